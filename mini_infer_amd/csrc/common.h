@@ -179,5 +179,5 @@ __device__ __forceinline__ void mi_store_cols(T* p, const float (&v)[V]) {
   }
 }
 
-static inline int ceil_div(int a, int b) { return (a + b - 1) / b; }
+static __host__ __device__ inline int ceil_div(int a, int b) { return (a + b - 1) / b; }
 static inline int64_t ceil_div64(int64_t a, int64_t b) { return (a + b - 1) / b; }

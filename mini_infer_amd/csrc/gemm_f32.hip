@@ -1,173 +1,299 @@
 // True float32 matrix product for the 32-bit path: C[M,N] = A[M,K] * W[N,K]^T.
-// Plain FMA, no reduced-precision matrix mode.  Each output element is summed by
-// one thread in the order of k, so a row's result does not depend on how many other
-// rows are in the batch or on where its tile lies.  The sum is carried in 64-bit and
-// rounded to float32 once, when it is written: an output differs from the exact product
-// of its float32 operands by that one rounding (relative 2.5e-8 on average), whatever K
-// is.  (Float32 sums in 16-deep slices added up with compensation measured 8e-8 at K =
-// 4,096, a plain float32 sum 2.7e-6; over 32 layers such errors are what the logits show.)
+// No reduced-precision matrix mode: float32 values are widened to 64-bit (exactly) and
+// multiplied and summed by the matrix cores' 64-bit instruction, and the sum is rounded to
+// float32 once, when it is written: an output differs from the exact product of its float32
+// operands by that one rounding (relative 2.5e-8 on average), whatever K is.  (Float32 sums
+// in 16-deep slices added up with compensation measured 8e-8 at K = 4,096, a plain float32
+// sum 2.7e-6; over 32 layers such errors are what the logits show.)
 //
-// 64x64 output tile per 256-thread block, 16-deep K slices staged in LDS, 4x4
-// outputs per thread.  Any M, N, K; rows of A and W may have strides.
+// Every output is summed in one fixed order that depends on K alone, in both kernels here, so
+// a row gives the same bits however many other rows its step has and wherever its tile lies:
+// K is cut into SEGMENTS runs of whole 32-value slices; inside a run one accumulator takes,
+// slice by slice, the slice's lower and then upper 16 values, of these the values 0, 4, 8, 12
+// first, then 1, 5, 9, 13 and so on (a lane of the matrix instruction's operand holds four
+// values that lie side by side, one of them per instruction); the runs' sums are added in
+// order.  Values past K are zeros and add nothing, exactly.
+//
+// What bounds it: the 64-bit matrix instruction (16x16x4) takes 64 cycles a SIMD, 76 TFLOP/s on
+// the whole part (the vector pipe's 64-bit multiply-add reached 51, and needs a widened operand
+// in registers for every one of them; the instruction shares it among 16 products).
 #include "common.h"
 
-#define BM 64
-#define BN 64
-#define BK 16
+typedef double f64x4_t __attribute__((ext_vector_type(4)));
 
+#define SEGMENTS 8
+#define SLICE 32       // values of K a step: one 128-byte line of a row
+#define BN 64
+
+static __host__ __device__ inline int segment_slices(int k) { return (k + SEGMENTS * SLICE - 1) / (SEGMENTS * SLICE); }
+
+__device__ __forceinline__ f64x4_t mma(float a, float w, f64x4_t acc) {
+  return __builtin_amdgcn_mfma_f64_16x16x4f64((double)a, (double)w, acc, 0, 0, 0);
+}
+
+// four values of a row from `at` on, zeros past its end
+template <bool ALIGNED>
+__device__ __forceinline__ float4 four_of_row(const float* row, int at, int k) {
+  if constexpr (ALIGNED) return at < k ? *reinterpret_cast<const float4*>(row + at) : make_float4(0.f, 0.f, 0.f, 0.f);
+  return make_float4(at < k ? row[at] : 0.f, at + 1 < k ? row[at + 1] : 0.f, at + 2 < k ? row[at + 2] : 0.f,
+                     at + 3 < k ? row[at + 3] : 0.f);
+}
+
+// Many rows: a block of 4 waves owns BM x 64 outputs, STAGE slices of both operands in LDS, the next ones in
+// flight in registers.  With 64 cycles an instruction the LDS is idle most of the time, so small tiles cost
+// nothing.  BM = 64 (a wave 32 x 32), one slice a stage, where there are at least four blocks a CU to cover one
+// another's barriers and loads; else BM = 32 (a wave 32 x 16): twice the blocks, four slices a stage.
+// ALIGNED: 16-byte loads (K, both row strides multiples of 4 values, both matrices on 16 bytes).
+template <int BM, int STAGE, bool ALIGNED>
 __global__ __launch_bounds__(256) void gemm_f32_kernel(const float* __restrict__ a, int64_t lda,
                                                        const float* __restrict__ w, int64_t ldw,
-                                                       float* __restrict__ c, int64_t ldc, int m,
-                                                       int n, int k) {
-  __shared__ float a_s[BK][BM + 4];
-  __shared__ float w_s[BK][BN + 4];
+                                                       float* __restrict__ c, int64_t ldc, int m, int n, int k) {
+  constexpr int LDS_ROW = STAGE * SLICE + 4;  // floats: 16-byte reads of 16 rows fall on different banks
+  constexpr int CT = BM == 64 ? 2 : 1;  // 16-column tiles of a wave (it has two tiles of rows)
+  constexpr int AL = STAGE * BM / 32, WL = STAGE * BN / 32;  // 16-byte pieces a thread stages
+  __shared__ __attribute__((aligned(16))) float a_s[BM][LDS_ROW];
+  __shared__ __attribute__((aligned(16))) float w_s[BN][LDS_ROW];
+  const int tid = threadIdx.x, wave = tid / MI_WAVE, lane = tid % MI_WAVE;
+  const int row0 = blockIdx.y * BM, col0 = blockIdx.x * BN;
+  const int wave_row = BM == 64 ? wave / 2 * 32 : 0, wave_col = BM == 64 ? wave % 2 * 32 : wave * 16;
+  const int r = lane % 16, quad = lane / 16;
+  constexpr int LANES = STAGE * SLICE / 4, ROWS = 256 / LANES;  // threads a row, rows a pass of the block's loads
+  const int l_row = tid / LANES, l_k = tid % LANES * 4;
 
-  const int tid = threadIdx.x;
-  const int row0 = blockIdx.y * BM;
-  const int col0 = blockIdx.x * BN;
-  const int ty = tid / 16, tx = tid % 16;
-
-  // loader mapping: thread loads 4 consecutive k of one row
-  const int l_row = tid / 4;
-  const int l_k = (tid % 4) * 4;
-
-  double acc[4][4];
+  float4 a_next[AL], w_next[WL];
+  auto fetch = [&](int k0) {
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = 0.0;
-
-  for (int k0 = 0; k0 < k; k0 += BK) {
-    {
-      const int r = row0 + l_row;
-      const float* src = a + (int64_t)r * lda + k0 + l_k;
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        a_s[l_k + i][l_row] = (r < m && k0 + l_k + i < k) ? src[i] : 0.f;
+    for (int i = 0; i < AL; ++i) {
+      const int row = row0 + l_row + ROWS * i;
+      a_next[i] = row < m ? four_of_row<ALIGNED>(a + (int64_t)row * lda, k0 + l_k, k) : make_float4(0.f, 0.f, 0.f, 0.f);
     }
-    {
-      const int r = col0 + l_row;
-      const float* src = w + (int64_t)r * ldw + k0 + l_k;
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
-        w_s[l_k + i][l_row] = (r < n && k0 + l_k + i < k) ? src[i] : 0.f;
+    for (int i = 0; i < WL; ++i) {
+      const int row = col0 + l_row + ROWS * i;
+      w_next[i] = row < n ? four_of_row<ALIGNED>(w + (int64_t)row * ldw, k0 + l_k, k) : make_float4(0.f, 0.f, 0.f, 0.f);
     }
+  };
+  f64x4_t total[2][CT], acc[2][CT];
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < CT; ++j) total[i][j] = acc[i][j] = f64x4_t{0.0, 0.0, 0.0, 0.0};
+
+  const int run = segment_slices(k), slices = ceil_div(k, SLICE);
+  int left = run;  // slices until the run's sum is complete
+  fetch(0);
+  for (int slice0 = 0; slice0 < slices; slice0 += STAGE) {
+    __syncthreads();  // the last slices' reads are done
+#pragma unroll
+    for (int i = 0; i < AL; ++i) *reinterpret_cast<float4*>(&a_s[l_row + ROWS * i][l_k]) = a_next[i];
+#pragma unroll
+    for (int i = 0; i < WL; ++i) *reinterpret_cast<float4*>(&w_s[l_row + ROWS * i][l_k]) = w_next[i];
     __syncthreads();
+    if (slice0 + STAGE < slices) fetch((slice0 + STAGE) * SLICE);
 #pragma unroll
-    for (int kk = 0; kk < BK; ++kk) {
-      double av[4], wv[4];
+    for (int slice = 0; slice < STAGE; ++slice) {  // (a slice past the last one is zeros)
 #pragma unroll
-      for (int i = 0; i < 4; ++i) av[i] = (double)a_s[kk][ty * 4 + i];
+      for (int half = 0; half < 2; ++half) {
+        const int at = SLICE * slice + 16 * half + 4 * quad;
+        float av[2][4], wv[CT][4];
 #pragma unroll
-      for (int j = 0; j < 4; ++j) wv[j] = (double)w_s[kk][tx * 4 + j];
+        for (int i = 0; i < 2; ++i)
+          *reinterpret_cast<float4*>(av[i]) = *reinterpret_cast<const float4*>(&a_s[wave_row + 16 * i + r][at]);
 #pragma unroll
-      for (int i = 0; i < 4; ++i)
+        for (int j = 0; j < CT; ++j)
+          *reinterpret_cast<float4*>(wv[j]) = *reinterpret_cast<const float4*>(&w_s[wave_col + 16 * j + r][at]);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = fma(av[i], wv[j], acc[i][j]);
-    }
-    __syncthreads();
-  }
-
+        for (int s = 0; s < 4; ++s)
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int r = row0 + ty * 4 + i;
-    if (r >= m) continue;
+          for (int i = 0; i < 2; ++i)
 #pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      const int col = col0 + tx * 4 + j;
-      if (col < n) c[(int64_t)r * ldc + col] = (float)acc[i][j];
-    }
-  }
-}
-
-// The same product for at most 16 rows (decode): a 64x64 tile would be three quarters empty and
-// its 16-byte loads per thread leave most of the memory system idle.  A block owns all rows
-// and 32 or 64 features; W is staged 64 deep (256 contiguous bytes of a row by a few threads),
-// and a thread sums one row x two or four features.  Every output is summed EXACTLY as above (in
-// the order of k, in 64-bit, rounded once); so a row gives the same bits whichever of the two
-// kernels its step takes.
-#define RM 16
-#define RK 64
-
-// TN = features per thread (the block owns 16 * TN): the more, the less is read from LDS per
-// product, the fewer blocks.
-template <int TN>
-__global__ __launch_bounds__(256) void gemm_f32_rows_kernel(const float* __restrict__ a, int64_t lda,
-                                                            const float* __restrict__ w, int64_t ldw,
-                                                            float* __restrict__ c, int64_t ldc, int m,
-                                                            int n, int k, int aligned) {
-  constexpr int RN = 16 * TN;
-  constexpr int W_PER = RN * RK / 256;  // consecutive k of one feature a thread stages: 8 or 16
-  __shared__ float a_s[RK][RM + 1];
-  __shared__ __attribute__((aligned(16))) float w_s[RK][RN + 4];
-  const int tid = threadIdx.x;
-  const int col0 = blockIdx.x * RN;
-  const int row = tid / 16, tx = tid % 16;  // this thread's outputs: row, features col0 + TN*tx ..
-  // loaders: W: W_PER consecutive k of one feature; A: 4 consecutive k of row tid / 16
-  const int w_feature = tid / (RK / W_PER), w_k = (tid % (RK / W_PER)) * W_PER;
-  const int w_row = col0 + w_feature;
-  const int a_row = tid / 16, a_k = (tid % 16) * 4;
-  double acc[TN];
-#pragma unroll
-  for (int j = 0; j < TN; ++j) acc[j] = 0.0;
-  for (int k0 = 0; k0 < k; k0 += RK) {
-    {
-      const float* src = w + (int64_t)w_row * ldw + k0 + w_k;
-      float v[W_PER];
-      if (aligned && w_row < n && k0 + w_k + W_PER <= k) {
-#pragma unroll
-        for (int i = 0; i < W_PER; i += 4) {
-          const float4 q = *reinterpret_cast<const float4*>(src + i);
-          v[i] = q.x; v[i + 1] = q.y; v[i + 2] = q.z; v[i + 3] = q.w;
-        }
-      } else {
-#pragma unroll
-        for (int i = 0; i < W_PER; ++i) v[i] = (w_row < n && k0 + w_k + i < k) ? src[i] : 0.f;
+            for (int j = 0; j < CT; ++j) acc[i][j] = mma(av[i][s], wv[j][s], acc[i][j]);
       }
+      if (--left == 0) {
+        left = run;
 #pragma unroll
-      for (int i = 0; i < W_PER; ++i) w_s[w_k + i][w_feature] = v[i];
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+          for (int j = 0; j < CT; ++j) {
+            total[i][j] += acc[i][j];
+            acc[i][j] = f64x4_t{0.0, 0.0, 0.0, 0.0};
+          }
+      }
     }
-    {
-      const float* src = a + (int64_t)a_row * lda + k0 + a_k;
-#pragma unroll
-      for (int i = 0; i < 4; ++i) a_s[a_k + i][a_row] = (a_row < m && k0 + a_k + i < k) ? src[i] : 0.f;
-    }
-    __syncthreads();
-    // (staged values past K are zeros: they add nothing, exactly)
-#pragma unroll
-    for (int kk = 0; kk < RK; ++kk) {
-      const double av = (double)a_s[kk][row];
-#pragma unroll
-      for (int j = 0; j < TN; ++j) acc[j] = fma(av, (double)w_s[kk][TN * tx + j], acc[j]);
-    }
-    __syncthreads();
   }
-  if (row < m) {
 #pragma unroll
-    for (int j = 0; j < TN; ++j) {
-      const int col = col0 + TN * tx + j;
-      if (col < n) c[(int64_t)row * ldc + col] = (float)acc[j];
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < CT; ++j) total[i][j] += acc[i][j];  // (the last run may be short)
+#pragma unroll
+  for (int i = 0; i < 2; ++i)
+#pragma unroll
+    for (int j = 0; j < CT; ++j)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        // (the 64-bit instruction's result: register e of a lane is row 4 * e + lane / 16)
+        const int row = row0 + wave_row + 16 * i + 4 * e + quad, col = col0 + wave_col + 16 * j + r;
+        if (row < m && col < n) c[(int64_t)row * ldc + col] = (float)total[i][j][e];
+      }
+}
+
+// Few rows (decode): bound by reading W once.  A block owns 16 * RT rows and 16 * FT features; its 8 waves take
+// one run of K each (the order above), every wave streams its part of the weights from memory, two slices ahead,
+// and the runs' sums meet in LDS.  LINES: whole lines of W, non-temporal, brought into operand order by lane
+// exchanges (common.h): rows of W on 128 bytes, K a multiple of 32, A on 16 bytes; else guarded single values.
+// Rows past m and features past n repeat the last one and are not written.
+template <int RT, int FT, bool LINES>
+__global__ __launch_bounds__(SEGMENTS * MI_WAVE) void gemm_f32_rows_kernel(const float* __restrict__ a, int64_t lda,
+                                                            const float* __restrict__ w, int64_t ldw,
+                                                            float* __restrict__ c, int64_t ldc, int m, int n, int k) {
+  __shared__ double sums[SEGMENTS][RT * FT][16][17];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / MI_WAVE), lane = threadIdx.x % MI_WAVE;
+  const int col0 = blockIdx.x * 16 * FT;
+  const int r = lane % 16, quad = lane / 16;
+  const float* a_row[RT];
+  f64x4_t acc[RT][FT];
+#pragma unroll
+  for (int i = 0; i < RT; ++i) {
+    a_row[i] = a + (int64_t)min(16 * i + r, m - 1) * lda;
+#pragma unroll
+    for (int f = 0; f < FT; ++f) acc[i][f] = f64x4_t{0.0, 0.0, 0.0, 0.0};
+  }
+  const int run = segment_slices(k), slices = ceil_div(k, SLICE);
+  const int first = min(wave * run, slices), last = min(first + run, slices);
+
+  if constexpr (LINES) {
+    // (offsets from the first of the block's rows: at most 32 rows of at most 2^26 bytes)
+    uint32_t lower[FT], upper[FT];
+#pragma unroll
+    for (int f = 0; f < FT; ++f) {
+      const int row = 16 * f + line_row_of_lane(lane), most = n - 1 - col0;
+      lower[f] = (uint32_t)min(row, most) * (uint32_t)(ldw * 4) + line_chunk_of_lane(lane);
+      upper[f] = (uint32_t)min(row + 8, most) * (uint32_t)(ldw * 4) + line_chunk_of_lane(lane);
     }
+    const float* w_block = w + (int64_t)col0 * ldw;
+    constexpr int AHEAD = 2;
+    bf16x8_t lo[AHEAD][FT], hi[AHEAD][FT];  // 16-byte pieces; what they hold is float32
+    float4 av[AHEAD][RT][2];
+    auto fetch = [&](int slot, int slice) {
+#pragma unroll
+      for (int f = 0; f < FT; ++f) load_line_pair(w_block, 2 * (int64_t)slice, lower[f], upper[f], lo[slot][f], hi[slot][f]);
+#pragma unroll
+      for (int i = 0; i < RT; ++i) {
+        av[slot][i][0] = *reinterpret_cast<const float4*>(a_row[i] + slice * SLICE + 4 * quad);
+        av[slot][i][1] = *reinterpret_cast<const float4*>(a_row[i] + slice * SLICE + 16 + 4 * quad);
+      }
+    };
+#pragma unroll
+    for (int s = 0; s < AHEAD; ++s)
+      if (first + s < last) fetch(s, first + s);
+    for (int at = first; at < last; at += AHEAD) {
+#pragma unroll
+      for (int s = 0; s < AHEAD; ++s) {
+        if (at + s < last) {
+          float wv[FT][2][4], xv[RT][2][4];
+#pragma unroll
+          for (int f = 0; f < FT; ++f) {
+            lines_to_operands(lo[s][f], hi[s][f]);
+            __builtin_memcpy(wv[f][0], &lo[s][f], 16);
+            __builtin_memcpy(wv[f][1], &hi[s][f], 16);
+          }
+          __builtin_memcpy(xv, av[s], sizeof(xv));
+          if (at + s + AHEAD < last) fetch(s, at + s + AHEAD);
+#pragma unroll
+          for (int half = 0; half < 2; ++half)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+              for (int i = 0; i < RT; ++i)
+#pragma unroll
+                for (int f = 0; f < FT; ++f) acc[i][f] = mma(xv[i][half][e], wv[f][half][e], acc[i][f]);
+        }
+      }
+    }
+  } else {
+    for (int slice = first; slice < last; ++slice) {
+#pragma unroll
+      for (int half = 0; half < 2; ++half) {
+        const int at = slice * SLICE + 16 * half + 4 * quad;
+        float xv[RT][4], wv[FT][4];
+#pragma unroll
+        for (int i = 0; i < RT; ++i) *reinterpret_cast<float4*>(xv[i]) = four_of_row<false>(a_row[i], at, k);
+#pragma unroll
+        for (int f = 0; f < FT; ++f)
+          *reinterpret_cast<float4*>(wv[f]) = four_of_row<false>(w + (int64_t)min(col0 + 16 * f + r, n - 1) * ldw, at, k);
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+#pragma unroll
+          for (int i = 0; i < RT; ++i)
+#pragma unroll
+            for (int f = 0; f < FT; ++f) acc[i][f] = mma(xv[i][e], wv[f][e], acc[i][f]);
+      }
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < RT; ++i)
+#pragma unroll
+    for (int f = 0; f < FT; ++f)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) sums[wave][i * FT + f][4 * e + quad][r] = acc[i][f][e];
+  __syncthreads();
+  for (int at = threadIdx.x; at < 256 * RT * FT; at += SEGMENTS * MI_WAVE) {
+    const int tile = at / 256, row = tile / FT * 16 + at / 16 % 16, col = col0 + tile % FT * 16 + at % 16;
+    double total = 0.0;
+#pragma unroll
+    for (int s = 0; s < SEGMENTS; ++s) total += sums[s][tile][at / 16 % 16][at % 16];
+    if (row < m && col < n) c[(int64_t)row * ldc + col] = (float)total;
   }
 }
 
+template <int BM, int STAGE>
+static void launch_tiles(const float* a, int64_t lda, const float* w, int64_t ldw, float* c, int64_t ldc, int m, int n,
+                         int k, bool aligned, hipStream_t stream) {
+  dim3 grid(ceil_div(n, BN), ceil_div(m, BM));
+  if (aligned) gemm_f32_kernel<BM, STAGE, true><<<grid, 256, 0, stream>>>(a, lda, w, ldw, c, ldc, m, n, k);
+  else gemm_f32_kernel<BM, STAGE, false><<<grid, 256, 0, stream>>>(a, lda, w, ldw, c, ldc, m, n, k);
+}
+
+template <int RT, int FT>
+static void launch_rows(const float* a, int64_t lda, const float* w, int64_t ldw, float* c, int64_t ldc, int m, int n,
+                        int k, bool lines, hipStream_t stream) {
+  const int grid = ceil_div(n, 16 * FT), block = SEGMENTS * MI_WAVE;
+  if (lines) gemm_f32_rows_kernel<RT, FT, true><<<grid, block, 0, stream>>>(a, lda, w, ldw, c, ldc, m, n, k);
+  else gemm_f32_rows_kernel<RT, FT, false><<<grid, block, 0, stream>>>(a, lda, w, ldw, c, ldc, m, n, k);
+}
+
+// Which kernel, with microseconds at rows x N x K (weights from memory).  Before: 64-bit multiply-adds on the vector
+// pipe, 4 x 4 outputs a thread, and a kernel of its own for up to 16 rows only.
+//     3 x 2048 x 2048     75.6 ->   9.0     20 x  2048 x 2048   317 ->  15.0     509 x  2048 x 2048    327 ->  88
+//     3 x 16384 x 2048     107 ->  30.7     20 x 16384 x 2048   349 ->  46.0     509 x  3072 x 2048    378 -> 125
+//     3 x 128256 x 2048    419 ->   192     60 x  2048 x 2048   320 ->  26.3     509 x 16384 x 2048   1060 -> 580
+//     3 x 2048 x 8192      322 ->  28.1     60 x 16384 x 2048   355 -> 102       509 x  2048 x 8192   1340 -> 345
+// 3 rows of 16,384 features and more run at the rate of a large copy; 580 us is 59 TFLOP/s, where the vendor
+// library's 64-bit product reaches 64.  Two tiles of features a wave from 8,192 on (fewer blocks below that would
+// leave CUs idle).  Up to 32 rows the streaming kernel always (20 x 128256 x 2048: 325 against 320 for the tiles,
+// 20 x 16384: 46 against 66); up to 64 rows where there are few features (60 x 2048: 26 against 64; 60 x 128256:
+// 810 against 580, every block reads all the rows' activations).
 extern "C" int mi_gemm_f32(const float* a, int64_t lda, const float* w, int64_t ldw, float* c,
                            int64_t ldc, int m, int n, int k, hipStream_t stream) {
   MI_REQUIRE(m >= 0 && n > 0 && k > 0, "gemm_f32: bad sizes m=%d n=%d k=%d", m, n, k);
   MI_REQUIRE(lda >= k && ldw >= k && ldc >= n, "gemm_f32: a row stride is shorter than its row");
-  MI_REQUIRE(ceil_div(m, BM) <= 65535, "gemm_f32: m=%d is too large for one call", m);
+  MI_REQUIRE(ceil_div(m, 64) <= 65535, "gemm_f32: m=%d is too large for one call", m);
   if (m == 0) return MI_OK;
-  if (m <= RM) {
-    const int aligned = ldw % 4 == 0 && ((uintptr_t)w % 16 == 0) ? 1 : 0;
-    // (four features a thread where that still leaves a block for every CU; measured at 8B sizes,
-    // 8 rows: 34.7 ms a step this way, 45.5 with four or eight everywhere, 36.5 with two everywhere)
-    if (n >= 8192) gemm_f32_rows_kernel<4><<<ceil_div(n, 64), 256, 0, stream>>>(a, lda, w, ldw, c, ldc, m, n, k, aligned);
-    else gemm_f32_rows_kernel<2><<<ceil_div(n, 32), 256, 0, stream>>>(a, lda, w, ldw, c, ldc, m, n, k, aligned);
+  const bool a16 = lda % 4 == 0 && (uintptr_t)a % 16 == 0, w16 = ldw % 4 == 0 && (uintptr_t)w % 16 == 0;
+  const bool wide = n >= 8192;
+  if (m <= 32 || (m <= 64 && !wide)) {
+    // (the streaming loads' offsets reach over a block's 32 features in 32 bits: ldw under 2^24 values)
+    const bool lines = a16 && k % SLICE == 0 && ldw % 32 == 0 && (uintptr_t)w % 128 == 0 && ldw < (1 << 24);
+    if (m > 32) launch_rows<4, 1>(a, lda, w, ldw, c, ldc, m, n, k, lines, stream);
+    else if (m > 16) launch_rows<2, 1>(a, lda, w, ldw, c, ldc, m, n, k, lines, stream);
+    else if (wide) launch_rows<1, 2>(a, lda, w, ldw, c, ldc, m, n, k, lines, stream);
+    else launch_rows<1, 1>(a, lda, w, ldw, c, ldc, m, n, k, lines, stream);
     MI_CHECK_LAUNCH("gemm_f32 (few rows)");
     return MI_OK;
   }
-  dim3 grid(ceil_div(n, BN), ceil_div(m, BM));
-  gemm_f32_kernel<<<grid, 256, 0, stream>>>(a, lda, w, ldw, c, ldc, m, n, k);
+  const bool aligned = a16 && w16 && k % 4 == 0;
+  if ((int64_t)ceil_div(n, BN) * ceil_div(m, 64) < 1024 && m <= 32 * 65535) launch_tiles<32, 4>(a, lda, w, ldw, c, ldc, m, n, k, aligned, stream);
+  else launch_tiles<64, 1>(a, lda, w, ldw, c, ldc, m, n, k, aligned, stream);
   MI_CHECK_LAUNCH("gemm_f32");
   return MI_OK;
 }

@@ -118,6 +118,25 @@ def test_gemm_f32_is_true_float32(m, n, k):
     assert torch.equal(ops.gemm_f32(wide[:, :k], w), ops.gemm_f32(wide[:, :k].contiguous(), w))
 
 
+@pytest.mark.parametrize("m,n,k", [(1, 16, 32), (16, 8200, 96), (17, 33, 544), (32, 100, 2048), (33, 8, 352), (64, 50, 257), (65, 130, 4096),
+                                   (50, 8192, 160), (700, 6200, 100), (90, 70, 36)])
+def test_gemm_f32_kernels_and_alignments_agree(m, n, k):
+    """Every kernel (few rows in 1, 2 or 4 tiles, large and small blocks) and both ways of loading (16 bytes, single values) sum
+    an output in the same order: the same bits, and the exact product rounded once (half an ulp, plus what 64-bit sums lose)."""
+    from mini_infer_amd import ops
+
+    a, w = _rand(m, k, seed=31), _rand(n, k, seed=32)
+    out = ops.gemm_f32(a, w)
+    exact = a.double() @ w.double().T
+    assert ((out.double() - exact).abs() <= 2.0 ** -24 * exact.abs() + 1e-12 * math.sqrt(k)).all()
+    for rows in (1, 16, 17, 40, 65):
+        if rows < m:
+            assert torch.equal(ops.gemm_f32(a[:rows], w), out[:rows]), rows
+    odd_a, odd_w = torch.zeros(m, k + 1, device=DEV), torch.zeros(n, k + 3, device=DEV)
+    odd_a[:, 1:], odd_w[:, 3:] = a, w
+    assert torch.equal(ops.gemm_f32(odd_a[:, 1:], odd_w[:, 3:]), out)
+
+
 @pytest.mark.parametrize(
     "m,n,k",
     [(1, 4096, 4096), (8, 6144, 4096), (16, 96, 64), (7, 301, 96), (13, 130, 160), (16, 1000, 14336),
