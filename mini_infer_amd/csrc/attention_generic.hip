@@ -1,6 +1,6 @@
 // Paged causal attention, plain-FMA version: the float32 path of the engine and
-// the fallback for sizes the matrix-core kernels refuse.  One 64-lane wave per
-// (query token, key/value head, up to 4 query heads of its group, key split).
+// the fallback for sizes the matrix-core kernels refuse.  One 64-lane wave, or four that share
+// its keys, per (query token, key/value head, up to 4 query heads of its group, key split).
 // Lanes own keys while scores are computed (one key row per lane, q broadcast
 // from LDS) and own output dims while values are accumulated.  The softmax is an
 // online one (running max).  For bfloat16 inputs the scores, the softmax's sum and the
@@ -61,9 +61,17 @@ __device__ __forceinline__ S head_gate(const T* gate, int64_t at) {
   else return mi_logistic(to_f32(gate[at]));
 }
 
-// VEC: head_dim is a multiple of 16 (16-byte loads, no guards inside a row)
-template <typename T, int VPL, bool VEC>
-__global__ __launch_bounds__(64) void attn_generic_kernel(
+// a lane's value as a scalar; the lane number is the same for the whole wave
+__device__ __forceinline__ float from_lane(float v, int lane) {
+  return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(v), lane));
+}
+
+// VEC: head_dim is a multiple of 16 (16-byte loads, no guards inside a row).
+// WAVES: the block's waves take every WAVES-th 64 keys of the range and are merged in S at the end.  One wave walks
+// its keys at the latency of its loads and instructions, and a few decoded tokens are too few waves to hide that;
+// measured at attn_generic_launch.
+template <typename T, int VPL, bool VEC, int WAVES>
+__global__ __launch_bounds__(64 * WAVES) void attn_generic_kernel(
     const T* __restrict__ q, int64_t q_row_stride, const T* __restrict__ k_pages,
     const T* __restrict__ v_pages, const int* __restrict__ block_table, int max_blocks,
     const int* __restrict__ token_request, const int* __restrict__ positions, T* __restrict__ out,
@@ -84,10 +92,11 @@ __global__ __launch_bounds__(64) void attn_generic_kernel(
   const int nh = min(GT, group - g0);
   const int head0 = kvh * group + g0;
   const int split = blockIdx.z;
-  const int lane = threadIdx.x;
+  const int lane = threadIdx.x % MI_WAVE;
+  const int wave = WAVES == 1 ? 0 : __builtin_amdgcn_readfirstlane(threadIdx.x / MI_WAVE);
 
   const T* q_row = q + (int64_t)t * q_row_stride + (int64_t)head0 * head_dim;
-  for (int i = lane; i < GT * head_dim; i += MI_WAVE)
+  for (int i = threadIdx.x; i < GT * head_dim; i += WAVES * MI_WAVE)
     q_lds[i] = (i < nh * head_dim) ? (S)to_f32(q_row[i]) * (S)scale : (S)0;
   __syncthreads();
 
@@ -116,7 +125,7 @@ __global__ __launch_bounds__(64) void attn_generic_kernel(
 #pragma unroll
   for (int g = 0; g < GT; ++g) slope[g] = (slopes != nullptr && g < nh) ? slopes[head0 + g] : 0.f;
 
-  for (int base = a; base < b; base += MI_WAVE) {
+  for (int base = a + wave * MI_WAVE; base < b; base += WAVES * MI_WAVE) {
     const int key = base + lane;
     const bool valid = key < b;
     int row_idx = 0;
@@ -138,30 +147,35 @@ __global__ __launch_bounds__(64) void attn_generic_kernel(
       for (int g = 0; g < GT; ++g)
 #pragma unroll
         for (int e = 0; e < 4; ++e) s4[g][e] = 0;
-      for (int d = 0; d < head_dim; d += KV) {
-        float kf[KV];
+      // (16 values of the key row at a time where rows are whole 16s: their loads are in flight together)
+      constexpr int RUN = VEC ? 16 : KV;
+      for (int d0 = 0; d0 < head_dim; d0 += RUN) {
+        float kf[RUN];
         if constexpr (VEC) {
-          const Pack<T, KV> kk = *reinterpret_cast<const Pack<T, KV>*>(k_row + d);
 #pragma unroll
-          for (int e = 0; e < KV; ++e) kf[e] = to_f32(kk.v[e]);
+          for (int at = 0; at < RUN; at += KV) {
+            const Pack<T, KV> kk = *reinterpret_cast<const Pack<T, KV>*>(k_row + d0 + at);
+#pragma unroll
+            for (int e = 0; e < KV; ++e) kf[at + e] = to_f32(kk.v[e]);
+          }
         } else {
           // pairs of elements; an even head size ends after the first or the second pair
-          const Pack<T, 2> k0 = *reinterpret_cast<const Pack<T, 2>*>(k_row + d);
+          const Pack<T, 2> k0 = *reinterpret_cast<const Pack<T, 2>*>(k_row + d0);
           kf[0] = to_f32(k0.v[0]);
           kf[1] = to_f32(k0.v[1]);
           kf[2] = kf[3] = 0.f;
-          if (d + 2 < head_dim) {
-            const Pack<T, 2> k1 = *reinterpret_cast<const Pack<T, 2>*>(k_row + d + 2);
+          if (d0 + 2 < head_dim) {
+            const Pack<T, 2> k1 = *reinterpret_cast<const Pack<T, 2>*>(k_row + d0 + 2);
             kf[2] = to_f32(k1.v[0]);
             kf[3] = to_f32(k1.v[1]);
           }
         }
 #pragma unroll
-        for (int e = 0; e < KV; ++e) {
-          if (!VEC && d + e >= head_dim) break;
+        for (int e = 0; e < RUN; ++e) {
+          if (!VEC && d0 + e >= head_dim) break;
 #pragma unroll
           for (int g = 0; g < GT; ++g) {
-            const S qv = q_lds[g * head_dim + d + e];
+            const S qv = q_lds[g * head_dim + d0 + e];
             if constexpr (sizeof(S) == 8) s4[g][e % 4] = fma(qv, (S)kf[e], s4[g][e % 4]);
             else s4[g][e % 4] = fmaf(qv, kf[e], s4[g][e % 4]);
           }
@@ -194,35 +208,84 @@ __global__ __launch_bounds__(64) void attn_generic_kernel(
       for (int v = 0; v < VPL; ++v) acc[g][v] *= (S)alpha;
       m[g] = m_new;
     }
+    // value rows eight at a time, so that eight loads are in flight (past the last key: that key again, weight 0)
+    constexpr int BATCH = 8;
     const int n_valid = min(MI_WAVE, b - base);
-    for (int j = 0; j < n_valid; ++j) {
-      const int rj = __shfl(row_idx, j, MI_WAVE);
-      float vv[VPL];
+    for (int j0 = 0; j0 < n_valid; j0 += BATCH) {
+      float vv[BATCH][VPL];
 #pragma unroll
-      for (int v = 0; v < VPL; ++v) vv[v] = 0.f;
-      if (owns_dims) {
-        const T* v_row = v_pages + (int64_t)rj * v_row_stride + lane * VPL;
-        if constexpr (VEC || VPL <= 2) {  // (an even head size: a pair never straddles the row's end)
-          const Pack<T, VPL> pk = *reinterpret_cast<const Pack<T, VPL>*>(v_row);
+      for (int u = 0; u < BATCH; ++u) {
+        const int rj = __builtin_amdgcn_readlane(row_idx, min(j0 + u, n_valid - 1));
 #pragma unroll
-          for (int v = 0; v < VPL; ++v) vv[v] = to_f32(pk.v[v]);
-        } else {
+        for (int v = 0; v < VPL; ++v) vv[u][v] = 0.f;
+        if (owns_dims) {
+          const T* v_row = v_pages + (int64_t)rj * v_row_stride + lane * VPL;
+          if constexpr (VEC || VPL <= 2) {  // (an even head size: a pair never straddles the row's end)
+            const Pack<T, VPL> pk = *reinterpret_cast<const Pack<T, VPL>*>(v_row);
 #pragma unroll
-          for (int v = 0; v < VPL; v += 2) {
-            if (lane * VPL + v < v_dim) {
-              const Pack<T, 2> pk = *reinterpret_cast<const Pack<T, 2>*>(v_row + v);
-              vv[v] = to_f32(pk.v[0]);
-              vv[v + 1] = to_f32(pk.v[1]);
+            for (int v = 0; v < VPL; ++v) vv[u][v] = to_f32(pk.v[v]);
+          } else {
+#pragma unroll
+            for (int v = 0; v < VPL; v += 2) {
+              if (lane * VPL + v < v_dim) {
+                const Pack<T, 2> pk = *reinterpret_cast<const Pack<T, 2>*>(v_row + v);
+                vv[u][v] = to_f32(pk.v[0]);
+                vv[u][v + 1] = to_f32(pk.v[1]);
+              }
             }
           }
         }
       }
 #pragma unroll
-      for (int g = 0; g < GT; ++g) {
-        const float pj = __shfl(p[g], j, MI_WAVE);
+      for (int u = 0; u < BATCH; ++u) {
+        if (j0 + u < n_valid) {
 #pragma unroll
-        for (int v = 0; v < VPL; ++v) acc[g][v] += (S)pj * (S)vv[v];
+          for (int g = 0; g < GT; ++g) {
+            const float pj = from_lane(p[g], j0 + u);
+#pragma unroll
+            for (int v = 0; v < VPL; ++v) acc[g][v] += (S)pj * (S)vv[u][v];
+          }
+        }
       }
+    }
+  }
+
+  if constexpr (WAVES > 1) {  // wave 0 takes over what the others have, in their order
+    S* merge = q_lds + GT * head_dim;  // [WAVES - 1][GT][VPL + 1][64], then their maxima
+    float* maxima = reinterpret_cast<float*>(merge + (WAVES - 1) * GT * (VPL + 1) * MI_WAVE);
+    if (wave > 0) {
+#pragma unroll
+      for (int g = 0; g < GT; ++g) {
+        S* to = merge + ((wave - 1) * GT + g) * (VPL + 1) * MI_WAVE + lane;
+#pragma unroll
+        for (int v = 0; v < VPL; ++v) to[v * MI_WAVE] = acc[g][v];
+        to[VPL * MI_WAVE] = l[g];
+        if (lane == 0) maxima[(wave - 1) * GT + g] = m[g];
+      }
+    }
+    __syncthreads();
+    if (wave > 0) return;
+#pragma unroll
+    for (int g = 0; g < GT; ++g) {
+      float top = m[g];
+#pragma unroll
+      for (int w = 0; w < WAVES - 1; ++w) top = fmaxf(top, maxima[w * GT + g]);
+      // (a wave without keys has the maximum -inf and nothing to add)
+      const S own = m[g] == -INFINITY ? (S)0 : (S)exp((double)m[g] - (double)top);
+      l[g] *= own;
+#pragma unroll
+      for (int v = 0; v < VPL; ++v) acc[g][v] *= own;
+#pragma unroll
+      for (int w = 0; w < WAVES - 1; ++w) {
+        const float m_w = maxima[w * GT + g];
+        if (m_w == -INFINITY) continue;
+        const S weight = (S)exp((double)m_w - (double)top);
+        const S* from = merge + (w * GT + g) * (VPL + 1) * MI_WAVE + lane;
+#pragma unroll
+        for (int v = 0; v < VPL; ++v) acc[g][v] += from[v * MI_WAVE] * weight;
+        l[g] += from[VPL * MI_WAVE] * weight;
+      }
+      m[g] = top;
     }
   }
 
@@ -357,18 +420,35 @@ static int attn_generic_launch(const void* q, int64_t q_row_stride, const void* 
   if (v_row_stride <= 0) v_row_stride = v_dim;
   const int group = q_heads / kv_heads;
   dim3 grid(num_tokens, kv_heads * ceil_div(group, GT), num_splits);
-  const size_t lds = sizeof(typename SumType<T>::type) * GT * head_dim;
+  using S = typename SumType<T>::type;
+  const size_t lds = sizeof(S) * GT * head_dim;
   const bool vec = head_dim % 16 == 0 && v_dim % 16 == 0 && v_row_stride % 16 == 0;
-#define MI_ATTN_LAUNCH(VPL, VEC)                                                                  \
-  attn_generic_kernel<T, VPL, VEC><<<grid, MI_WAVE, lds, stream>>>(                               \
+  // Four waves a range in the 32-bit path where one wave a range is fewer than two waves a SIMD (decode; values of
+  // up to 128 dims, which the merging's LDS holds).  One layer, 32 heads of 64 over 8 key/value heads, microseconds
+  // before and now: 3 tokens of up to 600 positions 113 -> 17.4, a prompt of 509 tokens 247 -> 148 (the batched
+  // loads alone, one wave a range).
+  const bool four = sizeof(S) == 8 && v_dim <= 128 && (int64_t)grid.x * grid.y * grid.z < 2048;
+#define MI_ATTN_LAUNCH_WAVES(VPL, VEC, WAVES, LDS)                                                \
+  attn_generic_kernel<T, VPL, VEC, WAVES><<<grid, WAVES * MI_WAVE, LDS, stream>>>(                \
       (const T*)q, q_row_stride, (const T*)k_pages, (const T*)v_pages, block_table, max_blocks,   \
       token_request, positions, (T*)out, out_row_stride, part_acc, part_ml, q_heads, kv_heads,    \
       head_dim, page_size, scale, window, num_splits, slopes, v_dim, v_row_stride, has_sink, sink_logit, mask_chunk, \
       softcap, sinks, (const T*)gate, gate_row_stride)
+#define MI_ATTN_LAUNCH(VPL, VEC)                                                                  \
+  do {                                                                                            \
+    if constexpr (sizeof(S) == 8 && VPL <= 2) {                                                   \
+      if (four) {                                                                                 \
+        MI_ATTN_LAUNCH_WAVES(VPL, VEC, 4, lds + 3 * GT * ((VPL + 1) * MI_WAVE * sizeof(S) + sizeof(float))); \
+        break;                                                                                    \
+      }                                                                                           \
+    }                                                                                             \
+    MI_ATTN_LAUNCH_WAVES(VPL, VEC, 1, lds);                                                       \
+  } while (0)
   if (v_dim <= 64) { if (vec) MI_ATTN_LAUNCH(1, true); else MI_ATTN_LAUNCH(1, false); }
   else if (v_dim <= 128) { if (vec) MI_ATTN_LAUNCH(2, true); else MI_ATTN_LAUNCH(2, false); }
   else if (v_dim <= 256) { if (vec) MI_ATTN_LAUNCH(4, true); else MI_ATTN_LAUNCH(4, false); }
   else { if (vec) MI_ATTN_LAUNCH(8, true); else MI_ATTN_LAUNCH(8, false); }
+#undef MI_ATTN_LAUNCH_WAVES
 #undef MI_ATTN_LAUNCH
   MI_CHECK_LAUNCH("attn_generic");
   if (num_splits > 1) {

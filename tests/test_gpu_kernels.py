@@ -649,6 +649,20 @@ def test_paged_attention_with_request_boundaries_known_on_the_device_only(mode, 
     assert np.abs(out.double().cpu().numpy() - expected).max() < _tol(dtype, 2)
 
 
+@pytest.mark.parametrize("q_heads,kv_heads,head_dim", [(8, 2, 64), (3, 3, 30), (10, 2, 128), (4, 1, 98)])
+@pytest.mark.parametrize("lengths", [[1], [63, 64, 65], [255, 256, 257, 300], [1, 2, 130, 511, 1030]])
+def test_paged_attention_float32_four_waves_a_range(q_heads, kv_heads, head_dim, lengths):
+    """Few decoded tokens in 32 bits: four waves share a range's keys (none, one or several 64s each, the last one short) and
+    are merged in 64 bits.  A weight of a key is rounded to float32 once (2^-24 relative), so is the result: 4e-7 of the largest
+    value leaves those two, and the partial results of cut ranges, room to add up."""
+    page_size = 16
+    case = _paged_case(torch.float32, q_heads, kv_heads, head_dim, page_size, lengths, [1] * len(lengths), seed=41)
+    scale = 1.0 / math.sqrt(head_dim)
+    out = _attend(case, q_heads, kv_heads, head_dim, scale, None, max(lengths))
+    expected = _attention_expected(case, scale, None)
+    assert np.abs(out.double().cpu().numpy() - expected).max() < 4e-7 * max(1.0, np.abs(expected).max())
+
+
 @pytest.mark.parametrize("window", [None, 700])
 def test_paged_attention_whole_long_prompts_many_tiles(window):
     """Whole prompts of a few thousand tokens beside a short one: dozens of tiles per head,
