@@ -1,0 +1,316 @@
+// Recurrences with a matrix state per head, over many tokens of a request, on the matrix cores.
+//
+//     S_t = a_t S_(t-1) + k_t u_t^T        o_t = S_t^T q_t        (S is dim x vdim, float32)
+//
+// Tokens are taken CHUNK at a time.  With G_i the product of a chunk's decays up to its token i (all factors below
+// are quotients G_i / G_j with j <= i, so at most 1) and S0 the state before it:
+//
+//     O = G Q S0 + W U            W_ij = (G_i / G_j) (q_i . k_j)   for j <= i
+//     S = G_last S0 + K^T (G_last / G) U
+//
+// where U's rows are the (scaled) values, or, for the gated delta rule,
+//
+//     U = T w (V - G K S0)        T = (1 + L)^-1,  L_ij = w_i (G_i / G_j) (k_i . k_j) for j < i.
+//
+// W, T and the factors do not depend on the state: a first launch makes them for all chunks and heads side by side
+// (delta_chunks.hip, decay_chunks.hip).  What is left is a walk over the chunks, here: a block keeps 16 columns of a
+// head's S, in the layout in which the matrix instruction leaves its results, which is also the layout of its second
+// operand with the rows of S in another order; its 4 waves own a quarter of the rows each, their partial K S0 and
+// Q S0 meet in LDS (one barrier a chunk), and everything after that is registers.  All operands are float32 and so is
+// the matrix instruction (16x16x4, 154 TFLOP/s): nothing is rounded that the token-by-token form keeps.
+//
+// What bounds it: the chain of one chunk after another. Measured at 2,048 tokens, one wave a SIMD: 2.9 us a chunk for
+// the delta rule (32 heads of 128 x 128: 68 matrix instructions a wave, 35 cycles each, make 1.0 us of it; the rest is
+// issuing some 30 loads of operands one chunk ahead and the exchange through LDS), 1.6 us for the others. Whole calls
+// with the first launch and the norm, token by token before: delta rule 896 -> 225 us, decay per head (64 heads of
+// 128 x 64) 717 -> 118, decay per channel (16 heads of 128 x 256) 772 -> 146. Waiting for everything in flight at the
+// barrier cost 2 us a chunk more. A chunk of 32: at twice that W and T (quadratic) weigh as much as the products with
+// the state, and the inverse no longer stays in a wave's registers.
+#pragma once
+#include "common.h"
+
+#define CHUNK 32
+
+namespace chunk_scan {
+
+enum { PER_CHANNEL = 0, PER_HEAD = 1, DELTA = 2 };
+
+typedef float f32x4_t __attribute__((ext_vector_type(4)));
+
+// What the first launch leaves, per chunk (a request's chunks lie one after another from `first_chunk` on).
+struct Made {
+  float* q;       // [chunks][shares][CHUNK][pad]; PER_CHANNEL: times G_i
+  float* k;       // the same (DELTA only)
+  float* kt;      // [chunks][shares][pad][CHUNK]; PER_CHANNEL: times G_last / G_j
+  float* within;  // W [chunks][heads][CHUNK][CHUNK]; PER_HEAD: for U = V, its columns times the step sizes
+  float* solve;   // T w, the same (DELTA only)
+  float* factor;  // [chunks][heads][2][CHUNK]: G, and G_last / G (PER_HEAD: times the step sizes); not PER_CHANNEL
+  float* fade;    // G_last: PER_CHANNEL [chunks][heads][pad]
+  int shares;     // rows q and k are shared by heads / shares heads
+};
+
+// The chunk number of a request's first chunk: requests' chunks never meet, since b + cu[b] / CHUNK grows by at least
+// the chunks of request b from one request to the next.
+__device__ __forceinline__ int first_chunk(int cu_b, int b) { return cu_b / CHUNK + b; }
+static inline int64_t chunk_count(int tokens, int requests) { return (int64_t)tokens / CHUNK + requests; }
+
+// Which request a chunk number belongs to: all threads of the block call this; -1: no request's.
+__device__ __forceinline__ int request_of_chunk(int chunk, const int* __restrict__ cu, int requests, int* shared_answer) {
+  if (threadIdx.x == 0) *shared_answer = -1;
+  __syncthreads();
+  for (int b = threadIdx.x; b < requests; b += blockDim.x) {
+    const int first = first_chunk(cu[b], b), tokens = cu[b + 1] - cu[b];
+    if (chunk >= first && chunk < first + (tokens + CHUNK - 1) / CHUNK) *shared_answer = b;
+  }
+  __syncthreads();
+  return *shared_answer;
+}
+
+// N values of a row from `at` on as float32, zeros from `dim` on (or all of them); `eights`: rows lie on 16 bytes in whole 8s.
+template <int N>
+__device__ __forceinline__ void row_values(const bf16_t* row, int at, int dim, bool eights, bool in, float (&v)[N]) {
+  static_assert(N % 8 == 0, "eight values a load");
+  if (eights) {
+#pragma unroll
+    for (int e = 0; e < N; e += 8) {
+      const bool has = in && at + e < dim;
+      const uint4 got = *reinterpret_cast<const uint4*>(row + (at + e < dim ? at + e : 0));
+      const uint32_t keep = has ? ~0u : 0u;
+      const uint32_t words[4] = {got.x & keep, got.y & keep, got.z & keep, got.w & keep};
+#pragma unroll
+      for (int w = 0; w < 4; ++w) {
+        v[e + 2 * w] = __uint_as_float(words[w] << 16);
+        v[e + 2 * w + 1] = __uint_as_float(words[w] & 0xFFFF0000u);
+      }
+    }
+  } else {
+#pragma unroll
+    for (int e = 0; e < N; ++e) v[e] = in && at + e < dim ? to_f32(row[at + e]) : 0.f;
+  }
+}
+static inline bool in_eights(const void* rows, int64_t stride, int64_t column, int dim) {
+  return (uintptr_t)rows % 16 == 0 && stride % 8 == 0 && column % 8 == 0 && dim % 8 == 0;
+}
+
+struct WalkArgs {
+  Made made;
+  const bf16_t* v;  // value rows
+  int64_t v_stride;  // under MAX_ROW values: offsets inside a chunk are 32-bit
+  int v_col;  // first column of head 0
+  const float* skip;  // PER_HEAD: per head, times the value, added to the read-out; may be null
+  float* state;       // [slots + 1][heads][vdim][pad]
+  int64_t state_stride;
+  const int *cu, *slots;
+  int num_slots;
+  float* out;  // float32 [tokens, heads * vdim]
+  int heads, vdim;
+};
+constexpr int64_t MAX_ROW = 1 << 24;
+
+__device__ __forceinline__ f32x4_t mma(float a, float b, f32x4_t acc) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, acc, 0, 0, 0); }
+__device__ __forceinline__ f32x4_t mma4(const float4& a, const f32x4_t& b, f32x4_t acc) {
+  acc = mma(a.x, b[0], acc), acc = mma(a.y, b[1], acc), acc = mma(a.z, b[2], acc);
+  return mma(a.w, b[3], acc);
+}
+__device__ __forceinline__ float4 load4(const float* p) { return *reinterpret_cast<const float4*>(p); }
+__device__ __forceinline__ f32x4_t scaled(const float4& s, const f32x4_t& v) { return f32x4_t{s.x * v[0], s.y * v[1], s.z * v[2], s.w * v[3]}; }
+
+// A barrier for LDS alone: __syncthreads() would also wait for the next chunk's operands, which are in flight (5.3 us a
+// chunk with it).
+__device__ __forceinline__ void lds_barrier() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+  __builtin_amdgcn_s_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+// One chunk's operands in a lane's registers.  Row tiles t of 16 tokens; a lane's four of a tile: tokens 16 t + 4 * (lane / 16) ..,
+// or, as first operand, token 16 t + lane % 16 and four rows of S (or tokens) side by side.
+template <int DT, int MODE>
+struct Operands {
+  float4 q[2][DT], k[MODE == DELTA ? 2 : 1][DT], kt[2][DT];
+  float4 within[2], solve[MODE == DELTA ? 3 : 1];
+  float4 g[2], tail[2], fade[MODE == PER_CHANNEL ? DT : 1];
+  float g_last;
+  uint32_t v[2][4];  // as read
+};
+
+// grid: heads * column blocks (the heads side by side, so that an XCD's blocks share their chunk data), requests; 256 threads.
+// DT: 16-row tiles of S a wave keeps; pad = 64 * DT.  One wave a SIMD walks, so what a chunk costs is what a wave issues:
+// addresses are a base that is the same for the wave plus a lane's offset made once, without branches (at the end of
+// one everything in flight would be waited for) and multiplications.
+template <int DT, int MODE>
+__global__ __launch_bounds__(256, MODE == DELTA || DT > 2 ? 1 : 2) void walk_kernel(WalkArgs p) {
+  constexpr int PAD = 64 * DT;
+  constexpr int SUMS = MODE == DELTA ? 4 : 2;
+  __shared__ f32x4_t parts[2][4][SUMS][MI_WAVE];
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / MI_WAVE), lane = threadIdx.x % MI_WAVE;
+  const int head = blockIdx.x % p.heads, b = blockIdx.y;
+  const uint32_t r = lane % 16, quad = lane / 16;
+  const int col = blockIdx.x / p.heads * 16 + r;
+  const bool live = col < p.vdim;
+  const int first = p.cu[b], last = p.cu[b + 1];
+  if (last <= first) return;
+  const int slot = p.slots[b];
+  const int row0 = 16 * DT * wave;  // of S
+  float* mine = p.state + (int64_t)((slot < 0 || slot >= p.num_slots) ? p.num_slots : slot) * p.state_stride +
+                ((int64_t)head * p.vdim + (live ? col : 0)) * PAD + row0 + 4 * quad;
+  f32x4_t S[DT];
+#pragma unroll
+  for (int d = 0; d < DT; ++d) S[d] = live ? *reinterpret_cast<const f32x4_t*>(mine + 16 * d) : f32x4_t{0.f, 0.f, 0.f, 0.f};
+  const int share = head / (p.heads / p.made.shares);
+  const int chunk0 = first_chunk(first, b), chunks = (last - first + CHUNK - 1) / CHUNK;
+  const float skip = (MODE == PER_HEAD && p.skip) ? p.skip[head] : 0.f;
+  const int out_stride = p.heads * p.vdim;
+  // a lane's offsets
+  const uint32_t at_row = r * PAD + 4 * quad, at_column = r * CHUNK + 4 * quad;
+  uint32_t v_at[2][4], out_at[4];
+#pragma unroll
+  for (int e = 0; e < 4; ++e) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t) v_at[t][e] = (16 * t + 4 * quad + e) * (uint32_t)p.v_stride;
+    out_at[e] = (16 * (wave & 1) + 4 * quad + e) * (uint32_t)out_stride + (uint32_t)col;
+  }
+  const uint32_t v_lane = live ? (uint32_t)col : 0u;
+
+  auto fetch = [&](int n, Operands<DT, MODE>& o) {
+    const int64_t chunk = chunk0 + n, rows = chunk * p.made.shares + share, of = chunk * p.heads + head;
+    const float *q = p.made.q + rows * CHUNK * PAD + row0, *kt = p.made.kt + rows * PAD * CHUNK + row0 * CHUNK;
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int d = 0; d < DT; ++d) {
+        o.q[t][d] = load4(q + 16 * t * PAD + 16 * d + at_row);
+        o.kt[t][d] = load4(kt + 16 * d * CHUNK + 16 * t + at_column);
+      }
+    if constexpr (MODE == DELTA) {
+      const float* k = p.made.k + rows * CHUNK * PAD + row0;
+#pragma unroll
+      for (int t = 0; t < 2; ++t)
+#pragma unroll
+        for (int d = 0; d < DT; ++d) o.k[t][d] = load4(k + 16 * t * PAD + 16 * d + at_row);
+      const float* solve = p.made.solve + of * CHUNK * CHUNK;
+      o.solve[0] = load4(solve + at_column);
+      o.solve[1] = load4(solve + 16 * CHUNK + at_column);
+      o.solve[2] = load4(solve + 16 * CHUNK + 16 + at_column);
+    }
+    // (row tile 0 or 1 of the read-outs, which waves 0 and 1 finish)
+    const float* within = p.made.within + of * CHUNK * CHUNK + 16 * (wave & 1) * CHUNK;
+    o.within[0] = load4(within + at_column);
+    o.within[1] = load4(within + 16 + at_column);
+    if constexpr (MODE == PER_CHANNEL) {
+      const float* fade = p.made.fade + of * PAD + row0;
+#pragma unroll
+      for (int d = 0; d < DT; ++d) o.fade[d] = load4(fade + 16 * d + 4 * quad);
+    } else {
+      const float* factor = p.made.factor + of * 2 * CHUNK;
+      if constexpr (MODE == DELTA) {
+        o.g[0] = load4(factor + 4 * quad);
+        o.g[1] = load4(factor + 16 + 4 * quad);
+      } else {
+        o.g[0] = load4(factor + 16 * (wave & 1) + 4 * quad);
+      }
+      o.tail[0] = load4(factor + CHUNK + 4 * quad);
+      o.tail[1] = load4(factor + CHUNK + 16 + 4 * quad);
+      o.g_last = factor[CHUNK - 1];
+    }
+    // (of tokens past the last one the last one's)
+    const int t0 = first + n * CHUNK;
+    const bf16_t* v = p.v + (int64_t)t0 * p.v_stride + p.v_col + (int64_t)head * p.vdim;
+    const uint32_t most = (uint32_t)(last - 1 - t0) * (uint32_t)p.v_stride;
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o.v[t][e] = *reinterpret_cast<const uint16_t*>(v + (min(v_at[t][e], most) + v_lane));
+  };
+  auto step = [&](int n, const Operands<DT, MODE>& o) {
+    // values; of tokens past the last one zeros (by their bits: a choice would be compiled into a branch around the load,
+    // and every load waited for by itself)
+    const int nt = last - first - n * CHUNK;
+    f32x4_t v[2];
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const uint32_t keep = (int)(16 * t + 4 * quad + e) < nt ? 0xFFFF0000u : 0u;
+        v[t][e] = __uint_as_float((o.v[t][e] << 16) & keep);
+      }
+    const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
+    f32x4_t sum[SUMS];
+#pragma unroll
+    for (int t = 0; t < SUMS; ++t) sum[t] = zero;
+#pragma unroll
+    for (int d = 0; d < DT; ++d)
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        sum[t] = mma4(o.q[t][d], S[d], sum[t]);
+        if constexpr (MODE == DELTA) sum[2 + t] = mma4(o.k[t][d], S[d], sum[2 + t]);
+      }
+    // (two buffers: a wave that runs ahead writes the other one, and cannot pass the next barrier)
+#pragma unroll
+    for (int t = 0; t < SUMS; ++t) parts[n & 1][wave][t][lane] = sum[t];
+    lds_barrier();
+    auto whole = [&](int t) {
+      return (parts[n & 1][0][t][lane] + parts[n & 1][1][t][lane]) + (parts[n & 1][2][t][lane] + parts[n & 1][3][t][lane]);
+    };
+    f32x4_t u[2] = {v[0], v[1]};
+    if constexpr (MODE == DELTA) {
+#pragma unroll
+      for (int t = 0; t < 2; ++t) u[t] -= scaled(o.g[t], whole(2 + t));
+      const f32x4_t upper = mma4(o.solve[0], u[0], zero), lower = mma4(o.solve[1], u[0], zero);
+      u[1] = lower + mma4(o.solve[2], u[1], zero);
+      u[0] = upper;
+    }
+    f32x4_t tail[2];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) {
+      if constexpr (MODE == PER_CHANNEL) tail[t] = u[t];
+      else tail[t] = scaled(o.tail[t], u[t]);
+    }
+#pragma unroll
+    for (int d = 0; d < DT; ++d) {
+      if constexpr (MODE == PER_CHANNEL) S[d] = scaled(o.fade[d], S[d]);
+      else S[d] *= o.g_last;
+    }
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int d = 0; d < DT; ++d) S[d] = mma4(o.kt[t][d], tail[t], S[d]);
+    if (wave < 2) {
+      f32x4_t read = whole(wave);
+      if constexpr (MODE != PER_CHANNEL) read = scaled(MODE == DELTA && wave == 1 ? o.g[1] : o.g[0], read);
+      read += mma4(o.within[0], u[0], zero);
+      if (wave == 1) read += mma4(o.within[1], u[1], zero);
+      if constexpr (MODE == PER_HEAD) read += skip * (wave == 0 ? v[0] : v[1]);
+      float* out = p.out + (int64_t)(first + n * CHUNK) * out_stride + (int64_t)head * p.vdim;
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+        if ((int)(16 * wave + 4 * quad + e) < nt && live) out[out_at[e]] = read[e];
+    }
+  };
+  // (two sets of operands: a third, two chunks ahead, measured 188 -> 185 us and cost the second block of a CU)
+  Operands<DT, MODE> even, odd;
+  fetch(0, even);
+  for (int n = 0; n + 1 < chunks; n += 2) {
+    fetch(n + 1, odd);
+    step(n, even);
+    fetch(min(n + 2, chunks - 1), even);
+    step(n + 1, odd);
+  }
+  if (chunks & 1) step(chunks - 1, even);
+  if (live) {
+#pragma unroll
+    for (int d = 0; d < DT; ++d) *reinterpret_cast<f32x4_t*>(mine + 16 * d) = S[d];
+  }
+}
+
+template <int MODE>
+static int launch_walk(const WalkArgs& p, int pad, int requests, hipStream_t stream) {
+  dim3 grid(p.heads * ceil_div(p.vdim, 16), requests);
+  if (pad == 64) walk_kernel<1, MODE><<<grid, 256, 0, stream>>>(p);
+  else if (pad == 128) walk_kernel<2, MODE><<<grid, 256, 0, stream>>>(p);
+  else walk_kernel<4, MODE><<<grid, 256, 0, stream>>>(p);
+  MI_CHECK_LAUNCH("chunk_walk");
+  return MI_OK;
+}
+
+}  // namespace chunk_scan

@@ -23,6 +23,7 @@
 // outputs are read in the element type); in the 32-bit engine the scalar gates, the unit norms
 // and the read-out's norm are evaluated in 64-bit and rounded once.
 #include "common.h"
+#include "delta_rule.h"
 
 #include <math.h>
 
@@ -258,7 +259,8 @@ __device__ __forceinline__ float lanes_sum(float v) {
 // sums over R lanes by register moves.  Counters at heads of 128 x 128, 16 lanes a column: 100
 // vector instructions and 6 LDS reads a token and wave, one wave a SIMD, a token every 250 issue
 // turns.  32 lanes a column (half the work a wave, two waves a SIMD, twice the LDS reads a CU)
-// measured no faster, 961 against 912 us for 2,048 tokens, so 16 it is.
+// measured no faster, 961 against 912 us for 2,048 tokens, so 16 it is.  Long portions of bfloat16 steps go in chunks
+// (delta_chunks.hip); this kernel has decoded tokens, short portions and the 32-bit engine.
 template <typename T, int R, int ROWS>
 __global__ __launch_bounds__(256) void gated_delta_kernel(
     const T* __restrict__ qkv, int64_t qkv_stride, const T* __restrict__ proj, int64_t proj_stride, int col_b,
@@ -578,18 +580,14 @@ extern "C" int mi_gated_delta_rows(int dim, int vdim) {
   return lanes * rows;
 }
 
-extern "C" int mi_gated_delta(int dtype, const void* qkv, int64_t qkv_stride, const void* proj, int64_t proj_stride,
-                              int col_b, int col_a, int col_g, const float* a_log, const float* dt_bias,
-                              const float* norm_weight, float* state, int64_t state_stride, const int* cu,
-                              const int* slots, float* readout, void* out, int64_t out_stride, int num_tokens, int num_requests, int heads,
-                              int kv_heads, int dim, int vdim, int dim_pad, float eps, int num_slots, hipStream_t stream) {
+int mi_gated_delta_check(int64_t qkv_stride, int64_t proj_stride, int col_b, int col_a, int col_g, const float* state,
+                         int64_t state_stride, int64_t out_stride, int num_requests, int heads, int kv_heads, int dim, int vdim,
+                         int dim_pad, float eps, int num_slots) {
   MI_REQUIRE(num_requests >= 0 && heads > 0 && kv_heads > 0 && heads % kv_heads == 0,
              "gated_delta: bad sizes requests=%d heads=%d kv_heads=%d", num_requests, heads, kv_heads);
   MI_REQUIRE(dim > 0 && dim <= 256, "gated_delta: dim=%d must be 1..256", dim);
   MI_REQUIRE(vdim > 0 && vdim <= 256, "gated_delta: vdim=%d must be 1..256", vdim);
-  int lanes = 0, rows = 0;
-  delta_layout(dim, vdim, &lanes, &rows);
-  const int pad = lanes * rows;
+  const int pad = mi_gated_delta_rows(dim, vdim);
   MI_REQUIRE(qkv_stride >= 2 * (int64_t)kv_heads * dim + (int64_t)heads * vdim && out_stride >= (int64_t)heads * vdim,
              "gated_delta: row strides shorter than a row");
   MI_REQUIRE(dim_pad == pad && state_stride >= (int64_t)heads * vdim * pad && state_stride % 4 == 0 &&
@@ -601,7 +599,35 @@ extern "C" int mi_gated_delta(int dtype, const void* qkv, int64_t qkv_stride, co
              "gated_delta: the gates' columns lie outside a row of the projections");
   MI_REQUIRE(eps > 0.f, "gated_delta: eps must be positive, got %g", (double)eps);
   MI_REQUIRE(num_slots >= 1 && num_requests <= 65535, "gated_delta: bad slot or request count");
+  return MI_OK;
+}
+
+int mi_delta_readout_norm(int dtype, const float* readout, const void* proj, int64_t proj_stride, int col_g, const float* norm_weight,
+                          void* out, int64_t out_stride, int num_tokens, int heads, int vdim, float eps, hipStream_t stream) {
+  if (num_tokens > 0) {
+    dim3 ngrid(num_tokens, min(ceil_div(heads, 4), 64));
+    if (dtype == MI_F32)
+      delta_readout_norm_kernel<float><<<ngrid, 256, 0, stream>>>(readout, (const float*)proj, proj_stride, col_g, norm_weight,
+                                                                  (float*)out, out_stride, heads, vdim, eps);
+    else
+      delta_readout_norm_kernel<bf16_t><<<ngrid, 256, 0, stream>>>(readout, (const bf16_t*)proj, proj_stride, col_g, norm_weight,
+                                                                   (bf16_t*)out, out_stride, heads, vdim, eps);
+    MI_CHECK_LAUNCH("delta_readout_norm");
+  }
+  return MI_OK;
+}
+
+extern "C" int mi_gated_delta(int dtype, const void* qkv, int64_t qkv_stride, const void* proj, int64_t proj_stride,
+                              int col_b, int col_a, int col_g, const float* a_log, const float* dt_bias,
+                              const float* norm_weight, float* state, int64_t state_stride, const int* cu,
+                              const int* slots, float* readout, void* out, int64_t out_stride, int num_tokens, int num_requests, int heads,
+                              int kv_heads, int dim, int vdim, int dim_pad, float eps, int num_slots, hipStream_t stream) {
+  const int bad = mi_gated_delta_check(qkv_stride, proj_stride, col_b, col_a, col_g, state, state_stride, out_stride, num_requests, heads,
+                                       kv_heads, dim, vdim, dim_pad, eps, num_slots);
+  if (bad != MI_OK) return bad;
   MI_REQUIRE(dtype == MI_F32 || dtype == MI_BF16, "gated_delta: unknown dtype %d", dtype);
+  int lanes = 0, rows = 0;
+  delta_layout(dim, vdim, &lanes, &rows);
   if (num_requests == 0) return MI_OK;
   MI_REQUIRE(readout != nullptr, "gated_delta: no buffer for the read-outs");
   const int cols = 256 / lanes, chunks = ceil_div(vdim, cols);
@@ -620,15 +646,5 @@ extern "C" int mi_gated_delta(int dtype, const void* qkv, int64_t qkv_stride, co
 #undef MI_DELTA_LANES
 #undef MI_DELTA_LAUNCH
   MI_CHECK_LAUNCH("gated_delta");
-  if (num_tokens > 0) {
-    dim3 ngrid(num_tokens, min(ceil_div(heads, 4), 64));
-    if (dtype == MI_F32)
-      delta_readout_norm_kernel<float><<<ngrid, 256, 0, stream>>>(readout, (const float*)proj, proj_stride, col_g, norm_weight,
-                                                                  (float*)out, out_stride, heads, vdim, eps);
-    else
-      delta_readout_norm_kernel<bf16_t><<<ngrid, 256, 0, stream>>>(readout, (const bf16_t*)proj, proj_stride, col_g, norm_weight,
-                                                                   (bf16_t*)out, out_stride, heads, vdim, eps);
-    MI_CHECK_LAUNCH("delta_readout_norm");
-  }
-  return MI_OK;
+  return mi_delta_readout_norm(dtype, readout, proj, proj_stride, col_g, norm_weight, out, out_stride, num_tokens, heads, vdim, eps, stream);
 }

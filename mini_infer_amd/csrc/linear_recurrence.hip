@@ -26,6 +26,7 @@
 // in the element type); in the 32-bit engine decays, step sizes, the read-out's sums and the
 // norm's statistics are evaluated in 64-bit and rounded once.
 #include "common.h"
+#include "linear_recurrence.h"
 
 #include <math.h>
 
@@ -95,16 +96,7 @@ __device__ __forceinline__ double lanes_sum(double v) {
   return v;
 }
 
-// log(1 + e) for 0 <= e <= 1 on the hardware's logarithm (one ulp), with the series where 1 + e
-// would round e away
-__device__ __forceinline__ float log1p_small(float e) {
-  return e < 1e-3f ? e * (1.f - e * (0.5f - e * 0.33333334f)) : 0.6931471805599453f * __builtin_amdgcn_logf(1.f + e);
-}
-// log(logistic(z)) = -softplus(-z), and softplus, float32 on the hardware's exponential and logarithm
-__device__ __forceinline__ float soft_plus_fast(float z) {
-  return fmaxf(z, 0.f) + log1p_small(__builtin_amdgcn_exp2f(-fabsf(z) * 1.4426950408889634f));
-}
-
+// Decoded tokens, short portions and the 32-bit engine; long portions of bfloat16 steps go in chunks (decay_chunks.hip).
 // 256 threads keep 256 / L columns of a head's S, L lanes a column, R rows a lane.  Tokens are
 // taken SCAN_TILE at a time: a tile's rows are asked of memory while the tile before it is
 // walked (they wait in registers), then all threads turn them into float32 q, k, decays and
@@ -194,7 +186,7 @@ __global__ __launch_bounds__(256) void decay_scan_kernel(ScanArgs p) {
         float av = 0.f;
         if (d < p.dim) {
           if constexpr (WIDE) av = (float)exp(log_logistic<double>((double)g_raw[i] + (double)ch_bias[i]) * (double)p.inv_tau);
-          else av = __builtin_amdgcn_exp2f(-soft_plus_fast(-(g_raw[i] + ch_bias[i])) * (p.inv_tau * 1.4426950408889634f));
+          else av = mi_channel_decay(g_raw[i] + ch_bias[i], p.inv_tau);
         }
         a_lds[at] = av;
       }
@@ -205,7 +197,7 @@ __global__ __launch_bounds__(256) void decay_scan_kernel(ScanArgs p) {
         a_lds[tid] = (float)exp(-rate_wide * step);
         dt_lds[tid] = (float)step;
       } else {
-        const float step = soft_plus_fast(g_raw[0] + head_bias);
+        const float step = mi_soft_plus_fast(g_raw[0] + head_bias);
         a_lds[tid] = __builtin_amdgcn_exp2f(-rate * step);
         dt_lds[tid] = step;
       }
@@ -375,17 +367,9 @@ extern "C" int mi_decay_scan_dim_pad(int dim) {
   return rows * lanes;
 }
 
-// mode 0: decay per key channel (gate: [tokens, heads * dim] logits, gate_bias [heads * dim], inv_tau);
-// mode 1: decay per head (gate: [tokens, heads] raw step sizes, gate_bias [heads], rate [heads], skip [heads] or null).
-// q, k: rows holding `groups` heads of `dim` from q_col / k_col on (head h reads group h / (heads / groups));
-// v: rows holding `heads` heads of `vdim` from v_col on.  state float32 [slots + 1][heads][vdim][dim_pad].
-// out float32 [tokens, heads * vdim].
-extern "C" int mi_decay_scan(int dtype, int mode, const void* q, int64_t q_stride, int q_col, const void* k, int64_t k_stride,
-                             int k_col, const void* v, int64_t v_stride, int v_col, const void* gate, int64_t gate_stride,
-                             int gate_col, const float* gate_bias, const float* rate, const float* skip, float inv_tau,
-                             float q_scale, float* state, int64_t state_stride, const int* cu, const int* slots, int num_slots,
-                             float* out, int num_tokens, int num_requests, int heads, int groups, int dim, int vdim,
-                             hipStream_t stream) {
+int mi_decay_scan_check(int dtype, int mode, int64_t q_stride, int q_col, int64_t k_stride, int k_col, int64_t v_stride, int v_col,
+                        int64_t gate_stride, int gate_col, const float* gate_bias, const float* rate, const float* state,
+                        int64_t state_stride, int num_slots, int num_tokens, int num_requests, int heads, int groups, int dim, int vdim) {
   MI_REQUIRE(num_tokens >= 0 && num_requests >= 0 && heads > 0 && groups > 0 && dim > 0 && vdim > 0,
              "decay_scan: bad sizes tokens=%d requests=%d heads=%d groups=%d dim=%d vdim=%d", num_tokens, num_requests, heads,
              groups, dim, vdim);
@@ -402,6 +386,23 @@ extern "C" int mi_decay_scan(int dtype, int mode, const void* q, int64_t q_strid
   MI_REQUIRE(state_stride >= (int64_t)heads * vdim * mi_decay_scan_dim_pad(dim) && ((uintptr_t)state % 16 == 0) &&
                  state_stride % 4 == 0,
              "decay_scan: the state rows are too short or not 16-byte aligned");
+  return MI_OK;
+}
+
+// mode 0: decay per key channel (gate: [tokens, heads * dim] logits, gate_bias [heads * dim], inv_tau);
+// mode 1: decay per head (gate: [tokens, heads] raw step sizes, gate_bias [heads], rate [heads], skip [heads] or null).
+// q, k: rows holding `groups` heads of `dim` from q_col / k_col on (head h reads group h / (heads / groups));
+// v: rows holding `heads` heads of `vdim` from v_col on.  state float32 [slots + 1][heads][vdim][dim_pad].
+// out float32 [tokens, heads * vdim].
+extern "C" int mi_decay_scan(int dtype, int mode, const void* q, int64_t q_stride, int q_col, const void* k, int64_t k_stride,
+                             int k_col, const void* v, int64_t v_stride, int v_col, const void* gate, int64_t gate_stride,
+                             int gate_col, const float* gate_bias, const float* rate, const float* skip, float inv_tau,
+                             float q_scale, float* state, int64_t state_stride, const int* cu, const int* slots, int num_slots,
+                             float* out, int num_tokens, int num_requests, int heads, int groups, int dim, int vdim,
+                             hipStream_t stream) {
+  const int bad = mi_decay_scan_check(dtype, mode, q_stride, q_col, k_stride, k_col, v_stride, v_col, gate_stride, gate_col, gate_bias,
+                                      rate, state, state_stride, num_slots, num_tokens, num_requests, heads, groups, dim, vdim);
+  if (bad != MI_OK) return bad;
   if (num_tokens == 0 || num_requests == 0) return MI_OK;
   ScanArgs p;
   p.q = q, p.k = k, p.v = v, p.gate = gate;

@@ -98,6 +98,11 @@ _SIGNATURES: dict[str, list] = {
         c_int, _P, c_int64, _P, c_int64, c_int, c_int, c_int, _P, _P, _P, _P, c_int64, _P, _P, _P, _P, c_int64,
         c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_int, _P,
     ],
+    "mi_gated_delta_chunks": [
+        _P, c_int64, _P, c_int64, c_int, c_int, c_int, _P, _P, _P, _P, c_int64, _P, _P, _P, _P, _P, c_int64, c_int, c_int, c_int, c_int,
+        c_int, c_int, c_int, c_float, c_int, _P,
+    ],
+    "mi_gated_delta_chunks_scratch": [c_int, c_int, c_int, c_int, c_int, c_int],
     "mi_gated_delta_rows": [c_int, c_int],
     "mi_latent_prepare": [
         c_int, _P, c_int64, c_int, c_int, c_int, c_int, _P, _P, _P, _P, _P, _P, c_int64, _P, c_int, c_int, c_int, c_int,
@@ -111,6 +116,11 @@ _SIGNATURES: dict[str, list] = {
     "mi_streams_update_norm": [
         c_int, _P, c_int64, _P, c_int64, c_float, c_float, _P, _P, _P, _P, _P, _P, _P, c_int, c_int, c_int, c_float, _P,
     ],
+    "mi_decay_scan_chunks": [
+        c_int, _P, c_int64, c_int, _P, c_int64, c_int, _P, c_int64, c_int, _P, c_int64, c_int, _P, _P, _P, c_float,
+        c_float, _P, c_int64, _P, _P, c_int, _P, _P, c_int, c_int, c_int, c_int, c_int, c_int, _P,
+    ],
+    "mi_decay_scan_chunks_scratch": [c_int, c_int, c_int, c_int, c_int, c_int],
     "mi_decay_scan_dim_pad": [c_int],
     "mi_decay_scan": [
         c_int, c_int, _P, c_int64, c_int, _P, c_int64, c_int, _P, c_int64, c_int, _P, c_int64, c_int, _P, _P, _P, c_float,
@@ -160,6 +170,9 @@ _SIGNATURES: dict[str, list] = {
 }
 
 
+_INT64_RESULTS = {"mi_gated_delta_chunks_scratch", "mi_decay_scan_chunks_scratch"}  # (sizes; every other entry point returns an int status)
+
+
 def _declare(lib: ctypes.CDLL) -> None:
     lib.mi_last_error.restype = ctypes.c_char_p
     lib.mi_last_error.argtypes = []
@@ -167,7 +180,7 @@ def _declare(lib: ctypes.CDLL) -> None:
     lib.mi_abi_version.argtypes = []
     for name, argtypes in _SIGNATURES.items():
         fn = getattr(lib, name)
-        fn.restype = c_int
+        fn.restype = c_int64 if name in _INT64_RESULTS else c_int
         fn.argtypes = argtypes
 
 

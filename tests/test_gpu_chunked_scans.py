@@ -1,0 +1,129 @@
+"""The recurrences with a matrix state taken 32 tokens at a time, against the recurrence itself in 64 bits and
+against the kernels that walk token by token."""
+
+from __future__ import annotations
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+SIZES = [([32, 31, 33, 1], 4, 2, 64, 64), ([200], 2, 2, 128, 128), ([97, 64, 5], 6, 3, 96, 80), ([129], 2, 1, 256, 250), ([65, 100], 3, 3, 20, 30)]
+
+
+def _rel(got, exact):
+    return float((got.double() - exact).norm() / exact.norm())
+
+
+def _state(generator, requests, shape, dim):
+    state = torch.zeros(requests + 2, *shape, device=DEV)
+    state[..., :dim] = torch.randn(requests + 2, *shape[:-1], dim, generator=generator, device=DEV) * 0.3
+    return state
+
+
+def _boundaries(lengths):
+    return torch.tensor([0, *torch.tensor(lengths).cumsum(0).tolist()], dtype=torch.int32, device=DEV)
+
+
+def _rows(generator, tokens, width, odd):
+    """bfloat16 rows; `odd`: of a buffer whose rows do not lie on 16 bytes."""
+    wide = torch.randn(tokens, width + (3 if odd else 0), generator=generator, device=DEV).bfloat16()
+    return wide[:, 3:] if odd else wide
+
+
+def _both(monkeypatch, call, state):
+    """What `call(state)` gives in chunks and token by token, with the state each leaves."""
+    from mini_infer_amd.ops import kernels
+
+    made = []
+    for chunks in (True, False):
+        monkeypatch.setattr(kernels, "chunked_scan_pays", lambda tokens, requests, chunks=chunks: chunks)
+        left = state.clone()
+        made.append((call(left), left))
+    return made
+
+
+def _check(chunked, walked, state, exact_out, exact_state, requests, dim, out_floor):
+    (out, left), (out_walked, left_walked) = chunked, walked
+    # float32 sums of up to 256 products and 32 tokens between two roundings of the state: a few 1e-7; never twice as far as
+    # the kernel that rounds the state at every token
+    assert _rel(left[:requests], exact_state) < max(4e-7, 2 * _rel(left_walked[:requests], exact_state))
+    assert torch.equal(left[requests:], state[requests:])  # rows of other slots are not touched
+    assert (left[..., dim:] == 0).all()
+    assert _rel(out, exact_out) < max(out_floor, 2 * _rel(out_walked, exact_out))
+
+
+@pytest.mark.parametrize("lengths,heads,kv_heads,dim,vdim", SIZES)
+@pytest.mark.parametrize("odd", [False, True])
+@pytest.mark.parametrize("fast", [False, True])
+def test_gated_delta_in_chunks(monkeypatch, lengths, heads, kv_heads, dim, vdim, odd, fast):
+    from mini_infer_amd import ops
+
+    g = torch.Generator(device=DEV).manual_seed(7)
+    tokens, requests = sum(lengths), len(lengths)
+    qkv, proj = _rows(g, tokens, 2 * kv_heads * dim + heads * vdim, odd), _rows(g, tokens, 2 * heads + heads * vdim, odd)
+    a_log = torch.log(1 + 15 * torch.rand(heads, generator=g, device=DEV))
+    dt_bias = torch.full((heads,), 1.0 if fast else -4.0, device=DEV)  # fast: a state is forgotten within a few tokens
+    weight = torch.ones(vdim, device=DEV)
+    state = _state(g, requests, ops.delta_state_shape(heads, dim, vdim), dim)
+    cu, slots = _boundaries(lengths), torch.arange(requests, dtype=torch.int32, device=DEV)
+    chunked, walked = _both(monkeypatch, lambda s: ops.gated_delta(
+        qkv, proj, 0, heads, 2 * heads, a_log, dt_bias, weight, s, cu, slots, heads=heads, kv_heads=kv_heads, dim=dim, vdim=vdim, eps=1e-6), state)
+
+    q, k, v = qkv.double().split([kv_heads * dim, kv_heads * dim, heads * vdim], 1)
+    q, k = (x.view(tokens, kv_heads, dim) for x in (q, k))
+    q, k = ((x / torch.sqrt((x * x).sum(-1, keepdim=True) + 1e-6)).repeat_interleave(heads // kv_heads, 1) for x in (q, k))
+    v, p = v.view(tokens, heads, vdim), proj.double()
+    write = torch.sigmoid(p[:, :heads])
+    decay = torch.exp(-torch.exp(a_log.double()) * torch.nn.functional.softplus(p[:, heads : 2 * heads] + dt_bias.double()))
+    out, left = torch.empty(tokens, heads, vdim, dtype=torch.float64, device=DEV), []
+    for b in range(requests):
+        S = state[b].double()[..., :dim].transpose(1, 2)
+        for t in range(int(cu[b]), int(cu[b + 1])):
+            S = S * decay[t, :, None, None]
+            S = S + k[t, :, :, None] * (write[t, :, None] * (v[t] - (k[t, :, None] @ S).squeeze(1)))[:, None]
+            out[t] = (q[t, :, None] @ S).squeeze(1) * dim ** -0.5
+        left.append(torch.nn.functional.pad(S.transpose(1, 2), (0, state.shape[-1] - dim)))
+    out = out / torch.sqrt((out * out).mean(-1, keepdim=True) + 1e-6) * torch.nn.functional.silu(p[:, 2 * heads :].view(tokens, heads, vdim))
+    _check(chunked, walked, state, out.flatten(1), torch.stack(left), requests, dim, 2.0 ** -8)
+
+
+@pytest.mark.parametrize("lengths,heads,groups,dim,vdim", SIZES)
+@pytest.mark.parametrize("odd", [False, True])
+@pytest.mark.parametrize("per_head", [False, True])
+@pytest.mark.parametrize("fast", [False, True])
+def test_decaying_state_in_chunks(monkeypatch, lengths, heads, groups, dim, vdim, odd, per_head, fast):
+    from mini_infer_amd import ops
+
+    if dim <= 32:
+        dim = 40  # (narrower keys stay with the token-by-token kernel)
+    g = torch.Generator(device=DEV).manual_seed(9)
+    tokens, requests = sum(lengths), len(lengths)
+    q, k, v = (_rows(g, tokens, n, odd) for n in (groups * dim, groups * dim, heads * vdim))
+    gate = _rows(g, tokens, heads if per_head else heads * dim, odd) * (20.0 if fast else 1.0)
+    bias = torch.full((heads if per_head else heads * dim,), -3.0 if per_head else 0.1, device=DEV)
+    rate = torch.log(1 + 15 * torch.rand(heads, generator=g, device=DEV)) if per_head else None
+    skip = torch.randn(heads, generator=g, device=DEV) if per_head else None
+    state = _state(g, requests, ops.decay_state_shape(heads, dim, vdim), dim)
+    cu, slots = _boundaries(lengths), torch.arange(requests, dtype=torch.int32, device=DEV)
+    chunked, walked = _both(monkeypatch, lambda s: ops.decay_scan(
+        q, 0, k, 0, v, 0, gate, 0, bias, s, cu, slots, heads=heads, groups=groups, dim=dim, vdim=vdim, per_head=per_head, rate=rate, skip=skip,
+        inv_tau=0.0625, q_scale=0.125), state)
+
+    qd, kd = (x.double().view(tokens, groups, dim).repeat_interleave(heads // groups, 1) for x in (q, k))
+    x, z = v.double().view(tokens, heads, vdim), gate.double() + bias.double()
+    if per_head:
+        step = torch.nn.functional.softplus(z)
+        decay, u = torch.exp(-torch.exp(rate.double()) * step)[..., None], x * step[..., None]
+    else:
+        decay, u = torch.sigmoid(z).pow(0.0625).view(tokens, heads, dim), x
+    out, left = torch.empty(tokens, heads, vdim, dtype=torch.float64, device=DEV), []
+    for b in range(requests):
+        S = state[b].double()[..., :dim].transpose(1, 2)
+        for t in range(int(cu[b]), int(cu[b + 1])):
+            S = decay[t, :, :, None] * S + kd[t, :, :, None] * u[t, :, None]
+            out[t] = (qd[t, :, None] @ S).squeeze(1) * 0.125
+        left.append(torch.nn.functional.pad(S.transpose(1, 2), (0, state.shape[-1] - dim)))
+    if per_head:
+        out = out + skip.double()[:, None] * x
+    _check(chunked, walked, state, out.flatten(1), torch.stack(left), requests, dim, 4e-7)
