@@ -53,6 +53,27 @@ def _check(chunked, walked, state, exact_out, exact_state, requests, dim, out_fl
     assert _rel(out, exact_out) < max(out_floor, 2 * _rel(out_walked, exact_out))
 
 
+def _exact_delta(qkv, proj, a_log, dt_bias, state, cu, heads, kv_heads, dim, vdim):
+    """Normed and gated read-outs (norm weight 1) and the states left, in 64 bits."""
+    tokens = qkv.shape[0]
+    q, k, v = qkv.double().split([kv_heads * dim, kv_heads * dim, heads * vdim], 1)
+    q, k = (x.view(tokens, kv_heads, dim) for x in (q, k))
+    q, k = ((x / torch.sqrt((x * x).sum(-1, keepdim=True) + 1e-6)).repeat_interleave(heads // kv_heads, 1) for x in (q, k))
+    v, p = v.view(tokens, heads, vdim), proj.double()
+    write = torch.sigmoid(p[:, :heads])
+    decay = torch.exp(-torch.exp(a_log.double()) * torch.nn.functional.softplus(p[:, heads : 2 * heads] + dt_bias.double()))
+    out, left = torch.empty(tokens, heads, vdim, dtype=torch.float64, device=DEV), []
+    for b in range(cu.numel() - 1):
+        S = state[b].double()[..., :dim].transpose(1, 2)
+        for t in range(int(cu[b]), int(cu[b + 1])):
+            S = S * decay[t, :, None, None]
+            S = S + k[t, :, :, None] * (write[t, :, None] * (v[t] - (k[t, :, None] @ S).squeeze(1)))[:, None]
+            out[t] = (q[t, :, None] @ S).squeeze(1) * dim ** -0.5
+        left.append(torch.nn.functional.pad(S.transpose(1, 2), (0, state.shape[-1] - dim)))
+    out = out / torch.sqrt((out * out).mean(-1, keepdim=True) + 1e-6) * torch.nn.functional.silu(p[:, 2 * heads :].view(tokens, heads, vdim))
+    return out.flatten(1), torch.stack(left)
+
+
 @pytest.mark.parametrize("lengths,heads,kv_heads,dim,vdim", SIZES)
 @pytest.mark.parametrize("odd", [False, True])
 @pytest.mark.parametrize("fast", [False, True])
@@ -70,22 +91,31 @@ def test_gated_delta_in_chunks(monkeypatch, lengths, heads, kv_heads, dim, vdim,
     chunked, walked = _both(monkeypatch, lambda s: ops.gated_delta(
         qkv, proj, 0, heads, 2 * heads, a_log, dt_bias, weight, s, cu, slots, heads=heads, kv_heads=kv_heads, dim=dim, vdim=vdim, eps=1e-6), state)
 
-    q, k, v = qkv.double().split([kv_heads * dim, kv_heads * dim, heads * vdim], 1)
-    q, k = (x.view(tokens, kv_heads, dim) for x in (q, k))
-    q, k = ((x / torch.sqrt((x * x).sum(-1, keepdim=True) + 1e-6)).repeat_interleave(heads // kv_heads, 1) for x in (q, k))
-    v, p = v.view(tokens, heads, vdim), proj.double()
-    write = torch.sigmoid(p[:, :heads])
-    decay = torch.exp(-torch.exp(a_log.double()) * torch.nn.functional.softplus(p[:, heads : 2 * heads] + dt_bias.double()))
-    out, left = torch.empty(tokens, heads, vdim, dtype=torch.float64, device=DEV), []
-    for b in range(requests):
-        S = state[b].double()[..., :dim].transpose(1, 2)
-        for t in range(int(cu[b]), int(cu[b + 1])):
-            S = S * decay[t, :, None, None]
-            S = S + k[t, :, :, None] * (write[t, :, None] * (v[t] - (k[t, :, None] @ S).squeeze(1)))[:, None]
-            out[t] = (q[t, :, None] @ S).squeeze(1) * dim ** -0.5
-        left.append(torch.nn.functional.pad(S.transpose(1, 2), (0, state.shape[-1] - dim)))
-    out = out / torch.sqrt((out * out).mean(-1, keepdim=True) + 1e-6) * torch.nn.functional.silu(p[:, 2 * heads :].view(tokens, heads, vdim))
-    _check(chunked, walked, state, out.flatten(1), torch.stack(left), requests, dim, 2.0 ** -8)
+    out, left = _exact_delta(qkv, proj, a_log, dt_bias, state, cu, heads, kv_heads, dim, vdim)
+    _check(chunked, walked, state, out, left, requests, dim, 2.0 ** -8)
+
+
+@pytest.mark.parametrize("lengths", [[1], [1, 1, 1], [1, 0, 3, 0, 0], [0, 2]])
+@pytest.mark.parametrize("heads,kv_heads,dim,vdim", [(4, 2, 64, 64), (6, 3, 96, 80), (2, 1, 256, 250), (3, 3, 20, 30), (2, 2, 128, 128)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_gated_delta_of_decoded_tokens(lengths, heads, kv_heads, dim, vdim, dtype):
+    """No more tokens than requests: one launch, whichever request the tokens belong to."""
+    from mini_infer_amd import ops
+
+    g = torch.Generator(device=DEV).manual_seed(11)
+    tokens, requests = sum(lengths), len(lengths)
+    qkv, proj = (_rows(g, tokens, n, True).to(dtype) for n in (2 * kv_heads * dim + heads * vdim, 2 * heads + heads * vdim))
+    a_log, dt_bias = torch.rand(heads, generator=g, device=DEV), torch.full((heads,), -2.0, device=DEV)
+    weight = 1 + 0.1 * torch.randn(vdim, generator=g, device=DEV)
+    before = _state(g, requests, ops.delta_state_shape(heads, dim, vdim), dim)
+    state = before.clone()
+    cu, slots = _boundaries(lengths), torch.arange(requests, dtype=torch.int32, device=DEV)
+    got = ops.gated_delta(qkv, proj, 0, heads, 2 * heads, a_log, dt_bias, weight, state, cu, slots, heads=heads, kv_heads=kv_heads, dim=dim,
+                          vdim=vdim, eps=1e-6)
+    out, left = _exact_delta(qkv, proj, a_log, dt_bias, before, cu, heads, kv_heads, dim, vdim)
+    # float32 state: a few roundings a token; what is written is rounded to the element type once
+    assert _rel(state[:requests], left) < 2e-7 and torch.equal(state[requests:], before[requests:])
+    assert _rel(got, out * weight.double().repeat(heads)) < (2.0 ** -8 if dtype == torch.bfloat16 else 3e-7)
 
 
 @pytest.mark.parametrize("lengths,heads,groups,dim,vdim", SIZES)
