@@ -42,7 +42,7 @@ __device__ __forceinline__ float4 four_of_row(const float* row, int at, int k) {
 // Many rows: a block of 4 waves owns BM x 64 outputs, STAGE slices of both operands in LDS, the next ones in
 // flight in registers.  With 64 cycles an instruction the LDS is idle most of the time, so small tiles cost
 // nothing.  BM = 64 (a wave 32 x 32), one slice a stage, where there are at least four blocks a CU to cover one
-// another's barriers and loads; else BM = 32 (a wave 32 x 16): twice the blocks, four slices a stage.
+// another's barriers and loads; else BM = 32 (a wave 32 x 16): twice the blocks, four slices a stage where a run is whole stages, else one.
 // ALIGNED: 16-byte loads (K, both row strides multiples of 4 values, both matrices on 16 bytes).
 template <int BM, int STAGE, bool ALIGNED>
 __global__ __launch_bounds__(256) void gemm_f32_kernel(const float* __restrict__ a, int64_t lda,
@@ -60,17 +60,25 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const float* __restrict__
   constexpr int LANES = STAGE * SLICE / 4, ROWS = 256 / LANES;  // threads a row, rows a pass of the block's loads
   const int l_row = tid / LANES, l_k = tid % LANES * 4;
 
+  // (rows past the last one repeat it and are not written: no branch around a load but one for the whole block, where K
+  // ends inside a stage; with a branch around each load 509 x 2048 x 2048 took 91 us instead of 87)
+  const float *a_row[AL], *w_row[WL];
+#pragma unroll
+  for (int i = 0; i < AL; ++i) a_row[i] = a + (int64_t)min(row0 + l_row + ROWS * i, m - 1) * lda + (ALIGNED ? l_k : 0);
+#pragma unroll
+  for (int i = 0; i < WL; ++i) w_row[i] = w + (int64_t)min(col0 + l_row + ROWS * i, n - 1) * ldw + (ALIGNED ? l_k : 0);
   float4 a_next[AL], w_next[WL];
   auto fetch = [&](int k0) {
+    if (ALIGNED && k0 + STAGE * SLICE <= k) {
 #pragma unroll
-    for (int i = 0; i < AL; ++i) {
-      const int row = row0 + l_row + ROWS * i;
-      a_next[i] = row < m ? four_of_row<ALIGNED>(a + (int64_t)row * lda, k0 + l_k, k) : make_float4(0.f, 0.f, 0.f, 0.f);
-    }
+      for (int i = 0; i < AL; ++i) a_next[i] = *reinterpret_cast<const float4*>(a_row[i] + k0);
 #pragma unroll
-    for (int i = 0; i < WL; ++i) {
-      const int row = col0 + l_row + ROWS * i;
-      w_next[i] = row < n ? four_of_row<ALIGNED>(w + (int64_t)row * ldw, k0 + l_k, k) : make_float4(0.f, 0.f, 0.f, 0.f);
+      for (int i = 0; i < WL; ++i) w_next[i] = *reinterpret_cast<const float4*>(w_row[i] + k0);
+    } else {
+#pragma unroll
+      for (int i = 0; i < AL; ++i) a_next[i] = four_of_row<ALIGNED>(a_row[i] - (ALIGNED ? l_k : 0), k0 + l_k, k);
+#pragma unroll
+      for (int i = 0; i < WL; ++i) w_next[i] = four_of_row<ALIGNED>(w_row[i] - (ALIGNED ? l_k : 0), k0 + l_k, k);
     }
   };
   f64x4_t total[2][CT], acc[2][CT];
@@ -109,16 +117,19 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const float* __restrict__
 #pragma unroll
             for (int j = 0; j < CT; ++j) acc[i][j] = mma(av[i][s], wv[j][s], acc[i][j]);
       }
-      if (--left == 0) {
-        left = run;
+    }
+    // (runs are whole stages: looked at after every slice, the sums went through other registers and back each time, with
+    // the matrix pipe drained: 87 us instead of 82 at 509 x 2048 x 2048)
+    left -= STAGE;
+    if (left == 0) {
+      left = run;
 #pragma unroll
-        for (int i = 0; i < 2; ++i)
+      for (int i = 0; i < 2; ++i)
 #pragma unroll
-          for (int j = 0; j < CT; ++j) {
-            total[i][j] += acc[i][j];
-            acc[i][j] = f64x4_t{0.0, 0.0, 0.0, 0.0};
-          }
-      }
+        for (int j = 0; j < CT; ++j) {
+          total[i][j] += acc[i][j];
+          acc[i][j] = f64x4_t{0.0, 0.0, 0.0, 0.0};
+        }
     }
   }
 #pragma unroll
@@ -264,10 +275,10 @@ static void launch_rows(const float* a, int64_t lda, const float* w, int64_t ldw
 
 // Which kernel, with microseconds at rows x N x K (weights from memory).  Before: 64-bit multiply-adds on the vector
 // pipe, 4 x 4 outputs a thread, and a kernel of its own for up to 16 rows only.
-//     3 x 2048 x 2048     75.6 ->   9.0     20 x  2048 x 2048   317 ->  15.0     509 x  2048 x 2048    327 ->  88
-//     3 x 16384 x 2048     107 ->  30.7     20 x 16384 x 2048   349 ->  46.0     509 x  3072 x 2048    378 -> 125
+//     3 x 2048 x 2048     75.6 ->   9.0     20 x  2048 x 2048   317 ->  15.0     509 x  2048 x 2048    327 ->  82
+//     3 x 16384 x 2048     107 ->  30.7     20 x 16384 x 2048   349 ->  46.0     509 x  3072 x 2048    378 -> 117
 //     3 x 128256 x 2048    419 ->   192     60 x  2048 x 2048   320 ->  26.3     509 x 16384 x 2048   1060 -> 580
-//     3 x 2048 x 8192      322 ->  28.1     60 x 16384 x 2048   355 -> 102       509 x  2048 x 8192   1340 -> 345
+//     3 x 2048 x 8192      322 ->  28.1     60 x 16384 x 2048   355 -> 102       509 x  2048 x 8192   1340 -> 316
 // 3 rows of 16,384 features and more run at the rate of a large copy; 580 us is 59 TFLOP/s, where the vendor
 // library's 64-bit product reaches 64.  Two tiles of features a wave from 8,192 on (fewer blocks below that would
 // leave CUs idle).  Up to 32 rows the streaming kernel always (20 x 128256 x 2048: 325 against 320 for the tiles,
@@ -292,8 +303,10 @@ extern "C" int mi_gemm_f32(const float* a, int64_t lda, const float* w, int64_t 
     return MI_OK;
   }
   const bool aligned = a16 && w16 && k % 4 == 0;
-  if ((int64_t)ceil_div(n, BN) * ceil_div(m, 64) < 1024 && m <= 32 * 65535) launch_tiles<32, 4>(a, lda, w, ldw, c, ldc, m, n, k, aligned, stream);
-  else launch_tiles<64, 1>(a, lda, w, ldw, c, ldc, m, n, k, aligned, stream);
+  const bool many_blocks = (int64_t)ceil_div(n, BN) * ceil_div(m, 64) >= 1024 || m > 32 * 65535;
+  if (many_blocks) launch_tiles<64, 1>(a, lda, w, ldw, c, ldc, m, n, k, aligned, stream);
+  else if (segment_slices(k) % 4 == 0) launch_tiles<32, 4>(a, lda, w, ldw, c, ldc, m, n, k, aligned, stream);
+  else launch_tiles<32, 1>(a, lda, w, ldw, c, ldc, m, n, k, aligned, stream);
   MI_CHECK_LAUNCH("gemm_f32");
   return MI_OK;
 }

@@ -119,7 +119,7 @@ def test_gemm_f32_is_true_float32(m, n, k):
 
 
 @pytest.mark.parametrize("m,n,k", [(1, 16, 32), (16, 8200, 96), (17, 33, 544), (32, 100, 2048), (33, 8, 352), (64, 50, 257), (65, 130, 4096),
-                                   (50, 8192, 160), (700, 6200, 100), (90, 70, 36)])
+                                   (50, 8192, 160), (700, 6200, 100), (90, 70, 36), (80, 70, 900)])
 def test_gemm_f32_kernels_and_alignments_agree(m, n, k):
     """Every kernel (few rows in 1, 2 or 4 tiles, large and small blocks) and both ways of loading (16 bytes, single values) sum
     an output in the same order: the same bits, and the exact product rounded once (half an ulp, plus what 64-bit sums lose)."""
