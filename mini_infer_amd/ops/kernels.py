@@ -1954,7 +1954,7 @@ def delta_state_shape(heads: int, dim: int, vdim: int) -> tuple[int, int, int]:
     return (heads, vdim, 64 if dim <= 64 else (128 if dim <= 128 else 256))
 
 
-def chunked_scan_pays(tokens: int, requests: int) -> bool:
+def chunked_scan_pays(tokens: int, requests: int, widest: int) -> bool:
     """Whether a recurrence over a step's rows is taken 32 tokens at a time on the matrix cores rather than token by token.
     Token by token a step takes about as long as its longest portion (0.3 to 0.45 microseconds a token at heads of 128 x 128);
     a chunk takes 1.6 to 3 microseconds, but a request with a single token costs as much as one with 32.  Measured, token by
@@ -2000,7 +2000,7 @@ def gated_delta(
     out = torch.empty((qkv.shape[0], heads * vdim), dtype=qkv.dtype, device=qkv.device)
     readout = torch.empty((qkv.shape[0], heads * vdim), dtype=torch.float32, device=qkv.device)  # S^T q before its norm
     lib = library.load()
-    if qkv.dtype == torch.bfloat16 and chunked_scan_pays(qkv.shape[0], requests):
+    if qkv.dtype == torch.bfloat16 and chunked_scan_pays(qkv.shape[0], requests, max(qkv.stride(0), heads * vdim)):
         floats = lib.mi_gated_delta_chunks_scratch(qkv.shape[0], requests, heads, kv_heads, dim, vdim)
         if floats > 0:
             scratch = torch.empty(floats, dtype=torch.float32, device=qkv.device)
@@ -2390,7 +2390,7 @@ def decay_scan(
         raise KernelShapeError("decay_scan: one more boundary than requests")
     out = torch.empty((tokens, heads * vdim), dtype=torch.float32, device=q.device)
     lib = library.load()
-    if q.dtype == torch.bfloat16 and chunked_scan_pays(tokens, requests):
+    if q.dtype == torch.bfloat16 and chunked_scan_pays(tokens, requests, max(v.stride(0), heads * vdim)):
         floats = lib.mi_decay_scan_chunks_scratch(int(per_head), tokens, requests, heads, groups, dim)
         if floats > 0:
             scratch = torch.empty(floats, dtype=torch.float32, device=q.device)

@@ -37,7 +37,7 @@ def _both(monkeypatch, call, state):
 
     made = []
     for chunks in (True, False):
-        monkeypatch.setattr(kernels, "chunked_scan_pays", lambda tokens, requests, chunks=chunks: chunks)
+        monkeypatch.setattr(kernels, "chunked_scan_pays", lambda tokens, requests, widest, chunks=chunks: chunks)
         left = state.clone()
         made.append((call(left), left))
     return made
