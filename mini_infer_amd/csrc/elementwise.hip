@@ -502,8 +502,6 @@ __global__ __launch_bounds__(256) void rope_kv_write_kernel(
 // The same for the usual layout (halves paired, every size a multiple of 4), four
 // elements per thread and step: 8- and 16-byte loads and stores instead of single
 // elements.  Arithmetic and rounding are those of the kernel above.
-typedef __attribute__((__vector_size__(8 * sizeof(__bf16)))) __bf16 bf16x8_vec;
-
 template <typename T>
 __global__ __launch_bounds__(256) void rope_kv_write_vec4_kernel(
     T* __restrict__ qkv, int64_t row_stride, const float* __restrict__ cos_t,
@@ -580,42 +578,12 @@ __global__ __launch_bounds__(256) void rope_kv_write_vec4_kernel(
     load_biased(k_col + h * head_dim + d, x);
     store4(k_pages + (((int64_t)page * kv_heads + h) * page_size + off) * head_dim + d, x);
   }
-  if (v_transposed && page_size % 8 == 0) {
-    // Transposed value pages keep a dim's slots side by side: where this step's tokens fill a
-    // whole page in order (a prompt's portion), a dim's row of the page is written at once
-    // (page_size elements in a row instead of one at a time); the page's tokens share the
-    // (head, dim) rows among them, each taking one page_size-th of them (all of them on the
-    // page's first token measured 18.1 us for 2,048 tokens of 8 heads of 128, shared out 11 us).
-    const int lead = t - off;
-    bool whole_page = lead >= 0 && lead + page_size <= num_tokens;
-    if (whole_page) {
-      for (int i = 0; i < page_size; ++i) whole_page = whole_page && slot_mapping[lead + i] == page * page_size + i;
-    }
-    if (whole_page) {
-      const int rows_each = (kv_heads * v_dim + page_size - 1) / page_size;
-      const int e_end = min((off + 1) * rows_each, kv_heads * v_dim);
-      for (int e = off * rows_each + first; e < e_end; e += stride) {
-        const int h = e / v_dim, d = e % v_dim;
-        T* dst = v_pages + ((int64_t)page * kv_heads + h) * page_size * v_dim + (int64_t)d * page_size;
-        const T* src = qkv + (int64_t)lead * row_stride + v_col + h * v_dim + d;
-        const float more = bias ? bias[v_col + h * v_dim + d] : 0.f;
-        for (int i0 = 0; i0 < page_size; i0 += 8) {
-          if constexpr (sizeof(T) == 2) {
-            bf16x8_vec x;
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-              x[i] = src[(int64_t)(i0 + i) * row_stride];
-              if (bias) x[i] = (bf16_t)((float)x[i] + more);
-            }
-            *reinterpret_cast<bf16x8_vec*>(dst + i0) = x;
-          } else {
-#pragma unroll
-            for (int i = 0; i < 8; ++i) dst[i0 + i] = from_f32<T>(to_f32(src[(int64_t)(i0 + i) * row_stride]) + more);
-          }
-        }
-      }
-      return;
-    }
+  if (v_transposed && mi_fills_page(slot_mapping, t, page, off, page_size, num_tokens)) {
+    mi_write_page_rows(v_pages, t, page, off, page_size, kv_heads, v_dim, first, stride, [&](int token, int e) {
+      const float x = to_f32(qkv[(int64_t)token * row_stride + v_col + e]);
+      return bias ? x + bias[v_col + e] : x;
+    });
+    return;
   }
   const int dim4 = v_dim / 4;
   for (int e = first; e < kv_heads * dim4; e += stride) {

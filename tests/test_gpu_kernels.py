@@ -997,3 +997,50 @@ def test_kernels_refuse_what_they_do_not_take():
         ops.add_rmsnorm(None, torch.zeros(2, 8, device=DEV), torch.ones(9, device=DEV), 1e-5)
     with pytest.raises(KernelShapeError):
         ops.gemm_f32(torch.zeros(2, 8, device=DEV), torch.zeros(3, 9, device=DEV))
+
+
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("q_heads,kv_heads,dim,rotary,vdim,page,first", [(24, 8, 128, 128, 128, 16, 13), (3, 2, 72, 8, 24, 8, 8),
+                                                                       (2, 1, 264, 256, 36, 8, 3), (5, 5, 8, 0, 4, 16, 0)])
+def test_portions_that_fill_pages_write_what_single_tokens_write(dtype, q_heads, kv_heads, dim, rotary, vdim, page, first):
+    """A page of transposed values that a step fills in order is written a dim's row at once, the others an element at a
+    time; and a head by a part of a wave.  Token by token no page is filled: the same bits."""
+    from mini_infer_amd import ops
+
+    tokens, q_width, k_width, v_width = 43, q_heads * dim, kv_heads * dim, kv_heads * vdim
+    rows = _rand(tokens, q_width + k_width + v_width, dtype=dtype, seed=3)
+    angles, other = _rand(tokens, rotary // 2, seed=4), _rand(tokens, v_width, dtype=dtype, seed=5)
+    q_weight, k_weight, mix = _rand(q_width, seed=6), _rand(k_width, seed=7), torch.tensor([0.3], device=DEV)
+    slots = torch.arange(first, first + tokens, dtype=torch.int32, device=DEV)
+    slots[20] = -1  # a row that writes nowhere: its page is not filled
+    made = []
+    for step in (tokens, 1):
+        left = []
+        for op in range(2):
+            qkv = rows.clone()
+            k_pages = torch.zeros(1 + (first + tokens) // page, kv_heads, page, dim, dtype=dtype, device=DEV)
+            v_pages = torch.zeros(1 + (first + tokens) // page, kv_heads, vdim, page, dtype=dtype, device=DEV)
+            for t in range(0, tokens, step):
+                part = slice(t, t + step)
+                if op == 0:
+                    ops.head_norm_rope_kv_write(qkv[part], angles[part].cos(), angles[part].sin(), slots[part].contiguous(), k_pages, v_pages,
+                                                q_weight[:dim].contiguous(), k_weight[:dim].contiguous(), 1e-5, q_heads=q_heads, kv_heads=kv_heads,
+                                                head_dim=dim, rotary_dim=rotary, v_head_dim=vdim, v_transposed=True)
+                else:
+                    ops.qkv_norm_write(qkv[part], q_weight, k_weight, slots[part].contiguous(), k_pages, v_pages, q_width=q_width,
+                                       kv_heads=kv_heads, head_dim=dim, v_head_dim=vdim, eps=1e-5, other_values=other[part], mix=mix,
+                                       v_transposed=True)
+            left += [qkv, k_pages, v_pages]
+        made.append(left)
+    for whole, single in zip(*made):
+        assert torch.equal(whole, single)
+    normed = rows[:, :q_width].double().view(tokens, q_heads, dim)
+    normed = normed / torch.sqrt((normed * normed).mean(-1, keepdim=True) + 1e-5) * q_weight[:dim].double()
+    turned = normed.clone()
+    if rotary:
+        cos, sin = angles.double().cos()[:, None], angles.double().sin()[:, None]
+        lo, hi = normed[..., : rotary // 2], normed[..., rotary // 2 : rotary]
+        turned[..., :rotary] = torch.cat((lo * cos - hi * sin, hi * cos + lo * sin), -1)
+    got = made[0][0][:, :q_width].double().view(tokens, q_heads, dim)
+    # one rounding to the element type, and a few float32 roundings before it
+    assert (got - turned).abs().max() <= (2.0 ** -8 if dtype == torch.bfloat16 else 1e-6) * turned.abs().max()
