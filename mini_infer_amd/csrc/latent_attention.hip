@@ -10,6 +10,7 @@
 //                    into the token's slot of the key pages as one row [c | r]; each head's
 //                    rotated query part goes behind that head's folded part in the query rows
 //                    the attention reads ([head][rank + rot]).
+//   latent_expand_pages   for steps in which every request begins: keys and values written out per head.
 //
 // Rotation pairs entry 2i with 2i+1; cos and sin come as float32 tables [tokens, rot/2].
 #include "common.h"
@@ -99,71 +100,141 @@ __global__ __launch_bounds__(256) void latent_prepare_kernel(
   }
 }
 
-// Keys and values written out per head, for a prompt that is in the step from its first token:
-// one row [q | k | v] per token with heads of D = dim + rot columns each,
-//   q head: [query's plain part | its rotated part]      k head: [W_uk c | rotated shared part]
-//   v head: [W_uv c | zeros up to D]
-// which the paged attention kernels take like any other stacked projection.
+// Keys and values written out per head into pages of the step's own, for prompts that are in the step from their first
+// token, and the queries' rotation:
+//   q head: [plain part | rotated part], in place or into rows of their own      k head: [W_uk c | rotated shared part]
+//   v head: [W_uv c | zeros up to v_width], transposed: a dim's slots side by side
+// which the paged attention kernels take.  A block makes a page of some heads whole, zeros behind a request's last token
+// included.  Bound by the bytes: each value is read and written once, 16 bytes a thread (EIGHTS: sizes and strides in
+// whole 8s; without, an element a thread).  1,501 tokens of 24 heads of 128 + 64, 128 wide values (50 MB,
+// 10.5 us at the rate of a large copy): 14.7 us, for 46.4 as one row [q | k | v] a token, a fill of the pages and a copy into them.
 template <typename T>
-__global__ __launch_bounds__(256) void latent_expand_kernel(
-    const T* __restrict__ proj, int64_t proj_stride, int q_head_width, int q_rot_at, int r_col,
-    const T* __restrict__ k_up, int64_t k_up_stride, const T* __restrict__ v_up, int64_t v_up_stride,
-    const float* __restrict__ cos_t, const float* __restrict__ sin_t, T* __restrict__ qkv, int64_t qkv_stride, int heads,
-    int dim, int rot, int vdim, const T* __restrict__ down, int64_t down_stride) {
-  const int t = blockIdx.x;
-  const int half = rot / 2, D = dim + rot;
-  const T* row = proj + (int64_t)t * proj_stride;
-  const float* c = cos_t + (int64_t)t * half;
-  const float* s = sin_t + (int64_t)t * half;
-  T* out = qkv + (int64_t)t * qkv_stride;
-  const T* ku = k_up + (int64_t)t * k_up_stride;
-  const T* vu = v_up + (int64_t)t * v_up_stride;
-  for (int e = threadIdx.x; e < heads * D; e += blockDim.x) {
-    const int h = e / D, d = e % D;
-    T qv, kv;
-    if (d < dim) {
-      qv = row[h * q_head_width + d];  // (plain parts lie in front of a query head: q_rot_at == dim)
-      kv = ku[h * dim + d];
-    } else {
-      const int i = (d - dim) / 2, odd = (d - dim) & 1;
-      const T* qx = row + h * q_head_width + q_rot_at + 2 * i;
-      const T* kx = (down != nullptr ? down + (int64_t)t * down_stride : row) + r_col + 2 * i;
-      const float q0 = to_f32(qx[0]), q1 = to_f32(qx[1]), k0 = to_f32(kx[0]), k1 = to_f32(kx[1]);
-      qv = from_f32<T>(odd ? q1 * c[i] + q0 * s[i] : q0 * c[i] - q1 * s[i]);
-      kv = from_f32<T>(odd ? k1 * c[i] + k0 * s[i] : k0 * c[i] - k1 * s[i]);
+struct BitsOf {
+  using type = uint32_t;
+};
+template <>
+struct BitsOf<bf16_t> {
+  using type = uint16_t;
+};
+
+template <typename T, bool EIGHTS>
+__global__ __launch_bounds__(256) void latent_expand_pages_kernel(
+    const T* proj, int64_t proj_stride, const T* __restrict__ shared_key, int64_t shared_stride, const T* __restrict__ k_up,
+    int64_t k_up_stride, const T* __restrict__ v_up, int64_t v_up_stride, const float* __restrict__ cos_t,
+    const float* __restrict__ sin_t, T* queries, int64_t queries_stride, T* __restrict__ k_pages, T* __restrict__ v_pages,
+    const int* __restrict__ page_first, const int* __restrict__ page_tokens, int heads, int dim, int rot, int vdim, int v_width,
+    int page_size, int heads_each) {
+  constexpr int V = EIGHTS ? 8 : 1;
+  struct alignas(V * sizeof(T) < 16 ? V * sizeof(T) : 16) Piece {
+    T v[V];
+  };
+  const int page = blockIdx.x, h0 = blockIdx.y * heads_each, nh = min(heads_each, heads - h0);
+  const int t0 = page_first[page], n = page_tokens[page];
+  const int D = dim + rot, half = rot / 2, pieces = D / V;
+  const bool copies = queries != proj;
+  for (int i = threadIdx.x; i < page_size * nh * pieces; i += blockDim.x) {
+    const int d = i % pieces * V, h = h0 + i / pieces % nh, off = i / (pieces * nh);
+    T* k_at = k_pages + (((int64_t)page * heads + h) * page_size + off) * D + d;
+    Piece k;
+    if (off >= n) {
+#pragma unroll
+      for (int j = 0; j < V; ++j) k.v[j] = from_f32<T>(0.f);
+      *reinterpret_cast<Piece*>(k_at) = k;
+      continue;
     }
-    out[e] = qv;
-    out[(int64_t)heads * D + e] = kv;
-    out[2 * (int64_t)heads * D + e] = d < vdim ? vu[h * vdim + d] : from_f32<T>(0.f);
+    const int64_t t = t0 + off;
+    const T* q_from = proj + t * proj_stride + (int64_t)h * D + d;
+    T* q_to = queries + t * queries_stride + (int64_t)h * D + d;
+    if (d < dim) {
+      *reinterpret_cast<Piece*>(k_at) = *reinterpret_cast<const Piece*>(k_up + t * k_up_stride + (int64_t)h * dim + d);
+      if (copies) *reinterpret_cast<Piece*>(q_to) = *reinterpret_cast<const Piece*>(q_from);
+      continue;
+    }
+    const T* shared = shared_key + t * shared_stride + (d - dim);
+    const float *c = cos_t + t * half + (d - dim) / 2, *s = sin_t + t * half + (d - dim) / 2;
+    if constexpr (EIGHTS) {
+      const Piece q = *reinterpret_cast<const Piece*>(q_from), r = *reinterpret_cast<const Piece*>(shared);
+      float cj[4], sj[4];
+      mi_load_cols<float, 4>(c, cj);
+      mi_load_cols<float, 4>(s, sj);
+      Piece turned;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const float q0 = to_f32(q.v[2 * j]), q1 = to_f32(q.v[2 * j + 1]), k0 = to_f32(r.v[2 * j]), k1 = to_f32(r.v[2 * j + 1]);
+        turned.v[2 * j] = from_f32<T>(q0 * cj[j] - q1 * sj[j]);
+        turned.v[2 * j + 1] = from_f32<T>(q1 * cj[j] + q0 * sj[j]);
+        k.v[2 * j] = from_f32<T>(k0 * cj[j] - k1 * sj[j]);
+        k.v[2 * j + 1] = from_f32<T>(k1 * cj[j] + k0 * sj[j]);
+      }
+      *reinterpret_cast<Piece*>(q_to) = turned;
+    } else {
+      const int odd = (d - dim) & 1;
+      const float q0 = to_f32(q_from[-odd]), q1 = to_f32(q_from[1 - odd]), k0 = to_f32(shared[-odd]), k1 = to_f32(shared[1 - odd]);
+      q_to[0] = from_f32<T>(odd ? q1 * *c + q0 * *s : q0 * *c - q1 * *s);
+      k.v[0] = from_f32<T>(odd ? k1 * *c + k0 * *s : k0 * *c - k1 * *s);
+    }
+    *reinterpret_cast<Piece*>(k_at) = k;
+  }
+  // (tokens past the last one and columns past the values: the last ones' bits, masked; a choice would be a branch a load)
+  using Bits = typename BitsOf<T>::type;
+  for (int i = threadIdx.x; i < nh * v_width; i += blockDim.x) {
+    const int h = h0 + i / v_width, d = i % v_width;
+    const Bits* from = reinterpret_cast<const Bits*>(v_up) + (int64_t)h * vdim + min(d, vdim - 1);
+    Bits* to = reinterpret_cast<Bits*>(v_pages) + (((int64_t)page * heads + h) * v_width + d) * page_size;
+    for (int o = 0; o < page_size; o += V) {
+      struct alignas(V * sizeof(Bits) < 16 ? V * sizeof(Bits) : 16) Slots {
+        Bits v[V];
+      } x;
+#pragma unroll
+      for (int j = 0; j < V; ++j) x.v[j] = from[(int64_t)(t0 + min(o + j, n - 1)) * v_up_stride];
+#pragma unroll
+      for (int j = 0; j < V; ++j) x.v[j] &= (Bits)(o + j < n && d < vdim ? ~0u : 0u);
+      *reinterpret_cast<Slots*>(to + o) = x;
+    }
   }
 }
 
 }  // namespace
 
-extern "C" int mi_latent_expand(int dtype, const void* proj, int64_t proj_stride, int q_head_width, int q_rot_at, int r_col,
-                                const void* k_up, int64_t k_up_stride, const void* v_up, int64_t v_up_stride,
-                                const float* cos_t, const float* sin_t, void* qkv, int64_t qkv_stride, int num_tokens,
-                                int heads, int dim, int rot, int vdim, const void* down, int64_t down_stride,
-                                hipStream_t stream) {
-  MI_REQUIRE(num_tokens >= 0 && heads > 0 && dim > 0 && rot >= 0 && rot % 2 == 0 && vdim > 0 && vdim <= dim + rot,
-             "latent_expand: bad sizes tokens=%d heads=%d dim=%d rot=%d vdim=%d", num_tokens, heads, dim, rot, vdim);
-  MI_REQUIRE(q_rot_at == dim && q_head_width >= dim + rot, "latent_expand: a query head is [plain (dim) | to rotate (rot)]");
-  MI_REQUIRE(proj_stride >= (int64_t)heads * q_head_width && (down != nullptr ? down_stride : proj_stride) >= r_col + (int64_t)rot && r_col >= 0 &&
-                 k_up_stride >= (int64_t)heads * dim && v_up_stride >= (int64_t)heads * vdim &&
-                 qkv_stride >= 3 * (int64_t)heads * (dim + rot),
-             "latent_expand: row strides shorter than a row");
-  MI_REQUIRE(dtype == MI_F32 || dtype == MI_BF16, "latent_expand: unknown dtype %d", dtype);
-  if (num_tokens == 0) return MI_OK;
-  if (dtype == MI_F32)
-    latent_expand_kernel<float><<<num_tokens, 256, 0, stream>>>(
-        (const float*)proj, proj_stride, q_head_width, q_rot_at, r_col, (const float*)k_up, k_up_stride, (const float*)v_up,
-        v_up_stride, cos_t, sin_t, (float*)qkv, qkv_stride, heads, dim, rot, vdim, (const float*)down, down_stride);
-  else
-    latent_expand_kernel<bf16_t><<<num_tokens, 256, 0, stream>>>(
-        (const bf16_t*)proj, proj_stride, q_head_width, q_rot_at, r_col, (const bf16_t*)k_up, k_up_stride,
-        (const bf16_t*)v_up, v_up_stride, cos_t, sin_t, (bf16_t*)qkv, qkv_stride, heads, dim, rot, vdim, (const bf16_t*)down,
-        down_stride);
-  MI_CHECK_LAUNCH("latent_expand");
+// proj: query heads [plain (dim) | to rotate (rot)] from column 0 on; shared_key: the shared part's rows, from its first
+// column.  queries: rows of heads * (dim + rot), or proj itself (its heads are then rotated in place).  page_first,
+// page_tokens: per page its first token and how many it holds, 1 .. page_size; every token lies in one page.
+extern "C" int mi_latent_expand_pages(int dtype, const void* proj, int64_t proj_stride, const void* shared_key, int64_t shared_stride,
+                                      const void* k_up, int64_t k_up_stride, const void* v_up, int64_t v_up_stride,
+                                      const float* cos_t, const float* sin_t, void* queries, int64_t queries_stride, void* k_pages,
+                                      void* v_pages, const int* page_first, const int* page_tokens, int num_pages, int heads, int dim,
+                                      int rot, int vdim, int v_width, int page_size, hipStream_t stream) {
+  MI_REQUIRE(num_pages >= 0 && heads > 0 && dim > 0 && rot >= 0 && rot % 2 == 0 && vdim > 0 && v_width >= vdim && page_size > 0,
+             "latent_expand_pages: bad sizes pages=%d heads=%d dim=%d rot=%d vdim=%d v_width=%d page_size=%d", num_pages, heads, dim,
+             rot, vdim, v_width, page_size);
+  MI_REQUIRE(proj_stride >= (int64_t)heads * (dim + rot) && queries_stride >= (int64_t)heads * (dim + rot) && shared_stride >= rot &&
+                 k_up_stride >= (int64_t)heads * dim && v_up_stride >= (int64_t)heads * vdim,
+             "latent_expand_pages: row strides shorter than a row");
+  MI_REQUIRE(dtype == MI_F32 || dtype == MI_BF16, "latent_expand_pages: unknown dtype %d", dtype);
+  const bool eights = dim % 8 == 0 && rot % 8 == 0 && page_size % 8 == 0 &&
+                      (proj_stride | shared_stride | k_up_stride | queries_stride) % 8 == 0 &&
+                      ((uintptr_t)proj | (uintptr_t)shared_key | (uintptr_t)k_up | (uintptr_t)cos_t | (uintptr_t)sin_t |
+                       (uintptr_t)queries | (uintptr_t)k_pages | (uintptr_t)v_pages) % 16 == 0;
+  MI_REQUIRE(queries != proj || (eights && queries_stride == proj_stride), "latent_expand_pages: rows that cannot be rotated in place");
+  if (num_pages == 0) return MI_OK;
+  const int heads_each = 4;
+  MI_REQUIRE(ceil_div(heads, heads_each) <= 65535 && (int64_t)page_size * heads_each * (dim + rot) <= 2147483647,
+             "latent_expand_pages: heads=%d or page_size=%d is too large", heads, page_size);
+  dim3 grid(num_pages, ceil_div(heads, heads_each));
+#define MI_EXPAND(T, EIGHTS)                                                                                                   \
+  latent_expand_pages_kernel<T, EIGHTS><<<grid, 256, 0, stream>>>(                                                             \
+      (const T*)proj, proj_stride, (const T*)shared_key, shared_stride, (const T*)k_up, k_up_stride, (const T*)v_up, v_up_stride, \
+      cos_t, sin_t, (T*)queries, queries_stride, (T*)k_pages, (T*)v_pages, page_first, page_tokens, heads, dim, rot, vdim, v_width, \
+      page_size, heads_each)
+  if (dtype == MI_F32) {
+    if (eights) MI_EXPAND(float, true);
+    else MI_EXPAND(float, false);
+  } else {
+    if (eights) MI_EXPAND(bf16_t, true);
+    else MI_EXPAND(bf16_t, false);
+  }
+#undef MI_EXPAND
+  MI_CHECK_LAUNCH("latent_expand_pages");
   return MI_OK;
 }
 

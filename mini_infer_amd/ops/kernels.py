@@ -2074,38 +2074,58 @@ def latent_prepare(
     )
 
 
-def latent_expand(
-    proj: torch.Tensor, k_up: torch.Tensor, v_up: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, *, heads: int,
-    dim: int, rot: int, vdim: int, r_col: int, down: torch.Tensor | None = None,
+def latent_expand_pages(
+    proj: torch.Tensor, k_up: torch.Tensor, v_up: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, k_pages: torch.Tensor,
+    v_pages: torch.Tensor, page_first: torch.Tensor, page_tokens: torch.Tensor, *, heads: int, dim: int, rot: int, vdim: int,
+    r_col: int, down: torch.Tensor | None = None,
 ) -> torch.Tensor:
-    """One row [q | k | v] per token with `heads` heads of D = dim + rot columns each, from a latent
-    attention layer's projections (`proj`: query heads [plain (dim) | to rotate (rot)] from column 0
-    on, the shared part to rotate from `r_col` on), the keys' plain parts `k_up` [T, heads*dim] and the
-    values `v_up` [T, heads*vdim] (padded with zeros to D): what the paged attention kernels take."""
-    _need_cuda(proj, k_up, v_up, cos, sin)
-    for name, t in (("proj", proj), ("k_up", k_up), ("v_up", v_up)):
+    """Keys and values of a latent attention layer written out per head into pages that hold the step's tokens alone, and the
+    queries rotated: what the paged attention kernels take.
+
+    `proj`: query heads [plain (dim) | to rotate (rot)] from column 0 on; the shared part to rotate from column `r_col` on of
+    `down`, or of `proj` without it; the keys' plain parts `k_up` [T, heads*dim] and the values `v_up` [T, heads*vdim].
+    `k_pages` [pages, heads, page_size, dim + rot] and `v_pages` [pages, heads, width, page_size] (width at least `vdim`, the
+    rest zeros) are written whole, slots without a token with zeros.  `page_first`, `page_tokens` (int32): per page its first
+    token and how many it holds (1 to page_size); together all tokens, each in one page.
+
+    Returns rows [T, >= heads * (dim + rot)] with the rotated queries in the first columns: `proj` itself, rotated in place,
+    where its rows allow 16-byte accesses, else rows of their own."""
+    _need_cuda(proj, k_up, v_up, cos, sin, k_pages, v_pages, page_first, page_tokens)
+    for name, t in (("proj", proj), ("k_up", k_up), ("v_up", v_up), ("down", proj if down is None else down)):
         if t.dim() != 2 or t.stride(1) != 1 or t.dtype != proj.dtype or t.shape[0] != proj.shape[0]:
-            raise KernelShapeError(f"latent_expand: {name} must be rows of the step in {proj.dtype} with unit inner stride")
-    _need_contiguous("cos", cos)
-    _need_contiguous("sin", sin)
+            raise KernelShapeError(f"latent_expand_pages: {name} must be rows of the step in {proj.dtype} with unit inner stride")
+    for name, t in (("cos", cos), ("sin", sin), ("k_pages", k_pages), ("v_pages", v_pages), ("page_first", page_first),
+                    ("page_tokens", page_tokens)):
+        _need_contiguous(name, t)
     tokens, width = proj.shape[0], dim + rot
     if cos.dtype != torch.float32 or tuple(cos.shape) != (tokens, rot // 2) or sin.shape != cos.shape or sin.dtype != torch.float32:
-        raise KernelShapeError(f"latent_expand: cos/sin must be float32 [{tokens}, {rot // 2}]")
-    if down is not None and (down.dim() != 2 or down.stride(1) != 1 or down.dtype != proj.dtype or down.shape[0] != tokens
-                             or down.shape[1] < r_col + rot):
-        raise KernelShapeError("latent_expand: the rows that hold the shared part do not fit")
-    if k_up.shape[1] != heads * dim or v_up.shape[1] != heads * vdim or vdim > width or proj.shape[1] < max(
-            heads * width, 0 if down is not None else r_col + rot):
-        raise KernelShapeError("latent_expand: the projections do not hold what the sizes say")
-    qkv = torch.empty((tokens, 3 * heads * width), dtype=proj.dtype, device=proj.device)
+        raise KernelShapeError(f"latent_expand_pages: cos/sin must be float32 [{tokens}, {rot // 2}]")
+    holds_shared = proj if down is None else down
+    if holds_shared.shape[1] < r_col + rot or r_col < 0:
+        raise KernelShapeError("latent_expand_pages: the rows that hold the shared part do not fit")
+    if k_up.shape[1] != heads * dim or v_up.shape[1] != heads * vdim or proj.shape[1] < heads * width:
+        raise KernelShapeError("latent_expand_pages: the projections do not hold what the sizes say")
+    pages, page_size = k_pages.shape[0], k_pages.shape[2]
+    if k_pages.dtype != proj.dtype or v_pages.dtype != proj.dtype or tuple(k_pages.shape) != (pages, heads, page_size, width) or (
+        v_pages.dim() != 4 or v_pages.shape[2] < vdim or tuple(v_pages.shape) != (pages, heads, v_pages.shape[2], page_size)
+    ):
+        raise KernelShapeError("latent_expand_pages: the pages do not hold such keys and transposed values")
+    _need_int32("page_first", page_first)
+    _need_int32("page_tokens", page_tokens)
+    if page_first.numel() != pages or page_tokens.numel() != pages:
+        raise KernelShapeError("latent_expand_pages: one first token and one count per page")
+    shared = holds_shared[:, r_col:]
+    in_eights = all(n % 8 == 0 for n in (dim, rot, page_size, proj.stride(0), shared.stride(0), k_up.stride(0))) and all(
+        t.data_ptr() % 16 == 0 for t in (proj, shared, k_up, cos, sin, k_pages, v_pages))
+    queries = proj if in_eights else torch.empty((tokens, heads * width), dtype=proj.dtype, device=proj.device)
     library.check(
-        library.load().mi_latent_expand(
-            _dtype_code(proj), _ptr(proj), proj.stride(0), width, dim, int(r_col), _ptr(k_up), k_up.stride(0), _ptr(v_up),
-            v_up.stride(0), _ptr(cos), _ptr(sin), _ptr(qkv), qkv.stride(0), tokens, heads, dim, rot, vdim,
-            _ptr(down), 0 if down is None else down.stride(0), _stream(),
+        library.load().mi_latent_expand_pages(
+            _dtype_code(proj), _ptr(proj), proj.stride(0), shared.data_ptr(), shared.stride(0), _ptr(k_up), k_up.stride(0),
+            _ptr(v_up), v_up.stride(0), _ptr(cos), _ptr(sin), _ptr(queries), queries.stride(0), _ptr(k_pages), _ptr(v_pages),
+            _ptr(page_first), _ptr(page_tokens), pages, heads, dim, rot, vdim, v_pages.shape[2], page_size, _stream(),
         )
     )
-    return qkv
+    return queries
 
 
 PER_HEAD_MAX_ROWS = 256  # rows up to which the engine's own product head by head is taken

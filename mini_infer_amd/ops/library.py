@@ -108,9 +108,9 @@ _SIGNATURES: dict[str, list] = {
         c_int, _P, c_int64, c_int, c_int, c_int, c_int, _P, _P, _P, _P, _P, _P, c_int64, _P, c_int, c_int, c_int, c_int,
         c_float, _P, c_int64, _P,
     ],
-    "mi_latent_expand": [
-        c_int, _P, c_int64, c_int, c_int, c_int, _P, c_int64, _P, c_int64, _P, _P, _P, c_int64, c_int, c_int, c_int, c_int,
-        c_int, _P, c_int64, _P,
+    "mi_latent_expand_pages": [
+        c_int, _P, c_int64, _P, c_int64, _P, c_int64, _P, c_int64, _P, _P, _P, c_int64, _P, _P, _P, _P, c_int, c_int, c_int, c_int,
+        c_int, c_int, c_int, _P,
     ],
     "mi_embed_norm_streams": [c_int, _P, _P, _P, _P, c_int, c_int, c_int, c_int, c_float, _P],
     "mi_streams_update_norm": [

@@ -163,9 +163,9 @@ class LatentAttention(Mixer):
         cu = ctx.host_cu_seqlens_q
         return all(ctx.host_seq_lens[b] == cu[b + 1] - cu[b] for b in range(len(ctx.host_seq_lens)))
 
-    def _own_pages(self, ctx: StepContext) -> tuple[torch.Tensor, torch.Tensor, int]:
-        """Write slots, block table and page count of pages that hold this step's tokens alone, each
-        request from a page of its own on (made once a step, on the host, for all layers that expand)."""
+    def _own_pages(self, ctx: StepContext) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
+        """Pages that hold this step's tokens alone, each request from a page of its own on: per page its first token and how
+        many it holds, and the block table (made once a step, on the host, for all layers that expand)."""
         key = ("latent_attention_own_pages", ctx.page_size)
         if key not in ctx.shared:
             import numpy as np
@@ -174,13 +174,15 @@ class LatentAttention(Mixer):
             lengths = cu[1:] - cu[:-1]
             pages = -(-lengths // page)
             first = np.concatenate([[0], np.cumsum(pages)])
-            request_of = np.repeat(np.arange(len(lengths)), lengths)
-            slots = first[request_of] * page + (np.arange(cu[-1]) - cu[request_of])
+            request_of = np.repeat(np.arange(len(lengths)), pages)
+            inside = (np.arange(first[-1]) - first[request_of]) * page
             table = np.zeros((len(lengths), max(1, int(pages.max()))), dtype=np.int32)
             for b, count in enumerate(pages):
                 table[b, :count] = first[b] + np.arange(count)
-            both = torch.from_numpy(np.concatenate([slots.astype(np.int32), table.reshape(-1)])).to(self.device)
-            ctx.shared[key] = (both[: slots.size], both[slots.size:].view(table.shape), int(first[-1]))
+            count = np.minimum(page, lengths[request_of] - inside)
+            all_of = torch.from_numpy(np.concatenate([cu[request_of] + inside, count, table.reshape(-1)]).astype(np.int32)).to(self.device)
+            n = int(first[-1])
+            ctx.shared[key] = (all_of[:n], all_of[n : 2 * n], all_of[2 * n :].view(table.shape))
         return ctx.shared[key]
 
     def _forward_expanded(self, proj: torch.Tensor, down, c_col: int, gate: torch.Tensor | None, ctx: StepContext,
@@ -194,24 +196,26 @@ class LatentAttention(Mixer):
             cache.k_pages, None, heads=heads, q_head_width=self.q_head_width, q_rot_at=dim, c_col=c_col,
             rank=rank, rot=rot, eps=self.norm_eps, latent_out=latent, down=down,
         )
-        qkv = ops.latent_expand(proj, self.up_k.forward(latent), self.up_v.forward(latent), rotary.cos, rotary.sin, heads=heads,
-                                dim=dim, rot=rot, vdim=vdim, r_col=c_col + rank, down=down)
-        slots, table, pages = self._own_pages(ctx)
-        # (zeroed: the kernel multiplies what lies past a request's last key by a weight of zero)
-        k_own = torch.zeros((pages, heads, ctx.page_size, width), dtype=proj.dtype, device=proj.device)
-        v_own = torch.zeros((pages, heads, width, ctx.page_size), dtype=proj.dtype, device=proj.device)
-        nothing = torch.empty((tokens, 0), dtype=torch.float32, device=proj.device)
-        ops.rope_kv_write(qkv, nothing, nothing, slots, k_own, v_own, q_heads=heads, kv_heads=heads, head_dim=width,
-                          rotary_dim=0, v_transposed=True)
-        mixed = ops.paged_attention(
-            qkv, k_own, v_own, table, ctx.token_request, ctx.positions, ctx.cu_seqlens_q, ctx.host_cu_seqlens_q, q_heads=heads,
-            kv_heads=heads, head_dim=width, scale=self.scale, window=self.window, max_seq_len=ctx.max_q_len, v_transposed=True,
-            sinks=self.sinks,
+        page_first, page_tokens, table = self._own_pages(ctx)
+        # (values of a width the attention kernel does not take are padded with zeros to the keys')
+        v_width = vdim if ops.mfma_attention_supported(self.dtype, width, ctx.page_size, vdim) else width
+        k_own = torch.empty((page_first.numel(), heads, ctx.page_size, width), dtype=proj.dtype, device=proj.device)
+        v_own = torch.empty((page_first.numel(), heads, v_width, ctx.page_size), dtype=proj.dtype, device=proj.device)
+        queries = ops.latent_expand_pages(
+            proj, self.up_k.forward(latent), self.up_v.forward(latent), rotary.cos, rotary.sin, k_own, v_own, page_first, page_tokens,
+            heads=heads, dim=dim, rot=rot, vdim=vdim, r_col=c_col + rank, down=down,
         )
-        if gate is not None:  # (the padding of the value heads leaves with it)
+        mixed = ops.paged_attention(
+            queries, k_own, v_own, table, ctx.token_request, ctx.positions, ctx.cu_seqlens_q, ctx.host_cu_seqlens_q, q_heads=heads,
+            kv_heads=heads, head_dim=width, scale=self.scale, window=self.window, max_seq_len=ctx.max_q_len, v_transposed=True,
+            sinks=self.sinks, v_head_dim=v_width,
+        )
+        if gate is not None:  # (padding of the value heads leaves with it)
             packed = torch.empty((tokens, heads, vdim), dtype=mixed.dtype, device=mixed.device)
-            ops.gate_heads(mixed.unflatten(1, (heads, width)), gate, packed)
+            ops.gate_heads(mixed.unflatten(1, (heads, v_width)), gate, packed)
             return self.out.forward(packed.view(tokens, heads * vdim))
+        if v_width == vdim:
+            return self.out.forward(mixed)
         if self._out_padded is None:  # W_o with zero columns under the padding of every value head
             assert self.out.weight is not None
             padded = torch.zeros((self.hidden_size, heads, width), dtype=self.out.weight.dtype, device=self.out.weight.device)

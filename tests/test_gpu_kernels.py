@@ -1044,3 +1044,48 @@ def test_portions_that_fill_pages_write_what_single_tokens_write(dtype, q_heads,
     got = made[0][0][:, :q_width].double().view(tokens, q_heads, dim)
     # one rounding to the element type, and a few float32 roundings before it
     assert (got - turned).abs().max() <= (2.0 ** -8 if dtype == torch.bfloat16 else 1e-6) * turned.abs().max()
+
+
+@pytest.mark.parametrize("heads,dim,rot,vdim,v_width,page,spare", [(5, 128, 64, 128, 128, 16, 8), (32, 16, 16, 12, 32, 8, 0), (3, 20, 12, 20, 32, 16, 0),
+                                                                   (4, 64, 0, 64, 64, 16, 3), (1, 24, 8, 7, 32, 4, 0)])
+@pytest.mark.parametrize("apart", [False, True])
+def test_latent_keys_and_values_of_a_step_in_pages(heads, dim, rot, vdim, v_width, page, spare, apart):
+    """Pages written whole, zeros where no token lies; queries rotated in place where rows allow it, else beside."""
+    from mini_infer_amd import ops
+
+    lengths, width = [1, 33, 16, 40], dim + rot
+    tokens = sum(lengths)
+    held = _rand(tokens, rot + 8, dtype=torch.bfloat16, seed=2)
+    proj = _rand(tokens, heads * width + (0 if apart else rot) + spare, dtype=torch.bfloat16, seed=3)
+    shared = held[:, 8:] if apart else proj[:, heads * width : heads * width + rot]
+    before, shared = proj.clone(), shared.clone()
+    k_up, v_up = _rand(tokens, heads * dim, dtype=torch.bfloat16, seed=4), _rand(tokens, heads * vdim + spare, dtype=torch.bfloat16, seed=5)[:, : heads * vdim]
+    angles = _rand(tokens, rot // 2, seed=6)
+    first, count, start = [], [], 0
+    for n in lengths:
+        for at in range(0, n, page):
+            first.append(start + at), count.append(min(page, n - at))
+        start += n
+    k_pages = torch.full((len(first), heads, page, width), float("nan"), dtype=torch.bfloat16, device=DEV)
+    v_pages = torch.full((len(first), heads, v_width, page), float("nan"), dtype=torch.bfloat16, device=DEV)
+    ints = [torch.tensor(x, dtype=torch.int32, device=DEV) for x in (first, count)]
+    queries = ops.latent_expand_pages(proj, k_up, v_up, angles.cos(), angles.sin(), k_pages, v_pages, *ints, heads=heads, dim=dim, rot=rot,
+                                      vdim=vdim, r_col=8 if apart else heads * width, down=held if apart else None)
+
+    def turned(x):  # [..., rot], pairs side by side
+        pairs = x.float().unflatten(-1, (rot // 2, 2))
+        cos, sin = (f().view(tokens, *[1] * (pairs.dim() - 3), rot // 2) for f in (angles.cos, angles.sin))
+        return torch.stack((pairs[..., 0] * cos - pairs[..., 1] * sin, pairs[..., 1] * cos + pairs[..., 0] * sin), -1).flatten(-2)
+
+    q = before[:, : heads * width].view(tokens, heads, width)
+    want_q = torch.cat((q[..., :dim].float(), turned(q[..., dim:])), -1)
+    want_k = torch.cat((k_up.view(tokens, heads, dim).float(), turned(shared)[:, None].expand(tokens, heads, rot)), -1)
+    got_q = queries[:, : heads * width].view(tokens, heads, width).float()
+    # (one rounding to bfloat16, of sums of two products)
+    assert ((got_q - want_q).abs() <= 2.0 ** -8 * want_q.abs() + 1e-6).all()
+    assert torch.equal(proj[:, heads * width :], before[:, heads * width :])
+    for p, (t, n) in enumerate(zip(first, count)):
+        got_k, got_v = k_pages[p].transpose(0, 1).float(), v_pages[p].permute(2, 0, 1)
+        assert ((got_k[:n] - want_k[t : t + n]).abs() <= 2.0 ** -8 * want_k[t : t + n].abs() + 1e-6).all() and (got_k[n:] == 0).all()
+        assert torch.equal(got_v[:n, :, :vdim], v_up[t : t + n].view(n, heads, vdim))
+        assert (got_v[n:] == 0).all() and (got_v[:, :, vdim:] == 0).all()
