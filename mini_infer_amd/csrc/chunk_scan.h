@@ -19,13 +19,16 @@
 // Q S0 meet in LDS (one barrier a chunk), and everything after that is registers.  All operands are float32 and so is
 // the matrix instruction (16x16x4, 154 TFLOP/s): nothing is rounded that the token-by-token form keeps.
 //
-// What bounds it: the chain of one chunk after another. Measured at 2,048 tokens, one wave a SIMD: 2.9 us a chunk for
+// What bounds it: the chain of one chunk after another.  Measured at 2,048 tokens, one wave a SIMD: 2.3 us a chunk for
 // the delta rule (32 heads of 128 x 128: 68 matrix instructions a wave, 35 cycles each, make 1.0 us of it; the rest is
-// issuing some 30 loads of operands one chunk ahead and the exchange through LDS), 1.6 us for the others. Whole calls
-// with the first launch and the norm, token by token before: delta rule 896 -> 225 us, decay per head (64 heads of
-// 128 x 64) 717 -> 118, decay per channel (16 heads of 128 x 256) 772 -> 146. Waiting for everything in flight at the
-// barrier cost 2 us a chunk more. A chunk of 32: at twice that W and T (quadratic) weigh as much as the products with
-// the state, and the inverse no longer stays in a wave's registers.
+// the way through LDS and back, and 0.4 us that the loads of the next chunk's operands cost beside it), 1.6 us for the
+// others.  A block's loads are limited by what the CU's L1 returns, not by their latency, so what all four waves need (W, T,
+// the factors, the values) is brought once, a piece a thread, and goes through LDS under the barrier that is there
+// anyway: 187 -> 145 us for the delta rule, 83 -> 70 and 81 -> 72 for the others (3B sizes, 1,777 tokens), against each
+// wave loading all of it.  Whole calls with the first launch and the norm, token by token before: delta rule 896 -> 184 us,
+// decay per head (64 heads of 128 x 64) 717 -> 117, decay per channel (16 heads of 128 x 256) 774 -> 144.  Waiting for
+// everything in flight at the barrier cost 2 us a chunk more.  A chunk of 32: at twice that W and T (quadratic) weigh as much
+// as the products with the state, and the inverse no longer stays in a wave's registers.
 #pragma once
 #include "common.h"
 
@@ -123,15 +126,26 @@ __device__ __forceinline__ void lds_barrier() {
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
 }
 
-// One chunk's operands in a lane's registers.  Row tiles t of 16 tokens; a lane's four of a tile: tokens 16 t + 4 * (lane / 16) ..,
-// or, as first operand, token 16 t + lane % 16 and four rows of S (or tokens) side by side.
+// One chunk's operands on their way, in a thread's registers.  Rows of S of the wave's own, in the order of the matrix
+// instruction's operands: row tiles t of 16 tokens, token 16 t + lane % 16 and four rows of S (or, of kt, a row of S and four
+// tokens) side by side.  What all waves read: a piece of it, which goes through LDS.
 template <int DT, int MODE>
 struct Operands {
   float4 q[2][DT], k[MODE == DELTA ? 2 : 1][DT], kt[2][DT];
-  float4 within[2], solve[MODE == DELTA ? 3 : 1];
-  float4 g[2], tail[2], fade[MODE == PER_CHANNEL ? DT : 1];
-  float g_last;
-  uint32_t v[2][4];  // as read
+  float4 fade[MODE == PER_CHANNEL ? DT : 1];
+  float4 within, solve;  // four values of a row of W and of T
+  float factor;          // one of the 64 factors
+  uint32_t v[2];         // two columns of a token's values, as read
+};
+
+// What the block's waves share of a chunk.  (Rows of 36: 16-byte reads of 16 rows fall on different banks.)
+constexpr int LDS_ROW = CHUNK + 4;
+template <int MODE>
+struct Shared {
+  float within[CHUNK * LDS_ROW];
+  float solve[MODE == DELTA ? CHUNK * LDS_ROW : 4];
+  float v[16 * LDS_ROW];  // [column][token]
+  float factor[2 * CHUNK];
 };
 
 // grid: heads * column blocks (the heads side by side, so that an XCD's blocks share their chunk data), requests; 256 threads.
@@ -143,6 +157,7 @@ __global__ __launch_bounds__(256, MODE == DELTA || DT > 2 ? 1 : 2) void walk_ker
   constexpr int PAD = 64 * DT;
   constexpr int SUMS = MODE == DELTA ? 4 : 2;
   __shared__ f32x4_t parts[2][4][SUMS][MI_WAVE];
+  __shared__ __align__(16) Shared<MODE> shared[2];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / MI_WAVE), lane = threadIdx.x % MI_WAVE;
   const int head = blockIdx.x % p.heads, b = blockIdx.y;
   const uint32_t r = lane % 16, quad = lane / 16;
@@ -162,15 +177,13 @@ __global__ __launch_bounds__(256, MODE == DELTA || DT > 2 ? 1 : 2) void walk_ker
   const float skip = (MODE == PER_HEAD && p.skip) ? p.skip[head] : 0.f;
   const int out_stride = p.heads * p.vdim;
   // a lane's offsets
-  const uint32_t at_row = r * PAD + 4 * quad, at_column = r * CHUNK + 4 * quad;
-  uint32_t v_at[2][4], out_at[4];
+  const uint32_t at_row = r * PAD + 4 * quad, at_column = r * CHUNK + 4 * quad, in_lds = r * LDS_ROW + 4 * quad;
+  uint32_t out_at[4];
 #pragma unroll
-  for (int e = 0; e < 4; ++e) {
-#pragma unroll
-    for (int t = 0; t < 2; ++t) v_at[t][e] = (16 * t + 4 * quad + e) * (uint32_t)p.v_stride;
-    out_at[e] = (16 * (wave & 1) + 4 * quad + e) * (uint32_t)out_stride + (uint32_t)col;
-  }
-  const uint32_t v_lane = live ? (uint32_t)col : 0u;
+  for (int e = 0; e < 4; ++e) out_at[e] = (16 * (wave & 1) + 4 * quad + e) * (uint32_t)out_stride + (uint32_t)col;
+  // values a thread brings: token 8 * wave + lane / 8 of the chunk, columns lane % 8 and 8 further
+  const uint32_t v_token = 8 * wave + lane / 8, v_at = v_token * (uint32_t)p.v_stride;
+  const uint32_t v_first = (uint32_t)min((int)(col - r) + lane % 8, p.vdim - 1), v_second = (uint32_t)min((int)(col - r) + lane % 8 + 8, p.vdim - 1);
 
   auto fetch = [&](int n, Operands<DT, MODE>& o) {
     const int64_t chunk = chunk0 + n, rows = chunk * p.made.shares + share, of = chunk * p.heads + head;
@@ -188,52 +201,25 @@ __global__ __launch_bounds__(256, MODE == DELTA || DT > 2 ? 1 : 2) void walk_ker
       for (int t = 0; t < 2; ++t)
 #pragma unroll
         for (int d = 0; d < DT; ++d) o.k[t][d] = load4(k + 16 * t * PAD + 16 * d + at_row);
-      const float* solve = p.made.solve + of * CHUNK * CHUNK;
-      o.solve[0] = load4(solve + at_column);
-      o.solve[1] = load4(solve + 16 * CHUNK + at_column);
-      o.solve[2] = load4(solve + 16 * CHUNK + 16 + at_column);
+      o.solve = load4(p.made.solve + of * CHUNK * CHUNK + 4 * threadIdx.x);
     }
-    // (row tile 0 or 1 of the read-outs, which waves 0 and 1 finish)
-    const float* within = p.made.within + of * CHUNK * CHUNK + 16 * (wave & 1) * CHUNK;
-    o.within[0] = load4(within + at_column);
-    o.within[1] = load4(within + 16 + at_column);
+    o.within = load4(p.made.within + of * CHUNK * CHUNK + 4 * threadIdx.x);
     if constexpr (MODE == PER_CHANNEL) {
       const float* fade = p.made.fade + of * PAD + row0;
 #pragma unroll
       for (int d = 0; d < DT; ++d) o.fade[d] = load4(fade + 16 * d + 4 * quad);
     } else {
-      const float* factor = p.made.factor + of * 2 * CHUNK;
-      if constexpr (MODE == DELTA) {
-        o.g[0] = load4(factor + 4 * quad);
-        o.g[1] = load4(factor + 16 + 4 * quad);
-      } else {
-        o.g[0] = load4(factor + 16 * (wave & 1) + 4 * quad);
-      }
-      o.tail[0] = load4(factor + CHUNK + 4 * quad);
-      o.tail[1] = load4(factor + CHUNK + 16 + 4 * quad);
-      o.g_last = factor[CHUNK - 1];
+      o.factor = p.made.factor[of * 2 * CHUNK + lane];
     }
     // (of tokens past the last one the last one's)
     const int t0 = first + n * CHUNK;
     const bf16_t* v = p.v + (int64_t)t0 * p.v_stride + p.v_col + (int64_t)head * p.vdim;
-    const uint32_t most = (uint32_t)(last - 1 - t0) * (uint32_t)p.v_stride;
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) o.v[t][e] = *reinterpret_cast<const uint16_t*>(v + (min(v_at[t][e], most) + v_lane));
+    const uint32_t v_row = min(v_at, (uint32_t)(last - 1 - t0) * (uint32_t)p.v_stride);
+    o.v[0] = *reinterpret_cast<const uint16_t*>(v + (v_row + v_first));
+    o.v[1] = *reinterpret_cast<const uint16_t*>(v + (v_row + v_second));
   };
   auto step = [&](int n, const Operands<DT, MODE>& o) {
-    // values; of tokens past the last one zeros (by their bits: a choice would be compiled into a branch around the load,
-    // and every load waited for by itself)
     const int nt = last - first - n * CHUNK;
-    f32x4_t v[2];
-#pragma unroll
-    for (int t = 0; t < 2; ++t)
-#pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const uint32_t keep = (int)(16 * t + 4 * quad + e) < nt ? 0xFFFF0000u : 0u;
-        v[t][e] = __uint_as_float((o.v[t][e] << 16) & keep);
-      }
     const f32x4_t zero = {0.f, 0.f, 0.f, 0.f};
     f32x4_t sum[SUMS];
 #pragma unroll
@@ -248,28 +234,54 @@ __global__ __launch_bounds__(256, MODE == DELTA || DT > 2 ? 1 : 2) void walk_ker
     // (two buffers: a wave that runs ahead writes the other one, and cannot pass the next barrier)
 #pragma unroll
     for (int t = 0; t < SUMS; ++t) parts[n & 1][wave][t][lane] = sum[t];
+    Shared<MODE>& both = shared[n & 1];
+    const int piece = threadIdx.x / 8 * LDS_ROW + threadIdx.x % 8 * 4;
+    *reinterpret_cast<float4*>(&both.within[piece]) = o.within;
+    if constexpr (MODE == DELTA) *reinterpret_cast<float4*>(&both.solve[piece]) = o.solve;
+    if constexpr (MODE != PER_CHANNEL) {
+      if (wave == 0) both.factor[lane] = o.factor;
+    }
+    {  // (of tokens past the last one zeros, by their bits: a choice would be compiled into a branch around the load, and every
+       // load waited for by itself)
+      const uint32_t keep = (int)v_token < nt ? 0xFFFF0000u : 0u;
+      both.v[lane % 8 * LDS_ROW + v_token] = __uint_as_float((o.v[0] << 16) & keep);
+      both.v[(lane % 8 + 8) * LDS_ROW + v_token] = __uint_as_float((o.v[1] << 16) & keep);
+    }
     lds_barrier();
+    f32x4_t v[2];
+#pragma unroll
+    for (int t = 0; t < 2; ++t) v[t] = *reinterpret_cast<const f32x4_t*>(&both.v[in_lds + 16 * t]);
+    float4 g[2], tails[2];
+    float g_last = 1.f;
+    if constexpr (MODE != PER_CHANNEL) {
+#pragma unroll
+      for (int t = 0; t < 2; ++t) {
+        g[t] = load4(&both.factor[16 * t + 4 * quad]);
+        tails[t] = load4(&both.factor[CHUNK + 16 * t + 4 * quad]);
+      }
+      g_last = both.factor[CHUNK - 1];
+    }
     auto whole = [&](int t) {
       return (parts[n & 1][0][t][lane] + parts[n & 1][1][t][lane]) + (parts[n & 1][2][t][lane] + parts[n & 1][3][t][lane]);
     };
     f32x4_t u[2] = {v[0], v[1]};
     if constexpr (MODE == DELTA) {
 #pragma unroll
-      for (int t = 0; t < 2; ++t) u[t] -= scaled(o.g[t], whole(2 + t));
-      const f32x4_t upper = mma4(o.solve[0], u[0], zero), lower = mma4(o.solve[1], u[0], zero);
-      u[1] = lower + mma4(o.solve[2], u[1], zero);
+      for (int t = 0; t < 2; ++t) u[t] -= scaled(g[t], whole(2 + t));
+      const f32x4_t upper = mma4(load4(&both.solve[in_lds]), u[0], zero), lower = mma4(load4(&both.solve[16 * LDS_ROW + in_lds]), u[0], zero);
+      u[1] = lower + mma4(load4(&both.solve[16 * LDS_ROW + 16 + in_lds]), u[1], zero);
       u[0] = upper;
     }
     f32x4_t tail[2];
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
       if constexpr (MODE == PER_CHANNEL) tail[t] = u[t];
-      else tail[t] = scaled(o.tail[t], u[t]);
+      else tail[t] = scaled(tails[t], u[t]);
     }
 #pragma unroll
     for (int d = 0; d < DT; ++d) {
       if constexpr (MODE == PER_CHANNEL) S[d] = scaled(o.fade[d], S[d]);
-      else S[d] *= o.g_last;
+      else S[d] *= g_last;
     }
 #pragma unroll
     for (int t = 0; t < 2; ++t)
@@ -277,9 +289,10 @@ __global__ __launch_bounds__(256, MODE == DELTA || DT > 2 ? 1 : 2) void walk_ker
       for (int d = 0; d < DT; ++d) S[d] = mma4(o.kt[t][d], tail[t], S[d]);
     if (wave < 2) {
       f32x4_t read = whole(wave);
-      if constexpr (MODE != PER_CHANNEL) read = scaled(MODE == DELTA && wave == 1 ? o.g[1] : o.g[0], read);
-      read += mma4(o.within[0], u[0], zero);
-      if (wave == 1) read += mma4(o.within[1], u[1], zero);
+      if constexpr (MODE != PER_CHANNEL) read = scaled(wave == 1 ? g[1] : g[0], read);
+      const float* within = &both.within[16 * wave * LDS_ROW + in_lds];
+      read += mma4(load4(within), u[0], zero);
+      if (wave == 1) read += mma4(load4(within + 16), u[1], zero);
       if constexpr (MODE == PER_HEAD) read += skip * (wave == 0 ? v[0] : v[1]);
       float* out = p.out + (int64_t)(first + n * CHUNK) * out_stride + (int64_t)head * p.vdim;
 #pragma unroll
@@ -287,7 +300,7 @@ __global__ __launch_bounds__(256, MODE == DELTA || DT > 2 ? 1 : 2) void walk_ker
         if ((int)(16 * wave + 4 * quad + e) < nt && live) out[out_at[e]] = read[e];
     }
   };
-  // (two sets of operands: a third, two chunks ahead, measured 188 -> 185 us and cost the second block of a CU)
+  // (two sets of operands: with a third, two chunks ahead, 162 us instead of 145)
   Operands<DT, MODE> even, odd;
   fetch(0, even);
   for (int n = 0; n + 1 < chunks; n += 2) {
