@@ -1957,12 +1957,13 @@ def delta_state_shape(heads: int, dim: int, vdim: int) -> tuple[int, int, int]:
 def chunked_scan_pays(tokens: int, requests: int, widest: int) -> bool:
     """Whether a recurrence over a step's rows is taken 32 tokens at a time on the matrix cores rather than token by token.
     Token by token a step takes about as long as its longest portion (0.3 to 0.45 microseconds a token at heads of 128 x 128);
-    a chunk takes 1.6 to 3 microseconds, but a request with a single token costs as much as one with 32.  Measured, token by
-    token against in chunks, microseconds: delta rule, 32 heads of 128 x 128: 2,048 tokens 896 / 225, 512 tokens 236 / 74, a
-    portion of 256 beside 15 single tokens 134 / 126, 4 portions of 16 32 / 45, 30 single tokens 65 / 140; a decay per head, 64
-    heads of 128 x 64: 2,048 tokens 717 / 118; 48 heads: 64 tokens 23.5 / 23.3, 256 beside 15 single tokens 304 / 53; a decay
-    per channel, 16 heads of 128 x 256: 2,048 tokens 772 / 146."""
-    return tokens >= 64 + 3 * requests
+    a chunk takes 1.6 to 2.3 microseconds, but a request with a single token costs as much as one with 32.  Measured, token by
+    token against in chunks, microseconds: delta rule, 32 heads of 128 x 128: 2,048 tokens 894 / 184, 512 tokens 230 / 63, a
+    portion of 256 beside 15 single tokens 133 / 88, 4 portions of 16 32 / 35, 30 single tokens 42 / 91; a decay per head, 64
+    heads of 128 x 64: 2,048 tokens 717 / 117; 48 heads: 64 tokens 23.6 / 26.4, 256 beside 15 single tokens 302 / 48; a decay
+    per channel, 16 heads of 128 x 256: 2,048 tokens 774 / 144.  `widest`: values from one row to the next of the widest operand
+    or result; the chunks' kernels reach over their 32 rows in 32 bits."""
+    return tokens >= 64 + 3 * requests and widest < 2**24
 
 
 def gated_delta(

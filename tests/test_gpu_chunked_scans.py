@@ -157,3 +157,24 @@ def test_decaying_state_in_chunks(monkeypatch, lengths, heads, groups, dim, vdim
     if per_head:
         out = out + skip.double()[:, None] * x
     _check(chunked, walked, state, out.flatten(1), torch.stack(left), requests, dim, 4e-7)
+
+
+def test_rows_too_far_apart_for_chunks_go_token_by_token():
+    from mini_infer_amd import ops
+
+    heads, kv_heads, dim, vdim, tokens = 2, 1, 64, 64, 70
+    g = torch.Generator(device=DEV).manual_seed(5)
+    qkv = torch.randn(tokens, 2 * kv_heads * dim + heads * vdim, generator=g, device=DEV).bfloat16()
+    far = torch.empty(tokens, 2**24, dtype=torch.bfloat16, device=DEV)[:, : qkv.shape[1]]
+    far.copy_(qkv)
+    proj = torch.randn(tokens, 2 * heads + heads * vdim, generator=g, device=DEV).bfloat16()
+    a_log, dt_bias, weight = torch.zeros(heads, device=DEV), torch.full((heads,), -2.0, device=DEV), torch.ones(vdim, device=DEV)
+    before = _state(g, 1, ops.delta_state_shape(heads, dim, vdim), dim)
+    cu, slots = _boundaries([tokens]), torch.zeros(1, dtype=torch.int32, device=DEV)
+    out, left = _exact_delta(qkv, proj, a_log, dt_bias, before, cu, heads, kv_heads, dim, vdim)
+    for rows in (qkv, far):
+        state = before.clone()
+        got = ops.gated_delta(rows, proj, 0, heads, 2 * heads, a_log, dt_bias, weight, state, cu, slots, heads=heads, kv_heads=kv_heads,
+                              dim=dim, vdim=vdim, eps=1e-6)
+        # as in the tests above: float32 states; read-outs rounded to bfloat16 once
+        assert _rel(state[:1], left) < 4e-7 and _rel(got, out) < 2.0 ** -8
