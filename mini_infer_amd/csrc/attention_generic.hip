@@ -426,7 +426,7 @@ static int attn_generic_launch(const void* q, int64_t q_row_stride, const void* 
   // Four waves a range in the 32-bit path where one wave a range is fewer than two waves a SIMD (decode; values of
   // up to 128 dims, which the merging's LDS holds).  One layer, 32 heads of 64 over 8 key/value heads, microseconds
   // before and now: 3 tokens of up to 600 positions 113 -> 17.4, a prompt of 509 tokens 247 -> 148 (the batched
-  // loads alone, one wave a range).
+  // loads alone, one wave a range; such prompts now take attention_prompt_f32.hip, 66).
   const bool four = sizeof(S) == 8 && v_dim <= 128 && (int64_t)grid.x * grid.y * grid.z < 2048;
 #define MI_ATTN_LAUNCH_WAVES(VPL, VEC, WAVES, LDS)                                                \
   attn_generic_kernel<T, VPL, VEC, WAVES><<<grid, WAVES * MI_WAVE, LDS, stream>>>(                \

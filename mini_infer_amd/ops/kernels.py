@@ -1165,6 +1165,22 @@ def paged_attention(
         return out
 
     assert chunk is None  # (a chunked mask on plain pages has gone to the general entry point above)
+    # float32 steps with many tokens a request: 16 rows a block on the matrix cores' 64-bit instruction.  (Below a block a CU
+    # keys have to be cut into ranges; a tile whose tokens are different requests' walks one's keys after another's.)
+    if (
+        q.dtype == torch.float32 and slopes is None and not force_plain and host_cu_seqlens_q is not None
+        and tokens >= 32 * num_requests and lib.mi_attn_prompt_f32_blocks(tokens, q_heads, kv_heads, head_dim, page_size) >= 256
+        and q.stride(0) % 4 == 0 and out.stride(0) % 4 == 0
+        and all(t.data_ptr() % 16 == 0 for t in (q, k_pages, v_pages, out))
+    ):
+        library.check(
+            lib.mi_attn_prompt_f32(
+                _ptr(q), q.stride(0), _ptr(k_pages), _ptr(v_pages), _ptr(block_table), block_table.shape[1], _ptr(token_request),
+                _ptr(positions), _ptr(out), out.stride(0), tokens, q_heads, kv_heads, head_dim, page_size, num_pages, float(scale),
+                int(window or 0), _stream(),
+            )
+        )
+        return out
     splits = attention_splits(tokens * kv_heads * math.ceil(group / 4), max_seq_len)
     part_acc, part_ml = partials(splits)
     library.check(

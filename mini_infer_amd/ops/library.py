@@ -60,6 +60,10 @@ _SIGNATURES: dict[str, list] = {
         c_int, _P, c_int64, _P, _P, _P, c_int, _P, _P, _P, c_int64, _P, _P, c_int, c_int, c_int,
         c_int, c_int, c_int, c_float, c_int, c_int, _P, _P,
     ],
+    "mi_attn_prompt_f32_blocks": [c_int, c_int, c_int, c_int, c_int],
+    "mi_attn_prompt_f32": [
+        _P, c_int64, _P, _P, _P, c_int, _P, _P, _P, c_int64, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_int, _P,
+    ],
     "mi_attn_mfma": [
         _P, c_int64, _P, _P, _P, c_int, _P, _P, c_int, c_int, c_int, _P, c_int64, _P, _P, c_int,
         c_int, c_int, c_int, c_int, c_float, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_int, _P, _P, c_float, c_int, _P,
@@ -170,7 +174,7 @@ _SIGNATURES: dict[str, list] = {
 }
 
 
-_INT64_RESULTS = {"mi_gated_delta_chunks_scratch", "mi_decay_scan_chunks_scratch"}  # (sizes; every other entry point returns an int status)
+_INT64_RESULTS = {"mi_gated_delta_chunks_scratch", "mi_decay_scan_chunks_scratch", "mi_attn_prompt_f32_blocks"}  # (sizes; every other entry point returns an int status)
 
 
 def _declare(lib: ctypes.CDLL) -> None:

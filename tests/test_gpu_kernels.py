@@ -1089,3 +1089,43 @@ def test_latent_keys_and_values_of_a_step_in_pages(heads, dim, rot, vdim, v_widt
         assert ((got_k[:n] - want_k[t : t + n]).abs() <= 2.0 ** -8 * want_k[t : t + n].abs() + 1e-6).all() and (got_k[n:] == 0).all()
         assert torch.equal(got_v[:n, :, :vdim], v_up[t : t + n].view(n, heads, vdim))
         assert (got_v[n:] == 0).all() and (got_v[:, :, vdim:] == 0).all()
+
+
+@pytest.mark.parametrize("q_heads,kv_heads,dim,page,window,lengths,contexts", [
+    (32, 8, 64, 16, None, [131], [0]), (24, 8, 128, 16, 37, [100, 66, 1, 33], [0, 50, 200, 7]), (40, 2, 64, 32, None, [130, 61], [3, 0]),
+    (16, 16, 64, 16, 1, [300], [70]), (32, 2, 64, 48, 100, [257], [1000])])
+def test_prompt_attention_float32(q_heads, kv_heads, dim, page, window, lengths, contexts):
+    """Row tiles across requests, groups that leave rows idle or need several blocks, windows, keys past the last one that are
+    no numbers; against the plain kernel."""
+    from mini_infer_amd import ops
+    from mini_infer_amd.ops import library
+
+    tokens = sum(lengths)
+    assert library.load().mi_attn_prompt_f32_blocks(tokens, q_heads, kv_heads, dim, page) >= 256 and tokens >= 32 * len(lengths)
+    pages_of = [-(-(n + c) // page) for n, c in zip(lengths, contexts)]
+    order = torch.randperm(sum(pages_of), generator=torch.Generator().manual_seed(1)).int()
+    table = torch.zeros(len(lengths), max(pages_of), dtype=torch.int32)
+    at = 0
+    k_pages, v_pages = (_rand(sum(pages_of), kv_heads, page, dim, seed=s) for s in (2, 3))
+    for b, count in enumerate(pages_of):
+        table[b, :count] = order[at : at + count]
+        at += count
+        past = lengths[b] + contexts[b] - (count - 1) * page
+        for pages in (k_pages, v_pages):
+            pages[int(table[b, count - 1]), :, past:] = float("nan")
+    last = int(table[-1, (lengths[-1] + contexts[-1] - 1) // page]), (lengths[-1] + contexts[-1] - 1) % page
+    v_pages[last[0], :, last[1]] = float("inf")  # the last token's own value: the tokens before it do not see it
+    ints = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)
+    requests = ints([b for b, n in enumerate(lengths) for _ in range(n)])
+    positions = ints([c + i for n, c in zip(lengths, contexts) for i in range(n)])
+    cu = [0, *torch.tensor(lengths).cumsum(0).tolist()]
+    q = _rand(tokens, q_heads * dim + 4, seed=4)
+    got, plain = (
+        ops.paged_attention(q, k_pages, v_pages, table.to(DEV), requests, positions, ints(cu), cu, q_heads=q_heads, kv_heads=kv_heads,
+                            head_dim=dim, scale=dim ** -0.5, window=window, max_seq_len=max(n + c for n, c in zip(lengths, contexts)),
+                            force_plain=plain)
+        for plain in (False, True))
+    assert torch.isinf(got[-1]).all() and torch.isinf(plain[-1]).all()
+    # both round a result once; the plain kernel also each weight (weights sum to one) and, with cut keys, each part
+    most = float(v_pages[torch.isfinite(v_pages)].abs().max())
+    assert (got[:-1] - plain[:-1]).abs().max() <= 4 * 2.0 ** -24 * most
