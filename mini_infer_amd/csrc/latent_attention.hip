@@ -150,6 +150,7 @@ __global__ __launch_bounds__(256) void latent_expand_pages_kernel(
       if (copies) *reinterpret_cast<Piece*>(q_to) = *reinterpret_cast<const Piece*>(q_from);
       continue;
     }
+    // (which of the two products is fused is said, so that both forms, and steps of any size, round alike)
     const T* shared = shared_key + t * shared_stride + (d - dim);
     const float *c = cos_t + t * half + (d - dim) / 2, *s = sin_t + t * half + (d - dim) / 2;
     if constexpr (EIGHTS) {
@@ -161,17 +162,17 @@ __global__ __launch_bounds__(256) void latent_expand_pages_kernel(
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const float q0 = to_f32(q.v[2 * j]), q1 = to_f32(q.v[2 * j + 1]), k0 = to_f32(r.v[2 * j]), k1 = to_f32(r.v[2 * j + 1]);
-        turned.v[2 * j] = from_f32<T>(q0 * cj[j] - q1 * sj[j]);
-        turned.v[2 * j + 1] = from_f32<T>(q1 * cj[j] + q0 * sj[j]);
-        k.v[2 * j] = from_f32<T>(k0 * cj[j] - k1 * sj[j]);
-        k.v[2 * j + 1] = from_f32<T>(k1 * cj[j] + k0 * sj[j]);
+        turned.v[2 * j] = from_f32<T>(fmaf(q0, cj[j], -(q1 * sj[j])));
+        turned.v[2 * j + 1] = from_f32<T>(fmaf(q1, cj[j], q0 * sj[j]));
+        k.v[2 * j] = from_f32<T>(fmaf(k0, cj[j], -(k1 * sj[j])));
+        k.v[2 * j + 1] = from_f32<T>(fmaf(k1, cj[j], k0 * sj[j]));
       }
       *reinterpret_cast<Piece*>(q_to) = turned;
     } else {
       const int odd = (d - dim) & 1;
       const float q0 = to_f32(q_from[-odd]), q1 = to_f32(q_from[1 - odd]), k0 = to_f32(shared[-odd]), k1 = to_f32(shared[1 - odd]);
-      q_to[0] = from_f32<T>(odd ? q1 * *c + q0 * *s : q0 * *c - q1 * *s);
-      k.v[0] = from_f32<T>(odd ? k1 * *c + k0 * *s : k0 * *c - k1 * *s);
+      q_to[0] = from_f32<T>(odd ? fmaf(q1, *c, q0 * *s) : fmaf(q0, *c, -(q1 * *s)));
+      k.v[0] = from_f32<T>(odd ? fmaf(k1, *c, k0 * *s) : fmaf(k0, *c, -(k1 * *s)));
     }
     *reinterpret_cast<Piece*>(k_at) = k;
   }
