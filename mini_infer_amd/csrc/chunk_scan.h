@@ -211,10 +211,10 @@ __global__ __launch_bounds__(256, MODE == DELTA || DT > 2 ? 1 : 2) void walk_ker
     } else {
       o.factor = p.made.factor[of * 2 * CHUNK + lane];
     }
-    // (of tokens past the last one the last one's)
+    // (of tokens past the last one the last one's; the rest of the request may be more rows than 32 bits reach over)
     const int t0 = first + n * CHUNK;
     const bf16_t* v = p.v + (int64_t)t0 * p.v_stride + p.v_col + (int64_t)head * p.vdim;
-    const uint32_t v_row = min(v_at, (uint32_t)(last - 1 - t0) * (uint32_t)p.v_stride);
+    const uint32_t v_row = min(v_at, (uint32_t)min(CHUNK - 1, last - 1 - t0) * (uint32_t)p.v_stride);
     o.v[0] = *reinterpret_cast<const uint16_t*>(v + (v_row + v_first));
     o.v[1] = *reinterpret_cast<const uint16_t*>(v + (v_row + v_second));
   };

@@ -178,3 +178,36 @@ def test_rows_too_far_apart_for_chunks_go_token_by_token():
                               dim=dim, vdim=vdim, eps=1e-6)
         # as in the tests above: float32 states; read-outs rounded to bfloat16 once
         assert _rel(state[:1], left) < 4e-7 and _rel(got, out) < 2.0 ** -8
+
+
+@pytest.mark.parametrize("kind", ["delta", "per_head", "per_channel"])
+def test_a_rest_of_more_values_than_32_bits_count(kind):
+    """520 value rows 2^23 apart: 519 of them are past 2^32 values.  The same bits as of rows side by side."""
+    from mini_infer_amd import ops
+
+    heads, groups, dim, vdim, tokens = 2, 1, 64, 64, 520
+    g = torch.Generator(device=DEV).manual_seed(13)
+    q, k, v = (torch.randn(tokens, n, generator=g, device=DEV).bfloat16() for n in (groups * dim, groups * dim, heads * vdim))
+    rows = torch.cat([q, k, v], 1) if kind == "delta" else v
+    far = torch.empty(tokens, 2**23, dtype=torch.bfloat16, device=DEV)[:, : rows.shape[1]]
+    far.copy_(rows)
+    cu, slots = _boundaries([tokens]), torch.zeros(1, dtype=torch.int32, device=DEV)
+    made = []
+    if kind == "delta":
+        proj = torch.randn(tokens, 2 * heads + heads * vdim, generator=g, device=DEV).bfloat16()
+        a_log, dt_bias, weight = torch.zeros(heads, device=DEV), torch.full((heads,), -2.0, device=DEV), torch.ones(vdim, device=DEV)
+        before = _state(g, 1, ops.delta_state_shape(heads, dim, vdim), dim)
+        for x in (rows, far):
+            state = before.clone()
+            made.append((ops.gated_delta(x, proj, 0, heads, 2 * heads, a_log, dt_bias, weight, state, cu, slots, heads=heads,
+                                         kv_heads=groups, dim=dim, vdim=vdim, eps=1e-6), state))
+    else:
+        per_head = kind == "per_head"
+        gates = heads if per_head else heads * dim
+        gate, bias = torch.randn(tokens, gates, generator=g, device=DEV).bfloat16(), torch.zeros(gates, device=DEV)
+        before = _state(g, 1, ops.decay_state_shape(heads, dim, vdim), dim)
+        for x in (rows, far):
+            state = before.clone()
+            made.append((ops.decay_scan(q, 0, k, 0, x, 0, gate, 0, bias, state, cu, slots, heads=heads, groups=groups, dim=dim, vdim=vdim,
+                                        per_head=per_head, rate=torch.zeros(heads, device=DEV) if per_head else None, inv_tau=0.0625), state))
+    assert torch.equal(made[0][0], made[1][0]) and torch.equal(made[0][1], made[1][1])
