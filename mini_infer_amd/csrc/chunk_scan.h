@@ -29,6 +29,13 @@
 // decay per head (64 heads of 128 x 64) 717 -> 117, decay per channel (16 heads of 128 x 256) 774 -> 144.  Waiting for
 // everything in flight at the barrier cost 2 us a chunk more.  A chunk of 32: at twice that W and T (quadratic) weigh as much
 // as the products with the state, and the inverse no longer stays in a wave's registers.
+//
+// Only finite numbers may be taken like this: the zeros of W and T above the diagonal make NaN of an infinite value, for
+// tokens before it, and quotients behind a decay of zero are infinity less infinity.  So each wave adds up zero times
+// (G_last / G) U, which is the same in all four and holds whatever was not finite in values, gates, and (for the delta rule by
+// itself, else through the factors) queries and keys; if that is not zero at the end the block leaves the state as it found it
+// and sets its flag, and a last launch takes the flagged columns again with the token-by-token kernel.  That launch costs 3 us
+// where nothing is flagged; a verdict at the end of a block that needed a barrier cost another 0.3 us a block.
 #pragma once
 #include "common.h"
 
@@ -47,7 +54,8 @@ struct Made {
   float* kt;      // [chunks][shares][pad][CHUNK]; PER_CHANNEL: times G_last / G_j
   float* within;  // W [chunks][heads][CHUNK][CHUNK]; PER_HEAD: for U = V, its columns times the step sizes
   float* solve;   // T w, the same (DELTA only)
-  float* factor;  // [chunks][heads][2][CHUNK]: G, and G_last / G (PER_HEAD: times the step sizes); not PER_CHANNEL
+  float* factor;  // [chunks][heads][2][CHUNK]: G, and G_last / G (PER_HEAD: times the step sizes); PER_CHANNEL [chunks][heads]: 0
+                  // (NaN: of a token, or PER_CHANNEL of a chunk, whose query, key or decay is not finite)
   float* fade;    // G_last: PER_CHANNEL [chunks][heads][pad]
   int shares;     // rows q and k are shared by heads / shares heads
 };
@@ -56,6 +64,7 @@ struct Made {
 // the chunks of request b from one request to the next.
 __device__ __forceinline__ int first_chunk(int cu_b, int b) { return cu_b / CHUNK + b; }
 static inline int64_t chunk_count(int tokens, int requests) { return (int64_t)tokens / CHUNK + requests; }
+static inline int64_t flag_count(int requests, int heads, int vdim) { return (int64_t)requests * heads * ceil_div(vdim, 16); }
 
 // Which request a chunk number belongs to: all threads of the block call this; -1: no request's.
 __device__ __forceinline__ int request_of_chunk(int chunk, const int* __restrict__ cu, int requests, int* shared_answer) {
@@ -106,6 +115,7 @@ struct WalkArgs {
   const int *cu, *slots;
   int num_slots;
   float* out;  // float32 [tokens, heads * vdim]
+  int* again;  // [requests][heads][column blocks of 16]: 1 where the columns are to be taken token by token
   int heads, vdim;
 };
 constexpr int64_t MAX_ROW = 1 << 24;
@@ -134,7 +144,7 @@ struct Operands {
   float4 q[2][DT], k[MODE == DELTA ? 2 : 1][DT], kt[2][DT];
   float4 fade[MODE == PER_CHANNEL ? DT : 1];
   float4 within, solve;  // four values of a row of W and of T
-  float factor;          // one of the 64 factors
+  float factor;          // one of the 64 factors; PER_CHANNEL: the chunk's only one
   uint32_t v[2];         // two columns of a token's values, as read
 };
 
@@ -164,7 +174,11 @@ __global__ __launch_bounds__(256, MODE == DELTA || DT > 2 ? 1 : 2) void walk_ker
   const int col = blockIdx.x / p.heads * 16 + r;
   const bool live = col < p.vdim;
   const int first = p.cu[b], last = p.cu[b + 1];
-  if (last <= first) return;
+  int* flag = p.again + ((int64_t)b * p.heads + head) * ((p.vdim + 15) / 16) + blockIdx.x / p.heads;
+  if (last <= first) {
+    if (threadIdx.x == 0) *flag = 0;
+    return;
+  }
   const int slot = p.slots[b];
   const int row0 = 16 * DT * wave;  // of S
   float* mine = p.state + (int64_t)((slot < 0 || slot >= p.num_slots) ? p.num_slots : slot) * p.state_stride +
@@ -175,6 +189,7 @@ __global__ __launch_bounds__(256, MODE == DELTA || DT > 2 ? 1 : 2) void walk_ker
   const int share = head / (p.heads / p.made.shares);
   const int chunk0 = first_chunk(first, b), chunks = (last - first + CHUNK - 1) / CHUNK;
   const float skip = (MODE == PER_HEAD && p.skip) ? p.skip[head] : 0.f;
+  float zeros[2] = {0.f, 0.f};  // unless something is not finite
   const int out_stride = p.heads * p.vdim;
   // a lane's offsets
   const uint32_t at_row = r * PAD + 4 * quad, at_column = r * CHUNK + 4 * quad, in_lds = r * LDS_ROW + 4 * quad;
@@ -208,6 +223,7 @@ __global__ __launch_bounds__(256, MODE == DELTA || DT > 2 ? 1 : 2) void walk_ker
       const float* fade = p.made.fade + of * PAD + row0;
 #pragma unroll
       for (int d = 0; d < DT; ++d) o.fade[d] = load4(fade + 16 * d + 4 * quad);
+      o.factor = p.made.factor[of];
     } else {
       o.factor = p.made.factor[of * 2 * CHUNK + lane];
     }
@@ -240,6 +256,8 @@ __global__ __launch_bounds__(256, MODE == DELTA || DT > 2 ? 1 : 2) void walk_ker
     if constexpr (MODE == DELTA) *reinterpret_cast<float4*>(&both.solve[piece]) = o.solve;
     if constexpr (MODE != PER_CHANNEL) {
       if (wave == 0) both.factor[lane] = o.factor;
+    } else if (threadIdx.x == 0) {
+      both.factor[0] = o.factor;
     }
     {  // (of tokens past the last one zeros, by their bits: a choice would be compiled into a branch around the load, and every
        // load waited for by itself)
@@ -261,6 +279,7 @@ __global__ __launch_bounds__(256, MODE == DELTA || DT > 2 ? 1 : 2) void walk_ker
       }
       g_last = both.factor[CHUNK - 1];
     }
+    if constexpr (MODE == PER_CHANNEL) zeros[0] += both.factor[0];
     auto whole = [&](int t) {
       return (parts[n & 1][0][t][lane] + parts[n & 1][1][t][lane]) + (parts[n & 1][2][t][lane] + parts[n & 1][3][t][lane]);
     };
@@ -277,6 +296,8 @@ __global__ __launch_bounds__(256, MODE == DELTA || DT > 2 ? 1 : 2) void walk_ker
     for (int t = 0; t < 2; ++t) {
       if constexpr (MODE == PER_CHANNEL) tail[t] = u[t];
       else tail[t] = scaled(tails[t], u[t]);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) zeros[t] = fmaf(0.f, tail[t][e], zeros[t]);
     }
 #pragma unroll
     for (int d = 0; d < DT; ++d) {
@@ -310,7 +331,9 @@ __global__ __launch_bounds__(256, MODE == DELTA || DT > 2 ? 1 : 2) void walk_ker
     step(n + 1, odd);
   }
   if (chunks & 1) step(chunks - 1, even);
-  if (live) {
+  const bool again = __ballot(!(zeros[0] + zeros[1] == 0.f)) != 0;  // (the same in all waves: so are all that zeros were made of)
+  if (threadIdx.x == 0) *flag = again;
+  if (live && !again) {
 #pragma unroll
     for (int d = 0; d < DT; ++d) *reinterpret_cast<f32x4_t*>(mine + 16 * d) = S[d];
   }

@@ -216,5 +216,22 @@ __device__ __forceinline__ void mi_write_page_rows(T* v_pages, int t, int page, 
   }
 }
 
+// Blocks of a launch that looks for flagged work and usually finds none.
+constexpr int AGAIN_BLOCKS = 512;
+
+// Calls take(i) for every i < total with flagged(i), an item a block at a time; all 256 threads of the block call this.
+template <typename F, typename G>
+__device__ __forceinline__ void mi_take_flagged(int64_t total, F flagged, G take) {
+  for (int64_t base = blockIdx.x; base < total; base += (int64_t)256 * gridDim.x) {
+    const int64_t mine = base + (int64_t)threadIdx.x * gridDim.x;
+    if (!__syncthreads_or(mine < total && flagged(mine))) continue;
+    for (int64_t i = base; i < min(total, base + (int64_t)256 * gridDim.x); i += gridDim.x) {
+      if (!flagged(i)) continue;
+      take(i);
+      __syncthreads();
+    }
+  }
+}
+
 static __host__ __device__ inline int ceil_div(int a, int b) { return (a + b - 1) / b; }
 static inline int64_t ceil_div64(int64_t a, int64_t b) { return (a + b - 1) / b; }

@@ -25,6 +25,7 @@ template <int DT>
 __global__ __launch_bounds__(256) void head_decay_chunk_kernel(RowArgs p, Made made) {
   constexpr int PAD = 64 * DT, ROW = PAD + 4, EACH = PAD / 8, INNER = CHUNK * (CHUNK + 4);
   __shared__ __align__(16) float q_s[CHUNK * ROW], k_s[CHUNK * ROW], qk_s[INNER];
+  __shared__ float zeros_s[CHUNK];
   __shared__ int which;
   const int chunk = blockIdx.x, share = blockIdx.y;
   const int b = request_of_chunk(chunk, p.cu, p.requests, &which);
@@ -39,6 +40,12 @@ __global__ __launch_bounds__(256) void head_decay_chunk_kernel(RowArgs p, Made m
     float qv[EACH], kv[EACH];
     row_values(q, sub * EACH, p.dim, p.eights, token < nt, qv);
     row_values(k, sub * EACH, p.dim, p.eights, token < nt, kv);
+    float zeros = 0.f;  // unless something is not finite
+#pragma unroll
+    for (int e = 0; e < EACH; ++e) zeros = fmaf(0.f, kv[e], fmaf(0.f, qv[e], zeros));
+#pragma unroll
+    for (int off = 1; off < 8; off <<= 1) zeros += __shfl_xor(zeros, off, MI_WAVE);
+    if (sub == 0) zeros_s[token] = zeros;
 #pragma unroll
     for (int e = 0; e < EACH; e += 4) {
       const float4 q4 = make_float4(qv[e] * p.q_scale, qv[e + 1] * p.q_scale, qv[e + 2] * p.q_scale, qv[e + 3] * p.q_scale);
@@ -81,7 +88,7 @@ __global__ __launch_bounds__(256) void head_decay_chunk_kernel(RowArgs p, Made m
     if (lane < CHUNK) {
       float* factor = made.factor + of * 2 * CHUNK + lane;
       factor[0] = __builtin_amdgcn_exp2f((float)sum);
-      factor[CHUNK] = __builtin_amdgcn_exp2f((float)(__shfl(sum, CHUNK - 1, CHUNK) - sum)) * dt;
+      factor[CHUNK] = __builtin_amdgcn_exp2f((float)(__shfl(sum, CHUNK - 1, CHUNK) - sum)) * dt + zeros_s[lane];
     }
     float* within = made.within + of * CHUNK * CHUNK + i0;
 #pragma unroll
@@ -112,6 +119,7 @@ __global__ __launch_bounds__(256) void channel_decay_chunk_kernel(RowArgs p, Mad
   if (b < 0) return;
   const int t0 = p.cu[b] + (chunk - first_chunk(p.cu[b], b)) * CHUNK, nt = min(CHUNK, p.cu[b + 1] - t0);
   const int tid = threadIdx.x, share = head / (p.heads / p.groups);
+  int odd = 0;
   {
     const int token = tid / 8, sub = tid % 8;
     const int64_t row = t0 + min(token, nt - 1);
@@ -122,16 +130,20 @@ __global__ __launch_bounds__(256) void channel_decay_chunk_kernel(RowArgs p, Mad
     row_values(k, sub * EACH, p.dim, p.eights, token < nt, kv);
     row_values(gate, sub * EACH, p.dim, p.eights, token < nt, av);
     const float* bias = p.gate_bias + (int64_t)head * p.dim;
+    float zeros = 0.f;
 #pragma unroll
     for (int e = 0; e < EACH; ++e) {
       const int d = sub * EACH + e;
       const float a = mi_channel_decay(av[e] + bias[min(d, p.dim - 1)], p.inv_tau);
       q_s[token * ROW + d] = qv[e] * p.q_scale;
       k_s[token * ROW + d] = kv[e];
+      zeros = fmaf(0.f, qv[e], zeros) + 0.f * kv[e] + 0.f * a;
       a_s[token * ROW + d] = token < nt && d < p.dim ? a : 1.f;
     }
+    odd = !(zeros == 0.f);
   }
-  __syncthreads();
+  odd = __syncthreads_or(odd);
+  if (tid == 0) made.factor[(int64_t)chunk * p.heads + head] = odd ? NAN : 0.f;
   for (int d = tid; d < PAD; d += 256) {
     const int64_t of = (int64_t)chunk * made.shares + head;  // (rows of a head of its own)
     double product = 1.0, tail = 1.0;  // (rounded once, where they are used)
@@ -187,11 +199,12 @@ int made_shares(int mode, int heads, int groups) { return mode == PER_CHANNEL ? 
 }  // namespace
 
 // Floats of scratch that mi_decay_scan_chunks takes; 0: sizes it does not take.
-extern "C" int64_t mi_decay_scan_chunks_scratch(int mode, int num_tokens, int num_requests, int heads, int groups, int dim) {
+extern "C" int64_t mi_decay_scan_chunks_scratch(int mode, int num_tokens, int num_requests, int heads, int groups, int dim, int vdim) {
   const int pad = mi_decay_scan_dim_pad(dim);
-  if (num_tokens <= 0 || num_requests <= 0 || num_requests > 65535 || dim > 256 || pad < 64 || heads <= 0 || heads > 65535 || groups <= 0) return 0;
+  if (num_tokens <= 0 || num_requests <= 0 || num_requests > 65535 || dim > 256 || pad < 64 || heads <= 0 || heads > 65535 || groups <= 0 || vdim <= 0) return 0;
   return chunk_count(num_tokens, num_requests) * ((int64_t)2 * made_shares(mode, heads, groups) * CHUNK * pad +
-                                                  (int64_t)heads * (CHUNK * CHUNK + (mode == PER_CHANNEL ? pad : 2 * CHUNK)));
+                                                  (int64_t)heads * (CHUNK * CHUNK + (mode == PER_CHANNEL ? pad + 1 : 2 * CHUNK))) +
+         flag_count(num_requests, heads, vdim);
 }
 
 // As mi_decay_scan for bfloat16, with `scratch` on 16 bytes.
@@ -205,15 +218,17 @@ extern "C" int mi_decay_scan_chunks(int mode, const void* q, int64_t q_stride, i
                                       rate, state, state_stride, num_slots, num_tokens, num_requests, heads, groups, dim, vdim);
   if (bad != MI_OK) return bad;
   if (num_tokens == 0 || num_requests == 0) return MI_OK;
-  MI_REQUIRE(mi_decay_scan_chunks_scratch(mode, num_tokens, num_requests, heads, groups, dim) > 0, "decay_scan_chunks: sizes it does not take");
+  MI_REQUIRE(mi_decay_scan_chunks_scratch(mode, num_tokens, num_requests, heads, groups, dim, vdim) > 0, "decay_scan_chunks: sizes it does not take");
   MI_REQUIRE(scratch != nullptr && (uintptr_t)scratch % 16 == 0, "decay_scan_chunks: no scratch");
   const int pad = mi_decay_scan_dim_pad(dim);
   const int64_t chunks = chunk_count(num_tokens, num_requests), rows = chunks * made_shares(mode, heads, groups) * CHUNK * pad;
   MI_REQUIRE(chunks <= 2147483647 && v_stride < MAX_ROW && (int64_t)heads * vdim < MAX_ROW, "decay_scan_chunks: sizes it does not take");
   Made made;
   made.q = scratch, made.kt = made.q + rows, made.within = made.kt + rows;
-  made.factor = made.fade = made.within + chunks * heads * CHUNK * CHUNK;
+  made.fade = made.within + chunks * heads * CHUNK * CHUNK;
+  made.factor = made.fade + (mode == PER_CHANNEL ? chunks * heads * pad : 0);
   made.k = made.solve = nullptr;
+  int* again = reinterpret_cast<int*>(made.factor + chunks * heads * (mode == PER_CHANNEL ? 1 : 2 * CHUNK));
   made.shares = made_shares(mode, heads, groups);
   RowArgs a;
   a.q = (const bf16_t*)q, a.k = (const bf16_t*)k, a.gate = (const bf16_t*)gate;
@@ -243,7 +258,10 @@ extern "C" int mi_decay_scan_chunks(int mode, const void* q, int64_t q_stride, i
   p.made = made;
   p.v = (const bf16_t*)v, p.v_stride = v_stride, p.v_col = v_col, p.skip = skip;
   p.state = state, p.state_stride = state_stride, p.cu = cu, p.slots = slots, p.num_slots = num_slots;
-  p.out = out, p.heads = heads, p.vdim = vdim;
-  return mode == PER_CHANNEL ? launch_walk<PER_CHANNEL>(p, pad, num_requests, stream)
-                             : launch_walk<PER_HEAD>(p, pad, num_requests, stream);
+  p.out = out, p.again = again, p.heads = heads, p.vdim = vdim;
+  const int walked = mode == PER_CHANNEL ? launch_walk<PER_CHANNEL>(p, pad, num_requests, stream) : launch_walk<PER_HEAD>(p, pad, num_requests, stream);
+  if (walked != MI_OK) return walked;
+  return mi_decay_scan_again(mode, q, q_stride, q_col, k, k_stride, k_col, v, v_stride, v_col, gate, gate_stride, gate_col, gate_bias, rate,
+                             skip, inv_tau, q_scale, state, state_stride, cu, slots, num_slots, out, again, num_requests, heads, groups, dim,
+                             vdim, stream);
 }

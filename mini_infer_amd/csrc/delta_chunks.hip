@@ -140,9 +140,10 @@ __global__ __launch_bounds__(256) void delta_chunk_kernel(const bf16_t* __restri
 
 // Floats of scratch that mi_gated_delta_chunks takes; 0: sizes it does not take.
 extern "C" int64_t mi_gated_delta_chunks_scratch(int num_tokens, int num_requests, int heads, int kv_heads, int dim, int vdim) {
-  if (num_tokens <= 0 || num_requests <= 0 || dim > 256 || vdim > 256 || heads <= 0 || kv_heads <= 0 || kv_heads > 65535) return 0;
+  if (num_tokens <= 0 || num_requests <= 0 || dim > 256 || vdim > 256 || vdim <= 0 || heads <= 0 || kv_heads <= 0 || kv_heads > 65535) return 0;
   const int pad = mi_gated_delta_rows(dim, vdim);
-  return chunk_count(num_tokens, num_requests) * ((int64_t)3 * kv_heads * CHUNK * pad + (int64_t)heads * (2 * CHUNK * CHUNK + 2 * CHUNK));
+  return chunk_count(num_tokens, num_requests) * ((int64_t)3 * kv_heads * CHUNK * pad + (int64_t)heads * (2 * CHUNK * CHUNK + 2 * CHUNK)) +
+         flag_count(num_requests, heads, vdim);
 }
 
 // As mi_gated_delta for bfloat16, with `scratch` on 16 bytes.
@@ -164,6 +165,7 @@ extern "C" int mi_gated_delta_chunks(const void* qkv, int64_t qkv_stride, const 
   made.within = made.kt + rows, made.solve = made.within + chunks * heads * CHUNK * CHUNK;
   made.factor = made.solve + chunks * heads * CHUNK * CHUNK;
   made.fade = nullptr;
+  int* again = reinterpret_cast<int*>(made.factor + chunks * heads * 2 * CHUNK);
   made.shares = kv_heads;
   dim3 grid((unsigned)chunks, kv_heads);
 #define MI_DELTA_CHUNKS(DT)                                                                                              \
@@ -180,8 +182,11 @@ extern "C" int mi_gated_delta_chunks(const void* qkv, int64_t qkv_stride, const 
   p.v = (const bf16_t*)qkv, p.v_stride = qkv_stride, p.v_col = 2 * kv_heads * dim;
   p.skip = nullptr;
   p.state = state, p.state_stride = state_stride, p.cu = cu, p.slots = slots, p.num_slots = num_slots;
-  p.out = readout, p.heads = heads, p.vdim = vdim;
+  p.out = readout, p.again = again, p.heads = heads, p.vdim = vdim;
   const int walked = launch_walk<DELTA>(p, dim_pad, num_requests, stream);
   if (walked != MI_OK) return walked;
+  const int redone = mi_delta_again(qkv, qkv_stride, proj, proj_stride, col_b, col_a, a_log, dt_bias, state, state_stride, cu, slots, readout,
+                                    again, num_requests, heads, kv_heads, dim, vdim, num_slots, stream);
+  if (redone != MI_OK) return redone;
   return mi_delta_readout_norm(MI_BF16, readout, proj, proj_stride, col_g, norm_weight, out, out_stride, num_tokens, heads, vdim, eps, stream);
 }

@@ -2428,7 +2428,7 @@ def decay_scan(
     out = torch.empty((tokens, heads * vdim), dtype=torch.float32, device=q.device)
     lib = library.load()
     if q.dtype == torch.bfloat16 and chunked_scan_pays(tokens, requests, max(v.stride(0), heads * vdim)):
-        floats = lib.mi_decay_scan_chunks_scratch(int(per_head), tokens, requests, heads, groups, dim)
+        floats = lib.mi_decay_scan_chunks_scratch(int(per_head), tokens, requests, heads, groups, dim, vdim)
         if floats > 0:
             scratch = torch.empty(floats, dtype=torch.float32, device=q.device)
             library.check(

@@ -124,7 +124,7 @@ _SIGNATURES: dict[str, list] = {
         c_int, _P, c_int64, c_int, _P, c_int64, c_int, _P, c_int64, c_int, _P, c_int64, c_int, _P, _P, _P, c_float,
         c_float, _P, c_int64, _P, _P, c_int, _P, _P, c_int, c_int, c_int, c_int, c_int, c_int, _P,
     ],
-    "mi_decay_scan_chunks_scratch": [c_int, c_int, c_int, c_int, c_int, c_int],
+    "mi_decay_scan_chunks_scratch": [c_int, c_int, c_int, c_int, c_int, c_int, c_int],
     "mi_decay_scan_dim_pad": [c_int],
     "mi_decay_scan": [
         c_int, c_int, _P, c_int64, c_int, _P, c_int64, c_int, _P, c_int64, c_int, _P, c_int64, c_int, _P, _P, _P, c_float,

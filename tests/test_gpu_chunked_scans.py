@@ -211,3 +211,45 @@ def test_a_rest_of_more_values_than_32_bits_count(kind):
             made.append((ops.decay_scan(q, 0, k, 0, x, 0, gate, 0, bias, state, cu, slots, heads=heads, groups=groups, dim=dim, vdim=vdim,
                                         per_head=per_head, rate=torch.zeros(heads, device=DEV) if per_head else None, inv_tau=0.0625), state))
     assert torch.equal(made[0][0], made[1][0]) and torch.equal(made[0][1], made[1][1])
+
+
+@pytest.mark.parametrize("dim,vdim", [(40, 64), (128, 128), (256, 250)])
+@pytest.mark.parametrize("what", ["value inf", "value nan", "k inf", "q inf", "state inf", "gate inf", "gate -inf", "gate nan"])
+@pytest.mark.parametrize("kind", ["delta", "per_head", "per_channel"])
+def test_what_is_not_finite_goes_token_by_token(monkeypatch, kind, what, dim, vdim):
+    """A value, key, query, state or gate in the middle of a chunk that is no finite number reaches what it reaches in the
+    token-by-token kernels: earlier tokens, other heads, other columns and other requests keep their numbers."""
+    from mini_infer_amd import ops
+
+    heads, groups, lengths, at, column = 4, 2, [50, 70], 50 + 32 + 9, 21
+    tokens, requests = sum(lengths), len(lengths)
+    g = torch.Generator(device=DEV).manual_seed(17)
+    q, k, v = (torch.randn(tokens, n, generator=g, device=DEV).bfloat16() for n in (groups * dim, groups * dim, heads * vdim))
+    per_channel = heads * dim if kind == "per_channel" else heads
+    gate = torch.randn(tokens, per_channel, generator=g, device=DEV).bfloat16()
+    shape = ops.delta_state_shape(heads, dim, vdim) if kind == "delta" else ops.decay_state_shape(heads, dim, vdim)
+    state = _state(g, requests, shape, dim)
+    name, bad = what.split()
+    if name == "state":
+        state[1, 1, column, 3] = float(bad)
+    else:
+        rows = {"value": (v, vdim + column), "k": (k, 7), "q": (q, 7), "gate": (gate, per_channel // heads)}[name]
+        rows[0][at, rows[1]] = float(bad)
+    cu, slots = _boundaries(lengths), torch.arange(requests, dtype=torch.int32, device=DEV)
+    if kind == "delta":
+        qkv = torch.cat([q, k, v], 1)
+        proj = torch.cat([torch.randn(tokens, heads, generator=g, device=DEV).bfloat16(), gate, torch.randn(tokens, heads * vdim, generator=g, device=DEV).bfloat16()], 1)
+        a_log, dt_bias, weight = torch.zeros(heads, device=DEV), torch.full((heads,), -2.0, device=DEV), torch.ones(vdim, device=DEV)
+        call = lambda s: ops.gated_delta(qkv, proj, 0, heads, 2 * heads, a_log, dt_bias, weight, s, cu, slots, heads=heads, kv_heads=groups, dim=dim, vdim=vdim, eps=1e-6)  # noqa: E731
+    else:
+        per_head = kind == "per_head"
+        bias, rate = torch.zeros(per_channel, device=DEV), torch.zeros(heads, device=DEV) if per_head else None
+        call = lambda s: ops.decay_scan(q, 0, k, 0, v, 0, gate, 0, bias, s, cu, slots, heads=heads, groups=groups, dim=dim, vdim=vdim, per_head=per_head, rate=rate, inv_tau=0.0625)  # noqa: E731
+    (out, left), (out_walked, left_walked) = _both(monkeypatch, call, state)
+    out, out_walked = out.double(), out_walked.double()
+    for got, walked in ((out, out_walked), (left.double(), left_walked.double())):
+        assert torch.equal(got.isnan(), walked.isnan()) and torch.equal(got.isinf(), walked.isinf()) and torch.equal(got[got.isinf()], walked[walked.isinf()])
+        finite = walked.isfinite()
+        # (bounds of the tests above: twice the error of one side against 64 bits)
+        assert float((got - walked)[finite].norm() / walked[finite].norm()) < (2.0 ** -7 if kind == "delta" and got is out else 8e-7)
+    assert out[: 50 if name == "state" else at].isfinite().all()
