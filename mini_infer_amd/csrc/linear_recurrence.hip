@@ -104,7 +104,7 @@ __device__ __forceinline__ double lanes_sum(double v) {
 // step sizes in LDS, and the walk reads LDS only, each token's operands one token ahead.  In LDS
 // a lane's run of R entries is followed by four unused ones where runs of 32 or 64 bytes would
 // otherwise meet 2 or 4 to a bank in a 16-byte read of all lanes.
-template <typename T, int MODE, int R, int L>
+template <typename T, int MODE, int R, int L, bool AGAIN>
 __device__ __forceinline__ void decay_scan_columns(const ScanArgs& p, int b, int head, int col0) {
   using A = typename Wide<T>::type;
   constexpr bool WIDE = sizeof(T) == 4;
@@ -128,7 +128,7 @@ __device__ __forceinline__ void decay_scan_columns(const ScanArgs& p, int b, int
   const int first = p.cu[b], last = p.cu[b + 1];
   if (last <= first) return;
   // (of columns taken again the flagged ones: the others' states have been advanced)
-  if (p.again != nullptr) live = live && p.again[((int64_t)b * p.heads + head) * ((p.vdim + 15) / 16) + min(col, p.vdim - 1) / 16] != 0;
+  if constexpr (AGAIN) live = live && p.again[((int64_t)b * p.heads + head) * ((p.vdim + 15) / 16) + min(col, p.vdim - 1) / 16] != 0;
   const int slot = p.slots[b];
   float* mine = p.state + (int64_t)((slot < 0 || slot >= p.num_slots) ? p.num_slots : slot) * p.state_stride +
                 ((int64_t)head * p.vdim + (live ? col : 0)) * DP + part * R;
@@ -281,7 +281,7 @@ __device__ __forceinline__ void decay_scan_columns(const ScanArgs& p, int b, int
 
 template <typename T, int MODE, int R, int L>
 __global__ __launch_bounds__(256) void decay_scan_kernel(ScanArgs p) {
-  decay_scan_columns<T, MODE, R, L>(p, blockIdx.x, blockIdx.y, blockIdx.z * (256 / L));
+  decay_scan_columns<T, MODE, R, L, false>(p, blockIdx.x, blockIdx.y, blockIdx.z * (256 / L));
 }
 
 // the same for columns that the chunks' walk has flagged
@@ -297,7 +297,7 @@ __global__ __launch_bounds__(256) void decay_scan_again_kernel(ScanArgs p, int r
         for (int f = i % blocks * (COLS / 16); f < min((int)(i % blocks + 1) * (COLS / 16), flags); ++f) any = any || of[f] != 0;
         return any;
       },
-      [&](int64_t i) { decay_scan_columns<bf16_t, MODE, R, L>(p, i / blocks / p.heads, i / blocks % p.heads, i % blocks * COLS); });
+      [&](int64_t i) { decay_scan_columns<bf16_t, MODE, R, L, true>(p, i / blocks / p.heads, i / blocks % p.heads, i % blocks * COLS); });
 }
 
 // rows per lane and lanes per column for a head whose keys are `dim` wide

@@ -1970,28 +1970,61 @@ def delta_state_shape(heads: int, dim: int, vdim: int) -> tuple[int, int, int]:
     return (heads, vdim, 64 if dim <= 64 else (128 if dim <= 128 else 256))
 
 
-def chunked_scan_pays(tokens: int, requests: int, widest: int) -> bool:
-    """Whether a recurrence over a step's rows is taken 32 tokens at a time on the matrix cores rather than token by token.
-    Token by token a step takes about as long as its longest portion (0.3 to 0.45 microseconds a token at heads of 128 x 128);
-    a chunk takes 1.6 to 2.3 microseconds, but a request with a single token costs as much as one with 32.  Measured, token by
-    token against in chunks, microseconds: delta rule, 32 heads of 128 x 128: 2,048 tokens 894 / 184, 512 tokens 230 / 63, a
-    portion of 256 beside 15 single tokens 133 / 88, 4 portions of 16 32 / 35, 30 single tokens 42 / 91; a decay per head, 64
-    heads of 128 x 64: 2,048 tokens 717 / 117; 48 heads: 64 tokens 23.6 / 26.4, 256 beside 15 single tokens 302 / 48; a decay
-    per channel, 16 heads of 128 x 256: 2,048 tokens 774 / 144.  `widest`: values from one row to the next of the widest operand
+# Microseconds of a recurrence over a step's rows with keys of up to so many columns: token by token (the launches, a request and a
+# token on a full chip, a token of the longest portion) and in chunks of 32 (the launches, a request on a full chip, a chunk of the
+# longest portion).  Fitted to 1,508 measured pairs: 1 to 100 requests of 8 to 512 tokens, single tokens beside one portion, 4 to 80
+# heads of 64 to 512 columns; half of the times are within 5 %.
+_SCAN_TIMES = {
+    ("delta", 64): (6.95, 0.89, 0.093, 0.288, 18.3, 2.33, 1.82),
+    ("delta", 128): (8.39, 2.13, 0.161, 0.428, 21, 3.14, 2.26),
+    ("delta", 256): (7.82, 3.4, 0.288, 0.62, 24.7, 7.38, 4.32),
+    ("per_head", 64): (3.85, 0.356, 0.0355, 0.252, 13.4, 0.971, 1.13),
+    ("per_head", 128): (3.43, 0.851, 0.0864, 0.303, 14, 1.68, 1.52),
+    ("per_head", 256): (2.44, 2.06, 0.19, 0.472, 16.4, 3.59, 2.36),
+    ("per_channel", 64): (3.98, 0.361, 0.0473, 0.267, 17.5, 1.57, 1.05),
+    ("per_channel", 128): (3.28, 1.18, 0.121, 0.348, 23.4, 2.35, 1.71),
+    ("per_channel", 256): (1.11, 3.09, 0.256, 0.58, 31.6, 5.51, 3.08),
+}
+
+
+def scan_times(kind: str, tokens: int, requests: int, longest: int | None, heads: int, dim: int, vdim: int) -> tuple[float, float]:
+    """About how many microseconds a recurrence takes token by token and in chunks.  A long portion is a chain of tokens (0.3 to 0.45
+    microseconds each at keys of 128) or of chunks (1.5 to 2.3), but a chunk costs the same with one token in it.  `longest`: tokens
+    of the step's longest portion; None (a recorded step): as if it were one portion beside single tokens, a scheduler's ordinary step."""
+    launches, request, token, chain, chunk_launches, chunk_request, chunk_chain = _SCAN_TIMES[kind, 64 if dim <= 64 else 128 if dim <= 128 else 256]
+    longest = max(1, tokens - requests + 1) if longest is None else longest
+    full = heads * -(-vdim // 16) / 256  # of the chip, by one request
+    if kind != "delta" and requests % 8 == 0 and longest * requests >= 2 * tokens:
+        # (that kernel's blocks go round the requests first, so of 8, 16, .. requests one has all its blocks on one of the 8 XCDs: 256
+        # tokens of 48 heads of 128 x 64 beside 15 single tokens take 288 microseconds, beside 14 or 16 of them 95)
+        chain *= max(1.0, 4 * full)
+    walked = launches + request * requests * full + max(token * tokens * full, chain * longest)
+    return walked, chunk_launches + chunk_request * requests * full + chunk_chain * longest / 32
+
+
+def chunked_scan_pays(walked: float, chunked: float, widest: int) -> bool:
+    """Whether a recurrence over a step's rows is taken 32 tokens at a time on the matrix cores rather than token by token, from
+    what `scan_times` expects of the two.  At this margin 1 of 1,508 measured steps is slower than token by token (6 %), and
+    together they are 1.17 times as fast (1.19 with the better one each time).  Microseconds, token by token against in chunks, of
+    the delta rule with 32 heads of 128 x 128: 2,048 tokens 887 / 181, 70 tokens 39 / 29, 256 beside 15 single tokens 161 / 83, 16
+    portions of 32 116 / 74, not taken: 4 of 20 33 / 33, 16 of 8 60 / 70, 100 of 4 243 / 331; a decay per head, 48 heads of 128 x 64:
+    2,048 tokens 705 / 117, 16 portions of 32 43 / 36, not taken: 16 of 16 25 / 36; per channel, 12 heads of 128 x 256: 2,048 tokens
+    818 / 125, 32 portions of 32 112 / 75, not taken: 4 of 64 29 / 37.  `widest`: values from one row to the next of the widest operand
     or result; the chunks' kernels reach over their 32 rows in 32 bits."""
-    return tokens >= 64 + 3 * requests and widest < 2**24
+    return chunked < 0.85 * walked and widest < 2**24
 
 
 def gated_delta(
     qkv: torch.Tensor, proj: torch.Tensor, col_b: int, col_a: int, col_g: int, a_log: torch.Tensor, dt_bias: torch.Tensor,
     norm_weight: torch.Tensor, state: torch.Tensor, cu_seqlens: torch.Tensor, slots: torch.Tensor, *, heads: int,
-    kv_heads: int, dim: int, vdim: int, eps: float,
+    kv_heads: int, dim: int, vdim: int, eps: float, longest: int | None = None,
 ) -> torch.Tensor:
     """The gated delta rule over the rows of a step.  `qkv` [T, 2*kv_heads*dim + heads*vdim]: the
     convolved q | k | v; `proj` [T, ...]: the rows that hold, from columns `col_b`, `col_a`
     (heads each) and `col_g` (heads*vdim) on, the projections of the write gate, the decay and
     the output gate.  `state` float32 [slots + 1, *delta_state_shape(...)] is advanced in
-    place.  Returns `rms_norm(S^T q) * norm_weight * silu(g)` [T, heads*vdim]."""
+    place.  Returns `rms_norm(S^T q) * norm_weight * silu(g)` [T, heads*vdim].  `longest`: tokens of the
+    step's longest portion where the host knows them (it only helps to choose the faster kernel)."""
     _need_cuda(qkv, proj, a_log, dt_bias, norm_weight, state, cu_seqlens, slots)
     for name, t in (("a_log", a_log), ("dt_bias", dt_bias), ("norm_weight", norm_weight), ("cu_seqlens", cu_seqlens), ("slots", slots)):
         _need_contiguous(name, t)
@@ -2017,7 +2050,9 @@ def gated_delta(
     out = torch.empty((qkv.shape[0], heads * vdim), dtype=qkv.dtype, device=qkv.device)
     readout = torch.empty((qkv.shape[0], heads * vdim), dtype=torch.float32, device=qkv.device)  # S^T q before its norm
     lib = library.load()
-    if qkv.dtype == torch.bfloat16 and chunked_scan_pays(qkv.shape[0], requests, max(qkv.stride(0), heads * vdim)):
+    if qkv.dtype == torch.bfloat16 and chunked_scan_pays(
+        *scan_times("delta", qkv.shape[0], requests, longest, heads, dim, vdim), max(qkv.stride(0), heads * vdim)
+    ):
         floats = lib.mi_gated_delta_chunks_scratch(qkv.shape[0], requests, heads, kv_heads, dim, vdim)
         if floats > 0:
             scratch = torch.empty(floats, dtype=torch.float32, device=qkv.device)
@@ -2389,7 +2424,7 @@ def decay_scan(
     q: torch.Tensor, q_col: int, k: torch.Tensor, k_col: int, v: torch.Tensor, v_col: int, gate: torch.Tensor, gate_col: int,
     gate_bias: torch.Tensor, state: torch.Tensor, cu_seqlens: torch.Tensor, slots: torch.Tensor, *, heads: int, groups: int,
     dim: int, vdim: int, per_head: bool, rate: torch.Tensor | None = None, skip: torch.Tensor | None = None,
-    inv_tau: float = 1.0, q_scale: float = 1.0,
+    inv_tau: float = 1.0, q_scale: float = 1.0, longest: int | None = None,
 ) -> torch.Tensor:
     """The recurrence `S <- diag(a) S + k v^T; o = S^T q` over the rows of a step, per request and
     head, float32 state [slots + 1, *decay_state_shape(...)] advanced in place; returns the
@@ -2400,7 +2435,7 @@ def decay_scan(
     `per_head=False`: `gate` rows hold heads*dim logits z from `gate_col` on and
     `a = logistic(z + gate_bias) ** inv_tau`, q enters times `q_scale`.  `per_head=True`: `gate`
     rows hold `heads` raw step sizes, `dt = softplus(raw + gate_bias)`, `a = exp(-exp(rate) * dt)`,
-    v enters times dt and the read-out gets `skip[h] * v` added."""
+    v enters times dt and the read-out gets `skip[h] * v` added.  `longest`: as `gated_delta`."""
     _need_cuda(q, k, v, gate, gate_bias, state, cu_seqlens, slots, rate, skip)
     for name, t in (("gate_bias", gate_bias), ("cu_seqlens", cu_seqlens), ("slots", slots), ("rate", rate), ("skip", skip)):
         _need_contiguous(name, t)
@@ -2427,7 +2462,9 @@ def decay_scan(
         raise KernelShapeError("decay_scan: one more boundary than requests")
     out = torch.empty((tokens, heads * vdim), dtype=torch.float32, device=q.device)
     lib = library.load()
-    if q.dtype == torch.bfloat16 and chunked_scan_pays(tokens, requests, max(v.stride(0), heads * vdim)):
+    if q.dtype == torch.bfloat16 and chunked_scan_pays(
+        *scan_times("per_head" if per_head else "per_channel", tokens, requests, longest, heads, dim, vdim), max(v.stride(0), heads * vdim)
+    ):
         floats = lib.mi_decay_scan_chunks_scratch(int(per_head), tokens, requests, heads, groups, dim, vdim)
         if floats > 0:
             scratch = torch.empty(floats, dtype=torch.float32, device=q.device)

@@ -32,6 +32,11 @@ from mini_infer_amd.registry import register_mixer
 DEFAULT_NAMES = {"z": "z", "x": "x", "g": "g", "o": "o", "z_bias": "z.b", "x_bias": "x.b"}
 
 
+def _longest(ctx: StepContext) -> int | None:
+    """Tokens of the step's longest portion, where the host knows the step's boundaries."""
+    return ctx.max_q_len if ctx.host_cu_seqlens_q is not None else None
+
+
 class MinGRU(Mixer):
     graph_safe = True
 
@@ -83,9 +88,7 @@ class MinGRU(Mixer):
             gated = ops.linear_gru(x, self.zxg.weight, self.bias_z, self.bias_x, cache.state, ctx.state_slots)
             return self.out.forward(gated)
         projected = self.zxg.forward(x)
-        # (the most rows a request brings: known only where the host knows the step's boundaries)
-        max_rows = ctx.max_q_len if ctx.host_cu_seqlens_q is not None else None
-        gated = ops.gated_scan(projected, self.bias_z, self.bias_x, cache.state, ctx.cu_seqlens_q, ctx.state_slots, max_rows)
+        gated = ops.gated_scan(projected, self.bias_z, self.bias_x, cache.state, ctx.cu_seqlens_q, ctx.state_slots, _longest(ctx))
         return self.out.forward(gated)
 
 
@@ -190,7 +193,7 @@ class GatedDeltaRule(Mixer):
         mixed = ops.gated_delta(
             qkv, proj, self.col_write, self.col_decay, self.col_gate, self.rate, self.step_bias, self.norm_weight,
             cache.state["recurrent"], ctx.cu_seqlens_q, ctx.state_slots, heads=self.num_heads, kv_heads=self.num_kv_heads,
-            dim=self.head_dim, vdim=self.v_head_dim, eps=self.norm_eps,
+            dim=self.head_dim, vdim=self.v_head_dim, eps=self.norm_eps, longest=_longest(ctx),
         )
         return self.out.forward(mixed)
 
@@ -274,7 +277,7 @@ class GatedLinearAttention(Mixer):
         readout = ops.decay_scan(
             proj, 0, proj, self.col_k, proj, self.col_v, logits, 0, self.decay_bias, cache.state, ctx.cu_seqlens_q,
             ctx.state_slots, heads=self.num_heads, groups=self.num_heads, dim=self.head_dim, vdim=self.v_head_dim,
-            per_head=False, inv_tau=1.0 / self.tau, q_scale=self.head_dim ** -0.5,
+            per_head=False, inv_tau=1.0 / self.tau, q_scale=self.head_dim ** -0.5, longest=_longest(ctx),
         )
         mixed = ops.readout_gate_norm(readout, proj[:, self.col_gate:], self.norm_weight, group_width=self.v_head_dim,
                                       gate_first=False, eps=self.norm_eps)
@@ -383,7 +386,7 @@ class StateSpaceDuality(Mixer):
         readout = ops.decay_scan(
             conv, self.inner + span, conv, self.inner, conv, 0, proj, self.inner + self.channels, self.step_bias,
             cache.state["recurrent"], ctx.cu_seqlens_q, ctx.state_slots, heads=self.num_heads, groups=self.groups,
-            dim=self.state_size, vdim=self.v_head_dim, per_head=True, rate=self.rate, skip=self.skip,
+            dim=self.state_size, vdim=self.v_head_dim, per_head=True, rate=self.rate, skip=self.skip, longest=_longest(ctx),
         )
         mixed = ops.readout_gate_norm(readout, proj, self.norm_weight, group_width=self.inner // self.norm_groups,
                                       gate_first=True, eps=self.norm_eps)

@@ -253,3 +253,35 @@ def test_what_is_not_finite_goes_token_by_token(monkeypatch, kind, what, dim, vd
         # (bounds of the tests above: twice the error of one side against 64 bits)
         assert float((got - walked)[finite].norm() / walked[finite].norm()) < (2.0 ** -7 if kind == "delta" and got is out else 8e-7)
     assert out[: 50 if name == "state" else at].isfinite().all()
+
+
+@pytest.mark.parametrize("kind", ["delta", "per_head", "per_channel"])
+@pytest.mark.parametrize("lengths,known,chunks", [
+    ([300], True, True), ([300], False, True), ([1] * 15 + [300], True, True), ([64] * 20, False, True),
+    ([8] * 20, True, False), ([16] * 8, True, False), ([5] * 60, True, False), ([1] * 40, False, False), ([20] * 4, True, False), ([1] * 40, True, False),
+])
+def test_which_steps_go_in_chunks(monkeypatch, kind, lengths, known, chunks):
+    """The rule by itself, on both sides of its line, with what the host knows of the portions and without."""
+    from mini_infer_amd import ops
+    from mini_infer_amd.ops import library
+
+    lib, calls = library.load(), []
+    for name in ("mi_gated_delta_chunks", "mi_decay_scan_chunks"):
+        entry = getattr(lib, name)
+        monkeypatch.setattr(lib, name, lambda *args, entry=entry: (calls.append(1), entry(*args))[1])
+    heads, groups, dim, vdim, tokens = 16, 16, 128, 128, sum(lengths)
+    cu, slots = _boundaries(lengths), torch.arange(len(lengths), dtype=torch.int32, device=DEV)
+    rows = lambda n: torch.zeros(tokens, n, dtype=torch.bfloat16, device=DEV)  # noqa: E731
+    longest = max(lengths) if known else None
+    if kind == "delta":
+        state = torch.zeros(len(lengths) + 1, *ops.delta_state_shape(heads, dim, vdim), device=DEV)
+        per_head = torch.zeros(heads, device=DEV)
+        ops.gated_delta(rows(2 * groups * dim + heads * vdim), rows(2 * heads + heads * vdim), 0, heads, 2 * heads, per_head, per_head,
+                        torch.ones(vdim, device=DEV), state, cu, slots, heads=heads, kv_heads=groups, dim=dim, vdim=vdim, eps=1e-6, longest=longest)
+    else:
+        state = torch.zeros(len(lengths) + 1, *ops.decay_state_shape(heads, dim, vdim), device=DEV)
+        gates = heads if kind == "per_head" else heads * dim
+        ops.decay_scan(rows(groups * dim), 0, rows(groups * dim), 0, rows(heads * vdim), 0, rows(gates), 0, torch.zeros(gates, device=DEV), state,
+                       cu, slots, heads=heads, groups=groups, dim=dim, vdim=vdim, per_head=kind == "per_head",
+                       rate=torch.zeros(heads, device=DEV) if kind == "per_head" else None, longest=longest)
+    assert len(calls) == int(chunks)
