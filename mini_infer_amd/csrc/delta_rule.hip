@@ -513,15 +513,12 @@ __global__ __launch_bounds__(256) void delta_readout_norm_kernel(const float* __
 // Decoded tokens: the rule, the read-outs' norm and the gate in one launch, a block per (request, head), bound by
 // reading and writing the state once.  A wave keeps 16 columns, LPC = pad / 4 lanes a column with four rows each, so every
 // load and store covers whole lines; all of a wave's state is asked for before anything else, and the unit norms and
-// gates are made by every wave for itself meanwhile: no tile in LDS, one barrier (for the norm's sum).  A request may
-// bring several tokens (they are walked, at a memory latency each), but steps of more than one a request go to the
-// kernels above.  30 requests, 24 heads of 128 x 128 (94 MB of state): 84 + 7 us for two launches before, 29 now.
-template <int LPC>
-__device__ __forceinline__ float column_sum(float v) {
-  v = lanes_sum<(LPC < 32 ? LPC : 32)>(v);
-  if constexpr (LPC == 64) v += __shfl_xor(v, 32, MI_WAVE);
-  return v;
-}
+// gates are made by every wave for itself meanwhile: no tile in LDS, one barrier (for the norm's sum).  A request's second
+// token would be walked at a memory latency (3 us), so only steps known to bring single tokens come here.  Microseconds of the
+// two launches above and of this one: bfloat16, 24 heads of 128 x 128: 1 request 9.2 / 8.0, 30 requests (94 MB of state) 51 / 28,
+// 512 requests 821 / 346; float32, 32 heads of 64 x 128: 4 requests 11.7 / 10.8, 128 requests 145 / 109.  Keys of 129 columns and more
+// (16 heads of 256 x 256, 30 requests: 92 / 183), float32 ones of 65 and more (64-bit gates and norms by every wave: 24 heads of 128 x
+// 128, 30 requests, 48 / 64) and few float32 heads (32 of 64 x 128, 1 request: 8.3 / 9.8) stay with the two launches.
 __device__ __forceinline__ double wide_sum(double v, int lanes) {
   for (int off = 1; off < lanes; off <<= 1) v += __shfl_xor(v, off, MI_WAVE);
   return v;
@@ -580,8 +577,8 @@ __global__ __launch_bounds__(1024) void gated_delta_token_kernel(
       float qq = 0.f, kk = 0.f;
 #pragma unroll
       for (int e = 0; e < 4; ++e) qq = fmaf(q[e], q[e], qq), kk = fmaf(k[e], k[e], kk);
-      q_inv = rsqrtf(column_sum<LPC>(qq) + 1e-6f) * (1.0f / sqrtf((float)dim));
-      k_inv = rsqrtf(column_sum<LPC>(kk) + 1e-6f);
+      q_inv = rsqrtf(lanes_sum<LPC>(qq) + 1e-6f) * (1.0f / sqrtf((float)dim));
+      k_inv = rsqrtf(lanes_sum<LPC>(kk) + 1e-6f);
       const float z = a_raw + bias, soft = z > 20.f ? z : log1pf(expf(z));
       decay = expf(-expf(rate_log) * soft);
       write = 1.f / (1.f + expf(-b_raw));
@@ -592,11 +589,11 @@ __global__ __launch_bounds__(1024) void gated_delta_token_kernel(
     A square = 0;
 #pragma unroll
     for (int n = 0; n < N; ++n) {
-      const float seen = column_sum<LPC>(fmaf(s[n].x, k[0], s[n].y * k[1]) + fmaf(s[n].z, k[2], s[n].w * k[3])) * decay;
+      const float seen = lanes_sum<LPC>(fmaf(s[n].x, k[0], s[n].y * k[1]) + fmaf(s[n].z, k[2], s[n].w * k[3])) * decay;
       const float u = write * (v[n] - seen);
       s[n].x = fmaf(k[0], u, s[n].x * decay), s[n].y = fmaf(k[1], u, s[n].y * decay);
       s[n].z = fmaf(k[2], u, s[n].z * decay), s[n].w = fmaf(k[3], u, s[n].w * decay);
-      read[n] = column_sum<LPC>(fmaf(s[n].x, q[0], s[n].y * q[1]) + fmaf(s[n].z, q[2], s[n].w * q[3]));
+      read[n] = lanes_sum<LPC>(fmaf(s[n].x, q[0], s[n].y * q[1]) + fmaf(s[n].z, q[2], s[n].w * q[3]));
       if (col0 + n * SIDE < vdim) square += (A)read[n] * (A)read[n];
     }
 #pragma unroll
@@ -774,11 +771,12 @@ int mi_delta_readout_norm(int dtype, const float* readout, const void* proj, int
   return MI_OK;
 }
 
+// single_tokens: no request brings more than one token.
 extern "C" int mi_gated_delta(int dtype, const void* qkv, int64_t qkv_stride, const void* proj, int64_t proj_stride,
                               int col_b, int col_a, int col_g, const float* a_log, const float* dt_bias,
                               const float* norm_weight, float* state, int64_t state_stride, const int* cu,
                               const int* slots, float* readout, void* out, int64_t out_stride, int num_tokens, int num_requests, int heads,
-                              int kv_heads, int dim, int vdim, int dim_pad, float eps, int num_slots, hipStream_t stream) {
+                              int kv_heads, int dim, int vdim, int dim_pad, float eps, int num_slots, int single_tokens, hipStream_t stream) {
   const int bad = mi_gated_delta_check(qkv_stride, proj_stride, col_b, col_a, col_g, state, state_stride, out_stride, num_requests, heads,
                                        kv_heads, dim, vdim, dim_pad, eps, num_slots);
   if (bad != MI_OK) return bad;
@@ -787,21 +785,17 @@ extern "C" int mi_gated_delta(int dtype, const void* qkv, int64_t qkv_stride, co
   delta_layout(dim, vdim, &lanes, &rows);
   if (num_requests == 0) return MI_OK;
   MI_REQUIRE(readout != nullptr, "gated_delta: no buffer for the read-outs");
-  if (num_tokens <= num_requests) {
+  const int pad = lanes * rows;
+  if (single_tokens && (dtype == MI_BF16 ? pad <= 128 : pad == 64 && (int64_t)heads * num_requests >= 128)) {
     dim3 tgrid(heads, num_requests);
     const int threads = ceil_div(vdim, 16) * MI_WAVE;
 #define MI_DELTA_TOKEN(T, LPC)                                                                                            \
   gated_delta_token_kernel<T, LPC><<<tgrid, threads, 0, stream>>>(                                                        \
       (const T*)qkv, qkv_stride, (const T*)proj, proj_stride, col_b, col_a, col_g, a_log, dt_bias, norm_weight, state,    \
       state_stride, cu, slots, (T*)out, out_stride, heads, kv_heads, dim, vdim, eps, num_slots)
-#define MI_DELTA_TOKEN_LANES(T)                \
-  if (pad == 64) MI_DELTA_TOKEN(T, 16);        \
-  else if (pad == 128) MI_DELTA_TOKEN(T, 32);  \
-  else MI_DELTA_TOKEN(T, 64);
-    const int pad = lanes * rows;
-    if (dtype == MI_F32) { MI_DELTA_TOKEN_LANES(float) }
-    else { MI_DELTA_TOKEN_LANES(bf16_t) }
-#undef MI_DELTA_TOKEN_LANES
+    if (dtype == MI_F32) MI_DELTA_TOKEN(float, 16);
+    else if (pad == 64) MI_DELTA_TOKEN(bf16_t, 16);
+    else MI_DELTA_TOKEN(bf16_t, 32);
 #undef MI_DELTA_TOKEN
     MI_CHECK_LAUNCH("gated_delta (a token a request)");
     return MI_OK;

@@ -2070,7 +2070,7 @@ def gated_delta(
             _dtype_code(qkv), _ptr(qkv), qkv.stride(0), _ptr(proj), proj.stride(0), int(col_b), int(col_a), int(col_g),
             _ptr(a_log), _ptr(dt_bias), _ptr(norm_weight), _ptr(state), state.stride(0), _ptr(cu_seqlens), _ptr(slots),
             _ptr(readout), _ptr(out), out.stride(0), qkv.shape[0], requests, heads, kv_heads, dim, vdim, shape[2], float(eps),
-            state.shape[0] - 1, _stream(),
+            state.shape[0] - 1, int(longest == 1), _stream(),
         )
     )
     return out

@@ -100,7 +100,7 @@ _SIGNATURES: dict[str, list] = {
     ],
     "mi_gated_delta": [
         c_int, _P, c_int64, _P, c_int64, c_int, c_int, c_int, _P, _P, _P, _P, c_int64, _P, _P, _P, _P, c_int64,
-        c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_int, _P,
+        c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_int, c_int, _P,
     ],
     "mi_gated_delta_chunks": [
         _P, c_int64, _P, c_int64, c_int, c_int, c_int, _P, _P, _P, _P, c_int64, _P, _P, _P, _P, _P, c_int64, c_int, c_int, c_int, c_int,

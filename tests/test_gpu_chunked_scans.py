@@ -285,3 +285,43 @@ def test_which_steps_go_in_chunks(monkeypatch, kind, lengths, known, chunks):
                        cu, slots, heads=heads, groups=groups, dim=dim, vdim=vdim, per_head=kind == "per_head",
                        rate=torch.zeros(heads, device=DEV) if kind == "per_head" else None, longest=longest)
     assert len(calls) == int(chunks)
+
+
+@pytest.mark.parametrize("lengths", [[1], [1, 0, 1, 1], [0, 3, 1, 0]])
+@pytest.mark.parametrize("heads,kv_heads,dim,vdim", [(3, 3, 20, 30), (4, 2, 64, 250), (128, 4, 64, 40), (2, 1, 65, 16), (2, 2, 128, 128), (2, 1, 129, 40)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_gated_delta_of_steps_said_to_be_single_tokens(lengths, heads, kv_heads, dim, vdim, dtype):
+    """On both sides of the key widths that the one launch takes; right also where a request brings more after all."""
+    from mini_infer_amd import ops
+
+    g = torch.Generator(device=DEV).manual_seed(19)
+    tokens, requests = sum(lengths), len(lengths)
+    qkv, proj = (_rows(g, tokens, n, True).to(dtype) for n in (2 * kv_heads * dim + heads * vdim, 2 * heads + heads * vdim))
+    a_log, dt_bias, weight = torch.rand(heads, generator=g, device=DEV), torch.full((heads,), -2.0, device=DEV), torch.ones(vdim, device=DEV)
+    before = _state(g, requests, ops.delta_state_shape(heads, dim, vdim), dim)
+    state = before.clone()
+    cu, slots = _boundaries(lengths), torch.arange(requests, dtype=torch.int32, device=DEV)
+    got = ops.gated_delta(qkv, proj, 0, heads, 2 * heads, a_log, dt_bias, weight, state, cu, slots, heads=heads, kv_heads=kv_heads, dim=dim,
+                          vdim=vdim, eps=1e-6, longest=1)
+    out, left = _exact_delta(qkv, proj, a_log, dt_bias, before, cu, heads, kv_heads, dim, vdim)
+    # as for decoded tokens above
+    assert _rel(state[:requests], left) < 2e-7 and torch.equal(state[requests:], before[requests:])
+    assert _rel(got, out) < (2.0 ** -8 if dtype == torch.bfloat16 else 3e-7)
+
+
+def test_a_recorded_step_is_not_taken_for_single_tokens():
+    """No more tokens than requests, but one request's: the bits of the two launches, which steps of single tokens do not take."""
+    from mini_infer_amd import ops
+
+    heads, dim, tokens, requests = 4, 128, 8, 8
+    g = torch.Generator(device=DEV).manual_seed(23)
+    qkv, proj = (torch.randn(tokens, n, generator=g, device=DEV).bfloat16() for n in (3 * heads * dim, 2 * heads + heads * dim))
+    a_log, dt_bias, weight = torch.zeros(heads, device=DEV), torch.full((heads,), -2.0, device=DEV), torch.ones(dim, device=DEV)
+    before = _state(g, requests, ops.delta_state_shape(heads, dim, dim), dim)
+    made = []
+    for count in (requests, 1):  # (with one request there are more tokens than requests)
+        state = before.clone()
+        cu = torch.tensor([0] + [tokens] * count, dtype=torch.int32, device=DEV)
+        made.append((ops.gated_delta(qkv, proj, 0, heads, 2 * heads, a_log, dt_bias, weight, state, cu, torch.arange(count, dtype=torch.int32, device=DEV),
+                                     heads=heads, kv_heads=heads, dim=dim, vdim=dim, eps=1e-6), state))
+    assert torch.equal(made[0][0], made[1][0]) and torch.equal(made[0][1], made[1][1])
