@@ -110,6 +110,8 @@ __global__ __launch_bounds__(64 * WAVES) void attn_generic_kernel(
   const int a = lo + split * chunk;
   const int b = min(a + chunk, hi);
   const int* bt = block_table + (int64_t)req * max_blocks;
+  const bool merges = WAVES > 1 && b - a > MI_WAVE;  // (else wave 0 has all keys)
+  if (!merges && wave > 0) return;
 
   float m[GT];
   S l[GT], acc[GT][VPL];
@@ -250,7 +252,7 @@ __global__ __launch_bounds__(64 * WAVES) void attn_generic_kernel(
     }
   }
 
-  if constexpr (WAVES > 1) {  // wave 0 takes over what the others have, in their order
+  if (merges) {  // wave 0 takes over what the others have, in their order
     S* merge = q_lds + GT * head_dim;  // [WAVES - 1][GT][VPL + 1][64], then their maxima
     float* maxima = reinterpret_cast<float*>(merge + (WAVES - 1) * GT * (VPL + 1) * MI_WAVE);
     if (wave > 0) {
@@ -424,10 +426,17 @@ static int attn_generic_launch(const void* q, int64_t q_row_stride, const void* 
   const size_t lds = sizeof(S) * GT * head_dim;
   const bool vec = head_dim % 16 == 0 && v_dim % 16 == 0 && v_row_stride % 16 == 0;
   // Four waves a range in the 32-bit path where one wave a range is fewer than two waves a SIMD (decode; values of
-  // up to 128 dims, which the merging's LDS holds).  One layer, 32 heads of 64 over 8 key/value heads, microseconds
-  // before and now: 3 tokens of up to 600 positions 113 -> 17.4, a prompt of 509 tokens 247 -> 148 (the batched
-  // loads alone, one wave a range; such prompts now take attention_prompt_f32.hip, 66).
-  const bool four = sizeof(S) == 8 && v_dim <= 128 && (int64_t)grid.x * grid.y * grid.z < 2048;
+  // up to 128 dims, which the merging's LDS holds) and the ranges are long enough for the blocks, of which three run
+  // on a CU at once instead of twelve.  Microseconds a layer with one wave and with four: 24 heads of 128 over 8: 30 tokens of
+  // 100 positions (240 blocks) 40 / 36, 60 of 200 113 / 47, 100 of 100 (800 blocks) 63 / 74, 100 of 200 115 / 82, 200 of 100 (1,600)
+  // 69 / 108, 200 of 400 313 / 299; 32 heads of 64 over 8: 30 of 200 44 / 20, 100 of 100 30 / 35, 200 of 200 60 / 60.  (One wave before
+  // its loads were batched: a prompt of 509 tokens 247, then 148; such prompts now take attention_prompt_f32.hip, 66.)
+  const int64_t blocks = (int64_t)grid.x * grid.y * grid.z;
+  int64_t keys = (int64_t)max_blocks * page_size;  // the most a range can have
+  if (window > 0) keys = keys < window ? keys : window;
+  if (mask_chunk > 0) keys = keys < mask_chunk ? keys : mask_chunk;
+  keys = ceil_div64(keys, num_splits);
+  const bool four = sizeof(S) == 8 && v_dim <= 128 && blocks < 2048 && keys > MI_WAVE * ceil_div64(blocks, 768);
 #define MI_ATTN_LAUNCH_WAVES(VPL, VEC, WAVES, LDS)                                                \
   attn_generic_kernel<T, VPL, VEC, WAVES><<<grid, WAVES * MI_WAVE, LDS, stream>>>(                \
       (const T*)q, q_row_stride, (const T*)k_pages, (const T*)v_pages, block_table, max_blocks,   \

@@ -1129,3 +1129,33 @@ def test_prompt_attention_float32(q_heads, kv_heads, dim, page, window, lengths,
     # both round a result once; the plain kernel also each weight (weights sum to one) and, with cut keys, each part
     most = float(v_pages[torch.isfinite(v_pages)].abs().max())
     assert (got[:-1] - plain[:-1]).abs().max() <= 4 * 2.0 ** -24 * most
+
+
+@pytest.mark.parametrize("q_heads,kv_heads,dim,requests,longest,window", [
+    (24, 8, 128, 90, 128, None), (24, 8, 128, 110, 128, None), (24, 8, 128, 110, 130, None), (6, 3, 80, 300, 300, 65), (4, 4, 64, 2, 65, None),
+    (8, 8, 64, 260, 20, None)])
+def test_decoded_tokens_attention_float32(q_heads, kv_heads, dim, requests, longest, window):
+    """On both sides of the line between one wave and four a block; contexts of 1, 64 and 65 keys, which leave waves idle, and the
+    longest, in one launch; in 64 bits."""
+    from mini_infer_amd import ops
+
+    page = 16
+    keys = [(1, 64, 65, longest)[b % 4] if longest >= 65 else 1 + b % longest for b in range(requests)]
+    keys = [min(n, longest) for n in keys]
+    blocks = max(-(-n // page) for n in keys)
+    k_pages, v_pages = (_rand(requests * blocks, kv_heads, page, dim, seed=s) for s in (2, 3))
+    table = torch.randperm(requests * blocks, generator=torch.Generator().manual_seed(1)).int().view(requests, blocks).to(DEV)
+    q = _rand(requests, q_heads * dim, seed=4)
+    ints = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)  # noqa: E731
+    cu = list(range(requests + 1))
+    got = ops.paged_attention(q, k_pages, v_pages, table, ints(cu[:-1]), ints([n - 1 for n in keys]), ints(cu), cu, q_heads=q_heads,
+                              kv_heads=kv_heads, head_dim=dim, scale=dim ** -0.5, window=window, max_seq_len=max(keys))
+    seen = torch.arange(blocks * page, device=DEV)[None] < ints(keys)[:, None]
+    if window is not None:
+        seen &= torch.arange(blocks * page, device=DEV)[None] >= ints(keys)[:, None] - window
+    k, v = (pages[table.long()].transpose(2, 3).reshape(requests, -1, kv_heads, dim).repeat_interleave(q_heads // kv_heads, 2).double() for pages in (k_pages, v_pages))
+    scores = (q.view(requests, 1, q_heads, dim).double() * k).sum(-1) * dim ** -0.5
+    weights = torch.softmax(scores.masked_fill(~seen[..., None], float("-inf")), 1)
+    want = (weights[..., None] * v).sum(1).flatten(1)
+    # a weight and the result are rounded once each (weights sum to one)
+    assert (got.double() - want).abs().max() <= 3 * 2.0 ** -24 * float(v_pages.abs().max())
