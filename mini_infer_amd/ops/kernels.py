@@ -1165,33 +1165,54 @@ def paged_attention(
         return out
 
     assert chunk is None  # (a chunked mask on plain pages has gone to the general entry point above)
-    # float32 steps with many tokens a request: 16 rows a block on the matrix cores' 64-bit instruction.  (Below a block a CU
-    # keys have to be cut into ranges; a tile whose tokens are different requests' walks one's keys after another's.)
-    if (
-        q.dtype == torch.float32 and slopes is None and not force_plain and host_cu_seqlens_q is not None
-        and tokens >= 32 * num_requests and lib.mi_attn_prompt_f32_blocks(tokens, q_heads, kv_heads, head_dim, page_size) >= 256
-        and q.stride(0) % 4 == 0 and out.stride(0) % 4 == 0
-        and all(t.data_ptr() % 16 == 0 for t in (q, k_pages, v_pages, out))
-    ):
-        library.check(
-            lib.mi_attn_prompt_f32(
-                _ptr(q), q.stride(0), _ptr(k_pages), _ptr(v_pages), _ptr(block_table), block_table.shape[1], _ptr(token_request),
-                _ptr(positions), _ptr(out), out.stride(0), tokens, q_heads, kv_heads, head_dim, page_size, num_pages, float(scale),
-                int(window or 0), _stream(),
-            )
+    # float32 portions of many tokens: 16 rows a block on the matrix cores' 64-bit instruction.  Leading requests that bring a
+    # single token go to the plain kernel by themselves, as above: in a tile each of them would walk its keys after another's (15
+    # of 2,000 positions beside a portion of 1,024, 24 heads of 128 over 8: 988 microseconds together, 424 apart; 8 over 8 1,885 / 275).
+    single = 0
+    if q.dtype == torch.float32 and slopes is None and not force_plain and host_cu_seqlens_q is not None:
+        q_lens = [host_cu_seqlens_q[b + 1] - host_cu_seqlens_q[b] for b in range(num_requests)]
+        while single < num_requests and q_lens[single] == 1:
+            single += 1
+        portions = q_lens[single:]
+        by_tiles = (
+            prompt_tiles_pay(portions, lib.mi_attn_prompt_f32_blocks(tokens - single, q_heads, kv_heads, head_dim, page_size))
+            and q.stride(0) % 4 == 0 and out.stride(0) % 4 == 0
+            and all(t.data_ptr() % 16 == 0 for t in (q, k_pages, v_pages, out))
         )
-        return out
-    splits = attention_splits(tokens * kv_heads * math.ceil(group / 4), max_seq_len)
-    part_acc, part_ml = partials(splits)
+        if by_tiles:
+            library.check(
+                lib.mi_attn_prompt_f32(
+                    _ptr(q) + 4 * single * q.stride(0), q.stride(0), _ptr(k_pages), _ptr(v_pages), _ptr(block_table), block_table.shape[1],
+                    _ptr(token_request) + 4 * single, _ptr(positions) + 4 * single, _ptr(out) + 4 * single * out.stride(0), out.stride(0),
+                    tokens - single, q_heads, kv_heads, head_dim, page_size, num_pages, float(scale), int(window or 0), _stream(),
+                )
+            )
+            if single == 0:
+                return out
+        else:
+            single = 0
+    rows = single if single else tokens
+    splits = attention_splits(rows * kv_heads * math.ceil(group / 4), max_seq_len)
+    part_acc, part_ml = partials(splits, rows)
     library.check(
         lib.mi_attn_generic(
             _dtype_code(q), _ptr(q), q.stride(0), _ptr(k_pages), _ptr(v_pages), _ptr(block_table),
             block_table.shape[1], _ptr(token_request), _ptr(positions), _ptr(out), out.stride(0),
-            _ptr(part_acc), _ptr(part_ml), tokens, q_heads, kv_heads, head_dim, page_size, num_pages,
+            _ptr(part_acc), _ptr(part_ml), rows, q_heads, kv_heads, head_dim, page_size, num_pages,
             float(scale), int(window or 0), splits, _ptr(slopes), _stream(),
         )
     )
     return out
+
+
+def prompt_tiles_pay(portions: list[int], blocks: int) -> bool:
+    """Whether float32 portions go to the kernel with 16 rows a tile, which starts `blocks` blocks for them (0: sizes it does not
+    take).  Microseconds a layer in the plain kernel and in tiles: 24 heads of 128 over 8: 160 tokens (256 blocks) 51 / 22, 256 tokens
+    behind 3,000 positions 1,630 / 412, 8 portions of 40 behind 1,000 positions 570 / 159; 16 portions of 16 (not taken) 19 / 26.  A
+    tile walks the keys of its requests one after another, so few of them may be short: 8 heads of 128 over 8 (16 tokens a tile), 10
+    single tokens of 1,000 positions behind a portion of 1,024 980 / 674, 30 of 3,000 behind one of 300 (not taken) 1,863 / 3,084."""
+    short = sum(n < 16 for n in portions)
+    return blocks >= 256 and sum(portions) >= max(32 * len(portions), 64 * short)
 
 
 GENERAL_ATTENTION_MAX_KEY_DIM = 1024

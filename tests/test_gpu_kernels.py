@@ -1159,3 +1159,36 @@ def test_decoded_tokens_attention_float32(q_heads, kv_heads, dim, requests, long
     want = (weights[..., None] * v).sum(1).flatten(1)
     # a weight and the result are rounded once each (weights sum to one)
     assert (got.double() - want).abs().max() <= 3 * 2.0 ** -24 * float(v_pages.abs().max())
+
+
+@pytest.mark.parametrize("q_heads,kv_heads,dim,lengths,contexts,launches", [
+    (24, 8, 128, [1, 1, 1, 200], [700, 0, 64, 30], ["tiles", "plain"]), (8, 8, 64, [1] * 5 + [300, 290], [90] * 7, ["tiles", "plain"]),
+    (24, 8, 128, [1, 1, 60], [70, 3, 0], ["plain"]), (8, 8, 64, [520] + [1] * 9, [20] * 10, ["plain"]), (24, 8, 128, [170], [9], ["tiles"])])
+def test_mixed_step_attention_float32(monkeypatch, q_heads, kv_heads, dim, lengths, contexts, launches):
+    """Leading single tokens apart from the portions, where those go in tiles; all in one plain launch else.  In 64 bits."""
+    from mini_infer_amd import ops
+    from mini_infer_amd.ops import library
+
+    lib, taken = library.load(), []
+    for kind, name in (("tiles", "mi_attn_prompt_f32"), ("plain", "mi_attn_generic")):
+        entry = getattr(lib, name)
+        monkeypatch.setattr(lib, name, lambda *args, kind=kind, entry=entry: (taken.append(kind), entry(*args))[1])
+    page, keys = 16, [n + c for n, c in zip(lengths, contexts)]
+    blocks = max(-(-n // page) for n in keys)
+    k_pages, v_pages = (_rand(len(lengths) * blocks, kv_heads, page, dim, seed=s) for s in (2, 3))
+    table = torch.randperm(len(lengths) * blocks, generator=torch.Generator().manual_seed(1)).int().view(-1, blocks).to(DEV)
+    ints = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)  # noqa: E731
+    cu = [0, *torch.tensor(lengths).cumsum(0).tolist()]
+    q = _rand(cu[-1], q_heads * dim + 4, seed=4)[:, : q_heads * dim]
+    positions = [c + i for n, c in zip(lengths, contexts) for i in range(n)]
+    got = ops.paged_attention(q, k_pages, v_pages, table, ints([b for b, n in enumerate(lengths) for _ in range(n)]), ints(positions), ints(cu), cu,
+                              q_heads=q_heads, kv_heads=kv_heads, head_dim=dim, scale=dim ** -0.5, window=None, max_seq_len=max(keys))
+    assert taken == launches
+    for b, n in enumerate(lengths):
+        k, v = (pages[table[b].long()].transpose(1, 2).reshape(-1, kv_heads, dim).repeat_interleave(q_heads // kv_heads, 1).double() for pages in (k_pages, v_pages))
+        rows = slice(cu[b], cu[b + 1])
+        scores = torch.matmul(q[rows].view(n, q_heads, dim).double().transpose(0, 1), k.permute(1, 2, 0).contiguous()) * dim ** -0.5
+        scores.masked_fill_(torch.arange(k.shape[0], device=DEV)[None] > ints(positions[rows])[:, None], float("-inf"))
+        want = torch.matmul(torch.softmax(scores, -1), v.transpose(0, 1).contiguous()).transpose(0, 1).flatten(1)
+        # a weight and the result are rounded once each (weights sum to one), and each part where keys are cut
+        assert (got[rows].double() - want).abs().max() <= 4 * 2.0 ** -24 * float(v_pages.abs().max())
