@@ -200,11 +200,13 @@ __global__ __launch_bounds__(64 * WAVES) void attn_generic_kernel(
 #pragma unroll
     for (int g = 0; g < GT; ++g) {
       const float m_new = fmaxf(m[g], wave_max(s[g]));
-      const float alpha = expf(m[g] - m_new);
+      // (a wave that has seen scores of -inf alone so far, of infinite keys say: weight 0, not the exponential of inf less inf)
+      const float top = WAVES > 1 && m_new == -INFINITY ? 0.f : m_new;
+      const float alpha = expf(m[g] - top);
       // (64-bit sums: the difference is taken and the exponential made before anything is
       // rounded to float32, so a key's weight is off by one rounding, not by the score's)
-      if constexpr (sizeof(S) == 8) p[g] = valid ? (float)exp(s_sum[g] - (S)m_new) : 0.f;
-      else p[g] = valid ? expf(s_sum[g] - m_new) : 0.f;
+      if constexpr (sizeof(S) == 8) p[g] = valid ? (float)exp(s_sum[g] - (S)top) : 0.f;
+      else p[g] = valid ? expf(s_sum[g] - top) : 0.f;
       l[g] = l[g] * (S)alpha + wave_sum((S)p[g]);
 #pragma unroll
       for (int v = 0; v < VPL; ++v) acc[g][v] *= (S)alpha;

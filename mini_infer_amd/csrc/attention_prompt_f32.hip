@@ -131,7 +131,8 @@ __global__ __launch_bounds__(WAVES * MI_WAVE, HD == 64 ? 2 : 1) void attn_prompt
       double p[4];
 #pragma unroll
       for (int e = 0; e < 4; ++e) {
-        p[e] = sees[e] ? exp(score[e] - (double)m[e]) : 0.0;
+        // (scores of -inf alone so far, of an infinite key say: weight 0, not the exponential of inf less inf)
+        p[e] = sees[e] ? exp(score[e] - (m[e] == -INFINITY ? 0.0 : (double)m[e])) : 0.0;
         l[e] += p[e];
         mine[(4 * e + quad) * P_ROW + c] = p[e];
       }

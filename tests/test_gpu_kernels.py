@@ -1192,3 +1192,30 @@ def test_mixed_step_attention_float32(monkeypatch, q_heads, kv_heads, dim, lengt
         want = torch.matmul(torch.softmax(scores, -1), v.transpose(0, 1).contiguous()).transpose(0, 1).flatten(1)
         # a weight and the result are rounded once each (weights sum to one), and each part where keys are cut
         assert (got[rows].double() - want).abs().max() <= 4 * 2.0 ** -24 * float(v_pages.abs().max())
+
+
+@pytest.mark.parametrize("tokens,plain", [(520, False), (520, True), (1, True)])
+@pytest.mark.parametrize("low", [[16], [32, 33], list(range(64, 128)), list(range(100, 300))])
+def test_scores_of_minus_infinity_have_no_weight_float32(tokens, plain, low):
+    """Keys whose scores are -inf (an infinite element), also where a tile of keys, or all that a wave has seen so far, has no
+    others: left out, as a score that is very low is."""
+    from mini_infer_amd import ops
+
+    q_heads, kv_heads, dim, page, length = 8, 8, 64, 16, 520 if tokens > 1 else 500
+    k_pages, v_pages = (_rand(-(-length // page), kv_heads, page, dim, seed=s) for s in (2, 3))
+    flat = k_pages.transpose(1, 2).reshape(-1, kv_heads, dim)
+    flat[low, :, 0] = float("inf")
+    k_pages = flat.view(-1, page, kv_heads, dim).transpose(1, 2).contiguous()
+    q = _rand(tokens, q_heads * dim, seed=4)
+    q.view(tokens, q_heads, dim)[:, :, 0] = -1.0 - q.view(tokens, q_heads, dim)[:, :, 0].abs()
+    first = 0 if tokens > 1 else length - 1
+    ints = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)  # noqa: E731
+    got = ops.paged_attention(q, k_pages, v_pages, torch.arange(len(k_pages), dtype=torch.int32, device=DEV)[None], ints([0] * tokens),
+                              ints([first + i for i in range(tokens)]), ints([0, tokens]), [0, tokens], q_heads=q_heads, kv_heads=kv_heads, head_dim=dim,
+                              scale=dim ** -0.5, window=None, max_seq_len=first + tokens, force_plain=plain)
+    v = v_pages.transpose(1, 2).reshape(-1, kv_heads, dim).double()
+    scores = torch.matmul(q.view(tokens, q_heads, dim).double().transpose(0, 1), flat.double().permute(1, 2, 0).contiguous()) * dim ** -0.5
+    scores.masked_fill_(torch.arange(len(flat), device=DEV)[None] > (first + torch.arange(tokens, device=DEV))[:, None], float("-inf"))
+    want = torch.matmul(torch.softmax(scores, -1), v.transpose(0, 1).contiguous()).transpose(0, 1).flatten(1)
+    assert want.isfinite().all() and got.isfinite().all()
+    assert (got.double() - want).abs().max() <= 4 * 2.0 ** -24 * float(v_pages.abs().max())
