@@ -148,12 +148,31 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const float* __restrict__
       }
 }
 
+// The same without a branch around the load, for loads that stay in flight (the row's first values where it has ended, masked).
+template <bool ALIGNED>
+__device__ __forceinline__ float4 four_in_flight(const float* row, int at, int k) {
+  uint32_t bits[4];
+  if constexpr (ALIGNED) {
+    const uint4 got = *reinterpret_cast<const uint4*>(row + (at < k ? at : 0));
+    bits[0] = got.x, bits[1] = got.y, bits[2] = got.z, bits[3] = got.w;
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e) bits[e] = __float_as_uint(row[at + e < k ? at + e : 0]);
+  }
+#pragma unroll
+  for (int e = 0; e < 4; ++e) bits[e] &= at + e < k ? ~0u : 0u;
+  return make_float4(__uint_as_float(bits[0]), __uint_as_float(bits[1]), __uint_as_float(bits[2]), __uint_as_float(bits[3]));
+}
+
 // Few rows (decode): bound by reading W once.  A block owns 16 * RT rows and 16 * FT features; its 8 waves take
 // one run of K each (the order above), every wave streams its part of the weights from memory, two slices ahead,
 // and the runs' sums meet in LDS.  LINES: whole lines of W, non-temporal, brought into operand order by lane
-// exchanges (common.h): rows of W on 128 bytes, K a multiple of 32, A on 16 bytes; else guarded single values.
+// exchanges (common.h): rows of W on 128 bytes, K a multiple of 32, A on 16 bytes.  PIECES: 16 bytes a load in operand order
+// (K and both strides in whole 4s, both matrices on 16 bytes); VALUES: single ones.
 // Rows past m and features past n repeat the last one and are not written.
-template <int RT, int FT, bool LINES>
+enum { VALUES = 0, PIECES = 1, LINES = 2 };
+
+template <int RT, int FT, int FORM>
 __global__ __launch_bounds__(SEGMENTS * MI_WAVE) void gemm_f32_rows_kernel(const float* __restrict__ a, int64_t lda,
                                                             const float* __restrict__ w, int64_t ldw,
                                                             float* __restrict__ c, int64_t ldc, int m, int n, int k) {
@@ -172,7 +191,7 @@ __global__ __launch_bounds__(SEGMENTS * MI_WAVE) void gemm_f32_rows_kernel(const
   const int run = segment_slices(k), slices = ceil_div(k, SLICE);
   const int first = min(wave * run, slices), last = min(first + run, slices);
 
-  if constexpr (LINES) {
+  if constexpr (FORM == LINES) {
     // (offsets from the first of the block's rows: at most 32 rows of at most 2^26 bytes)
     uint32_t lower[FT], upper[FT];
 #pragma unroll
@@ -222,22 +241,41 @@ __global__ __launch_bounds__(SEGMENTS * MI_WAVE) void gemm_f32_rows_kernel(const
       }
     }
   } else {
-    for (int slice = first; slice < last; ++slice) {
+    constexpr int AHEAD = 2;
+    const float* w_row[FT];
+#pragma unroll
+    for (int f = 0; f < FT; ++f) w_row[f] = w + (int64_t)min(col0 + 16 * f + r, n - 1) * ldw;
+    float4 wv[AHEAD][FT][2], xv[AHEAD][RT][2];
+    auto fetch = [&](int slot, int slice) {
 #pragma unroll
       for (int half = 0; half < 2; ++half) {
         const int at = slice * SLICE + 16 * half + 4 * quad;
-        float xv[RT][4], wv[FT][4];
 #pragma unroll
-        for (int i = 0; i < RT; ++i) *reinterpret_cast<float4*>(xv[i]) = four_of_row<false>(a_row[i], at, k);
+        for (int f = 0; f < FT; ++f) wv[slot][f][half] = four_in_flight<FORM == PIECES>(w_row[f], at, k);
 #pragma unroll
-        for (int f = 0; f < FT; ++f)
-          *reinterpret_cast<float4*>(wv[f]) = four_of_row<false>(w + (int64_t)min(col0 + 16 * f + r, n - 1) * ldw, at, k);
+        for (int i = 0; i < RT; ++i) xv[slot][i][half] = four_in_flight<FORM == PIECES>(a_row[i], at, k);
+      }
+    };
 #pragma unroll
-        for (int e = 0; e < 4; ++e)
+    for (int s = 0; s < AHEAD; ++s)
+      if (first + s < last) fetch(s, first + s);
+    for (int at = first; at < last; at += AHEAD) {
 #pragma unroll
-          for (int i = 0; i < RT; ++i)
+      for (int s = 0; s < AHEAD; ++s) {
+        if (at + s < last) {
+          float ws[FT][2][4], xs[RT][2][4];
+          __builtin_memcpy(ws, wv[s], sizeof(ws));
+          __builtin_memcpy(xs, xv[s], sizeof(xs));
+          if (at + s + AHEAD < last) fetch(s, at + s + AHEAD);
 #pragma unroll
-            for (int f = 0; f < FT; ++f) acc[i][f] = mma(xv[i][e], wv[f][e], acc[i][f]);
+          for (int half = 0; half < 2; ++half)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+              for (int i = 0; i < RT; ++i)
+#pragma unroll
+                for (int f = 0; f < FT; ++f) acc[i][f] = mma(xs[i][half][e], ws[f][half][e], acc[i][f]);
+        }
       }
     }
   }
@@ -267,10 +305,11 @@ static void launch_tiles(const float* a, int64_t lda, const float* w, int64_t ld
 
 template <int RT, int FT>
 static void launch_rows(const float* a, int64_t lda, const float* w, int64_t ldw, float* c, int64_t ldc, int m, int n,
-                        int k, bool lines, hipStream_t stream) {
+                        int k, int form, hipStream_t stream) {
   const int grid = ceil_div(n, 16 * FT), block = SEGMENTS * MI_WAVE;
-  if (lines) gemm_f32_rows_kernel<RT, FT, true><<<grid, block, 0, stream>>>(a, lda, w, ldw, c, ldc, m, n, k);
-  else gemm_f32_rows_kernel<RT, FT, false><<<grid, block, 0, stream>>>(a, lda, w, ldw, c, ldc, m, n, k);
+  if (form == LINES) gemm_f32_rows_kernel<RT, FT, LINES><<<grid, block, 0, stream>>>(a, lda, w, ldw, c, ldc, m, n, k);
+  else if (form == PIECES) gemm_f32_rows_kernel<RT, FT, PIECES><<<grid, block, 0, stream>>>(a, lda, w, ldw, c, ldc, m, n, k);
+  else gemm_f32_rows_kernel<RT, FT, VALUES><<<grid, block, 0, stream>>>(a, lda, w, ldw, c, ldc, m, n, k);
 }
 
 // Which kernel, with microseconds at rows x N x K (weights from memory).  Before: 64-bit multiply-adds on the vector
@@ -283,7 +322,9 @@ static void launch_rows(const float* a, int64_t lda, const float* w, int64_t ldw
 // library's 64-bit product reaches 64.  Two tiles of features a wave from 8,192 on (fewer blocks below that would
 // leave CUs idle).  Up to 32 rows the streaming kernel always (20 x 128256 x 2048: 325 against 320 for the tiles,
 // 20 x 16384: 46 against 66); up to 64 rows where there are few features (60 x 2048: 26 against 64; 60 x 128256:
-// 810 against 580, every block reads all the rows' activations).
+// 810 against 580, every block reads all the rows' activations).  Rows off whole lines, 16-byte pieces (single values waited for one
+// by one before): 1 x 128256 x 2052 684 -> 267, 32 rows 1,410 -> 509; 16 x 4096 x 4096, rows not on a line, 66 -> 23; single values, 8 x
+// 32000 x 4095 415 -> 218.
 extern "C" int mi_gemm_f32(const float* a, int64_t lda, const float* w, int64_t ldw, float* c,
                            int64_t ldc, int m, int n, int k, hipStream_t stream) {
   MI_REQUIRE(m >= 0 && n > 0 && k > 0, "gemm_f32: bad sizes m=%d n=%d k=%d", m, n, k);
@@ -295,10 +336,11 @@ extern "C" int mi_gemm_f32(const float* a, int64_t lda, const float* w, int64_t 
   if (m <= 32 || (m <= 64 && !wide)) {
     // (the streaming loads' offsets reach over a block's 32 features in 32 bits: ldw under 2^24 values)
     const bool lines = a16 && k % SLICE == 0 && ldw % 32 == 0 && (uintptr_t)w % 128 == 0 && ldw < (1 << 24);
-    if (m > 32) launch_rows<4, 1>(a, lda, w, ldw, c, ldc, m, n, k, lines, stream);
-    else if (m > 16) launch_rows<2, 1>(a, lda, w, ldw, c, ldc, m, n, k, lines, stream);
-    else if (wide) launch_rows<1, 2>(a, lda, w, ldw, c, ldc, m, n, k, lines, stream);
-    else launch_rows<1, 1>(a, lda, w, ldw, c, ldc, m, n, k, lines, stream);
+    const int form = lines ? LINES : a16 && w16 && k % 4 == 0 ? PIECES : VALUES;
+    if (m > 32) launch_rows<4, 1>(a, lda, w, ldw, c, ldc, m, n, k, form, stream);
+    else if (m > 16) launch_rows<2, 1>(a, lda, w, ldw, c, ldc, m, n, k, form, stream);
+    else if (wide) launch_rows<1, 2>(a, lda, w, ldw, c, ldc, m, n, k, form, stream);
+    else launch_rows<1, 1>(a, lda, w, ldw, c, ldc, m, n, k, form, stream);
     MI_CHECK_LAUNCH("gemm_f32 (few rows)");
     return MI_OK;
   }

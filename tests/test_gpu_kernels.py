@@ -1219,3 +1219,26 @@ def test_scores_of_minus_infinity_have_no_weight_float32(tokens, plain, low):
     want = torch.matmul(torch.softmax(scores, -1), v.transpose(0, 1).contiguous()).transpose(0, 1).flatten(1)
     assert want.isfinite().all() and got.isfinite().all()
     assert (got.double() - want).abs().max() <= 4 * 2.0 ** -24 * float(v_pages.abs().max())
+
+
+@pytest.mark.parametrize("m", [1, 16, 17, 33, 64])
+@pytest.mark.parametrize("n,k", [(40, 4), (33, 36), (8200, 100), (100, 2052), (17, 63), (8193, 258)])
+def test_few_rows_of_gemm_f32_off_whole_lines(m, n, k):
+    """Rows of W that end inside a line or start off one: loads by 16 bytes and by single values, whose masked parts (infinite
+    first values here) add nothing; the bits of 16-byte rows, of single values and of many rows are the same."""
+    from mini_infer_amd import ops
+
+    a, w = _rand(m, k, seed=31), _rand(n, k, seed=32)
+    a[:, 0], w[:, 0] = 1.0, float("inf")  # (every sum is infinite, so an addend of 0 * inf would show as NaN)
+    assert torch.isinf(ops.gemm_f32(a, w)).all()
+    w[:, 0] = 0.5
+    out = ops.gemm_f32(a, w)
+    exact = a.double() @ w.double().T
+    assert ((out.double() - exact).abs() <= 2.0 ** -24 * exact.abs() + 1e-12 * math.sqrt(k)).all()
+    for before_a, before_w in ((4, 4), (0, 4), (4, 0), (1, 4), (4, 3)):
+        off_a, off_w = torch.full((m, k + 4), 3.0, device=DEV), torch.full((n, k + 4), 5.0, device=DEV)
+        off_a, off_w = off_a[:, before_a : before_a + k], off_w[:, before_w : before_w + k]
+        off_a.copy_(a), off_w.copy_(w)
+        assert torch.equal(ops.gemm_f32(off_a, off_w), out), (before_a, before_w)
+    many = torch.cat([a, torch.ones(70, k, device=DEV)])
+    assert torch.equal(ops.gemm_f32(many, w)[:m], out)
