@@ -738,12 +738,12 @@ extern "C" int mi_route_top_k(int dtype, const void* x, int64_t x_stride, const 
   const int per_block = lds_for(4) <= 64 * 1024 ? 4 : (lds_for(2) <= 64 * 1024 ? 2 : 1);
   MI_REQUIRE(lds_for(per_block) <= 64 * 1024, "route_top_k: rows of %d do not fit the block's staging", width);
   // A wave walks one router row after another, at the latency of its loads: as many waves as a block may have while the
-  // blocks have a CU each, ten where they share them.  Microseconds with 256, 640 and 1,024 threads (rows x width, outputs):
-  // 300 x 3072, 18: 19.9, 10.8, 10.5; 1501 x 3072, 18: 21.3, 15.4, 18.5; 1000 x 2048, 64: 46.8, 26.7, 22.8; 2048 x 4096,
-  // 64: 68.4, 52.4, 52.9.
+  // blocks have a CU each, ten where two share one, and four where enough blocks do (three and more; rows of 40 KB and more
+  // leave room for fewer).  Microseconds with 256, 640 and 1,024 threads (rows x width, outputs): 300 x 3072, 18: 19.9, 10.8, 10.5;
+  // 1501 x 3072, 18: 21.3, 15.4, 18.5; 1000 x 2048, 64: 46.8, 26.7, 22.8; 2048 x 4096, 64: 68.4, 52.4, 52.9; 4000 x 3072, 18: 26.4,
+  // 30.2, 31.9; 16000 x 2048, 256: 617, 709, 684; 4000 x 7168, 256 (57 KB a block): 722, 531, 518.
   const int blocks = ceil_div(num_tokens, per_block);
-  const int threads = blocks <= 256 ? 1024 : 640;
-
+  const int threads = blocks <= 256 ? 1024 : (blocks <= 512 || lds_for(per_block) > 40 * 1024 ? 640 : 256);
 #define MI_ROUTE(T, R)                                                                                               \
   route_top_k_kernel<T, R><<<blocks, threads, lds_for(R), stream>>>((const T*)x, x_stride, router, correction, gate_row, \
                                                                     chosen, weights, shared_gate, num_tokens, width,    \

@@ -1242,3 +1242,17 @@ def test_few_rows_of_gemm_f32_off_whole_lines(m, n, k):
         assert torch.equal(ops.gemm_f32(off_a, off_w), out), (before_a, before_w)
     many = torch.cat([a, torch.ones(70, k, device=DEV)])
     assert torch.equal(ops.gemm_f32(many, w)[:m], out)
+
+
+@pytest.mark.parametrize("tokens,width", [(1025, 512), (2049, 512), (2051, 6000)])
+def test_router_block_sizes_give_the_same_bits(tokens, width):
+    """Sixteen, ten and four waves a block, by how many blocks there are and how much LDS one takes."""
+    from mini_infer_amd import ops
+
+    x, router = _rand(tokens, width, dtype=torch.bfloat16, seed=51), _rand(10, width, seed=52, scale=0.05)
+    chosen, weights, _ = ops.route_top_k(x, router, None, None, top=3, route_scale=1.0)
+    for at in range(0, tokens, 500):
+        some, their, _ = ops.route_top_k(x[at : at + 500], router, None, None, top=3, route_scale=1.0)
+        assert torch.equal(chosen[at : at + 500], some) and torch.equal(weights[at : at + 500], their)
+    want = torch.softmax(x.double() @ router.double().T, 1).gather(1, chosen.long())
+    assert ((weights.double() - want).abs() <= 1e-5 * want).all()  # float32 sums of `width` products, and exponentials of them
