@@ -165,7 +165,7 @@ __global__ __launch_bounds__(256) void head_norm_rope_kv_write_vec_kernel(
   if (slot < 0) return;
   const int first = blockIdx.y * blockDim.x + threadIdx.x, stride = gridDim.y * blockDim.x;
   const int v_col = (q_heads + kv_heads) * head_dim;
-  if (v_transposed && mi_fills_page(slot_mapping, t, page, off, page_size, gridDim.x)) {
+  if (v_transposed && (int)gridDim.x >= MI_LOOK_FOR_PAGES && mi_fills_page(slot_mapping, t, page, off, page_size, gridDim.x)) {
     mi_write_page_rows(v_pages, t, page, off, page_size, kv_heads, v_dim, first, stride,
                        [&](int token, int e) { return to_f32(qkv[(int64_t)token * row_stride + v_col + e]); });
     return;

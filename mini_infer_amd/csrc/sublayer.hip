@@ -750,7 +750,7 @@ __global__ __launch_bounds__(1024) void qkv_norm_write_kernel(
     store_cols<T, VEC>(k_pages + (((int64_t)page * kv_heads + h) * page_size + off) * head_dim + d, raw);
   }
   const A lam = (other != nullptr) ? (A)mix[0] : (A)0;
-  if (v_transposed && VEC > 1 && mi_fills_page(slot_mapping, t, page, off, page_size, gridDim.x)) {
+  if (v_transposed && VEC > 1 && (int)gridDim.x >= MI_LOOK_FOR_PAGES && mi_fills_page(slot_mapping, t, page, off, page_size, gridDim.x)) {
     mi_write_page_rows(v_pages, t, page, off, page_size, kv_heads, v_dim, (int)threadIdx.x, (int)blockDim.x, [&](int token, int e) {
       const float own = to_f32(qkv[(int64_t)token * row_stride + q_width + k_width + e]);
       if (other == nullptr) return own;

@@ -1000,14 +1000,15 @@ def test_kernels_refuse_what_they_do_not_take():
 
 
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("tokens", [43, 150])  # (steps of fewer than 128 tokens do not look for pages)
 @pytest.mark.parametrize("q_heads,kv_heads,dim,rotary,vdim,page,first", [(24, 8, 128, 128, 128, 16, 13), (3, 2, 72, 8, 24, 8, 8),
                                                                        (2, 1, 264, 256, 36, 8, 3), (5, 5, 8, 0, 4, 16, 0)])
-def test_portions_that_fill_pages_write_what_single_tokens_write(dtype, q_heads, kv_heads, dim, rotary, vdim, page, first):
+def test_portions_that_fill_pages_write_what_single_tokens_write(dtype, tokens, q_heads, kv_heads, dim, rotary, vdim, page, first):
     """A page of transposed values that a step fills in order is written a dim's row at once, the others an element at a
     time; and a head by a part of a wave.  Token by token no page is filled: the same bits."""
     from mini_infer_amd import ops
 
-    tokens, q_width, k_width, v_width = 43, q_heads * dim, kv_heads * dim, kv_heads * vdim
+    q_width, k_width, v_width = q_heads * dim, kv_heads * dim, kv_heads * vdim
     rows = _rand(tokens, q_width + k_width + v_width, dtype=dtype, seed=3)
     angles, other = _rand(tokens, rotary // 2, seed=4), _rand(tokens, v_width, dtype=dtype, seed=5)
     q_weight, k_weight, mix = _rand(q_width, seed=6), _rand(k_width, seed=7), torch.tensor([0.3], device=DEV)
