@@ -395,13 +395,17 @@ __global__ __launch_bounds__(1024) void readout_gate_norm_kernel(const float* __
   A r;
   if constexpr (sizeof(A) == 8) r = 1.0 / sqrt(ss / (double)group_width + (double)eps);
   else r = 1.0f / sqrtf(ss / (float)group_width + eps);
+  int first_weight = c0 < group_width ? ((int)at + c0) % weight_period : 0;
+  const int weights_on = ONE ? 0 : step % weight_period;
   for (int c = c0; c < group_width; c += step) {
     if constexpr (!ONE) {
       mi_load_cols<float, V>(orow + c, y);
       mi_load_cols<T, V>(grow + c, z);
     }
     float res[V];
-    int of_weight = ((int)at + c) % weight_period;  // (one division; the next columns' count on)
+    int of_weight = first_weight;  // (one division; the next columns' count on)
+    first_weight += weights_on;
+    if (first_weight >= weight_period) first_weight -= weight_period;
 #pragma unroll
     for (int j = 0; j < V; ++j) {
       const A w = (A)weight[of_weight];
@@ -514,6 +518,7 @@ extern "C" int mi_readout_gate_norm(int dtype, const float* o, const void* gate,
 #define MI_READOUT_OF(TT)                   \
   if (wide && one) MI_READOUT(TT, 4, true); \
   else if (wide) MI_READOUT(TT, 4, false);  \
+  else if (one) MI_READOUT(TT, 1, true);    \
   else MI_READOUT(TT, 1, false)
   if (dtype == MI_F32) {
     MI_READOUT_OF(float);

@@ -1257,3 +1257,21 @@ def test_router_block_sizes_give_the_same_bits(tokens, width):
         assert torch.equal(chosen[at : at + 500], some) and torch.equal(weights[at : at + 500], their)
     want = torch.softmax(x.double() @ router.double().T, 1).gather(1, chosen.long())
     assert ((weights.double() - want).abs() <= 1e-5 * want).all()  # float32 sums of `width` products, and exponentials of them
+
+
+@pytest.mark.parametrize("groups,group,period", [(5, 63, 63), (3, 1023, 3069), (2, 1025, 1025), (3, 2050, 6150), (1, 4100, 41), (7, 9, 3), (2, 4096, 8192)])
+@pytest.mark.parametrize("gate_first", [False, True])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_readout_norm_groups_of_any_size(groups, group, period, gate_first, dtype):
+    """Groups that the threads hold at once and that they do not, by fours and by single columns, weights that wrap inside a group."""
+    from mini_infer_amd import ops
+
+    width = groups * group
+    o, gate, weight = _rand(5, width, seed=61), _rand(5, width + 1, dtype=dtype, seed=62)[:, 1:], 1 + 0.2 * _rand(period, seed=63)
+    got = ops.readout_gate_norm(o, gate, weight, group_width=group, gate_first=gate_first, eps=1e-5).double()
+    silu = gate.double() * torch.sigmoid(gate.double())
+    y = (o.double() * silu if gate_first else o.double()).view(5, groups, group)
+    y = (y / torch.sqrt((y * y).mean(-1, keepdim=True) + 1e-5)).view(5, width) * weight.double().repeat(width // period)
+    want = y if gate_first else y * silu
+    # one rounding to the element type, and a few float32 roundings before it
+    assert ((got - want).abs() <= (2.0 ** -8 if dtype == torch.bfloat16 else 1e-5) * want.abs() + 1e-6).all()
