@@ -2201,6 +2201,22 @@ def latent_expand_pages(
     return queries
 
 
+def latent_expand(
+    proj: torch.Tensor, k_up: torch.Tensor, v_up: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, *, heads: int,
+    dim: int, rot: int, vdim: int, r_col: int, down: torch.Tensor | None = None,
+) -> torch.Tensor:
+    """The same as one row [q | k | v] per token with `heads` heads of dim + rot columns each (values padded with zeros), for callers
+    that write pages of their own: pages of one token, put side by side."""
+    tokens, width = proj.shape[0], dim + rot
+    if vdim > width:
+        raise KernelShapeError(f"latent_expand: values of {vdim} do not fit heads of {width}")
+    keys, values = (torch.empty((tokens, heads, *last), dtype=proj.dtype, device=proj.device) for last in ((1, width), (width, 1)))
+    first = torch.arange(tokens, dtype=torch.int32, device=proj.device)
+    queries = latent_expand_pages(proj, k_up, v_up, cos, sin, keys, values, first, torch.ones_like(first), heads=heads, dim=dim, rot=rot,
+                                  vdim=vdim, r_col=r_col, down=down)
+    return torch.cat([queries[:, : heads * width], keys.flatten(1), values.flatten(1)], 1)
+
+
 PER_HEAD_MAX_ROWS = 256  # rows up to which the engine's own product head by head is taken
 
 

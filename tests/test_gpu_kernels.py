@@ -1275,3 +1275,33 @@ def test_readout_norm_groups_of_any_size(groups, group, period, gate_first, dtyp
     want = y if gate_first else y * silu
     # one rounding to the element type, and a few float32 roundings before it
     assert ((got - want).abs() <= (2.0 ** -8 if dtype == torch.bfloat16 else 1e-5) * want.abs() + 1e-6).all()
+
+
+@pytest.mark.parametrize("heads,dim,rot,vdim,spare", [(5, 128, 64, 128, 8), (3, 20, 12, 20, 0), (4, 64, 0, 30, 3), (2, 24, 8, 32, 1)])
+@pytest.mark.parametrize("apart", [False, True])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_latent_heads_as_one_row_a_token(heads, dim, rot, vdim, spare, apart, dtype):
+    from mini_infer_amd import ops
+
+    tokens, width = 37, dim + rot
+    held = _rand(tokens, spare + rot, dtype=dtype, seed=2)
+    proj = _rand(tokens, heads * width + (0 if apart else spare + rot), dtype=dtype, seed=1)
+    before, shared = proj.clone(), held[:, spare:] if apart else proj[:, heads * width + spare :]
+    k_up, v_up = _rand(tokens, heads * dim, dtype=dtype, seed=3), _rand(tokens, heads * vdim, dtype=dtype, seed=4)
+    angles = _rand(tokens, rot // 2, seed=5)
+    got = ops.latent_expand(proj, k_up, v_up, angles.cos(), angles.sin(), heads=heads, dim=dim, rot=rot, vdim=vdim,
+                            r_col=spare if apart else heads * width + spare, down=held if apart else None)
+    assert torch.equal(proj, before) and got.shape == (tokens, 3 * heads * width)
+
+    def turned(x):  # [tokens, heads, rot], pairs side by side
+        pairs, cos, sin = x.double().unflatten(-1, (rot // 2, 2)), angles.double().cos()[:, None], angles.double().sin()[:, None]
+        return torch.stack((pairs[..., 0] * cos - pairs[..., 1] * sin, pairs[..., 1] * cos + pairs[..., 0] * sin), -1).flatten(-2)
+
+    q, k, v = got.double().view(tokens, 3, heads, width).unbind(1)
+    want_q = before[:, : heads * width].double().view(tokens, heads, width)
+    assert torch.equal(q[..., :dim], want_q[..., :dim]) and torch.equal(k[..., :dim], k_up.double().view(tokens, heads, dim))
+    assert torch.equal(v[..., :vdim], v_up.double().view(tokens, heads, vdim)) and (v[..., vdim:] == 0).all()
+    for made, source in ((q, want_q[..., dim:]), (k, shared[:, None].expand(tokens, heads, rot))):
+        want = turned(source)
+        # one rounding to the element type, of sums of two float32 products with float32 sines
+        assert ((made[..., dim:] - want).abs() <= (2.0 ** -8 if dtype == torch.bfloat16 else 1e-6) * (want.abs() + 1)).all()
