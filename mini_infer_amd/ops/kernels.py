@@ -2150,7 +2150,7 @@ def latent_prepare(
 def latent_expand_pages(
     proj: torch.Tensor, k_up: torch.Tensor, v_up: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, k_pages: torch.Tensor,
     v_pages: torch.Tensor, page_first: torch.Tensor, page_tokens: torch.Tensor, *, heads: int, dim: int, rot: int, vdim: int,
-    r_col: int, down: torch.Tensor | None = None,
+    r_col: int, down: torch.Tensor | None = None, in_place: bool = False,
 ) -> torch.Tensor:
     """Keys and values of a latent attention layer written out per head into pages that hold the step's tokens alone, and the
     queries rotated: what the paged attention kernels take.
@@ -2161,8 +2161,8 @@ def latent_expand_pages(
     rest zeros) are written whole, slots without a token with zeros.  `page_first`, `page_tokens` (int32): per page its first
     token and how many it holds (1 to page_size); together all tokens, each in one page.
 
-    Returns rows [T, >= heads * (dim + rot)] with the rotated queries in the first columns: `proj` itself, rotated in place,
-    where its rows allow 16-byte accesses, else rows of their own."""
+    Returns rows [T, >= heads * (dim + rot)] with the rotated queries in the first columns.  `in_place`: the caller has no more use
+    for the queries as they are; `proj` itself is returned, rotated in place, where its rows allow 16-byte accesses."""
     _need_cuda(proj, k_up, v_up, cos, sin, k_pages, v_pages, page_first, page_tokens)
     for name, t in (("proj", proj), ("k_up", k_up), ("v_up", v_up), ("down", proj if down is None else down)):
         if t.dim() != 2 or t.stride(1) != 1 or t.dtype != proj.dtype or t.shape[0] != proj.shape[0]:
@@ -2188,9 +2188,9 @@ def latent_expand_pages(
     if page_first.numel() != pages or page_tokens.numel() != pages:
         raise KernelShapeError("latent_expand_pages: one first token and one count per page")
     shared = holds_shared[:, r_col:]
-    in_eights = all(n % 8 == 0 for n in (dim, rot, page_size, proj.stride(0), shared.stride(0), k_up.stride(0))) and all(
+    in_place = in_place and all(n % 8 == 0 for n in (dim, rot, page_size, proj.stride(0), shared.stride(0), k_up.stride(0))) and all(
         t.data_ptr() % 16 == 0 for t in (proj, shared, k_up, cos, sin, k_pages, v_pages))
-    queries = proj if in_eights else torch.empty((tokens, heads * width), dtype=proj.dtype, device=proj.device)
+    queries = proj if in_place else torch.empty((tokens, heads * width), dtype=proj.dtype, device=proj.device)
     library.check(
         library.load().mi_latent_expand_pages(
             _dtype_code(proj), _ptr(proj), proj.stride(0), shared.data_ptr(), shared.stride(0), _ptr(k_up), k_up.stride(0),

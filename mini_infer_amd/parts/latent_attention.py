@@ -206,7 +206,7 @@ class LatentAttention(Mixer):
         v_own = torch.empty((page_first.numel(), heads, v_width, ctx.page_size), dtype=proj.dtype, device=proj.device)
         queries = ops.latent_expand_pages(
             proj, self.up_k.forward(latent), self.up_v.forward(latent), rotary.cos, rotary.sin, k_own, v_own, page_first, page_tokens,
-            heads=heads, dim=dim, rot=rot, vdim=vdim, r_col=c_col + rank, down=down,
+            heads=heads, dim=dim, rot=rot, vdim=vdim, r_col=c_col + rank, down=down, in_place=True,
         )
         mixed = ops.paged_attention(
             queries, k_own, v_own, table, ctx.token_request, ctx.positions, ctx.cu_seqlens_q, ctx.host_cu_seqlens_q, q_heads=heads,

@@ -1305,3 +1305,24 @@ def test_latent_heads_as_one_row_a_token(heads, dim, rot, vdim, spare, apart, dt
         want = turned(source)
         # one rounding to the element type, of sums of two float32 products with float32 sines
         assert ((made[..., dim:] - want).abs() <= (2.0 ** -8 if dtype == torch.bfloat16 else 1e-6) * (want.abs() + 1)).all()
+
+
+@pytest.mark.parametrize("dim,spare", [(128, 0), (20, 0), (128, 3)])
+def test_latent_queries_are_rotated_in_place_only_when_asked_to(dim, spare):
+    """The same bits either way; without `in_place` the projections stay as they are, whatever their alignment."""
+    from mini_infer_amd import ops
+
+    heads, rot, tokens, page = 3, 64, 21, 16
+    proj = _rand(tokens, heads * (dim + rot) + rot + spare, dtype=torch.bfloat16, seed=1)[:, spare:]
+    before, angles = proj.clone(), _rand(tokens, rot // 2, seed=5)
+    k_up, v_up = (_rand(tokens, heads * dim, dtype=torch.bfloat16, seed=s) for s in (3, 4))
+    ints = lambda x: torch.tensor(x, dtype=torch.int32, device=DEV)  # noqa: E731
+    made = []
+    for in_place in (False, True):
+        k_pages, v_pages = (torch.zeros(2, heads, *shape, dtype=torch.bfloat16, device=DEV) for shape in ((page, dim + rot), (dim, page)))
+        rows = ops.latent_expand_pages(proj, k_up, v_up, angles.cos(), angles.sin(), k_pages, v_pages, ints([0, 16]), ints([16, 5]), heads=heads,
+                                       dim=dim, rot=rot, vdim=dim, r_col=heads * (dim + rot), in_place=in_place)
+        made.append((rows[:, : heads * (dim + rot)].clone(), k_pages, v_pages))
+        if not in_place:
+            assert torch.equal(proj, before)
+    assert all(torch.equal(a, b) for a, b in zip(*made))
