@@ -8,7 +8,8 @@ import torch
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
-SIZES = [([32, 31, 33, 1], 4, 2, 64, 64), ([200], 2, 2, 128, 128), ([97, 64, 5], 6, 3, 96, 80), ([129], 2, 1, 256, 250), ([65, 100], 3, 3, 20, 30)]
+SIZES = [([32, 31, 33, 1], 4, 2, 64, 64), ([200], 2, 2, 128, 128), ([97, 64, 5], 6, 3, 96, 80), ([129], 2, 1, 256, 250), ([65, 100], 3, 3, 20, 30),
+         ([0, 70, 0, 33, 0], 18, 2, 64, 40)]  # (requests without tokens; more heads that share keys than a block takes at once)
 
 
 def _rel(got, exact):
@@ -31,15 +32,27 @@ def _rows(generator, tokens, width, odd):
     return wide[:, 3:] if odd else wide
 
 
+def _calls_in_chunks(monkeypatch):
+    """A list that grows by one with every call of the chunks' entry points."""
+    from mini_infer_amd.ops import library
+
+    lib, calls = library.load(), []
+    for name in ("mi_gated_delta_chunks", "mi_decay_scan_chunks"):
+        entry = getattr(lib, name)
+        monkeypatch.setattr(lib, name, lambda *args, entry=entry: (calls.append(1), entry(*args))[1])
+    return calls
+
+
 def _both(monkeypatch, call, state):
     """What `call(state)` gives in chunks and token by token, with the state each leaves."""
     from mini_infer_amd.ops import kernels
 
-    made = []
+    made, calls = [], _calls_in_chunks(monkeypatch)
     for chunks in (True, False):
-        monkeypatch.setattr(kernels, "chunked_scan_pays", lambda tokens, requests, widest, chunks=chunks: chunks)
+        monkeypatch.setattr(kernels, "chunked_scan_pays", lambda walked, chunked, widest, chunks=chunks: chunks)
         left = state.clone()
         made.append((call(left), left))
+        assert len(calls) == 1  # (the first call in chunks indeed, the second not)
     return made
 
 
@@ -263,12 +276,8 @@ def test_what_is_not_finite_goes_token_by_token(monkeypatch, kind, what, dim, vd
 def test_which_steps_go_in_chunks(monkeypatch, kind, lengths, known, chunks):
     """The rule by itself, on both sides of its line, with what the host knows of the portions and without."""
     from mini_infer_amd import ops
-    from mini_infer_amd.ops import library
 
-    lib, calls = library.load(), []
-    for name in ("mi_gated_delta_chunks", "mi_decay_scan_chunks"):
-        entry = getattr(lib, name)
-        monkeypatch.setattr(lib, name, lambda *args, entry=entry: (calls.append(1), entry(*args))[1])
+    calls = _calls_in_chunks(monkeypatch)
     heads, groups, dim, vdim, tokens = 16, 16, 128, 128, sum(lengths)
     cu, slots = _boundaries(lengths), torch.arange(len(lengths), dtype=torch.int32, device=DEV)
     rows = lambda n: torch.zeros(tokens, n, dtype=torch.bfloat16, device=DEV)  # noqa: E731
