@@ -31,9 +31,10 @@
 // as the products with the state, and the inverse no longer stays in a wave's registers.
 //
 // Only finite numbers may be taken like this: the zeros of W and T above the diagonal make NaN of an infinite value, for
-// tokens before it, and quotients behind a decay of zero are infinity less infinity.  So each wave adds up zero times
+// tokens before it, quotients behind a decay of zero are infinity less infinity, and a chunk's decays together may be zero, which
+// makes NaN of an infinite state that each by itself leaves infinite.  So each wave adds up zero times
 // (G_last / G) U, which is the same in all four and holds whatever was not finite in values, gates, and (for the delta rule by
-// itself, else through the factors) queries and keys; if that is not zero at the end the block leaves the state as it found it
+// itself, else through the factors and Q S0) queries, keys and the state; if that is not zero at the end the block leaves the state as it found it
 // and sets its flag, and a last launch takes the flagged columns again with the token-by-token kernel.  That launch costs 3 us
 // where nothing is flagged; a verdict at the end of a block that needed a barrier cost another 0.3 us a block.
 #pragma once
@@ -279,10 +280,11 @@ __global__ __launch_bounds__(256, MODE == DELTA || DT > 2 ? 1 : 2) void walk_ker
       }
       g_last = both.factor[CHUNK - 1];
     }
-    if constexpr (MODE == PER_CHANNEL) zeros[0] += both.factor[0];
     auto whole = [&](int t) {
       return (parts[n & 1][0][t][lane] + parts[n & 1][1][t][lane]) + (parts[n & 1][2][t][lane] + parts[n & 1][3][t][lane]);
     };
+    if constexpr (MODE == PER_CHANNEL) zeros[0] += both.factor[0];
+    if constexpr (MODE != DELTA) zeros[0] = fmaf(0.f, whole(0)[0], zeros[0]);  // (any token's: each meets all rows of S)
     f32x4_t u[2] = {v[0], v[1]};
     if constexpr (MODE == DELTA) {
 #pragma unroll

@@ -227,7 +227,7 @@ def test_a_rest_of_more_values_than_32_bits_count(kind):
 
 
 @pytest.mark.parametrize("dim,vdim", [(40, 64), (128, 128), (256, 250)])
-@pytest.mark.parametrize("what", ["value inf", "value nan", "k inf", "q inf", "state inf", "gate inf", "gate -inf", "gate nan"])
+@pytest.mark.parametrize("what", ["value inf", "value nan", "k inf", "q inf", "state inf", "state inf forgotten", "gate inf", "gate -inf", "gate nan"])
 @pytest.mark.parametrize("kind", ["delta", "per_head", "per_channel"])
 def test_what_is_not_finite_goes_token_by_token(monkeypatch, kind, what, dim, vdim):
     """A value, key, query, state or gate in the middle of a chunk that is no finite number reaches what it reaches in the
@@ -242,7 +242,9 @@ def test_what_is_not_finite_goes_token_by_token(monkeypatch, kind, what, dim, vd
     gate = torch.randn(tokens, per_channel, generator=g, device=DEV).bfloat16()
     shape = ops.delta_state_shape(heads, dim, vdim) if kind == "delta" else ops.decay_state_shape(heads, dim, vdim)
     state = _state(g, requests, shape, dim)
-    name, bad = what.split()
+    name, bad, *forgotten = what.split()
+    if forgotten:  # (a chunk's decays together are zero in float32, none of them by itself)
+        gate[50:] = 40.0 if kind != "per_channel" else -100.0
     if name == "state":
         state[1, 1, column, 3] = float(bad)
     else:
