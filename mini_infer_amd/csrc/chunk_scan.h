@@ -32,11 +32,12 @@
 //
 // Only finite numbers may be taken like this: the zeros of W and T above the diagonal make NaN of an infinite value, for
 // tokens before it, quotients behind a decay of zero are infinity less infinity, and a chunk's decays together may be zero, which
-// makes NaN of an infinite state that each by itself leaves infinite.  So each wave adds up zero times
-// (G_last / G) U, which is the same in all four and holds whatever was not finite in values, gates, and (for the delta rule by
-// itself, else through the factors and Q S0) queries, keys and the state; if that is not zero at the end the block leaves the state as it found it
-// and sets its flag, and a last launch takes the flagged columns again with the token-by-token kernel.  That launch costs 3 us
-// where nothing is flagged; a verdict at the end of a block that needed a barrier cost another 0.3 us a block.
+// makes NaN of an infinite state that each by itself leaves infinite.  Whatever is not finite in the state, the values, the
+// gates, and (for the delta rule by itself, else through the factors) in queries and keys stays in S to the end: products with
+// zero keep it.  So where a block's S does not end finite it leaves the state as it found it and sets its flag, and a last
+// launch takes the flagged columns again with the token-by-token kernel.  That launch costs 3 us where nothing is flagged, and the
+// barrier at a block's end 0.3 us; sums of what a chunk adds and of Q S0, the same in all waves and without a barrier, cost more
+// (77.6 us for the 70 of a decay per head).
 #pragma once
 #include "common.h"
 
@@ -55,9 +56,9 @@ struct Made {
   float* kt;      // [chunks][shares][pad][CHUNK]; PER_CHANNEL: times G_last / G_j
   float* within;  // W [chunks][heads][CHUNK][CHUNK]; PER_HEAD: for U = V, its columns times the step sizes
   float* solve;   // T w, the same (DELTA only)
-  float* factor;  // [chunks][heads][2][CHUNK]: G, and G_last / G (PER_HEAD: times the step sizes); PER_CHANNEL [chunks][heads]: 0
-                  // (NaN: of a token, or PER_CHANNEL of a chunk, whose query, key or decay is not finite)
-  float* fade;    // G_last: PER_CHANNEL [chunks][heads][pad]
+  float* factor;  // G, and G_last / G (PER_HEAD: times the step sizes, NaN of a token whose query or key is not finite)
+                  // [chunks][heads][2][CHUNK]; not PER_CHANNEL
+  float* fade;    // G_last: PER_CHANNEL [chunks][heads][pad]; NaN where a query, key or decay of the chunk is not finite
   int shares;     // rows q and k are shared by heads / shares heads
 };
 
@@ -145,7 +146,7 @@ struct Operands {
   float4 q[2][DT], k[MODE == DELTA ? 2 : 1][DT], kt[2][DT];
   float4 fade[MODE == PER_CHANNEL ? DT : 1];
   float4 within, solve;  // four values of a row of W and of T
-  float factor;          // one of the 64 factors; PER_CHANNEL: the chunk's only one
+  float factor;          // one of the 64 factors
   uint32_t v[2];         // two columns of a token's values, as read
 };
 
@@ -190,7 +191,6 @@ __global__ __launch_bounds__(256, MODE == DELTA || DT > 2 ? 1 : 2) void walk_ker
   const int share = head / (p.heads / p.made.shares);
   const int chunk0 = first_chunk(first, b), chunks = (last - first + CHUNK - 1) / CHUNK;
   const float skip = (MODE == PER_HEAD && p.skip) ? p.skip[head] : 0.f;
-  float zeros[2] = {0.f, 0.f};  // unless something is not finite
   const int out_stride = p.heads * p.vdim;
   // a lane's offsets
   const uint32_t at_row = r * PAD + 4 * quad, at_column = r * CHUNK + 4 * quad, in_lds = r * LDS_ROW + 4 * quad;
@@ -224,7 +224,6 @@ __global__ __launch_bounds__(256, MODE == DELTA || DT > 2 ? 1 : 2) void walk_ker
       const float* fade = p.made.fade + of * PAD + row0;
 #pragma unroll
       for (int d = 0; d < DT; ++d) o.fade[d] = load4(fade + 16 * d + 4 * quad);
-      o.factor = p.made.factor[of];
     } else {
       o.factor = p.made.factor[of * 2 * CHUNK + lane];
     }
@@ -257,8 +256,6 @@ __global__ __launch_bounds__(256, MODE == DELTA || DT > 2 ? 1 : 2) void walk_ker
     if constexpr (MODE == DELTA) *reinterpret_cast<float4*>(&both.solve[piece]) = o.solve;
     if constexpr (MODE != PER_CHANNEL) {
       if (wave == 0) both.factor[lane] = o.factor;
-    } else if (threadIdx.x == 0) {
-      both.factor[0] = o.factor;
     }
     {  // (of tokens past the last one zeros, by their bits: a choice would be compiled into a branch around the load, and every
        // load waited for by itself)
@@ -283,8 +280,6 @@ __global__ __launch_bounds__(256, MODE == DELTA || DT > 2 ? 1 : 2) void walk_ker
     auto whole = [&](int t) {
       return (parts[n & 1][0][t][lane] + parts[n & 1][1][t][lane]) + (parts[n & 1][2][t][lane] + parts[n & 1][3][t][lane]);
     };
-    if constexpr (MODE == PER_CHANNEL) zeros[0] += both.factor[0];
-    if constexpr (MODE != DELTA) zeros[0] = fmaf(0.f, whole(0)[0], zeros[0]);  // (any token's: each meets all rows of S)
     f32x4_t u[2] = {v[0], v[1]};
     if constexpr (MODE == DELTA) {
 #pragma unroll
@@ -298,8 +293,6 @@ __global__ __launch_bounds__(256, MODE == DELTA || DT > 2 ? 1 : 2) void walk_ker
     for (int t = 0; t < 2; ++t) {
       if constexpr (MODE == PER_CHANNEL) tail[t] = u[t];
       else tail[t] = scaled(tails[t], u[t]);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) zeros[t] = fmaf(0.f, tail[t][e], zeros[t]);
     }
 #pragma unroll
     for (int d = 0; d < DT; ++d) {
@@ -333,7 +326,10 @@ __global__ __launch_bounds__(256, MODE == DELTA || DT > 2 ? 1 : 2) void walk_ker
     step(n + 1, odd);
   }
   if (chunks & 1) step(chunks - 1, even);
-  const bool again = __ballot(!(zeros[0] + zeros[1] == 0.f)) != 0;  // (the same in all waves: so are all that zeros were made of)
+  f32x4_t zeros = {0.f, 0.f, 0.f, 0.f};  // unless something is not finite
+#pragma unroll
+  for (int d = 0; d < DT; ++d) zeros += 0.f * S[d];
+  const bool again = __syncthreads_or(!((zeros[0] + zeros[1]) + (zeros[2] + zeros[3]) == 0.f));
   if (threadIdx.x == 0) *flag = again;
   if (live && !again) {
 #pragma unroll

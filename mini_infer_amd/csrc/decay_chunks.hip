@@ -143,7 +143,6 @@ __global__ __launch_bounds__(256) void channel_decay_chunk_kernel(RowArgs p, Mad
     odd = !(zeros == 0.f);
   }
   odd = __syncthreads_or(odd);
-  if (tid == 0) made.factor[(int64_t)chunk * p.heads + head] = odd ? NAN : 0.f;
   for (int d = tid; d < PAD; d += 256) {
     const int64_t of = (int64_t)chunk * made.shares + head;  // (rows of a head of its own)
     double product = 1.0, tail = 1.0;  // (rounded once, where they are used)
@@ -152,7 +151,7 @@ __global__ __launch_bounds__(256) void channel_decay_chunk_kernel(RowArgs p, Mad
       product *= (double)a_s[i * ROW + d];
       made.q[(of * CHUNK + i) * PAD + d] = (float)((double)q_s[i * ROW + d] * product);
     }
-    made.fade[((int64_t)chunk * p.heads + head) * PAD + d] = (float)product;
+    made.fade[((int64_t)chunk * p.heads + head) * PAD + d] = odd ? NAN : (float)product;
     float four[4];
     float* kt = made.kt + (of * PAD + d) * CHUNK;
 #pragma unroll
@@ -203,7 +202,7 @@ extern "C" int64_t mi_decay_scan_chunks_scratch(int mode, int num_tokens, int nu
   const int pad = mi_decay_scan_dim_pad(dim);
   if (num_tokens <= 0 || num_requests <= 0 || num_requests > 65535 || dim > 256 || pad < 64 || heads <= 0 || heads > 65535 || groups <= 0 || vdim <= 0) return 0;
   return chunk_count(num_tokens, num_requests) * ((int64_t)2 * made_shares(mode, heads, groups) * CHUNK * pad +
-                                                  (int64_t)heads * (CHUNK * CHUNK + (mode == PER_CHANNEL ? pad + 1 : 2 * CHUNK))) +
+                                                  (int64_t)heads * (CHUNK * CHUNK + (mode == PER_CHANNEL ? pad : 2 * CHUNK))) +
          flag_count(num_requests, heads, vdim);
 }
 
@@ -228,7 +227,7 @@ extern "C" int mi_decay_scan_chunks(int mode, const void* q, int64_t q_stride, i
   made.fade = made.within + chunks * heads * CHUNK * CHUNK;
   made.factor = made.fade + (mode == PER_CHANNEL ? chunks * heads * pad : 0);
   made.k = made.solve = nullptr;
-  int* again = reinterpret_cast<int*>(made.factor + chunks * heads * (mode == PER_CHANNEL ? 1 : 2 * CHUNK));
+  int* again = reinterpret_cast<int*>(made.factor + (mode == PER_CHANNEL ? 0 : chunks * heads * 2 * CHUNK));
   made.shares = made_shares(mode, heads, groups);
   RowArgs a;
   a.q = (const bf16_t*)q, a.k = (const bf16_t*)k, a.gate = (const bf16_t*)gate;
