@@ -14,7 +14,7 @@ from pathlib import Path
 from mini_infer_amd.exceptions import ExtensionMissingError, KernelShapeError
 from mini_infer_amd.ops import build as _build
 
-ABI_VERSION = 37
+ABI_VERSION = 38
 
 _lib: ctypes.CDLL | None = None
 _lib_path: Path | None = None
@@ -177,11 +177,14 @@ _SIGNATURES: dict[str, list] = {
 _INT64_RESULTS = {"mi_gated_delta_chunks_scratch", "mi_decay_scan_chunks_scratch", "mi_attn_prompt_f32_blocks"}  # (sizes; every other entry point returns an int status)
 
 
-def _declare(lib: ctypes.CDLL) -> None:
+def _declare(lib: ctypes.CDLL, path: Path) -> None:
+    found = lib.mi_abi_version()  # (an int without arguments, as undeclared functions are; an older library may lack others)
+    if found != ABI_VERSION:
+        raise ExtensionMissingError(
+            f"{path} has ABI version {found}, this package needs {ABI_VERSION}; rebuild it"
+        )
     lib.mi_last_error.restype = ctypes.c_char_p
     lib.mi_last_error.argtypes = []
-    lib.mi_abi_version.restype = c_int
-    lib.mi_abi_version.argtypes = []
     for name, argtypes in _SIGNATURES.items():
         fn = getattr(lib, name)
         fn.restype = c_int64 if name in _INT64_RESULTS else c_int
@@ -212,12 +215,7 @@ def load(rebuild_if_stale: bool = True) -> ctypes.CDLL:
         lib = ctypes.CDLL(str(path))
     except OSError as err:
         raise ExtensionMissingError(f"cannot load {path}: {err}") from err
-    _declare(lib)
-    found = lib.mi_abi_version()
-    if found != ABI_VERSION:
-        raise ExtensionMissingError(
-            f"{path} has ABI version {found}, this package needs {ABI_VERSION}; rebuild it"
-        )
+    _declare(lib, path)
     _lib, _lib_path = lib, path
     return lib
 
