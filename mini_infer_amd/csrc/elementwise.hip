@@ -166,7 +166,7 @@ extern "C" int mi_begin_step(int* ids, const int* from_rows, const int* source, 
 //   out[b] = weight * s * rsqrt(mean(s^2) + eps)
 // One block per output row; with `rows`, output row b reads input row rows[b].
 // The delta may come in pieces: `partials` [num_partials][all rows][hidden] float32, the
-// sums of a product over ranges of K (gemm_mid_bf16.hip); they are added in order and
+// sums of a product over ranges of K (gemm_tiles_bf16.hip); they are added in order and
 // rounded to T, which gives the delta the product would have written itself.
 // ---------------------------------------------------------------------------
 

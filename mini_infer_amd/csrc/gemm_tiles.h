@@ -1,0 +1,126 @@
+// The kernel of gemm_tiles_bf16.hip and gemm_tiles_gated_bf16.hip, and the shapes that they compile it for.
+#pragma once
+
+#include "tile_product.h"
+
+// Of the 20 shapes measured those that are the best anywhere by more than 1 %.
+#define GEMM_TILE_SHAPES(X) \
+  X(1, 2, 2, 2, 2, 6)  /* 32 x 64 */ \
+  X(1, 4, 2, 2, 2, 6)  /* 32 x 128 */ \
+  X(1, 2, 2, 3, 2, 5)  /* 48 x 64 */ \
+  X(1, 2, 2, 4, 2, 5)  /* 64 x 64 */ \
+  X(1, 4, 2, 4, 2, 6)  /* 64 x 128 */ \
+  X(1, 2, 2, 5, 2, 4)  /* 80 x 64 */ \
+  X(2, 2, 2, 3, 2, 6)  /* 96 x 64 */ \
+  X(1, 4, 2, 6, 2, 5)  /* 96 x 128 */ \
+  X(2, 2, 2, 4, 2, 6)  /* 128 x 64 */ \
+  X(2, 2, 2, 4, 4, 5)  /* 128 x 128 */ \
+  X(1, 4, 2, 9, 2, 4)  /* 144 x 128 */ \
+  X(2, 4, 1, 5, 4, 3)  /* 160 x 256 */ \
+  X(2, 2, 2, 6, 4, 3)  /* 192 x 128 */ \
+  X(2, 4, 1, 8, 4, 2)  /* 256 x 256 */
+#define GEMM_TILE_ODD_SHAPE 1, 2, 2, 4, 2, 5  // of a K of odd 32s
+
+// pieces of 32 of K of range `range` of `ranges`, and the first of them; ranges are whole steps of 64
+struct KRange {
+  int first, halves;
+};
+__host__ __device__ __forceinline__ KRange k_range(int k, int steps_each, int range) {
+  const int first = range * steps_each * 2;
+  return {first, min(steps_each * 2, k / 32 - first)};
+}
+
+// (the second bound: two blocks a CU where LDS holds two)
+template <class T, bool GATED, bool ONCE, bool ODD>
+__global__ __launch_bounds__(T::THREADS, T::RING * 4 <= 163840 ? 2 : 1) void gemm_tiles_kernel(
+    const bf16_t* __restrict__ a, int64_t lda, const bf16_t* __restrict__ w, int64_t ldw, void* __restrict__ out, int64_t ldc,
+    int kind, float scale, bool vec, int m, int n, int k, int steps_each, int row_tiles, int feature_tiles, int total) {
+  __shared__ __align__(16) bf16_t ring[T::RING];
+  // Consecutive places go to one XCD (workgroups are dealt to the 8 of them in turn): the row tiles that read the same
+  // rows of W run at the same time behind one L2.
+  const int place = (blockIdx.x % 8) * (gridDim.x / 8) + blockIdx.x / 8;
+  if (place >= total) return;
+  const int row_tile = place % row_tiles, rest = place / row_tiles;
+  const int feature_tile = rest % feature_tiles, range = rest / feature_tiles;
+  const KRange part = k_range(k, steps_each, range);
+  constexpr int FEATURES = GATED ? T::BN / 2 : T::BN;
+  const int r0 = row_tile * T::BM, f0 = feature_tile * FEATURES;
+  a += part.first * 32;
+  w += part.first * 32;
+  T tile;
+  tile.template run<ONCE, ODD>(
+      ring, part.halves, [&](int r) { return a + (int64_t)min(r0 + r, m - 1) * lda; },
+      [&](int r) {
+        if constexpr (GATED) {  // of a wave's tiles of W the first half are gate rows, the second the up rows of the same features
+          constexpr int HALF = T::NT / 2;
+          const int t = r / 16 % T::NT;
+          const int f = min(f0 + (r / (T::NT * 16) * HALF + t % HALF) * 16 + r % 16, n - 1);
+          return w + (int64_t)(t < HALF ? f : f + n) * ldw;
+        } else {
+          return w + (int64_t)min(f0 + r, n - 1) * ldw;
+        }
+      });
+#pragma unroll
+  for (int i = 0; i < T::MT; ++i) {
+    const int row = r0 + tile.row(i);
+    if (!tile.mine(i) || row >= m) continue;
+#pragma unroll
+    for (int j = 0; j < (GATED ? T::NT / 2 : T::NT); ++j) {
+      const int f = f0 + (GATED ? (tile.wn * (T::NT / 2) + j) * 16 + tile.quad * 4 : tile.feature(j));
+      float v[4];
+#pragma unroll
+      for (int c = 0; c < 4; ++c) {
+        v[c] = tile.acc[j][i][c];
+        if constexpr (GATED) {
+          const float g = to_f32(from_f32<bf16_t>(v[c])), u = to_f32(from_f32<bf16_t>(tile.acc[j + T::NT / 2][i][c]));
+          v[c] = g / (1.f + expf(-g)) * u;
+        } else if (kind == 2) {
+          v[c] = to_f32(from_f32<bf16_t>(v[c])) * scale;
+        }
+      }
+      const bool whole = vec && f + 4 <= n;
+      if (!GATED && kind != 0) {
+        float* o = kind == 1 ? (float*)out + ((int64_t)range * m + row) * n + f : (float*)out + (int64_t)row * ldc + f;
+        if (whole) {
+          mi_store_cols<float, 4>(o, v);
+        } else {
+#pragma unroll
+          for (int c = 0; c < 4; ++c)
+            if (f + c < n) o[c] = v[c];
+        }
+      } else {
+        bf16_t* o = (bf16_t*)out + (int64_t)row * ldc + f;
+        if (whole) {
+          mi_store_cols<bf16_t, 4>(o, v);
+        } else {
+#pragma unroll
+          for (int c = 0; c < 4; ++c)
+            if (f + c < n) o[c] = from_f32<bf16_t>(v[c]);
+        }
+      }
+    }
+  }
+}
+
+struct GemmTilesLaunch {
+  const void *a, *w;
+  void* out;
+  int64_t lda, ldw, ldc;
+  int kind;
+  float scale;
+  bool vec;
+  int m, n, k, steps_each;
+  hipStream_t stream;
+};
+
+template <class T, bool GATED, bool ODD>
+static void gemm_tiles_launch(const GemmTilesLaunch& l) {
+  const int row_tiles = ceil_div(l.m, T::BM), feature_tiles = ceil_div(l.n, GATED ? T::BN / 2 : T::BN);
+  const int total = row_tiles * feature_tiles * ceil_div(ceil_div(l.k, 64), l.steps_each);
+  const auto kernel = row_tiles == 1 ? gemm_tiles_kernel<T, GATED, true, ODD> : gemm_tiles_kernel<T, GATED, false, ODD>;
+  kernel<<<ceil_div(total, 8) * 8, T::THREADS, 0, l.stream>>>((const bf16_t*)l.a, l.lda, (const bf16_t*)l.w, l.ldw, l.out, l.ldc, l.kind,
+                                                             l.scale, l.vec, l.m, l.n, l.k, l.steps_each, row_tiles, feature_tiles, total);
+}
+
+// gemm_tiles_gated_bf16.hip
+void gemm_tiles_gated_launch(int shape, bool odd, const GemmTilesLaunch& l);

@@ -7,7 +7,9 @@ refuses a size.  There is no CPU path: a CPU tensor is an error.
 
 from __future__ import annotations
 
+import ctypes
 import dataclasses
+import functools
 import math
 
 import torch
@@ -400,6 +402,9 @@ def gemm_skinny_bf16(a: torch.Tensor, w: torch.Tensor) -> torch.Tensor:
     return c
 
 
+HEAD_TILES_MAX_ROWS = 256
+
+
 def linear_f32_out(x: torch.Tensor, weight: torch.Tensor, scale: float = 1.0, scale_row: torch.Tensor | None = None) -> torch.Tensor:
     """`x @ weight.T` as float32, times `scale`, whatever the operands' dtype: what an output head returns.
     `scale_row`: the scale once more as a float32 tensor of one entry on the device (with it the widening and
@@ -407,8 +412,9 @@ def linear_f32_out(x: torch.Tensor, weight: torch.Tensor, scale: float = 1.0, sc
 
     Few bfloat16 rows: the weight-streaming kernel writes float32 itself (no cast launch); its
     values are those of `linear(...).float()`, rounded to bfloat16 on the way, so that a row's
-    logits do not depend on how many rows its step had.  More rows: the vendor library's
-    product, cast.  float32 operands: `gemm_f32`."""
+    logits do not depend on how many rows its step had.  Up to 256 rows of a large vocabulary: the same values from tiles
+    (128256 x 3072 at 24 / 64 / 256 rows 140 / 164 / 210 us against the vendor product and its cast's 166 / 192 / 307).
+    More rows: the vendor library's product, cast.  float32 operands: `gemm_f32`."""
     if x.dtype == torch.float32:
         logits = gemm_f32(x, weight)
         return logits if scale == 1.0 else logits.mul_(scale)
@@ -433,6 +439,10 @@ def linear_f32_out(x: torch.Tensor, weight: torch.Tensor, scale: float = 1.0, sc
             )
         )
         return out
+    if x.dim() == 2 and SKINNY_MAX_ROWS < x.shape[0] <= HEAD_TILES_MAX_ROWS and weight.shape[0] >= 16000 and _rows_of_bf16(x, weight):
+        m, n = x.shape[0], weight.shape[0]
+        _, shape, _ = _tiles_plan(m, n, x.shape[1], False, 1, False, 0.0, 0.0)
+        return _tiles(2, x, weight, torch.empty((m, n), dtype=torch.float32, device=x.device), n, shape, 1, float(scale))
     product = torch.matmul(x, weight.t())
     if scale == 1.0:
         return product.float()
@@ -480,57 +490,125 @@ def partial_sums_pay(m: int, n: int, k: int) -> bool:
     return m > SKINNY_MAX_ROWS and n <= 4096 and 2048 <= k <= 4096
 
 
+@functools.lru_cache(maxsize=8192)
+def _tiles_plan(m: int, n: int, k: int, gated: bool, most_ranges: int, same_order: bool, sum_base: float, sum_each: float) -> tuple[float, int, int]:
+    """(microseconds expected, tile shape, ranges of K) of the best way to make a product in tiles (csrc/gemm_tiles_bf16.hip)."""
+    shape, ranges, micros = ctypes.c_int(), ctypes.c_int(), ctypes.c_float()
+    library.check(
+        library.load().mi_gemm_tiles_plan(m, n, k, int(gated), most_ranges, int(same_order), sum_base, sum_each,
+                                          ctypes.addressof(shape), ctypes.addressof(ranges), ctypes.addressof(micros))
+    )
+    return micros.value, shape.value, ranges.value
+
+
+def _rows_of_bf16(x: torch.Tensor, weight: torch.Tensor) -> bool:
+    """Whether both are matrices of bfloat16 rows on 16 bytes that fit one another, K in whole 32s."""
+    return (
+        x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and x.dim() == 2 and weight.dim() == 2
+        and x.shape[1] == weight.shape[1] and x.stride(1) == 1 and weight.stride(1) == 1 and x.shape[0] > 0 and weight.shape[0] > 0
+        and x.data_ptr() % 16 == 0 and weight.data_ptr() % 16 == 0
+        and bool(library.load().mi_gemm_tiles_take(x.shape[0], weight.shape[0], x.shape[1], x.stride(0), weight.stride(0)))
+    )
+
+
+def _tiles(kind: int, x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor, n: int, shape: int, ranges: int, scale: float = 1.0) -> torch.Tensor:
+    library.check(
+        library.load().mi_gemm_tiles_bf16(kind, _ptr(x), x.stride(0), _ptr(weight), weight.stride(0), _ptr(out), out.stride(-2), scale,
+                                          x.shape[0], n, x.shape[1], shape, ranges, _stream())
+    )
+    return out
+
+
 def linear_partial_sums(x: torch.Tensor, weight: torch.Tensor) -> PartialSums:
-    """`x @ weight.T` for up to 128 bfloat16 rows as float32 sums over ranges of K."""
+    """`x @ weight.T` for up to 128 bfloat16 rows as float32 sums over ranges of K; the ranges, and the order in which each is
+    summed, depend on the matrix alone."""
     _need_cuda(x, weight)
     if x.dtype != torch.bfloat16 or weight.dtype != torch.bfloat16 or x.dim() != 2 or weight.dim() != 2:
         raise KernelShapeError("linear_partial_sums takes 2-D bfloat16 tensors")
     m, k = x.shape
     n = weight.shape[0]
-    lib = library.load()
-    if (
-        weight.shape[1] != k
-        or x.stride(1) != 1
-        or weight.stride(1) != 1
-        or not lib.mi_gemm_mid_bf16_supported(m, n, k, x.stride(0), weight.stride(0))
-    ):
+    if not 1 <= m <= PARTIAL_SUMS_MAX_ROWS or not _rows_of_bf16(x, weight):
         raise KernelShapeError(
             f"linear_partial_sums takes 1 to 128 rows, K a multiple of 32, rows aligned to 16 bytes; "
             f"got x {tuple(x.shape)} strides {x.stride()}, weight {tuple(weight.shape)} strides {weight.stride()}"
         )
-    ranges = lib.mi_gemm_mid_bf16_ranges(n, k)
-    if ranges < 1:
-        raise KernelShapeError("linear_partial_sums: cannot read the device's compute unit count")
+    _, shape, ranges = _tiles_plan(m, n, k, False, 16, True, 0.0, 0.0)
     pieces = torch.empty((ranges, m, n), dtype=torch.float32, device=x.device)
-    library.check(
-        lib.mi_gemm_mid_partial_bf16(_ptr(x), x.stride(0), _ptr(weight), weight.stride(0), _ptr(pieces), m, n, k, _stream())
-    )
-    return PartialSums(pieces, torch.bfloat16)
+    return PartialSums(_tiles(1, x, weight, pieces, n, shape, ranges), torch.bfloat16)
+
+
+def sum_pieces(pieces: torch.Tensor) -> torch.Tensor:
+    """The sum over the first axis of contiguous float32 pieces, in order, as bfloat16."""
+    _need_cuda(pieces)
+    _need_contiguous("pieces", pieces)
+    if pieces.dtype != torch.float32 or pieces.dim() != 3 or pieces.numel() == 0:
+        raise KernelShapeError(f"sum_pieces takes float32 [pieces, rows, columns], got {tuple(pieces.shape)} {pieces.dtype}")
+    out = torch.empty(pieces.shape[1:], dtype=torch.bfloat16, device=pieces.device)
+    library.check(library.load().mi_sum_pieces(_ptr(pieces), _ptr(out), pieces.shape[0], out.numel(), _stream()))
+    return out
+
+
+SUM_LAUNCH_MICROS = 4.0  # of a launch that adds pieces up, beside their bytes
+SUM_BYTES_A_MICRO = 5e6
+TILES_MAX_ROWS = 1024
+
+
+@functools.lru_cache(maxsize=8192)
+def tiles_for(m: int, n: int, k: int, partial_ok: bool) -> tuple[int, int] | None:
+    """(tile shape, ranges of K) where a bfloat16 product of more rows than `gemm_skinny_bf16` takes is made in tiles; None: by the
+    vendor library.  Over 61 matrices (n 1024 to 28672, k 1536 to 14336) the tiles took, as a geometric mean of the library's time,
+    where the sum over ranges is left to the consumer / made here, its launch included:
+
+        rows           17    32    64    128   192   256   272   320   400   600   900
+        all in tiles   1.51  1.46  1.44  1.33  1.42  1.22  1.13  1.11  1.06  1.01  0.96
+                       1.22  1.17  1.20  1.19  1.33  1.17  1.08  1.06  1.04  0.99  0.95
+        by this rule   1.51  1.46  1.44  1.34  1.42  1.23  1.11  1.10  1.07  1.05  1.02
+                       1.17  1.16  1.16  1.19  1.29  1.18  1.07  1.06  1.05  1.04  1.02
+
+    The library does not cut K and so leaves CUs idle where there are few features; from 256 rows on it is about as fast as whole
+    tiles, and cutting has to pay.  It is faster (tiles 0.75 to 0.95) for the widest matrices, and where the whole product takes
+    it less than 9 microseconds and the sum needs a launch of its own."""
+    if not SKINNY_MAX_ROWS < m <= TILES_MAX_ROWS:
+        return None
+    if n >= 16000 and m > 80 or not partial_ok and n * k < 8_000_000:
+        return None
+    each = m * n * 4 / SUM_BYTES_A_MICRO
+    whole, _, _ = _tiles_plan(m, n, k, False, 1, False, 0.0, 0.0)
+    micros, shape, ranges = _tiles_plan(m, n, k, False, 16, False, 0.0 if partial_ok else SUM_LAUNCH_MICROS, each)
+    if m > 256 and micros > 0.88 * whole:
+        return None
+    return shape, ranges
+
+
+@functools.lru_cache(maxsize=8192)
+def gated_tiles_for(m: int, n: int, k: int) -> int | None:
+    """The tile shape where the gated product of n features is made in tiles, or None.  Up to 32 rows the streaming product
+    (`gemm_skinny_swiglu_bf16`) gives a row the same bits as it gets in a step of its own; tiles are not faster everywhere there (gate|up
+    at 24 rows: 16384 x 3072 19.8 against 23.9 us, 28672 x 4096 50.8 against 47.1).  Above, measured against the vendor product
+    and `silu_mul`, tiles are 1.0 to 1.9 times as fast up to 200 rows, and beyond as long as tiles of up to 192 x 128 are what pays
+    (7168 x 4096 at 256 / 600 rows 32.5 / 48.2 against 43.8 / 53.8, 16384 x 2048 at 271 / 320 29.4 / 30.8 against 33.3 /
+    33.9); where there is work for larger ones the library is faster by as much as 1.3."""
+    if not SKINNY_WIDE_MAX_ROWS < m <= 768:
+        return None
+    _, shape, _ = _tiles_plan(m, n, k, True, 1, False, 0.0, 0.0)
+    if m > 200 and library.load().mi_gemm_tiles_area(shape) > 192 * 128:
+        return None
+    return shape
 
 
 def linear(x: torch.Tensor, weight: torch.Tensor, partial_ok: bool = False) -> torch.Tensor | PartialSums:
     """`x @ weight.T` without bias.
 
-    float32 runs the hand-written true-float32 kernel.  bfloat16 with at most 16
-    rows (decode) runs the hand-written weight-streaming kernel; more rows go to
-    the vendor GEMM library through torch, as the reference's engine does
+    float32 runs the hand-written true-float32 kernel.  bfloat16 with at most 16 rows (decode) runs the hand-written
+    weight-streaming kernel, some tens to some hundreds of rows the tiles of `gemm_tiles_bf16` where they are faster
+    (`tiles_for`); the rest goes to the vendor GEMM library through torch, as the reference's engine does
     (distributed/linear.py:167, `F.linear` -> the vendor BLAS).
-    With `partial_ok` the result may come as `PartialSums` where that pays
-    (`partial_sums_pay`: up to 128 rows, few features, a long K).
+    With `partial_ok` the result may come as `PartialSums` where that pays.
     """
     if x.dtype == torch.float32:
         return gemm_f32(x, weight)
     _need_cuda(x, weight)
-    plain = x.dtype == torch.bfloat16 and weight.dtype == torch.bfloat16 and x.dim() == 2 and weight.dim() == 2
-    plain = plain and x.stride(1) == 1 and weight.stride(1) == 1 and weight.shape[1] == x.shape[1]
-    if (
-        partial_ok
-        and plain
-        and partial_sums_pay(x.shape[0], weight.shape[0], x.shape[1])
-        and x.shape[1] % 32 == 0
-        and x.stride(0) % 8 == 0
-        and weight.stride(0) % 8 == 0
-    ):
+    if partial_ok and x.dim() == 2 and weight.dim() == 2 and partial_sums_pay(x.shape[0], weight.shape[0], x.shape[1]) and _rows_of_bf16(x, weight):
         return linear_partial_sums(x, weight)
     if (
         x.dtype == torch.bfloat16
@@ -540,6 +618,14 @@ def linear(x: torch.Tensor, weight: torch.Tensor, partial_ok: bool = False) -> t
         and skinny_gemm_takes(x.shape[0], x.shape[1], x.stride(0), weight.stride(0))
     ):
         return gemm_skinny_bf16(x, weight)
+    if x.dim() == 2 and x.shape[0] <= TILES_MAX_ROWS and _rows_of_bf16(x, weight):
+        m, n = x.shape[0], weight.shape[0]
+        plan = tiles_for(m, n, x.shape[1], partial_ok)
+        if plan is not None:
+            if plan[1] == 1:
+                return _tiles(0, x, weight, torch.empty((m, n), dtype=torch.bfloat16, device=x.device), n, *plan)
+            pieces = _tiles(1, x, weight, torch.empty((plan[1], m, n), dtype=torch.float32, device=x.device), n, *plan)
+            return PartialSums(pieces, torch.bfloat16) if partial_ok else sum_pieces(pieces)
     return torch.matmul(x, weight.t())
 
 
@@ -664,8 +750,8 @@ def qkv_rope_write(
 def linear_swiglu(x: "torch.Tensor | ScaledRows", gate_up_weight: torch.Tensor) -> torch.Tensor:
     """`silu(x @ gate.T) * (x @ up.T)` with `gate_up_weight` = [gate; up] stacked, [2I, K].
 
-    bfloat16 with at most 32 rows runs as ONE hand-written kernel (the product with the
-    activation in its last step); otherwise the product and `silu_mul` run in turn.
+    bfloat16 with at most 32 rows, and up to some hundreds where that is faster (`gated_tiles_for`), runs as ONE
+    hand-written kernel (the product with the activation in its last step); otherwise the product and `silu_mul` run in turn.
     Both ways round the two products to the element type before the activation, so given
     the same rows a token's result does not depend on which one ran.  `x` may be
     `ScaledRows`: the rows' factors are then applied to the sums of the two products (the same
@@ -691,6 +777,12 @@ def linear_swiglu(x: "torch.Tensor | ScaledRows", gate_up_weight: torch.Tensor) 
             scaled, x = x, values
         else:
             x = x.finish()
+    if scaled is None and x.dim() == 2 and SKINNY_WIDE_MAX_ROWS < x.shape[0] <= TILES_MAX_ROWS and _rows_of_bf16(x, gate_up_weight):
+        _need_cuda(x, gate_up_weight)
+        m, n = x.shape[0], rows // 2
+        shape = gated_tiles_for(m, n, width)
+        if shape is not None:
+            return _tiles(3, x, gate_up_weight, torch.empty((m, n), dtype=torch.bfloat16, device=x.device), n, shape, 1)
     if (
         x.dtype == torch.bfloat16
         and gate_up_weight.dtype == torch.bfloat16

@@ -14,7 +14,7 @@ from pathlib import Path
 from mini_infer_amd.exceptions import ExtensionMissingError, KernelShapeError
 from mini_infer_amd.ops import build as _build
 
-ABI_VERSION = 38
+ABI_VERSION = 39
 
 _lib: ctypes.CDLL | None = None
 _lib_path: Path | None = None
@@ -34,9 +34,11 @@ _SIGNATURES: dict[str, list] = {
     "mi_gemm_f32": [_P, c_int64, _P, c_int64, _P, c_int64, c_int, c_int, c_int, _P],
     "mi_gemm_skinny_bf16": [_P, c_int64, _P, c_int64, _P, c_int64, c_int, c_int, c_int, _P],
     "mi_gemm_skinny_f32out_bf16": [_P, c_int64, _P, c_int64, _P, c_int64, c_int, c_int, c_int, c_float, _P],
-    "mi_gemm_mid_partial_bf16": [_P, c_int64, _P, c_int64, _P, c_int, c_int, c_int, _P],
-    "mi_gemm_mid_bf16_ranges": [c_int, c_int],
-    "mi_gemm_mid_bf16_supported": [c_int, c_int, c_int, c_int64, c_int64],
+    "mi_gemm_tiles_plan": [c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_float, _P, _P, _P],
+    "mi_gemm_tiles_area": [c_int],
+    "mi_gemm_tiles_take": [c_int, c_int, c_int, c_int64, c_int64],
+    "mi_gemm_tiles_bf16": [c_int, _P, c_int64, _P, c_int64, _P, c_int64, c_float, c_int, c_int, c_int, c_int, c_int, _P],
+    "mi_sum_pieces": [_P, _P, c_int, c_int64, _P],
     "mi_gemm_skinny_attn_bf16_supported": [c_int, c_int, c_int],
     "mi_gemm_skinny_attn_bf16": [_P, _P, c_int, c_int, c_int, _P, c_int64, _P, c_int64, c_int, c_int, _P],
     "mi_gemm_skinny_swiglu_bf16": [_P, c_int64, _P, c_int64, _P, c_int64, c_int, c_int, c_int, _P],

@@ -192,6 +192,68 @@ def test_linear_in_partial_sums_then_norm_is_linear_then_norm(m, n, k):
         assert torch.equal(out_a, out_b) and torch.equal(res_a, res_b)
 
 
+def _tile_shapes():
+    """(rows, features) of every tile shape, from the list that the kernels are compiled for."""
+    import re
+    from pathlib import Path
+
+    import mini_infer_amd
+
+    text = (Path(mini_infer_amd.__file__).parent / "csrc" / "gemm_tiles.h").read_text()
+    found = [[int(v) for v in m.split(",")] for m in re.findall(r"^  X\(([0-9, ]+)\)", text, re.M)]
+    return [(wm * mt * 16, wn * nt * 16) for wm, wn, _, mt, nt, _ in found]
+
+
+@pytest.mark.parametrize("shape", range(len(_tile_shapes())))
+def test_products_in_tiles(shape):
+    """Every shape at the edges of its tiles, whole, over ranges of K, as float32 times a number, and gated; K of one step, of fewer steps than
+    the ring has stages, of odd 32s, and of ranges of unequal length; rows of a wider buffer; a row of infinities stays alone."""
+    from mini_infer_amd.ops import kernels
+
+    bm, bn = _tile_shapes()[shape]
+    cases = [(bm, bn, 64, 1), (bm + 1, bn + 1, 128, 2), (bm - 1, bn - 3, 320, 1), (2 * bm + 5, 2 * bn + 4, 64 * 11, 3), (1, 5, 32, 1),
+             (17, bn + 62, 96, 1), (bm, 70, 64 * 7 + 32, 2), (3, 2 * bn, 1024, 16)]
+    for m, n, k, ranges in cases:
+        a = _rand(m, k + 8, dtype=torch.bfloat16, seed=41)[:, :k]
+        w = _rand(2 * n, k, dtype=torch.bfloat16, seed=42, scale=0.05)
+        if m > 2:
+            a[m - 1] = float("inf")
+        exact = a.double() @ w.double().T
+        finite = slice(0, m - 1 if m > 2 else m)
+        bound = 2.0 ** -8 * float(exact[finite].abs().max()) + 1e-6  # (float32 sums of exact products, one rounding)
+        pieces = kernels._tiles(1, a, w, torch.full((ranges, m, 2 * n), 7.0, device=DEV), 2 * n, shape, ranges)
+        assert (pieces.double().sum(0) - exact)[finite].abs().max() < 2.0 ** -20 * k * float(exact[finite].abs().max()) + 1e-6
+        if ranges == 1:
+            out = kernels._tiles(0, a, w, torch.full((m, 2 * n + 3), 7.0, dtype=torch.bfloat16, device=DEV)[:, : 2 * n], 2 * n, shape, 1)
+            assert (out.double() - exact)[finite].abs().max() < bound, (m, n, k)
+            scaled = kernels._tiles(2, a, w, torch.empty(m, 2 * n, device=DEV), 2 * n, shape, 1, 0.25)
+            assert torch.equal(scaled[finite], out.float()[finite] * 0.25)
+            gated = kernels._tiles(3, a, w, torch.empty(m, n, dtype=torch.bfloat16, device=DEV), n, shape, 1)
+            g, u = out.double()[:, :n], out.double()[:, n:]
+            wanted = (g / (1.0 + torch.exp(-g)) * u)[finite]
+            # (a product may come out one rounding apart: the gated tile sums the same pieces in the same order, so it does not)
+            assert (gated.double()[finite] - wanted).abs().max() < 2.0 ** -8 * float(wanted.abs().max()) + 1e-6, (m, n, k)
+
+
+@pytest.mark.parametrize("m,n,k", [(17, 3072, 3072), (33, 2048, 8192), (271, 3072, 8192), (100, 8192, 2048), (24, 1000, 8224), (400, 2048, 8192)])
+def test_linear_of_some_tens_to_some_hundreds_of_rows(m, n, k):
+    """`linear` through tiles, with and without a consumer for the pieces; operands that the tiles do not take (rows off 16 bytes) go on
+    being taken."""
+    from mini_infer_amd import ops
+    from mini_infer_amd.ops import kernels
+
+    a, w = _rand(m, k, dtype=torch.bfloat16, seed=43), _rand(n, k, dtype=torch.bfloat16, seed=44, scale=0.05)
+    expected = a.double() @ w.double().T
+    bound = 2.0 ** -8 * float(expected.abs().max()) + 1e-6
+    assert kernels.tiles_for(m, n, k, True) is not None
+    left = ops.linear(a, w, partial_ok=True)
+    left = left.finish() if isinstance(left, ops.PartialSums) else left
+    off = _rand(m * k + 4, dtype=torch.bfloat16, seed=45)[4:].view(m, k).copy_(a)
+    for got in (left, ops.linear(a, w), ops.linear(off, w)):
+        assert got.dtype == torch.bfloat16 and (got.double() - expected).abs().max() < bound
+    assert torch.equal(kernels.sum_pieces(_rand(3, 5, 7, seed=46)), _rand(3, 5, 7, seed=46).sum(0).bfloat16())
+
+
 def test_linear_leaves_partial_sums_only_where_asked_and_where_it_pays():
     from mini_infer_amd import ops
     from mini_infer_amd.exceptions import KernelShapeError
