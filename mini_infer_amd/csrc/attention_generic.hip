@@ -338,12 +338,19 @@ __global__ __launch_bounds__(512) void attn_reduce_kernel(const float* __restric
                                                          const float* __restrict__ part_ml,
                                                          T* __restrict__ out, int64_t out_row_stride,
                                                          int q_heads, int head_dim, int num_splits,
+                                                         int lead_tokens, int lead_splits,
                                                          int has_sink, float sink_logit, const float* __restrict__ sinks,
                                                          const T* __restrict__ gate, int64_t gate_row_stride) {
   using S = typename SumType<T>::type;
   const int t = blockIdx.x, h = blockIdx.y;
   const int lane = threadIdx.x % MI_WAVE;
-  const int64_t base = ((int64_t)t * q_heads + h) * num_splits;
+  int64_t base = ((int64_t)t * q_heads + h) * num_splits;
+  if (t < lead_tokens) {
+    num_splits = lead_splits;
+    base = ((int64_t)t * q_heads + h) * num_splits;
+  } else {
+    base += (int64_t)lead_tokens * q_heads * (lead_splits - num_splits);
+  }
   constexpr int BATCH = 8;
   // Few splits of a head of at most 128 dims (the usual decode step): every partial value
   // this lane needs is requested up front, together with the (max, sum) pairs, so the
@@ -465,7 +472,7 @@ static int attn_generic_launch(const void* q, int64_t q_row_stride, const void* 
   if (num_splits > 1) {
     dim3 rgrid(num_tokens, q_heads);
     attn_reduce_kernel<T><<<rgrid, reduce_threads(v_dim), 0, stream>>>(part_acc, part_ml, (T*)out, out_row_stride,
-                                                         q_heads, v_dim, num_splits, has_sink, sink_logit, sinks,
+                                                         q_heads, v_dim, num_splits, 0, 1, has_sink, sink_logit, sinks,
                                                          (const T*)gate, gate_row_stride);
     MI_CHECK_LAUNCH("attn_reduce");
   }
@@ -564,17 +571,17 @@ extern "C" int mi_attn_general(int dtype, const void* q, int64_t q_row_stride, c
                                       softcap, sinks, gate, gate_row_stride);
 }
 
-// The combining step alone, for partials written by the matrix-core kernel.
+// The combining step alone, for partials written by the matrix-core kernel (attention_mfma.h says what the lead tokens are).
 extern "C" int mi_attn_reduce_bf16(const float* part_acc, const float* part_ml, void* out,
                                    int64_t out_row_stride, int num_tokens, int q_heads,
-                                   int head_dim, int num_splits, int has_sink, float sink_logit,
+                                   int head_dim, int num_splits, int lead_tokens, int lead_splits, int has_sink, float sink_logit,
                                    const float* sinks, const void* gate, int64_t gate_row_stride, hipStream_t stream) {
   if (num_tokens == 0) return MI_OK;
   MI_REQUIRE(q_heads <= 65535, "attn_reduce: too many heads");
   dim3 rgrid(num_tokens, q_heads);
   attn_reduce_kernel<bf16_t><<<rgrid, reduce_threads(head_dim), 0, stream>>>(part_acc, part_ml, (bf16_t*)out,
                                                             out_row_stride, q_heads, head_dim,
-                                                            num_splits, has_sink, sink_logit, sinks,
+                                                            num_splits, lead_tokens, lead_splits, has_sink, sink_logit, sinks,
                                                             (const bf16_t*)gate, gate_row_stride);
   MI_CHECK_LAUNCH("attn_reduce");
   return MI_OK;

@@ -1043,6 +1043,7 @@ def paged_attention(
     softcap: float | None = None,
     gate: torch.Tensor | None = None,
     out: torch.Tensor | None = None,
+    host_seq_lens: list[int] | None = None,
 ) -> torch.Tensor | AttentionPieces:
     """Causal attention of every token over its request's pages; returns [T, q_heads*head_dim].
 
@@ -1078,7 +1079,9 @@ def paged_attention(
     `host_cu_seqlens_q=None`: the boundaries are known on the device only (a step that is
     recorded once and replayed with other boundaries); the launch is then shaped by the number
     of tokens and requests alone, with as many tiles as any division of the tokens among the
-    requests can need, and requests without tokens are allowed.
+    requests can need, and requests without tokens are allowed.  `host_seq_lens` (optional): how many
+    positions each request holds with this step's tokens; where a step brings portions beside single tokens, each
+    of the two is cut by its own keys.
     bfloat16 caches with transposed values run on the matrix cores; everything else
     (float32, other head or page sizes) runs the plain kernel.
     """
@@ -1167,19 +1170,36 @@ def paged_attention(
 
     gate_args = (v_dim, _ptr(gate), 0 if gate is None else gate.stride(0))
 
-    def seen(tokens_per_tile: int) -> int:
-        """The most keys the tokens of one tile see (a chunked mask hides all but a chunk's)."""
-        return max_seq_len if chunk is None else min(max_seq_len, chunk + tokens_per_tile - 1)
+    def seen(tokens_per_tile: int, most: int = max_seq_len) -> int:
+        """The most keys the tokens of one tile see (a chunked mask hides all but a chunk's) of requests of at most `most` positions."""
+        return most if chunk is None else min(most, chunk + tokens_per_tile - 1)
+
+    def mixed(singles: int, num_tiles: int, single_splits: int, tile_splits: int) -> None:
+        """Portions and single tokens as one launch (csrc/attention_mixed.hip); `singles` < 0: found on the device."""
+        lead = max(singles, 0)
+        rows = (lead * (single_splits if single_splits > 1 else 0) + (tokens - lead) * (tile_splits if tile_splits > 1 else 0)) * q_heads
+        pieces = torch.empty((rows * (v_dim + 2),), dtype=torch.float32, device=q.device) if rows else None
+        library.check(
+            lib.mi_attn_mixed(
+                _ptr(q), q.stride(0), _ptr(k_pages), _ptr(v_pages), _ptr(block_table), block_table.shape[1], _ptr(cu_seqlens_q),
+                _ptr(positions), num_requests, tokens, singles, num_tiles, _ptr(out), out.stride(0), _ptr(pieces),
+                None if pieces is None else _ptr(pieces) + 4 * rows * v_dim, q_heads, kv_heads, head_dim, page_size, num_pages,
+                float(scale), int(window or 0), single_splits, tile_splits, int(has_sink), float(sink_logit or 0.0), int(chunk or 0),
+                _ptr(sinks), _ptr(slopes), float(softcap or 0.0), _ptr(gate), 0 if gate is None else gate.stride(0), _stream(),
+            )
+        )
 
     if use_mfma and host_cu_seqlens_q is None:
-        # boundaries on the device only: one launch in the prefill shape, every wave finding its
-        # tile's request itself; a request of q tokens has ceil(q / tile) tiles, at most
-        # tokens // tile + requests of them in all, and the tiles past the real ones find nothing
+        # boundaries on the device only: one launch, every wave finding its tile's request itself; a request of q tokens has
+        # ceil(q / tile) tiles, at most tokens // tile + requests of them in all, and the tiles past the real ones find nothing
         shape = ATTN_SHAPE_PREFILL
         tokens_per_tile = lib.mi_attn_mfma_tokens_per_tile(q_heads, kv_heads, shape)
         num_tiles = tokens // tokens_per_tile + num_requests
         head_blocks = -(-group // min(group, 128))
         splits = min(16, attention_splits(num_tiles * kv_heads * head_blocks, seen(tokens_per_tile), target=512, min_keys=128))
+        if num_requests > 1 and lib.mi_attn_mixed_supported(head_dim, v_dim, page_size):
+            mixed(-1, num_tiles, splits, splits)
+            return out
         part_acc, part_ml = partials(splits)
         library.check(
             lib.mi_attn_mfma(
@@ -1195,6 +1215,12 @@ def paged_attention(
         q_lens = [host_cu_seqlens_q[b + 1] - host_cu_seqlens_q[b] for b in range(num_requests)]
         max_blocks = block_table.shape[1]
 
+        def wide_prefill(lens: list[int]) -> bool:
+            if head_dim > 128:
+                return False
+            wide_tile = lib.mi_attn_mfma_tokens_per_tile(q_heads, kv_heads, ATTN_SHAPE_PREFILL_WIDE)
+            return sum(-(-n // wide_tile) for n in lens) * kv_heads * -(-group // min(group, 256)) >= WIDE_PREFILL_MIN_BLOCKS
+
         def run(first: int, last: int, leave_pieces: bool = False) -> AttentionPieces | None:
             """Requests [first, last) of the step in one launch."""
             lens = q_lens[first:last]
@@ -1203,11 +1229,8 @@ def paged_attention(
             run_tokens = host_cu_seqlens_q[last] - first_token
             decode_only = max(lens) <= 1
             shape = ATTN_SHAPE_DECODE if decode_only else ATTN_SHAPE_PREFILL
-            if not decode_only and head_dim <= 128:
-                wide_tile = lib.mi_attn_mfma_tokens_per_tile(q_heads, kv_heads, ATTN_SHAPE_PREFILL_WIDE)
-                wide_blocks = sum(-(-n // wide_tile) for n in lens) * kv_heads * -(-group // min(group, 256))
-                if wide_blocks >= WIDE_PREFILL_MIN_BLOCKS:
-                    shape = ATTN_SHAPE_PREFILL_WIDE
+            if not decode_only and wide_prefill(lens):
+                shape = ATTN_SHAPE_PREFILL_WIDE
             tokens_per_tile = lib.mi_attn_mfma_tokens_per_tile(q_heads, kv_heads, shape)
             # 2: exactly one token per request (the kernel then needs no request boundaries)
             one_tile_per_request = 2 if (decode_only and min(lens) == 1) else int(max(lens) <= tokens_per_tile)
@@ -1247,8 +1270,18 @@ def paged_attention(
         while leading_single < num_requests and q_lens[leading_single] == 1:
             leading_single += 1
         if 0 < leading_single < num_requests:
-            run(0, leading_single)
-            run(leading_single, num_requests)
+            most = host_seq_lens or [max_seq_len] * num_requests
+            lens = q_lens[leading_single:]
+            if not lib.mi_attn_mixed_supported(head_dim, v_dim, page_size) or wide_prefill(lens):
+                run(0, leading_single)
+                run(leading_single, num_requests)
+                return out
+            tile = lib.mi_attn_mfma_tokens_per_tile(q_heads, kv_heads, ATTN_SHAPE_PREFILL)
+            num_tiles = sum(-(-n // tile) for n in lens)
+            # (portions are cut from 512 keys on only: a portion of 256 tokens in two ranges would need the combining launch for all its rows)
+            mixed(leading_single, num_tiles,
+                  min(16, attention_splits(leading_single * kv_heads * -(-group // 16), seen(1, max(most[:leading_single])), target=256, min_keys=128)),
+                  min(16, attention_splits(num_tiles * kv_heads * -(-group // 128), seen(tile, max(most[leading_single:])), target=512, min_keys=256)))
         else:
             pieces = run(0, num_requests, leave_pieces=not combine and not has_sink and chunk is None and gate is None and v_dim == head_dim
                          and leading_single == num_requests)

@@ -14,7 +14,7 @@ from pathlib import Path
 from mini_infer_amd.exceptions import ExtensionMissingError, KernelShapeError
 from mini_infer_amd.ops import build as _build
 
-ABI_VERSION = 39
+ABI_VERSION = 40
 
 _lib: ctypes.CDLL | None = None
 _lib_path: Path | None = None
@@ -70,6 +70,11 @@ _SIGNATURES: dict[str, list] = {
         _P, c_int64, _P, _P, _P, c_int, _P, _P, c_int, c_int, c_int, _P, c_int64, _P, _P, c_int,
         c_int, c_int, c_int, c_int, c_float, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_int, _P, _P, c_float, c_int, _P,
         c_int64, _P,
+    ],
+    "mi_attn_mixed_supported": [c_int, c_int, c_int],
+    "mi_attn_mixed": [
+        _P, c_int64, _P, _P, _P, c_int, _P, _P, c_int, c_int, c_int, c_int, _P, c_int64, _P, _P, c_int, c_int, c_int, c_int, c_int, c_float,
+        c_int, c_int, c_int, c_int, c_float, c_int, _P, _P, c_float, _P, c_int64, _P,
     ],
     "mi_gemm_skinny_addnorm_pieces": [c_int],
     "mi_gemm_skinny_addnorm_bf16": [

@@ -354,6 +354,7 @@ class GQAttention(Mixer):
             kv_heads=self.num_kv_heads, head_dim=self.head_dim, scale=self.scale, window=self.window,
             max_seq_len=ctx.max_seq_len, v_transposed=cache.v_transposed, combine=not few, slopes=self.slopes,
             v_head_dim=self.v_head_dim, sink_logit=self.sink_logit, chunk=self.chunk, gate=gate, out=out,
+            host_seq_lens=ctx.host_seq_lens,
         )
 
 
@@ -532,7 +533,7 @@ class WholeNormAttention(GQAttention):
             ctx.positions, ctx.cu_seqlens_q, ctx.host_cu_seqlens_q, q_heads=self.num_heads,
             kv_heads=self.num_kv_heads, head_dim=self.head_dim, scale=self.scale, window=self.window,
             max_seq_len=ctx.max_seq_len, v_transposed=cache.v_transposed, slopes=self.slopes,
-            v_head_dim=self.v_head_dim, sinks=self.sinks, softcap=self.softcap,
+            v_head_dim=self.v_head_dim, sinks=self.sinks, softcap=self.softcap, host_seq_lens=ctx.host_seq_lens,
         )
         return self.out.forward(attended)
 

@@ -725,6 +725,45 @@ def test_paged_attention_float32_four_waves_a_range(q_heads, kv_heads, head_dim,
     assert np.abs(out.double().cpu().numpy() - expected).max() < 4e-7 * max(1.0, np.abs(expected).max())
 
 
+@pytest.mark.parametrize("q_heads,kv_heads,head_dim,window", [(32, 8, 64, None), (24, 8, 128, None), (40, 2, 128, 130), (3, 3, 64, 40)])
+@pytest.mark.parametrize("lengths,q_lens", [
+    ([1, 2], [1, 2]), ([300, 33, 600], [1, 1, 256]), ([2000, 1, 31, 900, 700, 50], [1, 1, 1, 40, 200, 1]), ([90, 43, 3000], [1, 43, 85]),
+])
+@pytest.mark.parametrize("on_device", [False, True])
+def test_paged_attention_of_portions_beside_single_tokens_in_one_launch(monkeypatch, q_heads, kv_heads, head_dim, window, lengths, q_lens, on_device):
+    """Both parts whole and in key ranges, tiles of 42, 16 and 128 tokens with and without rests, a single token behind the portions (on the
+    device it has a decode block, else a tile); boundaries known and found on the device, there with a request that brings nothing.
+    Sinks, caps, slopes, chunks and gates: as in launches of their own, but for the ranges' order (bfloat16 results)."""
+    from mini_infer_amd import ops
+    from mini_infer_amd.ops import kernels
+
+    case = _paged_case(torch.bfloat16, q_heads, kv_heads, head_dim, 16, lengths, q_lens, seed=17, v_transposed=True)
+    lib, taken = kernels.library.load(), []
+    launch = lib.mi_attn_mixed
+    monkeypatch.setattr(lib, "mi_attn_mixed", lambda *a: (taken.append(a[10]), launch(*a))[1])
+    tokens, scale = case["q"].shape[0], head_dim ** -0.5
+    table, cu, host_cu, held = case["block_table"], case["cu"], case["host_cu"], list(lengths)
+    if on_device:
+        table, cu, host_cu, held = torch.cat([table, torch.zeros_like(table[:1])]), torch.cat([cu, cu[-1:]]), None, None
+
+    def attend(**more):
+        return ops.paged_attention(case["q"], case["k_pages"], case["v_pages"], table, case["token_request"], case["positions"], cu, host_cu,
+                                   q_heads=q_heads, kv_heads=kv_heads, head_dim=head_dim, scale=scale, window=window, max_seq_len=max(lengths),
+                                   v_transposed=True, host_seq_lens=held, **more)
+
+    leading = next(i for i, n in enumerate(q_lens) if n > 1)
+    got = attend()
+    assert taken == [-1 if on_device else leading]
+    assert np.abs(got.double().cpu().numpy() - _attention_expected(case, scale, window)).max() < _tol(torch.bfloat16, 2)
+    options = {"sinks": _rand(q_heads, seed=1), "softcap": 5.0, "slopes": _rand(q_heads, seed=2).abs() * 0.02, "chunk": 100,
+               "gate": _rand(tokens, q_heads, seed=3, dtype=torch.bfloat16)}
+    wide = torch.zeros((tokens, q_heads * head_dim + 8), dtype=torch.bfloat16, device=DEV)
+    got = attend(out=wide[:, 4:-4], **options)
+    assert len(taken) == 2 and not wide[:, :4].any() and not wide[:, -4:].any()
+    monkeypatch.setattr(lib, "mi_attn_mixed_supported", lambda *a: 0)
+    assert (got.float() - attend(**options).float()).abs().max() < _tol(torch.bfloat16, 2) and len(taken) == 2
+
+
 @pytest.mark.parametrize("window", [None, 700])
 def test_paged_attention_whole_long_prompts_many_tiles(window):
     """Whole prompts of a few thousand tokens beside a short one: dozens of tiles per head,
