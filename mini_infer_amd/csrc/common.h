@@ -95,6 +95,16 @@ __device__ __forceinline__ void lines_to_operands(bf16x8_t& lower_rows, bf16x8_t
 __device__ __forceinline__ int line_row_of_lane(int lane) { return lane / 8; }
 __device__ __forceinline__ uint32_t line_chunk_of_lane(int lane) { return (uint32_t)(lane % 8) * 16u; }
 
+// One of the loads below by itself.
+__device__ __forceinline__ bf16x8_t load_line(const void* matrix, int64_t first_kstep, uint32_t at) {
+  using global_bytes = const __attribute__((address_space(1))) char;
+  using global_chunk = const __attribute__((address_space(1))) bf16x8_t;
+  uint64_t base_bits = reinterpret_cast<uint64_t>(matrix) + (uint64_t)first_kstep * 64u;
+  asm("" : "+s"(base_bits));
+  asm("" : "+v"(at));
+  return __builtin_nontemporal_load((global_chunk*)((global_bytes*)base_bits + at));
+}
+
 // The two loads of a pair of k-steps, non-temporal: base (uniform, kept in scalar registers) + the
 // lane's offsets.
 __device__ __forceinline__ void load_line_pair(const void* matrix, int64_t first_kstep, uint32_t lower_at,

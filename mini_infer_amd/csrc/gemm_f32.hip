@@ -164,7 +164,7 @@ __device__ __forceinline__ float4 four_in_flight(const float* row, int at, int k
   return make_float4(__uint_as_float(bits[0]), __uint_as_float(bits[1]), __uint_as_float(bits[2]), __uint_as_float(bits[3]));
 }
 
-// Few rows (decode): bound by reading W once.  A block owns 16 * RT rows and 16 * FT features; its 8 waves take
+// Few rows (decode; those that gemm_f32_few_kernel does not take): bound by reading W once.  A block owns 16 * RT rows and 16 * FT features; its 8 waves take
 // one run of K each (the order above), every wave streams its part of the weights from memory, two slices ahead,
 // and the runs' sums meet in LDS.  LINES: whole lines of W, non-temporal, brought into operand order by lane
 // exchanges (common.h): rows of W on 128 bytes, K a multiple of 32, A on 16 bytes.  PIECES: 16 bytes a load in operand order
@@ -295,12 +295,115 @@ __global__ __launch_bounds__(SEGMENTS * MI_WAVE) void gemm_f32_rows_kernel(const
   }
 }
 
+// The same for up to 4 * G rows, of which the instruction above would leave most of its 16 idle: the 64-bit instruction of
+// four 4x4 products (4x4x4) takes a quarter of its time and keeps W where it has it (a lane's feature is lane % 16, its piece of K lane / 16; a
+// row of A is lane % 4), and sums in the same order, so a row gives the same bits.  Rows of A go through LDS, a wave's own run of them
+// CHUNK slices at a time: read from memory like W, they were a load for every one of W's (gate|up at 3 rows without them 27 -> 25 us, without
+// the products 21).  Form LINES only.  A block owns FEATURES features and all of K, eight waves a run each; 8 features where 16 would
+// leave half of the CUs without a block (the upper eight of the operand then repeat the lower ones and are not written).
+//
+// Deeper prefetch is no better (the output head at 8 slices 192 us, 151 at 2 and 4): blocks beside one another on a CU cover the
+// waits.  Microseconds at 3 rows (1B sizes), before -> after: q|k|v 3072 x 2048 9.3 -> 7.9, o 2048 x 2048 8.8 -> 7.0, down 2048 x 8192
+// 28.4 -> 20.4, gate|up 16384 x 2048 30.4 -> 22.6, head 128256 x 2048 180 -> 151 (6.9 TB/s); at 7 rows (two slices ahead) 9.1 -> 8.8, 8.9 -> 8.7,
+// 30.7 -> 25.7, 184 -> 180, and above 16 slices a run no better than with one 16 x 16 product (2048 x 8192 29.1 against 28.5, 4096 x 14336
+// 48.8 / 47.6), so those stay.
+template <int G, int FEATURES>
+__global__ __launch_bounds__(SEGMENTS * MI_WAVE) void gemm_f32_few_kernel(const float* __restrict__ a, int64_t lda,
+                                                           const float* __restrict__ w, int64_t ldw,
+                                                           float* __restrict__ c, int64_t ldc, int m, int n, int k, int chunk) {
+  extern __shared__ __attribute__((aligned(16))) float4 staged[];  // [wave][slice of the chunk][group of rows][half][piece of K][row]
+  __shared__ double sums[SEGMENTS][G][MI_WAVE];
+  constexpr int AHEAD = G == 1 ? 4 : 2;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / MI_WAVE), lane = threadIdx.x % MI_WAVE;
+  const int col0 = blockIdx.x * FEATURES, most = n - 1 - col0;
+  const int run = segment_slices(k), slices = ceil_div(k, SLICE);
+  const int first = min(wave * run, slices), last = min(first + run, slices);
+  const uint32_t lower = (uint32_t)min(line_row_of_lane(lane), most) * (uint32_t)(ldw * 4) + line_chunk_of_lane(lane);
+  const uint32_t upper = FEATURES == 8 ? lower : (uint32_t)min(line_row_of_lane(lane) + 8, most) * (uint32_t)(ldw * 4) + line_chunk_of_lane(lane);
+  const float* w_block = w + (int64_t)col0 * ldw;
+  bf16x8_t lo[AHEAD], hi[AHEAD];  // 16-byte pieces; what they hold is float32
+  auto fetch = [&](int slot, int slice) {
+    if constexpr (FEATURES == 8) lo[slot] = load_line(w_block, 2 * (int64_t)slice, lower);
+    else load_line_pair(w_block, 2 * (int64_t)slice, lower, upper, lo[slot], hi[slot]);
+  };
+  float4* mine = staged + wave * chunk * (32 * G);
+  auto stage = [&](int from, int upto) {
+    const int piece = lane % 16, row = lane / 16;  // two slices a load
+    for (int s = from; s < upto; s += 2) {
+      if (s + piece / 8 < upto) {
+#pragma unroll
+        for (int g = 0; g < G; ++g)
+          mine[((s - from + piece / 8) * G + g) * 32 + piece % 8 * 4 + row] =
+              *reinterpret_cast<const float4*>(a + (int64_t)min(g * 4 + row, m - 1) * lda + (int64_t)s * SLICE + piece * 4);
+      }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // (nobody else reads them: no barrier)
+  };
+  double acc[G];
+#pragma unroll
+  for (int g = 0; g < G; ++g) acc[g] = 0.0;
+#pragma unroll
+  for (int s = 0; s < AHEAD; ++s)
+    if (first + s < last) fetch(s, first + s);
+  const float4* from = mine + lane / 16 * 4 + lane % 4;
+  for (int begin = first; begin < last; begin += chunk) {
+    const int end = min(begin + chunk, last);
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    stage(begin, end);
+    for (int at = begin; at < end; at += AHEAD) {
+#pragma unroll
+      for (int s = 0; s < AHEAD; ++s) {
+        if (at + s < end) {
+          float wv[2][4], xv[G][2][4];
+          if constexpr (FEATURES == 8) hi[s] = lo[s];
+          lines_to_operands(lo[s], hi[s]);
+          __builtin_memcpy(wv[0], &lo[s], 16);
+          __builtin_memcpy(wv[1], &hi[s], 16);
+#pragma unroll
+          for (int g = 0; g < G; ++g)
+#pragma unroll
+            for (int half = 0; half < 2; ++half) {
+              const float4 x = from[((at + s - begin) * G + g) * 32 + half * 16];
+              __builtin_memcpy(xv[g][half], &x, 16);
+            }
+          if (at + s + AHEAD < last) fetch(s, at + s + AHEAD);
+#pragma unroll
+          for (int half = 0; half < 2; ++half)
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+              for (int g = 0; g < G; ++g)
+                acc[g] = __builtin_amdgcn_mfma_f64_4x4x4f64((double)xv[g][half][e], (double)wv[half][e], acc[g], 0, 0, 0);
+        }
+      }
+    }
+  }
+#pragma unroll
+  for (int g = 0; g < G; ++g) sums[wave][g][lane] = acc[g];
+  __syncthreads();
+  if (wave < G) {
+    double total = 0.0;
+#pragma unroll
+    for (int s = 0; s < SEGMENTS; ++s) total += sums[s][wave][lane];
+    const int row = wave * 4 + lane / 16, f = lane % 16;  // (the instruction's result: row lane / 16, feature lane % 16)
+    if (f < FEATURES && row < m && col0 + f < n) c[(int64_t)row * ldc + col0 + f] = (float)total;
+  }
+}
+
 template <int BM, int STAGE>
 static void launch_tiles(const float* a, int64_t lda, const float* w, int64_t ldw, float* c, int64_t ldc, int m, int n,
                          int k, bool aligned, hipStream_t stream) {
   dim3 grid(ceil_div(n, BN), ceil_div(m, BM));
   if (aligned) gemm_f32_kernel<BM, STAGE, true><<<grid, 256, 0, stream>>>(a, lda, w, ldw, c, ldc, m, n, k);
   else gemm_f32_kernel<BM, STAGE, false><<<grid, 256, 0, stream>>>(a, lda, w, ldw, c, ldc, m, n, k);
+}
+
+template <int G, int FEATURES>
+static void launch_few(const float* a, int64_t lda, const float* w, int64_t ldw, float* c, int64_t ldc, int m, int n, int k,
+                       hipStream_t stream) {
+  const int chunk = min(segment_slices(k), 16 / G);
+  gemm_f32_few_kernel<G, FEATURES><<<ceil_div(n, FEATURES), SEGMENTS * MI_WAVE, SEGMENTS * chunk * G * 32 * sizeof(float4), stream>>>(
+      a, lda, w, ldw, c, ldc, m, n, k, chunk);
 }
 
 template <int RT, int FT>
@@ -312,7 +415,8 @@ static void launch_rows(const float* a, int64_t lda, const float* w, int64_t ldw
   else gemm_f32_rows_kernel<RT, FT, VALUES><<<grid, block, 0, stream>>>(a, lda, w, ldw, c, ldc, m, n, k);
 }
 
-// Which kernel, with microseconds at rows x N x K (weights from memory).  Before: 64-bit multiply-adds on the vector
+// Which kernel, with microseconds at rows x N x K (weights from memory; 3 rows: in one 16 x 16 product, for groups of four see
+// gemm_f32_few_kernel).  Before: 64-bit multiply-adds on the vector
 // pipe, 4 x 4 outputs a thread, and a kernel of its own for up to 16 rows only.
 //     3 x 2048 x 2048     75.6 ->   9.0     20 x  2048 x 2048   317 ->  15.0     509 x  2048 x 2048    327 ->  82
 //     3 x 16384 x 2048     107 ->  30.7     20 x 16384 x 2048   349 ->  46.0     509 x  3072 x 2048    378 -> 117
@@ -337,7 +441,11 @@ extern "C" int mi_gemm_f32(const float* a, int64_t lda, const float* w, int64_t 
     // (the streaming loads' offsets reach over a block's 32 features in 32 bits: ldw under 2^24 values)
     const bool lines = a16 && k % SLICE == 0 && ldw % 32 == 0 && (uintptr_t)w % 128 == 0 && ldw < (1 << 24);
     const int form = lines ? LINES : a16 && w16 && k % 4 == 0 ? PIECES : VALUES;
-    if (m > 32) launch_rows<4, 1>(a, lda, w, ldw, c, ldc, m, n, k, form, stream);
+    const bool half_empty = ceil_div(n, 16) <= 128;
+    if (lines && m <= (segment_slices(k) <= 16 ? 8 : 4)) {
+      if (m > 4) half_empty ? launch_few<2, 8>(a, lda, w, ldw, c, ldc, m, n, k, stream) : launch_few<2, 16>(a, lda, w, ldw, c, ldc, m, n, k, stream);
+      else half_empty ? launch_few<1, 8>(a, lda, w, ldw, c, ldc, m, n, k, stream) : launch_few<1, 16>(a, lda, w, ldw, c, ldc, m, n, k, stream);
+    } else if (m > 32) launch_rows<4, 1>(a, lda, w, ldw, c, ldc, m, n, k, form, stream);
     else if (m > 16) launch_rows<2, 1>(a, lda, w, ldw, c, ldc, m, n, k, form, stream);
     else if (wide) launch_rows<1, 2>(a, lda, w, ldw, c, ldc, m, n, k, form, stream);
     else launch_rows<1, 1>(a, lda, w, ldw, c, ldc, m, n, k, form, stream);

@@ -118,6 +118,19 @@ def test_gemm_f32_is_true_float32(m, n, k):
     assert torch.equal(ops.gemm_f32(wide[:, :k], w), ops.gemm_f32(wide[:, :k].contiguous(), w))
 
 
+@pytest.mark.parametrize("m", [1, 3, 4, 5, 8])
+@pytest.mark.parametrize("n,k", [(5, 32), (8, 288), (17, 544), (2041, 1056), (2048, 4352), (2050, 2080), (2064, 4096), (9000, 256)])
+def test_few_rows_of_gemm_f32_in_groups_of_four(m, n, k):
+    """One and two groups of four rows, 8 and 16 features a block with a rest, runs of K of none, one, some and more slices than a stage
+    holds: the bits that a row gets among 20 (which are made otherwise), and the exact product rounded once."""
+    from mini_infer_amd import ops
+
+    a, w = _rand(20, k, seed=33), _rand(n, k, seed=34)
+    out, exact = ops.gemm_f32(a[:m], w), a[:m].double() @ w.double().T
+    assert torch.equal(out, ops.gemm_f32(a, w)[:m])
+    assert ((out.double() - exact).abs() <= 2.0 ** -24 * exact.abs() + 1e-12 * math.sqrt(k)).all()
+
+
 @pytest.mark.parametrize("m,n,k", [(1, 16, 32), (16, 8200, 96), (17, 33, 544), (32, 100, 2048), (33, 8, 352), (64, 50, 257), (65, 130, 4096),
                                    (50, 8192, 160), (700, 6200, 100), (90, 70, 36), (80, 70, 900)])
 def test_gemm_f32_kernels_and_alignments_agree(m, n, k):
