@@ -70,6 +70,11 @@ __device__ __forceinline__ float from_lane(float v, int lane) {
 // WAVES: the block's waves take every WAVES-th 64 keys of the range and are merged in S at the end.  One wave walks
 // its keys at the latency of its loads and instructions, and a few decoded tokens are too few waves to hide that;
 // measured at attn_generic_launch.
+// With several waves (rows in whole 16s) 32 value rows are asked for at once instead of 8, the first of them with the first
+// values of the key rows, before the scores.  A few decoded tokens give a wave one or two 64s of keys, and its time is the waits one after another.  A layer with its
+// combining launch, 3 requests of up to 600 positions, 24 heads of 128 over 8: 43.1 -> 25.1 us (30 of 200: 42.8 -> 21.1); 32 heads of 64 over
+// 8: 21.9 -> 19.5.  (64 value rows, or all 64 values of a key row: the same for heads of 128 and 36 us for heads of 64, where the compiler
+// makes one long straight run of it.)
 template <typename T, int VPL, bool VEC, int WAVES>
 __global__ __launch_bounds__(64 * WAVES) void attn_generic_kernel(
     const T* __restrict__ q, int64_t q_row_stride, const T* __restrict__ k_pages,
@@ -83,6 +88,7 @@ __global__ __launch_bounds__(64 * WAVES) void attn_generic_kernel(
   extern __shared__ __align__(8) unsigned char q_lds_bytes[];
   S* q_lds = reinterpret_cast<S*>(q_lds_bytes);  // [GT][head_dim], pre-multiplied by the scale
   constexpr int KV = VEC ? 16 / sizeof(T) : 4;  // elements per step along a key row
+  constexpr bool DEEP = VEC && WAVES > 1;
 
   const int t = blockIdx.x;
   const int group = q_heads / kv_heads;
@@ -138,9 +144,57 @@ __global__ __launch_bounds__(64 * WAVES) void attn_generic_kernel(
       s[g] = -INFINITY;
       s_sum[g] = 0;
     }
-    if (valid) {
-      const int page = bt[key / page_size];
-      row_idx = (page * kv_heads + kvh) * page_size + key % page_size;
+    // value rows BATCH at a time, whose loads are in flight together (past the last key: that key again, weight 0)
+    constexpr int BATCH = DEEP ? 32 : 8;
+    const int n_valid = min(MI_WAVE, b - base);
+    float vv[BATCH][VPL];
+    auto load_values = [&](int j0) {
+#pragma unroll
+      for (int u = 0; u < BATCH; ++u) {
+        const int rj = __builtin_amdgcn_readlane(row_idx, min(j0 + u, n_valid - 1));
+#pragma unroll
+        for (int v = 0; v < VPL; ++v) vv[u][v] = 0.f;
+        if (owns_dims) {
+          const T* v_row = v_pages + (int64_t)rj * v_row_stride + lane * VPL;
+          if constexpr (VEC || VPL <= 2) {  // (an even head size: a pair never straddles the row's end)
+            const Pack<T, VPL> pk = *reinterpret_cast<const Pack<T, VPL>*>(v_row);
+#pragma unroll
+            for (int v = 0; v < VPL; ++v) vv[u][v] = to_f32(pk.v[v]);
+          } else {
+#pragma unroll
+            for (int v = 0; v < VPL; v += 2) {
+              if (lane * VPL + v < v_dim) {
+                const Pack<T, 2> pk = *reinterpret_cast<const Pack<T, 2>*>(v_row + v);
+                vv[u][v] = to_f32(pk.v[0]);
+                vv[u][v + 1] = to_f32(pk.v[1]);
+              }
+            }
+          }
+        }
+      }
+    };
+    // (16 values of the key row at a time where rows are whole 16s: their loads are in flight together)
+    constexpr int RUN = VEC ? 16 : KV;
+    float kf[RUN];
+    auto load_key = [&](const T* k_row, int d0) {
+#pragma unroll
+      for (int at = 0; at < RUN; at += KV) {
+        const Pack<T, KV> kk = *reinterpret_cast<const Pack<T, KV>*>(k_row + d0 + at);
+#pragma unroll
+        for (int e = 0; e < KV; ++e) kf[at + e] = to_f32(kk.v[e]);
+      }
+    };
+    if constexpr (DEEP) {  // (all lanes, those past the last key with it)
+      const int real = min(key, b - 1), page = bt[real / page_size];
+      row_idx = (page * kv_heads + kvh) * page_size + real % page_size;
+      load_key(k_pages + (int64_t)row_idx * head_dim, 0);
+      load_values(0);
+    }
+    if (DEEP || valid) {
+      if constexpr (!DEEP) {
+        const int page = bt[key / page_size];
+        row_idx = (page * kv_heads + kvh) * page_size + key % page_size;
+      }
       const T* k_row = k_pages + (int64_t)row_idx * head_dim;
       // four running sums per score (dims d, d+1, d+2, d+3 of every group of four), added
       // at the end: shorter chains of roundings than one sum over the whole head
@@ -149,17 +203,11 @@ __global__ __launch_bounds__(64 * WAVES) void attn_generic_kernel(
       for (int g = 0; g < GT; ++g)
 #pragma unroll
         for (int e = 0; e < 4; ++e) s4[g][e] = 0;
-      // (16 values of the key row at a time where rows are whole 16s: their loads are in flight together)
-      constexpr int RUN = VEC ? 16 : KV;
       for (int d0 = 0; d0 < head_dim; d0 += RUN) {
-        float kf[RUN];
-        if constexpr (VEC) {
-#pragma unroll
-          for (int at = 0; at < RUN; at += KV) {
-            const Pack<T, KV> kk = *reinterpret_cast<const Pack<T, KV>*>(k_row + d0 + at);
-#pragma unroll
-            for (int e = 0; e < KV; ++e) kf[at + e] = to_f32(kk.v[e]);
-          }
+        if constexpr (DEEP) {
+          if (d0 > 0) load_key(k_row, d0);
+        } else if constexpr (VEC) {
+          load_key(k_row, d0);
         } else {
           // pairs of elements; an even head size ends after the first or the second pair
           const Pack<T, 2> k0 = *reinterpret_cast<const Pack<T, 2>*>(k_row + d0);
@@ -193,7 +241,7 @@ __global__ __launch_bounds__(64 * WAVES) void attn_generic_kernel(
           else s_sum[g] = softcap * tanhf(s_sum[g] / softcap);
         }
         s_sum[g] += (S)slope[g] * distance;
-        s[g] = (float)s_sum[g];
+        s[g] = !DEEP || valid ? (float)s_sum[g] : -INFINITY;
       }
     }
     float p[GT];
@@ -212,34 +260,8 @@ __global__ __launch_bounds__(64 * WAVES) void attn_generic_kernel(
       for (int v = 0; v < VPL; ++v) acc[g][v] *= (S)alpha;
       m[g] = m_new;
     }
-    // value rows eight at a time, so that eight loads are in flight (past the last key: that key again, weight 0)
-    constexpr int BATCH = 8;
-    const int n_valid = min(MI_WAVE, b - base);
     for (int j0 = 0; j0 < n_valid; j0 += BATCH) {
-      float vv[BATCH][VPL];
-#pragma unroll
-      for (int u = 0; u < BATCH; ++u) {
-        const int rj = __builtin_amdgcn_readlane(row_idx, min(j0 + u, n_valid - 1));
-#pragma unroll
-        for (int v = 0; v < VPL; ++v) vv[u][v] = 0.f;
-        if (owns_dims) {
-          const T* v_row = v_pages + (int64_t)rj * v_row_stride + lane * VPL;
-          if constexpr (VEC || VPL <= 2) {  // (an even head size: a pair never straddles the row's end)
-            const Pack<T, VPL> pk = *reinterpret_cast<const Pack<T, VPL>*>(v_row);
-#pragma unroll
-            for (int v = 0; v < VPL; ++v) vv[u][v] = to_f32(pk.v[v]);
-          } else {
-#pragma unroll
-            for (int v = 0; v < VPL; v += 2) {
-              if (lane * VPL + v < v_dim) {
-                const Pack<T, 2> pk = *reinterpret_cast<const Pack<T, 2>*>(v_row + v);
-                vv[u][v] = to_f32(pk.v[0]);
-                vv[u][v + 1] = to_f32(pk.v[1]);
-              }
-            }
-          }
-        }
-      }
+      if (!DEEP || j0 > 0) load_values(j0);
 #pragma unroll
       for (int u = 0; u < BATCH; ++u) {
         if (j0 + u < n_valid) {
@@ -255,41 +277,43 @@ __global__ __launch_bounds__(64 * WAVES) void attn_generic_kernel(
   }
 
   if (merges) {  // wave 0 takes over what the others have, in their order
-    S* merge = q_lds + GT * head_dim;  // [WAVES - 1][GT][VPL + 1][64], then their maxima
+    S* merge = q_lds + GT * head_dim;  // [WAVES - 1][GT][VPL + 1][64], then [WAVES][GT] maxima
     float* maxima = reinterpret_cast<float*>(merge + (WAVES - 1) * GT * (VPL + 1) * MI_WAVE);
-    if (wave > 0) {
 #pragma unroll
-      for (int g = 0; g < GT; ++g) {
+    for (int g = 0; g < GT; ++g) {
+      if (wave > 0) {
         S* to = merge + ((wave - 1) * GT + g) * (VPL + 1) * MI_WAVE + lane;
 #pragma unroll
         for (int v = 0; v < VPL; ++v) to[v * MI_WAVE] = acc[g][v];
         to[VPL * MI_WAVE] = l[g];
-        if (lane == 0) maxima[(wave - 1) * GT + g] = m[g];
       }
+      if (lane == 0) maxima[wave * GT + g] = m[g];
     }
     __syncthreads();
     if (wave > 0) return;
+    // (a lane makes the weight of one wave and head: the sixteen 64-bit exponentials one after another took 0.8 us more)
+    const float its = lane < WAVES * GT ? maxima[lane] : -INFINITY;
+    float top = its;
+#pragma unroll
+    for (int off = GT; off < WAVES * GT; off <<= 1) top = fmaxf(top, __shfl_xor(top, off, MI_WAVE));
+    // (a wave without keys has the maximum -inf and nothing to add)
+    const double weight = its == -INFINITY ? 0.0 : exp((double)its - (double)top);
 #pragma unroll
     for (int g = 0; g < GT; ++g) {
-      float top = m[g];
-#pragma unroll
-      for (int w = 0; w < WAVES - 1; ++w) top = fmaxf(top, maxima[w * GT + g]);
-      // (a wave without keys has the maximum -inf and nothing to add)
-      const S own = m[g] == -INFINITY ? (S)0 : (S)exp((double)m[g] - (double)top);
+      const S own = (S)__shfl(weight, g, MI_WAVE);
       l[g] *= own;
 #pragma unroll
       for (int v = 0; v < VPL; ++v) acc[g][v] *= own;
 #pragma unroll
-      for (int w = 0; w < WAVES - 1; ++w) {
-        const float m_w = maxima[w * GT + g];
-        if (m_w == -INFINITY) continue;
-        const S weight = (S)exp((double)m_w - (double)top);
-        const S* from = merge + (w * GT + g) * (VPL + 1) * MI_WAVE + lane;
+      for (int w = 1; w < WAVES; ++w) {
+        if (from_lane(its, w * GT + g) == -INFINITY) continue;
+        const S its_weight = (S)__shfl(weight, w * GT + g, MI_WAVE);
+        const S* from = merge + ((w - 1) * GT + g) * (VPL + 1) * MI_WAVE + lane;
 #pragma unroll
-        for (int v = 0; v < VPL; ++v) acc[g][v] += from[v * MI_WAVE] * weight;
-        l[g] += from[VPL * MI_WAVE] * weight;
+        for (int v = 0; v < VPL; ++v) acc[g][v] += from[v * MI_WAVE] * its_weight;
+        l[g] += from[VPL * MI_WAVE] * its_weight;
       }
-      m[g] = top;
+      m[g] = from_lane(top, g);
     }
   }
 
@@ -456,7 +480,7 @@ static int attn_generic_launch(const void* q, int64_t q_row_stride, const void* 
   do {                                                                                            \
     if constexpr (sizeof(S) == 8 && VPL <= 2) {                                                   \
       if (four) {                                                                                 \
-        MI_ATTN_LAUNCH_WAVES(VPL, VEC, 4, lds + 3 * GT * ((VPL + 1) * MI_WAVE * sizeof(S) + sizeof(float))); \
+        MI_ATTN_LAUNCH_WAVES(VPL, VEC, 4, lds + 3 * GT * (VPL + 1) * MI_WAVE * sizeof(S) + 4 * GT * sizeof(float)); \
         break;                                                                                    \
       }                                                                                           \
     }                                                                                             \
