@@ -121,6 +121,14 @@ __device__ __forceinline__ void load_line_pair(const void* matrix, int64_t first
   upper_rows = __builtin_nontemporal_load((global_chunk*)(base + upper_at));
 }
 
+// (float32 elements: evaluated in 64-bit and rounded once; the float32 exponential and two more
+// roundings put the result 4.7e-8 away on average, twice what rounding alone costs)
+template <typename T>
+__device__ __forceinline__ float silu_times(float g, float u) {
+  if constexpr (sizeof(T) == 4) return (float)((double)g / (1.0 + exp(-(double)g)) * (double)u);
+  else return g / (1.f + expf(-g)) * u;
+}
+
 // 1 / (1 + exp(-z)) in float32 on the hardware's exponential and reciprocal (v_exp_f32, v_rcp_f32:
 // one ulp each).  The library's expf and an IEEE division cost some 70 instructions per gate,
 // and a prompt's gated recurrence was bound by them, not by memory (2,048 x 4,096 gates: 17 us

@@ -659,14 +659,6 @@ extern "C" int mi_rope_kv_write(int dtype, void* qkv, int64_t row_stride, const 
 // out[t, i] = silu(gate_up[t, i]) * gate_up[t, I + i],  silu(g) = g / (1 + exp(-g))
 // ---------------------------------------------------------------------------
 
-// (float32 elements: evaluated in 64-bit and rounded once; the float32 exponential and two more
-// roundings put the result 4.7e-8 away on average, twice what rounding alone costs)
-template <typename T>
-__device__ __forceinline__ float silu_times(float g, float u) {
-  if constexpr (sizeof(T) == 4) return (float)((double)g / (1.0 + exp(-(double)g)) * (double)u);
-  else return g / (1.f + expf(-g)) * u;
-}
-
 template <typename T, int VEC>
 __global__ __launch_bounds__(256) void silu_mul_kernel(const T* __restrict__ gate_up,
                                                        T* __restrict__ out, int inter) {

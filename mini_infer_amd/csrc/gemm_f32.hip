@@ -307,7 +307,11 @@ __global__ __launch_bounds__(SEGMENTS * MI_WAVE) void gemm_f32_rows_kernel(const
 // 28.4 -> 20.4, gate|up 16384 x 2048 30.4 -> 22.6, head 128256 x 2048 180 -> 151 (6.9 TB/s); at 7 rows (two slices ahead) 9.1 -> 8.8, 8.9 -> 8.7,
 // 30.7 -> 25.7, 184 -> 180, and above 16 slices a run no better than with one 16 x 16 product (2048 x 8192 29.1 against 28.5, 4096 x 14336
 // 48.8 / 47.6), so those stay.
-template <int G, int FEATURES>
+//
+// GATED: W is [gate; up], n features each; a block's operand holds the gate rows of 8 features and the up rows of the same, and
+// silu(gate) * up is written, both products rounded to float32 first, as silu_mul takes them (the same bits, a launch less: 1B with 3 requests
+// decoding 1,688 -> 1,658 us a step).
+template <int G, int FEATURES, bool GATED = false>
 __global__ __launch_bounds__(SEGMENTS * MI_WAVE) void gemm_f32_few_kernel(const float* __restrict__ a, int64_t lda,
                                                            const float* __restrict__ w, int64_t ldw,
                                                            float* __restrict__ c, int64_t ldc, int m, int n, int k, int chunk) {
@@ -315,11 +319,12 @@ __global__ __launch_bounds__(SEGMENTS * MI_WAVE) void gemm_f32_few_kernel(const 
   __shared__ double sums[SEGMENTS][G][MI_WAVE];
   constexpr int AHEAD = G == 1 ? 4 : 2;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / MI_WAVE), lane = threadIdx.x % MI_WAVE;
-  const int col0 = blockIdx.x * FEATURES, most = n - 1 - col0;
+  static_assert(!GATED || FEATURES == 16, "a block's operand holds both matrices' rows");
+  const int col0 = blockIdx.x * (GATED ? 8 : FEATURES), most = n - 1 - col0;
   const int run = segment_slices(k), slices = ceil_div(k, SLICE);
   const int first = min(wave * run, slices), last = min(first + run, slices);
   const uint32_t lower = (uint32_t)min(line_row_of_lane(lane), most) * (uint32_t)(ldw * 4) + line_chunk_of_lane(lane);
-  const uint32_t upper = FEATURES == 8 ? lower : (uint32_t)min(line_row_of_lane(lane) + 8, most) * (uint32_t)(ldw * 4) + line_chunk_of_lane(lane);
+  const uint32_t upper = GATED ? lower + (uint32_t)n * (uint32_t)(ldw * 4) : FEATURES == 8 ? lower : (uint32_t)min(line_row_of_lane(lane) + 8, most) * (uint32_t)(ldw * 4) + line_chunk_of_lane(lane);
   const float* w_block = w + (int64_t)col0 * ldw;
   bf16x8_t lo[AHEAD], hi[AHEAD];  // 16-byte pieces; what they hold is float32
   auto fetch = [&](int slot, int slice) {
@@ -386,7 +391,12 @@ __global__ __launch_bounds__(SEGMENTS * MI_WAVE) void gemm_f32_few_kernel(const 
 #pragma unroll
     for (int s = 0; s < SEGMENTS; ++s) total += sums[s][wave][lane];
     const int row = wave * 4 + lane / 16, f = lane % 16;  // (the instruction's result: row lane / 16, feature lane % 16)
-    if (f < FEATURES && row < m && col0 + f < n) c[(int64_t)row * ldc + col0 + f] = (float)total;
+    if constexpr (GATED) {
+      const float up = __shfl_down((float)total, 8, MI_WAVE);
+      if (f < 8 && row < m && col0 + f < n) c[(int64_t)row * ldc + col0 + f] = silu_times<float>((float)total, up);
+    } else {
+      if (f < FEATURES && row < m && col0 + f < n) c[(int64_t)row * ldc + col0 + f] = (float)total;
+    }
   }
 }
 
@@ -398,11 +408,11 @@ static void launch_tiles(const float* a, int64_t lda, const float* w, int64_t ld
   else gemm_f32_kernel<BM, STAGE, false><<<grid, 256, 0, stream>>>(a, lda, w, ldw, c, ldc, m, n, k);
 }
 
-template <int G, int FEATURES>
+template <int G, int FEATURES, bool GATED = false>
 static void launch_few(const float* a, int64_t lda, const float* w, int64_t ldw, float* c, int64_t ldc, int m, int n, int k,
                        hipStream_t stream) {
   const int chunk = min(segment_slices(k), 16 / G);
-  gemm_f32_few_kernel<G, FEATURES><<<ceil_div(n, FEATURES), SEGMENTS * MI_WAVE, SEGMENTS * chunk * G * 32 * sizeof(float4), stream>>>(
+  gemm_f32_few_kernel<G, FEATURES, GATED><<<ceil_div(n, GATED ? 8 : FEATURES), SEGMENTS * MI_WAVE, SEGMENTS * chunk * G * 32 * sizeof(float4), stream>>>(
       a, lda, w, ldw, c, ldc, m, n, k, chunk);
 }
 
@@ -413,6 +423,29 @@ static void launch_rows(const float* a, int64_t lda, const float* w, int64_t ldw
   if (form == LINES) gemm_f32_rows_kernel<RT, FT, LINES><<<grid, block, 0, stream>>>(a, lda, w, ldw, c, ldc, m, n, k);
   else if (form == PIECES) gemm_f32_rows_kernel<RT, FT, PIECES><<<grid, block, 0, stream>>>(a, lda, w, ldw, c, ldc, m, n, k);
   else gemm_f32_rows_kernel<RT, FT, VALUES><<<grid, block, 0, stream>>>(a, lda, w, ldw, c, ldc, m, n, k);
+}
+
+// Whether gemm_f32_few_kernel is the faster one (figures there).
+static bool few_rows_take(int m, int k) { return m <= (segment_slices(k) <= 16 ? 8 : 4); }
+
+// Whole lines of W, rows of A on 16 bytes; the streaming loads' offsets reach over `rows` rows of W in 32 bits.
+static bool whole_lines(const float* a, int64_t lda, const float* w, int64_t ldw, int k, int64_t rows) {
+  return lda % 4 == 0 && (uintptr_t)a % 16 == 0 && k % SLICE == 0 && ldw % 32 == 0 && (uintptr_t)w % 128 == 0 && rows * ldw < (1 << 29);
+}
+
+// silu(a * gate^T) * (a * up^T) of a few rows, w = [gate; up] of n rows each.
+extern "C" int mi_gemm_f32_swiglu_takes(const float* a, int64_t lda, const float* w, int64_t ldw, int m, int n, int k) {
+  return m >= 1 && n >= 1 && k >= 1 && lda >= k && ldw >= k && few_rows_take(m, k) && whole_lines(a, lda, w, ldw, k, (int64_t)n + 8) ? 1 : 0;
+}
+
+extern "C" int mi_gemm_f32_swiglu(const float* a, int64_t lda, const float* w, int64_t ldw, float* c, int64_t ldc, int m, int n, int k,
+                                  hipStream_t stream) {
+  MI_REQUIRE(mi_gemm_f32_swiglu_takes(a, lda, w, ldw, m, n, k) && ldc >= n, "gemm_f32_swiglu: m=%d n=%d k=%d lda=%lld ldw=%lld ldc=%lld is not taken", m,
+             n, k, (long long)lda, (long long)ldw, (long long)ldc);
+  if (m > 4) launch_few<2, 16, true>(a, lda, w, ldw, c, ldc, m, n, k, stream);
+  else launch_few<1, 16, true>(a, lda, w, ldw, c, ldc, m, n, k, stream);
+  MI_CHECK_LAUNCH("gemm_f32_swiglu");
+  return MI_OK;
 }
 
 // Which kernel, with microseconds at rows x N x K (weights from memory; 3 rows: in one 16 x 16 product, for groups of four see
@@ -438,11 +471,10 @@ extern "C" int mi_gemm_f32(const float* a, int64_t lda, const float* w, int64_t 
   const bool a16 = lda % 4 == 0 && (uintptr_t)a % 16 == 0, w16 = ldw % 4 == 0 && (uintptr_t)w % 16 == 0;
   const bool wide = n >= 8192;
   if (m <= 32 || (m <= 64 && !wide)) {
-    // (the streaming loads' offsets reach over a block's 32 features in 32 bits: ldw under 2^24 values)
-    const bool lines = a16 && k % SLICE == 0 && ldw % 32 == 0 && (uintptr_t)w % 128 == 0 && ldw < (1 << 24);
+    const bool lines = whole_lines(a, lda, w, ldw, k, 32);
     const int form = lines ? LINES : a16 && w16 && k % 4 == 0 ? PIECES : VALUES;
     const bool half_empty = ceil_div(n, 16) <= 128;
-    if (lines && m <= (segment_slices(k) <= 16 ? 8 : 4)) {
+    if (lines && few_rows_take(m, k)) {
       if (m > 4) half_empty ? launch_few<2, 8>(a, lda, w, ldw, c, ldc, m, n, k, stream) : launch_few<2, 16>(a, lda, w, ldw, c, ldc, m, n, k, stream);
       else half_empty ? launch_few<1, 8>(a, lda, w, ldw, c, ldc, m, n, k, stream) : launch_few<1, 16>(a, lda, w, ldw, c, ldc, m, n, k, stream);
     } else if (m > 32) launch_rows<4, 1>(a, lda, w, ldw, c, ldc, m, n, k, form, stream);

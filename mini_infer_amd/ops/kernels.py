@@ -751,8 +751,8 @@ def linear_swiglu(x: "torch.Tensor | ScaledRows", gate_up_weight: torch.Tensor) 
     """`silu(x @ gate.T) * (x @ up.T)` with `gate_up_weight` = [gate; up] stacked, [2I, K].
 
     bfloat16 with at most 32 rows, and up to some hundreds where that is faster (`gated_tiles_for`), runs as ONE
-    hand-written kernel (the product with the activation in its last step); otherwise the product and `silu_mul` run in turn.
-    Both ways round the two products to the element type before the activation, so given
+    hand-written kernel (the product with the activation in its last step), and so do up to 8 float32 rows (4 of a long K);
+    otherwise the product and `silu_mul` run in turn.  Both ways round the two products to the element type before the activation, so given
     the same rows a token's result does not depend on which one ran.  `x` may be
     `ScaledRows`: the rows' factors are then applied to the sums of the two products (the same
     kernel with one more step), or to `x` first where that kernel does not take the shapes.
@@ -812,6 +812,16 @@ def linear_swiglu(x: "torch.Tensor | ScaledRows", gate_up_weight: torch.Tensor) 
             )
         )
         return out
+    if (
+        x.dtype == torch.float32 and gate_up_weight.dtype == torch.float32 and x.dim() == 2 and x.shape[1] == width
+        and x.stride(1) == 1 and gate_up_weight.stride(1) == 1 and x.shape[0] > 0 and rows > 0 and x.is_cuda and gate_up_weight.is_cuda
+    ):
+        lib, m, n = library.load(), x.shape[0], rows // 2
+        matrices = (_ptr(x), x.stride(0), _ptr(gate_up_weight), gate_up_weight.stride(0))
+        if lib.mi_gemm_f32_swiglu_takes(*matrices, m, n, width):
+            out = torch.empty((m, n), dtype=torch.float32, device=x.device)
+            library.check(lib.mi_gemm_f32_swiglu(*matrices, _ptr(out), n, m, n, width, _stream()))
+            return out
     return silu_mul(linear(x, gate_up_weight))
 
 

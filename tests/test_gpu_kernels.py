@@ -131,6 +131,20 @@ def test_few_rows_of_gemm_f32_in_groups_of_four(m, n, k):
     assert ((out.double() - exact).abs() <= 2.0 ** -24 * exact.abs() + 1e-12 * math.sqrt(k)).all()
 
 
+@pytest.mark.parametrize("m", [1, 4, 5, 8])
+@pytest.mark.parametrize("n,k", [(1, 32), (8, 288), (13, 2080), (700, 4096), (64, 4352)])
+def test_gated_product_of_a_few_float32_rows(m, n, k):
+    """The launch with the activation in its last step (4 rows and 8, a rest of features; above 16 slices a run 8 rows go the other way)
+    gives the bits of the product and `silu_mul` in turn."""
+    from mini_infer_amd import ops
+    from mini_infer_amd.ops import library
+
+    x, w = _rand(m, k, seed=35), _rand(2 * n, k, seed=36, scale=k ** -0.5)
+    taken = library.load().mi_gemm_f32_swiglu_takes(x.data_ptr(), k, w.data_ptr(), k, m, n, k)
+    assert taken == (m <= 4 or k <= 4096)
+    assert torch.equal(ops.linear_swiglu(x, w), ops.silu_mul(ops.gemm_f32(x, w)))
+
+
 @pytest.mark.parametrize("m,n,k", [(1, 16, 32), (16, 8200, 96), (17, 33, 544), (32, 100, 2048), (33, 8, 352), (64, 50, 257), (65, 130, 4096),
                                    (50, 8192, 160), (700, 6200, 100), (90, 70, 36), (80, 70, 900)])
 def test_gemm_f32_kernels_and_alignments_agree(m, n, k):
