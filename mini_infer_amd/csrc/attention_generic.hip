@@ -70,12 +70,9 @@ __device__ __forceinline__ float from_lane(float v, int lane) {
 // WAVES: the block's waves take every WAVES-th 64 keys of the range and are merged in S at the end.  One wave walks
 // its keys at the latency of its loads and instructions, and a few decoded tokens are too few waves to hide that;
 // measured at attn_generic_launch.
-// With several waves (rows in whole 16s) 32 value rows are asked for at once instead of 8, the first of them with the first
-// values of the key rows, before the scores.  A few decoded tokens give a wave one or two 64s of keys, and its time is the waits one after another.  A layer with its
-// combining launch, 3 requests of up to 600 positions, 24 heads of 128 over 8: 43.1 -> 25.1 us (30 of 200: 42.8 -> 21.1); 32 heads of 64 over
-// 8: 21.9 -> 19.5.  (64 value rows, or all 64 values of a key row: the same for heads of 128 and 36 us for heads of 64, where the compiler
-// makes one long straight run of it.)
-template <typename T, int VPL, bool VEC, int WAVES>
+// DEEP (several waves, rows in whole 16s): 32 value rows are asked for at once instead of 8, the first of them with the first
+// values of the key rows, before the scores; measured at attn_generic_launch.
+template <typename T, int VPL, bool VEC, int WAVES, bool DEEP = false>
 __global__ __launch_bounds__(64 * WAVES) void attn_generic_kernel(
     const T* __restrict__ q, int64_t q_row_stride, const T* __restrict__ k_pages,
     const T* __restrict__ v_pages, const int* __restrict__ block_table, int max_blocks,
@@ -88,7 +85,6 @@ __global__ __launch_bounds__(64 * WAVES) void attn_generic_kernel(
   extern __shared__ __align__(8) unsigned char q_lds_bytes[];
   S* q_lds = reinterpret_cast<S*>(q_lds_bytes);  // [GT][head_dim], pre-multiplied by the scale
   constexpr int KV = VEC ? 16 / sizeof(T) : 4;  // elements per step along a key row
-  constexpr bool DEEP = VEC && WAVES > 1;
 
   const int t = blockIdx.x;
   const int group = q_heads / kv_heads;
@@ -147,8 +143,7 @@ __global__ __launch_bounds__(64 * WAVES) void attn_generic_kernel(
     // value rows BATCH at a time, whose loads are in flight together (past the last key: that key again, weight 0)
     constexpr int BATCH = DEEP ? 32 : 8;
     const int n_valid = min(MI_WAVE, b - base);
-    float vv[BATCH][VPL];
-    auto load_values = [&](int j0) {
+    auto load_values = [&](int j0, float (&vv)[BATCH][VPL]) {
 #pragma unroll
       for (int u = 0; u < BATCH; ++u) {
         const int rj = __builtin_amdgcn_readlane(row_idx, min(j0 + u, n_valid - 1));
@@ -173,22 +168,17 @@ __global__ __launch_bounds__(64 * WAVES) void attn_generic_kernel(
         }
       }
     };
-    // (16 values of the key row at a time where rows are whole 16s: their loads are in flight together)
-    constexpr int RUN = VEC ? 16 : KV;
-    float kf[RUN];
-    auto load_key = [&](const T* k_row, int d0) {
-#pragma unroll
-      for (int at = 0; at < RUN; at += KV) {
-        const Pack<T, KV> kk = *reinterpret_cast<const Pack<T, KV>*>(k_row + d0 + at);
-#pragma unroll
-        for (int e = 0; e < KV; ++e) kf[at + e] = to_f32(kk.v[e]);
-      }
-    };
+    float key_early[DEEP ? 16 : 1], value_early[BATCH][VPL];
     if constexpr (DEEP) {  // (all lanes, those past the last key with it)
       const int real = min(key, b - 1), page = bt[real / page_size];
       row_idx = (page * kv_heads + kvh) * page_size + real % page_size;
-      load_key(k_pages + (int64_t)row_idx * head_dim, 0);
-      load_values(0);
+#pragma unroll
+      for (int at = 0; at < 16; at += KV) {
+        const Pack<T, KV> kk = *reinterpret_cast<const Pack<T, KV>*>(k_pages + (int64_t)row_idx * head_dim + at);
+#pragma unroll
+        for (int e = 0; e < KV; ++e) key_early[at + e] = to_f32(kk.v[e]);
+      }
+      load_values(0, value_early);
     }
     if (DEEP || valid) {
       if constexpr (!DEEP) {
@@ -203,11 +193,20 @@ __global__ __launch_bounds__(64 * WAVES) void attn_generic_kernel(
       for (int g = 0; g < GT; ++g)
 #pragma unroll
         for (int e = 0; e < 4; ++e) s4[g][e] = 0;
+      // (16 values of the key row at a time where rows are whole 16s: their loads are in flight together)
+      constexpr int RUN = VEC ? 16 : KV;
       for (int d0 = 0; d0 < head_dim; d0 += RUN) {
-        if constexpr (DEEP) {
-          if (d0 > 0) load_key(k_row, d0);
+        float kf[RUN];
+        if (DEEP && d0 == 0) {
+#pragma unroll
+          for (int e = 0; e < RUN; ++e) kf[e] = key_early[DEEP ? e : 0];
         } else if constexpr (VEC) {
-          load_key(k_row, d0);
+#pragma unroll
+          for (int at = 0; at < RUN; at += KV) {
+            const Pack<T, KV> kk = *reinterpret_cast<const Pack<T, KV>*>(k_row + d0 + at);
+#pragma unroll
+            for (int e = 0; e < KV; ++e) kf[at + e] = to_f32(kk.v[e]);
+          }
         } else {
           // pairs of elements; an even head size ends after the first or the second pair
           const Pack<T, 2> k0 = *reinterpret_cast<const Pack<T, 2>*>(k_row + d0);
@@ -261,7 +260,15 @@ __global__ __launch_bounds__(64 * WAVES) void attn_generic_kernel(
       m[g] = m_new;
     }
     for (int j0 = 0; j0 < n_valid; j0 += BATCH) {
-      if (!DEEP || j0 > 0) load_values(j0);
+      float vv[BATCH][VPL];
+      if (DEEP && j0 == 0) {
+#pragma unroll
+        for (int u = 0; u < BATCH; ++u)
+#pragma unroll
+          for (int v = 0; v < VPL; ++v) vv[u][v] = value_early[u][v];
+      } else {
+        load_values(j0, vv);
+      }
 #pragma unroll
       for (int u = 0; u < BATCH; ++u) {
         if (j0 + u < n_valid) {
@@ -464,14 +471,21 @@ static int attn_generic_launch(const void* q, int64_t q_row_stride, const void* 
   // 100 positions (240 blocks) 40 / 36, 60 of 200 113 / 47, 100 of 100 (800 blocks) 63 / 74, 100 of 200 115 / 82, 200 of 100 (1,600)
   // 69 / 108, 200 of 400 313 / 299; 32 heads of 64 over 8: 30 of 200 44 / 20, 100 of 100 30 / 35, 200 of 200 60 / 60.  (One wave before
   // its loads were batched: a prompt of 509 tokens 247, then 148; such prompts now take attention_prompt_f32.hip, 66.)
+  //
+  // Up to three blocks a CU a wave has one or two 64s of keys and its time is the waits one after another, so that more loads in flight
+  // (DEEP) are worth two blocks a CU at once instead of three.  A layer with its combining launch: 24 heads of 128 over 8, 3 tokens of
+  // up to 600 positions 43.1 -> 25.1 us, 30 of 200 (240 blocks) 42.8 -> 21.1, 32 heads, 8 of 2,000 (512) 63.4 -> 41.8; 32 heads of 64 over 8,
+  // 3 of 600 21.9 -> 19.5, 60 of 200 (480) 22.0 -> 20.1, 15 of 1,500 (960, not taken) 43.5 / 41.5, 128 of one prompt (1,024, not taken)
+  // 22.0 / 27.9.  (64 value rows, or all 64 values of a key row: the same for heads of 128 and 36 us for heads of 64, where the
+  // compiler makes one long straight run of it.)
   const int64_t blocks = (int64_t)grid.x * grid.y * grid.z;
   int64_t keys = (int64_t)max_blocks * page_size;  // the most a range can have
   if (window > 0) keys = keys < window ? keys : window;
   if (mask_chunk > 0) keys = keys < mask_chunk ? keys : mask_chunk;
   keys = ceil_div64(keys, num_splits);
   const bool four = sizeof(S) == 8 && v_dim <= 128 && blocks < 2048 && keys > MI_WAVE * ceil_div64(blocks, 768);
-#define MI_ATTN_LAUNCH_WAVES(VPL, VEC, WAVES, LDS)                                                \
-  attn_generic_kernel<T, VPL, VEC, WAVES><<<grid, WAVES * MI_WAVE, LDS, stream>>>(                \
+#define MI_ATTN_LAUNCH_WAVES(VPL, VEC, WAVES, DEEP, LDS)                                          \
+  attn_generic_kernel<T, VPL, VEC, WAVES, DEEP><<<grid, WAVES * MI_WAVE, LDS, stream>>>(                \
       (const T*)q, q_row_stride, (const T*)k_pages, (const T*)v_pages, block_table, max_blocks,   \
       token_request, positions, (T*)out, out_row_stride, part_acc, part_ml, q_heads, kv_heads,    \
       head_dim, page_size, scale, window, num_splits, slopes, v_dim, v_row_stride, has_sink, sink_logit, mask_chunk, \
@@ -480,11 +494,13 @@ static int attn_generic_launch(const void* q, int64_t q_row_stride, const void* 
   do {                                                                                            \
     if constexpr (sizeof(S) == 8 && VPL <= 2) {                                                   \
       if (four) {                                                                                 \
-        MI_ATTN_LAUNCH_WAVES(VPL, VEC, 4, lds + 3 * GT * (VPL + 1) * MI_WAVE * sizeof(S) + 4 * GT * sizeof(float)); \
+        const size_t merge = 3 * GT * (VPL + 1) * MI_WAVE * sizeof(S) + 4 * GT * sizeof(float);   \
+        if (VEC && blocks <= 768) MI_ATTN_LAUNCH_WAVES(VPL, VEC, 4, VEC, lds + merge);            \
+        else MI_ATTN_LAUNCH_WAVES(VPL, VEC, 4, false, lds + merge);                               \
         break;                                                                                    \
       }                                                                                           \
     }                                                                                             \
-    MI_ATTN_LAUNCH_WAVES(VPL, VEC, 1, lds);                                                       \
+    MI_ATTN_LAUNCH_WAVES(VPL, VEC, 1, false, lds);                                                       \
   } while (0)
   if (v_dim <= 64) { if (vec) MI_ATTN_LAUNCH(1, true); else MI_ATTN_LAUNCH(1, false); }
   else if (v_dim <= 128) { if (vec) MI_ATTN_LAUNCH(2, true); else MI_ATTN_LAUNCH(2, false); }
