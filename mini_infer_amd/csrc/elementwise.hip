@@ -502,12 +502,17 @@ __global__ __launch_bounds__(256) void rope_kv_write_kernel(
 // The same for the usual layout (halves paired, every size a multiple of 4), four
 // elements per thread and step: 8- and 16-byte loads and stores instead of single
 // elements.  Arithmetic and rounding are those of the kernel above.
-template <typename T>
+//
+// PIECES: the projection comes as `num_pieces` float32 sums over ranges of K, [piece][token][width], whose sum in order, rounded to T,
+// is what is rotated and written; rotated queries go to qkv (of any width), nothing else does.  (A launch that adds them by itself: 4.7 us
+// a layer more at 33 to 64 rows.)
+template <typename T, bool PIECES = false>
 __global__ __launch_bounds__(256) void rope_kv_write_vec4_kernel(
     T* __restrict__ qkv, int64_t row_stride, const float* __restrict__ cos_t,
     const float* __restrict__ sin_t, const int* __restrict__ slot_mapping, T* __restrict__ k_pages,
     T* __restrict__ v_pages, int q_heads, int kv_heads, int head_dim, int rotary_dim, int page_size,
-    int v_transposed, int num_tokens, int blocks_y, int v_dim, const float* __restrict__ bias) {
+    int v_transposed, int num_tokens, int blocks_y, int v_dim, const float* __restrict__ bias,
+    const float* __restrict__ pieces, int num_pieces, int width) {
   const int t = blockIdx.x;
   const int first = blockIdx.y * blockDim.x + threadIdx.x;
   const int stride = blockDim.x * blocks_y;
@@ -519,7 +524,21 @@ __global__ __launch_bounds__(256) void rope_kv_write_vec4_kernel(
 
   // four of the row's columns, their biases added
   auto load_biased = [&](int column, float v[4]) {
-    load4(row + column, v);
+    if constexpr (PIECES) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] = 0.f;
+#pragma unroll 4
+      for (int p = 0; p < num_pieces; ++p) {
+        float more[4];
+        load4(pieces + ((int64_t)p * num_tokens + t) * width + column, more);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] += more[i];
+      }
+#pragma unroll
+      for (int i = 0; i < 4; ++i) v[i] = to_f32(from_f32<T>(v[i]));
+    } else {
+      load4(row + column, v);
+    }
     if (bias) {
       float more[4];
       load4(bias + column, more);
@@ -549,7 +568,7 @@ __global__ __launch_bounds__(256) void rope_kv_write_vec4_kernel(
     store4(x + half + j, hi);
   }
   const int pass4 = (head_dim - rotary_dim) / 4;
-  if (bias) {  // (without one the dims that are not rotated stay as they are)
+  if (bias || PIECES) {  // (otherwise the dims that are not rotated stay as they are)
     for (int e = first; e < q_heads * pass4; e += stride) {
       const int column = (e / pass4) * head_dim + rotary_dim + (e % pass4) * 4;
       float x[4];
@@ -580,7 +599,13 @@ __global__ __launch_bounds__(256) void rope_kv_write_vec4_kernel(
   }
   if (v_transposed && mi_fills_page(slot_mapping, t, page, off, page_size, num_tokens)) {
     mi_write_page_rows(v_pages, t, page, off, page_size, kv_heads, v_dim, first, stride, [&](int token, int e) {
-      const float x = to_f32(qkv[(int64_t)token * row_stride + v_col + e]);
+      float x = 0.f;
+      if constexpr (PIECES) {
+        for (int p = 0; p < num_pieces; ++p) x += pieces[((int64_t)p * num_tokens + token) * width + v_col + e];
+        x = to_f32(from_f32<T>(x));
+      } else {
+        x = to_f32(qkv[(int64_t)token * row_stride + v_col + e]);
+      }
       return bias ? x + bias[v_col + e] : x;
     });
     return;
@@ -601,19 +626,31 @@ __global__ __launch_bounds__(256) void rope_kv_write_vec4_kernel(
 }
 
 // bias: float32 [q heads | k heads | v heads], added to the projection's columns before anything else, or null
+// Whether mi_rope_kv_write adds up a projection left in pieces (bfloat16, tensors on 16 bytes, value heads in whole 4s).
+extern "C" int mi_rope_takes_pieces(int head_dim, int rotary_dim, int interleaved) {
+  return !interleaved && head_dim > 0 && head_dim % 4 == 0 && rotary_dim % 8 == 0 ? 1 : 0;
+}
+
+// pieces (may be null): [num_pieces][num_tokens][width] float32, the projection's sums over ranges of K; qkv then takes the rotated
+// queries only.
 extern "C" int mi_rope_kv_write(int dtype, void* qkv, int64_t row_stride, const float* cos_t,
                                 const float* sin_t, const int* slot_mapping, void* k_pages,
                                 void* v_pages, int num_tokens, int q_heads, int kv_heads,
                                 int head_dim, int rotary_dim, int interleaved, int page_size,
-                                int num_pages, int v_transposed, int v_head_dim, const float* bias, hipStream_t stream) {
+                                int num_pages, int v_transposed, int v_head_dim, const float* bias, const float* pieces,
+                                int num_pieces, int width, hipStream_t stream) {
   if (v_head_dim <= 0) v_head_dim = head_dim;  // values as wide as keys
   MI_REQUIRE(num_tokens >= 0 && q_heads >= 0 && kv_heads >= 0 && head_dim > 0,
              "rope_kv_write: bad sizes tokens=%d q_heads=%d kv_heads=%d head_dim=%d", num_tokens,
              q_heads, kv_heads, head_dim);
   MI_REQUIRE(rotary_dim >= 0 && rotary_dim <= head_dim && rotary_dim % 2 == 0,
              "rope_kv_write: rotary_dim=%d must be even and at most head_dim=%d", rotary_dim, head_dim);
-  MI_REQUIRE(row_stride >= (int64_t)(q_heads + kv_heads) * head_dim + (int64_t)kv_heads * v_head_dim,
+  const int64_t projected = (int64_t)(q_heads + kv_heads) * head_dim + (int64_t)kv_heads * v_head_dim;
+  MI_REQUIRE(row_stride >= (pieces ? (int64_t)q_heads * head_dim : projected),
              "rope_kv_write: row stride %lld is shorter than the q, k and v heads", (long long)row_stride);
+  MI_REQUIRE(!pieces || (num_pieces >= 1 && width >= projected && width % 4 == 0 && (uintptr_t)pieces % 16 == 0 && dtype == MI_BF16 &&
+                         mi_rope_takes_pieces(head_dim, rotary_dim, interleaved) && v_head_dim % 4 == 0),
+             "rope_kv_write: %d pieces of rows of %d are not taken", num_pieces, width);
   MI_REQUIRE(kv_heads == 0 || slot_mapping == nullptr || (page_size > 0 && num_pages > 0 && k_pages && v_pages),
              "rope_kv_write: pages are needed to write keys and values");
   MI_REQUIRE(dtype == MI_F32 || dtype == MI_BF16, "rope_kv_write: unknown dtype %d", dtype);
@@ -622,6 +659,7 @@ extern "C" int mi_rope_kv_write(int dtype, void* qkv, int64_t row_stride, const 
   const size_t elem = dtype == MI_F32 ? 4 : 2;
   const bool aligned = ((uintptr_t)qkv | (uintptr_t)cos_t | (uintptr_t)sin_t | (uintptr_t)k_pages |
                         (uintptr_t)v_pages | (uintptr_t)(row_stride * elem) | (uintptr_t)bias) % 16 == 0;
+  MI_REQUIRE(aligned || !pieces, "rope_kv_write: pieces go with tensors on 16 bytes");
   if (!interleaved && aligned && head_dim % 4 == 0 && rotary_dim % 8 == 0 && v_head_dim % 4 == 0) {
     const int items = max(q_heads * (rotary_dim / 8), kv_heads * (max(head_dim, v_head_dim) / 4));
     const int blocks_y = min((num_tokens >= 512) ? 2 : 16, max(1, ceil_div(items, 256)));
@@ -629,11 +667,12 @@ extern "C" int mi_rope_kv_write(int dtype, void* qkv, int64_t row_stride, const 
     if (dtype == MI_F32) {
       rope_kv_write_vec4_kernel<float><<<grid, 256, 0, stream>>>(
           (float*)qkv, row_stride, cos_t, sin_t, slot_mapping, (float*)k_pages, (float*)v_pages,
-          q_heads, kv_heads, head_dim, rotary_dim, page_size, v_transposed, num_tokens, blocks_y, v_head_dim, bias);
+          q_heads, kv_heads, head_dim, rotary_dim, page_size, v_transposed, num_tokens, blocks_y, v_head_dim, bias, nullptr, 0, 0);
     } else {
-      rope_kv_write_vec4_kernel<bf16_t><<<grid, 256, 0, stream>>>(
-          (bf16_t*)qkv, row_stride, cos_t, sin_t, slot_mapping, (bf16_t*)k_pages, (bf16_t*)v_pages,
-          q_heads, kv_heads, head_dim, rotary_dim, page_size, v_transposed, num_tokens, blocks_y, v_head_dim, bias);
+      const auto kernel = pieces ? rope_kv_write_vec4_kernel<bf16_t, true> : rope_kv_write_vec4_kernel<bf16_t>;
+      kernel<<<grid, 256, 0, stream>>>((bf16_t*)qkv, row_stride, cos_t, sin_t, slot_mapping, (bf16_t*)k_pages, (bf16_t*)v_pages, q_heads,
+                                       kv_heads, head_dim, rotary_dim, page_size, v_transposed, num_tokens, blocks_y, v_head_dim, bias, pieces,
+                                       num_pieces, width);
     }
     MI_CHECK_LAUNCH("rope_kv_write");
     return MI_OK;

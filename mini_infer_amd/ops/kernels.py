@@ -271,8 +271,13 @@ def rope_table(positions: torch.Tensor, inv_freq: torch.Tensor, amplitude: float
     return cos, sin
 
 
+def rope_takes_partial_sums(head_dim: int, rotary_dim: int, interleaved: bool) -> bool:
+    """Whether `rope_kv_write` takes the projection of such heads as `PartialSums`."""
+    return bool(library.load().mi_rope_takes_pieces(head_dim, rotary_dim, int(interleaved)))
+
+
 def rope_kv_write(
-    qkv: torch.Tensor,
+    qkv: "torch.Tensor | PartialSums",
     cos: torch.Tensor,
     sin: torch.Tensor,
     slot_mapping: torch.Tensor | None,
@@ -287,8 +292,9 @@ def rope_kv_write(
     v_transposed: bool = False,
     v_head_dim: int | None = None,
     bias: torch.Tensor | None = None,
-) -> None:
-    """Rotate q in place inside `qkv`; rotate k and write k, v into their page slots.
+) -> torch.Tensor:
+    """Rotate q in place inside `qkv`, rotate k and write k, v into their page slots; returns `qkv`.  A projection that comes as
+    `PartialSums` (`rope_takes_partial_sums`) is added up on the way: what is returned then holds the rotated queries alone.
     `v_head_dim`: the width of a value head where it is not the keys' (`head_dim`).
     `bias` (float32, one number per column of q, k and v): added to the projection before anything else.
 
@@ -297,6 +303,14 @@ def rope_kv_write(
     [num_pages, kv_heads, head_dim, page_size] with `v_transposed`.  `kv_heads=0`
     rotates q only.
     """
+    pieces, width = None, 0
+    if isinstance(qkv, PartialSums):
+        pieces, width = qkv.pieces, qkv.pieces.shape[2]
+        _need_cuda(pieces)
+        _need_contiguous("pieces", pieces)
+        if width < (q_heads + kv_heads) * head_dim + kv_heads * (head_dim if v_head_dim is None else int(v_head_dim)):
+            raise KernelShapeError(f"qkv rows hold {width} values, fewer than the q, k and v heads need")
+        qkv = torch.empty((pieces.shape[1], q_heads * head_dim), dtype=qkv.dtype, device=pieces.device)
     _need_cuda(qkv, cos, sin, slot_mapping, k_pages, v_pages)
     _need_contiguous("cos", cos)
     _need_contiguous("sin", sin)
@@ -308,7 +322,7 @@ def rope_kv_write(
         raise KernelShapeError(f"qkv must be [T, width] with unit inner stride, got {qkv.stride()}")
     tokens = qkv.shape[0]
     v_dim = head_dim if v_head_dim is None else int(v_head_dim)
-    if qkv.shape[1] < (q_heads + kv_heads) * head_dim + kv_heads * v_dim:
+    if pieces is None and qkv.shape[1] < (q_heads + kv_heads) * head_dim + kv_heads * v_dim:
         raise KernelShapeError(
             f"qkv rows hold {qkv.shape[1]} values, fewer than the q, k and v heads need: "
             f"{(q_heads + kv_heads) * head_dim + kv_heads * v_dim}"
@@ -341,9 +355,11 @@ def rope_kv_write(
         lib.mi_rope_kv_write(
             _dtype_code(qkv), _ptr(qkv), qkv.stride(0), _ptr(cos), _ptr(sin), _ptr(slot_mapping),
             _ptr(k_pages), _ptr(v_pages), tokens, q_heads, kv_heads, head_dim, rotary_dim,
-            int(interleaved), page_size, num_pages, int(v_transposed), v_dim, _ptr(bias), _stream(),
+            int(interleaved), page_size, num_pages, int(v_transposed), v_dim, _ptr(bias), _ptr(pieces),
+            0 if pieces is None else pieces.shape[0], width, _stream(),
         )
     )
+    return qkv
 
 
 def silu_mul(gate_up: torch.Tensor) -> torch.Tensor:

@@ -14,7 +14,7 @@ from pathlib import Path
 from mini_infer_amd.exceptions import ExtensionMissingError, KernelShapeError
 from mini_infer_amd.ops import build as _build
 
-ABI_VERSION = 41
+ABI_VERSION = 42
 
 _lib: ctypes.CDLL | None = None
 _lib_path: Path | None = None
@@ -26,9 +26,10 @@ _SIGNATURES: dict[str, list] = {
     "mi_begin_step": [_P, _P, _P, c_int, c_int, c_int, _P, _P, _P, c_int, c_int, _P],
     "mi_add_rmsnorm": [c_int, _P, _P, _P, _P, _P, c_int, c_int, c_float, _P, c_int, c_int64, _P],
     "mi_rope_table": [_P, _P, _P, _P, c_int, c_int, c_float, _P],
+    "mi_rope_takes_pieces": [c_int, c_int, c_int],
     "mi_rope_kv_write": [
         c_int, _P, c_int64, _P, _P, _P, _P, _P, c_int, c_int, c_int, c_int, c_int, c_int, c_int,
-        c_int, c_int, c_int, _P, _P,
+        c_int, c_int, c_int, _P, _P, c_int, c_int, _P,
     ],
     "mi_silu_mul": [c_int, _P, _P, c_int, c_int, _P],
     "mi_gemm_f32": [_P, c_int64, _P, c_int64, _P, c_int64, c_int, c_int, c_int, _P],

@@ -288,7 +288,12 @@ class GQAttention(Mixer):
             )
             return self._project(self._attend(queries, ctx, cache))
         if writes_cache:
-            qkv = self.qkv.forward(x)
+            # A projection left in pieces is added up by the rotation's launch, in steps of single tokens: 8B sizes, 40 of them,
+            # 4,650 -> 4,500 us a step.  A portion's values are written a page at a time, sixteen tokens a thread, and all their
+            # pieces there cost more than a launch (60 tokens beside 9 single ones, 8B 5,420 -> 5,950; 100 beside 10, 1B 1,567 -> 1,851).
+            in_pieces = (ctx.max_q_len == 1 and rotary is not None and self._same_widths and self._plain_heads
+                         and ops.rope_takes_partial_sums(self.head_dim, rotary.rotary_dim, rotary.interleaved))
+            qkv = self.qkv.forward(x, partial_ok=in_pieces)
             kv_heads, slots = self.num_kv_heads, ctx.slot_mapping[cache.group]
         else:
             # reads another call's keys and values: only q is projected
@@ -309,7 +314,7 @@ class GQAttention(Mixer):
                 v_head_dim=self.v_head_dim,
             )
         else:
-            ops.rope_kv_write(
+            qkv = ops.rope_kv_write(
                 qkv, cos, sin, slots, cache.k_pages, cache.v_pages,
                 q_heads=self.num_heads, kv_heads=kv_heads, head_dim=self.head_dim,
                 rotary_dim=rotary_dim, interleaved=interleaved, v_transposed=cache.v_transposed,

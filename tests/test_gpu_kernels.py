@@ -477,6 +477,30 @@ def test_rope_kv_write(dtype, q_heads, kv_heads, head_dim, rotary_dim, interleav
         assert torch.equal(qkv[0, : q_heads * head_dim], original[0, : q_heads * head_dim])
 
 
+@pytest.mark.parametrize("transposed", [False, True])
+@pytest.mark.parametrize("q_heads,kv_heads,head_dim,rotary_dim,extra,writes", [
+    (24, 8, 128, 128, 0, True), (3, 1, 64, 32, 4, True), (4, 2, 72, 8, 0, True), (8, 2, 64, 64, 0, False)])
+@pytest.mark.parametrize("tokens,pieces", [(1, 2), (17, 3), (700, 16)])
+def test_rope_kv_write_of_a_projection_in_pieces(q_heads, kv_heads, head_dim, rotary_dim, extra, writes, transposed, tokens, pieces):
+    """The bits of the same with the pieces added up first (`PartialSums.finish`): whole heads and parts rotated, pages filled whole and
+    not, a token without a slot, a step that writes nothing."""
+    from mini_infer_amd import ops
+
+    page, width = 16, (q_heads + 2 * kv_heads) * head_dim + extra
+    sums = ops.PartialSums(_rand(pieces, tokens, width, seed=1), torch.bfloat16)
+    cos, sin = _rand(tokens, rotary_dim // 2, seed=2), _rand(tokens, rotary_dim // 2, seed=3)
+    slots = torch.arange(5, tokens + 5, dtype=torch.int32, device=DEV)
+    slots[tokens // 2] = -1
+    results = []
+    for qkv in (sums, sums.finish()):
+        k_pages = torch.zeros((tokens // page + 2, kv_heads, page, head_dim), dtype=torch.bfloat16, device=DEV)
+        v_pages = torch.zeros_like(k_pages.transpose(2, 3).contiguous() if transposed else k_pages)
+        queries = ops.rope_kv_write(qkv, cos, sin, slots if writes else None, k_pages, v_pages, q_heads=q_heads, kv_heads=kv_heads if writes else 0,
+                                    head_dim=head_dim, rotary_dim=rotary_dim, v_transposed=transposed)
+        results.append((queries[:, : q_heads * head_dim], k_pages, v_pages))
+    assert all(torch.equal(a, b) for a, b in zip(*results)) and bool(results[0][1].any()) == (writes and tokens > 1)
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("page_size", [16, 8])
 @pytest.mark.parametrize("more_pages", [0, 40])  # 40 more whole pages: the rows of a prompt's portion
