@@ -578,11 +578,13 @@ def tiles_for(m: int, n: int, k: int, partial_ok: bool) -> tuple[int, int] | Non
         rows           17    32    64    128   192   256   272   320   400   600   900
         all in tiles   1.51  1.46  1.44  1.33  1.42  1.22  1.13  1.11  1.06  1.01  0.96
                        1.22  1.17  1.20  1.19  1.33  1.17  1.08  1.06  1.04  0.99  0.95
-        by this rule   1.51  1.46  1.44  1.34  1.42  1.23  1.11  1.10  1.07  1.05  1.02
-                       1.17  1.16  1.16  1.19  1.29  1.18  1.07  1.06  1.05  1.04  1.02
+        by this rule   1.51  1.46  1.44  1.34  1.42  1.23  1.13  1.11  1.07  1.05  1.02
+                       1.17  1.16  1.16  1.19  1.29  1.18  1.08  1.06  1.05  1.04  1.02
 
-    The library does not cut K and so leaves CUs idle where there are few features; from 256 rows on it is about as fast as whole
-    tiles, and cutting has to pay.  It is faster (tiles 0.75 to 0.95) for the widest matrices, and where the whole product takes
+    The library does not cut K and so leaves CUs idle where there are few features; from some 300 rows on it is about as fast as whole
+    tiles, and cutting has to pay.  (Up to 320 rows tiles without that: they are as fast or faster, 3072 x 3072 at 271 rows 15.3 against
+    19.7 us, 5120 x 3072 20.8 / 20.7, at worst 10240 x 3072 31.3 / 28.8; and a call of the library costs the host 20 us, one of these 8, of
+    which a step of that many tokens at 3B widths waits for the host.)  It is faster (tiles 0.75 to 0.95) for the widest matrices, and where the whole product takes
     it less than 9 microseconds and the sum needs a launch of its own."""
     if not SKINNY_MAX_ROWS < m <= TILES_MAX_ROWS:
         return None
@@ -591,7 +593,7 @@ def tiles_for(m: int, n: int, k: int, partial_ok: bool) -> tuple[int, int] | Non
     each = m * n * 4 / SUM_BYTES_A_MICRO
     whole, _, _ = _tiles_plan(m, n, k, False, 1, False, 0.0, 0.0)
     micros, shape, ranges = _tiles_plan(m, n, k, False, 16, False, 0.0 if partial_ok else SUM_LAUNCH_MICROS, each)
-    if m > 256 and micros > 0.88 * whole:
+    if m > 320 and micros > 0.88 * whole:
         return None
     return shape, ranges
 
