@@ -2845,8 +2845,36 @@ def embed_pair_hash(
     return out, cast
 
 
+@dataclasses.dataclass
+class ExpertRows:
+    """The rows that a token's chosen experts made (`experts_by_expert(leave_rows=True)`), not added up yet:
+    `sum_k weights[t, k] * made[t * top + k] (+ shared_gate[t] * shared[t])`, a choice past the real experts standing for `x[t]`
+    itself.  `scale_add_norm` adds them on its way; anything else calls `finish()`."""
+
+    made: torch.Tensor  # [tokens * top, width]
+    chosen: torch.Tensor
+    weights: torch.Tensor | None
+    x: torch.Tensor
+    shared: torch.Tensor | None
+    shared_gate: torch.Tensor | None
+    experts: int
+    top: int
+
+    def operands(self) -> tuple:
+        """(made, chosen, weights, x, its stride, shared, its stride, gate) as the library takes them."""
+        return (_ptr(self.made), _ptr(self.chosen), _ptr(self.weights), _ptr(self.x), self.x.stride(0), _ptr(self.shared),
+                0 if self.shared is None else self.shared.stride(0), _ptr(self.shared_gate))
+
+    def finish(self) -> torch.Tensor:
+        out = torch.empty((self.made.shape[0] // self.top, self.made.shape[1]), dtype=self.made.dtype, device=self.made.device)
+        made, *others = self.operands()
+        library.check(library.load().mi_expert_combine(
+            _dtype_code(self.made), made, None, *others, _ptr(out), out.shape[0], out.shape[1], self.experts, self.top, _stream()))
+        return out
+
+
 def scale_add_norm(
-    residual: torch.Tensor, y: torch.Tensor | None, scale: torch.Tensor | None, factor: torch.Tensor, alpha: float,
+    residual: torch.Tensor, y: "torch.Tensor | ExpertRows | None", scale: torch.Tensor | None, factor: torch.Tensor, alpha: float,
     eps: float, dtype: torch.dtype, rows: torch.Tensor | None = None, want_cast: bool = True,
 ) -> torch.Tensor | None:
     """The norm behind the sum: `x <- rms_norm(alpha * x + scale * y) * factor` row by row, in place
@@ -2854,6 +2882,12 @@ def scale_add_norm(
     is `alpha * x + y`; without `y` the row is normed as it is).  With `want_cast` the new rows are
     returned in `dtype` as well.  With `rows` (int32) only those rows are normed, the stream stays
     as it was and the normed rows come back [len(rows), H]."""
+    experts = (None, None, None, None, 0, None, 0, None, 0, 0)
+    picked = rows is not None and y is not None
+    if isinstance(y, ExpertRows):
+        if y.made.dtype != dtype or tuple(y.made.shape) != (residual.shape[0] * y.top, residual.shape[1]):
+            raise KernelShapeError(f"scale_add_norm: experts' rows {tuple(y.made.shape)} {y.made.dtype} do not fit the stream {tuple(residual.shape)} in {dtype}")
+        experts, y = (*y.operands(), y.experts, y.top), None
     _need_cuda(residual, y, scale, factor, rows)
     for name, t in (("residual", residual), ("scale", scale), ("factor", factor), ("rows", rows)):
         _need_contiguous(name, t)
@@ -2866,14 +2900,14 @@ def scale_add_norm(
         raise KernelShapeError(f"scale_add_norm: y {tuple(y.shape)} {y.dtype} does not fit the stream {(tokens, hidden)} in {dtype}")
     if factor.numel() != hidden or (scale is not None and scale.numel() != hidden):
         raise KernelShapeError(f"scale_add_norm: one factor (and one scale) per column of {hidden}")
-    if rows is not None and y is not None:
+    if picked:
         raise KernelShapeError("scale_add_norm: rows are picked for the norm alone")
     count = tokens if rows is None else rows.numel()
     cast = torch.empty((count, hidden), dtype=dtype, device=residual.device) if (want_cast or rows is not None) else None
     library.check(
         library.load().mi_scale_add_norm(
             F32 if dtype == torch.float32 else BF16, _ptr(residual), _ptr(y), 0 if y is None else y.stride(0), _ptr(scale),
-            _ptr(factor), _ptr(rows), _ptr(cast), count, hidden, float(alpha), float(eps), _stream(),
+            _ptr(factor), _ptr(rows), _ptr(cast), count, hidden, float(alpha), float(eps), *experts, _stream(),
         )
     )
     return cast
@@ -3161,7 +3195,8 @@ def experts_by_expert(
     x: torch.Tensor, gate_up: torch.Tensor, down: torch.Tensor, chosen: torch.Tensor, weights: torch.Tensor,
     shared: torch.Tensor | None = None, shared_gate: torch.Tensor | None = None, tiles: str | None = None, *,
     activation: str = "silu_gated", weight_on: str = "output", combine: bool = True, lists: ExpertLists | None = None,
-) -> "torch.Tensor | SummedRows | WeightedRows":
+    leave_rows: bool = False,
+) -> "torch.Tensor | SummedRows | WeightedRows | ExpertRows":
     """The same sum as `experts_few_rows`, expert by expert without the host knowing anything: one small
     kernel lists the (row, expert) pairs by expert, then every chosen expert's block streams its
     weights once for up to eight of the expert's rows at a time (the rows wait in LDS), and one kernel adds
@@ -3171,7 +3206,7 @@ def experts_by_expert(
     expert's rows a pass, and "lds", tiles of 128 rows x 128 features with both operands staged through LDS
     (rows in steps of 64 elements).  `combine=False`
     (no shared or identity experts): the rows are left for a norm to add up (`SummedRows`; weights on the
-    output: `WeightedRows`).
+    output: `WeightedRows`).  `leave_rows`: the sum of any experts is left to a norm behind it (`ExpertRows`).
     `lists`: the pairs by expert where `route_top_k` has made them already."""
     tokens, width, experts, ff, top = _check_experts(x, gate_up, down, chosen, weights, shared, shared_gate, activation, weight_on)
     mode, on_input, on_output = _expert_weights(activation, weights, weight_on)
@@ -3207,11 +3242,8 @@ def experts_by_expert(
                                          width, experts, ff, width, many, _stream()))
     if not combine:
         return SummedRows(made, top) if on_output is None else WeightedRows(made, weights)
-    out = torch.empty((tokens, width), dtype=x.dtype, device=x.device)
-    library.check(lib.mi_expert_combine(
-        code, _ptr(made), None, _ptr(chosen), _ptr(on_output), _ptr(x), x.stride(0), _ptr(shared),
-        0 if shared is None else shared.stride(0), _ptr(shared_gate), _ptr(out), tokens, width, experts, top, _stream()))
-    return out
+    rows = ExpertRows(made, chosen, on_output, x, shared, shared_gate, experts, top)
+    return rows if leave_rows else rows.finish()
 
 
 def experts_grouped(

@@ -14,7 +14,7 @@ from pathlib import Path
 from mini_infer_amd.exceptions import ExtensionMissingError, KernelShapeError
 from mini_infer_amd.ops import build as _build
 
-ABI_VERSION = 42
+ABI_VERSION = 43
 
 _lib: ctypes.CDLL | None = None
 _lib_path: Path | None = None
@@ -147,7 +147,9 @@ _SIGNATURES: dict[str, list] = {
     ],
     "mi_gated_mul": [c_int, c_int, _P, c_int64, _P, c_int64, _P, c_int64, c_int, c_int, _P],
     "mi_embed_pair_hash": [c_int, _P, _P, _P, _P, _P, _P, _P, _P, c_int64, c_int, _P, _P, c_int, c_int, c_int, c_int, c_int, c_int, _P],
-    "mi_scale_add_norm": [c_int, _P, _P, c_int64, _P, _P, _P, _P, c_int, c_int, c_float, c_float, _P],
+    "mi_scale_add_norm": [
+        c_int, _P, _P, c_int64, _P, _P, _P, _P, c_int, c_int, c_float, c_float, _P, _P, _P, _P, c_int64, _P, c_int64, _P, c_int, c_int, _P,
+    ],
     "mi_norm_rows": [c_int, _P, c_int64, _P, _P, c_int64, c_int, c_int, c_float, _P],
     "mi_qkv_norm_write": [
         c_int, _P, c_int64, _P, _P, _P, c_int64, _P, _P, _P, _P, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int,

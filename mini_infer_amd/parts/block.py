@@ -467,6 +467,8 @@ class PostNormBlock(Block):
         super().__init__(dtype, device)
         self.mixer_norm, self.mixer, self.ffn_norm, self.feed_forward = mixer_norm, mixer, ffn_norm, feed_forward
         self.hidden_size, self.alpha, self.layer_scale, self.names = hidden_size, float(alpha), bool(layer_scale), names
+        if getattr(ffn_norm, "takes_expert_rows", False) and hasattr(feed_forward, "leave_expert_rows"):
+            feed_forward.leave_expert_rows = True
         self.mixer_scale: torch.Tensor | None = None
         self.ffn_scale: torch.Tensor | None = None
 

@@ -355,6 +355,8 @@ class RoutedExperts(FeedForward):
         self.down: torch.Tensor | None = None  # [experts, hidden, ff]
         # set by a block whose norms add up `ops.SummedRows` on their way
         self.leave_rows_apart = False
+        # set by a block whose norm adds up `ops.ExpertRows` on its way
+        self.leave_expert_rows = False
         self.force_form: str | None = None  # "few", "by_expert" or "grouped": for tests and measurements
 
     def _expert_name(self, prefix: str, e: int, which: str) -> str:
@@ -431,6 +433,8 @@ class RoutedExperts(FeedForward):
         elif by_expert:
             run = ops.experts_by_expert
             how["lists"] = lists[0]
+            # (float32 rows are the stream itself, which that norm writes)
+            how["leave_rows"] = self.leave_expert_rows and x.dtype != torch.float32
             how["combine"] = not (self.leave_rows_apart and shared is None and (self.weight_on == "input" or not self.identity))
         else:
             run = ops.experts_few_rows

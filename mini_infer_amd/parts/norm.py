@@ -199,9 +199,11 @@ class PostRMSNorm(Norm):
     def load_params(self, prefix: str, get: TensorGetter) -> None:
         self.factor = (get(prefix + self.name).float() + self.weight_offset).contiguous()
 
+    takes_expert_rows = True
+
     def norm_sum(self, y, residual, scale=None, alpha=1.0, want_cast=False):
         assert self.factor is not None, "norm used before its weight was loaded"
-        y = y.finish() if hasattr(y, "finish") else y
+        y = y.finish() if hasattr(y, "finish") and not isinstance(y, ops.ExpertRows) else y
         return ops.scale_add_norm(residual, y, scale, self.factor, alpha, self.eps, self.dtype, want_cast=want_cast)
 
     def forward(self, delta, residual: torch.Tensor, rows: torch.Tensor | None = None) -> torch.Tensor:

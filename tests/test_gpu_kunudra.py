@@ -166,6 +166,28 @@ def test_the_norm_behind_the_sum(dtype, width, scaled):
     np.testing.assert_allclose(picked.float().cpu().numpy(), again, rtol=0, atol=tolerance(dtype, 4))
 
 
+@pytest.mark.parametrize("tokens,width", [(1, 4096), (8, 1030), (5, 16404), (300, 3072), (300, 4100)])
+@pytest.mark.parametrize("dtype", ["bfloat16", "float32"])
+@pytest.mark.parametrize("shared,gated,weighted", [(True, False, True), (True, True, False), (False, False, True)])
+def test_norm_that_adds_up_the_experts_rows(tokens, width, dtype, shared, gated, weighted):
+    """The bits of `ExpertRows.finish` followed by the norm: identity experts, a choice that is none, with a shared expert, its gate and
+    without; columns kept in registers and made again, single and in fours."""
+    from mini_infer_amd import ops
+
+    g = torch.Generator().manual_seed(7)
+    rand = lambda *shape: torch.randn(shape, generator=g).to("cuda")  # noqa: E731
+    top, experts, kind = 3, 5, TORCH[dtype]
+    chosen = torch.randint(-1, experts + 2, (tokens, top), generator=g).to("cuda", torch.int32)
+    rows = ops.ExpertRows(rand(tokens * top, width).to(kind), chosen, rand(tokens, top) if weighted else None, rand(tokens, width).to(kind),
+                          rand(tokens, width).to(kind) if shared else None, rand(tokens) if gated else None, experts, top)
+    stream, scale, factor = rand(tokens, width), rand(width), rand(width)
+    results = []
+    for y in (rows, rows.finish()):
+        own = stream.clone()
+        results.append((ops.scale_add_norm(own, y, scale if weighted else None, factor, 1.6, 1e-6, kind), own))
+    assert all(torch.equal(a, b) for a, b in zip(*results)) and results[0][1].isfinite().all()
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("width, extra", [(7, 3), (80, 144), (300, 0)])
 def test_a_norm_over_the_first_columns_of_wider_rows(dtype, width, extra):
