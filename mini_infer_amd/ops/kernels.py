@@ -1815,14 +1815,14 @@ class StreamUpdate:
 
         x += scale * (a + b + bias) + shift
 
-    `a`, `b`: a layer's sublayer outputs [T, H] in the compute dtype (either may be None; `b` may be
+    `a`, `b`: a layer's sublayer outputs [T, H] in the compute dtype (either may be None or `PartialSums`; `b` may be
     `WeightedRows`);
     `bias`, `shift`: float32 [H] or None.  A norm that knows it makes the update and its own
     statistics in one launch (`stream_update_norm`); anything else calls `finish()`, which
     returns the whole right-hand side as one float32 tensor to add."""
 
-    a: torch.Tensor | None
-    b: "torch.Tensor | WeightedRows | None" = None
+    a: "torch.Tensor | PartialSums | None"
+    b: "torch.Tensor | PartialSums | WeightedRows | None" = None
     bias: torch.Tensor | None = None
     shift: torch.Tensor | None = None
     scale: float = 1.0
@@ -1836,7 +1836,7 @@ class StreamUpdate:
         total = None
         for part in (self.a, self.b, self.bias):
             if part is not None:
-                part = part.finish() if isinstance(part, WeightedRows) else part
+                part = part.finish() if isinstance(part, (WeightedRows, PartialSums)) else part
                 total = part.float() if total is None else total + part.float()
         if total is not None:
             total = total * self.scale
@@ -1855,14 +1855,23 @@ def stream_update_norm(
     new rows times `weight` (compute dtype) -> [T, H] or [len(rows), H]; `weight=None`: the
     update alone."""
     update = update if update is not None else StreamUpdate(None)
-    b, b_weights, pieces = update.b, None, 1
+    a, b, b_weights, pieces, sums = update.a, update.b, None, 1, []
+    for part in (a, b):
+        partial = part.pieces if isinstance(part, PartialSums) else None
+        _need_cuda(partial)
+        _need_contiguous("partial sums", partial)
+        if partial is not None and (part.dtype != torch.bfloat16 or partial.dtype != torch.float32 or tuple(partial.shape[1:]) != tuple(residual.shape)):
+            raise KernelShapeError(f"stream update: sums {tuple(partial.shape)} of {part.dtype} do not fit the stream {tuple(residual.shape)}")
+        sums += [_ptr(partial), 0 if partial is None else partial.shape[0]]
+    dtype_of_sums = torch.bfloat16 if any(sums) else None
+    a, b = (None if isinstance(part, PartialSums) else part for part in (a, b))
     if isinstance(b, WeightedRows):
         b, b_weights, pieces = b.rows, b.weights, b.weights.shape[1]
         _need_contiguous("b's weights", b_weights)
         _need_f32("b's weights", b_weights)
         if b_weights.shape[0] != residual.shape[0]:
             raise KernelShapeError(f"stream update: weights of {b_weights.shape[0]} tokens for {residual.shape[0]} rows")
-    _need_cuda(update.a, b, b_weights, update.bias, update.shift, residual, weight, rows)
+    _need_cuda(a, b, b_weights, update.bias, update.shift, residual, weight, rows)
     for name, t in (("residual", residual), ("weight", weight), ("rows", rows), ("bias", update.bias), ("shift", update.shift)):
         _need_contiguous(name, t)
     _need_int32("rows", rows)
@@ -1870,8 +1879,10 @@ def stream_update_norm(
     _need_f32("bias", update.bias)
     _need_f32("shift", update.shift)
     tokens, hidden = residual.shape
-    dtype = weight.dtype if weight is not None else (update.a.dtype if update.a is not None else torch.float32)
-    for name, t, count in (("a", update.a, tokens), ("b", b, tokens * pieces)):
+    dtype = weight.dtype if weight is not None else (a.dtype if a is not None else dtype_of_sums or torch.float32)
+    if dtype_of_sums is not None and dtype != dtype_of_sums:
+        raise KernelShapeError(f"stream update: sums of bfloat16 products in a step of {dtype}")
+    for name, t, count in (("a", a, tokens), ("b", b, tokens * pieces)):
         if t is not None and (t.dim() != 2 or tuple(t.shape) != (count, hidden) or t.stride(1) != 1 or t.dtype != dtype):
             raise KernelShapeError(f"stream update: {name} {tuple(t.shape)} {t.dtype} does not fit the stream {(tokens, hidden)} in {dtype}")
     for name, t in (("bias", update.bias), ("shift", update.shift), ("weight", weight)):
@@ -1884,9 +1895,9 @@ def stream_update_norm(
     code = F32 if dtype == torch.float32 else BF16
     library.check(
         library.load().mi_stream_update_norm(
-            code, _ptr(update.a), 0 if update.a is None else update.a.stride(0), _ptr(b),
+            code, _ptr(a), 0 if a is None else a.stride(0), _ptr(b),
             0 if b is None else b.stride(0), _ptr(b_weights), pieces, _ptr(update.bias), _ptr(update.shift), float(update.scale),
-            _ptr(residual), _ptr(weight), _ptr(out), _ptr(rows), n_out, hidden, float(eps), _stream(),
+            _ptr(residual), _ptr(weight), _ptr(out), _ptr(rows), n_out, hidden, float(eps), *sums, tokens, _stream(),
         )
     )
     return out

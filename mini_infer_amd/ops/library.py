@@ -14,7 +14,7 @@ from pathlib import Path
 from mini_infer_amd.exceptions import ExtensionMissingError, KernelShapeError
 from mini_infer_amd.ops import build as _build
 
-ABI_VERSION = 43
+ABI_VERSION = 44
 
 _lib: ctypes.CDLL | None = None
 _lib_path: Path | None = None
@@ -103,7 +103,9 @@ _SIGNATURES: dict[str, list] = {
         c_int, _P, c_int64, _P, _P, _P, c_int, _P, _P, _P, c_int64, _P, _P, c_int, c_int, c_int, c_int, c_int,
         c_int64, c_int, c_int, c_float, c_int, c_int, _P, c_int, c_float, c_int, c_float, _P, _P, c_int64, _P,
     ],
-    "mi_stream_update_norm": [c_int, _P, c_int64, _P, c_int64, _P, c_int, _P, _P, c_float, _P, _P, _P, _P, c_int, c_int, c_float, _P],
+    "mi_stream_update_norm": [
+        c_int, _P, c_int64, _P, c_int64, _P, c_int, _P, _P, c_float, _P, _P, _P, _P, c_int, c_int, c_float, _P, c_int, _P, c_int, c_int, _P,
+    ],
     "mi_clamped_glu": [c_int, _P, c_int64, _P, _P, c_int64, c_int, c_int, c_float, c_float, _P],
     "mi_short_conv": [
         c_int, _P, c_int64, _P, _P, c_int64, _P, _P, _P, _P, c_int64, c_int, c_int, c_int, c_int, c_int, _P, c_int, _P,

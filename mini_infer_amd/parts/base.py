@@ -194,6 +194,7 @@ class Norm(Part):
     """
 
     takes_partial_sums = False
+    takes_sums_in_updates = False  # an `ops.StreamUpdate` may hold them
     takes_pending_products = False
     emit_scaled_rows = False
     # the part that consumes this norm's output, set by the block together with

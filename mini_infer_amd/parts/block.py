@@ -150,6 +150,11 @@ class ParallelBlock(Block):
         self.joint = None
         self.beside = feed_forward  # what of the feed-forward is not made with the joint products
         self.emit_pending_output = self.emit_partial_sums = False
+        if not joint and norm.takes_sums_in_updates:
+            # (products left in pieces are added up by the launch that makes the update)
+            mixer.emit_partial_sums = True
+            if feed_forward is not None:
+                feed_forward.emit_partial_sums = True
         if joint:
             from mini_infer_amd.parts.joint import JointProducts
 
@@ -225,12 +230,13 @@ class ParallelBlock(Block):
             return self._forward_joint(h, ctx, cache, writes_cache)
         if hasattr(h, "finish"):
             h = h.finish()
-        mixed = self.mixer.forward(h, ctx, cache, writes_cache)
-        mixed = mixed.finish() if hasattr(mixed, "finish") else mixed
+        def made(part):
+            return part.finish() if hasattr(part, "finish") and not isinstance(part, ops.PartialSums) else part
+
+        mixed = made(self.mixer.forward(h, ctx, cache, writes_cache))
         fed = bias = None
         if self.feed_forward is not None:
-            fed = self.feed_forward.forward(h, ctx)
-            fed = fed.finish() if hasattr(fed, "finish") else fed
+            fed = made(self.feed_forward.forward(h, ctx))
             bias = getattr(self.feed_forward, "output_bias", None)
         return ops.StreamUpdate(mixed, fed, bias, None, self.scale)
 

@@ -277,7 +277,7 @@ class ClampedGatedFeedForward(FeedForward):
         assert self.gate_up.weight is not None
         # (few rows: the product, the biases, the clamps and the activation are one kernel)
         act = ops.linear_clamped_glu(x, self.gate_up.weight, self.gate_up_bias, self.limit, self.slope)
-        return self.down.forward(act)
+        return self.down.forward(act, partial_ok=self.emit_partial_sums)
 
 
 @register_feed_forward("clamped_glu")

@@ -218,13 +218,13 @@ class LatentAttention(Mixer):
         if gate is not None:  # (padding of the value heads leaves with it)
             packed = torch.empty((tokens, heads, vdim), dtype=mixed.dtype, device=mixed.device)
             ops.gate_heads(mixed.unflatten(1, (heads, v_width)), gate, packed)
-            return self.out.forward(packed.view(tokens, heads * vdim))
+            return self.out.forward(packed.view(tokens, heads * vdim), partial_ok=self.emit_partial_sums)
         if self._out_padded is None:  # W_o with zero columns under the padding of every value head
             assert self.out.weight is not None
             padded = torch.zeros((self.hidden_size, heads, width), dtype=self.out.weight.dtype, device=self.out.weight.device)
             padded[:, :, :vdim] = self.out.weight.view(self.hidden_size, heads, vdim)
             self._out_padded = padded.view(self.hidden_size, heads * width)
-        return ops.linear(mixed, self._out_padded)
+        return ops.linear(mixed, self._out_padded, partial_ok=self.emit_partial_sums)
 
     def forward(self, x, ctx: StepContext, cache: LayerCache, writes_cache: bool = True):
         assert cache.group is not None and cache.k_pages is not None
@@ -265,7 +265,7 @@ class LatentAttention(Mixer):
         values = torch.empty((tokens, heads * self.v_head_dim), dtype=proj.dtype, device=proj.device)
         ops.linear_per_head(mixed.unflatten(1, (heads, rank)), self.map_v, values.unflatten(1, (heads, self.v_head_dim)),
                             weight_kn=self.map_v_kn, gate=gate)
-        return self.out.forward(values)
+        return self.out.forward(values, partial_ok=self.emit_partial_sums)
 
 
 @register_mixer("latent_attention")

@@ -18,6 +18,7 @@ from mini_infer_amd.registry import register_norm
 class RMSNorm(Norm):
     graph_safe = True
     takes_partial_sums = True
+    takes_sums_in_updates = True
     takes_pending_products = True
 
     def __init__(self, hidden_size: int, eps: float, dtype: torch.dtype, device, name: str = "weight") -> None:

@@ -195,7 +195,7 @@ class GatedDeltaRule(Mixer):
             cache.state["recurrent"], ctx.cu_seqlens_q, ctx.state_slots, heads=self.num_heads, kv_heads=self.num_kv_heads,
             dim=self.head_dim, vdim=self.v_head_dim, eps=self.norm_eps, longest=_longest(ctx),
         )
-        return self.out.forward(mixed)
+        return self.out.forward(mixed, partial_ok=self.emit_partial_sums)
 
 
 @register_mixer("gated_delta_rule")

@@ -106,6 +106,27 @@ def test_the_stream_update_and_the_norm_behind_it(dtype, width, parts):
     np.testing.assert_allclose(np.broadcast_to(update.finish().cpu().numpy(), x.shape), new - x, rtol=0, atol=1e-5)
 
 
+@pytest.mark.parametrize("tokens,width", [(1, 2048), (30, 3072), (70, 1030), (3, 20000)])
+@pytest.mark.parametrize("kinds", [(3, 2), (1, None), (None, 16), (0, 5)])
+@pytest.mark.parametrize("picked", [False, True])
+def test_the_stream_update_of_products_left_in_pieces(tokens, width, kinds, picked):
+    """The bits of the same update with the pieces added up first; one side or both in 1 to 16 pieces, beside a tensor (0) and beside
+    nothing; columns kept and made again, single and in fours; all rows, and some with the stream left as it was."""
+    from mini_infer_amd import ops
+
+    g = torch.Generator().manual_seed(3)
+    rand = lambda *shape: torch.randn(shape, generator=g).to("cuda")  # noqa: E731
+    parts = [None if n is None else rand(tokens, width).bfloat16() if n == 0 else ops.PartialSums(rand(n, tokens, width), torch.bfloat16) for n in kinds]
+    stream, weight = rand(tokens, width), rand(width).bfloat16()
+    rows = torch.tensor([tokens - 1, 0], dtype=torch.int32, device="cuda") if picked else None
+    results = []
+    for a, b in (parts, [p.finish() if isinstance(p, ops.PartialSums) else p for p in parts]):
+        own = stream.clone()
+        update = ops.StreamUpdate(a, b, None, None, 0.5)
+        results.append((ops.stream_update_norm(update, own, weight, 1e-6, rows), own, update.finish()))
+    assert all(torch.equal(x, y) for x, y in zip(*results))
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("inter, limit", [(5, 0.7), (64, 1.5), (300, 3.0)])
 def test_the_clamped_gated_activation(dtype, inter, limit):
