@@ -97,7 +97,7 @@ __device__ __forceinline__ void add_up(const Sums& sums, int64_t place, float va
 
 // The new values of VEC columns of a row: x + scale * (a + b + bias) + shift, with b = sum_p
 // b_weights[p] * row p of `pieces` rows that lie b_stride apart (b_weights null: one row, as it is).
-template <typename T, int VEC>
+template <typename T, int VEC, bool SUMS>
 __device__ __forceinline__ void updated(const T* ar, const T* br, int64_t b_stride, const float* b_weights, int pieces,
                                         const float* bias, const float* shift, float scale, const float* x, int c,
                                         const Sums& a_sums, const Sums& b_sums, int64_t row_at, float value[VEC]) {
@@ -106,7 +106,7 @@ __device__ __forceinline__ void updated(const T* ar, const T* br, int64_t b_stri
 #pragma unroll
   for (int e = 0; e < VEC; ++e) av[e] = bv[e] = cv[e] = sv[e] = 0.f;
   if (ar) load_some<VEC>(ar + c, av);
-  if (a_sums.at) add_up<T, VEC>(a_sums, row_at + c, av);
+  if (SUMS && a_sums.at) add_up<T, VEC>(a_sums, row_at + c, av);
   double bw[VEC];  // (float32 elements: the weighted sum in 64-bit)
   if (b_weights) {
 #pragma unroll
@@ -123,7 +123,7 @@ __device__ __forceinline__ void updated(const T* ar, const T* br, int64_t b_stri
     }
   } else {
     if (br) load_some<VEC>(br + c, bv);
-    if (b_sums.at) add_up<T, VEC>(b_sums, row_at + c, bv);
+    if (SUMS && b_sums.at) add_up<T, VEC>(b_sums, row_at + c, bv);
     if constexpr (sizeof(T) == 4) {
 #pragma unroll
       for (int e = 0; e < VEC; ++e) bw[e] = (double)bv[e];
@@ -140,7 +140,8 @@ __device__ __forceinline__ void updated(const T* ar, const T* br, int64_t b_stri
 
 // One block a row.  `rows` (optional) lists the rows to norm; with it the stream is left as
 // it was (the rows' new values are used for the norm only), as the final norm wants it.
-template <typename T, int VEC>
+// SUMS: a product in pieces may be among the summands (with its registers seven waves a SIMD instead of eight: not for prompts).
+template <typename T, int VEC, bool SUMS>
 __global__ __launch_bounds__(1024) void stream_update_norm_kernel(
     const T* __restrict__ a, int64_t a_stride, const T* __restrict__ b, int64_t b_stride,
     const float* __restrict__ b_weights, int pieces, const float* __restrict__ bias, const float* __restrict__ shift, float scale, float* __restrict__ stream,
@@ -162,7 +163,7 @@ __global__ __launch_bounds__(1024) void stream_update_norm_kernel(
   int n = 0;
   for (int c = threadIdx.x * VEC; c < hidden; c += blockDim.x * VEC, ++n) {
     float value[VEC];
-    updated<T, VEC>(ar, br, b_stride, bwr, pieces, bias, shift, scale, x, c, a_sums, b_sums, (int64_t)t * hidden, value);
+    updated<T, VEC, SUMS>(ar, br, b_stride, bwr, pieces, bias, shift, scale, x, c, a_sums, b_sums, (int64_t)t * hidden, value);
 #pragma unroll
     for (int e = 0; e < VEC; ++e) {
       if constexpr (WIDE) squares_wide += (double)value[e] * (double)value[e];
@@ -193,7 +194,7 @@ __global__ __launch_bounds__(1024) void stream_update_norm_kernel(
     } else if (!rows) {
       load_some<VEC>(x + c, value);
     } else {  // made again: the stream was not written
-      updated<T, VEC>(ar, br, b_stride, bwr, pieces, bias, shift, scale, x, c, a_sums, b_sums, (int64_t)t * hidden, value);
+      updated<T, VEC, SUMS>(ar, br, b_stride, bwr, pieces, bias, shift, scale, x, c, a_sums, b_sums, (int64_t)t * hidden, value);
     }
     load_some<VEC>(weight + c, w);
 #pragma unroll
@@ -268,12 +269,13 @@ extern "C" int mi_stream_update_norm(int dtype, const void* a, int64_t a_stride,
   const bool vec = hidden % 4 == 0 && ((uintptr_t)a | (uintptr_t)b | (uintptr_t)weight | (uintptr_t)out | (uintptr_t)(a_stride * elem) |
                                        (uintptr_t)(b_stride * elem)) % 16 == 0 &&
                    ((uintptr_t)bias | (uintptr_t)shift | (uintptr_t)stream | (uintptr_t)a_sums | (uintptr_t)b_sums) % 16 == 0;
-#define MI_UPDATE_LAUNCH(T, VEC)                                                                                      \
-  stream_update_norm_kernel<T, VEC><<<num_out_rows, threads, 0, stream_handle>>>(                                     \
+#define MI_UPDATE_LAUNCH(T, VEC, SUMS)                                                                                \
+  stream_update_norm_kernel<T, VEC, SUMS><<<num_out_rows, threads, 0, stream_handle>>>(                               \
       (const T*)a, a_stride, (const T*)b, b_stride, b_weights, pieces, bias, shift, scale, stream, (const T*)weight, (T*)out, rows, hidden, eps, \
       Sums{a_sums, a_count, (int64_t)num_tokens * hidden}, Sums{b_sums, b_count, (int64_t)num_tokens * hidden})
-  if (dtype == MI_F32) { if (vec) MI_UPDATE_LAUNCH(float, 4); else MI_UPDATE_LAUNCH(float, 1); }
-  else { if (vec) MI_UPDATE_LAUNCH(bf16_t, 4); else MI_UPDATE_LAUNCH(bf16_t, 1); }
+  if (dtype == MI_F32) { if (vec) MI_UPDATE_LAUNCH(float, 4, false); else MI_UPDATE_LAUNCH(float, 1, false); }
+  else if (a_sums || b_sums) { if (vec) MI_UPDATE_LAUNCH(bf16_t, 4, true); else MI_UPDATE_LAUNCH(bf16_t, 1, true); }
+  else { if (vec) MI_UPDATE_LAUNCH(bf16_t, 4, false); else MI_UPDATE_LAUNCH(bf16_t, 1, false); }
 #undef MI_UPDATE_LAUNCH
   MI_CHECK_LAUNCH("stream_update_norm");
   return MI_OK;
