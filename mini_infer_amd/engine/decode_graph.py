@@ -184,8 +184,9 @@ class DecodeGraph:
         # No garbage collection while the stream records: a collector run frees whatever cyclic
         # garbage earlier work left (pinned buffers, events, other graphs), their destructors make
         # runtime calls that a recording stream forbids, and an error inside a destructor aborts.
+        # (Kept off, it has nothing to run; it need not run before.  That run was 27 ms of a process with torch and
+        # a model in it, most of a step's first pass.)
         collecting = gc.isenabled()
-        gc.collect()
         gc.disable()
         try:
             with torch.cuda.graph(graph):
