@@ -53,6 +53,10 @@ class DecoderModel:
         head = spec.head_description()
         self.head = HEADS.lookup(head["kind"])(head, dtype, device, shared)
         self.stream_vectors: dict[str, torch.Tensor] = {}  # float32 [rows, hidden], by checkpoint name
+        layer_parts = [part for block in self.blocks for part in block.parts()]
+        if any(getattr(part, "routes", False) for part in layer_parts):
+            for part in layer_parts:
+                part.steady = True
         # a product whose output only ever meets norms that can add up its pieces may leave them apart
         if self.final_norm.takes_partial_sums and all(block.takes_partial_sums for block in self.blocks):
             for block in self.blocks:

@@ -614,14 +614,15 @@ def gated_tiles_for(m: int, n: int, k: int) -> int | None:
     return shape
 
 
-def linear(x: torch.Tensor, weight: torch.Tensor, partial_ok: bool = False) -> torch.Tensor | PartialSums:
+def linear(x: torch.Tensor, weight: torch.Tensor, partial_ok: bool = False, steady: bool = False) -> torch.Tensor | PartialSums:
     """`x @ weight.T` without bias.
 
     float32 runs the hand-written true-float32 kernel.  bfloat16 with at most 16 rows (decode) runs the hand-written
     weight-streaming kernel, some tens to some hundreds of rows the tiles of `gemm_tiles_bf16` where they are faster
     (`tiles_for`); the rest goes to the vendor GEMM library through torch, as the reference's engine does
     (distributed/linear.py:167, `F.linear` -> the vendor BLAS).
-    With `partial_ok` the result may come as `PartialSums` where that pays.
+    With `partial_ok` the result may come as `PartialSums` where that pays.  `steady` (`Part.steady`): without those tiles, so that the
+    sums keep the order that they have in the library.
     """
     if x.dtype == torch.float32:
         return gemm_f32(x, weight)
@@ -636,7 +637,7 @@ def linear(x: torch.Tensor, weight: torch.Tensor, partial_ok: bool = False) -> t
         and skinny_gemm_takes(x.shape[0], x.shape[1], x.stride(0), weight.stride(0))
     ):
         return gemm_skinny_bf16(x, weight)
-    if x.dim() == 2 and x.shape[0] <= TILES_MAX_ROWS and _rows_of_bf16(x, weight):
+    if not steady and x.dim() == 2 and x.shape[0] <= TILES_MAX_ROWS and _rows_of_bf16(x, weight):
         m, n = x.shape[0], weight.shape[0]
         plan = tiles_for(m, n, x.shape[1], partial_ok)
         if plan is not None:
@@ -765,7 +766,7 @@ def qkv_rope_write(
     return q_out
 
 
-def linear_swiglu(x: "torch.Tensor | ScaledRows", gate_up_weight: torch.Tensor) -> torch.Tensor:
+def linear_swiglu(x: "torch.Tensor | ScaledRows", gate_up_weight: torch.Tensor, steady: bool = False) -> torch.Tensor:
     """`silu(x @ gate.T) * (x @ up.T)` with `gate_up_weight` = [gate; up] stacked, [2I, K].
 
     bfloat16 with at most 32 rows, and up to some hundreds where that is faster (`gated_tiles_for`), runs as ONE
@@ -795,7 +796,7 @@ def linear_swiglu(x: "torch.Tensor | ScaledRows", gate_up_weight: torch.Tensor) 
             scaled, x = x, values
         else:
             x = x.finish()
-    if scaled is None and x.dim() == 2 and SKINNY_WIDE_MAX_ROWS < x.shape[0] <= TILES_MAX_ROWS and _rows_of_bf16(x, gate_up_weight):
+    if not steady and scaled is None and x.dim() == 2 and SKINNY_WIDE_MAX_ROWS < x.shape[0] <= TILES_MAX_ROWS and _rows_of_bf16(x, gate_up_weight):
         _need_cuda(x, gate_up_weight)
         m, n = x.shape[0], rows // 2
         shape = gated_tiles_for(m, n, width)
@@ -840,7 +841,7 @@ def linear_swiglu(x: "torch.Tensor | ScaledRows", gate_up_weight: torch.Tensor) 
             out = torch.empty((m, n), dtype=torch.float32, device=x.device)
             library.check(lib.mi_gemm_f32_swiglu(*matrices, _ptr(out), n, m, n, width, _stream()))
             return out
-    return silu_mul(linear(x, gate_up_weight))
+    return silu_mul(linear(x, gate_up_weight, steady=steady))
 
 
 # Launch shapes of the matrix-core attention kernel: 128-row prefill blocks, two to a CU; decode
@@ -1072,6 +1073,7 @@ def paged_attention(
     gate: torch.Tensor | None = None,
     out: torch.Tensor | None = None,
     host_seq_lens: list[int] | None = None,
+    steady: bool = False,
 ) -> torch.Tensor | AttentionPieces:
     """Causal attention of every token over its request's pages; returns [T, q_heads*head_dim].
 
@@ -1109,7 +1111,8 @@ def paged_attention(
     of tokens and requests alone, with as many tiles as any division of the tokens among the
     requests can need, and requests without tokens are allowed.  `host_seq_lens` (optional): how many
     positions each request holds with this step's tokens; where a step brings portions beside single tokens, each
-    of the two is cut by its own keys.
+    of the two is cut by its own keys.  `steady` (`Part.steady`): portions and single tokens as launches of their own, their keys cut
+    alike, which keeps the order of the sums.
     bfloat16 caches with transposed values run on the matrix cores; everything else
     (float32, other head or page sizes) runs the plain kernel.
     """
@@ -1225,7 +1228,7 @@ def paged_attention(
         num_tiles = tokens // tokens_per_tile + num_requests
         head_blocks = -(-group // min(group, 128))
         splits = min(16, attention_splits(num_tiles * kv_heads * head_blocks, seen(tokens_per_tile), target=512, min_keys=128))
-        if num_requests > 1 and lib.mi_attn_mixed_supported(head_dim, v_dim, page_size):
+        if not steady and num_requests > 1 and lib.mi_attn_mixed_supported(head_dim, v_dim, page_size):
             mixed(-1, num_tiles, splits, splits)
             return out
         part_acc, part_ml = partials(splits)
@@ -1300,7 +1303,7 @@ def paged_attention(
         if 0 < leading_single < num_requests:
             most = host_seq_lens or [max_seq_len] * num_requests
             lens = q_lens[leading_single:]
-            if not lib.mi_attn_mixed_supported(head_dim, v_dim, page_size) or wide_prefill(lens):
+            if steady or not lib.mi_attn_mixed_supported(head_dim, v_dim, page_size) or wide_prefill(lens):
                 run(0, leading_single)
                 run(leading_single, num_requests)
                 return out
@@ -1767,7 +1770,8 @@ def linear_gru(
     return out
 
 
-def linear_gelu_table(x: torch.Tensor, weight: torch.Tensor, table: torch.Tensor, ids: torch.Tensor, first_col: int) -> torch.Tensor:
+def linear_gelu_table(x: torch.Tensor, weight: torch.Tensor, table: torch.Tensor, ids: torch.Tensor, first_col: int,
+                      steady: bool = False) -> torch.Tensor:
     """`gelu_tanh(x @ weight.T) * table[ids, first_col : first_col + N]`.  Few bfloat16 rows: one
     weight-streaming kernel with the activation and the gather in its last step; otherwise the
     product followed by `gated_table_rows`.  Both round the product to the element type first."""
@@ -1800,7 +1804,7 @@ def linear_gelu_table(x: torch.Tensor, weight: torch.Tensor, table: torch.Tensor
             )
         )
         return out
-    return gated_table_rows(linear(x, weight), table, ids, first_col)
+    return gated_table_rows(linear(x, weight, steady=steady), table, ids, first_col)
 
 
 # ----------------------------------------------------------------------------
@@ -1926,7 +1930,8 @@ def clamped_glu(
     return out
 
 
-def linear_clamped_glu(x: torch.Tensor, gate_up_weight: torch.Tensor, bias: torch.Tensor | None, limit: float, slope: float) -> torch.Tensor:
+def linear_clamped_glu(x: torch.Tensor, gate_up_weight: torch.Tensor, bias: torch.Tensor | None, limit: float, slope: float,
+                       steady: bool = False) -> torch.Tensor:
     """`clamped_glu(x @ [gate; up].T, bias, limit, slope)`.  bfloat16 with at most 32 rows runs as ONE
     kernel (the weight-streaming product with biases, clamps and activation in its last step);
     otherwise the product and `clamped_glu` run in turn.  Both round the two products to the element
@@ -1955,7 +1960,7 @@ def linear_clamped_glu(x: torch.Tensor, gate_up_weight: torch.Tensor, bias: torc
             )
         )
         return out
-    return clamped_glu(linear(x, gate_up_weight), bias, limit, slope)
+    return clamped_glu(linear(x, gate_up_weight, steady=steady), bias, limit, slope)
 
 
 @dataclasses.dataclass(frozen=True)
@@ -2076,7 +2081,7 @@ def layer_in(
     return q_out, gates
 
 
-def linear_geglu(x: torch.Tensor, gate_up_weight: torch.Tensor) -> torch.Tensor:
+def linear_geglu(x: torch.Tensor, gate_up_weight: torch.Tensor, steady: bool = False) -> torch.Tensor:
     """`gelu_tanh(x @ gate.T) * (x @ up.T)` with `gate_up_weight` = [gate; up] stacked, [2I, K].  bfloat16
     with at most 32 rows runs as ONE kernel (the weight-streaming product with the activation in its
     last step); otherwise the product and `gated_mul` run in turn.  Both round the two products to the
@@ -2102,7 +2107,7 @@ def linear_geglu(x: torch.Tensor, gate_up_weight: torch.Tensor) -> torch.Tensor:
             )
         )
         return out
-    both = linear(x, gate_up_weight)
+    both = linear(x, gate_up_weight, steady=steady)
     return gated_mul(both[:, : rows // 2], both[:, rows // 2 :], "gelu_tanh")
 
 
@@ -3315,10 +3320,10 @@ def experts_grouped(
             if count:
                 mine = sorted_rows[at:at + count]
                 if activation == "silu_gated":
-                    inner = linear_swiglu(mine, gate_up[e])
+                    inner = linear_swiglu(mine, gate_up[e], steady=True)
                 else:
-                    inner = weighted_squared_relu(linear(mine, gate_up[e]), sorted_weights[at:at + count].contiguous())
-                made.append(linear(inner, down[e]))
+                    inner = weighted_squared_relu(linear(mine, gate_up[e], steady=True), sorted_weights[at:at + count].contiguous())
+                made.append(linear(inner, down[e], steady=True))
                 at += count
         rows = torch.cat(made, dim=0) if made else torch.empty((1, width), dtype=x.dtype, device=x.device)
     out = torch.empty((tokens, width), dtype=x.dtype, device=x.device)

@@ -291,13 +291,13 @@ class GQAttention(Mixer):
             # A projection left in pieces is added up by the rotation's launch, in steps of single tokens: 8B sizes, 40 of them,
             # 4,650 -> 4,500 us a step.  A portion's values are written a page at a time, sixteen tokens a thread, and all their
             # pieces there cost more than a launch (60 tokens beside 9 single ones, 8B 5,420 -> 5,950; 100 beside 10, 1B 1,567 -> 1,851).
-            in_pieces = (ctx.max_q_len == 1 and rotary is not None and self._same_widths and self._plain_heads
+            in_pieces = (not self.steady and ctx.max_q_len == 1 and rotary is not None and self._same_widths and self._plain_heads
                          and ops.rope_takes_partial_sums(self.head_dim, rotary.rotary_dim, rotary.interleaved))
             qkv = self.qkv.forward(x, partial_ok=in_pieces)
             kv_heads, slots = self.num_kv_heads, ctx.slot_mapping[cache.group]
         else:
             # reads another call's keys and values: only q is projected
-            qkv = ops.linear(x, self.qkv.weight[:q_width])
+            qkv = ops.linear(x, self.qkv.weight[:q_width], steady=self.steady)
             kv_heads, slots = 0, None
         if rotary is not None:
             cos, sin, rotary_dim, interleaved = rotary.cos, rotary.sin, rotary.rotary_dim, rotary.interleaved
@@ -359,7 +359,7 @@ class GQAttention(Mixer):
             kv_heads=self.num_kv_heads, head_dim=self.head_dim, scale=self.scale, window=self.window,
             max_seq_len=ctx.max_seq_len, v_transposed=cache.v_transposed, combine=not few, slopes=self.slopes,
             v_head_dim=self.v_head_dim, sink_logit=self.sink_logit, chunk=self.chunk, gate=gate, out=out,
-            host_seq_lens=ctx.host_seq_lens,
+            host_seq_lens=ctx.host_seq_lens, steady=self.steady,
         )
 
 
@@ -417,7 +417,7 @@ class KeysAsValuesAttention(GQAttention):
             qk = self.qkv.forward(x)
             kv_heads, slots = self.num_kv_heads, ctx.slot_mapping[cache.group]
         else:
-            qk = ops.linear(x, self.qkv.weight[:q_width])
+            qk = ops.linear(x, self.qkv.weight[:q_width], steady=self.steady)
             kv_heads, slots = 0, None
         ops.qk_norm_kv_write(
             qk, self.q_norm, self.k_norm if writes_cache else None, slots, cache.k_pages, cache.v_pages,
@@ -526,7 +526,7 @@ class WholeNormAttention(GQAttention):
         else:
             if self.mix_key is not None:
                 raise NotImplementedError("a layer that shares values and reads another call's cache; not built")
-            qkv = ops.linear(x, self.qkv.weight[:q_width])
+            qkv = ops.linear(x, self.qkv.weight[:q_width], steady=self.steady)
             kv_heads, slots = 0, None
         ops.qkv_norm_write(
             qkv, self.q_norm, self.k_norm if writes_cache else None, slots, cache.k_pages, cache.v_pages,
@@ -538,7 +538,7 @@ class WholeNormAttention(GQAttention):
             ctx.positions, ctx.cu_seqlens_q, ctx.host_cu_seqlens_q, q_heads=self.num_heads,
             kv_heads=self.num_kv_heads, head_dim=self.head_dim, scale=self.scale, window=self.window,
             max_seq_len=ctx.max_seq_len, v_transposed=cache.v_transposed, slopes=self.slopes,
-            v_head_dim=self.v_head_dim, sinks=self.sinks, softcap=self.softcap, host_seq_lens=ctx.host_seq_lens,
+            v_head_dim=self.v_head_dim, sinks=self.sinks, softcap=self.softcap, host_seq_lens=ctx.host_seq_lens, steady=self.steady,
         )
         return self.out.forward(attended)
 

@@ -217,9 +217,9 @@ class ParallelBlock(Block):
             if (self.emit_pending_output and self.dtype == torch.bfloat16
                     and ops.pending_product_pays(inner.shape[0], *weight.shape, self.emit_partial_sums)):
                 return ops.PendingProduct(inner, weight)
-            return ops.linear(inner, weight, partial_ok=self.emit_partial_sums)
+            return ops.linear(inner, weight, partial_ok=self.emit_partial_sums, steady=self.steady)
         h = h.finish() if hasattr(h, "finish") else h
-        added = ops.linear(self.joint.inner_rows(h, ctx, cache, writes_cache), weight)
+        added = ops.linear(self.joint.inner_rows(h, ctx, cache, writes_cache), weight, steady=self.steady)
         return ops.StreamUpdate(added, None if self.beside is None else self.beside.forward(h, ctx), None, None, self.scale)
 
     def forward(self, delta, residual: torch.Tensor, ctx: StepContext, cache: LayerCache, writes_cache: bool = True):

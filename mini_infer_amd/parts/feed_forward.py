@@ -69,11 +69,11 @@ class SwiGLU(FeedForward):
         assert self.gate_up.weight is not None, "SwiGLU used before its weights were loaded"
         assert self.down.weight is not None
         if self.activation == "silu":
-            act = ops.linear_swiglu(x, self.gate_up.weight)
+            act = ops.linear_swiglu(x, self.gate_up.weight, steady=self.steady)
         else:
             if isinstance(x, ops.ScaledRows):
                 x = x.finish()
-            act = ops.linear_geglu(x, self.gate_up.weight)
+            act = ops.linear_geglu(x, self.gate_up.weight, steady=self.steady)
         if (
             self.emit_pending_output
             and self.dtype == torch.bfloat16
@@ -187,7 +187,7 @@ class TokenSideInput(FeedForward):
             x = x.finish()
         assert self.gate.weight is not None
         # (few rows: the gate product, its activation and the gather are one kernel)
-        gated = ops.linear_gelu_table(x, self.gate.weight, self.table.tensor, ctx.token_ids, self.first_col)
+        gated = ops.linear_gelu_table(x, self.gate.weight, self.table.tensor, ctx.token_ids, self.first_col, steady=self.steady)
         return self.proj.forward(gated)
 
 
@@ -276,7 +276,7 @@ class ClampedGatedFeedForward(FeedForward):
             x = x.finish()
         assert self.gate_up.weight is not None
         # (few rows: the product, the biases, the clamps and the activation are one kernel)
-        act = ops.linear_clamped_glu(x, self.gate_up.weight, self.gate_up_bias, self.limit, self.slope)
+        act = ops.linear_clamped_glu(x, self.gate_up.weight, self.gate_up_bias, self.limit, self.slope, steady=self.steady)
         return self.down.forward(act, partial_ok=self.emit_partial_sums)
 
 
@@ -314,6 +314,7 @@ class RoutedExperts(FeedForward):
     engine's own products once over all its rows.  Router, correction and the shared expert's gate row stay float32."""
 
     graph_safe = True
+    routes = True
 
     # rows * top pairs, times the bytes of an expert, from which on sorting by expert pays for the
     # launches of a loop over the experts (each pair reads its expert's weights once otherwise)

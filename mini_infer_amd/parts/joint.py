@@ -107,10 +107,11 @@ class JointProducts:
             self.mixer.forward_layer_in(h, self.input_weight, self.layout, ctx, cache, writes_cache, activated, mixed)
         else:
             h = h.finish() if isinstance(h, ops.ScaledRows) else h
+            steady = self.mixer.steady
             if self.partner is not None and self.dtype == torch.bfloat16 and rows.shape[0] * self.input_weight.shape[0] >= APART_IN_OUTPUTS:
-                own, gated = ops.linear(h, self.mixer.joint_input.weight), ops.linear(h, self.partner.gate_up.weight)
+                own, gated = ops.linear(h, self.mixer.joint_input.weight, steady=steady), ops.linear(h, self.partner.gate_up.weight, steady=steady)
             else:
-                columns = ops.linear(h, self.input_weight)
+                columns = ops.linear(h, self.input_weight, steady=steady)
                 own, gated = columns[:, : self.mixer_columns], columns[:, self.mixer_columns: self.mixer_columns + 2 * self.ff]
             self.mixer.forward_projected(own, ctx, cache, writes_cache, mixed)
             if self.partner is not None:
@@ -125,5 +126,5 @@ class JointProducts:
     def outputs(self, joined: torch.Tensor) -> tuple[torch.Tensor, torch.Tensor]:
         """The two parts of the last product of `inner_rows`."""
         assert self.partner is not None
-        return (ops.linear(joined[:, : self.inner], self.mixer.joint_output.weight),
-                ops.linear(joined[:, self.inner:], self.partner.down.weight))
+        return (ops.linear(joined[:, : self.inner], self.mixer.joint_output.weight, steady=self.mixer.steady),
+                ops.linear(joined[:, self.inner:], self.partner.down.weight, steady=self.mixer.steady))

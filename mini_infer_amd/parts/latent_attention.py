@@ -213,7 +213,7 @@ class LatentAttention(Mixer):
         mixed = ops.paged_attention(
             queries, k_own, v_own, table, ctx.token_request, ctx.positions, ctx.cu_seqlens_q, ctx.host_cu_seqlens_q, q_heads=heads,
             kv_heads=heads, head_dim=width, scale=self.scale, window=self.window, max_seq_len=ctx.max_q_len, v_transposed=True,
-            sinks=self.sinks, v_head_dim=v_width,
+            sinks=self.sinks, v_head_dim=v_width, steady=self.steady,
         )
         if gate is not None:  # (padding of the value heads leaves with it)
             packed = torch.empty((tokens, heads, vdim), dtype=mixed.dtype, device=mixed.device)
@@ -224,7 +224,7 @@ class LatentAttention(Mixer):
             padded = torch.zeros((self.hidden_size, heads, width), dtype=self.out.weight.dtype, device=self.out.weight.device)
             padded[:, :, :vdim] = self.out.weight.view(self.hidden_size, heads, vdim)
             self._out_padded = padded.view(self.hidden_size, heads * width)
-        return ops.linear(mixed, self._out_padded, partial_ok=self.emit_partial_sums)
+        return ops.linear(mixed, self._out_padded, partial_ok=self.emit_partial_sums, steady=self.steady)
 
     def forward(self, x, ctx: StepContext, cache: LayerCache, writes_cache: bool = True):
         assert cache.group is not None and cache.k_pages is not None

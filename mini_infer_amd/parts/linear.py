@@ -57,4 +57,4 @@ class Linear(Part):
     def forward(self, x: torch.Tensor, partial_ok: bool = False):
         """`x @ weight.T`; with `partial_ok` possibly as `ops.PartialSums` for a norm to add up."""
         assert self.weight is not None, "Linear used before its weight was loaded"
-        return ops.linear(x, self.weight, partial_ok=partial_ok)
+        return ops.linear(x, self.weight, partial_ok=partial_ok, steady=self.steady)

@@ -679,3 +679,34 @@ def test_the_replay_program_runs_a_trace_of_this_design(folders, tmp_path):
             assert_close(got[at: at + n], want, "float32", f"trace step {number} {rid}")
             fed[rid] += n
             at += n
+
+
+def test_steps_in_front_of_a_router_keep_the_order_of_their_sums(monkeypatch):
+    """A prompt, and a portion beside single tokens, of sizes that other designs make in tiles and attend to in one launch: here
+    neither runs (a rounding that falls the other way chooses another expert), and a product is the library's, bit for bit."""
+    from mini_infer_amd import ModelRunner, StepEntry, ops
+    from mini_infer_amd.models import architecture_for
+    from mini_infer_amd.ops import library
+
+    mlp = {"kind": "moe", "expert": {"ff": 256}, "shared": {"ff": 4096}, "router": {"experts": 8, "identity": 1, "top": 2, "scale": 2.5}}
+    layers = [tk.latent(8, 64, 32, 64, 256, 512, 0.1, 10000.0, mlp=tk.dense(4096)), tk.attention(8, 4, 64, 64, 0.125, window=128, mlp=mlp)]
+    raw = {"architecture": "Kunudra", "vocab": 512, "width": 1024, "norm": {"eps": 1e-6}, "postln_alpha": 1.6, "embedding": {}, "layers": layers}
+    arch = architecture_for(raw)
+    parsed = arch.parse_config(raw)
+    model = arch.make_model(parsed, torch.bfloat16, DEV)
+    specs, generator = model.param_specs(), torch.Generator().manual_seed(3)
+    model.load_params(lambda name: (0.02 * torch.randn(specs[name].shape, generator=generator)).to(DEV, TORCH.get(specs[name].dtype, torch.bfloat16)))
+    runner = ModelRunner(model, parsed, num_blocks=64, block_size=16, max_concurrent=4)
+    lib, taken = library.load(), []
+    for name in ("mi_gemm_tiles_bf16", "mi_attn_mixed"):
+        monkeypatch.setattr(lib, name, lambda *a, name=name, launch=getattr(lib, name): (taken.append(name), launch(*a))[1])
+    tokens = torch.randint(0, 512, (200,), generator=generator).tolist()
+    for i in (0, 1):
+        runner.step([StepEntry(i, tokens[:100 + i], [])])
+    runner.step([StepEntry(0, tokens[100:101], [0]), StepEntry(1, tokens[101:102], [0]), StepEntry(2, tokens[:60], [59])])
+    assert taken == []
+    x, w = dev(np.random.default_rng(1).normal(size=(100, 1024)), torch.bfloat16), dev(np.random.default_rng(2).normal(size=(8192, 1024)), torch.bfloat16)
+    assert torch.equal(ops.linear(x, w, steady=True), x @ w.t()) and torch.equal(ops.linear_swiglu(x, w, steady=True), ops.silu_mul(x @ w.t()))
+    assert taken == []
+    ops.linear(x, w)
+    assert taken == ["mi_gemm_tiles_bf16"]

@@ -74,3 +74,24 @@ def test_float32_models_are_wired_the_same_and_decide_at_run_time():
     # the flags say what a part MAY do; float32 parts then make every product themselves
     model = DecoderModel(_spec(tiny.TINY_A), torch.float32, "cpu")
     assert all(block.feed_forward.emit_pending_output for block in model.blocks)
+
+
+def test_every_part_of_a_design_with_routed_experts_keeps_the_order_of_its_sums():
+    """Wherever a rounding can reach a router; designs without one take the faster forms."""
+    import tiny_bemulorn
+    import tiny_figosun
+    import tiny_kunudra
+    import tiny_zekonex
+
+    seen = set()
+    for configs in (tiny_kunudra, tiny_figosun, tiny_bemulorn, tiny_zekonex):
+        for cfg in configs.CONFIGS.values():
+            cfg = cfg[0] if isinstance(cfg, tuple) else cfg
+            model = DecoderModel(_spec(cfg), torch.bfloat16, "cpu")
+            parts = [part for block in model.blocks for part in block.parts()]
+            assert len(parts) > 4 * len(model.blocks)
+            routed = any(layer["mlp"] is not None and layer["mlp"]["kind"] == "moe" for layer in cfg["layers"])
+            assert {part.steady for part in parts} == {routed}
+            seen.add(routed)
+    assert seen == {True, False}
+    assert not any(part.steady for block in DecoderModel(_spec(), torch.bfloat16, "cpu").blocks for part in block.parts())
