@@ -625,12 +625,12 @@ __global__ __launch_bounds__(256) void rope_kv_write_vec4_kernel(
   }
 }
 
-// bias: float32 [q heads | k heads | v heads], added to the projection's columns before anything else, or null
 // Whether mi_rope_kv_write adds up a projection left in pieces (bfloat16, tensors on 16 bytes, value heads in whole 4s).
 extern "C" int mi_rope_takes_pieces(int head_dim, int rotary_dim, int interleaved) {
   return !interleaved && head_dim > 0 && head_dim % 4 == 0 && rotary_dim % 8 == 0 ? 1 : 0;
 }
 
+// bias: float32 [q heads | k heads | v heads], added to the projection's columns before anything else, or null
 // pieces (may be null): [num_pieces][num_tokens][width] float32, the projection's sums over ranges of K; qkv then takes the rotated
 // queries only.
 extern "C" int mi_rope_kv_write(int dtype, void* qkv, int64_t row_stride, const float* cos_t,

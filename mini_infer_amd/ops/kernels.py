@@ -310,7 +310,8 @@ def rope_kv_write(
         _need_contiguous("pieces", pieces)
         if width < (q_heads + kv_heads) * head_dim + kv_heads * (head_dim if v_head_dim is None else int(v_head_dim)):
             raise KernelShapeError(f"qkv rows hold {width} values, fewer than the q, k and v heads need")
-        qkv = torch.empty((pieces.shape[1], q_heads * head_dim), dtype=qkv.dtype, device=pieces.device)
+        # (rows on 16 bytes, whatever the heads' number and size)
+        qkv = torch.empty((pieces.shape[1], -(-q_heads * head_dim // 8) * 8), dtype=qkv.dtype, device=pieces.device)[:, : q_heads * head_dim]
     _need_cuda(qkv, cos, sin, slot_mapping, k_pages, v_pages)
     _need_contiguous("cos", cos)
     _need_contiguous("sin", sin)

@@ -501,6 +501,26 @@ def test_rope_kv_write_of_a_projection_in_pieces(q_heads, kv_heads, head_dim, ro
     assert all(torch.equal(a, b) for a, b in zip(*results)) and bool(results[0][1].any()) == (writes and tokens > 1)
 
 
+@pytest.mark.parametrize("q_heads,kv_heads,head_dim,rotary_dim", [(5, 1, 20, 16), (3, 1, 100, 40), (7, 7, 12, 8)])
+def test_rope_kv_write_in_pieces_of_rows_that_are_not_whole_16_bytes(q_heads, kv_heads, head_dim, rotary_dim):
+    """Queries whose heads together are an odd number of 8 bytes: taken like any others that `rope_takes_partial_sums` answers for."""
+    from mini_infer_amd import ops
+
+    tokens, page, width = 20, 16, (q_heads + 2 * kv_heads) * head_dim
+    assert q_heads * head_dim % 8 == 4 and ops.rope_takes_partial_sums(head_dim, rotary_dim, False)
+    sums = ops.PartialSums(_rand(3, tokens, width, seed=1), torch.bfloat16)
+    cos, sin = _rand(tokens, rotary_dim // 2, seed=2), _rand(tokens, rotary_dim // 2, seed=3)
+    slots = torch.arange(tokens, dtype=torch.int32, device=DEV)
+    results = []
+    for qkv in (sums, sums.finish()):
+        k_pages = torch.zeros((2, kv_heads, page, head_dim), dtype=torch.bfloat16, device=DEV)
+        v_pages = torch.zeros((2, kv_heads, head_dim, page), dtype=torch.bfloat16, device=DEV)
+        queries = ops.rope_kv_write(qkv, cos, sin, slots, k_pages, v_pages, q_heads=q_heads, kv_heads=kv_heads, head_dim=head_dim,
+                                    rotary_dim=rotary_dim, v_transposed=True)
+        results.append((queries[:, : q_heads * head_dim], k_pages, v_pages))
+    assert all(torch.equal(a, b) for a, b in zip(*results)) and results[0][1].any()
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("page_size", [16, 8])
 @pytest.mark.parametrize("more_pages", [0, 40])  # 40 more whole pages: the rows of a prompt's portion
