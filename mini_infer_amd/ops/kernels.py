@@ -1301,7 +1301,7 @@ def paged_attention(
         leading_single = 0
         while leading_single < num_requests and q_lens[leading_single] == 1:
             leading_single += 1
-        if 0 < leading_single < num_requests:
+        if leading_single and host_cu_seqlens_q[leading_single] < tokens:  # (requests without tokens behind them go along)
             most = host_seq_lens or [max_seq_len] * num_requests
             lens = q_lens[leading_single:]
             if steady or not lib.mi_attn_mixed_supported(head_dim, v_dim, page_size) or wide_prefill(lens):

@@ -835,6 +835,16 @@ def test_paged_attention_of_portions_beside_single_tokens_in_one_launch(monkeypa
     assert (got.float() - attend(**options).float()).abs().max() < _tol(torch.bfloat16, 2) and len(taken) == 2
 
 
+@pytest.mark.parametrize("lengths,q_lens", [([30, 20], [1, 0]), ([300, 20, 900, 1], [1, 1, 0, 0]), ([30, 20, 9], [1, 0, 1]), ([600, 70, 300], [1, 0, 70])])
+def test_paged_attention_of_single_tokens_before_requests_without_tokens(lengths, q_lens):
+    """Boundaries known to the host, some requests of the step without tokens behind those with one."""
+    case = _paged_case(torch.bfloat16, 4, 2, 64, 16, lengths, q_lens, seed=19, v_transposed=True)
+    out = _attend(case, 4, 2, 64, 0.125, None, max(lengths))
+    with_tokens = [i for i, n in enumerate(q_lens) if n]
+    expected = _attention_expected({key: [case[key][i] for i in with_tokens] for key in ("qs", "ks", "vs")}, 0.125, None)
+    assert np.abs(out.double().cpu().numpy() - expected).max() < _tol(torch.bfloat16, 2)
+
+
 @pytest.mark.parametrize("window", [None, 700])
 def test_paged_attention_whole_long_prompts_many_tiles(window):
     """Whole prompts of a few thousand tokens beside a short one: dozens of tiles per head,
