@@ -281,6 +281,27 @@ def test_linear_of_some_tens_to_some_hundreds_of_rows(m, n, k):
     assert torch.equal(kernels.sum_pieces(_rand(3, 5, 7, seed=46)), _rand(3, 5, 7, seed=46).sum(0).bfloat16())
 
 
+@pytest.mark.parametrize("count,rows,columns,first", [(1, 1, 1, 0), (2, 17, 3072, 0), (16, 70, 1030, 0), (5, 3, 7, 0), (3, 5, 7, 1), (4, 6, 8, 2)])
+def test_partial_sums_finish_in_one_launch(monkeypatch, count, rows, columns, first):
+    """The sum in order, rounded once, by one launch of this library; pieces off 16 bytes and columns of wider pieces by torch, the same."""
+    from mini_infer_amd import ops
+    from mini_infer_amd.ops import library
+
+    lib, launches = library.load(), []
+    launch = lib.mi_sum_pieces
+    monkeypatch.setattr(lib, "mi_sum_pieces", lambda *a: (launches.append(a), launch(*a))[1])
+    pieces = _rand(first + count, rows, columns, seed=5)[first:]
+    expected = pieces[0].clone()
+    for piece in pieces[1:]:
+        expected += piece
+    finished = ops.PartialSums(pieces, torch.bfloat16).finish()
+    assert finished.dtype == torch.bfloat16 and torch.equal(finished, expected.bfloat16())
+    assert len(launches) == (first * rows * columns % 4 == 0)
+    wide = torch.cat([pieces, pieces], dim=2)[:, :, :columns]
+    assert torch.equal(ops.PartialSums(wide, torch.bfloat16).finish(), expected.bfloat16())
+    assert ops.PartialSums(pieces, torch.float32).finish().equal(expected)
+
+
 def test_linear_leaves_partial_sums_only_where_asked_and_where_it_pays():
     from mini_infer_amd import ops
     from mini_infer_amd.exceptions import KernelShapeError
