@@ -70,6 +70,8 @@ class DecoderModel:
         for layer, after in followers.items():
             if all(part.takes_pending_products for part in after):
                 self.blocks[layer].enable_pending_output()
+            if all(part.takes_sums_in_updates for part in after):
+                self.blocks[layer].enable_sums_in_updates()
 
     @property
     def vocab_size(self) -> int:

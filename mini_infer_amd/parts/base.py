@@ -430,6 +430,13 @@ class Block(Part):
     def enable_pending_output(self) -> None:
         pass
 
+    # Whether the block's `delta` may be an `ops.StreamUpdate` that holds `ops.PartialSums`; where all that follows a block says
+    # so, the model calls its `enable_sums_in_updates()`.
+    takes_sums_in_updates = False
+
+    def enable_sums_in_updates(self) -> None:
+        pass
+
     def cache_needs(self, page_size: int) -> CacheNeeds:
         """What the cache manager must keep for one call of this block: its mixer's needs, and what the
         block itself remembers of a request from step to step."""

@@ -78,6 +78,10 @@ class PreNormBlock(Block):
         if self.feed_forward.can_defer_output:
             self.feed_forward.emit_pending_output = True
 
+    @property
+    def takes_sums_in_updates(self) -> bool:  # type: ignore[override]
+        return self.mixer_norm.takes_sums_in_updates
+
     def _children(self):
         return (
             (self.names["mixer_norm"], self.mixer_norm),
@@ -150,11 +154,6 @@ class ParallelBlock(Block):
         self.joint = None
         self.beside = feed_forward  # what of the feed-forward is not made with the joint products
         self.emit_pending_output = self.emit_partial_sums = False
-        if not joint and norm.takes_sums_in_updates:
-            # (products left in pieces are added up by the launch that makes the update)
-            mixer.emit_partial_sums = True
-            if feed_forward is not None:
-                feed_forward.emit_partial_sums = True
         if joint:
             from mini_infer_amd.parts.joint import JointProducts
 
@@ -193,6 +192,17 @@ class ParallelBlock(Block):
 
     def enable_partial_sums(self) -> None:
         self.emit_partial_sums = self.joint is not None
+
+    @property
+    def takes_sums_in_updates(self) -> bool:  # type: ignore[override]
+        return self.norm.takes_sums_in_updates
+
+    def enable_sums_in_updates(self) -> None:
+        if self.joint is None and not self.steady:
+            # (products left in pieces are added up by the launch that makes the update)
+            self.mixer.emit_partial_sums = True
+            if self.feed_forward is not None:
+                self.feed_forward.emit_partial_sums = True
 
     def param_specs(self, prefix: str) -> dict[str, ParamSpec]:
         specs: dict[str, ParamSpec] = {}

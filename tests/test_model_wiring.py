@@ -95,3 +95,29 @@ def test_every_part_of_a_design_with_routed_experts_keeps_the_order_of_its_sums(
             seen.add(routed)
     assert seen == {True, False}
     assert not any(part.steady for block in DecoderModel(_spec(), torch.bfloat16, "cpu").blocks for part in block.parts())
+
+
+def test_a_parallel_layer_leaves_pieces_only_for_followers_that_add_them_up():
+    """What comes next in every place of the order decides, not the layer's own norm."""
+    import tiny_zekonex
+
+    cfg = tiny_zekonex.TINY_A
+    spec = _spec(cfg)
+    assert len(spec.layers) >= 3 and all(layer.block["kind"] == "parallel" for layer in spec.layers)
+
+    def leaving(spec):
+        model = DecoderModel(spec, torch.bfloat16, "cpu")
+        emits = [{part.emit_partial_sums for part in (block.mixer, block.feed_forward) if part is not None} for block in model.blocks]
+        assert all(len(each) == 1 for each in emits)
+        return [each.pop() for each in emits]
+
+    count = len(spec.layers)
+    assert leaving(spec) == [True] * count
+    plain = dict(spec.layers[1].block, norm={"kind": "test_wiring_plain_norm"})
+    changed = dataclasses.replace(spec, layers=[spec.layers[0], dataclasses.replace(spec.layers[1], block=plain), *spec.layers[2:]])
+    assert leaving(changed) == [False] + [True] * (count - 1)
+    ends = dataclasses.replace(spec, final_norm={"kind": "test_wiring_plain_norm"})
+    assert leaving(ends) == [True] * (count - 1) + [False]
+    # the first layer stands before the plain norm in one of its two places
+    again = dataclasses.replace(changed, order=[LayerCall(0), LayerCall(2 % count), LayerCall(0), LayerCall(1)])
+    assert leaving(again)[0] is False
