@@ -37,13 +37,13 @@ const Shape SHAPES[] = {GEMM_TILE_SHAPES(X)};
 #undef X
 constexpr int SHAPE_COUNT = sizeof(SHAPES) / sizeof(SHAPES[0]);
 constexpr int MOST_RANGES = 16;
-constexpr int CUS = 256;
 
 // Microseconds that a launch is expected to take (rows: of W, gate and up together).
-double gemm_tiles_micros(const Shape& s, int m, int rows, int k, int steps_each) {
+double gemm_tiles_micros(const Shape& s, int m, int rows, int k, int steps_each, int cus) {
   const int steps = ceil_div(k, 64), ranges = ceil_div(steps, steps_each);
   const int64_t blocks = (int64_t)ceil_div(m, s.rows) * ceil_div(rows, s.features) * ranges;
-  const int64_t a_cu = ceil_div64(ceil_div64(blocks, 8), CUS / 8);
+  const int xcds = max(1, cus / 32);  // (blocks are dealt to them in turn)
+  const int64_t a_cu = ceil_div64(ceil_div64(blocks, xcds), max(1, cus / xcds));
   const int together = s.ring_bytes * 2 <= 163840 ? 2 : 1;
   const double brought = (double)a_cu * steps_each * (s.rows + s.features) * 128;
   const double products = (double)a_cu * steps_each * s.rows * s.features * 128;
@@ -57,17 +57,17 @@ double gemm_tiles_micros(const Shape& s, int m, int rows, int k, int steps_each)
 // The best way to make a product: *shape and *ranges of K (1: whole), for a caller to whom sums over r > 1 ranges cost sum_base +
 // sum_each * r microseconds more than the whole product.  most_ranges: 1 whole products only.  same_order: ranges by n and k alone, and
 // every shape that is chosen sums a range in the same order, so that a row's sums do not depend on the other rows.
-// *micros: the expected microseconds, that extra included.
-extern "C" int mi_gemm_tiles_plan(int m, int n, int k, int gated, int most_ranges, int same_order, float sum_base, float sum_each, int* shape,
+// cus: the device's compute units.  *micros: the expected microseconds, that extra included.
+extern "C" int mi_gemm_tiles_plan(int m, int n, int k, int gated, int most_ranges, int same_order, float sum_base, float sum_each, int cus, int* shape,
                                   int* ranges, float* micros) {
-  MI_REQUIRE(m >= 1 && n >= 1 && k >= 1, "gemm_tiles_plan: m=%d n=%d k=%d", m, n, k);
+  MI_REQUIRE(m >= 1 && n >= 1 && k >= 1 && cus >= 1, "gemm_tiles_plan: m=%d n=%d k=%d on %d compute units", m, n, k, cus);
   const int rows = gated ? 2 * n : n;
   const int steps = ceil_div(k, 64);
   double best = INFINITY;
   *shape = 0, *ranges = 1;
   int from = 1, to = max(1, min(min(most_ranges, MOST_RANGES), steps / 4));
   if (same_order) {  // a block a CU with tiles of 64 features
-    to = max(1, min(min(MOST_RANGES, steps / 4), CUS / ceil_div(n, 64)));
+    to = max(1, min(min(MOST_RANGES, steps / 4), cus / ceil_div(n, 64)));
     from = to;
   }
   for (int i = 0; i < SHAPE_COUNT; ++i) {
@@ -75,7 +75,7 @@ extern "C" int mi_gemm_tiles_plan(int m, int n, int k, int gated, int most_range
     for (int r = from; r <= to; ++r) {
       const int each = ceil_div(steps, r), got = ceil_div(steps, each);
       if (got != r && !same_order) continue;
-      const double t = gemm_tiles_micros(SHAPES[i], m, rows, k, each) + (got > 1 ? sum_base + sum_each * got : 0.0);
+      const double t = gemm_tiles_micros(SHAPES[i], m, rows, k, each, cus) + (got > 1 ? sum_base + sum_each * got : 0.0);
       if (t < best) best = t, *shape = i, *ranges = got;
     }
   }

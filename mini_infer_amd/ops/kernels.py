@@ -460,7 +460,7 @@ def linear_f32_out(x: torch.Tensor, weight: torch.Tensor, scale: float = 1.0, sc
         return out
     if x.dim() == 2 and SKINNY_MAX_ROWS < x.shape[0] <= HEAD_TILES_MAX_ROWS and weight.shape[0] >= 16000 and _rows_of_bf16(x, weight):
         m, n = x.shape[0], weight.shape[0]
-        _, shape, _ = _tiles_plan(m, n, x.shape[1], False, 1, False, 0.0, 0.0)
+        _, shape, _ = _tiles_plan(m, n, x.shape[1], False, 1, False, 0.0, 0.0, _compute_units(x.device))
         return _tiles(2, x, weight, torch.empty((m, n), dtype=torch.float32, device=x.device), n, shape, 1, float(scale))
     product = torch.matmul(x, weight.t())
     if scale == 1.0:
@@ -509,12 +509,22 @@ def partial_sums_pay(m: int, n: int, k: int) -> bool:
     return m > SKINNY_MAX_ROWS and n <= 4096 and 2048 <= k <= 4096
 
 
+WHOLE_DEVICE_CUS = 256
+
+
+@functools.lru_cache(maxsize=None)
+def _compute_units(device: torch.device) -> int:
+    return torch.cuda.get_device_properties(device).multi_processor_count
+
+
 @functools.lru_cache(maxsize=8192)
-def _tiles_plan(m: int, n: int, k: int, gated: bool, most_ranges: int, same_order: bool, sum_base: float, sum_each: float) -> tuple[float, int, int]:
-    """(microseconds expected, tile shape, ranges of K) of the best way to make a product in tiles (csrc/gemm_tiles_bf16.hip)."""
+def _tiles_plan(m: int, n: int, k: int, gated: bool, most_ranges: int, same_order: bool, sum_base: float, sum_each: float,
+                cus: int = WHOLE_DEVICE_CUS) -> tuple[float, int, int]:
+    """(microseconds expected, tile shape, ranges of K) of the best way to make a product in tiles (csrc/gemm_tiles_bf16.hip) on a
+    device of `cus` compute units."""
     shape, ranges, micros = ctypes.c_int(), ctypes.c_int(), ctypes.c_float()
     library.check(
-        library.load().mi_gemm_tiles_plan(m, n, k, int(gated), most_ranges, int(same_order), sum_base, sum_each,
+        library.load().mi_gemm_tiles_plan(m, n, k, int(gated), most_ranges, int(same_order), sum_base, sum_each, cus,
                                           ctypes.addressof(shape), ctypes.addressof(ranges), ctypes.addressof(micros))
     )
     return micros.value, shape.value, ranges.value
@@ -551,7 +561,7 @@ def linear_partial_sums(x: torch.Tensor, weight: torch.Tensor) -> PartialSums:
             f"linear_partial_sums takes 1 to 128 rows, K a multiple of 32, rows aligned to 16 bytes; "
             f"got x {tuple(x.shape)} strides {x.stride()}, weight {tuple(weight.shape)} strides {weight.stride()}"
         )
-    _, shape, ranges = _tiles_plan(m, n, k, False, 16, True, 0.0, 0.0)
+    _, shape, ranges = _tiles_plan(m, n, k, False, 16, True, 0.0, 0.0, _compute_units(x.device))
     pieces = torch.empty((ranges, m, n), dtype=torch.float32, device=x.device)
     return PartialSums(_tiles(1, x, weight, pieces, n, shape, ranges), torch.bfloat16)
 
@@ -573,7 +583,7 @@ TILES_MAX_ROWS = 1024
 
 
 @functools.lru_cache(maxsize=8192)
-def tiles_for(m: int, n: int, k: int, partial_ok: bool) -> tuple[int, int] | None:
+def tiles_for(m: int, n: int, k: int, partial_ok: bool, cus: int = WHOLE_DEVICE_CUS) -> tuple[int, int] | None:
     """(tile shape, ranges of K) where a bfloat16 product of more rows than `gemm_skinny_bf16` takes is made in tiles; None: by the
     vendor library.  Over 61 matrices (n 1024 to 28672, k 1536 to 14336) the tiles took, as a geometric mean of the library's time,
     where the sum over ranges is left to the consumer / made here, its launch included:
@@ -594,15 +604,15 @@ def tiles_for(m: int, n: int, k: int, partial_ok: bool) -> tuple[int, int] | Non
     if n >= 16000 and m > 80 or not partial_ok and n * k < 8_000_000:
         return None
     each = m * n * 4 / SUM_BYTES_A_MICRO
-    whole, _, _ = _tiles_plan(m, n, k, False, 1, False, 0.0, 0.0)
-    micros, shape, ranges = _tiles_plan(m, n, k, False, 16, False, 0.0 if partial_ok else SUM_LAUNCH_MICROS, each)
+    whole, _, _ = _tiles_plan(m, n, k, False, 1, False, 0.0, 0.0, cus)
+    micros, shape, ranges = _tiles_plan(m, n, k, False, 16, False, 0.0 if partial_ok else SUM_LAUNCH_MICROS, each, cus)
     if m > 320 and micros > 0.88 * whole:
         return None
     return shape, ranges
 
 
 @functools.lru_cache(maxsize=8192)
-def gated_tiles_for(m: int, n: int, k: int) -> int | None:
+def gated_tiles_for(m: int, n: int, k: int, cus: int = WHOLE_DEVICE_CUS) -> int | None:
     """The tile shape where the gated product of n features is made in tiles, or None.  Up to 32 rows the streaming product
     (`gemm_skinny_swiglu_bf16`) gives a row the same bits as it gets in a step of its own; tiles are not faster everywhere there (gate|up
     at 24 rows: 16384 x 3072 19.8 against 23.9 us, 28672 x 4096 50.8 against 47.1).  Above, measured against the vendor product
@@ -611,7 +621,7 @@ def gated_tiles_for(m: int, n: int, k: int) -> int | None:
     33.9); where there is work for larger ones the library is faster by as much as 1.3."""
     if not SKINNY_WIDE_MAX_ROWS < m <= 768:
         return None
-    _, shape, _ = _tiles_plan(m, n, k, True, 1, False, 0.0, 0.0)
+    _, shape, _ = _tiles_plan(m, n, k, True, 1, False, 0.0, 0.0, cus)
     if m > 200 and library.load().mi_gemm_tiles_area(shape) > 192 * 128:
         return None
     return shape
@@ -642,7 +652,7 @@ def linear(x: torch.Tensor, weight: torch.Tensor, partial_ok: bool = False, stea
         return gemm_skinny_bf16(x, weight)
     if not steady and x.dim() == 2 and x.shape[0] <= TILES_MAX_ROWS and _rows_of_bf16(x, weight):
         m, n = x.shape[0], weight.shape[0]
-        plan = tiles_for(m, n, x.shape[1], partial_ok)
+        plan = tiles_for(m, n, x.shape[1], partial_ok, _compute_units(x.device))
         if plan is not None:
             if plan[1] == 1:
                 return _tiles(0, x, weight, torch.empty((m, n), dtype=torch.bfloat16, device=x.device), n, *plan)
@@ -802,7 +812,7 @@ def linear_swiglu(x: "torch.Tensor | ScaledRows", gate_up_weight: torch.Tensor, 
     if not steady and scaled is None and x.dim() == 2 and SKINNY_WIDE_MAX_ROWS < x.shape[0] <= TILES_MAX_ROWS and _rows_of_bf16(x, gate_up_weight):
         _need_cuda(x, gate_up_weight)
         m, n = x.shape[0], rows // 2
-        shape = gated_tiles_for(m, n, width)
+        shape = gated_tiles_for(m, n, width, _compute_units(x.device))
         if shape is not None:
             return _tiles(3, x, gate_up_weight, torch.empty((m, n), dtype=torch.bfloat16, device=x.device), n, shape, 1)
     if (

@@ -14,7 +14,7 @@ from pathlib import Path
 from mini_infer_amd.exceptions import ExtensionMissingError, KernelShapeError
 from mini_infer_amd.ops import build as _build
 
-ABI_VERSION = 44
+ABI_VERSION = 45
 
 _lib: ctypes.CDLL | None = None
 _lib_path: Path | None = None
@@ -37,7 +37,7 @@ _SIGNATURES: dict[str, list] = {
     "mi_gemm_f32_swiglu": [_P, c_int64, _P, c_int64, _P, c_int64, c_int, c_int, c_int, _P],
     "mi_gemm_skinny_bf16": [_P, c_int64, _P, c_int64, _P, c_int64, c_int, c_int, c_int, _P],
     "mi_gemm_skinny_f32out_bf16": [_P, c_int64, _P, c_int64, _P, c_int64, c_int, c_int, c_int, c_float, _P],
-    "mi_gemm_tiles_plan": [c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_float, _P, _P, _P],
+    "mi_gemm_tiles_plan": [c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_float, c_int, _P, _P, _P],
     "mi_gemm_tiles_area": [c_int],
     "mi_gemm_tiles_take": [c_int, c_int, c_int, c_int64, c_int64],
     "mi_gemm_tiles_bf16": [c_int, _P, c_int64, _P, c_int64, _P, c_int64, c_float, c_int, c_int, c_int, c_int, c_int, _P],
