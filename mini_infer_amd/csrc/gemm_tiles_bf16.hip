@@ -57,6 +57,10 @@ double gemm_tiles_micros(const Shape& s, int m, int rows, int k, int steps_each,
 // The best way to make a product: *shape and *ranges of K (1: whole), for a caller to whom sums over r > 1 ranges cost sum_base +
 // sum_each * r microseconds more than the whole product.  most_ranges: 1 whole products only.  same_order: ranges by n and k alone, and
 // every shape that is chosen sums a range in the same order, so that a row's sums do not depend on the other rows.
+// Where rows of W are a multiple of 16 KB long, up to 128 rows are not cut into ranges of K that begin 4 KB apart: all blocks then ask the
+// same memory channels at once, which the expected time does not know.  With the sum's launch, 8192 x 8192 at 17 / 64 rows in 4
+// ranges 35.3 / 36.7 us, in 2 29.8 / 32.2 (the vendor library 31.0 / 33.0), 4096 x 16384 at 24 / 64 rows in 8 ranges 47.3 / 50.7, in 4, which
+// begin 8 KB apart, 31.6 / 33.4 (the library 32.8 / 42.1).  More rows read little of W for what they multiply: 4096 x 8192 at 200 rows in 4 ranges 31.2, otherwise 36.6.
 // cus: the device's compute units.  *micros: the expected microseconds, that extra included.
 extern "C" int mi_gemm_tiles_plan(int m, int n, int k, int gated, int most_ranges, int same_order, float sum_base, float sum_each, int cus, int* shape,
                                   int* ranges, float* micros) {
@@ -75,6 +79,7 @@ extern "C" int mi_gemm_tiles_plan(int m, int n, int k, int gated, int most_range
     for (int r = from; r <= to; ++r) {
       const int each = ceil_div(steps, r), got = ceil_div(steps, each);
       if (got != r && !same_order) continue;
+      if (got > 1 && !same_order && m <= 128 && k % 8192 == 0 && each % 64 == 32) continue;  // (see above: the same memory channels)
       const double t = gemm_tiles_micros(SHAPES[i], m, rows, k, each, cus) + (got > 1 ? sum_base + sum_each * got : 0.0);
       if (t < best) best = t, *shape = i, *ranges = got;
     }

@@ -20,3 +20,18 @@ def test_a_plan_counts_the_compute_units_of_its_device(cus):
     part = kernels._tiles_plan(64, 4096, 4096, False, 16, False, 0.0, 0.0, cus)
     assert part[0] >= whole[0] and part[2] <= whole[2] and (cus == 256) == (part == whole)
     assert kernels._tiles_plan(64, 4096, 4096, False, 16, False, 0.0, 0.0) == whole
+
+
+@pytest.mark.parametrize("m", [17, 24, 32, 48, 64, 100, 128, 129, 200])
+@pytest.mark.parametrize("n", [2048, 4096, 8192, 10240])
+@pytest.mark.parametrize("k", [4096, 8192, 14336, 16384])
+@pytest.mark.parametrize("partial_ok", [False, True])
+def test_few_rows_are_not_cut_into_ranges_that_begin_4_kb_apart_in_rows_of_16(m, n, k, partial_ok):
+    """All blocks would ask the same memory channels; more rows, and rows of W of other lengths, are cut as before."""
+    _, _, ranges = kernels._tiles_plan(m, n, k, False, 16, False, 0.0 if partial_ok else 4.0, m * n * 4 / 5e6)
+    apart = -(-(k // 64) // ranges) * 128  # bytes
+    assert ranges == 1 or m > 128 or k % 8192 or apart % 8192 != 4096
+    if (m, n, k) == (17, 8192, 8192):
+        assert ranges == 2
+    if (m, n, k) == (200, 4096, 8192):
+        assert ranges == 4
