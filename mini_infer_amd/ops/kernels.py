@@ -595,9 +595,11 @@ def tiles_for(m: int, n: int, k: int, partial_ok: bool, cus: int = WHOLE_DEVICE_
                        1.17  1.16  1.16  1.19  1.29  1.18  1.08  1.06  1.05  1.04  1.02
 
     The library does not cut K and so leaves CUs idle where there are few features; from some 300 rows on it is about as fast as whole
-    tiles, and cutting has to pay.  (Up to 320 rows tiles without that: they are as fast or faster, 3072 x 3072 at 271 rows 15.3 against
-    19.7 us, 5120 x 3072 20.8 / 20.7, at worst 10240 x 3072 31.3 / 28.8; and a call of the library costs the host 20 us, one of these 8, of
-    which a step of that many tokens at 3B widths waits for the host.)  It is faster (tiles 0.75 to 0.95) for the widest matrices, and where the whole product takes
+    tiles, and cutting has to pay.  (Up to 288 rows tiles without that: 3072 x 3072 at 272 rows 15.8 against 17.5 us, 6144 x 4096 29.6 / 29.3,
+    5120 x 3072 21.8 / 20.7, at worst 9216 x 3072 32.2 / 28.7; and a call of the library costs the host 20 us, one of these 8, of which a
+    step of that many tokens at 3B widths waits for the host.  Up to 320 rows those that are cut, 2048 x 8192 at 300 rows 25.5 / 33.0, and
+    whole ones of matrices up to 4096 x 4096, 24.4 / 26.2; larger ones are slower from three tiles of 96 rows on, 5120 x 3072 25.6 / 22.3,
+    6144 x 4096 31.6 / 30.0, 5120 x 5120 40.9 / 37.5.)  It is faster (tiles 0.75 to 0.95) for the widest matrices, and where the whole product takes
     it less than 9 microseconds and the sum needs a launch of its own."""
     if not SKINNY_MAX_ROWS < m <= TILES_MAX_ROWS:
         return None
@@ -606,7 +608,7 @@ def tiles_for(m: int, n: int, k: int, partial_ok: bool, cus: int = WHOLE_DEVICE_
     each = m * n * 4 / SUM_BYTES_A_MICRO
     whole, _, _ = _tiles_plan(m, n, k, False, 1, False, 0.0, 0.0, cus)
     micros, shape, ranges = _tiles_plan(m, n, k, False, 16, False, 0.0 if partial_ok else SUM_LAUNCH_MICROS, each, cus)
-    if m > 320 and micros > 0.88 * whole:
+    if m > 320 and micros > 0.88 * whole or m > 288 and ranges == 1 and max(n, k) > 4096:
         return None
     return shape, ranges
 

@@ -35,3 +35,13 @@ def test_few_rows_are_not_cut_into_ranges_that_begin_4_kb_apart_in_rows_of_16(m,
         assert ranges == 2
     if (m, n, k) == (200, 4096, 8192):
         assert ranges == 4
+
+
+@pytest.mark.parametrize("n,k", [(5120, 3072), (6144, 4096), (6144, 3072), (5120, 5120), (3072, 8192)])
+def test_whole_tiles_of_large_matrices_end_at_288_rows(n, k):
+    """Where the library was measured faster; cut ones and small matrices go on to 320."""
+    assert kernels.tiles_for(288, n, k, False) is not None
+    for m in (289, 300, 320):
+        plan = kernels.tiles_for(m, n, k, False)
+        assert plan is None or plan[1] > 1
+    assert kernels.tiles_for(320, 3072, 3072, False) is not None and kernels.tiles_for(320, 2048, 8192, True)[1] > 1
