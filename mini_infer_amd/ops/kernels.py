@@ -618,13 +618,14 @@ def gated_tiles_for(m: int, n: int, k: int, cus: int = WHOLE_DEVICE_CUS) -> int 
     """The tile shape where the gated product of n features is made in tiles, or None.  Up to 32 rows the streaming product
     (`gemm_skinny_swiglu_bf16`) gives a row the same bits as it gets in a step of its own; tiles are not faster everywhere there (gate|up
     at 24 rows: 16384 x 3072 19.8 against 23.9 us, 28672 x 4096 50.8 against 47.1).  Above, measured against the vendor product
-    and `silu_mul`, tiles are 1.0 to 1.9 times as fast up to 200 rows, and beyond as long as tiles of up to 192 x 128 are what pays
+    and `silu_mul`, tiles are 1.0 to 1.9 times as fast up to 160 rows, and beyond as long as tiles of up to 192 x 128 are what pays
     (7168 x 4096 at 256 / 600 rows 32.5 / 48.2 against 43.8 / 53.8, 16384 x 2048 at 271 / 320 29.4 / 30.8 against 33.3 /
-    33.9); where there is work for larger ones the library is faster by as much as 1.3."""
+    33.9); where there is work for larger ones the library is faster by as much as 1.3 (28672 x 4096 at 193 rows 86.9 / 72.3, 57344 x
+    8192 at 161 / 192 rows 235 / 215 and 236 / 203; at 160 rows 181 / 196)."""
     if not SKINNY_WIDE_MAX_ROWS < m <= 768:
         return None
     _, shape, _ = _tiles_plan(m, n, k, True, 1, False, 0.0, 0.0, cus)
-    if m > 200 and library.load().mi_gemm_tiles_area(shape) > 192 * 128:
+    if m > 160 and library.load().mi_gemm_tiles_area(shape) > 192 * 128:
         return None
     return shape
 

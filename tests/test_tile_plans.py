@@ -45,3 +45,15 @@ def test_whole_tiles_of_large_matrices_end_at_288_rows(n, k):
         plan = kernels.tiles_for(m, n, k, False)
         assert plan is None or plan[1] > 1
     assert kernels.tiles_for(320, 3072, 3072, False) is not None and kernels.tiles_for(320, 2048, 8192, True)[1] > 1
+
+
+def test_gated_products_of_more_than_160_rows_take_no_tiles_above_192_by_128():
+    """Larger ones were measured slower than the library from there on."""
+    from mini_infer_amd.ops import library
+
+    for n, k in ((14336, 4096), (28672, 8192), (8192, 3072), (8192, 2048), (2048, 3072)):
+        assert kernels.gated_tiles_for(160, n, k) is not None
+        for m in (161, 176, 192, 193, 200, 256):
+            shape = kernels.gated_tiles_for(m, n, k)
+            assert shape is None or library.load().mi_gemm_tiles_area(shape) <= 192 * 128
+    assert kernels.gated_tiles_for(193, 14336, 4096) is None and kernels.gated_tiles_for(192, 14336, 4096) is not None
