@@ -88,8 +88,9 @@ extern "C" int mi_gemm_tiles_plan(int m, int n, int k, int gated, int most_range
   return MI_OK;
 }
 
-// Rows times features of a shape.
-extern "C" int mi_gemm_tiles_area(int shape) { return shape >= 0 && shape < SHAPE_COUNT ? SHAPES[shape].rows * SHAPES[shape].features : 0; }
+// Rows and features of a shape (0: there is none of that number).
+extern "C" int mi_gemm_tiles_rows(int shape) { return shape >= 0 && shape < SHAPE_COUNT ? SHAPES[shape].rows : 0; }
+extern "C" int mi_gemm_tiles_features(int shape) { return shape >= 0 && shape < SHAPE_COUNT ? SHAPES[shape].features : 0; }
 
 extern "C" int mi_gemm_tiles_take(int m, int n, int k, int64_t lda, int64_t ldw) {
   return m >= 1 && n >= 1 && k >= 32 && k % 32 == 0 && lda >= k && ldw >= k && lda % 8 == 0 && ldw % 8 == 0 &&

@@ -613,6 +613,12 @@ def tiles_for(m: int, n: int, k: int, partial_ok: bool, cus: int = WHOLE_DEVICE_
     return shape, ranges
 
 
+def tile_size(shape: int) -> tuple[int, int]:
+    """Rows and features of a tile shape; (0, 0): there is none of that number."""
+    lib = library.load()
+    return lib.mi_gemm_tiles_rows(shape), lib.mi_gemm_tiles_features(shape)
+
+
 @functools.lru_cache(maxsize=8192)
 def gated_tiles_for(m: int, n: int, k: int, cus: int = WHOLE_DEVICE_CUS) -> int | None:
     """The tile shape where the gated product of n features is made in tiles, or None.  Up to 32 rows the streaming product
@@ -625,7 +631,7 @@ def gated_tiles_for(m: int, n: int, k: int, cus: int = WHOLE_DEVICE_CUS) -> int 
     if not SKINNY_WIDE_MAX_ROWS < m <= 768:
         return None
     _, shape, _ = _tiles_plan(m, n, k, True, 1, False, 0.0, 0.0, cus)
-    if m > 160 and library.load().mi_gemm_tiles_area(shape) > 192 * 128:
+    if m > 160 and tile_size(shape)[0] * tile_size(shape)[1] > 192 * 128:
         return None
     return shape
 

@@ -14,7 +14,7 @@ from pathlib import Path
 from mini_infer_amd.exceptions import ExtensionMissingError, KernelShapeError
 from mini_infer_amd.ops import build as _build
 
-ABI_VERSION = 45
+ABI_VERSION = 46
 
 _lib: ctypes.CDLL | None = None
 _lib_path: Path | None = None
@@ -38,7 +38,8 @@ _SIGNATURES: dict[str, list] = {
     "mi_gemm_skinny_bf16": [_P, c_int64, _P, c_int64, _P, c_int64, c_int, c_int, c_int, _P],
     "mi_gemm_skinny_f32out_bf16": [_P, c_int64, _P, c_int64, _P, c_int64, c_int, c_int, c_int, c_float, _P],
     "mi_gemm_tiles_plan": [c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_float, c_int, _P, _P, _P],
-    "mi_gemm_tiles_area": [c_int],
+    "mi_gemm_tiles_rows": [c_int],
+    "mi_gemm_tiles_features": [c_int],
     "mi_gemm_tiles_take": [c_int, c_int, c_int, c_int64, c_int64],
     "mi_gemm_tiles_bf16": [c_int, _P, c_int64, _P, c_int64, _P, c_int64, c_float, c_int, c_int, c_int, c_int, c_int, _P],
     "mi_sum_pieces": [_P, _P, c_int, c_int64, _P],

@@ -219,47 +219,65 @@ def test_linear_in_partial_sums_then_norm_is_linear_then_norm(m, n, k):
         assert torch.equal(out_a, out_b) and torch.equal(res_a, res_b)
 
 
-def _tile_shapes():
-    """(rows, features) of every tile shape, from the list that the kernels are compiled for."""
-    import re
-    from pathlib import Path
-
-    import mini_infer_amd
-
-    text = (Path(mini_infer_amd.__file__).parent / "csrc" / "gemm_tiles.h").read_text()
-    found = [[int(v) for v in m.split(",")] for m in re.findall(r"^  X\(([0-9, ]+)\)", text, re.M)]
-    return [(wm * mt * 16, wn * nt * 16) for wm, wn, _, mt, nt, _ in found]
+TILE_SHAPES = 14
 
 
-@pytest.mark.parametrize("shape", range(len(_tile_shapes())))
-def test_products_in_tiles(shape):
-    """Every shape at the edges of its tiles, whole, over ranges of K, as float32 times a number, and gated; K of one step, of fewer steps than
-    the ring has stages, of odd 32s, and of ranges of unequal length; rows of a wider buffer; a row of infinities stays alone."""
+def test_every_tile_shape_is_tested():
     from mini_infer_amd.ops import kernels
 
-    bm, bn = _tile_shapes()[shape]
+    sizes = [kernels.tile_size(shape) for shape in range(TILE_SHAPES + 1)]
+    assert len(set(sizes)) == TILE_SHAPES + 1 and sizes[-1] == (0, 0)
+
+
+@pytest.mark.parametrize("shape", range(TILE_SHAPES))
+def test_products_in_tiles(shape):
+    """Every shape at the edges of its tiles, whole, over ranges of K, as float32 times a number, and gated; K of one step, of fewer steps than
+    the ring has stages, of odd 32s, and of ranges of unequal length; rows of a wider buffer, whose values beside and behind the result
+    stay, on boundaries of four values and off them; a row of infinities stays alone."""
+    from mini_infer_amd.ops import kernels
+
+    bm, bn = kernels.tile_size(shape)
     cases = [(bm, bn, 64, 1), (bm + 1, bn + 1, 128, 2), (bm - 1, bn - 3, 320, 1), (2 * bm + 5, 2 * bn + 4, 64 * 11, 3), (1, 5, 32, 1),
              (17, bn + 62, 96, 1), (bm, 70, 64 * 7 + 32, 2), (3, 2 * bn, 1024, 16)]
+
+    def made(kind, a, w, n, dtype, ranges=1, scale=1.0, spare=0):
+        """The product in the first columns of rows with `spare` more (over ranges: [ranges, m, n], contiguous) before more values."""
+        m = a.shape[0]
+        if kind == 1:
+            flat = torch.full((ranges * m * n + 64,), 7.0, device=DEV)
+            out, rest = flat[:-64].view(ranges, m, n), [flat[-64:]]
+        else:
+            wide = torch.full((m + 1, n + spare), 7.0, dtype=dtype, device=DEV)
+            out, rest = wide[:m, :n], [wide[:, n:], wide[m:]]
+        kernels._tiles(kind, a, w, out, n, shape, ranges, scale)
+        assert all((each == 7).all() for each in rest), (kind, a.shape, n, ranges, spare)
+        return out
+
     for m, n, k, ranges in cases:
         a = _rand(m, k + 8, dtype=torch.bfloat16, seed=41)[:, :k]
         w = _rand(2 * n, k, dtype=torch.bfloat16, seed=42, scale=0.05)
         if m > 2:
             a[m - 1] = float("inf")
-        exact = a.double() @ w.double().T
         finite = slice(0, m - 1 if m > 2 else m)
-        bound = 2.0 ** -8 * float(exact[finite].abs().max()) + 1e-6  # (float32 sums of exact products, one rounding)
-        pieces = kernels._tiles(1, a, w, torch.full((ranges, m, 2 * n), 7.0, device=DEV), 2 * n, shape, ranges)
-        assert (pieces.double().sum(0) - exact)[finite].abs().max() < 2.0 ** -20 * k * float(exact[finite].abs().max()) + 1e-6
+        exact = (a.double() @ w.double().T)[finite]
+        # (exact products in float32 sums of k terms and the ranges', each rounded or cut; then one rounding to 8 bits)
+        summed = 2.0 ** -23 * (k + ranges) * (a.double().abs() @ w.double().abs().T)[finite] + 1e-30
+        rounded = summed + 2.0 ** -8 * exact.abs()
+        pieces = made(1, a, w, 2 * n, torch.float32, ranges)
+        assert ((pieces.double().sum(0)[finite] - exact).abs() <= summed).all(), (m, n, k)
         if ranges == 1:
-            out = kernels._tiles(0, a, w, torch.full((m, 2 * n + 3), 7.0, dtype=torch.bfloat16, device=DEV)[:, : 2 * n], 2 * n, shape, 1)
-            assert (out.double() - exact)[finite].abs().max() < bound, (m, n, k)
-            scaled = kernels._tiles(2, a, w, torch.empty(m, 2 * n, device=DEV), 2 * n, shape, 1, 0.25)
-            assert torch.equal(scaled[finite], out.float()[finite] * 0.25)
-            gated = kernels._tiles(3, a, w, torch.empty(m, n, dtype=torch.bfloat16, device=DEV), n, shape, 1)
-            g, u = out.double()[:, :n], out.double()[:, n:]
-            wanted = (g / (1.0 + torch.exp(-g)) * u)[finite]
-            # (a product may come out one rounding apart: the gated tile sums the same pieces in the same order, so it does not)
-            assert (gated.double()[finite] - wanted).abs().max() < 2.0 ** -8 * float(wanted.abs().max()) + 1e-6, (m, n, k)
+            outs = [made(0, a, w, 2 * n, torch.bfloat16, spare=spare) for spare in (0, 3, -2 * n % 4 + 4)]
+            out = outs[0]
+            assert all(torch.equal(other[finite], out[finite]) for other in outs)
+            assert ((out[finite].double() - exact).abs() <= rounded).all(), (m, n, k)
+            for spare in (0, 1, -2 * n % 4):
+                assert torch.equal(made(2, a, w, 2 * n, torch.float32, scale=0.25, spare=spare)[finite], out.float()[finite] * 0.25)
+            g, u = out.double()[finite, :n], out.double()[finite, n:]
+            wanted = g / (1.0 + torch.exp(-g)) * u
+            for spare in (0, 3, -n % 4 + 4):
+                # (a product may come out one rounding apart: the gated tile sums the same pieces in the same order, so it does not)
+                gated = made(3, a, w, n, torch.bfloat16, spare=spare)[finite]
+                assert ((gated.double() - wanted).abs() <= 2.0 ** -8 * wanted.abs() + 1e-30).all(), (m, n, k)
 
 
 @pytest.mark.parametrize("m,n,k", [(17, 3072, 3072), (33, 2048, 8192), (271, 3072, 8192), (100, 8192, 2048), (24, 1000, 8224), (400, 2048, 8192)])
