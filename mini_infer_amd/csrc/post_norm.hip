@@ -42,7 +42,22 @@ __device__ __forceinline__ A block_add(A v, A* scratch) {
   __syncthreads();
   if (lane == 0) scratch[wave] = v;
   __syncthreads();
-  A parts[16];  // (a block's 16 waves at most: read at once, added in order)
+  A total = 0;
+  for (int w = 0; w < n_waves; ++w) total += scratch[w];
+  return total;
+}
+
+// The same, the waves' sums (16 at most) read at once and added in order.
+template <typename A>
+__device__ __forceinline__ A block_add_at_once(A v, A* scratch) {
+#pragma unroll
+  for (int off = MI_WAVE / 2; off > 0; off >>= 1) v = lane_add(v, off);
+  const int wave = threadIdx.x / MI_WAVE, lane = threadIdx.x % MI_WAVE;
+  const int n_waves = (blockDim.x + MI_WAVE - 1) / MI_WAVE;
+  __syncthreads();
+  if (lane == 0) scratch[wave] = v;
+  __syncthreads();
+  A parts[16];
 #pragma unroll
   for (int w = 0; w < 16; ++w) parts[w] = scratch[min(w, n_waves - 1)];
   A total = 0;
@@ -104,6 +119,65 @@ __global__ __launch_bounds__(256) void embed_pair_hash_kernel(
 
 // ---------------------------------------------------------------------------------------------
 
+template <typename T, int VEC>
+__global__ __launch_bounds__(1024) void scale_add_norm_kernel(
+    float* __restrict__ stream, const T* __restrict__ y, int64_t y_stride, const float* __restrict__ scale,
+    const float* __restrict__ factor, const int* __restrict__ rows, T* __restrict__ cast, int hidden, float alpha,
+    float eps) {
+  using A = typename WideOf<T>::type;
+  __shared__ A scratch[16];
+  const int t = rows != nullptr ? rows[blockIdx.x] : blockIdx.x;
+  float* x = stream + (int64_t)t * hidden;
+  const T* add = y != nullptr ? y + (int64_t)t * y_stride : nullptr;
+  // a row is at most a few thousand columns: the sums of a thread's columns stay in registers
+  // between the two passes where they fit (4 turns), and are made again where they do not
+  constexpr int KEPT = 4;
+  A kept[KEPT][VEC];
+  A squares = 0;
+  int turn = 0;
+  for (int c = threadIdx.x * VEC; c < hidden; c += blockDim.x * VEC, ++turn) {
+    float v[VEC], u[VEC], s[VEC];
+    mi_load_cols<float, VEC>(x + c, v);
+    if (add != nullptr) {
+      mi_load_cols<T, VEC>(add + c, u);
+      if (scale != nullptr) mi_load_cols<float, VEC>(scale + c, s);
+    }
+#pragma unroll
+    for (int j = 0; j < VEC; ++j) {
+      A sum = (A)v[j];
+      if (add != nullptr) sum = (A)alpha * (A)v[j] + (scale != nullptr ? (A)s[j] * (A)u[j] : (A)u[j]);
+      if (turn < KEPT) kept[turn][j] = sum;
+      squares += sum * sum;
+    }
+  }
+  const A inv = inv_root_of(block_add<A>(squares, scratch) / (A)hidden, (A)eps);
+  T* narrow = cast != nullptr ? cast + (int64_t)blockIdx.x * hidden : nullptr;
+  turn = 0;
+  for (int c = threadIdx.x * VEC; c < hidden; c += blockDim.x * VEC, ++turn) {
+    float f[VEC], r[VEC];
+    mi_load_cols<float, VEC>(factor + c, f);
+    if (turn < KEPT) {
+#pragma unroll
+      for (int j = 0; j < VEC; ++j) r[j] = (float)((kept[turn][j] * inv) * (A)f[j]);
+    } else {
+      float v[VEC], u[VEC], s[VEC];
+      mi_load_cols<float, VEC>(x + c, v);
+      if (add != nullptr) {
+        mi_load_cols<T, VEC>(add + c, u);
+        if (scale != nullptr) mi_load_cols<float, VEC>(scale + c, s);
+      }
+#pragma unroll
+      for (int j = 0; j < VEC; ++j) {
+        A sum = (A)v[j];
+        if (add != nullptr) sum = (A)alpha * (A)v[j] + (scale != nullptr ? (A)s[j] * (A)u[j] : (A)u[j]);
+        r[j] = (float)((sum * inv) * (A)f[j]);
+      }
+    }
+    if (rows == nullptr) mi_store_cols<float, VEC>(x + c, r);
+    if (narrow != nullptr) mi_store_cols<T, VEC>(narrow + c, r);
+  }
+}
+
 // The routed experts' rows of a token (made [pair][width], expert by expert as expert_combine in routed_experts.hip takes them), which
 // are added up here instead of there: y[t] = sum_k weights[t, k] * (row of choice k) + shared_gate[t] * shared[t], rounded to T.
 struct ExpertRows {
@@ -114,54 +188,46 @@ struct ExpertRows {
   int experts, top;
 };
 
-// A row is a chain: its columns, their squares over the block, the factors, the result; few rows (decode) are that chain's time.  So the
-// factors are asked for with the columns, and the turns whose columns are kept are counted when compiling, so that their loads are in
-// flight together.  With the experts' sum made here, 12 layers with 11 of routed experts: 8 rows of 4096 3,167 -> 3,108 us a step, 1,501
-// rows of 3072 6,778 -> 6,706.
-template <typename T, int VEC, bool EXPERTS>
-__global__ __launch_bounds__(1024) void scale_add_norm_kernel(
-    float* __restrict__ stream, const T* __restrict__ y, int64_t y_stride, const float* __restrict__ scale,
-    const float* __restrict__ factor, const int* __restrict__ rows, T* __restrict__ cast, int hidden, float alpha,
-    float eps, ExpertRows e) {
+// The same norm with the experts' sum made here.  A row is a chain: the choices, their rows, the squares over the block, the factors, the
+// result; few rows (decode) are that chain's time.  So the factors are asked for with the columns, and the turns whose columns are kept are
+// counted when compiling, so that their loads are in flight together.  Microseconds of expert_combine and the kernel above / of this / of
+// this with the loop above: 2 experts a token, 8 rows of 4096 7.9 / 5.5 / 6.6, 1,501 rows of 3072 19.4 / 12.8 / 13.5.  (Without experts the
+// loop above is as fast or faster: 8 rows of 1024 2.9 against 3.2, of 4096 4.4 / 4.2, 1,501 float32 rows of 3072 12.3 / 14.4.)
+template <typename T, int VEC>
+__global__ __launch_bounds__(1024) void experts_add_norm_kernel(
+    float* __restrict__ stream, const float* __restrict__ scale, const float* __restrict__ factor, T* __restrict__ cast, int hidden,
+    float alpha, float eps, ExpertRows e) {
   using A = typename WideOf<T>::type;
   __shared__ A scratch[16];
-  const int t = rows != nullptr ? rows[blockIdx.x] : blockIdx.x;
+  const int t = blockIdx.x;
   float* x = stream + (int64_t)t * hidden;
-  const T* add = y != nullptr ? y + (int64_t)t * y_stride : nullptr;
   auto sum_at = [&](int c, A (&sum)[VEC]) {
     float v[VEC], u[VEC], s[VEC];
     mi_load_cols<float, VEC>(x + c, v);
-    if constexpr (EXPERTS) {
-      A total[VEC];
+    A total[VEC];
 #pragma unroll
-      for (int j = 0; j < VEC; ++j) total[j] = 0;
-      for (int k = 0; k < e.top; ++k) {
-        const int64_t pair = (int64_t)t * e.top + k;
-        const int chosen = e.chosen[pair];
-        if (chosen < 0) continue;
-        const T* src = chosen >= e.experts ? (const T*)e.x + (int64_t)t * e.x_stride : (const T*)e.made + pair * hidden;
-        mi_load_cols<T, VEC>(src + c, u);
-        const A weight = e.weights != nullptr ? (A)e.weights[pair] : (A)1;
+    for (int j = 0; j < VEC; ++j) total[j] = 0;
+    for (int k = 0; k < e.top; ++k) {
+      const int64_t pair = (int64_t)t * e.top + k;
+      const int chosen = e.chosen[pair];
+      if (chosen < 0) continue;
+      const T* src = chosen >= e.experts ? (const T*)e.x + (int64_t)t * e.x_stride : (const T*)e.made + pair * hidden;
+      mi_load_cols<T, VEC>(src + c, u);
+      const A weight = e.weights != nullptr ? (A)e.weights[pair] : (A)1;
 #pragma unroll
-        for (int j = 0; j < VEC; ++j) total[j] += weight * (A)u[j];
-      }
-      if (e.shared != nullptr) {
-        mi_load_cols<T, VEC>((const T*)e.shared + (int64_t)t * e.shared_stride + c, u);
-        const A g = e.shared_gate != nullptr ? (A)e.shared_gate[t] : (A)1;
-#pragma unroll
-        for (int j = 0; j < VEC; ++j) total[j] += g * (A)u[j];
-      }
-#pragma unroll
-      for (int j = 0; j < VEC; ++j) u[j] = to_f32(from_f32<T>((float)total[j]));
-    } else if (add != nullptr) {
-      mi_load_cols<T, VEC>(add + c, u);
+      for (int j = 0; j < VEC; ++j) total[j] += weight * (A)u[j];
     }
-    const bool adds = EXPERTS || add != nullptr;
-    if (adds && scale != nullptr) mi_load_cols<float, VEC>(scale + c, s);
+    if (e.shared != nullptr) {
+      mi_load_cols<T, VEC>((const T*)e.shared + (int64_t)t * e.shared_stride + c, u);
+      const A g = e.shared_gate != nullptr ? (A)e.shared_gate[t] : (A)1;
+#pragma unroll
+      for (int j = 0; j < VEC; ++j) total[j] += g * (A)u[j];
+    }
+    if (scale != nullptr) mi_load_cols<float, VEC>(scale + c, s);
 #pragma unroll
     for (int j = 0; j < VEC; ++j) {
-      sum[j] = (A)v[j];
-      if (adds) sum[j] = (A)alpha * (A)v[j] + (scale != nullptr ? (A)s[j] * (A)u[j] : (A)u[j]);
+      const float y = to_f32(from_f32<T>((float)total[j]));
+      sum[j] = (A)alpha * (A)v[j] + (scale != nullptr ? (A)s[j] * (A)y : (A)y);
     }
   };
   constexpr int KEPT = 4;
@@ -185,13 +251,13 @@ __global__ __launch_bounds__(1024) void scale_add_norm_kernel(
 #pragma unroll
     for (int j = 0; j < VEC; ++j) squares += sum[j] * sum[j];
   }
-  const A inv = inv_root_of(block_add<A>(squares, scratch) / (A)hidden, (A)eps);
-  T* narrow = cast != nullptr ? cast + (int64_t)blockIdx.x * hidden : nullptr;
+  const A inv = inv_root_of(block_add_at_once<A>(squares, scratch) / (A)hidden, (A)eps);
+  T* narrow = cast != nullptr ? cast + (int64_t)t * hidden : nullptr;
   auto write = [&](int c, const A (&sum)[VEC], const float (&factors)[VEC]) {
     float r[VEC];
 #pragma unroll
     for (int j = 0; j < VEC; ++j) r[j] = (float)((sum[j] * inv) * (A)factors[j]);
-    if (rows == nullptr) mi_store_cols<float, VEC>(x + c, r);
+    mi_store_cols<float, VEC>(x + c, r);
     if (narrow != nullptr) mi_store_cols<T, VEC>(narrow + c, r);
   };
 #pragma unroll
@@ -282,9 +348,11 @@ extern "C" int mi_scale_add_norm(int dtype, float* stream_rows, const void* y, i
   const ExpertRows e = {made, x, shared, chosen, weights, shared_gate, x_stride, shared_stride, experts, top};
 #define MI_POST(T, VEC)                                                                                                    \
   do {                                                                                                                     \
-    const auto kernel = made != nullptr ? scale_add_norm_kernel<T, VEC, true> : scale_add_norm_kernel<T, VEC, false>;      \
-    kernel<<<num_rows, threads, 0, stream>>>(stream_rows, (const T*)y, y_stride, scale, factor, rows, (T*)cast, hidden, alpha, \
-                                             eps, e);                                                                      \
+    if (made != nullptr)                                                                                                   \
+      experts_add_norm_kernel<T, VEC><<<num_rows, threads, 0, stream>>>(stream_rows, scale, factor, (T*)cast, hidden, alpha, eps, e); \
+    else                                                                                                                   \
+      scale_add_norm_kernel<T, VEC><<<num_rows, threads, 0, stream>>>(stream_rows, (const T*)y, y_stride, scale, factor,   \
+                                                                      rows, (T*)cast, hidden, alpha, eps);                 \
   } while (0)
   if (dtype == MI_F32) {
     if (vec) MI_POST(float, 4);
