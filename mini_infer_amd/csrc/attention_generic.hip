@@ -473,7 +473,8 @@ static int attn_generic_launch(const void* q, int64_t q_row_stride, const void* 
   // its loads were batched: a prompt of 509 tokens 247, then 148; such prompts now take attention_prompt_f32.hip, 66.)
   //
   // Up to three blocks a CU a wave has one or two 64s of keys and its time is the waits one after another, so that more loads in flight
-  // (DEEP) are worth two blocks a CU at once instead of three.  A layer with its combining launch: 24 heads of 128 over 8, 3 tokens of
+  // (DEEP) are worth two blocks a CU at once instead of three; for values of up to 64 dims, of which less is in flight, as long as two
+  // a CU are all there are (32 heads of 64 over 8, 40 / 48 tokens of 700, 640 / 768 blocks, 44.2 / 45.3 us without and 49.6 / 56.9 with it).  A layer with its combining launch: 24 heads of 128 over 8, 3 tokens of
   // up to 600 positions 43.1 -> 25.1 us, 30 of 200 (240 blocks) 42.8 -> 21.1, 32 heads, 8 of 2,000 (512) 63.4 -> 41.8; 32 heads of 64 over 8,
   // 3 of 600 21.9 -> 19.5, 60 of 200 (480) 22.0 -> 20.1, 15 of 1,500 (960, not taken) 43.5 / 41.5, 128 of one prompt (1,024, not taken)
   // 22.0 / 27.9.  (64 value rows, or all 64 values of a key row: the same for heads of 128 and 36 us for heads of 64, where the
@@ -495,7 +496,7 @@ static int attn_generic_launch(const void* q, int64_t q_row_stride, const void* 
     if constexpr (sizeof(S) == 8 && VPL <= 2) {                                                   \
       if (four) {                                                                                 \
         const size_t merge = 3 * GT * (VPL + 1) * MI_WAVE * sizeof(S) + 4 * GT * sizeof(float);   \
-        if (VEC && blocks <= 768) MI_ATTN_LAUNCH_WAVES(VPL, VEC, 4, VEC, lds + merge);            \
+        if (VEC && blocks <= (VPL == 1 ? 512 : 768)) MI_ATTN_LAUNCH_WAVES(VPL, VEC, 4, VEC, lds + merge); \
         else MI_ATTN_LAUNCH_WAVES(VPL, VEC, 4, false, lds + merge);                               \
         break;                                                                                    \
       }                                                                                           \
