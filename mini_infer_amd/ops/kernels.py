@@ -430,9 +430,10 @@ def linear_f32_out(x: torch.Tensor, weight: torch.Tensor, scale: float = 1.0, sc
     the scaling of the library's product are one launch).
 
     Few bfloat16 rows: the weight-streaming kernel writes float32 itself (no cast launch); its
-    values are those of `linear(...).float()`, rounded to bfloat16 on the way, so that a row's
-    logits do not depend on how many rows its step had.  Up to 256 rows of a large vocabulary: the same values from tiles
-    (128256 x 3072 at 24 / 64 / 256 rows 140 / 164 / 210 us against the vendor product and its cast's 166 / 192 / 307).
+    values are those of `linear(...).float()`, rounded to bfloat16 on the way, so that up to 16 rows a row's
+    logits do not depend on how many its step had.  Up to 256 rows of a large vocabulary: rounded the same from tiles, whose sums
+    over K may be in another order with another number of rows (4e-5 from the library's in the 2-norm; 128256 x 3072 at 24 / 64 /
+    256 rows 140 / 164 / 210 us against the vendor product and its cast's 166 / 192 / 307).
     More rows: the vendor library's product, cast.  float32 operands: `gemm_f32`."""
     if x.dtype == torch.float32:
         logits = gemm_f32(x, weight)
@@ -483,25 +484,27 @@ PARTIAL_SUMS_MAX_ROWS = 128
 
 def partial_sums_pay(m: int, n: int, k: int) -> bool:
     """Whether a product of these sizes is left as sums over ranges of K when its caller
-    takes them (`linear(..., partial_ok=True)`).  Measured on MI355X, the product alone with
+    takes them (`linear(..., partial_ok=True)`), in an order that depends on the matrix alone (`linear_partial_sums`; what this leaves
+    aside above 16 rows `tiles_for` may still cut).  Measured on MI355X, the product alone with
     weights from memory, microseconds whole / in pieces (whole = `gemm_skinny_bf16` up to
-    16 rows, the vendor library above):
+    16 rows, the vendor library above; in pieces = tiles):
 
-                                  8 rows    12 rows   16 rows   32 rows   64 rows
-        4096 x 14336 (8B down)    22 / 23   26 / 24   28 / 24   34 / 25   39 / 28
-        8192 x 28672 (70B down)   77 / 85   81 / 86   89 / 87  101 / 89  144 / 100
-        3072 x 8192  (3B down)    12 / 18   14 / 18   16 / 19   17 / 20   23 / 22
-        4096 x 4096  (8B o)        8 / 10    9 / 10   10 / 10   13 / 11   15 / 13
-        3072 x 3072  (3B o)        7 / 8     7 / 8     8 / 8    11 / 9    16 / 11
-        8192 x 8192  (70B o)      24 / 36   23 / 36   25 / 35   31 / 38   34 / 40
+                                  8 rows     12 rows    16 rows    32 rows    64 rows
+        4096 x 14336 (8B down)    22 / 20    25 / 20    28 / 20    31 / 21    39 / 24
+        8192 x 28672 (70B down)   75 / 72    77 / 71    82 / 71    92 / 74   134 / 87
+        3072 x 8192  (3B down)    11 / 11    13 / 11    14 / 11    17 / 11    23 / 13
+        4096 x 4096  (8B o)      7.8 / 7.9  8.5 / 8.0  9.4 / 8.0   13 / 8.3   15 / 9.7
+        3072 x 3072  (3B o)      6.6 / 6.1  7.3 / 6.1  7.8 / 6.1   11 / 6.6   16 / 8.0
+        8192 x 8192  (70B o)      23 / 26    23 / 26    24 / 26    29 / 27    33 / 29
 
-    and at 96 / 128 rows 63 / 75 against 36 / 39 (8B down), 22 / 24 against 16 / 18 (8B o),
-    121 / 201 against 130 / 131 (70B down)
+    and at 96 / 128 rows 63 / 75 against 29 / 35 (8B down), 22 / 24 against 12 / 15 (8B o),
+    115 / 198 against 99 / 125 (70B down).  With the norm behind it, which adds the pieces up, 8B down at
+    8 / 16 rows 25.4 / 31.2 against 23.8 / 23.7, 3B down 13.9 / 17.5 against 15.0 / 15.1, 8B o 11.0 / 12.6 against 12.0 / 12.0.
 
-    (the norm that adds the pieces up costs about a microsecond more than one that does not),
-    so: a long K from 11 rows on (15 with more than 4096 features), a small square-ish product
-    where the weight-streaming kernel ends (17 rows), nothing else.  Whole decode steps at 8B
-    sizes and 8 rows run 2.4 % faster with the down product whole, at 16 rows 2.6 % slower."""
+    So: a long K from 11 rows on (15 with more than 4096 features), a small square-ish product
+    where the weight-streaming kernel ends (17 rows), nothing else.  (The lines were drawn for a slower product in pieces, and none of
+    what lies on its side is slower in pieces now; up to 16 rows a little more would be faster, K of 12,288 from 8 rows and of
+    8,192 from 12.  Up to 64 rows the fixed order costs nothing against the best cut, at 128 8B down with its norm 39.9 / 38.1.)"""
     if not 5 <= m <= PARTIAL_SUMS_MAX_ROWS or n > 8192:
         return False
     if k >= 12288:
@@ -622,8 +625,8 @@ def tile_size(shape: int) -> tuple[int, int]:
 @functools.lru_cache(maxsize=8192)
 def gated_tiles_for(m: int, n: int, k: int, cus: int = WHOLE_DEVICE_CUS) -> int | None:
     """The tile shape where the gated product of n features is made in tiles, or None.  Up to 32 rows the streaming product
-    (`gemm_skinny_swiglu_bf16`) gives a row the same bits as it gets in a step of its own; tiles are not faster everywhere there (gate|up
-    at 24 rows: 16384 x 3072 19.8 against 23.9 us, 28672 x 4096 50.8 against 47.1).  Above, measured against the vendor product
+    (`gemm_skinny_swiglu_bf16`) stands, because tiles are not faster everywhere there (gate|up at 24 rows: 16384 x 3072 19.8 against 23.9 us,
+    28672 x 4096 50.8 against 47.1) and no rule between the two has been measured.  Above, measured against the vendor product
     and `silu_mul`, tiles are 1.0 to 1.9 times as fast up to 160 rows, and beyond as long as tiles of up to 192 x 128 are what pays
     (7168 x 4096 at 256 / 600 rows 32.5 / 48.2 against 43.8 / 53.8, 16384 x 2048 at 271 / 320 29.4 / 30.8 against 33.3 /
     33.9); where there is work for larger ones the library is faster by as much as 1.3 (28672 x 4096 at 193 rows 86.9 / 72.3, 57344 x
@@ -1331,7 +1334,10 @@ def paged_attention(
                 return out
             tile = lib.mi_attn_mfma_tokens_per_tile(q_heads, kv_heads, ATTN_SHAPE_PREFILL)
             num_tiles = sum(-(-n // tile) for n in lens)
-            # (portions are cut from 512 keys on only: a portion of 256 tokens in two ranges would need the combining launch for all its rows)
+            # (portions are cut from 512 keys on only: a portion of 256 tokens in two ranges would need the combining launch for all its rows.
+            # Sixteen ranges at most, at any length: beside a portion of 256 one token at 16k / 32k / 128k positions, 24 heads of 128 over
+            # 8, takes 22.4 / 34.9 / 94.4 us, in 32 ranges, as it would have alone, 26.9 / 37.4 / 105; launched one after the other
+            # 47.6 / 59.5 / 116.  A portion at 8k / 32k beside a token at 700: 51.4 / 143 us, before 64.7 / 158.)
             mixed(leading_single, num_tiles,
                   min(16, attention_splits(leading_single * kv_heads * -(-group // 16), seen(1, max(most[:leading_single])), target=256, min_keys=128)),
                   min(16, attention_splits(num_tiles * kv_heads * -(-group // 128), seen(tile, max(most[leading_single:])), target=512, min_keys=256)))

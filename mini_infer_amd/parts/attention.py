@@ -289,7 +289,7 @@ class GQAttention(Mixer):
             return self._project(self._attend(queries, ctx, cache))
         if writes_cache:
             # A projection left in pieces is added up by the rotation's launch, in steps of single tokens: 8B sizes, 40 of them,
-            # 4,650 -> 4,500 us a step.  A portion's values are written a page at a time, sixteen tokens a thread, and all their
+            # 4,574 -> 4,494 us a step.  A portion's values are written a page at a time, sixteen tokens a thread, and all their
             # pieces there cost more than a launch (60 tokens beside 9 single ones, 8B 5,420 -> 5,950; 100 beside 10, 1B 1,567 -> 1,851).
             in_pieces = (not self.steady and ctx.max_q_len == 1 and rotary is not None and self._same_widths and self._plain_heads
                          and ops.rope_takes_partial_sums(self.head_dim, rotary.rotary_dim, rotary.interleaved))

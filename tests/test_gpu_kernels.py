@@ -874,6 +874,16 @@ def test_paged_attention_of_portions_beside_single_tokens_in_one_launch(monkeypa
     assert (got.float() - attend(**options).float()).abs().max() < _tol(torch.bfloat16, 2) and len(taken) == 2
 
 
+@pytest.mark.parametrize("q_heads,kv_heads,head_dim", [(6, 2, 128), (8, 1, 64)])
+@pytest.mark.parametrize("lengths,q_lens", [([20000, 300], [1, 300]), ([17, 9100], [1, 150]), ([12001, 8300, 8200], [1, 1, 33])])
+def test_paged_attention_of_long_contexts_beside_portions(q_heads, kv_heads, head_dim, lengths, q_lens):
+    """Thousands of positions on either side, and on both, cut into their most ranges."""
+    case = _paged_case(torch.bfloat16, q_heads, kv_heads, head_dim, 16, lengths, q_lens, seed=23, v_transposed=True)
+    scale = head_dim ** -0.5
+    out = _attend(case, q_heads, kv_heads, head_dim, scale, None, max(lengths))
+    assert np.abs(out.double().cpu().numpy() - _attention_expected(case, scale, None)).max() < _tol(torch.bfloat16, 2)
+
+
 @pytest.mark.parametrize("lengths,q_lens", [([30, 20], [1, 0]), ([300, 20, 900, 1], [1, 1, 0, 0]), ([30, 20, 9], [1, 0, 1]), ([600, 70, 300], [1, 0, 70])])
 def test_paged_attention_of_single_tokens_before_requests_without_tokens(lengths, q_lens):
     """Boundaries known to the host, some requests of the step without tokens behind those with one."""
