@@ -258,3 +258,16 @@ __device__ __forceinline__ void mi_take_flagged(int64_t total, F flagged, G take
 
 static __host__ __device__ inline int ceil_div(int a, int b) { return (a + b - 1) / b; }
 static inline int64_t ceil_div64(int64_t a, int64_t b) { return (a + b - 1) / b; }
+
+// Compute units of the current device (asked once per device).
+static inline int mi_compute_units() {
+  static int cached[64] = {0};
+  int device = 0;
+  if (hipGetDevice(&device) != hipSuccess || device < 0 || device >= 64) return 0;
+  if (cached[device] == 0) {
+    int count = 0;
+    if (hipDeviceGetAttribute(&count, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess) return 0;
+    cached[device] = count;
+  }
+  return cached[device];
+}

@@ -3,12 +3,22 @@
 // nothing the host has to know: the pairs are listed expert by expert on the device (`expert_sort`),
 // and a block finds its tile in that list.
 //
-// Both operands pass through LDS, 64 elements of K at a time, two buffers: while one is worked on, the next
-// is on its way straight from memory into LDS (no registers between).  A row of a buffer is 128 bytes, eight
-// chunks of 16; chunk c of row r lies at place c ^ (r % 8), so that the eight lanes that are served together
-// find their 16-byte pieces in different banks.  The waves stand 2 x 2 over the tile; MFMA 16x16x32 with
-// weight rows as the first operand and pairs as the second, so a lane ends with four consecutive features of
-// a pair.
+// The tiles are those of turns_product.h, 64, 128, 160 or 256 pairs x 256 weight rows, one block to a CU; all of them sum in the
+// same order, so which one is taken does not show in the results.  What bounds such a launch is the matrix cores, and the
+// last round of blocks, which may be nearly empty: 2,700 pairs over 16 experts are 22 to 50 row tiles, and a row tile more or less
+// decides whether it takes one round or two.  The host does not know how many pairs an expert got, so every block works out
+// from the list, before it looks for its tile, how long the launch takes in either size and takes the shortest: all
+// blocks see the same list and take the same.  Measured (microseconds, the pairs as routers spread them, 58 to 333 an expert;
+// before: tiles of 128 x 128 on two buffers, four waves in step, two blocks to a CU):
+//     experts x gate|up, down            pairs    before        now
+//     16 x 4096 x 3072, 3072 x 2048      1,942    133 +  40     102 +  42
+//                                        3,238    161 +  70     126 +  52
+//                                        4,122    173 +  70     123 +  56
+//     16 x 7168 x 4096, 4096 x 3584      2,612    261 + 153     210 + 124
+//                                        5,776    430 + 245     308 + 176
+// and over 120 such pairs of launches 1.17 times as fast from 96 to 200 pairs an expert, 1.23 beyond, and below, where the weights' bytes
+// bound both, 1.03 to 1.04 (a single launch at worst 0.93, both together 0.97).  A step of 1,501 tokens of 12 layers at the
+// first sizes 6,708 -> 6,429 us.
 //
 // Tiles are numbered expert by expert, within an expert feature tile by feature tile with the row tiles of one
 // feature tile side by side; each of the 8 XCDs takes one stretch of these numbers (workgroups are dealt
@@ -17,15 +27,62 @@
 //
 // MODE as in routed_experts.hip: 0 plain, 1 silu(gate) * up (a block then makes BN / 2 features: gate and up rows
 // side by side in its tile), 2 relu(weight * z)^2.
-#include "common.h"
+#include "turns_product.h"
 
 namespace {
 
-typedef float f32x4_e __attribute__((ext_vector_type(4)));
-typedef __attribute__((address_space(3))) void lds_void;
-typedef const __attribute__((address_space(1))) void global_void;
-
 #define TILE_K 64
+
+// The tiles, by rows, with the microseconds that a step of 64 of K takes one; a launch is expected to take, beside what any launch
+// does, the longer of its rounds of blocks, each its steps and ROUND_MICROS for beginning and end, and the bytes of W, once from memory
+// and again from cache for every row tile.  A fit to 840 launches in these four sizes (8 to 64 experts, 1024 to 7168 wide, 2 to
+// 1,240 pairs an expert, half of them gated; 12 % off): what it picks is 1 % slower than the best of the four.
+struct TileForm {
+  int rows;
+  float step_micros;
+};
+constexpr int FORMS = 4;
+constexpr int FORM_FEATURES = 256;  // weight rows of a tile, in all of them
+__host__ __device__ constexpr TileForm tile_form(int i) {
+  return i == 0 ? TileForm{64, 0.53f} : i == 1 ? TileForm{128, 0.86f} : i == 2 ? TileForm{160, 0.99f} : TileForm{256, 1.40f};
+}
+
+// The tile that a launch takes: row_tiles[f] of form f cover the pairs (0: not to be taken); used: experts with pairs; n, k: an expert's weight rows
+// and their length; cus: compute units, in 8 XCDs to which blocks are dealt in turn.
+__host__ __device__ inline int pick_form(const int (&row_tiles)[FORMS], int used, int n, int k, int cus) {
+  constexpr float ROUND_MICROS = 6.3f, FROM_MEMORY = 1.0e-7f, AGAIN = 0.85e-7f;  // a byte of W
+  const float steps = (float)(k / TILE_K);
+  int best = -1;
+  float least = 0.f;
+  for (int f = 0; f < FORMS; ++f) {
+    if (row_tiles[f] == 0) continue;
+    const int blocks = row_tiles[f] * ((n + FORM_FEATURES - 1) / FORM_FEATURES), rounds = ((blocks + 7) / 8 + cus / 8 - 1) / (cus / 8);
+    const float multiplied = (float)rounds * (steps * tile_form(f).step_micros + ROUND_MICROS);
+    const float brought = FROM_MEMORY * (float)used * (float)n * (float)k * 2.f + AGAIN * (float)blocks * steps * (FORM_FEATURES * TILE_K * 2.f);
+    const float micros = multiplied > brought ? multiplied : brought;
+    if (best < 0 || micros < least * 0.995f) best = f, least = micros;  // (level: the smaller one)
+  }
+  return best;
+}
+
+// The same on the device, from the list.  All threads of the block get the same answer.
+__device__ __forceinline__ int pick_form(const int* __restrict__ first, int experts, bool smallest, int n, int k, int cus) {
+  int row_tiles[FORMS] = {}, used = 0;
+  for (int e = threadIdx.x % MI_WAVE; e < experts; e += MI_WAVE) {
+    const int pairs = first[e + 1] - first[e];
+    used += pairs > 0;
+#pragma unroll
+    for (int f = 0; f < FORMS; ++f) row_tiles[f] += (pairs + tile_form(f).rows - 1) / tile_form(f).rows;
+  }
+#pragma unroll
+  for (int off = MI_WAVE / 2; off > 0; off >>= 1) {
+    used += __shfl_xor(used, off, MI_WAVE);
+#pragma unroll
+    for (int f = 0; f < FORMS; ++f) row_tiles[f] += __shfl_xor(row_tiles[f], off, MI_WAVE);
+  }
+  if (!smallest) row_tiles[0] = 0;
+  return __builtin_amdgcn_readfirstlane(pick_form(row_tiles, used, n, k, cus));
+}
 
 // Which tile this block works on: expert, first pair of the row tile (an index into `listed`), feature tile.
 // False: past the last tile.  All threads of the block get the same answer.
@@ -70,131 +127,55 @@ __device__ __forceinline__ bool find_tile(const int* __restrict__ first, int exp
   return false;
 }
 
-// (two blocks to a CU: without the bound the compiler spreads over more registers than two leave each)
-template <int MODE, int BM, int BN>
-__global__ __launch_bounds__(256, 2) void expert_tiles_lds_kernel(
-    const bf16_t* __restrict__ src, int64_t src_stride, int src_div, const bf16_t* __restrict__ weight,
+template <class T, int MODE>
+__device__ __forceinline__ void make_tile(
+    bf16_t* ring, const bf16_t* __restrict__ src, int64_t src_stride, int src_div, const bf16_t* __restrict__ weight,
     int64_t expert_stride, const int* __restrict__ listed, const int* __restrict__ first,
-    const float* __restrict__ pair_weight, bf16_t* __restrict__ out, int64_t out_stride, int experts, int k_dim,
-    int features, int feature_tiles) {
+    const float* __restrict__ pair_weight, bf16_t* __restrict__ out, int64_t out_stride, int experts, int k_dim, int features) {
   constexpr bool GATED = MODE == 1;
-  constexpr int WM = BM / 2, WN = BN / 2;     // a wave's share of the tile: pairs, weight rows
-  constexpr int MT = WM / 16, NT = WN / 16;   // in tiles of 16
-  constexpr int ROW = TILE_K;                 // elements of a row in LDS
-  constexpr int A_LOADS = BM / 32, B_LOADS = BN / 32;  // 8-row loads a wave makes for each operand
-  // (an array of its own for each buffer: the compiler then sees that what is fetched into one does not touch
-  // what is read from the other, and waits for nothing between)
-  __shared__ __align__(16) bf16_t pairs_even[BM * ROW], pairs_odd[BM * ROW];
-  __shared__ __align__(16) bf16_t rows_even[BN * ROW], rows_odd[BN * ROW];
-
+  constexpr int FEATURES = GATED ? T::BN / 2 : T::BN, HALF = T::NT / 2;
+  static_assert(T::BN == FORM_FEATURES);
+  const int feature_tiles = (features + FEATURES - 1) / FEATURES;
   int expert, row0, feature_tile;
-  if (!find_tile(first, experts, feature_tiles, BM, blockIdx.x, expert, row0, feature_tile)) return;
-  const int end = first[expert + 1];
-  const int wave = threadIdx.x / MI_WAVE, lane = threadIdx.x % MI_WAVE;
-  const int col = lane % 16, quad = lane / 16;
-  // a block's features: BN of them, or where they come in pairs BN / 2 (the tile's lower half of weight rows
-  // their gate rows, its upper half their up rows)
-  constexpr int FEATURES = GATED ? BN / 2 : BN;
-  const int f0 = feature_tile * FEATURES;
-
-  // what this lane fetches: 16 bytes of row 8 * load + lane / 8, chunk (lane % 8) ^ (lane / 8), of every load
-  const int chunk = (lane % 8) ^ (lane / 8);
-  const bf16_t* a_src[A_LOADS];
-  const bf16_t* b_src[B_LOADS];
-#pragma unroll
-  for (int i = 0; i < A_LOADS; ++i) {
-    const int r = (wave * A_LOADS + i) * 8 + lane / 8;
-    const int pair = listed[min(row0 + r, end - 1)];  // (past the expert's last pair: that one again, not written)
-    a_src[i] = src + (int64_t)(pair / src_div) * src_stride + chunk * 8;
-  }
+  if (!find_tile(first, experts, feature_tiles, T::BM, blockIdx.x, expert, row0, feature_tile)) return;
+  const int end = first[expert + 1], f0 = feature_tile * FEATURES;
   const bf16_t* w = weight + (int64_t)expert * expert_stride;
+  T tile;
+  tile.run(
+      ring, k_dim / TILE_K,
+      [&](int r) {  // (past the expert's last pair: that one again, not written)
+        return src + (int64_t)(listed[min(row0 + r, end - 1)] / src_div) * src_stride;
+      },
+      [&](int r) {
+        if constexpr (GATED) {  // of a wave's tiles of weight rows the first half are gate rows, the second the up rows of the same features
+          const int t = r / 16 % T::NT, f = min(f0 + (r / (T::NT * 16) * HALF + t % HALF) * 16 + r % 16, features - 1);
+          return w + (int64_t)(t < HALF ? f : f + features) * k_dim;
+        } else {
+          return w + (int64_t)min(f0 + r, features - 1) * k_dim;
+        }
+      });
 #pragma unroll
-  for (int i = 0; i < B_LOADS; ++i) {
-    const int r = (wave * B_LOADS + i) * 8 + lane / 8;
-    int row;
-    if constexpr (GATED) row = min(f0 + (r % FEATURES), features - 1) + (r / FEATURES) * features;
-    else row = min(f0 + r, features - 1);
-    b_src[i] = w + (int64_t)row * k_dim + chunk * 8;
-  }
-  auto fetch = [&](bf16_t* pairs_lds, bf16_t* rows_lds, int k) {
-#pragma unroll
-    for (int i = 0; i < A_LOADS; ++i)
-      __builtin_amdgcn_global_load_lds((global_void*)(a_src[i] + k),
-                                       (lds_void*)(&pairs_lds[(wave * A_LOADS + i) * 8 * ROW]), 16, 0, 0);
-#pragma unroll
-    for (int i = 0; i < B_LOADS; ++i)
-      __builtin_amdgcn_global_load_lds((global_void*)(b_src[i] + k),
-                                       (lds_void*)(&rows_lds[(wave * B_LOADS + i) * 8 * ROW]), 16, 0, 0);
-  };
-
-  const int m_half = wave / 2, n_half = wave % 2;
-  f32x4_e acc[NT][MT];
-#pragma unroll
-  for (int n = 0; n < NT; ++n)
-#pragma unroll
-    for (int m = 0; m < MT; ++m) acc[n][m] = f32x4_e{0.f, 0.f, 0.f, 0.f};
-
-  // weight-row tile n of this wave: gated, its first half are gate rows and its second the up rows of the same features
-  auto row_tile = [&](int n) {
-    if constexpr (GATED) return (n < NT / 2 ? n_half * (NT / 2) + n : NT + n_half * (NT / 2) + (n - NT / 2)) * 16;
-    else return (n_half * NT + n) * 16;
-  };
-
-  auto work = [&](const bf16_t* pairs_lds, const bf16_t* rows_lds) {
-#pragma unroll
-    for (int s = 0; s < TILE_K / 32; ++s) {
-      bf16x8_t a[NT], b[MT];
-      const int place = ((s * 4 + quad) ^ (col % 8)) * 8;
-#pragma unroll
-      for (int n = 0; n < NT; ++n) a[n] = *reinterpret_cast<const bf16x8_t*>(&rows_lds[(row_tile(n) + col) * ROW + place]);
-#pragma unroll
-      for (int m = 0; m < MT; ++m)
-        b[m] = *reinterpret_cast<const bf16x8_t*>(&pairs_lds[(m_half * WM + m * 16 + col) * ROW + place]);
-#pragma unroll
-      for (int n = 0; n < NT; ++n)
-#pragma unroll
-        for (int m = 0; m < MT; ++m) acc[n][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[n], b[m], acc[n][m], 0, 0, 0);
-    }
-  };
-  auto whole = [&]() {  // what was asked for last is there, for all waves, and nobody reads the other buffer any more
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-  };
-
-  fetch(pairs_even, rows_even, 0);
-  const int steps = k_dim / TILE_K;
-  for (int step = 0; step < steps; step += 2) {
-    whole();
-    if (step + 1 < steps) fetch(pairs_odd, rows_odd, (step + 1) * TILE_K);
-    work(pairs_even, rows_even);
-    if (step + 1 >= steps) break;
-    whole();
-    if (step + 2 < steps) fetch(pairs_even, rows_even, (step + 2) * TILE_K);
-    work(pairs_odd, rows_odd);
-  }
-
-#pragma unroll
-  for (int m = 0; m < MT; ++m) {
-    const int r = row0 + m_half * WM + m * 16 + col;
+  for (int m = 0; m < T::MT; ++m) {
+    const int r = row0 + tile.row(m);
     if (r >= end) continue;
     const int pair = listed[r];
     bf16_t* o = out + (int64_t)pair * out_stride;
     const float pw = MODE == 2 && pair_weight != nullptr ? pair_weight[pair] : 1.f;
 #pragma unroll
-    for (int n = 0; n < (GATED ? NT / 2 : NT); ++n) {
-      const int f = f0 + (GATED ? (n_half * (NT / 2) + n) * 16 : (n_half * NT + n) * 16) + 4 * quad;
+    for (int n = 0; n < (GATED ? HALF : T::NT); ++n) {
+      const int f = f0 + (GATED ? (tile.wn * HALF + n) * 16 + tile.quad * 4 : tile.feature(n));
       float v[4];
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         if constexpr (GATED) {
           // the two products as the element type holds them, then silu(gate) * up
-          const float g = to_f32(from_f32<bf16_t>(acc[n][m][j])), u = to_f32(from_f32<bf16_t>(acc[n + NT / 2][m][j]));
+          const float g = to_f32(from_f32<bf16_t>(tile.acc[n][m][j])), u = to_f32(from_f32<bf16_t>(tile.acc[n + HALF][m][j]));
           v[j] = g / (1.f + expf(-g)) * u;
         } else if constexpr (MODE == 2) {
-          const float z = fmaxf(pw * acc[n][m][j], 0.f);
+          const float z = fmaxf(pw * tile.acc[n][m][j], 0.f);
           v[j] = z * z;
         } else {
-          v[j] = acc[n][m][j];
+          v[j] = tile.acc[n][m][j];
         }
       }
       if (f + 4 <= features && out_stride % 4 == 0) {
@@ -208,21 +189,61 @@ __global__ __launch_bounds__(256, 2) void expert_tiles_lds_kernel(
   }
 }
 
-template <int MODE, int BM, int BN>
+using Tile64 = TurnsProduct<2, 4, 2, 4, 3>;
+using Tile128 = TurnsProduct<2, 4, 4, 4, 3>;
+using Tile160 = TurnsProduct<2, 4, 5, 4, 3>;
+using Tile256 = TurnsProduct<2, 4, 8, 4, 2>;
+
+template <int MODE>
+__global__ __launch_bounds__(512, 2) void expert_tiles_kernel(
+    const bf16_t* __restrict__ src, int64_t src_stride, int src_div, const bf16_t* __restrict__ weight,
+    int64_t expert_stride, const int* __restrict__ listed, const int* __restrict__ first,
+    const float* __restrict__ pair_weight, bf16_t* __restrict__ out, int64_t out_stride, int experts, int k_dim,
+    int features, bool smallest, int cus) {
+  __shared__ __align__(16) bf16_t ring[Tile160::RING];
+  static_assert(Tile160::RING >= Tile64::RING && Tile160::RING >= Tile128::RING && Tile160::RING >= Tile256::RING);
+  const int form = pick_form(first, experts, smallest, MODE == 1 ? 2 * features : features, k_dim, cus);
+#define MI_TILE(T) make_tile<T, MODE>(ring, src, src_stride, src_div, weight, expert_stride, listed, first, pair_weight, out, out_stride, experts, k_dim, features)
+  if (form == 0) MI_TILE(Tile64);
+  else if (form == 1) MI_TILE(Tile128);
+  else if (form == 2) MI_TILE(Tile160);
+  else if (form == 3) MI_TILE(Tile256);
+#undef MI_TILE
+}
+
+// Pairs an expert has on average up to which tiles of 64 may be taken (they were the best of the four up to 71): a launch has a block for
+// every tile that there can be of the smallest size, and the rest end when they have read the list.
+constexpr int SMALLEST_UP_TO = 96;
+
+template <int MODE>
 void launch_tiles(const void* src, int64_t src_stride, int src_div, const void* weight, const int* listed, const int* first,
-                  const float* pair_weight, void* out, int64_t out_stride, int pairs, int experts, int k_dim, int features,
+                  const float* pair_weight, void* out, int64_t out_stride, int pairs, int experts, int k_dim, int features, int cus,
                   hipStream_t stream) {
-  const int feature_tiles = ceil_div(features, MODE == 1 ? BN / 2 : BN);
-  const int most = feature_tiles * (pairs / BM + min(experts, pairs));  // (an expert's last tile may be a short one)
-  expert_tiles_lds_kernel<MODE, BM, BN><<<ceil_div(most, 8) * 8, 256, 0, stream>>>(
+  const int feature_tiles = ceil_div(features, MODE == 1 ? FORM_FEATURES / 2 : FORM_FEATURES);
+  const bool smallest = pairs <= (int64_t)SMALLEST_UP_TO * experts;
+  const int most = feature_tiles * (pairs / tile_form(smallest ? 0 : 1).rows + min(experts, pairs));  // (an expert's last tile may be a short one)
+  expert_tiles_kernel<MODE><<<ceil_div(most, 8) * 8, 512, 0, stream>>>(
       (const bf16_t*)src, src_stride, src_div, (const bf16_t*)weight, (int64_t)(MODE == 1 ? 2 : 1) * features * k_dim, listed,
-      first, pair_weight, (bf16_t*)out, out_stride, experts, k_dim, features, feature_tiles);
+      first, pair_weight, (bf16_t*)out, out_stride, experts, k_dim, features, smallest, cus);
 }
 
 }  // namespace
 
 // Whether rows of k_dim bfloat16 elements are taken.
 extern "C" int mi_expert_tiles_take(int k_dim) { return k_dim > 0 && k_dim % TILE_K == 0; }
+
+// Rows of the tile that a launch of n weight rows an expert takes where the experts got counts[0..experts) pairs (0: no pairs).
+extern "C" int mi_expert_tiles_rows(const int* counts, int experts, int n, int k_dim, int cus) {
+  int row_tiles[FORMS] = {}, used = 0;
+  int64_t pairs = 0;
+  for (int e = 0; e < experts; ++e) {
+    pairs += counts[e], used += counts[e] > 0;
+    for (int f = 0; f < FORMS; ++f) row_tiles[f] += ceil_div(counts[e], tile_form(f).rows);
+  }
+  if (pairs > (int64_t)SMALLEST_UP_TO * experts) row_tiles[0] = 0;
+  const int form = pick_form(row_tiles, used, n, k_dim, max(8, cus));
+  return form < 0 ? 0 : tile_form(form).rows;
+}
 
 // Arguments as mi_expert_rows (bfloat16 only), with the number of listed pairs.
 extern "C" int mi_expert_tiles(int mode, const void* src, int64_t src_stride, int src_div, const void* weight,
@@ -233,10 +254,11 @@ extern "C" int mi_expert_tiles(int mode, const void* src, int64_t src_stride, in
   MI_REQUIRE(mi_expert_tiles_take(k_dim) && src_stride % 8 == 0 && ((uintptr_t)src | (uintptr_t)weight) % 16 == 0 && (uintptr_t)out % 8 == 0,
              "expert_tiles: rows of %d elements are not taken %d at a time", k_dim, TILE_K);
   MI_REQUIRE(mode >= 0 && mode <= 2, "expert_tiles: mode %d", mode);
-  MI_REQUIRE((int64_t)ceil_div(features, 64) * ((int64_t)pairs / 128 + experts) < (1 << 30), "expert_tiles: too many tiles");
+  MI_REQUIRE((int64_t)ceil_div(features, 128) * ((int64_t)pairs / 64 + experts) < (1 << 30), "expert_tiles: too many tiles");
   if (pairs == 0) return MI_OK;
+  const int cus = max(8, mi_compute_units());
 #define MI_TILES(MODE) \
-  launch_tiles<MODE, 128, 128>(src, src_stride, src_div, weight, listed, first, pair_weight, out, out_stride, pairs, experts, k_dim, features, stream)
+  launch_tiles<MODE>(src, src_stride, src_div, weight, listed, first, pair_weight, out, out_stride, pairs, experts, k_dim, features, cus, stream)
   if (mode == 1) MI_TILES(1);
   else if (mode == 2) MI_TILES(2);
   else MI_TILES(0);

@@ -755,19 +755,6 @@ __global__ __launch_bounds__(64 * SK_WAVES) void gemm_skinny_bf16_kernel(
 #define SK_MAX_ROWS 16
 #define SK_WIDE_MAX_ROWS 32
 
-// Compute units of the current device (asked once per device).
-static int compute_units() {
-  static int cached[64] = {0};
-  int device = 0;
-  if (hipGetDevice(&device) != hipSuccess || device < 0 || device >= 64) return 0;
-  if (cached[device] == 0) {
-    int count = 0;
-    if (hipDeviceGetAttribute(&count, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess) return 0;
-    cached[device] = count;
-  }
-  return cached[device];
-}
-
 static bool skinny_takes(int m, int n, int k, int64_t lda, int64_t ldw, int max_rows) {
   return m >= 1 && m <= max_rows && n >= 1 && k >= 32 && k % 32 == 0 && lda % 8 == 0 && ldw % 8 == 0;
 }
@@ -810,7 +797,7 @@ static int skinny_plain(const void* a, int64_t lda, const void* w, int64_t ldw, 
   const bf16_t* ap = (const bf16_t*)a;
   const bf16_t* wp = (const bf16_t*)w;
   bf16_t* cp = (bf16_t*)c;
-  const int cus = compute_units();
+  const int cus = mi_compute_units();
   MI_REQUIRE(cus > 0, "gemm_skinny_bf16: cannot read the device's compute unit count");
   const int fpb = features_per_block_for(n, cus, 4);
   const int blocks = ceil_div(n, fpb);
@@ -897,7 +884,7 @@ extern "C" int mi_gemm_skinny_attn_bf16(const float* part_acc, const float* part
   args.num_splits = num_splits;
   args.attn_heads = heads;
   args.attn_head_dim = head_dim;
-  const int cus = compute_units();
+  const int cus = mi_compute_units();
   MI_REQUIRE(cus > 0, "gemm_skinny_attn_bf16: cannot read the device's compute unit count");
   const int fpb = features_per_block_for(n, cus, 4);
   const int blocks = ceil_div(n, fpb);
@@ -925,7 +912,7 @@ extern "C" int mi_gemm_skinny_attn_bf16(const float* part_acc, const float* part
 // pieces = mi_gemm_skinny_addnorm_pieces(n).  With part_acc the activations are the
 // uncombined key ranges of attn_mfma (as in mi_gemm_skinny_attn_bf16; a, lda unused).
 extern "C" int mi_gemm_skinny_addnorm_pieces(int n) {
-  const int cus = compute_units();
+  const int cus = mi_compute_units();
   if (cus <= 0 || n < 1) return 0;
   return ceil_div(n, features_per_block_for(n, cus, 4));
 }
@@ -964,7 +951,7 @@ extern "C" int mi_gemm_skinny_addnorm_bf16(const void* a, int64_t lda, const flo
   const bf16_t* ap = from_attention ? wp : (const bf16_t*)a;  // (never read when the activations are made in the kernel)
   if (from_attention) lda = ldw;
   bf16_t* cp = (bf16_t*)values;
-  const int cus = compute_units();
+  const int cus = mi_compute_units();
   MI_REQUIRE(cus > 0, "gemm_skinny_addnorm_bf16: cannot read the device's compute unit count");
   const int fpb = features_per_block_for(n, cus, 4);
   const int blocks = ceil_div(n, fpb);
@@ -1008,7 +995,7 @@ extern "C" int mi_gemm_skinny_swiglu_scaled_bf16(const void* a, int64_t lda, con
   args.sumsq_pieces = pieces;
   args.norm_eps = eps;
   args.norm_width = k;
-  const int cus = compute_units();
+  const int cus = mi_compute_units();
   MI_REQUIRE(cus > 0, "gemm_skinny_swiglu_scaled_bf16: cannot read the device's compute unit count");
   const int fpb = features_per_block_for(n, cus, 2);
   const int blocks = ceil_div(n, fpb);
@@ -1068,7 +1055,7 @@ static int skinny_gated(const void* a, int64_t lda, const void* w, int64_t ldw, 
   const bf16_t* ap = (const bf16_t*)a;
   const bf16_t* wp = (const bf16_t*)w;
   bf16_t* cp = (bf16_t*)out;
-  const int cus = compute_units();
+  const int cus = mi_compute_units();
   MI_REQUIRE(cus > 0, "gemm_skinny_swiglu_bf16: cannot read the device's compute unit count");
   const int fpb = features_per_block_for(n, cus, 2);  // two output tiles = four weight tiles
   const int blocks = ceil_div(n, fpb);
@@ -1120,7 +1107,7 @@ extern "C" int mi_gemm_skinny_gru_bf16(const void* a, int64_t lda, const void* w
   fold.gru_num_slots = num_slots;
   fold.gru_bz = bz;
   fold.gru_bx = bx;
-  const int cus = compute_units();
+  const int cus = mi_compute_units();
   MI_REQUIRE(cus > 0, "gemm_skinny_gru_bf16: cannot read the device's compute unit count");
   const int fpb = features_per_block_for(n, cus, 1);  // one output tile = three weight tiles
   const int blocks = ceil_div(n, fpb);
@@ -1171,7 +1158,7 @@ static int rope_product(const char* name, const void* a, int64_t lda, const floa
   fold.norm_eps = eps;
   fold.norm_width = k;
   // pairs per block: an even share over the CUs in whole rounds, as for the plain product
-  const int cus = compute_units();
+  const int cus = mi_compute_units();
   MI_REQUIRE(cus > 0, "%s: cannot read the device's compute unit count", name);
   const int total_pairs = n / 2;
   const int rounds = ceil_div(total_pairs, cus * 16);
@@ -1283,7 +1270,7 @@ extern "C" int mi_gemm_skinny_layer_in_bf16(const void* a, int64_t lda, const fl
   fold.sumsq_pieces = pieces;
   fold.norm_eps = eps;
   fold.norm_width = k;
-  const int cus = compute_units();
+  const int cus = mi_compute_units();
   MI_REQUIRE(cus > 0, "gemm_skinny_layer_in_bf16: cannot read the device's compute unit count");
   const int n = (int)(rows / 2);  // pairs
   const int fpb = features_per_block_for(n, cus, 2);

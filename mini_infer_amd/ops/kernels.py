@@ -3227,6 +3227,13 @@ def expert_tiles_take(x: torch.Tensor, ff: int) -> bool:
     return x.dtype == torch.bfloat16 and bool(lib.mi_expert_tiles_take(x.shape[1])) and bool(lib.mi_expert_tiles_take(ff))
 
 
+def expert_tile_rows(counts: list[int], weight_rows: int, k: int, cus: int = WHOLE_DEVICE_CUS) -> int:
+    """Rows of the tile that a launch of the tiles staged through LDS takes where the experts got `counts` pairs, `weight_rows` (gate and up
+    together) of `k` elements each."""
+    given = (ctypes.c_int * len(counts))(*counts)
+    return library.load().mi_expert_tiles_rows(ctypes.addressof(given), len(counts), weight_rows, k, cus)
+
+
 def expert_tiles_for(x: torch.Tensor, pairs: int, experts: int, ff: int) -> str:
     """The form in which `experts_by_expert` makes its products for `pairs` (row, choice) pairs."""
     if pairs >= EXPERT_LDS_TILES_MIN_ROWS * experts and expert_tiles_take(x, ff):
@@ -3247,8 +3254,8 @@ def experts_by_expert(
     a row's results in the order of its choices.  Four launches; an expert that many rows chose is read once
     per sixteen of them, not once per row.  `tiles` (default: by the average number of rows an expert
     gets): "rows" is that form; for prompts (bfloat16) "direct", blocks of 64 features that take 64 of an
-    expert's rows a pass, and "lds", tiles of 128 rows x 128 features with both operands staged through LDS
-    (rows in steps of 64 elements).  `combine=False`
+    expert's rows a pass, and "lds", tiles of 64 to 256 rows x 256 weight rows with both operands staged through LDS
+    (rows in steps of 64 elements; which of them, the device finds out from the list: `expert_tile_rows`).  `combine=False`
     (no shared or identity experts): the rows are left for a norm to add up (`SummedRows`; weights on the
     output: `WeightedRows`).  `leave_rows`: the sum of any experts is left to a norm behind it (`ExpertRows`).
     `lists`: the pairs by expert where `route_top_k` has made them already."""

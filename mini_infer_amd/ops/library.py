@@ -14,7 +14,7 @@ from pathlib import Path
 from mini_infer_amd.exceptions import ExtensionMissingError, KernelShapeError
 from mini_infer_amd.ops import build as _build
 
-ABI_VERSION = 46
+ABI_VERSION = 47
 
 _lib: ctypes.CDLL | None = None
 _lib_path: Path | None = None
@@ -177,6 +177,7 @@ _SIGNATURES: dict[str, list] = {
         c_int, c_int, c_int, _P, _P,
     ],
     "mi_expert_tiles_take": [c_int],
+    "mi_expert_tiles_rows": [_P, c_int, c_int, c_int, c_int],
     "mi_expert_tiles": [c_int, _P, c_int64, c_int, _P, _P, _P, _P, _P, c_int64, c_int, c_int, c_int, c_int, _P],
     "mi_gated_update_norm": [
         c_int, _P, _P, c_int64, c_int, _P, c_int64, _P, _P, _P, _P, _P, c_int, c_int, c_float, c_float, _P, c_int, _P,

@@ -388,6 +388,43 @@ def test_silu_gated_experts_in_tiles_staged_through_lds(rows, width, ff, experts
     assert (got - want).abs().max() < 2e-2 * max(1.0, want.abs().max())
 
 
+@pytest.mark.parametrize("activation", ["silu_gated", "squared_relu"])
+@pytest.mark.parametrize("rows, width, ff, counts, tile_rows", [
+    # (by the rule, for the first product: its 25,600 weight rows are 100 tiles for every row tile, and the rounds of 256 decide)
+    (40, 64, 128, [1, 16, 17, 6], 64), (230, 128, 12800, [97, 128], 128), (320, 192, 12800, [160, 129], 160), (520, 64, 12800, [255, 256], 256),
+    (511, 128, 12800, [255, 256], 256), (520, 320, 12800, [256, 241], 256), (300, 64, 12800, [160, 130], 160),
+    (300, 192, 320, [0, 127, 129, 0, 33], 64), (700, 320, 64, [1, 640, 3], 128), (64, 64, 64, [64], 64)])
+def test_expert_tiles_of_every_size(activation, rows, width, ff, counts, tile_rows):
+    """Tiles of 64, 128, 160 and 256 rows at their edges, one to five steps of 64 of K and more, features beside whole tiles, experts without
+    pairs: against float64.  A product rounds once to bfloat16 (2^-9), the activation's inputs and its output once each; the sums themselves are float32 over at
+    most 12,800 terms of their own size, 2^-12 of the result's; a pair's result is held against the largest."""
+    from mini_infer_amd import ops
+
+    features = 2 * ff if activation == "silu_gated" else ff
+    if activation != "silu_gated":  # (half the weight rows, so twice the experts)
+        rows, counts = 2 * rows, counts + counts
+    assert ops.kernels.expert_tile_rows(counts, features, width) == tile_rows
+    rng = np.random.default_rng(rows + width)
+    experts = len(counts)
+    x = dev(rng.standard_normal((rows, width)), torch.bfloat16)
+    up = dev(rng.standard_normal((experts, features, width)) / np.sqrt(width), torch.bfloat16)
+    down = dev(rng.standard_normal((experts, width, ff)) / np.sqrt(ff), torch.bfloat16)
+    picks = np.full(rows, experts, dtype=np.int32)  # (beyond the pairs: an expert without weights, whose result is the row itself)
+    picks[:sum(counts)] = rng.permutation(np.repeat(np.arange(experts, dtype=np.int32), counts))
+    chosen, w = ints(picks.tolist()).reshape(rows, 1), torch.ones((rows, 1), device=DEV)
+    got = ops.experts_by_expert(x, up, down, chosen, w, tiles="lds", activation=activation).double().cpu()
+    x64, u64, d64 = x.double().cpu(), up.double().cpu(), down.double().cpu()
+    for r in range(rows):
+        e = picks[r]
+        if e == experts:
+            want = x64[r]
+        else:
+            z = u64[e] @ x64[r]
+            act = torch.nn.functional.silu(z[:ff]) * z[ff:] if activation == "silu_gated" else torch.relu(z) ** 2
+            want = d64[e] @ act
+        assert (got[r] - want).abs().max() < 2 ** -6 * max(1.0, want.abs().max()), (r, e)
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("scores", ["logistic", "softmax"])
 @pytest.mark.parametrize("tokens, width, outputs, experts, top, corrected, gated", [

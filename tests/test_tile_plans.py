@@ -57,3 +57,24 @@ def test_gated_products_of_more_than_160_rows_take_no_tiles_above_192_by_128():
             shape = kernels.gated_tiles_for(m, n, k)
             assert shape is None or math.prod(kernels.tile_size(shape)) <= 192 * 128
     assert kernels.gated_tiles_for(193, 14336, 4096) is None and kernels.gated_tiles_for(192, 14336, 4096) is not None
+
+
+@pytest.mark.parametrize("counts, weight_rows, k, rows", [
+    ([4] * 16, 4096, 3072, 64),                    # few pairs an expert: the weights' bytes, and no row tile twice
+    ([100] * 16, 3072, 2048, 128),                 # one row tile an expert, one round of blocks
+    ([150] * 16, 4096, 3072, 160),                 # two of 128 would make two rounds
+    ([250] * 16, 4096, 3072, 256),
+    ([0, 0, 1, 0], 256, 64, 64),
+    ([0, 0], 256, 64, 0),                          # nobody chose any: nothing to do
+    ([10000], 28672, 4096, 256),
+])
+def test_expert_tiles_by_the_rounds_of_blocks_they_take(counts, weight_rows, k, rows):
+    assert kernels.expert_tile_rows(counts, weight_rows, k) == rows
+
+
+def test_expert_tiles_count_the_compute_units():
+    """A quarter of a device takes four rounds where the whole one takes one; tiles of 64 end at 96 pairs an expert on average."""
+    assert kernels.expert_tile_rows([130] * 16, 4096, 3072, 256) == 160
+    assert kernels.expert_tile_rows([96] * 2, 256, 64) == 64 and kernels.expert_tile_rows([97] * 2, 256, 64) == 128
+    for cus in (8, 64, 256):
+        assert kernels.expert_tile_rows([1, 300, 45], 512, 512, cus) in (64, 128, 160, 256)
