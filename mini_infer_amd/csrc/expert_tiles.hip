@@ -31,57 +31,23 @@
 
 namespace {
 
-#define TILE_K 64
-
-// The tiles, by rows, with the microseconds that a step of 64 of K takes one; a launch is expected to take, beside what any launch
-// does, the longer of its rounds of blocks, each its steps and ROUND_MICROS for beginning and end, and the bytes of W, once from memory
-// and again from cache for every row tile.  A fit to 840 launches in these four sizes (8 to 64 experts, 1024 to 7168 wide, 2 to
-// 1,240 pairs an expert, half of them gated; 12 % off): what it picks is 1 % slower than the best of the four.
-struct TileForm {
-  int rows;
-  float step_micros;
-};
-constexpr int FORMS = 4;
-constexpr int FORM_FEATURES = 256;  // weight rows of a tile, in all of them
-__host__ __device__ constexpr TileForm tile_form(int i) {
-  return i == 0 ? TileForm{64, 0.53f} : i == 1 ? TileForm{128, 0.86f} : i == 2 ? TileForm{160, 0.99f} : TileForm{256, 1.40f};
-}
-
-// The tile that a launch takes: row_tiles[f] of form f cover the pairs (0: not to be taken); used: experts with pairs; n, k: an expert's weight rows
-// and their length; cus: compute units, in 8 XCDs to which blocks are dealt in turn.
-__host__ __device__ inline int pick_form(const int (&row_tiles)[FORMS], int used, int n, int k, int cus) {
-  constexpr float ROUND_MICROS = 6.3f, FROM_MEMORY = 1.0e-7f, AGAIN = 0.85e-7f;  // a byte of W
-  const float steps = (float)(k / TILE_K);
-  int best = -1;
-  float least = 0.f;
-  for (int f = 0; f < FORMS; ++f) {
-    if (row_tiles[f] == 0) continue;
-    const int blocks = row_tiles[f] * ((n + FORM_FEATURES - 1) / FORM_FEATURES), rounds = ((blocks + 7) / 8 + cus / 8 - 1) / (cus / 8);
-    const float multiplied = (float)rounds * (steps * tile_form(f).step_micros + ROUND_MICROS);
-    const float brought = FROM_MEMORY * (float)used * (float)n * (float)k * 2.f + AGAIN * (float)blocks * steps * (FORM_FEATURES * TILE_K * 2.f);
-    const float micros = multiplied > brought ? multiplied : brought;
-    if (best < 0 || micros < least * 0.995f) best = f, least = micros;  // (level: the smaller one)
-  }
-  return best;
-}
-
 // The same on the device, from the list.  All threads of the block get the same answer.
 __device__ __forceinline__ int pick_form(const int* __restrict__ first, int experts, bool smallest, int n, int k, int cus) {
-  int row_tiles[FORMS] = {}, used = 0;
+  int row_tiles[TURNS_WIDE] = {}, used = 0;
   for (int e = threadIdx.x % MI_WAVE; e < experts; e += MI_WAVE) {
     const int pairs = first[e + 1] - first[e];
     used += pairs > 0;
 #pragma unroll
-    for (int f = 0; f < FORMS; ++f) row_tiles[f] += (pairs + tile_form(f).rows - 1) / tile_form(f).rows;
+    for (int f = 0; f < TURNS_WIDE; ++f) row_tiles[f] += (pairs + turns_form(f).rows - 1) / turns_form(f).rows;
   }
 #pragma unroll
   for (int off = MI_WAVE / 2; off > 0; off >>= 1) {
     used += __shfl_xor(used, off, MI_WAVE);
 #pragma unroll
-    for (int f = 0; f < FORMS; ++f) row_tiles[f] += __shfl_xor(row_tiles[f], off, MI_WAVE);
+    for (int f = 0; f < TURNS_WIDE; ++f) row_tiles[f] += __shfl_xor(row_tiles[f], off, MI_WAVE);
   }
   if (!smallest) row_tiles[0] = 0;
-  return __builtin_amdgcn_readfirstlane(pick_form(row_tiles, used, n, k, cus));
+  return __builtin_amdgcn_readfirstlane(turns_pick(row_tiles, used, n, k, cus));
 }
 
 // Which tile this block works on: expert, first pair of the row tile (an index into `listed`), feature tile.
@@ -133,8 +99,8 @@ __device__ __forceinline__ void make_tile(
     int64_t expert_stride, const int* __restrict__ listed, const int* __restrict__ first,
     const float* __restrict__ pair_weight, bf16_t* __restrict__ out, int64_t out_stride, int experts, int k_dim, int features) {
   constexpr bool GATED = MODE == 1;
-  constexpr int FEATURES = GATED ? T::BN / 2 : T::BN, HALF = T::NT / 2;
-  static_assert(T::BN == FORM_FEATURES);
+  constexpr int FEATURES = GATED ? T::BN / 2 : T::BN;
+  static_assert(T::BN == TURNS_FEATURES);
   const int feature_tiles = (features + FEATURES - 1) / FEATURES;
   int expert, row0, feature_tile;
   if (!find_tile(first, experts, feature_tiles, T::BM, blockIdx.x, expert, row0, feature_tile)) return;
@@ -142,57 +108,33 @@ __device__ __forceinline__ void make_tile(
   const bf16_t* w = weight + (int64_t)expert * expert_stride;
   T tile;
   tile.run(
-      ring, k_dim / TILE_K,
+      ring, k_dim / TURNS_K,
       [&](int r) {  // (past the expert's last pair: that one again, not written)
         return src + (int64_t)(listed[min(row0 + r, end - 1)] / src_div) * src_stride;
       },
-      [&](int r) {
-        if constexpr (GATED) {  // of a wave's tiles of weight rows the first half are gate rows, the second the up rows of the same features
-          const int t = r / 16 % T::NT, f = min(f0 + (r / (T::NT * 16) * HALF + t % HALF) * 16 + r % 16, features - 1);
-          return w + (int64_t)(t < HALF ? f : f + features) * k_dim;
-        } else {
-          return w + (int64_t)min(f0 + r, features - 1) * k_dim;
-        }
-      });
+      [&](int r) { return w + (int64_t)(GATED ? T::gated_row(r, f0, features) : min(f0 + r, features - 1)) * k_dim; });
+  tile.leave(ring, [&](float sum, int r) {
+    if (MODE != 2) return sum;
+    const float z = fmaxf((pair_weight != nullptr ? pair_weight[listed[min(row0 + r, end - 1)]] : 1.f) * sum, 0.f);
+    return z * z;
+  });
+  constexpr int CHUNKS = FEATURES / 8;
+  const bool whole = (uintptr_t)out % 16 == 0 && out_stride % 8 == 0;
+  for (int i = threadIdx.x; i < T::BM * CHUNKS; i += T::THREADS) {
+    const int row = i / CHUNKS, f = i % CHUNKS * 8;
+    if (row0 + row >= end || f0 + f >= features) continue;
+    const bf16_t* at = ring + row * T::MADE + (GATED ? T::gated_at(f) : f);
+    float v[8];
+    mi_load_8(at, v);
+    if constexpr (GATED) {  // the two products as the element type holds them, then silu(gate) * up
+      float u[8];
+      mi_load_8(at + T::PAIR, u);
 #pragma unroll
-  for (int m = 0; m < T::MT; ++m) {
-    const int r = row0 + tile.row(m);
-    if (r >= end) continue;
-    const int pair = listed[r];
-    bf16_t* o = out + (int64_t)pair * out_stride;
-    const float pw = MODE == 2 && pair_weight != nullptr ? pair_weight[pair] : 1.f;
-#pragma unroll
-    for (int n = 0; n < (GATED ? HALF : T::NT); ++n) {
-      const int f = f0 + (GATED ? (tile.wn * HALF + n) * 16 + tile.quad * 4 : tile.feature(n));
-      float v[4];
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        if constexpr (GATED) {
-          // the two products as the element type holds them, then silu(gate) * up
-          const float g = to_f32(from_f32<bf16_t>(tile.acc[n][m][j])), u = to_f32(from_f32<bf16_t>(tile.acc[n + HALF][m][j]));
-          v[j] = g / (1.f + expf(-g)) * u;
-        } else if constexpr (MODE == 2) {
-          const float z = fmaxf(pw * tile.acc[n][m][j], 0.f);
-          v[j] = z * z;
-        } else {
-          v[j] = tile.acc[n][m][j];
-        }
-      }
-      if (f + 4 <= features && out_stride % 4 == 0) {
-        mi_store_cols<bf16_t, 4>(o + f, v);
-      } else {
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          if (f + j < features) o[f + j] = from_f32<bf16_t>(v[j]);
-      }
+      for (int c = 0; c < 8; ++c) v[c] = silu_times<bf16_t>(v[c], u[c]);
     }
+    mi_store_8(out + (int64_t)listed[row0 + row] * out_stride, f0 + f, features, whole, v);
   }
 }
-
-using Tile64 = TurnsProduct<2, 4, 2, 4, 3>;
-using Tile128 = TurnsProduct<2, 4, 4, 4, 3>;
-using Tile160 = TurnsProduct<2, 4, 5, 4, 3>;
-using Tile256 = TurnsProduct<2, 4, 8, 4, 2>;
 
 template <int MODE>
 __global__ __launch_bounds__(512, 2) void expert_tiles_kernel(
@@ -200,14 +142,13 @@ __global__ __launch_bounds__(512, 2) void expert_tiles_kernel(
     int64_t expert_stride, const int* __restrict__ listed, const int* __restrict__ first,
     const float* __restrict__ pair_weight, bf16_t* __restrict__ out, int64_t out_stride, int experts, int k_dim,
     int features, bool smallest, int cus) {
-  __shared__ __align__(16) bf16_t ring[Tile160::RING];
-  static_assert(Tile160::RING >= Tile64::RING && Tile160::RING >= Tile128::RING && Tile160::RING >= Tile256::RING);
+  __shared__ __align__(16) bf16_t ring[TURNS_RING];
   const int form = pick_form(first, experts, smallest, MODE == 1 ? 2 * features : features, k_dim, cus);
-#define MI_TILE(T) make_tile<T, MODE>(ring, src, src_stride, src_div, weight, expert_stride, listed, first, pair_weight, out, out_stride, experts, k_dim, features)
-  if (form == 0) MI_TILE(Tile64);
-  else if (form == 1) MI_TILE(Tile128);
-  else if (form == 2) MI_TILE(Tile160);
-  else if (form == 3) MI_TILE(Tile256);
+#define MI_TILE(...) make_tile<__VA_ARGS__, MODE>(ring, src, src_stride, src_div, weight, expert_stride, listed, first, pair_weight, out, out_stride, experts, k_dim, features)
+  if (form == 0) MI_TILE(TurnsOf<0>::type);
+  else if (form == 1) MI_TILE(TurnsOf<1>::type);
+  else if (form == 2) MI_TILE(TurnsOf<2>::type);
+  else if (form == 3) MI_TILE(TurnsOf<3>::type);
 #undef MI_TILE
 }
 
@@ -219,9 +160,9 @@ template <int MODE>
 void launch_tiles(const void* src, int64_t src_stride, int src_div, const void* weight, const int* listed, const int* first,
                   const float* pair_weight, void* out, int64_t out_stride, int pairs, int experts, int k_dim, int features, int cus,
                   hipStream_t stream) {
-  const int feature_tiles = ceil_div(features, MODE == 1 ? FORM_FEATURES / 2 : FORM_FEATURES);
+  const int feature_tiles = ceil_div(features, MODE == 1 ? TURNS_FEATURES / 2 : TURNS_FEATURES);
   const bool smallest = pairs <= (int64_t)SMALLEST_UP_TO * experts;
-  const int most = feature_tiles * (pairs / tile_form(smallest ? 0 : 1).rows + min(experts, pairs));  // (an expert's last tile may be a short one)
+  const int most = feature_tiles * (pairs / turns_form(smallest ? 0 : 1).rows + min(experts, pairs));  // (an expert's last tile may be a short one)
   expert_tiles_kernel<MODE><<<ceil_div(most, 8) * 8, 512, 0, stream>>>(
       (const bf16_t*)src, src_stride, src_div, (const bf16_t*)weight, (int64_t)(MODE == 1 ? 2 : 1) * features * k_dim, listed,
       first, pair_weight, (bf16_t*)out, out_stride, experts, k_dim, features, smallest, cus);
@@ -230,19 +171,19 @@ void launch_tiles(const void* src, int64_t src_stride, int src_div, const void* 
 }  // namespace
 
 // Whether rows of k_dim bfloat16 elements are taken.
-extern "C" int mi_expert_tiles_take(int k_dim) { return k_dim > 0 && k_dim % TILE_K == 0; }
+extern "C" int mi_expert_tiles_take(int k_dim) { return k_dim > 0 && k_dim % TURNS_K == 0; }
 
 // Rows of the tile that a launch of n weight rows an expert takes where the experts got counts[0..experts) pairs (0: no pairs).
 extern "C" int mi_expert_tiles_rows(const int* counts, int experts, int n, int k_dim, int cus) {
-  int row_tiles[FORMS] = {}, used = 0;
+  int row_tiles[TURNS_WIDE] = {}, used = 0;
   int64_t pairs = 0;
   for (int e = 0; e < experts; ++e) {
     pairs += counts[e], used += counts[e] > 0;
-    for (int f = 0; f < FORMS; ++f) row_tiles[f] += ceil_div(counts[e], tile_form(f).rows);
+    for (int f = 0; f < TURNS_WIDE; ++f) row_tiles[f] += ceil_div(counts[e], turns_form(f).rows);
   }
   if (pairs > (int64_t)SMALLEST_UP_TO * experts) row_tiles[0] = 0;
-  const int form = pick_form(row_tiles, used, n, k_dim, max(8, cus));
-  return form < 0 ? 0 : tile_form(form).rows;
+  const int form = turns_pick(row_tiles, used, n, k_dim, max(8, cus));
+  return form < 0 ? 0 : turns_form(form).rows;
 }
 
 // Arguments as mi_expert_rows (bfloat16 only), with the number of listed pairs.
@@ -252,7 +193,7 @@ extern "C" int mi_expert_tiles(int mode, const void* src, int64_t src_stride, in
   MI_REQUIRE(pairs >= 0 && experts > 0 && features > 0 && src_div > 0 && src_stride >= k_dim && out_stride >= features,
              "expert_tiles: bad sizes pairs=%d experts=%d k=%d features=%d", pairs, experts, k_dim, features);
   MI_REQUIRE(mi_expert_tiles_take(k_dim) && src_stride % 8 == 0 && ((uintptr_t)src | (uintptr_t)weight) % 16 == 0 && (uintptr_t)out % 8 == 0,
-             "expert_tiles: rows of %d elements are not taken %d at a time", k_dim, TILE_K);
+             "expert_tiles: rows of %d elements are not taken %d at a time", k_dim, TURNS_K);
   MI_REQUIRE(mode >= 0 && mode <= 2, "expert_tiles: mode %d", mode);
   MI_REQUIRE((int64_t)ceil_div(features, 128) * ((int64_t)pairs / 64 + experts) < (1 << 30), "expert_tiles: too many tiles");
   if (pairs == 0) return MI_OK;

@@ -225,7 +225,120 @@ struct TurnsProduct {
     static constexpr int value = N;
   };
 
-  // Where the sums lie in the tile: acc[n][m][j] is row `row(m)`, row of W `feature(n) + j`.
-  __device__ __forceinline__ int row(int m) const { return (wm * MT + m) * 16 + col; }
-  __device__ __forceinline__ int feature(int n) const { return (wn * NT + n) * 16 + quad * 4; }
+  // The sums, each as value_of(sum, row of the tile) rounded to bfloat16, as rows of the tile in `ring`, MADE elements apart; all threads see them
+  // afterwards.  What follows reads them in a loop: written from registers, the last steps of 32 little tiles are 60 KB of instructions, which
+  // every launch fetches anew (2048 x 6144 x 4096 86 us alone, 101 in a kernel with four sizes of tiles).
+  static constexpr int MADE = BN + 8;
+  static_assert(BM * MADE <= 79872, "the tile fits the largest ring");
+  template <typename F>
+  __device__ __forceinline__ void leave(bf16_t* ring, F value_of) {
+    meet();  // (the group that is ahead does not write what the other still reads)
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+      const int r = (wm * MT + m) * 16 + col;
+#pragma unroll
+      for (int n = 0; n < NT; ++n) {
+        float v[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] = value_of(acc[n][m][j], r);
+        mi_store_cols<bf16_t, 4>(ring + r * MADE + (wn * NT + n) * 16 + quad * 4, v);
+      }
+    }
+    __syncthreads();
+  }
+  // Products of gate and up rows: of a wave's tiles of W the first half are gate rows, the second the up rows of the same features.  Which
+  // row of [gate; up] of `features` features each the tile's row r of W is, features from f0 on; and where the tile's feature f lies in
+  // what `leave` left, its up product PAIR further on.
+  static constexpr int PAIR = NT / 2 * 16;
+  static __device__ __forceinline__ int gated_row(int r, int f0, int features) {
+    const int t = r % (2 * PAIR), f = min(f0 + r / (2 * PAIR) * PAIR + t % PAIR, features - 1);
+    return t < PAIR ? f : f + features;
+  }
+  static __device__ __forceinline__ int gated_at(int f) { return f / PAIR * (2 * PAIR) + f % PAIR; }
 };
+
+// Eight bfloat16 values of LDS as floats, and eight floats as bfloat16 values of a row from column f on that has n of them (whole: 16 bytes at once).
+__device__ __forceinline__ void mi_load_8(const bf16_t* p, float (&v)[8]) {
+  const bf16x8_t got = *reinterpret_cast<const bf16x8_t*>(p);
+#pragma unroll
+  for (int i = 0; i < 8; ++i) v[i] = to_f32((bf16_t)got[i]);
+}
+__device__ __forceinline__ void mi_store_8(bf16_t* row, int f, int n, bool whole, const float (&v)[8]) {
+  if (whole && f + 8 <= n) {
+    bf16x8_t out;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) out[i] = from_f32<bf16_t>(v[i]);
+    *reinterpret_cast<bf16x8_t*>(row + f) = out;
+  } else {
+    for (int i = 0; i < 8 && f + i < n; ++i) row[f + i] = from_f32<bf16_t>(v[i]);
+  }
+}
+
+// The tiles that launches choose among, rows of A x rows of W, and the microseconds that a step of 64 of K takes one.
+// X(number, rows, rows of W, gate and up rows side by side?, microseconds a step, shape)
+#define TURNS_FORMS_OF(X) \
+  X(0, 64, 256, true, 0.556f, 2, 4, 2, 4, 3) \
+  X(1, 128, 256, true, 0.814f, 2, 4, 4, 4, 3) \
+  X(2, 160, 256, true, 0.943f, 2, 4, 5, 4, 3) \
+  X(3, 256, 256, true, 1.286f, 2, 4, 8, 4, 2) \
+  X(4, 64, 128, true, 0.345f, 2, 4, 2, 2, 4) \
+  X(5, 128, 128, true, 0.486f, 4, 2, 2, 4, 4) \
+  X(6, 160, 128, true, 0.603f, 2, 4, 5, 2, 4) \
+  X(7, 192, 128, true, 0.674f, 2, 4, 6, 2, 3) \
+  X(8, 256, 128, true, 0.786f, 4, 2, 4, 4, 3) \
+  X(9, 128, 192, false, 0.668f, 2, 4, 4, 3, 3) \
+  X(10, 192, 192, false, 0.847f, 2, 4, 6, 3, 3)
+constexpr int TURNS_K = 64;
+constexpr int TURNS_FORMS = 11;
+template <int F>
+struct TurnsOf;
+#define X(I, ROWS, FEATURES, GATED, MICROS, ...)                                                                 \
+  template <>                                                                                                    \
+  struct TurnsOf<I> {                                                                                            \
+    using type = TurnsProduct<__VA_ARGS__>;                                                                      \
+    static_assert(type::BM == ROWS && type::BN == FEATURES && type::RING <= 79872 && (!GATED || type::NT % 2 == 0)); \
+  };
+TURNS_FORMS_OF(X)
+#undef X
+constexpr int TURNS_RING = TurnsOf<2>::type::RING;  // the largest
+struct TurnsForm {
+  int rows, features;
+  bool gated;
+  float step_micros;
+};
+__host__ __device__ constexpr TurnsForm turns_form(int i) {
+  constexpr TurnsForm forms[TURNS_FORMS] = {
+#define X(I, ROWS, FEATURES, GATED, MICROS, ...) {ROWS, FEATURES, GATED, MICROS},
+      TURNS_FORMS_OF(X)
+#undef X
+  };
+  return forms[i];
+}
+
+// Microseconds of the rounds that `tiles` tiles of form f take on `each` compute units (of one XCD): the last one, where it does not fill them, is a
+// little shorter, because the card's power then lets the clock rise.  And of the bytes of `matrices` matrices of n rows of k elements that
+// `blocks` tiles read.
+__host__ __device__ inline float turns_rounds_micros(int f, int tiles, int each, int k) {
+  if (tiles == 0) return 0.f;
+  const int rounds = (tiles + each - 1) / each, idle = rounds * each - tiles;
+  return ((float)rounds - 0.29f * (float)idle / (float)each) * ((float)(k / TURNS_K) * turns_form(f).step_micros + 3.4f);
+}
+__host__ __device__ inline float turns_bytes_micros(int f, int matrices, int64_t blocks, int n, int k) {
+  return 2.33e-7f * (float)matrices * (float)n * (float)k * 2.f + 0.73e-7f * (float)blocks * (float)k * ((float)turns_form(f).features * 2.f);
+}
+
+// Of the first four forms (256 rows of W) the one that a launch takes, or -1: row_tiles[f] of form f cover the rows of A (0: not to be taken); matrices:
+// the matrices W, n rows of k elements each, that any of them reads; cus: compute units, in 8 XCDs to which blocks are dealt in turn.
+constexpr int TURNS_WIDE = 4, TURNS_FEATURES = 256;
+__host__ __device__ inline int turns_pick(const int (&row_tiles)[TURNS_WIDE], int matrices, int n, int k, int cus) {
+  int best = -1;
+  float least = 0.f;
+  for (int f = 0; f < TURNS_WIDE; ++f) {
+    if (row_tiles[f] == 0) continue;
+    const int blocks = row_tiles[f] * ((n + TURNS_FEATURES - 1) / TURNS_FEATURES);
+    const float multiplied = turns_rounds_micros(f, (blocks + 7) / 8, cus / 8, k), brought = turns_bytes_micros(f, matrices, blocks, n, k);
+    const float micros = multiplied > brought ? multiplied : brought;
+    if (best < 0 || micros < least * 0.995f) best = f, least = micros;  // (level: the smaller one)
+  }
+  return best;
+}

@@ -639,15 +639,70 @@ def gated_tiles_for(m: int, n: int, k: int, cus: int = WHOLE_DEVICE_CUS) -> int 
     return shape
 
 
+TURNS_MIN_ROWS = 321
+TURNS_NONE, TURNS_SILU, TURNS_CLAMPED, TURNS_GELU = range(4)
+TURNS_OUTPUTS_A_K = 400
+
+
+def _turns_take(x: torch.Tensor, weight: torch.Tensor) -> bool:
+    """Whether the product of these is made in the tiles of `gemm_turns_bf16`."""
+    return x.dim() == 2 and x.shape[0] >= TURNS_MIN_ROWS and turns_pay(x.shape[0], weight.shape[0], x.shape[1]) and _rows_of_bf16(x, weight)
+
+
+def turns_pay(m: int, n: int, k: int) -> bool:
+    """Whether a bfloat16 product of so many rows (n: gate and up together where it is gated, which is then one launch with its activation) is made in
+    the tiles of `gemm_turns_bf16`; otherwise `tiles_for`, `gated_tiles_for` or the vendor library.  Their sums have the same order, bit for bit, in all but a few of the library's kernels.  Microseconds of the library (or tiles, up to 1,024
+    rows) / these, weights from memory, over 12 matrices of 2048 x 2048 to 16384 x 2048 and 4096 x 14336:
+
+        rows                400            640            1024           1501           2048           4096
+        4096 x 14336        67 / 87        81 / 124       129 / 125      163 / 160      203 / 185      306 / 305
+        6144 x 4096         32 / 32        40 / 38        53 / 51        72 / 60        79 / 79        157 / 148
+        3072 x 8192         42 / 48        51 / 51        63 / 64        84 / 75        94 / 91        150 / 145
+        2048 x 8192         32 / 47        44 / 50        52 / 52        56 / 62        69 / 68        110 / 107
+        3072 x 3072         25 / 19        25 / 19        25 / 23        34 / 30        36 / 33        62 / 57
+        16384 x 2048        34 / 31        39 / 37        53 / 52        85 / 84        100 / 103      193 / 205
+
+    as a geometric mean over those matrices 1.08 up to 1,024 rows, 1.07 to 2,048, 1.05 beyond.  What they lose on is a long K with
+    few outputs: a block walks all of K, the library's smaller tiles and cut ranges finish earlier.  Left to those: fewer outputs than
+    `TURNS_OUTPUTS_A_K` for each element of K.  What is taken is at worst 0.94 as fast at these sizes (4096 x 4096 at 768 rows 33.2 / 35.5), and
+    of small matrices 1024 x 3072 at 2,048 rows 21.2 / 23.5, 512 x 512 at 500 rows 5.7 / 6.4, 1024 x 1024 at 1,100 11.1 / 9.8.
+
+    Gated, with the launch of the activation on the other side, gate|up 28672 x 4096 at 400 / 1,024 / 1,777 / 2,048 / 4,096 rows 106 / 203 / 432 / 373 / 693
+    against 97 / 184 / 327 / 346 / 658, 16384 x 3072 60 / 94 / 166 / 173 / 330 against 48 / 79 / 144 / 152 / 300, 7168 x 4096 36 / 61 / 92 / 94 /
+    184 against 34 / 57 / 84 / 90 / 178: 1.12 up to 1,024 rows, 1.16 to 2,048, 1.14 beyond, and never slower from 321 rows on."""
+    return m >= TURNS_MIN_ROWS and k % 64 == 0 and m * n >= TURNS_OUTPUTS_A_K * k
+
+
+def turns_plan(m: int, n: int, k: int, gated: bool = False, cus: int = WHOLE_DEVICE_CUS) -> tuple[list[int], float]:
+    """([rows and rows of W of the tiles, rows of those that the rest is cut into, tiles of an XCD that stay whole, all of its tiles],
+    microseconds expected) of a product of n features in the tiles of `gemm_turns_bf16`."""
+    plan, micros = (ctypes.c_int * 5)(), ctypes.c_float()
+    library.check(library.load().mi_gemm_turns_plan(m, n, k, int(gated), cus, ctypes.addressof(plan), ctypes.addressof(micros)))
+    return list(plan), micros.value
+
+
+def _turns(act: int, x: torch.Tensor, weight: torch.Tensor, n: int, bias: torch.Tensor | None = None, limit: float = 0.0, slope: float = 0.0,
+           only: int = -1, out: torch.Tensor | None = None) -> torch.Tensor:
+    """One launch of `gemm_turns_bf16`, into `out` (rows may be strided) if given; `only`: all tiles of that form."""
+    _need_cuda(x, weight, bias)
+    if out is None:
+        out = torch.empty((x.shape[0], n), dtype=torch.bfloat16, device=x.device)
+    library.check(
+        library.load().mi_gemm_turns_bf16(act, _ptr(x), x.stride(0), _ptr(weight), weight.stride(0), _ptr(bias), limit, slope, _ptr(out),
+                                          out.stride(0), x.shape[0], n, x.shape[1], only, _stream())
+    )
+    return out
+
+
 def linear(x: torch.Tensor, weight: torch.Tensor, partial_ok: bool = False, steady: bool = False) -> torch.Tensor | PartialSums:
     """`x @ weight.T` without bias.
 
     float32 runs the hand-written true-float32 kernel.  bfloat16 with at most 16 rows (decode) runs the hand-written
     weight-streaming kernel, some tens to some hundreds of rows the tiles of `gemm_tiles_bf16` where they are faster
-    (`tiles_for`); the rest goes to the vendor GEMM library through torch, as the reference's engine does
-    (distributed/linear.py:167, `F.linear` -> the vendor BLAS).
-    With `partial_ok` the result may come as `PartialSums` where that pays.  `steady` (`Part.steady`): without those tiles, so that the
-    sums keep the order that they have in the library.
+    (`tiles_for`), more rows mostly the tiles of `gemm_turns_bf16` (`turns_pay`); the rest goes to the vendor GEMM library through torch, as the
+    reference's engine does (distributed/linear.py:167, `F.linear` -> the vendor BLAS).
+    With `partial_ok` the result may come as `PartialSums` where that pays.  `steady` (`Part.steady`): without the tiles of
+    `gemm_tiles_bf16`, so that the sums keep the order that they have in the library and in `gemm_turns_bf16`.
     """
     if x.dtype == torch.float32:
         return gemm_f32(x, weight)
@@ -662,6 +717,8 @@ def linear(x: torch.Tensor, weight: torch.Tensor, partial_ok: bool = False, stea
         and skinny_gemm_takes(x.shape[0], x.shape[1], x.stride(0), weight.stride(0))
     ):
         return gemm_skinny_bf16(x, weight)
+    if _turns_take(x, weight):
+        return _turns(TURNS_NONE, x, weight, weight.shape[0])
     if not steady and x.dim() == 2 and x.shape[0] <= TILES_MAX_ROWS and _rows_of_bf16(x, weight):
         m, n = x.shape[0], weight.shape[0]
         plan = tiles_for(m, n, x.shape[1], partial_ok, _compute_units(x.device))
@@ -821,6 +878,8 @@ def linear_swiglu(x: "torch.Tensor | ScaledRows", gate_up_weight: torch.Tensor, 
             scaled, x = x, values
         else:
             x = x.finish()
+    if scaled is None and _turns_take(x, gate_up_weight):
+        return _turns(TURNS_SILU, x, gate_up_weight, rows // 2)
     if not steady and scaled is None and x.dim() == 2 and SKINNY_WIDE_MAX_ROWS < x.shape[0] <= TILES_MAX_ROWS and _rows_of_bf16(x, gate_up_weight):
         _need_cuda(x, gate_up_weight)
         m, n = x.shape[0], rows // 2
@@ -1988,6 +2047,10 @@ def linear_clamped_glu(x: torch.Tensor, gate_up_weight: torch.Tensor, bias: torc
             )
         )
         return out
+    if _turns_take(x, gate_up_weight) and limit > 0:
+        _need_contiguous("bias", bias)
+        _need_f32("bias", bias)
+        return _turns(TURNS_CLAMPED, x, gate_up_weight, rows // 2, bias, float(limit), float(slope))
     return clamped_glu(linear(x, gate_up_weight, steady=steady), bias, limit, slope)
 
 
@@ -2135,6 +2198,8 @@ def linear_geglu(x: torch.Tensor, gate_up_weight: torch.Tensor, steady: bool = F
             )
         )
         return out
+    if _turns_take(x, gate_up_weight):
+        return _turns(TURNS_GELU, x, gate_up_weight, rows // 2)
     both = linear(x, gate_up_weight, steady=steady)
     return gated_mul(both[:, : rows // 2], both[:, rows // 2 :], "gelu_tanh")
 

@@ -14,7 +14,7 @@ from pathlib import Path
 from mini_infer_amd.exceptions import ExtensionMissingError, KernelShapeError
 from mini_infer_amd.ops import build as _build
 
-ABI_VERSION = 47
+ABI_VERSION = 48
 
 _lib: ctypes.CDLL | None = None
 _lib_path: Path | None = None
@@ -177,6 +177,13 @@ _SIGNATURES: dict[str, list] = {
         c_int, c_int, c_int, _P, _P,
     ],
     "mi_expert_tiles_take": [c_int],
+    "mi_gemm_turns_plan": [c_int, c_int, c_int, c_int, c_int, _P, _P],
+    "mi_gemm_turns_rows": [c_int],
+    "mi_gemm_turns_features": [c_int],
+    "mi_gemm_turns_gated": [c_int],
+    "mi_gemm_turns_bf16": [
+        c_int, _P, c_int64, _P, c_int64, _P, c_float, c_float, _P, c_int64, c_int, c_int, c_int, c_int, _P,
+    ],
     "mi_expert_tiles_rows": [_P, c_int, c_int, c_int, c_int],
     "mi_expert_tiles": [c_int, _P, c_int64, c_int, _P, _P, _P, _P, _P, c_int64, c_int, c_int, c_int, c_int, _P],
     "mi_gated_update_norm": [

@@ -280,6 +280,91 @@ def test_products_in_tiles(shape):
                 assert ((gated.double() - wanted).abs() <= 2.0 ** -8 * wanted.abs() + 1e-30).all(), (m, n, k)
 
 
+def test_every_form_of_the_tiles_that_take_turns_is_tested():
+    from mini_infer_amd.ops import library
+
+    lib = library.load()
+    assert lib.mi_gemm_turns_rows(10) > 0 and lib.mi_gemm_turns_rows(11) == 0
+
+
+@pytest.mark.parametrize("form", range(-1, 11))
+def test_products_in_tiles_that_take_turns(form):
+    """Every form (-1: the plan's) at the edges of its tiles, plain and with each activation; K of one step, of fewer steps than the ring has stages and of
+    more; rows of a wider buffer, whose values beside and behind the result stay, on boundaries of eight values and off them; more row tiles
+    than stand side by side; a row of infinities stays alone."""
+    from mini_infer_amd import ops
+    from mini_infer_amd.exceptions import KernelShapeError
+    from mini_infer_amd.ops import kernels, library
+
+    lib = library.load()
+    bm, bn = (lib.mi_gemm_turns_rows(form), lib.mi_gemm_turns_features(form)) if form >= 0 else (256, 256)
+    half = bn // 2
+    cases = [(bm, half, 64), (bm + 1, half + 1, 128), (bm - 1, half - 3, 192), (2 * bm + 5, bn + 4, 320), (1, 5, 64), (9 * bm + 3, 70, 64 * 9)]
+    if form < 0:
+        cases += [(512, 16896, 64), (1000, 14400, 64)]  # (both cut the tiles of the last round)
+        assert any(kernels.turns_plan(m, 2 * n, k)[0][0] != kernels.turns_plan(m, 2 * n, k)[0][2] for m, n, k in cases)
+
+    def made(act, a, w, n, spare=0, bias=None):
+        m = a.shape[0]
+        wide = torch.full((m + 1, n + spare), 7.0, dtype=torch.bfloat16, device=DEV)
+        kernels._turns(act, a, w, n, bias, 3.0, 1.702, form, wide[:m, :n])
+        assert (wide[:m, n:] == 7).all() and (wide[m:] == 7).all(), (act, a.shape, n, spare)
+        return wide[:m, :n]
+
+    for m, n, k in cases:
+        a = _rand(m, k + 8, dtype=torch.bfloat16, seed=43)[:, :k]
+        w = _rand(2 * n, k, dtype=torch.bfloat16, seed=44, scale=0.05)
+        if m > 2:
+            a[m - 1] = float("inf")
+        finite = slice(0, m - 1 if m > 2 else m)
+        exact = (a.double() @ w.double().T)[finite]
+        # (float32 sums of k products, then one rounding to 8 bits)
+        bound = 2.0 ** -23 * k * (a.double().abs() @ w.double().abs().T)[finite] + 2.0 ** -8 * exact.abs() + 1e-30
+        out = made(kernels.TURNS_NONE, a, w, 2 * n)[finite]
+        assert ((out.double() - exact).abs() <= bound).all(), (m, n, k)
+        for spare in (3, -2 * n % 8 + 8):
+            assert torch.equal(made(kernels.TURNS_NONE, a, w, 2 * n, spare)[finite], out)
+        if form >= 0 and not lib.mi_gemm_turns_gated(form):
+            with pytest.raises(KernelShapeError):
+                made(kernels.TURNS_SILU, a, w, n)
+            continue
+        # the activation is that of the launch that would follow the product
+        bias = _rand(2 * n, seed=45)
+        for spare in (0, 3, -n % 8 + 8):
+            assert torch.equal(made(kernels.TURNS_SILU, a, w, n, spare)[finite], ops.silu_mul(out))
+            assert torch.equal(made(kernels.TURNS_GELU, a, w, n, spare)[finite], ops.gated_mul(out[:, :n], out[:, n:], "gelu_tanh"))
+            assert torch.equal(made(kernels.TURNS_CLAMPED, a, w, n, spare, bias)[finite], ops.clamped_glu(out, bias, 3.0, 1.702))
+            assert torch.equal(made(kernels.TURNS_CLAMPED, a, w, n, spare)[finite], ops.clamped_glu(out, None, 3.0, 1.702))
+
+
+@pytest.mark.parametrize("m, n, k", [(401, 2304, 2048), (640, 1000, 512), (2048, 1500, 1024)])
+def test_products_of_many_rows_go_through_the_tiles_that_take_turns(m, n, k, monkeypatch):
+    """Plain and gated, from the public entry points; K that is not whole 64s, rows off 16 bytes and few rows do not."""
+    from mini_infer_amd import ops
+    from mini_infer_amd.ops import kernels
+
+    taken = []
+    own = kernels._turns
+    monkeypatch.setattr(kernels, "_turns", lambda act, *rest, **more: (taken.append(act), own(act, *rest, **more))[1])
+    a, w = _rand(m, k + 40, dtype=torch.bfloat16, seed=46), _rand(2 * n, k + 40, dtype=torch.bfloat16, seed=47, scale=0.05)
+    exact = a[:, :k].double() @ w[:, :k].double().T
+    for steady in (False, True):
+        got = ops.linear(a[:, :k], w[:, :k], steady=steady)
+        assert (got.double() - exact).abs().max() < 2.0 ** -7 * exact.abs().max()
+    assert taken == [kernels.TURNS_NONE] * 2
+    g, u = exact[:, :n].float().bfloat16().double(), exact[:, n:].float().bfloat16().double()
+    for got, want in ((ops.linear_swiglu(a[:, :k], w[:, :k]), torch.nn.functional.silu(g) * u),
+                      (ops.linear_geglu(a[:, :k], w[:, :k]), torch.nn.functional.gelu(g, approximate="tanh") * u),
+                      (ops.linear_clamped_glu(a[:, :k], w[:, :k], None, 2.0, 1.702), g.clamp(max=2.0) * torch.sigmoid(1.702 * g.clamp(max=2.0)) * (u.clamp(-2.0, 2.0) + 1))):
+        assert (got.double() - want).abs().max() < 2.0 ** -6 * want.abs().max()
+    assert taken[2:] == [kernels.TURNS_SILU, kernels.TURNS_GELU, kernels.TURNS_CLAMPED]
+    del taken[:]
+    ops.linear(a[:, :k - 32], w[:, :k - 32])
+    ops.linear(a[:, 1:k + 1], w[:, 1:k + 1])
+    ops.linear(a[:320, :k], w[:, :k])
+    assert taken == []
+
+
 @pytest.mark.parametrize("m,n,k", [(17, 3072, 3072), (33, 2048, 8192), (271, 3072, 8192), (100, 8192, 2048), (24, 1000, 8224), (400, 2048, 8192)])
 def test_linear_of_some_tens_to_some_hundreds_of_rows(m, n, k):
     """`linear` through tiles, with and without a consumer for the pieces; operands that the tiles do not take (rows off 16 bytes) go on

@@ -78,3 +78,46 @@ def test_expert_tiles_count_the_compute_units():
     assert kernels.expert_tile_rows([96] * 2, 256, 64) == 64 and kernels.expert_tile_rows([97] * 2, 256, 64) == 128
     for cus in (8, 64, 256):
         assert kernels.expert_tile_rows([1, 300, 45], 512, 512, cus) in (64, 128, 160, 256)
+
+
+@pytest.mark.parametrize("gated", [False, True])
+@pytest.mark.parametrize("m, n, k", [(2048, 14336, 4096), (1777, 14336, 4096), (2048, 28672, 4096), (321, 64, 64), (4096, 4096, 14336), (700, 5000, 192),
+                                     (3000, 12288, 3072), (1, 1, 64), (100000, 128, 64)])
+def test_tiles_that_take_turns_cover_a_product_once(m, n, k, gated):
+    """What the launch works out block by block, over its plan: every row tile of every feature tile, whole or in as many parts as it is cut into."""
+    (rows, features, rest, whole, places), micros = kernels.turns_plan(m, n, k, gated)
+    row_tiles, feature_tiles = -(-m // rows), -(-n // (features // 2 if gated else features))
+    cut = rows // rest
+    assert rows % rest == 0 and micros > 0 and places == -(-row_tiles * feature_tiles // 8) and whole % 32 == 0 and places - whole < 32
+    seen = {}
+    for block in range(8 * (whole + (places - whole) * cut)):
+        xcd, at = block % 8, block // 8
+        part = at >= whole
+        place = xcd * places + (whole + (at - whole) // cut if part else at)
+        if place >= min((xcd + 1) * places, row_tiles * feature_tiles):
+            continue
+        band = place // (8 * feature_tiles)
+        in_band = min(8, row_tiles - band * 8)
+        left = place - band * 8 * feature_tiles
+        r0 = (band * 8 + left % in_band) * rows + ((at - whole) % cut * rest if part else 0)
+        seen.setdefault((r0, left // in_band), []).append(rest if part else rows)
+    made = {}
+    for (r0, tile), sizes in seen.items():
+        assert len(sizes) == 1 and 0 <= tile < feature_tiles
+        for r in range(r0, r0 + sizes[0], 64 if sizes[0] % 64 == 0 else 32):
+            assert (r, tile) not in made
+            made[(r, tile)] = True
+    step = 64 if rows % 64 == 0 and rest % 64 == 0 else 32
+    assert len(made) == row_tiles * rows // step * feature_tiles
+
+
+def test_the_rest_of_a_product_is_cut_where_whole_tiles_leave_units_idle():
+    assert kernels.turns_plan(2048, 14336, 4096, gated=True)[0] == [256, 256, 128, 96, 112]
+    assert kernels.turns_plan(1777, 14336, 4096, gated=True)[0] == [256, 256, 64, 96, 98]
+    assert kernels.turns_plan(4096, 14336, 4096, gated=True)[0][2:] == [256, 224, 224]
+
+
+@pytest.mark.parametrize("m, n, k, taken", [(321, 3072, 3072, False), (401, 3072, 3072, True), (320, 28672, 4096, False), (640, 4096, 14336, False),
+                                            (2048, 4096, 14336, True), (1501, 2048, 8192, False), (2048, 2048, 8192, True), (512, 4096, 4128, False)])
+def test_products_that_go_to_the_tiles_that_take_turns(m, n, k, taken):
+    assert kernels.turns_pay(m, n, k) == taken
