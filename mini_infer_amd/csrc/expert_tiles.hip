@@ -112,7 +112,7 @@ __device__ __forceinline__ void make_tile(
       [&](int r) {  // (past the expert's last pair: that one again, not written)
         return src + (int64_t)(listed[min(row0 + r, end - 1)] / src_div) * src_stride;
       },
-      [&](int r) { return w + (int64_t)(GATED ? T::gated_row(r, f0, features) : min(f0 + r, features - 1)) * k_dim; });
+      [&](int r) { return w + (int64_t)(GATED ? T::Pairs::row_of(r, f0, features) : min(f0 + r, features - 1)) * k_dim; });
   tile.leave(ring, [&](float sum, int r) {
     if (MODE != 2) return sum;
     const float z = fmaxf((pair_weight != nullptr ? pair_weight[listed[min(row0 + r, end - 1)]] : 1.f) * sum, 0.f);
@@ -123,12 +123,12 @@ __device__ __forceinline__ void make_tile(
   for (int i = threadIdx.x; i < T::BM * CHUNKS; i += T::THREADS) {
     const int row = i / CHUNKS, f = i % CHUNKS * 8;
     if (row0 + row >= end || f0 + f >= features) continue;
-    const bf16_t* at = ring + row * T::MADE + (GATED ? T::gated_at(f) : f);
+    const bf16_t* at = ring + row * T::MADE + (GATED ? T::Pairs::at(f) : f);
     float v[8];
     mi_load_8(at, v);
     if constexpr (GATED) {  // the two products as the element type holds them, then silu(gate) * up
       float u[8];
-      mi_load_8(at + T::PAIR, u);
+      mi_load_8(at + T::Pairs::PAIR, u);
 #pragma unroll
       for (int c = 0; c < 8; ++c) v[c] = silu_times<bf16_t>(v[c], u[c]);
     }

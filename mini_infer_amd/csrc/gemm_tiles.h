@@ -1,6 +1,7 @@
 // The kernel of gemm_tiles_bf16.hip and gemm_tiles_gated_bf16.hip, and the shapes that they compile it for.
 #pragma once
 
+#include "gated_tile.h"
 #include "tile_product.h"
 
 // Of the 20 shapes measured those that are the best anywhere by more than 1 %.
@@ -34,7 +35,7 @@ __host__ __device__ __forceinline__ KRange k_range(int k, int steps_each, int ra
 template <class T, bool GATED, bool ONCE, bool ODD>
 __global__ __launch_bounds__(T::THREADS, T::RING * 4 <= 163840 ? 2 : 1) void gemm_tiles_kernel(
     const bf16_t* __restrict__ a, int64_t lda, const bf16_t* __restrict__ w, int64_t ldw, void* __restrict__ out, int64_t ldc,
-    int kind, float scale, bool vec, int m, int n, int k, int steps_each, int row_tiles, int feature_tiles, int total) {
+    int kind, float scale, const GatedActivation how, bool vec, int m, int n, int k, int steps_each, int row_tiles, int feature_tiles, int total) {
   __shared__ __align__(16) bf16_t ring[T::RING];
   // Consecutive places go to one XCD (workgroups are dealt to the 8 of them in turn): the row tiles that read the same
   // rows of W run at the same time behind one L2.
@@ -51,35 +52,29 @@ __global__ __launch_bounds__(T::THREADS, T::RING * 4 <= 163840 ? 2 : 1) void gem
   tile.template run<ONCE, ODD>(
       ring, part.halves, [&](int r) { return a + (int64_t)min(r0 + r, m - 1) * lda; },
       [&](int r) {
-        if constexpr (GATED) {  // of a wave's tiles of W the first half are gate rows, the second the up rows of the same features
-          constexpr int HALF = T::NT / 2;
-          const int t = r / 16 % T::NT;
-          const int f = min(f0 + (r / (T::NT * 16) * HALF + t % HALF) * 16 + r % 16, n - 1);
-          return w + (int64_t)(t < HALF ? f : f + n) * ldw;
-        } else {
-          return w + (int64_t)min(f0 + r, n - 1) * ldw;
-        }
+        return w + (int64_t)(GATED ? GatedTile<T::NT>::row_of(r, f0, n) : min(f0 + r, n - 1)) * ldw;
       });
+  if constexpr (GATED) {
+    tile.leave(ring);
+#define MI_WRITE(ACT) write_activated<ACT, GatedTile<T::NT>, T::BM, T::BN, T::MADE, T::THREADS>(ring, how, (bf16_t*)out, ldc, vec, r0, m, f0, n)
+    if (kind == 4) MI_WRITE(ACT_CLAMPED);
+    else if (kind == 5) MI_WRITE(ACT_GELU);
+    else MI_WRITE(ACT_SILU);
+#undef MI_WRITE
+    return;
+  }
 #pragma unroll
   for (int i = 0; i < T::MT; ++i) {
     const int row = r0 + tile.row(i);
     if (!tile.mine(i) || row >= m) continue;
 #pragma unroll
-    for (int j = 0; j < (GATED ? T::NT / 2 : T::NT); ++j) {
-      const int f = f0 + (GATED ? (tile.wn * (T::NT / 2) + j) * 16 + tile.quad * 4 : tile.feature(j));
+    for (int j = 0; j < T::NT; ++j) {
+      const int f = f0 + tile.feature(j);
       float v[4];
 #pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        v[c] = tile.acc[j][i][c];
-        if constexpr (GATED) {
-          const float g = to_f32(from_f32<bf16_t>(v[c])), u = to_f32(from_f32<bf16_t>(tile.acc[j + T::NT / 2][i][c]));
-          v[c] = g / (1.f + expf(-g)) * u;
-        } else if (kind == 2) {
-          v[c] = to_f32(from_f32<bf16_t>(v[c])) * scale;
-        }
-      }
+      for (int c = 0; c < 4; ++c) v[c] = kind == 2 ? to_f32(from_f32<bf16_t>(tile.acc[j][i][c])) * scale : tile.acc[j][i][c];
       const bool whole = vec && f + 4 <= n;
-      if (!GATED && kind != 0) {
+      if (kind != 0) {
         float* o = kind == 1 ? (float*)out + ((int64_t)range * m + row) * n + f : (float*)out + (int64_t)row * ldc + f;
         if (whole) {
           mi_store_cols<float, 4>(o, v);
@@ -108,6 +103,7 @@ struct GemmTilesLaunch {
   int64_t lda, ldw, ldc;
   int kind;
   float scale;
+  GatedActivation how;
   bool vec;
   int m, n, k, steps_each;
   hipStream_t stream;
@@ -119,7 +115,7 @@ static void gemm_tiles_launch(const GemmTilesLaunch& l) {
   const int total = row_tiles * feature_tiles * ceil_div(ceil_div(l.k, 64), l.steps_each);
   const auto kernel = row_tiles == 1 ? gemm_tiles_kernel<T, GATED, true, ODD> : gemm_tiles_kernel<T, GATED, false, ODD>;
   kernel<<<ceil_div(total, 8) * 8, T::THREADS, 0, l.stream>>>((const bf16_t*)l.a, l.lda, (const bf16_t*)l.w, l.ldw, l.out, l.ldc, l.kind,
-                                                             l.scale, l.vec, l.m, l.n, l.k, l.steps_each, row_tiles, feature_tiles, total);
+                                                             l.scale, l.how, l.vec, l.m, l.n, l.k, l.steps_each, row_tiles, feature_tiles, total);
 }
 
 // gemm_tiles_gated_bf16.hip

@@ -14,16 +14,7 @@
 // (models/blocks/silu_mul_kernel.py:86-90).
 #include "turns_product.h"
 
-#include <math.h>
-
 namespace {
-
-enum { ACT_NONE = 0, ACT_SILU = 1, ACT_CLAMPED = 2, ACT_GELU = 3 };
-
-struct Activation {  // ACT_CLAMPED: float32 [2n] biases of gate and up (or null)
-  const float* bias;
-  float limit, slope;
-};
 
 // Which tiles a launch is made of: each of the 8 XCDs takes `places` tiles of form `form`, the first `whole` of them as they are, which fill
 // its compute units in whole rounds, the rest, which would leave some of them idle, cut into `cut` tiles of fewer rows (form `rest`).
@@ -33,7 +24,7 @@ struct TurnsPlan {
 
 template <class T, int ACT>
 __device__ __forceinline__ void make_tile(bf16_t* ring, const bf16_t* __restrict__ a, int64_t lda, const bf16_t* __restrict__ w, int64_t ldw,
-                                          bf16_t* __restrict__ out, int64_t ldo, const Activation& how, bool vec, int m, int n, int k, int r0,
+                                          bf16_t* __restrict__ out, int64_t ldo, const GatedActivation& how, bool vec, int m, int n, int k, int r0,
                                           int feature_tile) {
   constexpr bool GATED = ACT != ACT_NONE;
   constexpr int FEATURES = GATED ? T::BN / 2 : T::BN;
@@ -42,46 +33,25 @@ __device__ __forceinline__ void make_tile(bf16_t* ring, const bf16_t* __restrict
   T tile;
   tile.run(
       ring, k / TURNS_K, [&](int r) { return a + (int64_t)min(r0 + r, m - 1) * lda; },
-      [&](int r) { return w + (int64_t)(GATED ? T::gated_row(r, f0, n) : min(f0 + r, n - 1)) * ldw; });
+      [&](int r) { return w + (int64_t)(GATED ? T::Pairs::row_of(r, f0, n) : min(f0 + r, n - 1)) * ldw; });
   tile.leave(ring, [](float sum, int) { return sum; });
-  // (the two products as the element type holds them, then the arithmetic of silu_mul, clamped_glu, gated_mul)
-  constexpr int CHUNKS = FEATURES / 8;
-  float gate_bias[8] = {}, up_bias[8] = {};
-  if (ACT == ACT_CLAMPED && how.bias != nullptr) {  // (a thread's features are the same in every row)
-    static_assert(ACT != ACT_CLAMPED || T::THREADS % CHUNKS == 0);
-    const int f = f0 + (int)threadIdx.x % CHUNKS * 8;
-#pragma unroll
-    for (int c = 0; c < 8; ++c) gate_bias[c] = how.bias[min(f + c, n - 1)], up_bias[c] = how.bias[n + min(f + c, n - 1)];
-  }
-  for (int i = threadIdx.x; i < T::BM * CHUNKS; i += T::THREADS) {
-    const int row = i / CHUNKS, f = i % CHUNKS * 8;
-    if (r0 + row >= m || f0 + f >= n) continue;
-    const bf16_t* at = ring + row * T::MADE + (GATED ? T::gated_at(f) : f);
-    float v[8];
-    mi_load_8(at, v);
-    if constexpr (GATED) {
-      float u[8];
-      mi_load_8(at + T::PAIR, u);
-#pragma unroll
-      for (int c = 0; c < 8; ++c) {
-        if constexpr (ACT == ACT_CLAMPED) {
-          const float gate = fminf(v[c] + gate_bias[c], how.limit);
-          const float up = fminf(fmaxf(u[c] + up_bias[c], -how.limit), how.limit);
-          v[c] = gate * mi_logistic(how.slope * gate) * (up + 1.f);
-        } else if constexpr (ACT == ACT_GELU) {
-          v[c] = 0.5f * v[c] * (1.f + tanhf(0.7978845608028654f * (v[c] + 0.044715f * v[c] * v[c] * v[c]))) * u[c];
-        } else {
-          v[c] = silu_times<bf16_t>(v[c], u[c]);
-        }
-      }
+  if constexpr (GATED) {
+    write_activated<ACT, typename T::Pairs, T::BM, T::BN, T::MADE, T::THREADS>(ring, how, out, ldo, vec, r0, m, f0, n);
+  } else {
+    constexpr int CHUNKS = FEATURES / 8;
+    for (int i = threadIdx.x; i < T::BM * CHUNKS; i += T::THREADS) {
+      const int row = i / CHUNKS, f = i % CHUNKS * 8;
+      if (r0 + row >= m || f0 + f >= n) continue;
+      float v[8];
+      mi_load_8(ring + row * T::MADE + f, v);
+      mi_store_8(out + (int64_t)(r0 + row) * ldo, f0 + f, n, vec, v);
     }
-    mi_store_8(out + (int64_t)(r0 + row) * ldo, f0 + f, n, vec, v);
   }
 }
 
 template <int ACT>
 __global__ __launch_bounds__(512, 2) void gemm_turns_kernel(const bf16_t* __restrict__ a, int64_t lda, const bf16_t* __restrict__ w, int64_t ldw,
-                                                            bf16_t* __restrict__ out, int64_t ldo, const Activation how, bool vec, int m, int n, int k,
+                                                            bf16_t* __restrict__ out, int64_t ldo, const GatedActivation how, bool vec, int m, int n, int k,
                                                             int row_tiles, int feature_tiles, const TurnsPlan plan) {
   __shared__ __align__(16) bf16_t ring[TURNS_RING];
   // (workgroups are dealt to the XCDs in turn)
@@ -154,7 +124,7 @@ extern "C" int mi_gemm_turns_bf16(int act, const void* a, int64_t lda, const voi
   MI_REQUIRE(act >= 0 && act <= 3 && (act != ACT_CLAMPED || limit > 0.f), "gemm_turns_bf16: activation %d, limit %g", act, (double)limit);
   MI_REQUIRE((int64_t)ceil_div(m, 64) * ceil_div(n, 64) < (1 << 27), "gemm_turns_bf16: too many tiles");
   const bool vec = (uintptr_t)out % 16 == 0 && ldo % 8 == 0;
-  const Activation how = {bias, limit, slope};
+  const GatedActivation how = {bias, limit, slope};
   MI_REQUIRE(only >= -1 && only < TURNS_FORMS && (only < 0 || act == ACT_NONE || turns_form(only).gated), "gemm_turns_bf16: form %d", only);
   double micros;
   const TurnsPlan plan = turns_plan(m, n, k, act != ACT_NONE, only, max(8, mi_compute_units()), &micros);

@@ -30,7 +30,9 @@ struct TileProduct {
   static constexpr int STEP_K = 64;
   static constexpr int STAGE = (BM + BN) * STEP_K;  // elements
   static constexpr int EXCHANGE = WK == 1 ? 0 : WM * WN * NT * MT * MI_WAVE * 8;  // elements: float32 sums that change hands
-  static constexpr int RING = STAGES * STAGE > EXCHANGE ? STAGES * STAGE : EXCHANGE;
+  static constexpr int MADE = BN + 8;  // elements from one row that `leave` leaves to the next
+  static constexpr int WORK = STAGES * STAGE > EXCHANGE ? STAGES * STAGE : EXCHANGE;
+  static constexpr int RING = WORK > BM * MADE ? WORK : BM * MADE;
   static constexpr int LOADS = (BM + BN) / 8;  // of 8 rows x 128 bytes
   static constexpr int EACH = LOADS / WAVES, REST = LOADS % WAVES;  // a wave makes EACH, the first REST one more
   static constexpr int MOST = EACH + (REST > 0);
@@ -181,6 +183,21 @@ struct TileProduct {
         for (int m = 0; m < MT; ++m)
           if ((m < FIRST_M) == (wk == 0)) acc[n][m] += to[(n * MT + m) * MI_WAVE];
     }
+  }
+
+  // The sums rounded to bfloat16 as rows of the tile in `ring`, MADE elements apart; all threads see them afterwards.
+  __device__ __forceinline__ void leave(bf16_t* ring) {
+    __syncthreads();
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+      if (mine(m)) {
+#pragma unroll
+        for (int n = 0; n < NT; ++n) {
+          const float v[4] = {acc[n][m][0], acc[n][m][1], acc[n][m][2], acc[n][m][3]};
+          mi_store_cols<bf16_t, 4>(ring + row(m) * MADE + feature(n), v);
+        }
+      }
+    __syncthreads();
   }
 
   // Whether row tile m's sums are this wave's to write.

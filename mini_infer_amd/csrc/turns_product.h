@@ -14,7 +14,7 @@
 // one wave alone, so all tile shapes give the same bits as those.
 #pragma once
 
-#include "common.h"
+#include "gated_tile.h"
 
 typedef float f32x4_u __attribute__((ext_vector_type(4)));
 
@@ -246,33 +246,8 @@ struct TurnsProduct {
     }
     __syncthreads();
   }
-  // Products of gate and up rows: of a wave's tiles of W the first half are gate rows, the second the up rows of the same features.  Which
-  // row of [gate; up] of `features` features each the tile's row r of W is, features from f0 on; and where the tile's feature f lies in
-  // what `leave` left, its up product PAIR further on.
-  static constexpr int PAIR = NT / 2 * 16;
-  static __device__ __forceinline__ int gated_row(int r, int f0, int features) {
-    const int t = r % (2 * PAIR), f = min(f0 + r / (2 * PAIR) * PAIR + t % PAIR, features - 1);
-    return t < PAIR ? f : f + features;
-  }
-  static __device__ __forceinline__ int gated_at(int f) { return f / PAIR * (2 * PAIR) + f % PAIR; }
+  using Pairs = GatedTile<NT>;  // where the tile holds gate and up rows
 };
-
-// Eight bfloat16 values of LDS as floats, and eight floats as bfloat16 values of a row from column f on that has n of them (whole: 16 bytes at once).
-__device__ __forceinline__ void mi_load_8(const bf16_t* p, float (&v)[8]) {
-  const bf16x8_t got = *reinterpret_cast<const bf16x8_t*>(p);
-#pragma unroll
-  for (int i = 0; i < 8; ++i) v[i] = to_f32((bf16_t)got[i]);
-}
-__device__ __forceinline__ void mi_store_8(bf16_t* row, int f, int n, bool whole, const float (&v)[8]) {
-  if (whole && f + 8 <= n) {
-    bf16x8_t out;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) out[i] = from_f32<bf16_t>(v[i]);
-    *reinterpret_cast<bf16x8_t*>(row + f) = out;
-  } else {
-    for (int i = 0; i < 8 && f + i < n; ++i) row[f + i] = from_f32<bf16_t>(v[i]);
-  }
-}
 
 // The tiles that launches choose among, rows of A x rows of W, and the microseconds that a step of 64 of K takes one.
 // X(number, rows, rows of W, gate and up rows side by side?, microseconds a step, shape)

@@ -543,10 +543,11 @@ def _rows_of_bf16(x: torch.Tensor, weight: torch.Tensor) -> bool:
     )
 
 
-def _tiles(kind: int, x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor, n: int, shape: int, ranges: int, scale: float = 1.0) -> torch.Tensor:
+def _tiles(kind: int, x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor, n: int, shape: int, ranges: int, scale: float = 1.0,
+           bias: torch.Tensor | None = None, limit: float = 0.0, slope: float = 0.0) -> torch.Tensor:
     library.check(
         library.load().mi_gemm_tiles_bf16(kind, _ptr(x), x.stride(0), _ptr(weight), weight.stride(0), _ptr(out), out.stride(-2), scale,
-                                          x.shape[0], n, x.shape[1], shape, ranges, _stream())
+                                          _ptr(bias), limit, slope, x.shape[0], n, x.shape[1], shape, ranges, _stream())
     )
     return out
 
@@ -625,12 +626,14 @@ def tile_size(shape: int) -> tuple[int, int]:
 @functools.lru_cache(maxsize=8192)
 def gated_tiles_for(m: int, n: int, k: int, cus: int = WHOLE_DEVICE_CUS) -> int | None:
     """The tile shape where the gated product of n features is made in tiles, or None.  Up to 32 rows the streaming product
-    (`gemm_skinny_swiglu_bf16`) stands, because tiles are not faster everywhere there (gate|up at 24 rows: 16384 x 3072 19.8 against 23.9 us,
-    28672 x 4096 50.8 against 47.1) and no rule between the two has been measured.  Above, measured against the vendor product
-    and `silu_mul`, tiles are 1.0 to 1.9 times as fast up to 160 rows, and beyond as long as tiles of up to 192 x 128 are what pays
-    (7168 x 4096 at 256 / 600 rows 32.5 / 48.2 against 43.8 / 53.8, 16384 x 2048 at 271 / 320 29.4 / 30.8 against 33.3 /
-    33.9); where there is work for larger ones the library is faster by as much as 1.3 (28672 x 4096 at 193 rows 86.9 / 72.3, 57344 x
-    8192 at 161 / 192 rows 235 / 215 and 236 / 203; at 160 rows 181 / 196)."""
+    (`gemm_skinny_swiglu_bf16`) stands, in whose sums a row's result does not depend on how many other rows there are (tiles of 32 x 64 are
+    faster where they are a block a compute unit on most of them, gate|up at 17 / 24 / 32 rows 16384 x 3072 22.6 / 22.3 / 23.6 us against
+    19.3 / 18.7 / 19.1, 11008 x 2048 12.9 / 13.8 / 15.1 against 11.6 / 11.9 / 12.3, and level or slower elsewhere, 28672 x 4096 43.7 / 45.9 /
+    47.1 against 48.7 / 47.4 / 47.4).  Above, measured against the vendor product and the activation's launch, tiles are 1.0 to 1.9 times as fast up to
+    160 rows, and beyond as long as tiles of up to 192 x 128 are what pays (7168 x 4096 at 256 rows 32.5 against 43.8, 16384 x 2048 at
+    271 / 320 29.4 / 30.8 against 33.3 / 33.9; with the clamped activation 16384 x 3072 at 64 / 200 / 300 rows 24.7 / 39.9 / 46.5 against 22.1 / 36.1
+    / 44.1); where there is work for larger ones the library is faster by as much as 1.3 (28672 x 4096 at 193 rows 86.9 / 72.3, 57344 x 8192 at 161 /
+    192 rows 235 / 215 and 236 / 203; at 160 rows 181 / 196)."""
     if not SKINNY_WIDE_MAX_ROWS < m <= 768:
         return None
     _, shape, _ = _tiles_plan(m, n, k, True, 1, False, 0.0, 0.0, cus)
@@ -641,6 +644,7 @@ def gated_tiles_for(m: int, n: int, k: int, cus: int = WHOLE_DEVICE_CUS) -> int 
 
 TURNS_MIN_ROWS = 321
 TURNS_NONE, TURNS_SILU, TURNS_CLAMPED, TURNS_GELU = range(4)
+GATED_TILE_KINDS = {TURNS_SILU: 3, TURNS_CLAMPED: 4, TURNS_GELU: 5}  # of gemm_tiles_bf16
 TURNS_OUTPUTS_A_K = 400
 
 
@@ -692,6 +696,22 @@ def _turns(act: int, x: torch.Tensor, weight: torch.Tensor, n: int, bias: torch.
                                           out.stride(0), x.shape[0], n, x.shape[1], only, _stream())
     )
     return out
+
+
+def _gated_as_one(act: int, x: torch.Tensor, weight: torch.Tensor, steady: bool, bias: torch.Tensor | None = None, limit: float = 0.0,
+                  slope: float = 0.0) -> torch.Tensor | None:
+    """The gated product of more than 32 rows with its activation as one launch of tiles where that pays, else None."""
+    if _turns_take(x, weight):
+        return _turns(act, x, weight, weight.shape[0] // 2, bias, limit, slope)
+    if steady or x.dim() != 2 or not SKINNY_WIDE_MAX_ROWS < x.shape[0] <= TILES_MAX_ROWS or not _rows_of_bf16(x, weight):
+        return None
+    _need_cuda(x, weight, bias)
+    m, n = x.shape[0], weight.shape[0] // 2
+    shape = gated_tiles_for(m, n, x.shape[1], _compute_units(x.device))
+    if shape is None:
+        return None
+    out = torch.empty((m, n), dtype=torch.bfloat16, device=x.device)
+    return _tiles(GATED_TILE_KINDS[act], x, weight, out, n, shape, 1, bias=bias, limit=limit, slope=slope)
 
 
 def linear(x: torch.Tensor, weight: torch.Tensor, partial_ok: bool = False, steady: bool = False) -> torch.Tensor | PartialSums:
@@ -851,7 +871,7 @@ def qkv_rope_write(
 def linear_swiglu(x: "torch.Tensor | ScaledRows", gate_up_weight: torch.Tensor, steady: bool = False) -> torch.Tensor:
     """`silu(x @ gate.T) * (x @ up.T)` with `gate_up_weight` = [gate; up] stacked, [2I, K].
 
-    bfloat16 with at most 32 rows, and up to some hundreds where that is faster (`gated_tiles_for`), runs as ONE
+    bfloat16 with at most 32 rows, up to some hundreds where that is faster (`gated_tiles_for`) and most of more (`turns_pay`) runs as ONE
     hand-written kernel (the product with the activation in its last step), and so do up to 8 float32 rows (4 of a long K);
     otherwise the product and `silu_mul` run in turn.  Both ways round the two products to the element type before the activation, so given
     the same rows a token's result does not depend on which one ran.  `x` may be
@@ -878,14 +898,10 @@ def linear_swiglu(x: "torch.Tensor | ScaledRows", gate_up_weight: torch.Tensor, 
             scaled, x = x, values
         else:
             x = x.finish()
-    if scaled is None and _turns_take(x, gate_up_weight):
-        return _turns(TURNS_SILU, x, gate_up_weight, rows // 2)
-    if not steady and scaled is None and x.dim() == 2 and SKINNY_WIDE_MAX_ROWS < x.shape[0] <= TILES_MAX_ROWS and _rows_of_bf16(x, gate_up_weight):
-        _need_cuda(x, gate_up_weight)
-        m, n = x.shape[0], rows // 2
-        shape = gated_tiles_for(m, n, width, _compute_units(x.device))
-        if shape is not None:
-            return _tiles(3, x, gate_up_weight, torch.empty((m, n), dtype=torch.bfloat16, device=x.device), n, shape, 1)
+    if scaled is None:
+        made = _gated_as_one(TURNS_SILU, x, gate_up_weight, steady)
+        if made is not None:
+            return made
     if (
         x.dtype == torch.bfloat16
         and gate_up_weight.dtype == torch.bfloat16
@@ -2019,13 +2035,20 @@ def clamped_glu(
 
 def linear_clamped_glu(x: torch.Tensor, gate_up_weight: torch.Tensor, bias: torch.Tensor | None, limit: float, slope: float,
                        steady: bool = False) -> torch.Tensor:
-    """`clamped_glu(x @ [gate; up].T, bias, limit, slope)`.  bfloat16 with at most 32 rows runs as ONE
-    kernel (the weight-streaming product with biases, clamps and activation in its last step);
-    otherwise the product and `clamped_glu` run in turn.  Both round the two products to the element
-    type first and then do the same float32 arithmetic, so the results agree bit for bit."""
+    """`clamped_glu(x @ [gate; up].T, bias, limit, slope)`.  bfloat16 with at most 32 rows, up to some
+    hundreds where that is faster (`gated_tiles_for`) and most of more (`turns_pay`) runs as ONE kernel (the product with biases, clamps and
+    activation in its last step); otherwise the product and `clamped_glu` run in turn.  All round the two products to the
+    element type first and then do the same float32 arithmetic."""
     rows, width = gate_up_weight.shape
     if rows % 2 or (bias is not None and bias.numel() != rows):
         raise KernelShapeError(f"linear_clamped_glu: stacked weight of {rows} rows, bias of {None if bias is None else bias.numel()}")
+    if bias is not None:
+        _need_contiguous("bias", bias)
+        _need_f32("bias", bias)
+    if limit > 0:
+        made = _gated_as_one(TURNS_CLAMPED, x, gate_up_weight, steady, bias, float(limit), float(slope))
+        if made is not None:
+            return made
     if (
         x.dtype == torch.bfloat16
         and gate_up_weight.dtype == torch.bfloat16
@@ -2036,8 +2059,6 @@ def linear_clamped_glu(x: torch.Tensor, gate_up_weight: torch.Tensor, bias: torc
         and skinny_gemm_takes(x.shape[0], width, x.stride(0), gate_up_weight.stride(0), SKINNY_WIDE_MAX_ROWS)
     ):
         _need_cuda(x, gate_up_weight, bias)
-        _need_contiguous("bias", bias)
-        _need_f32("bias", bias)
         m, n = x.shape[0], rows // 2
         out = torch.empty((m, n), dtype=torch.bfloat16, device=x.device)
         library.check(
@@ -2047,10 +2068,6 @@ def linear_clamped_glu(x: torch.Tensor, gate_up_weight: torch.Tensor, bias: torc
             )
         )
         return out
-    if _turns_take(x, gate_up_weight) and limit > 0:
-        _need_contiguous("bias", bias)
-        _need_f32("bias", bias)
-        return _turns(TURNS_CLAMPED, x, gate_up_weight, rows // 2, bias, float(limit), float(slope))
     return clamped_glu(linear(x, gate_up_weight, steady=steady), bias, limit, slope)
 
 
@@ -2174,12 +2191,15 @@ def layer_in(
 
 def linear_geglu(x: torch.Tensor, gate_up_weight: torch.Tensor, steady: bool = False) -> torch.Tensor:
     """`gelu_tanh(x @ gate.T) * (x @ up.T)` with `gate_up_weight` = [gate; up] stacked, [2I, K].  bfloat16
-    with at most 32 rows runs as ONE kernel (the weight-streaming product with the activation in its
-    last step); otherwise the product and `gated_mul` run in turn.  Both round the two products to the
+    with at most 32 rows, up to some hundreds where that is faster (`gated_tiles_for`) and most of more (`turns_pay`) runs as ONE kernel (the
+    product with the activation in its last step); otherwise the product and `gated_mul` run in turn.  All round the two products to the
     element type first and then do the same float32 arithmetic."""
     rows, width = gate_up_weight.shape
     if rows % 2:
         raise KernelShapeError(f"linear_geglu: stacked weight has an odd number of rows ({rows})")
+    made = _gated_as_one(TURNS_GELU, x, gate_up_weight, steady)
+    if made is not None:
+        return made
     if (
         x.dtype == torch.bfloat16
         and gate_up_weight.dtype == torch.bfloat16
@@ -2198,8 +2218,6 @@ def linear_geglu(x: torch.Tensor, gate_up_weight: torch.Tensor, steady: bool = F
             )
         )
         return out
-    if _turns_take(x, gate_up_weight):
-        return _turns(TURNS_GELU, x, gate_up_weight, rows // 2)
     both = linear(x, gate_up_weight, steady=steady)
     return gated_mul(both[:, : rows // 2], both[:, rows // 2 :], "gelu_tanh")
 

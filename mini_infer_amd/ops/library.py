@@ -14,7 +14,7 @@ from pathlib import Path
 from mini_infer_amd.exceptions import ExtensionMissingError, KernelShapeError
 from mini_infer_amd.ops import build as _build
 
-ABI_VERSION = 48
+ABI_VERSION = 49
 
 _lib: ctypes.CDLL | None = None
 _lib_path: Path | None = None
@@ -41,7 +41,9 @@ _SIGNATURES: dict[str, list] = {
     "mi_gemm_tiles_rows": [c_int],
     "mi_gemm_tiles_features": [c_int],
     "mi_gemm_tiles_take": [c_int, c_int, c_int, c_int64, c_int64],
-    "mi_gemm_tiles_bf16": [c_int, _P, c_int64, _P, c_int64, _P, c_int64, c_float, c_int, c_int, c_int, c_int, c_int, _P],
+    "mi_gemm_tiles_bf16": [
+        c_int, _P, c_int64, _P, c_int64, _P, c_int64, c_float, _P, c_float, c_float, c_int, c_int, c_int, c_int, c_int, _P,
+    ],
     "mi_sum_pieces": [_P, _P, c_int, c_int64, _P],
     "mi_gemm_skinny_attn_bf16_supported": [c_int, c_int, c_int],
     "mi_gemm_skinny_attn_bf16": [_P, _P, c_int, c_int, c_int, _P, c_int64, _P, c_int64, c_int, c_int, _P],

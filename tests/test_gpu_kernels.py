@@ -231,16 +231,17 @@ def test_every_tile_shape_is_tested():
 
 @pytest.mark.parametrize("shape", range(TILE_SHAPES))
 def test_products_in_tiles(shape):
-    """Every shape at the edges of its tiles, whole, over ranges of K, as float32 times a number, and gated; K of one step, of fewer steps than
+    """Every shape at the edges of its tiles, whole, over ranges of K, as float32 times a number, and gated with each activation; K of one step, of fewer steps than
     the ring has stages, of odd 32s, and of ranges of unequal length; rows of a wider buffer, whose values beside and behind the result
     stay, on boundaries of four values and off them; a row of infinities stays alone."""
+    from mini_infer_amd import ops
     from mini_infer_amd.ops import kernels
 
     bm, bn = kernels.tile_size(shape)
     cases = [(bm, bn, 64, 1), (bm + 1, bn + 1, 128, 2), (bm - 1, bn - 3, 320, 1), (2 * bm + 5, 2 * bn + 4, 64 * 11, 3), (1, 5, 32, 1),
              (17, bn + 62, 96, 1), (bm, 70, 64 * 7 + 32, 2), (3, 2 * bn, 1024, 16)]
 
-    def made(kind, a, w, n, dtype, ranges=1, scale=1.0, spare=0):
+    def made(kind, a, w, n, dtype, ranges=1, scale=1.0, spare=0, bias=None):
         """The product in the first columns of rows with `spare` more (over ranges: [ranges, m, n], contiguous) before more values."""
         m = a.shape[0]
         if kind == 1:
@@ -249,7 +250,7 @@ def test_products_in_tiles(shape):
         else:
             wide = torch.full((m + 1, n + spare), 7.0, dtype=dtype, device=DEV)
             out, rest = wide[:m, :n], [wide[:, n:], wide[m:]]
-        kernels._tiles(kind, a, w, out, n, shape, ranges, scale)
+        kernels._tiles(kind, a, w, out, n, shape, ranges, scale, bias, 2.5, 1.702)
         assert all((each == 7).all() for each in rest), (kind, a.shape, n, ranges, spare)
         return out
 
@@ -278,6 +279,11 @@ def test_products_in_tiles(shape):
                 # (a product may come out one rounding apart: the gated tile sums the same pieces in the same order, so it does not)
                 gated = made(3, a, w, n, torch.bfloat16, spare=spare)[finite]
                 assert ((gated.double() - wanted).abs() <= 2.0 ** -8 * wanted.abs() + 1e-30).all(), (m, n, k)
+                # (and the other activations are those of the launch that would follow)
+                bias = _rand(2 * n, seed=48)
+                assert torch.equal(made(4, a, w, n, torch.bfloat16, spare=spare, bias=bias)[finite], ops.clamped_glu(out, bias, 2.5, 1.702)[finite])
+                assert torch.equal(made(4, a, w, n, torch.bfloat16, spare=spare)[finite], ops.clamped_glu(out, None, 2.5, 1.702)[finite])
+                assert torch.equal(made(5, a, w, n, torch.bfloat16, spare=spare)[finite], ops.gated_mul(out[:, :n], out[:, n:], "gelu_tanh")[finite])
 
 
 def test_every_form_of_the_tiles_that_take_turns_is_tested():
