@@ -169,15 +169,15 @@ class GQAttention(Mixer):
 
     def wants_scaled_rows(self, rows: int) -> bool:
         """Only where projection, rotation and cache write will run as the one kernel that
-        applies the rows' factors: few bfloat16 rows, whole heads rotated in half pairing."""
+        applies the rows' factors: few rows, whole heads rotated in half pairing."""
         layout = self.position.rotary_layout() if self.position is not None else None
+        takes = ops.scaled_rows_product_takes if self.dtype == torch.bfloat16 else ops.scaled_rows_product_takes_f32
         return (
-            self.dtype == torch.bfloat16
-            and self._same_widths
+            self._same_widths
             and self._plain_heads
             and layout == (self.head_dim, False)
             and self.head_dim % 32 == 0
-            and ops.scaled_rows_product_takes(rows, self.qkv.weight, self.hidden_size)
+            and takes(rows, self.qkv.weight, self.hidden_size)
         )
 
     def cache_needs(self, page_size: int) -> CacheNeeds:
@@ -268,19 +268,19 @@ class GQAttention(Mixer):
             x = x.finish() if isinstance(x, ops.ScaledRows) else x
             return self._project(self.forward_projected(self.qkv.forward(x), ctx, cache, writes_cache))
         rotary = self.position.rotary(ctx) if self.position is not None else None
+        if self.dtype == torch.bfloat16:
+            takes, project = ops.qkv_rope_write_takes, ops.qkv_rope_write
+        else:
+            takes, project = ops.qkv_rope_write_f32_takes, ops.qkv_rope_write_f32
+        as_one = rotary is not None and self._same_widths and self._plain_heads
         if isinstance(x, ops.ScaledRows) and not (
-            rotary is not None
-            and self._same_widths
-            and self._plain_heads
-            and ops.qkv_rope_write_takes(x, self.qkv.weight, self.head_dim, rotary.rotary_dim, rotary.interleaved)
+            as_one and takes(x, self.qkv.weight, self.head_dim, rotary.rotary_dim, rotary.interleaved)
         ):
             x = x.finish()  # rows but for their norm factors, and no kernel here that applies them
-        if rotary is not None and self._same_widths and self._plain_heads and ops.qkv_rope_write_takes(
-            x, self.qkv.weight, self.head_dim, rotary.rotary_dim, rotary.interleaved
-        ):
+        if as_one and takes(x, self.qkv.weight, self.head_dim, rotary.rotary_dim, rotary.interleaved):
             # few rows (decode): projection, rotation and cache write are one kernel
             kv_heads = self.num_kv_heads if writes_cache else 0
-            queries = ops.qkv_rope_write(
+            queries = project(
                 x, self.qkv.weight if writes_cache else self.qkv.weight[:q_width], rotary.cos, rotary.sin,
                 ctx.slot_mapping[cache.group] if writes_cache else None, cache.k_pages, cache.v_pages,
                 q_heads=self.num_heads, kv_heads=kv_heads, head_dim=self.head_dim,
@@ -333,10 +333,10 @@ class GQAttention(Mixer):
         """The output projection of what `_attend` returned; for few rows, where the block
         asked for it, not made here but handed on to the norm that follows."""
         assert self.out.weight is not None
-        if self.emit_pending_output and self.dtype == torch.bfloat16:
+        if self.emit_pending_output:
             rows = attended.tokens if isinstance(attended, ops.AttentionPieces) else attended.shape[0]
             q_width = self.num_heads * self.v_head_dim
-            if ops.pending_product_pays(rows, self.hidden_size, q_width, self.emit_partial_sums):
+            if ops.pending_product_pays(rows, self.hidden_size, q_width, self.emit_partial_sums and self.dtype == torch.bfloat16):
                 return ops.PendingProduct(attended, self.out.weight)
         if isinstance(attended, ops.AttentionPieces):
             return ops.linear_from_attention(attended, self.out.weight)
