@@ -4,112 +4,131 @@
 // and a block finds its tile in that list.
 //
 // The tiles are those of turns_product.h, 64, 128, 160 or 256 pairs x 256 weight rows, one block to a CU; all of them sum in the
-// same order, so which one is taken does not show in the results.  What bounds such a launch is the matrix cores, and the
-// last round of blocks, which may be nearly empty: 2,700 pairs over 16 experts are 22 to 50 row tiles, and a row tile more or less
-// decides whether it takes one round or two.  The host does not know how many pairs an expert got, so every block works out
-// from the list, before it looks for its tile, how long the launch takes in either size and takes the shortest: all
-// blocks see the same list and take the same.  Measured (microseconds, the pairs as routers spread them, 58 to 333 an expert;
-// before: tiles of 128 x 128 on two buffers, four waves in step, two blocks to a CU):
-//     experts x gate|up, down            pairs    before        now
-//     16 x 4096 x 3072, 3072 x 2048      1,942    133 +  40     102 +  42
-//                                        3,238    161 +  70     126 +  52
-//                                        4,122    173 +  70     123 +  56
-//     16 x 7168 x 4096, 4096 x 3584      2,612    261 + 153     210 + 124
-//                                        5,776    430 + 245     308 + 176
-// and over 120 such pairs of launches 1.17 times as fast from 96 to 200 pairs an expert, 1.23 beyond, and below, where the weights' bytes
-// bound both, 1.03 to 1.04 (a single launch at worst 0.93, both together 0.97).  A step of 1,501 tokens of 12 layers at the
-// first sizes 6,708 -> 6,429 us.
+// same order, so which one is taken does not show in the results.  What bounds such a launch is the weights' bytes up to some 150 pairs an
+// expert, the matrix cores beyond some 300, and anywhere the last round of blocks, which may be nearly empty: 2,700 pairs over 16 experts are 16 to 50
+// row tiles of 16 blocks, and an expert with 257 pairs more decides whether 256 CUs take one round or two.  So each expert's pairs are cut by
+// themselves (expert_cuts.h), whoever makes the list leaves the four ways to do so beside it, every block works out which of them its launch takes
+// (the host does not know how many pairs an expert got), and the largest tiles run first, so that the small ones fill the gaps.
+// Microseconds, gate and up + down, weights from memory, the pairs as routers spread them (two of 18 experts are not among the 16): all experts'
+// tiles alike, cut expert by expert:
+//     experts x gate|up, down          pairs     an expert        alike       by expert
+//     16 x 4096 x 3072, 3072 x 2048      700      25 to 88       81 +  51      71 +  47
+//                                      1,760      69 to 178      94 +  60      82 +  50
+//                                      2,670     101 to 284     146 +  59     108 +  58
+//                                      5,330     230 to 448     171 + 105     167 +  96
+//                                     10,700     334 to 1001    254 + 159     268 + 147
+//     16 x 7168 x 4096, 4096 x 3584    2,220      80 to 193     218 + 114     189 +  95
+//                                      3,560     122 to 407     290 + 168     250 + 141
+//     64 x 2048 x 2048, 2048 x 1024    5,800      35 to 173     165 +  84     133 +  61
+// A step of 1,501 tokens of 12 layers at the first sizes 6,055 -> 5,800 us.  (Tiles of 128 x 128 on two buffers, four waves in step, two blocks to a
+// CU, came before both: 1.17 to 1.23 times the time of tiles that are all alike from 96 pairs an expert on.)
 //
-// Tiles are numbered expert by expert, within an expert feature tile by feature tile with the row tiles of one
-// feature tile side by side; each of the 8 XCDs takes one stretch of these numbers (workgroups are dealt
-// to the XCDs in turn), so the row tiles that read the same weights run at the same time behind one
-// L2, and an expert's rows stay in it.
+// Each of the 8 XCDs takes an eighth of the tiles of every form (workgroups are dealt to the XCDs in turn), side by side in the list: an
+// expert's row tile by row tile, a row tile's feature tiles one after the other, so that its pairs' rows stay behind one L2.  (Tiles
+// dealt to the XCDs one by one, which brings every expert's rows into every L2: 16 x 4096 x 3072 with 5,330 pairs 157 -> 181.)
 //
 // MODE as in routed_experts.hip: 0 plain, 1 silu(gate) * up (a block then makes BN / 2 features: gate and up rows
 // side by side in its tile), 2 relu(weight * z)^2.
+#include "expert_cuts.h"
 #include "turns_product.h"
 
 namespace {
 
-// The same on the device, from the list.  All threads of the block get the same answer.
-__device__ __forceinline__ int pick_form(const int* __restrict__ first, int experts, bool smallest, int n, int k, int cus) {
-  int row_tiles[TURNS_WIDE] = {}, used = 0;
-  for (int e = threadIdx.x % MI_WAVE; e < experts; e += MI_WAVE) {
-    const int pairs = first[e + 1] - first[e];
-    used += pairs > 0;
+constexpr int TILE_FEATURES = 256;
+static_assert(cut_rows(0) == turns_form(0).rows && cut_rows(1) == turns_form(1).rows && cut_rows(2) == turns_form(2).rows && cut_rows(3) == turns_form(3).rows);
+
+// Microseconds of a launch over n weight rows of k elements an expert: what the compute units multiply, the largest tiles first, and what they
+// bring in, of which neither hides the other quite.  Fitted to 50 spreads of pairs over experts of five sizes, weights from memory: the cut with the least of
+// these is 0.5 % slower than the best one on average, 8 % at worst.
+__host__ __device__ inline float launch_micros(const CutSums& sums, int n, int k, int cus) {
+  const int feature_tiles = (n + TILE_FEATURES - 1) / TILE_FEATURES;
+  constexpr float STEP[CUT_FORMS] = {0.84f, 1.04f, 1.15f, 1.30f};  // of 64 of K, with the pairs' rows from L2 and the weights from memory
+  float micros[CUT_FORMS], work = 0.f, rows = 0.f;
+  int all = 0;
 #pragma unroll
-    for (int f = 0; f < TURNS_WIDE; ++f) row_tiles[f] += (pairs + turns_form(f).rows - 1) / turns_form(f).rows;
+  for (int f = 0; f < CUT_FORMS; ++f) {
+    micros[f] = (float)(k / TURNS_K) * STEP[f] + 5.9f;
+    work += micros[f] * (float)sums.tiles[f];
+    rows += (float)cut_rows(f) * (float)sums.tiles[f];
+    all += sums.tiles[f];
   }
+  auto at = [&](int place) {  // of the tile at a place in the launch's order
+    float of = 0.f;
+    int past = 0;
 #pragma unroll
-  for (int off = MI_WAVE / 2; off > 0; off >>= 1) {
-    used += __shfl_xor(used, off, MI_WAVE);
-#pragma unroll
-    for (int f = 0; f < TURNS_WIDE; ++f) row_tiles[f] += __shfl_xor(row_tiles[f], off, MI_WAVE);
-  }
-  if (!smallest) row_tiles[0] = 0;
-  return __builtin_amdgcn_readfirstlane(turns_pick(row_tiles, used, n, k, cus));
+    for (int f = CUT_FORMS - 1; f >= 0; --f) {
+      past += sums.tiles[f] * feature_tiles;
+      if (of == 0.f && place < past) of = micros[f];
+    }
+    return of;
+  };
+  float made = work * (float)feature_tiles / (float)cus;
+  const float first = at(0), next = at(cus), two = next > 0.f ? at(cus - 1) + next : 0.f, three = 3.f * at(2 * cus);
+  made = first > made ? first : made;
+  made = two > made ? two : made;
+  made = three > made ? three : made;
+  const float matrix = (float)n * (float)k * 2.f;
+  const float brought = 1.40e-7f * (float)sums.used * matrix + 0.78e-7f * rows * (float)feature_tiles * (float)k * 2.f +
+                        0.69e-7f * (float)(all - sums.used) * matrix + 1.11e-7f * (float)sums.again * matrix;
+  const float a = made * made, b = brought * brought;
+  return sqrtf(sqrtf(a * a + b * b));
 }
 
-// Which tile this block works on: expert, first pair of the row tile (an index into `listed`), feature tile.
-// False: past the last tile.  All threads of the block get the same answer.
-__device__ __forceinline__ bool find_tile(const int* __restrict__ first, int experts, int feature_tiles, int bm, int id,
-                                          int& expert, int& row0, int& feature_tile) {
-  const int lane = threadIdx.x % MI_WAVE;
-  // row tiles in all
-  int total = 0;
-  for (int base = 0; base < experts; base += MI_WAVE) {
-    const int e = base + lane;
-    int tiles = e < experts ? (first[e + 1] - first[e] + bm - 1) / bm : 0;
-#pragma unroll
-    for (int off = MI_WAVE / 2; off > 0; off >>= 1) tiles += __shfl_xor(tiles, off, MI_WAVE);
-    total += tiles;
-  }
-  total *= feature_tiles;
-  const int per = (total + 7) / 8;
-  const int place = (id % 8) * per + id / 8;
-  if (id / 8 >= per || place >= total) return false;
-  int before = 0;
-  for (int base = 0; base < experts; base += MI_WAVE) {
-    const int e = base + lane;
-    const int tiles = e < experts ? (first[e + 1] - first[e] + bm - 1) / bm : 0;
-    int upto = tiles;  // row tiles of the experts up to and including this lane's
-#pragma unroll
-    for (int off = 1; off < MI_WAVE; off <<= 1) {
-      const int other = __shfl_up(upto, off, MI_WAVE);
-      if (lane >= off) upto += other;
-    }
-    const uint64_t past = __ballot((before + upto) * feature_tiles > place);
-    if (past != 0) {
-      const int at = __builtin_ctzll(past);
-      const int mine = __shfl(tiles, at, MI_WAVE), start = before + __shfl(upto, at, MI_WAVE) - mine;
-      const int rest = place - start * feature_tiles;
-      expert = base + at;
-      row0 = first[expert] + (rest % mine) * bm;
-      feature_tile = rest / mine;
-      return true;
-    }
-    before += __shfl(upto, MI_WAVE - 1, MI_WAVE);
-  }
-  return false;
+__global__ __launch_bounds__(CUTS * MI_WAVE) void expert_plan_kernel(const int* __restrict__ first, int pairs, int experts, CutsPlan* __restrict__ plan) {
+  plan_cut(first, pairs, experts, __builtin_amdgcn_readfirstlane(threadIdx.x / MI_WAVE), plan);
 }
 
-template <class T, int MODE>
+// Which tile block `id` works on.  False: past the last one.  All threads of the block get the same answer.
+__device__ __forceinline__ bool find_tile(const CutsPlan* __restrict__ plan, int pairs, int experts, int n, int k, int cus, int id, RowTile& place,
+                                          int& feature_tile) {
+  const int lane = threadIdx.x % MI_WAVE, feature_tiles = (n + TILE_FEATURES - 1) / TILE_FEATURES;
+  const CutSums sums = plan->sums[min(lane, CUTS - 1)];  // a lane a cut
+  const float micros = launch_micros(sums, n, k, cus);
+  int cut = 0;
+  float least = 0.f;
+#pragma unroll
+  for (int c = CUTS - 1; c >= 0; --c) {
+    const float its = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(micros), c));
+    if (c == CUTS - 1 || its < least) cut = c, least = its;
+  }
+  // each XCD has an eighth of the tiles of every form, the largest first, side by side in the list; what is left over of one form goes to
+  // the XCDs behind those that got what was left over of the form before
+  int slot = id / 8, row_tile = 0, given = 0, at = -1;
+#pragma unroll
+  for (int f = CUT_FORMS - 1; f >= 0; --f) {
+    const int row_tiles = __builtin_amdgcn_readlane(sums.tiles[f], cut), tiles = row_tiles * feature_tiles, turn = (id - given) & 7;
+    const int mine = tiles / 8 + (turn < tiles % 8);
+    if (at < 0) {
+      if (slot < mine) at = turn * (tiles / 8) + min(turn, tiles % 8) + slot;
+      else slot -= mine, row_tile += row_tiles;
+    }
+    given += tiles;
+  }
+  if (at < 0) return false;
+  row_tile += at / feature_tiles;
+  feature_tile = at % feature_tiles;
+  const RowTile* list = row_tiles_of(plan, cut, pairs, experts) + row_tile;
+  place.expert = __builtin_amdgcn_readfirstlane(list->expert);
+  place.row0 = __builtin_amdgcn_readfirstlane(list->row0);
+  place.end = __builtin_amdgcn_readfirstlane(list->end);
+  place.form = __builtin_amdgcn_readfirstlane(list->form);
+  return true;
+}
+
+template <class T, int MODE, bool ONCE>
 __device__ __forceinline__ void make_tile(
     bf16_t* ring, const bf16_t* __restrict__ src, int64_t src_stride, int src_div, const bf16_t* __restrict__ weight,
-    int64_t expert_stride, const int* __restrict__ listed, const int* __restrict__ first,
-    const float* __restrict__ pair_weight, bf16_t* __restrict__ out, int64_t out_stride, int experts, int k_dim, int features) {
+    int64_t expert_stride, const int* __restrict__ listed,
+    const float* __restrict__ pair_weight, bf16_t* __restrict__ out, int64_t out_stride, int k_dim, int features, const RowTile& place, int feature_tile) {
   constexpr bool GATED = MODE == 1;
   constexpr int FEATURES = GATED ? T::BN / 2 : T::BN;
-  static_assert(T::BN == TURNS_FEATURES);
-  const int feature_tiles = (features + FEATURES - 1) / FEATURES;
-  int expert, row0, feature_tile;
-  if (!find_tile(first, experts, feature_tiles, T::BM, blockIdx.x, expert, row0, feature_tile)) return;
-  const int end = first[expert + 1], f0 = feature_tile * FEATURES;
+  static_assert(T::BN == TILE_FEATURES);
+  const int expert = place.expert, row0 = place.row0, end = place.end, f0 = feature_tile * FEATURES;
   const bf16_t* w = weight + (int64_t)expert * expert_stride;
   T tile;
-  tile.run(
+  tile.template run<ONCE>(
       ring, k_dim / TURNS_K,
-      [&](int r) {  // (past the expert's last pair: that one again, not written)
+      [&](int r) {  // (past the tile's last pair: that one again, not written)
         return src + (int64_t)(listed[min(row0 + r, end - 1)] / src_div) * src_stride;
       },
       [&](int r) { return w + (int64_t)(GATED ? T::Pairs::row_of(r, f0, features) : min(f0 + r, features - 1)) * k_dim; });
@@ -136,36 +155,37 @@ __device__ __forceinline__ void make_tile(
   }
 }
 
-template <int MODE>
+// ONCE: most experts have one row tile, so that nobody else reads its weights: past the caches (16 x 4096 x 3072 with 2,700 pairs 106 -> 98 us, and
+// 75 -> 67 with 400; with 12,000 pairs 265 -> 270).
+template <int MODE, bool ONCE>
 __global__ __launch_bounds__(512, 2) void expert_tiles_kernel(
     const bf16_t* __restrict__ src, int64_t src_stride, int src_div, const bf16_t* __restrict__ weight,
-    int64_t expert_stride, const int* __restrict__ listed, const int* __restrict__ first,
-    const float* __restrict__ pair_weight, bf16_t* __restrict__ out, int64_t out_stride, int experts, int k_dim,
-    int features, bool smallest, int cus) {
+    int64_t expert_stride, const int* __restrict__ listed, const CutsPlan* __restrict__ plan,
+    const float* __restrict__ pair_weight, bf16_t* __restrict__ out, int64_t out_stride, int pairs, int experts, int k_dim,
+    int features, int cus) {
   __shared__ __align__(16) bf16_t ring[TURNS_RING];
-  const int form = pick_form(first, experts, smallest, MODE == 1 ? 2 * features : features, k_dim, cus);
-#define MI_TILE(...) make_tile<__VA_ARGS__, MODE>(ring, src, src_stride, src_div, weight, expert_stride, listed, first, pair_weight, out, out_stride, experts, k_dim, features)
-  if (form == 0) MI_TILE(TurnsOf<0>::type);
-  else if (form == 1) MI_TILE(TurnsOf<1>::type);
-  else if (form == 2) MI_TILE(TurnsOf<2>::type);
-  else if (form == 3) MI_TILE(TurnsOf<3>::type);
+  RowTile place;
+  int feature_tile;
+  if (!find_tile(plan, pairs, experts, MODE == 1 ? 2 * features : features, k_dim, cus, blockIdx.x, place, feature_tile)) return;
+#define MI_TILE(...) \
+  make_tile<__VA_ARGS__, MODE, ONCE>(ring, src, src_stride, src_div, weight, expert_stride, listed, pair_weight, out, out_stride, k_dim, features, place, feature_tile)
+  if (place.form == 0) MI_TILE(TurnsOf<0>::type);
+  else if (place.form == 1) MI_TILE(TurnsOf<1>::type);
+  else if (place.form == 2) MI_TILE(TurnsOf<2>::type);
+  else MI_TILE(TurnsOf<3>::type);
 #undef MI_TILE
 }
 
-// Pairs an expert has on average up to which tiles of 64 may be taken (they were the best of the four up to 71): a launch has a block for
-// every tile that there can be of the smallest size, and the rest end when they have read the list.
-constexpr int SMALLEST_UP_TO = 96;
-
 template <int MODE>
-void launch_tiles(const void* src, int64_t src_stride, int src_div, const void* weight, const int* listed, const int* first,
+void launch_tiles(const void* src, int64_t src_stride, int src_div, const void* weight, const int* listed, const void* plan,
                   const float* pair_weight, void* out, int64_t out_stride, int pairs, int experts, int k_dim, int features, int cus,
                   hipStream_t stream) {
-  const int feature_tiles = ceil_div(features, MODE == 1 ? TURNS_FEATURES / 2 : TURNS_FEATURES);
-  const bool smallest = pairs <= (int64_t)SMALLEST_UP_TO * experts;
-  const int most = feature_tiles * (pairs / turns_form(smallest ? 0 : 1).rows + min(experts, pairs));  // (an expert's last tile may be a short one)
-  expert_tiles_kernel<MODE><<<ceil_div(most, 8) * 8, 512, 0, stream>>>(
-      (const bf16_t*)src, src_stride, src_div, (const bf16_t*)weight, (int64_t)(MODE == 1 ? 2 : 1) * features * k_dim, listed,
-      first, pair_weight, (bf16_t*)out, out_stride, experts, k_dim, features, smallest, cus);
+  const int feature_tiles = ceil_div(features, MODE == 1 ? TILE_FEATURES / 2 : TILE_FEATURES);
+  const int most = feature_tiles * most_row_tiles(pairs, experts, 0);
+  const auto kernel = pairs <= (int64_t)cut_rows(CUT_FORMS - 1) * experts ? expert_tiles_kernel<MODE, true> : expert_tiles_kernel<MODE, false>;
+  kernel<<<ceil_div(most, 8) * 8, 512, 0, stream>>>((const bf16_t*)src, src_stride, src_div, (const bf16_t*)weight,
+                                                    (int64_t)(MODE == 1 ? 2 : 1) * features * k_dim, listed, (const CutsPlan*)plan, pair_weight,
+                                                    (bf16_t*)out, out_stride, pairs, experts, k_dim, features, cus);
 }
 
 }  // namespace
@@ -173,33 +193,55 @@ void launch_tiles(const void* src, int64_t src_stride, int src_div, const void* 
 // Whether rows of k_dim bfloat16 elements are taken.
 extern "C" int mi_expert_tiles_take(int k_dim) { return k_dim > 0 && k_dim % TURNS_K == 0; }
 
-// Rows of the tile that a launch of n weight rows an expert takes where the experts got counts[0..experts) pairs (0: no pairs).
-extern "C" int mi_expert_tiles_rows(const int* counts, int experts, int n, int k_dim, int cus) {
-  int row_tiles[TURNS_WIDE] = {}, used = 0;
-  int64_t pairs = 0;
-  for (int e = 0; e < experts; ++e) {
-    pairs += counts[e], used += counts[e] > 0;
-    for (int f = 0; f < TURNS_WIDE; ++f) row_tiles[f] += ceil_div(counts[e], turns_form(f).rows);
+// How a launch of n weight rows an expert cuts experts with counts[0..experts) pairs: for each expert four numbers: full
+// tiles of the largest form, tiles behind them, the pairs in each of these and the rows of their form.
+extern "C" int mi_expert_tiles_cut(const int* counts, int experts, int n, int k_dim, int cus, int* cuts) {
+  MI_REQUIRE(counts && cuts && experts > 0 && n > 0 && mi_expert_tiles_take(k_dim), "expert_tiles_cut: experts=%d n=%d k=%d", experts, n, k_dim);
+  int best = -1;
+  float least = 0.f;
+  for (int c = CUTS - 1; c >= 0; --c) {
+    CutSums sums = {};
+    for (int e = 0; e < experts; ++e) add(sums, cover(counts[e], c));
+    const float micros = launch_micros(sums, n, k_dim, max(8, cus));
+    if (best < 0 || micros < least) best = c, least = micros;
   }
-  if (pairs > (int64_t)SMALLEST_UP_TO * experts) row_tiles[0] = 0;
-  const int form = turns_pick(row_tiles, used, n, k_dim, max(8, cus));
-  return form < 0 ? 0 : turns_form(form).rows;
+  for (int e = 0; e < experts; ++e) {
+    const Cover c = cover(counts[e], best);
+    cuts[4 * e] = c.full, cuts[4 * e + 1] = c.tiles, cuts[4 * e + 2] = c.each, cuts[4 * e + 3] = cut_rows(c.form);
+  }
+  return MI_OK;
 }
 
-// Arguments as mi_expert_rows (bfloat16 only), with the number of listed pairs.
+// 32-bit words of the plan that mi_expert_plan leaves for mi_expert_tiles, on 16 bytes.
+extern "C" int64_t mi_expert_plan_words(int pairs, int experts) {
+  if (pairs < 0 || experts < 1) return 0;
+  return (int64_t)(sizeof(CutsPlan) + row_tiles_before(CUTS, pairs, experts) * sizeof(RowTile)) / 4;
+}
+
+// (mi_expert_sort leaves the same where it is asked to)
+extern "C" int mi_expert_plan(const int* first, int pairs, int experts, void* plan, hipStream_t stream) {
+  MI_REQUIRE(pairs >= 0 && experts > 0 && first && plan && (uintptr_t)plan % 16 == 0, "expert_plan: pairs=%d experts=%d", pairs, experts);
+  if (pairs == 0) return MI_OK;
+  expert_plan_kernel<<<1, CUTS * MI_WAVE, 0, stream>>>(first, pairs, experts, (CutsPlan*)plan);
+  MI_CHECK_LAUNCH("expert_plan");
+  return MI_OK;
+}
+
+// Arguments as mi_expert_rows (bfloat16 only), with the number of pairs handed to the list, and the plan of mi_expert_plan for the list in place
+// of `first`.
 extern "C" int mi_expert_tiles(int mode, const void* src, int64_t src_stride, int src_div, const void* weight,
-                               const int* listed, const int* first, const float* pair_weight, void* out,
+                               const int* listed, const void* plan, const float* pair_weight, void* out,
                                int64_t out_stride, int pairs, int experts, int k_dim, int features, hipStream_t stream) {
   MI_REQUIRE(pairs >= 0 && experts > 0 && features > 0 && src_div > 0 && src_stride >= k_dim && out_stride >= features,
              "expert_tiles: bad sizes pairs=%d experts=%d k=%d features=%d", pairs, experts, k_dim, features);
   MI_REQUIRE(mi_expert_tiles_take(k_dim) && src_stride % 8 == 0 && ((uintptr_t)src | (uintptr_t)weight) % 16 == 0 && (uintptr_t)out % 8 == 0,
              "expert_tiles: rows of %d elements are not taken %d at a time", k_dim, TURNS_K);
-  MI_REQUIRE(mode >= 0 && mode <= 2, "expert_tiles: mode %d", mode);
+  MI_REQUIRE(mode >= 0 && mode <= 2 && (uintptr_t)plan % 16 == 0, "expert_tiles: mode %d", mode);
   MI_REQUIRE((int64_t)ceil_div(features, 128) * ((int64_t)pairs / 64 + experts) < (1 << 30), "expert_tiles: too many tiles");
   if (pairs == 0) return MI_OK;
   const int cus = max(8, mi_compute_units());
 #define MI_TILES(MODE) \
-  launch_tiles<MODE>(src, src_stride, src_div, weight, listed, first, pair_weight, out, out_stride, pairs, experts, k_dim, features, cus, stream)
+  launch_tiles<MODE>(src, src_stride, src_div, weight, listed, plan, pair_weight, out, out_stride, pairs, experts, k_dim, features, cus, stream)
   if (mode == 1) MI_TILES(1);
   else if (mode == 2) MI_TILES(2);
   else MI_TILES(0);

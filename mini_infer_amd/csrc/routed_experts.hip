@@ -29,6 +29,7 @@
 //                        expert reads, and W (w x) = w (W x), so no weighted copy of the rows is made
 // and EXPERT_PLAIN, the second product alone.
 #include "common.h"
+#include "expert_cuts.h"
 
 #include <math.h>
 
@@ -377,8 +378,9 @@ __device__ __forceinline__ void place_experts(int* count, int* __restrict__ firs
   if (lane == 0) first[experts] = at;
 }
 
+// `plan` (may be null): what expert_cuts.h says of the list; the first waves make it while the others list the pairs.
 __global__ __launch_bounds__(1024) void expert_sort_kernel(const int* __restrict__ chosen, int* __restrict__ listed,
-                                                           int* __restrict__ first, int pairs, int experts) {
+                                                           int* first, int pairs, int experts, CutsPlan* __restrict__ plan) {
   __shared__ int count[MI_SORT_MAX_EXPERTS + 1];
   for (int e = threadIdx.x; e <= experts; e += blockDim.x) count[e] = 0;
   __syncthreads();
@@ -389,6 +391,8 @@ __global__ __launch_bounds__(1024) void expert_sort_kernel(const int* __restrict
   __syncthreads();
   place_experts(count, first, experts);
   __syncthreads();
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / MI_WAVE);
+  if (plan != nullptr && wave < CUTS) plan_cut(first, pairs, experts, wave, plan);
   // (pairs of one expert in any order: each pair's result is its own)
   for (int p = threadIdx.x; p < pairs; p += blockDim.x) {
     const int e = chosen[p];
@@ -845,10 +849,12 @@ extern "C" int mi_expert_combine(int dtype, const void* made, const int* where, 
   return MI_OK;
 }
 
-extern "C" int mi_expert_sort(const int* chosen, int* listed, int* first, int pairs, int experts, hipStream_t stream) {
+// `plan`: mi_expert_plan_words words on 16 bytes, or null.
+extern "C" int mi_expert_sort(const int* chosen, int* listed, int* first, int pairs, int experts, void* plan, hipStream_t stream) {
   MI_REQUIRE(pairs >= 0 && experts > 0 && experts <= MI_SORT_MAX_EXPERTS, "expert_sort: %d pairs over %d experts (at most %d)", pairs,
              experts, MI_SORT_MAX_EXPERTS);
-  expert_sort_kernel<<<1, pairs > 256 ? 1024 : 256, 0, stream>>>(chosen, listed, first, pairs, experts);
+  MI_REQUIRE((uintptr_t)plan % 16 == 0, "expert_sort: the plan lies on 16 bytes");
+  expert_sort_kernel<<<1, pairs > 256 ? 1024 : 256, 0, stream>>>(chosen, listed, first, pairs, experts, pairs > 0 ? (CutsPlan*)plan : nullptr);
   MI_CHECK_LAUNCH("expert_sort");
   return MI_OK;
 }

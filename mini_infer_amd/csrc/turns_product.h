@@ -91,8 +91,9 @@ struct TurnsProduct {
   }
 
   // acc = the tile's sums over `steps` (at least one) times 64 of K; a_row(r) and w_row(r) give the first of them of the tile's row r,
-  // 0 <= r < BM, BN, on 16 bytes and readable.  Nothing of `ring` may be written before the block has met once more.
-  template <typename RowA, typename RowW>
+  // 0 <= r < BM, BN, on 16 bytes and readable.  Nothing of `ring` may be written before the block has met once more.  ONCE: nobody else reads
+  // these rows of W (they are then read past the caches).
+  template <bool ONCE = false, typename RowA, typename RowW>
   __device__ __forceinline__ void run(bf16_t* ring, int steps, RowA a_row, RowW w_row) {
     const bf16_t* src[MOST];
     const int chunk = ((lane % 8) ^ (lane / 8)) * 8;
@@ -110,7 +111,11 @@ struct TurnsProduct {
       bf16_t* at = ring + slot * STAGE + wave * 512;
 #pragma unroll
       for (int j = from; j < to; ++j) {
-        if (j < EACH || wave < REST) __builtin_amdgcn_global_load_lds((global_void*)src[j], (lds_void*)(at + j * (WAVES * 512)), 16, 0, 0);
+        const bool of_w = HALVES ? (j + 1) * WAVES * 8 <= BN : j * WAVES * 8 >= BM;
+        if (j < EACH || wave < REST) {
+          if (ONCE && of_w) __builtin_amdgcn_global_load_lds((global_void*)src[j], (lds_void*)(at + j * (WAVES * 512)), 16, 0, 2);
+          else __builtin_amdgcn_global_load_lds((global_void*)src[j], (lds_void*)(at + j * (WAVES * 512)), 16, 0, 0);
+        }
         src[j] += STEP_K;
       }
     };
@@ -300,20 +305,4 @@ __host__ __device__ inline float turns_rounds_micros(int f, int tiles, int each,
 }
 __host__ __device__ inline float turns_bytes_micros(int f, int matrices, int64_t blocks, int n, int k) {
   return 2.33e-7f * (float)matrices * (float)n * (float)k * 2.f + 0.73e-7f * (float)blocks * (float)k * ((float)turns_form(f).features * 2.f);
-}
-
-// Of the first four forms (256 rows of W) the one that a launch takes, or -1: row_tiles[f] of form f cover the rows of A (0: not to be taken); matrices:
-// the matrices W, n rows of k elements each, that any of them reads; cus: compute units, in 8 XCDs to which blocks are dealt in turn.
-constexpr int TURNS_WIDE = 4, TURNS_FEATURES = 256;
-__host__ __device__ inline int turns_pick(const int (&row_tiles)[TURNS_WIDE], int matrices, int n, int k, int cus) {
-  int best = -1;
-  float least = 0.f;
-  for (int f = 0; f < TURNS_WIDE; ++f) {
-    if (row_tiles[f] == 0) continue;
-    const int blocks = row_tiles[f] * ((n + TURNS_FEATURES - 1) / TURNS_FEATURES);
-    const float multiplied = turns_rounds_micros(f, (blocks + 7) / 8, cus / 8, k), brought = turns_bytes_micros(f, matrices, blocks, n, k);
-    const float micros = multiplied > brought ? multiplied : brought;
-    if (best < 0 || micros < least * 0.995f) best = f, least = micros;  // (level: the smaller one)
-  }
-  return best;
 }

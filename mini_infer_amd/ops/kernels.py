@@ -3241,10 +3241,18 @@ EXPERT_ACTIVATIONS = {"silu_gated": (1, 2), "squared_relu": (2, 1)}
 @dataclasses.dataclass
 class ExpertLists:
     """The (row, choice) pairs of a step listed expert by expert, on the device: expert e's are `listed[first[e] :
-    first[e + 1]]` (int32 [pairs] and [experts + 1])."""
+    first[e + 1]]` (int32 [pairs] and [experts + 1]); `plan`: how tiles staged through LDS may cut them, where those may be taken."""
 
     listed: torch.Tensor
     first: torch.Tensor
+    plan: torch.Tensor | None = None
+
+
+def _list_pairs(chosen: torch.Tensor, lists: ExpertLists, pairs: int, experts: int, planned: bool) -> None:
+    lib = library.load()
+    if planned:
+        lists.plan = torch.empty((lib.mi_expert_plan_words(pairs, experts),), dtype=torch.int32, device=chosen.device)
+    library.check(lib.mi_expert_sort(_ptr(chosen), _ptr(lists.listed), _ptr(lists.first), pairs, experts, _ptr(lists.plan), _stream()))
 
 
 def route_top_k(
@@ -3305,7 +3313,7 @@ def route_top_k(
         )
     )
     if lists is not None:
-        library.check(library.load().mi_expert_sort(_ptr(chosen), _ptr(lists.listed), _ptr(lists.first), tokens * top, experts, _stream()))
+        _list_pairs(chosen, lists, tokens * top, experts, x.dtype == torch.bfloat16 and tokens * top >= EXPERT_LDS_TILES_MIN_ROWS * experts)
         return chosen, weights, gates, lists
     return chosen, weights, gates
 
@@ -3428,11 +3436,13 @@ def expert_tiles_take(x: torch.Tensor, ff: int) -> bool:
     return x.dtype == torch.bfloat16 and bool(lib.mi_expert_tiles_take(x.shape[1])) and bool(lib.mi_expert_tiles_take(ff))
 
 
-def expert_tile_rows(counts: list[int], weight_rows: int, k: int, cus: int = WHOLE_DEVICE_CUS) -> int:
-    """Rows of the tile that a launch of the tiles staged through LDS takes where the experts got `counts` pairs, `weight_rows` (gate and up
-    together) of `k` elements each."""
-    given = (ctypes.c_int * len(counts))(*counts)
-    return library.load().mi_expert_tiles_rows(ctypes.addressof(given), len(counts), weight_rows, k, cus)
+def expert_tile_cuts(counts: list[int], weight_rows: int, k: int, cus: int = WHOLE_DEVICE_CUS) -> list[tuple[int, int, int, int]]:
+    """For each expert with `counts` pairs: the full tiles of 256 of them, the tiles behind those, the pairs in each of these and the rows of
+    their form, in a launch of the tiles staged through LDS with `weight_rows` (gate and up together) of `k` elements an expert."""
+    given, cuts = (ctypes.c_int * len(counts))(*counts), (ctypes.c_int * (4 * len(counts)))()
+    library.check(library.load().mi_expert_tiles_cut(ctypes.addressof(given), len(counts), weight_rows, k, cus,
+                                                     ctypes.addressof(cuts)))
+    return [tuple(cuts[4 * e:4 * e + 4]) for e in range(len(counts))]
 
 
 def expert_tiles_for(x: torch.Tensor, pairs: int, experts: int, ff: int) -> str:
@@ -3456,7 +3466,7 @@ def experts_by_expert(
     per sixteen of them, not once per row.  `tiles` (default: by the average number of rows an expert
     gets): "rows" is that form; for prompts (bfloat16) "direct", blocks of 64 features that take 64 of an
     expert's rows a pass, and "lds", tiles of 64 to 256 rows x 256 weight rows with both operands staged through LDS
-    (rows in steps of 64 elements; which of them, the device finds out from the list: `expert_tile_rows`).  `combine=False`
+    (rows in steps of 64 elements; which of them, the device finds out from the list: `expert_tile_cuts`).  `combine=False`
     (no shared or identity experts): the rows are left for a norm to add up (`SummedRows`; weights on the
     output: `WeightedRows`).  `leave_rows`: the sum of any experts is left to a norm behind it (`ExpertRows`).
     `lists`: the pairs by expert where `route_top_k` has made them already."""
@@ -3470,7 +3480,7 @@ def experts_by_expert(
     if lists is None:
         lists = ExpertLists(torch.empty((pairs,), dtype=torch.int32, device=x.device),
                             torch.empty((experts + 1,), dtype=torch.int32, device=x.device))
-        library.check(library.load().mi_expert_sort(_ptr(chosen), _ptr(lists.listed), _ptr(lists.first), pairs, experts, _stream()))
+        _list_pairs(chosen, lists, pairs, experts, tiles == "lds" or (tiles is None and expert_tiles_for(x, pairs, experts, ff) == "lds"))
     listed, first = lists.listed, lists.first
     if listed.numel() != pairs or first.numel() != experts + 1 or listed.dtype != torch.int32 or first.dtype != torch.int32:
         raise KernelShapeError("experts_by_expert: the lists are those of other pairs")
@@ -3483,9 +3493,13 @@ def experts_by_expert(
         raise KernelShapeError(f"experts_by_expert: tiles {tiles!r} for rows of {width} and {ff} {x.dtype}")
     many = int(tiles == "direct")
     if tiles == "lds":
-        library.check(lib.mi_expert_tiles(mode, _ptr(x), x.stride(0), top, _ptr(gate_up), _ptr(listed), _ptr(first),
+        plan = lists.plan
+        if plan is None:
+            plan = torch.empty((lib.mi_expert_plan_words(pairs, experts),), dtype=torch.int32, device=x.device)
+            library.check(lib.mi_expert_plan(_ptr(first), pairs, experts, _ptr(plan), _stream()))
+        library.check(lib.mi_expert_tiles(mode, _ptr(x), x.stride(0), top, _ptr(gate_up), _ptr(listed), _ptr(plan),
                                           _ptr(on_input), _ptr(act), ff, pairs, experts, width, ff, _stream()))
-        library.check(lib.mi_expert_tiles(0, _ptr(act), ff, 1, _ptr(down), _ptr(listed), _ptr(first), None, _ptr(made),
+        library.check(lib.mi_expert_tiles(0, _ptr(act), ff, 1, _ptr(down), _ptr(listed), _ptr(plan), None, _ptr(made),
                                           width, pairs, experts, ff, width, _stream()))
     else:
         library.check(lib.mi_expert_rows(code, mode, _ptr(x), x.stride(0), top, _ptr(gate_up), _ptr(listed), _ptr(first),

@@ -14,7 +14,7 @@ from pathlib import Path
 from mini_infer_amd.exceptions import ExtensionMissingError, KernelShapeError
 from mini_infer_amd.ops import build as _build
 
-ABI_VERSION = 50
+ABI_VERSION = 51
 
 _lib: ctypes.CDLL | None = None
 _lib_path: Path | None = None
@@ -176,7 +176,7 @@ _SIGNATURES: dict[str, list] = {
     "mi_weighted_squared_relu": [c_int, _P, c_int64, _P, _P, c_int64, c_int, c_int, _P],
     "mi_expert_down_combine": [c_int, _P, _P, _P, _P, _P, c_int64, _P, c_int64, _P, _P, c_int, c_int, c_int, c_int, c_int, _P],
     "mi_expert_combine": [c_int, _P, _P, _P, _P, _P, c_int64, _P, c_int64, _P, _P, c_int, c_int, c_int, c_int, _P],
-    "mi_expert_sort": [_P, _P, _P, c_int, c_int, _P],
+    "mi_expert_sort": [_P, _P, _P, c_int, c_int, _P, _P],
     "mi_expert_rows_at_once": [c_int, c_int],
     "mi_expert_rows": [c_int, c_int, _P, c_int64, c_int, _P, _P, _P, _P, _P, c_int64, c_int, c_int, c_int, c_int, _P],
     "mi_attn_latent_takes": [c_int, c_int],
@@ -193,7 +193,9 @@ _SIGNATURES: dict[str, list] = {
     "mi_gemm_turns_bf16": [
         c_int, _P, c_int64, _P, c_int64, _P, c_float, c_float, _P, c_int64, c_int, c_int, c_int, c_int, _P,
     ],
-    "mi_expert_tiles_rows": [_P, c_int, c_int, c_int, c_int],
+    "mi_expert_tiles_cut": [_P, c_int, c_int, c_int, c_int, _P],
+    "mi_expert_plan_words": [c_int, c_int],
+    "mi_expert_plan": [_P, c_int, c_int, _P, _P],
     "mi_expert_tiles": [c_int, _P, c_int64, c_int, _P, _P, _P, _P, _P, c_int64, c_int, c_int, c_int, c_int, _P],
     "mi_gated_update_norm": [
         c_int, _P, _P, c_int64, c_int, _P, c_int64, _P, _P, _P, _P, _P, c_int, c_int, c_float, c_float, _P, c_int, _P,
@@ -206,7 +208,7 @@ _SIGNATURES: dict[str, list] = {
 }
 
 
-_INT64_RESULTS = {"mi_gated_delta_chunks_scratch", "mi_decay_scan_chunks_scratch", "mi_attn_prompt_f32_blocks"}  # (sizes; every other entry point returns an int status)
+_INT64_RESULTS = {"mi_gated_delta_chunks_scratch", "mi_decay_scan_chunks_scratch", "mi_attn_prompt_f32_blocks", "mi_expert_plan_words"}  # (sizes; every other entry point returns an int status)
 
 
 def _declare(lib: ctypes.CDLL, path: Path) -> None:

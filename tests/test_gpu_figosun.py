@@ -389,12 +389,15 @@ def test_silu_gated_experts_in_tiles_staged_through_lds(rows, width, ff, experts
 
 
 @pytest.mark.parametrize("activation", ["silu_gated", "squared_relu"])
-@pytest.mark.parametrize("rows, width, ff, counts, tile_rows", [
-    # (by the rule, for the first product: its 25,600 weight rows are 100 tiles for every row tile, and the rounds of 256 decide)
-    (40, 64, 128, [1, 16, 17, 6], 64), (230, 128, 12800, [97, 128], 128), (320, 192, 12800, [160, 129], 160), (520, 64, 12800, [255, 256], 256),
-    (511, 128, 12800, [255, 256], 256), (520, 320, 12800, [256, 241], 256), (300, 64, 12800, [160, 130], 160),
-    (300, 192, 320, [0, 127, 129, 0, 33], 64), (700, 320, 64, [1, 640, 3], 128), (64, 64, 64, [64], 64)])
-def test_expert_tiles_of_every_size(activation, rows, width, ff, counts, tile_rows):
+@pytest.mark.parametrize("rows, width, ff, counts, forms", [
+    (40, 64, 128, [1, 16, 17, 6], [64, 64, 64, 64]), (230, 128, 12800, [97, 128], [128, 128]), (320, 192, 12800, [160, 129], [160, 160]),
+    (520, 64, 12800, [255, 256], [256, 256]), (511, 128, 12800, [255, 256], [256, 256]), (520, 320, 12800, [256, 241], [256, 256]),
+    (300, 64, 12800, [160, 65], [160, 128]), (300, 192, 320, [0, 127, 129, 0, 33], [64, 128, 128, 64, 64]),
+    (700, 320, 64, [1, 640, 3], [64, 128, 64]), (64, 64, 64, [64], [64]),
+    # several tiles an expert, as many pairs in each; full ones and a rest of another form, or of the same
+    (814, 64, 6400, [513, 0, 300], [256, 64, 160]), (620, 64, 12800, [513, 100], [64, 128]), (1030, 64, 12800, [512, 513], [256, 256]),
+    (760, 512, 6400, [700, 40], [256, 64])])
+def test_expert_tiles_of_every_size(activation, rows, width, ff, counts, forms):
     """Tiles of 64, 128, 160 and 256 rows at their edges, one to five steps of 64 of K and more, features beside whole tiles, experts without
     pairs: against float64.  A product rounds once to bfloat16 (2^-9), the activation's inputs and its output once each; the sums themselves are float32 over at
     most 12,800 terms of their own size, 2^-12 of the result's; a pair's result is held against the largest."""
@@ -402,8 +405,8 @@ def test_expert_tiles_of_every_size(activation, rows, width, ff, counts, tile_ro
 
     features = 2 * ff if activation == "silu_gated" else ff
     if activation != "silu_gated":  # (half the weight rows, so twice the experts)
-        rows, counts = 2 * rows, counts + counts
-    assert ops.kernels.expert_tile_rows(counts, features, width) == tile_rows
+        rows, counts, forms = 2 * rows, counts + counts, forms + forms
+    assert [form for _, _, _, form in ops.kernels.expert_tile_cuts(counts, features, width)] == forms
     rng = np.random.default_rng(rows + width)
     experts = len(counts)
     x = dev(rng.standard_normal((rows, width)), torch.bfloat16)

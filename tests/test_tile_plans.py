@@ -59,25 +59,27 @@ def test_gated_products_of_more_than_160_rows_take_no_tiles_above_192_by_128():
     assert kernels.gated_tiles_for(193, 14336, 4096) is None and kernels.gated_tiles_for(192, 14336, 4096) is not None
 
 
-@pytest.mark.parametrize("counts, weight_rows, k, rows", [
-    ([4] * 16, 4096, 3072, 64),                    # few pairs an expert: the weights' bytes, and no row tile twice
-    ([100] * 16, 3072, 2048, 128),                 # one row tile an expert, one round of blocks
-    ([150] * 16, 4096, 3072, 160),                 # two of 128 would make two rounds
-    ([250] * 16, 4096, 3072, 256),
-    ([0, 0, 1, 0], 256, 64, 64),
-    ([0, 0], 256, 64, 0),                          # nobody chose any: nothing to do
-    ([10000], 28672, 4096, 256),
+@pytest.mark.parametrize("counts, weight_rows, k, cuts", [
+    ([4] * 16, 4096, 3072, [(0, 1, 4, 64)] * 16),
+    ([100] * 16, 3072, 2048, [(0, 1, 100, 128)] * 16),
+    ([150, 40] * 8, 4096, 3072, [(0, 1, 150, 160), (0, 1, 40, 64)] * 8),         # each expert the smallest form that holds its pairs
+    ([250] * 16, 4096, 3072, [(0, 1, 250, 256)] * 16),
+    ([0, 0, 1, 0], 256, 64, [(0, 0, 0, 64)] * 2 + [(0, 1, 1, 64), (0, 0, 0, 64)]),
+    ([0, 0], 256, 64, [(0, 0, 0, 64)] * 2),                                      # nobody chose any: nothing to do
+    ([1, 300, 45], 512, 512, [(0, 1, 1, 64), (0, 3, 100, 128), (0, 1, 45, 64)]),  # few tiles: smaller ones
+    ([10000], 28672, 4096, [(39, 1, 16, 64)]),                                   # many: full ones and the smallest for the rest
 ])
-def test_expert_tiles_by_the_rounds_of_blocks_they_take(counts, weight_rows, k, rows):
-    assert kernels.expert_tile_rows(counts, weight_rows, k) == rows
+def test_expert_tiles_by_what_their_launch_takes(counts, weight_rows, k, cuts):
+    assert kernels.expert_tile_cuts(counts, weight_rows, k) == cuts
 
 
-def test_expert_tiles_count_the_compute_units():
-    """A quarter of a device takes four rounds where the whole one takes one; tiles of 64 end at 96 pairs an expert on average."""
-    assert kernels.expert_tile_rows([130] * 16, 4096, 3072, 256) == 160
-    assert kernels.expert_tile_rows([96] * 2, 256, 64) == 64 and kernels.expert_tile_rows([97] * 2, 256, 64) == 128
-    for cus in (8, 64, 256):
-        assert kernels.expert_tile_rows([1, 300, 45], 512, 512, cus) in (64, 128, 160, 256)
+@pytest.mark.parametrize("counts", [[1], [63, 64, 65], [255, 256, 257, 0, 1025], [160, 161, 320, 321, 512, 513], [7] * 200, [5000, 1, 0, 2049]])
+@pytest.mark.parametrize("weight_rows, k, cus", [(64, 64, 8), (4096, 3072, 256), (28672, 4096, 256), (640, 512, 64)])
+def test_expert_tiles_hold_every_pair(counts, weight_rows, k, cus):
+    for pairs, (full, tiles, each, rows) in zip(counts, kernels.expert_tile_cuts(counts, weight_rows, k, cus)):
+        assert rows in (64, 128, 160, 256) and each <= rows
+        assert full * 256 + tiles * each >= pairs > full * 256 or pairs == full == tiles == 0
+
 
 
 @pytest.mark.parametrize("gated", [False, True])
