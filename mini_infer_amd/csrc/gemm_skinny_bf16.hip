@@ -40,8 +40,8 @@ typedef __attribute__((__vector_size__(4 * sizeof(float)))) float f32x4_t;
 //   EPI_STORE_F32  c (float32) = float(bf16(product)): the output head's logits, which are
 //              wanted in float32 (no cast launch after the product).  Rounded to bfloat16 on the
 //              way like every product of this path, so that a position's logits are the same
-//              numbers whether its step had few rows (this kernel) or many (the vendor
-//              library's bfloat16 product, widened afterwards).
+//              numbers whether its step had few rows (this kernel) or many (a
+//              bfloat16 product, widened afterwards).
 //   EPI_GELU_TABLE  c = bf16(gelu_tanh(bf16(product)) * table[ids[row], col0 + feature]): a gate that
 //              multiplies a slice of a per-token table row (a side input that depends on the
 //              token's identity); the values are those of the product followed by gated_table_rows.

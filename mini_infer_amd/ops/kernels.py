@@ -434,7 +434,7 @@ def linear_f32_out(x: torch.Tensor, weight: torch.Tensor, scale: float = 1.0, sc
     logits do not depend on how many its step had.  Up to 256 rows of a large vocabulary: rounded the same from tiles, whose sums
     over K may be in another order with another number of rows (4e-5 from the library's in the 2-norm; 128256 x 3072 at 24 / 64 /
     256 rows 140 / 164 / 210 us against the vendor product and its cast's 166 / 192 / 307).
-    More rows: the vendor library's product, cast.  float32 operands: `gemm_f32`."""
+    More rows: `linear`, cast.  float32 operands: `gemm_f32`."""
     if x.dtype == torch.float32:
         logits = gemm_f32(x, weight)
         return logits if scale == 1.0 else logits.mul_(scale)
@@ -487,7 +487,7 @@ def partial_sums_pay(m: int, n: int, k: int) -> bool:
     takes them (`linear(..., partial_ok=True)`), in an order that depends on the matrix alone (`linear_partial_sums`; what this leaves
     aside above 16 rows `tiles_for` may still cut).  Measured on MI355X, the product alone with
     weights from memory, microseconds whole / in pieces (whole = `gemm_skinny_bf16` up to
-    16 rows, the vendor library above; in pieces = tiles):
+    16 rows, the vendor library above, with which these were measured; in pieces = tiles):
 
                                   8 rows     12 rows    16 rows    32 rows    64 rows
         4096 x 14336 (8B down)    22 / 20    25 / 20    28 / 20    31 / 21    39 / 24

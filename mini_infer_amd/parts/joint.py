@@ -12,8 +12,8 @@ both results are sums, the two last ones are one product with the matrices side 
 (the sum of the sublayers is then rounded once, not three times).  A layer is two products of
 twice the size with the mixer's own work between them: at few rows the weights of a whole layer stream
 through two launches, and the first of them ends with everything that follows it row by row
-(`ops.layer_in`).  For many rows the vendor library makes both products and the pieces of a very large one are
-faster apart, so a prompt takes the parts' own views of the stacked matrices where they are (`apart_in`,
+(`ops.layer_in`).  For many rows the pieces of a very large product were faster apart in the vendor library,
+which then made them all, so a prompt takes the parts' own views of the stacked matrices where they are (`apart_in`,
 `apart_out`).
 
 What a mixer that joins offers (`Mixer.can_join`): `joint_input` and `joint_output` (its first and

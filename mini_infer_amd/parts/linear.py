@@ -1,8 +1,8 @@
 """A bias-free linear map `y = x @ W.T` with W in [out, in] layout.
 
 The reference's linears are `F.linear` on the vendor BLAS
-(distributed/linear.py:6-14, :167).  Here bfloat16 of many rows uses the vendor GEMM too, fewer rows kernels of the
-engine's own (`ops.linear`), and float32 runs a hand-written true-float32 kernel.  Several checkpoint tensors can
+(distributed/linear.py:6-14, :167).  Here bfloat16 runs kernels of the engine's own, and the vendor GEMM where that is
+faster (`ops.linear`); float32 runs a hand-written true-float32 kernel.  Several checkpoint tensors can
 be stacked along the output axis at load (q|k|v, gate|up) so one product serves
 them all (distributed/linear.py:237-249 merges q, k, v the same way).
 """
