@@ -1,4 +1,4 @@
-// The kernel of gemm_tiles_bf16.hip and gemm_tiles_gated_bf16.hip, and the shapes that they compile it for.
+// The kernel of gemm_tiles_bf16.hip, gemm_tiles_gated_bf16.hip and gemm_tiles_rope_bf16.hip, and the shapes that they compile it for.
 #pragma once
 
 #include "gated_tile.h"
@@ -31,11 +31,26 @@ __host__ __device__ __forceinline__ KRange k_range(int k, int steps_each, int ra
   return {first, min(steps_each * 2, k / 32 - first)};
 }
 
+// Which rows of W stand beside one another in a tile: none, gate and up, or the two elements that are rotated together.
+enum { PAIRED_NOT = 0, PAIRED_GATED = 1, PAIRED_ROTARY = 2 };
+
+// (A type picked by comparing with one of those would put an unnamed enumeration into the kernel's symbol, which the compiler numbers otherwise for
+// the host than for the device: the kernel is then not found.)
+template <int PAIRED>
+struct PairedHow {
+  using type = GatedActivation;
+};
+template <>
+struct PairedHow<2> {
+  using type = RotaryWrite;
+};
+
 // (the second bound: two blocks a CU where LDS holds two)
-template <class T, bool GATED, bool ONCE, bool ODD>
+template <class T, int PAIRED, bool ONCE, bool ODD>
 __global__ __launch_bounds__(T::THREADS, T::RING * 4 <= 163840 ? 2 : 1) void gemm_tiles_kernel(
     const bf16_t* __restrict__ a, int64_t lda, const bf16_t* __restrict__ w, int64_t ldw, void* __restrict__ out, int64_t ldc,
-    int kind, float scale, const GatedActivation how, bool vec, int m, int n, int k, int steps_each, int row_tiles, int feature_tiles, int total) {
+    int kind, float scale, const typename PairedHow<PAIRED>::type how, bool vec, int m, int n, int k, int steps_each, int row_tiles, int feature_tiles,
+    int total) {
   __shared__ __align__(16) bf16_t ring[T::RING];
   // Consecutive places go to one XCD (workgroups are dealt to the 8 of them in turn): the row tiles that read the same
   // rows of W run at the same time behind one L2.
@@ -44,7 +59,7 @@ __global__ __launch_bounds__(T::THREADS, T::RING * 4 <= 163840 ? 2 : 1) void gem
   const int row_tile = place % row_tiles, rest = place / row_tiles;
   const int feature_tile = rest % feature_tiles, range = rest / feature_tiles;
   const KRange part = k_range(k, steps_each, range);
-  constexpr int FEATURES = GATED ? T::BN / 2 : T::BN;
+  constexpr int FEATURES = PAIRED != PAIRED_NOT ? T::BN / 2 : T::BN;
   const int r0 = row_tile * T::BM, f0 = feature_tile * FEATURES;
   a += part.first * 32;
   w += part.first * 32;
@@ -52,9 +67,14 @@ __global__ __launch_bounds__(T::THREADS, T::RING * 4 <= 163840 ? 2 : 1) void gem
   tile.template run<ONCE, ODD>(
       ring, part.halves, [&](int r) { return a + (int64_t)min(r0 + r, m - 1) * lda; },
       [&](int r) {
-        return w + (int64_t)(GATED ? GatedTile<T::NT>::row_of(r, f0, n) : min(f0 + r, n - 1)) * ldw;
+        if constexpr (PAIRED == PAIRED_ROTARY) return w + (int64_t)rotary_row_of(GatedTile<T::NT>::row_of(r, f0, n), n, how.head_dim) * ldw;
+        else return w + (int64_t)(PAIRED == PAIRED_GATED ? GatedTile<T::NT>::row_of(r, f0, n) : min(f0 + r, n - 1)) * ldw;
       });
-  if constexpr (GATED) {
+  if constexpr (PAIRED == PAIRED_ROTARY) {
+    tile.leave(ring);
+    write_rotated<GatedTile<T::NT>, T::BM, T::BN, T::MADE, T::THREADS>(ring, how, r0, m, f0, n);
+    return;
+  } else if constexpr (PAIRED == PAIRED_GATED) {
     tile.leave(ring);
 #define MI_WRITE(ACT) write_activated<ACT, GatedTile<T::NT>, T::BM, T::BN, T::MADE, T::THREADS>(ring, how, (bf16_t*)out, ldc, vec, r0, m, f0, n)
     if (kind == 4) MI_WRITE(ACT_CLAMPED);
@@ -104,18 +124,23 @@ struct GemmTilesLaunch {
   int kind;
   float scale;
   GatedActivation how;
+  RotaryWrite rotary;
   bool vec;
   int m, n, k, steps_each;
   hipStream_t stream;
 };
 
-template <class T, bool GATED, bool ODD>
+template <class T, int PAIRED, bool ODD>
 static void gemm_tiles_launch(const GemmTilesLaunch& l) {
-  const int row_tiles = ceil_div(l.m, T::BM), feature_tiles = ceil_div(l.n, GATED ? T::BN / 2 : T::BN);
+  const int row_tiles = ceil_div(l.m, T::BM), feature_tiles = ceil_div(l.n, PAIRED != PAIRED_NOT ? T::BN / 2 : T::BN);
   const int total = row_tiles * feature_tiles * ceil_div(ceil_div(l.k, 64), l.steps_each);
-  const auto kernel = row_tiles == 1 ? gemm_tiles_kernel<T, GATED, true, ODD> : gemm_tiles_kernel<T, GATED, false, ODD>;
+  const auto kernel = row_tiles == 1 ? gemm_tiles_kernel<T, PAIRED, true, ODD> : gemm_tiles_kernel<T, PAIRED, false, ODD>;
+  const auto& how = [&]() -> const auto& {
+    if constexpr (PAIRED == PAIRED_ROTARY) return l.rotary;
+    else return l.how;
+  }();
   kernel<<<ceil_div(total, 8) * 8, T::THREADS, 0, l.stream>>>((const bf16_t*)l.a, l.lda, (const bf16_t*)l.w, l.ldw, l.out, l.ldc, l.kind,
-                                                             l.scale, l.how, l.vec, l.m, l.n, l.k, l.steps_each, row_tiles, feature_tiles, total);
+                                                             l.scale, how, l.vec, l.m, l.n, l.k, l.steps_each, row_tiles, feature_tiles, total);
 }
 
 // gemm_tiles_gated_bf16.hip

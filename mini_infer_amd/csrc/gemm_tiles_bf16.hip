@@ -31,7 +31,7 @@ struct Shape {
 };
 template <class T, bool ODD = false>
 constexpr Shape shape() {
-  return {T::BM, T::BN, T::RING * 2, T::WK, gemm_tiles_launch<T, false, ODD>};
+  return {T::BM, T::BN, T::RING * 2, T::WK, gemm_tiles_launch<T, PAIRED_NOT, ODD>};
 }
 #define X(...) shape<TileProduct<__VA_ARGS__>>(),
 const Shape SHAPES[] = {GEMM_TILE_SHAPES(X)};
@@ -113,10 +113,10 @@ extern "C" int mi_gemm_tiles_bf16(int kind, const void* a, int64_t lda, const vo
   MI_REQUIRE(ceil_div(steps, each) == ranges, "gemm_tiles_bf16: %d steps of K do not make %d ranges", steps, ranges);
   const int element = kind == 1 || kind == 2 ? 4 : 2, at_once = kind >= 3 ? 8 : 4;
   const bool vec = (uintptr_t)out % (at_once * element) == 0 && (kind == 1 ? n : ldc) % at_once == 0;
-  const GemmTilesLaunch l = {a, w, out, lda, ldw, ldc, kind, scale, {bias, limit, slope}, vec, m, n, k, each, stream};
+  const GemmTilesLaunch l = {a, w, out, lda, ldw, ldc, kind, scale, {bias, limit, slope}, {}, vec, m, n, k, each, stream};
   const bool odd = k % 64 != 0;  // (one shape for these: nothing real is made so)
   if (kind >= 3) gemm_tiles_gated_launch(shape, odd, l);
-  else if (odd) gemm_tiles_launch<TileProduct<GEMM_TILE_ODD_SHAPE>, false, true>(l);
+  else if (odd) gemm_tiles_launch<TileProduct<GEMM_TILE_ODD_SHAPE>, PAIRED_NOT, true>(l);
   else SHAPES[shape].launch(l);
   MI_CHECK_LAUNCH("gemm_tiles_bf16");
   return MI_OK;

@@ -2,9 +2,9 @@
 #include "gemm_tiles.h"
 
 void gemm_tiles_gated_launch(int shape, bool odd, const GemmTilesLaunch& l) {
-#define X(...) gemm_tiles_launch<TileProduct<__VA_ARGS__>, true, false>,
+#define X(...) gemm_tiles_launch<TileProduct<__VA_ARGS__>, PAIRED_GATED, false>,
   static void (*const launches[])(const GemmTilesLaunch&) = {GEMM_TILE_SHAPES(X)};
 #undef X
-  if (odd) gemm_tiles_launch<TileProduct<GEMM_TILE_ODD_SHAPE>, true, true>(l);
+  if (odd) gemm_tiles_launch<TileProduct<GEMM_TILE_ODD_SHAPE>, PAIRED_GATED, true>(l);
   else launches[shape](l);
 }

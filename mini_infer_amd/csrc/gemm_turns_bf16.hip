@@ -22,9 +22,19 @@ struct TurnsPlan {
   int form, rest, cut, whole, places;
 };
 
+constexpr int ACT_ROTARY = 4;  // not an activation: [q | k | v] rotated and written (gated_tile.h)
+template <int ACT>
+struct TurnsHow {
+  using type = GatedActivation;
+};
+template <>
+struct TurnsHow<4> {
+  using type = RotaryWrite;
+};
+
 template <class T, int ACT>
 __device__ __forceinline__ void make_tile(bf16_t* ring, const bf16_t* __restrict__ a, int64_t lda, const bf16_t* __restrict__ w, int64_t ldw,
-                                          bf16_t* __restrict__ out, int64_t ldo, const GatedActivation& how, bool vec, int m, int n, int k, int r0,
+                                          bf16_t* __restrict__ out, int64_t ldo, const typename TurnsHow<ACT>::type& how, bool vec, int m, int n, int k, int r0,
                                           int feature_tile) {
   constexpr bool GATED = ACT != ACT_NONE;
   constexpr int FEATURES = GATED ? T::BN / 2 : T::BN;
@@ -33,9 +43,14 @@ __device__ __forceinline__ void make_tile(bf16_t* ring, const bf16_t* __restrict
   T tile;
   tile.run(
       ring, k / TURNS_K, [&](int r) { return a + (int64_t)min(r0 + r, m - 1) * lda; },
-      [&](int r) { return w + (int64_t)(GATED ? T::Pairs::row_of(r, f0, n) : min(f0 + r, n - 1)) * ldw; });
+      [&](int r) {
+        if constexpr (ACT == ACT_ROTARY) return w + (int64_t)rotary_row_of(HalvedTile<T::BN>::row_of(r, f0, n), n, how.head_dim) * ldw;
+        else return w + (int64_t)(GATED ? T::Pairs::row_of(r, f0, n) : min(f0 + r, n - 1)) * ldw;
+      });
   tile.leave(ring, [](float sum, int) { return sum; });
-  if constexpr (GATED) {
+  if constexpr (ACT == ACT_ROTARY) {
+    write_rotated<HalvedTile<T::BN>, T::BM, T::BN, T::MADE, T::THREADS>(ring, how, r0, m, f0, n);
+  } else if constexpr (GATED) {
     write_activated<ACT, typename T::Pairs, T::BM, T::BN, T::MADE, T::THREADS>(ring, how, out, ldo, vec, r0, m, f0, n);
   } else {
     constexpr int CHUNKS = FEATURES / 8;
@@ -51,7 +66,7 @@ __device__ __forceinline__ void make_tile(bf16_t* ring, const bf16_t* __restrict
 
 template <int ACT>
 __global__ __launch_bounds__(512, 2) void gemm_turns_kernel(const bf16_t* __restrict__ a, int64_t lda, const bf16_t* __restrict__ w, int64_t ldw,
-                                                            bf16_t* __restrict__ out, int64_t ldo, const GatedActivation how, bool vec, int m, int n, int k,
+                                                            bf16_t* __restrict__ out, int64_t ldo, const typename TurnsHow<ACT>::type how, bool vec, int m, int n, int k,
                                                             int row_tiles, int feature_tiles, const TurnsPlan plan) {
   __shared__ __align__(16) bf16_t ring[TURNS_RING];
   // (workgroups are dealt to the XCDs in turn)
@@ -67,7 +82,7 @@ __global__ __launch_bounds__(512, 2) void gemm_turns_kernel(const bf16_t* __rest
   const int form = cut ? plan.rest : plan.form;
   const int r0 = (band * BAND + rest % in_band) * turns_form(plan.form).rows + (cut ? behind % plan.cut * turns_form(plan.rest).rows : 0);
 #define X(I, ROWS, FEATURES, CAN_GATE, ...)                                                                                        \
-  if constexpr (ACT == ACT_NONE || CAN_GATE) {                                                                                     \
+  if constexpr (ACT == ACT_NONE || ACT == ACT_ROTARY || CAN_GATE) {                                                                             \
     if (form == I) make_tile<TurnsOf<I>::type, ACT>(ring, a, lda, w, ldw, out, ldo, how, vec, m, n, k, r0, rest / in_band);         \
   }
   TURNS_FORMS_OF(X)
@@ -139,5 +154,26 @@ extern "C" int mi_gemm_turns_bf16(int act, const void* a, int64_t lda, const voi
   else MI_LAUNCH(ACT_GELU);
 #undef MI_LAUNCH
   MI_CHECK_LAUNCH("gemm_turns_bf16");
+  return MI_OK;
+}
+
+// [q | k | v] rotated and written where it belongs in the last step; only: as above.
+extern "C" int mi_gemm_turns_rope(const void* a, int64_t lda, const void* w, int64_t ldw, void* q, int64_t ldq, const float* cos_t, const float* sin_t,
+                                  const int* slots, void* k_pages, void* v_pages, int m, int k, int q_heads, int kv_heads, int head_dim, int page_size,
+                                  int num_pages, int v_transposed, int only, hipStream_t stream) {
+  const RotaryWrite how = {cos_t, sin_t, slots, (bf16_t*)q, (bf16_t*)k_pages, (bf16_t*)v_pages, ldq, q_heads, kv_heads, head_dim, page_size, v_transposed};
+  MI_REQUIRE(rotary_write_fits(how, m, num_pages), "gemm_turns_rope: m=%d, %d + 2 * %d heads of %d, pages of %d", m, q_heads, kv_heads, head_dim, page_size);
+  MI_REQUIRE(k >= TURNS_K && k % TURNS_K == 0 && lda >= k && ldw >= k && lda % 8 == 0 && ldw % 8 == 0 && ((uintptr_t)a | (uintptr_t)w) % 16 == 0,
+             "gemm_turns_rope: takes K a multiple of 64 and rows on 16 bytes; got k=%d lda=%lld ldw=%lld", k, (long long)lda, (long long)ldw);
+  const int pairs = (q_heads + 2 * kv_heads) * (head_dim / 2);
+  MI_REQUIRE((int64_t)ceil_div(m, 64) * ceil_div(pairs, 64) < (1 << 27), "gemm_turns_rope: too many tiles");
+  MI_REQUIRE(only >= -1 && only < TURNS_FORMS, "gemm_turns_rope: form %d", only);
+  double micros;
+  const TurnsPlan plan = turns_plan(m, 2 * pairs, k, false, only, max(8, mi_compute_units()), &micros);
+  const TurnsForm form = turns_form(plan.form);
+  const int blocks = 8 * (plan.whole + (plan.places - plan.whole) * plan.cut);
+  gemm_turns_kernel<ACT_ROTARY><<<blocks, 512, 0, stream>>>((const bf16_t*)a, lda, (const bf16_t*)w, ldw, nullptr, 0, how, true, m, pairs, k,
+                                                            ceil_div(m, form.rows), ceil_div(pairs, form.features / 2), plan);
+  MI_CHECK_LAUNCH("gemm_turns_rope");
   return MI_OK;
 }

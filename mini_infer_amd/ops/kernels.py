@@ -868,6 +868,67 @@ def qkv_rope_write(
     return q_out
 
 
+def qkv_rope_write_many_plan(x: torch.Tensor, weight: torch.Tensor, head_dim: int, rotary_dim: int, interleaved: bool, steady: bool = False,
+                             in_pieces: bool = False, others: tuple[torch.Tensor | None, ...] = ()) -> int | None:
+    """How `qkv_rope_write_many` makes this product of many bfloat16 rows: the shape of its tiles, -1 for those of `gemm_turns_bf16`, or
+    None where `linear` with the same options does not make it in whole tiles, whose sums and so results these are; whole heads of a multiple of 16
+    rotated in half pairing.  Faster by the rotation's launch at every size measured (csrc/gated_tile.h: 33 to 2,048 rows; drawn steps of 3B and
+    8B sizes 1.01 to 1.04), so there is no other line.  `others`: the tensors that it reads and writes beside these, which have to lie on 16 bytes."""
+    if any(t is not None and t.data_ptr() % 16 != 0 for t in others):
+        return None
+    if not isinstance(x, torch.Tensor) or interleaved or rotary_dim != head_dim or head_dim % 16 != 0 or not _rows_of_bf16(x, weight) or x.shape[1] % 64 != 0:
+        return None
+    m, n, k = x.shape[0], weight.shape[0], x.shape[1]
+    if _turns_take(x, weight):
+        return -1
+    if steady or in_pieces or m <= SKINNY_WIDE_MAX_ROWS:
+        return None
+    plan = tiles_for(m, n, k, False, _compute_units(x.device))
+    return plan[0] if plan is not None and plan[1] == 1 else None
+
+
+def qkv_rope_write_many(
+    x: torch.Tensor, weight: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, slot_mapping: torch.Tensor | None,
+    k_pages: torch.Tensor | None, v_pages: torch.Tensor | None, *, q_heads: int, kv_heads: int, head_dim: int, v_transposed: bool = False,
+    plan: int,
+) -> torch.Tensor:
+    """`qkv_rope_write` for many rows, `plan` from `qkv_rope_write_many_plan`: `linear` and `rope_kv_write` as one kernel of tiles
+    (csrc/gated_tile.h); returns the rotated queries."""
+    _need_cuda(x, weight, cos, sin, slot_mapping, k_pages, v_pages)
+    for name, t in (("cos", cos), ("sin", sin), ("slot_mapping", slot_mapping), ("k_pages", k_pages), ("v_pages", v_pages)):
+        _need_contiguous(name, t)
+    _need_int32("slot_mapping", slot_mapping)
+    if not _rows_of_bf16(x, weight):
+        raise KernelShapeError(f"qkv_rope_write_many takes bfloat16 rows on 16 bytes, got x {tuple(x.shape)} {x.dtype} and weight {tuple(weight.shape)}")
+    m, k = x.shape
+    if weight.shape != ((q_heads + 2 * kv_heads) * head_dim, k):
+        raise KernelShapeError(f"qkv_rope_write_many: weight {tuple(weight.shape)} does not fit (q+2kv)*head_dim x {k}")
+    if cos.shape != (m, head_dim // 2) or sin.shape != cos.shape or cos.dtype != torch.float32 or sin.dtype != torch.float32:
+        raise KernelShapeError(f"cos/sin must be float32 [{m}, {head_dim // 2}], got {tuple(cos.shape)} {cos.dtype}")
+    page_size = num_pages = 0
+    if kv_heads > 0:
+        if slot_mapping is None or k_pages is None or v_pages is None:
+            raise KernelShapeError("writing keys and values needs slot_mapping, k_pages and v_pages")
+        if k_pages.dtype != torch.bfloat16 or v_pages.dtype != torch.bfloat16:
+            raise KernelShapeError("qkv_rope_write_many writes bfloat16 pages")
+        if k_pages.dim() != 4 or k_pages.shape[1] != kv_heads or k_pages.shape[3] != head_dim:
+            raise KernelShapeError(f"k_pages must be [num_pages, {kv_heads}, page_size, {head_dim}], got {tuple(k_pages.shape)}")
+        _check_v_pages(k_pages, v_pages, v_transposed)
+        if slot_mapping.numel() != m:
+            raise KernelShapeError("slot_mapping needs one entry per row")
+        num_pages, page_size = k_pages.shape[0], k_pages.shape[2]
+    q_out = torch.empty((m, q_heads * head_dim), dtype=torch.bfloat16, device=x.device)
+    lib = library.load()
+    pages = (_ptr(slot_mapping), _ptr(k_pages), _ptr(v_pages)) if kv_heads > 0 else (None, None, None)
+    library.check(
+        (lib.mi_gemm_turns_rope if plan < 0 else lib.mi_gemm_tiles_rope)(
+            _ptr(x), x.stride(0), _ptr(weight), weight.stride(0), _ptr(q_out), q_out.stride(0), _ptr(cos), _ptr(sin), *pages, m, k, q_heads,
+            kv_heads, head_dim, page_size, num_pages, int(v_transposed), plan, _stream(),
+        )
+    )
+    return q_out
+
+
 def linear_swiglu(x: "torch.Tensor | ScaledRows", gate_up_weight: torch.Tensor, steady: bool = False) -> torch.Tensor:
     """`silu(x @ gate.T) * (x @ up.T)` with `gate_up_weight` = [gate; up] stacked, [2I, K].
 

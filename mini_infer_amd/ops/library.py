@@ -14,7 +14,7 @@ from pathlib import Path
 from mini_infer_amd.exceptions import ExtensionMissingError, KernelShapeError
 from mini_infer_amd.ops import build as _build
 
-ABI_VERSION = 51
+ABI_VERSION = 52
 
 _lib: ctypes.CDLL | None = None
 _lib_path: Path | None = None
@@ -192,6 +192,12 @@ _SIGNATURES: dict[str, list] = {
     "mi_gemm_turns_gated": [c_int],
     "mi_gemm_turns_bf16": [
         c_int, _P, c_int64, _P, c_int64, _P, c_float, c_float, _P, c_int64, c_int, c_int, c_int, c_int, _P,
+    ],
+    "mi_gemm_tiles_rope": [
+        _P, c_int64, _P, c_int64, _P, c_int64, _P, _P, _P, _P, _P, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, _P,
+    ],
+    "mi_gemm_turns_rope": [
+        _P, c_int64, _P, c_int64, _P, c_int64, _P, _P, _P, _P, _P, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, _P,
     ],
     "mi_expert_tiles_cut": [_P, c_int, c_int, c_int, c_int, _P],
     "mi_expert_plan_words": [c_int, c_int],

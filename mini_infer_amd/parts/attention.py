@@ -287,6 +287,20 @@ class GQAttention(Mixer):
                 v_transposed=cache.v_transposed,
             )
             return self._project(self._attend(queries, ctx, cache))
+        # many rows: the same in tiles, where the projection alone would be whole tiles
+        many = None
+        if as_one and self.dtype == torch.bfloat16:
+            single = ctx.max_q_len == 1 and writes_cache
+            weight = self.qkv.weight if writes_cache else self.qkv.weight[:q_width]
+            many = ops.qkv_rope_write_many_plan(x, weight, self.head_dim, rotary.rotary_dim, rotary.interleaved, self.steady, single,
+                                                (rotary.cos, rotary.sin, cache.k_pages, cache.v_pages))
+        if many is not None:
+            queries = ops.qkv_rope_write_many(
+                x, weight, rotary.cos, rotary.sin, ctx.slot_mapping[cache.group] if writes_cache else None, cache.k_pages, cache.v_pages,
+                q_heads=self.num_heads, kv_heads=self.num_kv_heads if writes_cache else 0, head_dim=self.head_dim,
+                v_transposed=cache.v_transposed, plan=many,
+            )
+            return self._project(self._attend(queries, ctx, cache))
         if writes_cache:
             # A projection left in pieces is added up by the rotation's launch, in steps of single tokens: 8B sizes, 40 of them,
             # 4,574 -> 4,494 us a step.  A portion's values are written a page at a time, sixteen tokens a thread, and all their

@@ -1719,3 +1719,73 @@ def test_float32_rows_projected_rotated_and_written_as_one(m, hidden, heads, kv_
     torch.testing.assert_close(ops.qkv_rope_write_f32(rows, w, cos, sin, *where[2], **names), apart, **near)
     for ours, theirs in zip(caches[2], caches[0]):
         torch.testing.assert_close(ours, theirs, **near)
+
+
+@pytest.mark.parametrize("m,hidden,heads,kv_heads,head_dim,page", [
+    (33, 3072, 24, 8, 128, 16), (271, 3072, 24, 8, 128, 16), (97, 2048, 6, 1, 96, 8), (350, 256, 6, 2, 64, 16), (1030, 128, 3, 3, 32, 32),
+    (513, 64, 5, 1, 16, 12), (700, 128, 4, 0, 48, 16), (321, 192, 2, 2, 256, 4),
+])
+@pytest.mark.parametrize("transposed", [False, True])
+def test_many_rows_projected_rotated_and_written_as_one(m, hidden, heads, kv_heads, head_dim, page, transposed):
+    """In every tile that the kernel may take, against the same tile's plain product and `rope_kv_write`: the same bits, but where a rotation's two
+    products are fused differently, which may round the last bit of a bfloat16 the other way."""
+    from mini_infer_amd import ops
+    from mini_infer_amd.exceptions import KernelShapeError
+    from mini_infer_amd.ops import kernels, library
+
+    torch.manual_seed(m + hidden)
+    x = torch.randn(m, hidden, device="cuda").bfloat16()
+    n = (heads + 2 * kv_heads) * head_dim
+    w = (torch.randn(n, hidden, device="cuda") / hidden ** 0.5).bfloat16()
+    angle = torch.rand(m, head_dim // 2, device="cuda") * 6
+    cos, sin = angle.cos(), angle.sin()
+    # single slots, rows that are not written, a run from the middle of a page on and one that begins a page
+    pages = 2 * (m // page) + 20
+    free = torch.randperm(9 * page)[:9].tolist()
+    run = list(range(10 * page + 5, 10 * page + 5 + (m - 11) // 2))
+    slots = free + [-1, -1] + run
+    begin = (slots[-1] // page + 2) * page
+    slots = torch.tensor(slots + list(range(begin, begin + m - len(slots))), dtype=torch.int32, device="cuda")
+    assert slots.max() < pages * page and slots.unique().numel() == m - 1
+    sizes = (pages, max(kv_heads, 1), page, head_dim)
+    names = dict(q_heads=heads, kv_heads=kv_heads, head_dim=head_dim, v_transposed=transposed)
+
+    def caches():
+        return [torch.zeros(sizes, device="cuda", dtype=torch.bfloat16),
+                torch.zeros(sizes[:2] + (head_dim, page) if transposed else sizes, device="cuda", dtype=torch.bfloat16)]
+
+    def check(product, plan, form=-1):
+        theirs, ours = caches(), caches()
+        where = [(slots, *c) if kv_heads else (None, None, None) for c in (theirs, ours)]
+        apart = ops.rope_kv_write(product, cos, sin, *where[0], rotary_dim=head_dim, **names)[:, : heads * head_dim]
+        if form < 0:
+            one = ops.qkv_rope_write_many(x, w, cos, sin, *where[1], plan=plan, **names)
+        else:  # all tiles of that form
+            one = torch.empty(m, heads * head_dim, dtype=torch.bfloat16, device="cuda")
+            pointers = [None if t is None else t.data_ptr() for t in where[1]]
+            library.check(library.load().mi_gemm_turns_rope(
+                x.data_ptr(), x.stride(0), w.data_ptr(), w.stride(0), one.data_ptr(), one.stride(0), cos.data_ptr(), sin.data_ptr(), *pointers, m, hidden,
+                heads, kv_heads, head_dim, page, pages, int(transposed), form, torch.cuda.current_stream().cuda_stream))
+        torch.testing.assert_close(one, apart, rtol=2.0**-7, atol=2.0**-22 * 8)
+        assert (one != apart).float().mean() < 1e-3
+        torch.testing.assert_close(ours[0], theirs[0], rtol=2.0**-7, atol=2.0**-22 * 8)
+        assert torch.equal(ours[1], theirs[1])
+
+    if m > 320:
+        form = 0
+        while library.load().mi_gemm_turns_rows(form):
+            check(kernels._turns(0, x, w, n), -1, form)
+            form += 1
+    else:
+        shape = 0
+        while kernels.tile_size(shape)[0]:
+            plain = kernels._tiles(0, x, w, torch.empty((m, n), dtype=torch.bfloat16, device="cuda"), n, shape, 1)
+            check(plain, shape)
+            shape += 1
+    plan = ops.qkv_rope_write_many_plan(x, w, head_dim, head_dim, False)
+    if plan is not None:
+        check(ops.linear(x, w), plan)
+    with pytest.raises(KernelShapeError):
+        ops.qkv_rope_write_many(x[:, ::2], w[:, ::2], cos, sin, None, None, None, plan=-1, **names)
+    assert ops.qkv_rope_write_many_plan(x, w, head_dim, head_dim, True) is None
+    assert ops.qkv_rope_write_many_plan(x.float(), w.float(), head_dim, head_dim, False) is None
