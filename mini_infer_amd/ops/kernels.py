@@ -871,9 +871,19 @@ def qkv_rope_write(
 def qkv_rope_write_many_plan(x: torch.Tensor, weight: torch.Tensor, head_dim: int, rotary_dim: int, interleaved: bool, steady: bool = False,
                              in_pieces: bool = False, others: tuple[torch.Tensor | None, ...] = ()) -> int | None:
     """How `qkv_rope_write_many` makes this product of many bfloat16 rows: the shape of its tiles, -1 for those of `gemm_turns_bf16`, or
-    None where `linear` with the same options does not make it in whole tiles, whose sums and so results these are; whole heads of a multiple of 16
-    rotated in half pairing.  Faster by the rotation's launch at every size measured (csrc/gated_tile.h: 33 to 2,048 rows; drawn steps of 3B and
-    8B sizes 1.01 to 1.04), so there is no other line.  `others`: the tensors that it reads and writes beside these, which have to lie on 16 bytes."""
+    None: left to `linear` and `rope_kv_write`.  Whole heads of a multiple of 16, rotated in half pairing.  `others`: the tensors that it reads and
+    writes beside these, which have to lie on 16 bytes.
+
+    Where `linear` makes whole tiles these are they, with the same results.  Microseconds of the two launches / this one, weights from memory:
+
+        rows                100            200            271            330            1000           2048           8192
+        3072 x 2048         16.3 / 10.5    17.3 / 12.3    18.1 / 13.3    20.7 / 15.9    26.4 / 21.2    35.3 / 29.3    103 / 86
+        5120 x 3072         21.0 / 16.3    24.1 / 19.6    26.9 / 22.4    27.4 / 22.5    45.0 / 40.3    69.8 / 64.7    217 / 194
+        6144 x 4096         25.0 / 20.8    32.1 / 27.0    33.6 / 28.7    39.7 / 34.6    58.3 / 52.6    90.4 / 83.8    308 / 283
+        10240 x 8192        44.5 / 57.0    64.1 / 62.7    74.5 / 67.4    78.2 / 73.5    153 / 147      284 / 274      949 / 895
+
+    Up to 320 rows whole tiles are taken too where the library makes the product (3072 x 2048 above; 2304 x 768 11.3 to 13.3 / 6.3 to 8.3,
+    5120 x 3072 at 300 rows 27.1 / 25.4), as they lose less to it than the rotation's launch takes, but not where `linear` cuts K: 10240 x 8192 at 100 rows."""
     if any(t is not None and t.data_ptr() % 16 != 0 for t in others):
         return None
     if not isinstance(x, torch.Tensor) or interleaved or rotary_dim != head_dim or head_dim % 16 != 0 or not _rows_of_bf16(x, weight) or x.shape[1] % 64 != 0:
@@ -883,7 +893,10 @@ def qkv_rope_write_many_plan(x: torch.Tensor, weight: torch.Tensor, head_dim: in
         return -1
     if steady or in_pieces or m <= SKINNY_WIDE_MAX_ROWS:
         return None
-    plan = tiles_for(m, n, k, False, _compute_units(x.device))
+    cus = _compute_units(x.device)
+    plan = tiles_for(m, n, k, False, cus)
+    if plan is None and m < TURNS_MIN_ROWS and n < 16000:
+        return _tiles_plan(m, n, k, False, 1, False, 0.0, 0.0, cus)[1]
     return plan[0] if plan is not None and plan[1] == 1 else None
 
 

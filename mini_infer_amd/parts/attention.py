@@ -287,7 +287,7 @@ class GQAttention(Mixer):
                 v_transposed=cache.v_transposed,
             )
             return self._project(self._attend(queries, ctx, cache))
-        # many rows: the same in tiles, where the projection alone would be whole tiles
+        # many rows: the same in tiles
         many = None
         if as_one and self.dtype == torch.bfloat16:
             single = ctx.max_q_len == 1 and writes_cache
