@@ -256,6 +256,13 @@ __device__ __forceinline__ void mi_take_flagged(int64_t total, F flagged, G take
   }
 }
 
+// The two elements of a head that are rotated together.  Each is one product, rounded, and one fused multiply-add; which of an element's two products
+// is rounded shows in its last bit, and left to the compiler that differed from kernel to kernel.
+__device__ __forceinline__ void mi_rotate(float x0, float x1, float c, float s, float& y0, float& y1) {
+  y0 = __builtin_fmaf(x0, c, -(x1 * s));
+  y1 = __builtin_fmaf(x1, c, x0 * s);
+}
+
 static __host__ __device__ inline int ceil_div(int a, int b) { return (a + b - 1) / b; }
 static inline int64_t ceil_div64(int64_t a, int64_t b) { return (a + b - 1) / b; }
 

@@ -455,8 +455,10 @@ __global__ __launch_bounds__(256) void rope_kv_write_kernel(
     const int i1 = interleaved ? 2 * j + 1 : j + half;
     T* x = row + h * head_dim;
     const float x0 = biased(x, h * head_dim, i0), x1 = biased(x, h * head_dim, i1);
-    x[i0] = from_f32<T>(x0 * c[j] - x1 * s[j]);
-    x[i1] = from_f32<T>(x1 * c[j] + x0 * s[j]);
+    float y0, y1;
+    mi_rotate(x0, x1, c[j], s[j], y0, y1);
+    x[i0] = from_f32<T>(y0);
+    x[i1] = from_f32<T>(y1);
   }
   const int pass = head_dim - rotary_dim;
   if (bias) {  // (without one the dims that are not rotated stay as they are)
@@ -482,8 +484,10 @@ __global__ __launch_bounds__(256) void rope_kv_write_kernel(
     const T* x = k_row + h * head_dim;
     T* dst = k_pages + (((int64_t)page * kv_heads + h) * page_size + off) * head_dim;
     const float x0 = biased(x, k_col + h * head_dim, i0), x1 = biased(x, k_col + h * head_dim, i1);
-    dst[i0] = from_f32<T>(x0 * c[j] - x1 * s[j]);
-    dst[i1] = from_f32<T>(x1 * c[j] + x0 * s[j]);
+    float y0, y1;
+    mi_rotate(x0, x1, c[j], s[j], y0, y1);
+    dst[i0] = from_f32<T>(y0);
+    dst[i1] = from_f32<T>(y1);
   }
   for (int e = first; e < kv_heads * pass; e += stride) {
     const int h = e / pass, d = rotary_dim + e % pass;
@@ -553,10 +557,7 @@ __global__ __launch_bounds__(256) void rope_kv_write_vec4_kernel(
     load4(c + j, cj);
     load4(s + j, sj);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      lo[i] = x0[i] * cj[i] - x1[i] * sj[i];
-      hi[i] = x1[i] * cj[i] + x0[i] * sj[i];
-    }
+    for (int i = 0; i < 4; ++i) mi_rotate(x0[i], x1[i], cj[i], sj[i], lo[i], hi[i]);
   };
 
   for (int e = first; e < q_heads * half4; e += stride) {

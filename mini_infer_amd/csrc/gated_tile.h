@@ -145,10 +145,7 @@ __device__ __forceinline__ void write_rotated(const bf16_t* made, const RotaryWr
         *reinterpret_cast<float4*>(s + e) = *reinterpret_cast<const float4*>(how.sin + (int64_t)t * half + j + e);
       }
 #pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        lo[e] = x0[e] * c[e] - x1[e] * s[e];
-        hi[e] = x1[e] * c[e] + x0[e] * s[e];
-      }
+      for (int e = 0; e < 8; ++e) mi_rotate(x0[e], x1[e], c[e], s[e], lo[e], hi[e]);
       mi_store_8(dst, j, how.head_dim, true, lo);
       mi_store_8(dst, j + half, how.head_dim, true, hi);
     } else {

@@ -457,8 +457,7 @@ __global__ __launch_bounds__(SEGMENTS * MI_WAVE) void gemm_f32_few_kernel(const 
         float y0 = x0, y1 = x1;
         if (!is_value) {
           const float cj = with.cos_t[(int64_t)row * half_dim + d], sj = with.sin_t[(int64_t)row * half_dim + d];
-          y0 = x0 * cj - x1 * sj;
-          y1 = x1 * cj + x0 * sj;
+          mi_rotate(x0, x1, cj, sj, y0, y1);
         }
         if (rope_head < with.q_heads) {
           to[0] = y0;
