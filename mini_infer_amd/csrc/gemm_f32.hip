@@ -312,30 +312,26 @@ __global__ __launch_bounds__(SEGMENTS * MI_WAVE) void gemm_f32_rows_kernel(const
 // silu(gate) * up is written, both products rounded to float32 first, as silu_mul takes them (the same bits, a launch less: 1B with 3 requests
 // decoding 1,688 -> 1,658 us a step).
 //
-// What a step of few rows launched beside its products cost it more than the products' own ends: 1B with 3 requests, 4.6 us a norm, a
-// rotation with the cache write, 16 layers of 2 and 1.  So the product behind which a norm stands adds its rows to the residual itself
-// (FEW_ADD), the product behind the norm applies it (NORMED), and q|k|v are rotated and written where they belong (FEW_ROPE; a block holds 8
-// features of the first half of a head and the 8 that they are turned with).  Every block brings whole rows into LDS anyway: on
-// the way they are multiplied with the norm's weight (rounded to float32 once, as by the norm's own launch) and their squares added up in
-// 64 bits, and the rows' factors meet the 64-bit sums at the end.
-enum { FEW_PLAIN = 0, FEW_GATED = 1, FEW_ROPE = 2, FEW_ADD = 3 };
+// FEW_ROPE: q|k|v, rotated and written where they belong; a block holds 8 features of the first half of a head and the 8 that they are turned with.
+// 1B with 3 requests decoding 1,656 -> 1,619 us a step.  (With the norms in the products around them too, their factors applied to the 64-bit sums,
+// 1,571, but that rounds elsewhere than the norm's launch in front of more rows: a request's logits changed when a fifth one joined.  The
+// factor first, its sum in the order of that launch, has every block add up all rows' squares: o, norm and gate|up of 3 rows at those sizes 33.6 ->
+// 38.6 us.)
+enum { FEW_PLAIN = 0, FEW_GATED = 1, FEW_ROPE = 2 };
 
-struct FewRows {  // what a kind has beside the product (see the entries)
-  const float* norm_weight;  // NORMED: [k]
-  float eps;
-  const float *cos_t, *sin_t;  // FEW_ROPE: [m][half]
+struct FewRows {  // what FEW_ROPE has beside the product (see the entry)
+  const float *cos_t, *sin_t;  // [m][half]
   const int* slots;
   float *k_pages, *v_pages;
   int q_heads, kv_heads, head_dim, page_size, v_transposed;
 };
 
-template <int G, int FEATURES, int KIND = FEW_PLAIN, bool NORMED = false>
+template <int G, int FEATURES, int KIND = FEW_PLAIN>
 __global__ __launch_bounds__(SEGMENTS * MI_WAVE) void gemm_f32_few_kernel(const float* __restrict__ a, int64_t lda,
                                                            const float* __restrict__ w, int64_t ldw,
                                                            float* __restrict__ c, int64_t ldc, int m, int n, int k, int chunk, FewRows with) {
   extern __shared__ __attribute__((aligned(16))) float4 staged[];  // [wave][slice of the chunk][group of rows][half][piece of K][row]
   __shared__ double sums[SEGMENTS][G][MI_WAVE];
-  __shared__ double squares[NORMED ? SEGMENTS : 1][4 * G];
   constexpr int AHEAD = G == 1 ? 4 : 2;
   constexpr bool PAIRED = KIND == FEW_GATED || KIND == FEW_ROPE;  // the operand's upper 8 features belong to its lower 8
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / MI_WAVE), lane = threadIdx.x % MI_WAVE;
@@ -354,34 +350,20 @@ __global__ __launch_bounds__(SEGMENTS * MI_WAVE) void gemm_f32_few_kernel(const 
   const int row = wave * 4 + lane / 16, f = lane % 16;  // (the instruction's result: row lane / 16, feature lane % 16)
   const bool written = wave < G && row < m && f < (PAIRED ? 8 : FEATURES) && f <= most;
   float* const to = c + (int64_t)row * ldc + col0 + f;
-  float residual = 0.f;
-  if constexpr (KIND == FEW_ADD) {
-    if (written) residual = *to;
-  }
   bf16x8_t lo[AHEAD], hi[AHEAD];  // 16-byte pieces; what they hold is float32
   auto fetch = [&](int slot, int slice) {
     if constexpr (FEATURES == 8) lo[slot] = load_line(w_block, 2 * (int64_t)slice, lower);
     else load_line_pair(w_block, 2 * (int64_t)slice, lower, upper, lo[slot], hi[slot]);
   };
   float4* mine = staged + wave * chunk * (32 * G);
-  double square[G];
-#pragma unroll
-  for (int g = 0; g < G; ++g) square[g] = 0.0;
   auto stage = [&](int from, int upto) {
     const int piece = lane % 16, row = lane / 16;  // two slices a load
     for (int s = from; s < upto; s += 2) {
       if (s + piece / 8 < upto) {
-        float4 by;
-        if constexpr (NORMED) by = *reinterpret_cast<const float4*>(with.norm_weight + (int64_t)s * SLICE + piece * 4);
 #pragma unroll
-        for (int g = 0; g < G; ++g) {
-          float4 x = *reinterpret_cast<const float4*>(a + (int64_t)min(g * 4 + row, m - 1) * lda + (int64_t)s * SLICE + piece * 4);
-          if constexpr (NORMED) {
-            square[g] += (double)x.x * (double)x.x + (double)x.y * (double)x.y + ((double)x.z * (double)x.z + (double)x.w * (double)x.w);
-            x = float4{by.x * x.x, by.y * x.y, by.z * x.z, by.w * x.w};
-          }
-          mine[((s - from + piece / 8) * G + g) * 32 + piece % 8 * 4 + row] = x;
-        }
+        for (int g = 0; g < G; ++g)
+          mine[((s - from + piece / 8) * G + g) * 32 + piece % 8 * 4 + row] =
+              *reinterpret_cast<const float4*>(a + (int64_t)min(g * 4 + row, m - 1) * lda + (int64_t)s * SLICE + piece * 4);
       }
     }
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");  // (nobody else reads them: no barrier)
@@ -427,25 +409,11 @@ __global__ __launch_bounds__(SEGMENTS * MI_WAVE) void gemm_f32_few_kernel(const 
   }
 #pragma unroll
   for (int g = 0; g < G; ++g) sums[wave][g][lane] = acc[g];
-  if constexpr (NORMED) {
-#pragma unroll
-    for (int g = 0; g < G; ++g) {
-#pragma unroll
-      for (int off = 8; off > 0; off >>= 1) square[g] += __shfl_xor(square[g], off, MI_WAVE);
-      if (lane % 16 == 0) squares[wave][g * 4 + lane / 16] = square[g];
-    }
-  }
   __syncthreads();
   if (wave < G) {
     double total = 0.0;
 #pragma unroll
     for (int s = 0; s < SEGMENTS; ++s) total += sums[s][wave][lane];
-    if constexpr (NORMED) {
-      double all = 0.0;
-#pragma unroll
-      for (int s = 0; s < SEGMENTS; ++s) all += squares[s][row];
-      total *= 1.0 / sqrt(all / (double)k + (double)with.eps);
-    }
     if constexpr (KIND == FEW_GATED) {
       const float up = __shfl_down((float)total, 8, MI_WAVE);
       if (written) *to = silu_times<float>((float)total, up);
@@ -475,8 +443,6 @@ __global__ __launch_bounds__(SEGMENTS * MI_WAVE) void gemm_f32_few_kernel(const 
           }
         }
       }
-    } else if constexpr (KIND == FEW_ADD) {
-      if (written) *to = residual + (float)total;
     } else {
       if (written) *to = (float)total;
     }
@@ -491,21 +457,20 @@ static void launch_tiles(const float* a, int64_t lda, const float* w, int64_t ld
   else gemm_f32_kernel<BM, STAGE, false><<<grid, 256, 0, stream>>>(a, lda, w, ldw, c, ldc, m, n, k);
 }
 
-template <int G, int FEATURES, int KIND = FEW_PLAIN, bool NORMED = false>
+template <int G, int FEATURES, int KIND = FEW_PLAIN>
 static void launch_few(const float* a, int64_t lda, const float* w, int64_t ldw, float* c, int64_t ldc, int m, int n, int k,
                        hipStream_t stream, const FewRows& with = FewRows()) {
   const int chunk = min(segment_slices(k), 16 / G);
   const int blocks = KIND == FEW_ROPE ? (with.q_heads + 2 * with.kv_heads) * (with.head_dim / 16) : ceil_div(n, KIND == FEW_GATED ? 8 : FEATURES);
-  gemm_f32_few_kernel<G, FEATURES, KIND, NORMED><<<blocks, SEGMENTS * MI_WAVE, SEGMENTS * chunk * G * 32 * sizeof(float4), stream>>>(
+  gemm_f32_few_kernel<G, FEATURES, KIND><<<blocks, SEGMENTS * MI_WAVE, SEGMENTS * chunk * G * 32 * sizeof(float4), stream>>>(
       a, lda, w, ldw, c, ldc, m, n, k, chunk, with);
 }
 
-// A launch of a kind for one or two groups of four rows, or for one whose norm is to be applied.
+// A launch of a kind for one or two groups of four rows.
 template <int FEATURES, int KIND>
 static void launch_few_of(const float* a, int64_t lda, const float* w, int64_t ldw, float* c, int64_t ldc, int m, int n, int k,
-                          hipStream_t stream, const FewRows& with) {
-  if (with.norm_weight) launch_few<1, FEATURES, KIND, true>(a, lda, w, ldw, c, ldc, m, n, k, stream, with);
-  else if (m > 4) launch_few<2, FEATURES, KIND>(a, lda, w, ldw, c, ldc, m, n, k, stream, with);
+                          hipStream_t stream, const FewRows& with = FewRows()) {
+  if (m > 4) launch_few<2, FEATURES, KIND>(a, lda, w, ldw, c, ldc, m, n, k, stream, with);
   else launch_few<1, FEATURES, KIND>(a, lda, w, ldw, c, ldc, m, n, k, stream, with);
 }
 
@@ -531,42 +496,12 @@ extern "C" int mi_gemm_f32_swiglu_takes(const float* a, int64_t lda, const float
   return m >= 1 && n >= 1 && k >= 1 && lda >= k && ldw >= k && few_rows_take(m, k) && whole_lines(a, lda, w, ldw, k, (int64_t)n + 8) ? 1 : 0;
 }
 
-// Rows whose norm the product behind it applies (and that the product before it adds to): one group.  Microseconds for o, norm and
-// gate|up with launches of their own / in two, weights from memory: hidden 2048 and 8,192 features 3 rows 33.6 / 32.4, 8 rows 38.7 / 39.0;
-// 4096 and 14,336 94.3 / 92.0 and 101.9 / 106.8; 1024 and 3,072 16.2 / 14.7 and 17.4 / 16.0.  Down, norm, q|k|v, rotation and
-// write at 3 rows 34.5 / 30.4, 70.8 / 63.7 and 19.6 / 15.6.  1B with 3 requests decoding 1,660 -> 1,571 us a step.
-extern "C" int mi_gemm_f32_most_normed_rows() { return 4; }
-
-static bool norm_fits(const float* norm_weight, float eps, int m) {
-  return norm_weight == nullptr || ((uintptr_t)norm_weight % 16 == 0 && eps > 0.f && m <= mi_gemm_f32_most_normed_rows());
-}
-
-// norm_weight [k] (on 16 bytes; null: rows as they are): an RMS norm to apply to the rows, 4 at most, first.
 extern "C" int mi_gemm_f32_swiglu(const float* a, int64_t lda, const float* w, int64_t ldw, float* c, int64_t ldc, int m, int n, int k,
-                                  const float* norm_weight, float eps, hipStream_t stream) {
+                                  hipStream_t stream) {
   MI_REQUIRE(mi_gemm_f32_swiglu_takes(a, lda, w, ldw, m, n, k) && ldc >= n, "gemm_f32_swiglu: m=%d n=%d k=%d lda=%lld ldw=%lld ldc=%lld is not taken", m,
              n, k, (long long)lda, (long long)ldw, (long long)ldc);
-  MI_REQUIRE(norm_fits(norm_weight, eps, m), "gemm_f32_swiglu: a norm is for 4 rows at most, its weight on 16 bytes, its epsilon positive");
-  FewRows with = {};
-  with.norm_weight = norm_weight;
-  with.eps = eps;
-  launch_few_of<16, FEW_GATED>(a, lda, w, ldw, c, ldc, m, n, k, stream, with);
+  launch_few_of<16, FEW_GATED>(a, lda, w, ldw, c, ldc, m, n, k, stream);
   MI_CHECK_LAUNCH("gemm_f32_swiglu");
-  return MI_OK;
-}
-
-// residual += a * w^T for a few rows, each product rounded to float32 first.
-extern "C" int mi_gemm_f32_add_takes(const float* a, int64_t lda, const float* w, int64_t ldw, int m, int n, int k) {
-  return m >= 1 && m <= mi_gemm_f32_most_normed_rows() && n >= 1 && k >= 1 && lda >= k && ldw >= k && whole_lines(a, lda, w, ldw, k, 16) ? 1 : 0;
-}
-
-extern "C" int mi_gemm_f32_add(const float* a, int64_t lda, const float* w, int64_t ldw, float* residual, int64_t ldr, int m, int n, int k,
-                               hipStream_t stream) {
-  MI_REQUIRE(mi_gemm_f32_add_takes(a, lda, w, ldw, m, n, k) && ldr >= n && residual, "gemm_f32_add: m=%d n=%d k=%d lda=%lld ldw=%lld ldr=%lld is not taken",
-             m, n, k, (long long)lda, (long long)ldw, (long long)ldr);
-  if (ceil_div(n, 16) <= 128) launch_few<1, 8, FEW_ADD>(a, lda, w, ldw, residual, ldr, m, n, k, stream);
-  else launch_few<1, 16, FEW_ADD>(a, lda, w, ldw, residual, ldr, m, n, k, stream);
-  MI_CHECK_LAUNCH("gemm_f32_add");
   return MI_OK;
 }
 
@@ -576,19 +511,15 @@ extern "C" int mi_gemm_f32_rope_takes(const float* a, int64_t lda, const float* 
 }
 
 // The stacked q|k|v product of a few rows, whole heads rotated in half pairing (cos_t, sin_t [m][head_dim / 2]): queries to q_out, keys and
-// values to their slots (kv_heads = 0: queries alone; a slot below 0 is not written).  The norm as for mi_gemm_f32_swiglu.
+// values to their slots (kv_heads = 0: queries alone; a slot below 0 is not written).
 extern "C" int mi_gemm_f32_rope(const float* a, int64_t lda, const float* w, int64_t ldw, float* q_out, int64_t ldq, const float* cos_t,
                                 const float* sin_t, const int* slots, float* k_pages, float* v_pages, int m, int k, int q_heads, int kv_heads,
-                                int head_dim, int page_size, int num_pages, int v_transposed, const float* norm_weight, float eps,
-                                hipStream_t stream) {
+                                int head_dim, int page_size, int num_pages, int v_transposed, hipStream_t stream) {
   MI_REQUIRE(mi_gemm_f32_rope_takes(a, lda, w, ldw, m, k, head_dim) && q_heads >= 1 && kv_heads >= 0 && q_out && cos_t && sin_t &&
                  ldq >= (int64_t)q_heads * head_dim && ((int64_t)q_heads + 2 * (int64_t)kv_heads) * head_dim < (1ll << 31),
              "gemm_f32_rope: m=%d k=%d lda=%lld ldw=%lld heads %d and %d of %d is not taken", m, k, (long long)lda, (long long)ldw, q_heads, kv_heads, head_dim);
   MI_REQUIRE(kv_heads == 0 || (slots && k_pages && v_pages && page_size > 0 && num_pages > 0), "gemm_f32_rope: keys and values need pages and slots");
-  MI_REQUIRE(norm_fits(norm_weight, eps, m), "gemm_f32_rope: a norm is for 4 rows at most, its weight on 16 bytes, its epsilon positive");
   FewRows with = {};
-  with.norm_weight = norm_weight;
-  with.eps = eps;
   with.cos_t = cos_t;
   with.sin_t = sin_t;
   with.slots = slots;

@@ -958,13 +958,8 @@ def linear_swiglu(x: "torch.Tensor | ScaledRows", gate_up_weight: torch.Tensor, 
     rows, width = gate_up_weight.shape
     if rows % 2:
         raise KernelShapeError(f"linear_swiglu: stacked weight has an odd number of rows ({rows})")
-    scaled = unnormed = None
-    if isinstance(x, UnnormedRows):
-        if scaled_rows_product_takes_f32(x.values.shape[0], gate_up_weight, x.values.shape[1]):
-            unnormed, x = x, x.values
-        else:
-            x = x.finish()
-    elif isinstance(x, ScaledRows):
+    scaled = None
+    if isinstance(x, ScaledRows):
         values = x.values
         if (
             _scaled_rows_fit(x)
@@ -1018,10 +1013,8 @@ def linear_swiglu(x: "torch.Tensor | ScaledRows", gate_up_weight: torch.Tensor, 
         matrices = (_ptr(x), x.stride(0), _ptr(gate_up_weight), gate_up_weight.stride(0))
         if lib.mi_gemm_f32_swiglu_takes(*matrices, m, n, width):
             out = torch.empty((m, n), dtype=torch.float32, device=x.device)
-            library.check(lib.mi_gemm_f32_swiglu(*matrices, _ptr(out), n, m, n, width, *_norm_of(unnormed), _stream()))
+            library.check(lib.mi_gemm_f32_swiglu(*matrices, _ptr(out), n, m, n, width, _stream()))
             return out
-    if unnormed is not None:
-        x = unnormed.finish()
     return silu_mul(linear(x, gate_up_weight, steady=steady))
 
 
@@ -1154,85 +1147,22 @@ class ScaledRows:
         return (self.values.float() * factor[:, None]).to(self.values.dtype)
 
 
-@dataclasses.dataclass
-class UnnormedRows(ScaledRows):
-    """Float32 rows whose RMS norm is still to be applied: `values` [T, H] is the residual stream itself, `weight` [H] the norm's (no
-    sums of squares come along).  The products that take them (`linear_swiglu`, `qkv_rope_write_f32`) norm what they read; anything else
-    calls `finish()`.  To be read before the residual stream is added to again."""
-
-    weight: torch.Tensor
-
-    def finish(self) -> torch.Tensor:
-        return add_rmsnorm(None, self.values, self.weight, self.eps)
-
-
-def _norm_of(rows: UnnormedRows | None) -> tuple:
-    """Weight and epsilon as the float32 products of few rows take a norm."""
-    return (None, 0.0) if rows is None else (_ptr(rows.weight), rows.eps)
-
-
-def scaled_rows_product_takes_f32(rows: int, weight: torch.Tensor | None, norm_width: int) -> bool:
-    """`scaled_rows_product_takes` for float32: 4 rows at most, on whole lines (csrc/gemm_f32.hip has both ways' times)."""
-    if weight is None or weight.dtype != torch.float32 or weight.dim() != 2 or weight.stride(1) != 1 or weight.shape[1] != norm_width:
-        return False
-    lib = library.load()
-    return (rows <= lib.mi_gemm_f32_most_normed_rows()
-            and bool(lib.mi_gemm_f32_swiglu_takes(None, norm_width, _ptr(weight), weight.stride(0), rows, weight.shape[0] // 2, norm_width)))
-
-
-def linear_add_norm_f32_takes(pending: PendingProduct, residual: torch.Tensor, norm_weight: torch.Tensor) -> bool:
-    """Whether `linear_add_norm_f32` runs: at most 4 rows, on whole lines."""
-    x, weight = pending.x, pending.weight
-    return (
-        isinstance(x, torch.Tensor) and x.dtype == weight.dtype == residual.dtype == norm_weight.dtype == torch.float32
-        and x.dim() == weight.dim() == 2 and x.shape[1] == weight.shape[1] and x.stride(1) == 1 and weight.stride(1) == 1
-        and residual.is_cuda and residual.is_contiguous() and tuple(residual.shape) == (x.shape[0], weight.shape[0])
-        and norm_weight.is_contiguous() and tuple(norm_weight.shape) == (weight.shape[0],) and norm_weight.data_ptr() % 16 == 0
-        and bool(library.load().mi_gemm_f32_add_takes(_ptr(x), x.stride(0), _ptr(weight), weight.stride(0), x.shape[0], *weight.shape))
-    )
-
-
-def linear_add_norm_f32(pending: PendingProduct, residual: torch.Tensor, norm_weight: torch.Tensor, eps: float) -> UnnormedRows:
-    """`linear_add_norm` for a few float32 rows: `residual += x @ weight.T` in one kernel, the norm of the sum left to the product that
-    reads it."""
-    x, weight = pending.x, pending.weight
-    if not linear_add_norm_f32_takes(pending, residual, norm_weight):
-        raise KernelShapeError(
-            f"linear_add_norm_f32 takes float32, at most 4 rows on whole lines; got weight {tuple(weight.shape)} {weight.dtype}, "
-            f"residual {tuple(residual.shape)} {residual.dtype}"
-        )
-    _need_cuda(x, weight, norm_weight)
-    m, n = residual.shape
-    library.check(
-        library.load().mi_gemm_f32_add(_ptr(x), x.stride(0), _ptr(weight), weight.stride(0), _ptr(residual), residual.stride(0), m, n,
-                                       weight.shape[1], _stream())
-    )
-    return UnnormedRows(residual, None, float(eps), norm_weight)
-
-
-def qkv_rope_write_f32_takes(x: "torch.Tensor | UnnormedRows", weight: torch.Tensor, head_dim: int, rotary_dim: int, interleaved: bool) -> bool:
+def qkv_rope_write_f32_takes(x: "torch.Tensor | ScaledRows", weight: torch.Tensor, head_dim: int, rotary_dim: int, interleaved: bool) -> bool:
     """Whether `qkv_rope_write_f32` runs these operands: float32 rows, 8 at most, whole heads of a multiple of 16 rotated in half pairing."""
-    if isinstance(x, ScaledRows):
-        if not isinstance(x, UnnormedRows) or x.values.shape[0] > library.load().mi_gemm_f32_most_normed_rows():
-            return False
-        x = x.values
     return (
-        x.dtype == weight.dtype == torch.float32 and x.is_cuda and x.dim() == weight.dim() == 2 and x.shape[1] == weight.shape[1]
+        isinstance(x, torch.Tensor) and x.dtype == weight.dtype == torch.float32 and x.is_cuda and x.dim() == weight.dim() == 2 and x.shape[1] == weight.shape[1]
         and x.stride(1) == 1 and weight.stride(1) == 1 and not interleaved and rotary_dim == head_dim
         and bool(library.load().mi_gemm_f32_rope_takes(_ptr(x), x.stride(0), _ptr(weight), weight.stride(0), x.shape[0], x.shape[1], head_dim))
     )
 
 
 def qkv_rope_write_f32(
-    x: "torch.Tensor | UnnormedRows", weight: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, slot_mapping: torch.Tensor | None,
+    x: torch.Tensor, weight: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, slot_mapping: torch.Tensor | None,
     k_pages: torch.Tensor | None, v_pages: torch.Tensor | None, *, q_heads: int, kv_heads: int, head_dim: int, v_transposed: bool = False,
 ) -> torch.Tensor:
-    """`qkv_rope_write` for a few float32 rows: `linear` and `rope_kv_write` as one kernel; returns the rotated queries.  `x` may be
-    `UnnormedRows`, normed on the way."""
+    """`qkv_rope_write` for a few float32 rows: `linear` and `rope_kv_write` as one kernel, with the same results; returns the rotated queries."""
     if not qkv_rope_write_f32_takes(x, weight, head_dim, head_dim, False):
         raise KernelShapeError(f"qkv_rope_write_f32 takes a few float32 rows and heads of a multiple of 16, got a weight {tuple(weight.shape)} {weight.dtype}")
-    unnormed = x if isinstance(x, UnnormedRows) else None
-    x = x if unnormed is None else unnormed.values
     _need_cuda(x, weight, cos, sin, slot_mapping, k_pages, v_pages)
     for name, t in (("cos", cos), ("sin", sin), ("slot_mapping", slot_mapping), ("k_pages", k_pages), ("v_pages", v_pages)):
         _need_contiguous(name, t)
@@ -1259,7 +1189,7 @@ def qkv_rope_write_f32(
     library.check(
         library.load().mi_gemm_f32_rope(
             _ptr(x), x.stride(0), _ptr(weight), weight.stride(0), _ptr(q_out), q_out.stride(0), _ptr(cos), _ptr(sin), *pages, m, k, q_heads,
-            kv_heads, head_dim, page_size, num_pages, int(v_transposed), *_norm_of(unnormed), _stream(),
+            kv_heads, head_dim, page_size, num_pages, int(v_transposed), _stream(),
         )
     )
     return q_out

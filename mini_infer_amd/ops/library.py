@@ -14,7 +14,7 @@ from pathlib import Path
 from mini_infer_amd.exceptions import ExtensionMissingError, KernelShapeError
 from mini_infer_amd.ops import build as _build
 
-ABI_VERSION = 52
+ABI_VERSION = 53
 
 _lib: ctypes.CDLL | None = None
 _lib_path: Path | None = None
@@ -34,13 +34,10 @@ _SIGNATURES: dict[str, list] = {
     "mi_silu_mul": [c_int, _P, _P, c_int, c_int, _P],
     "mi_gemm_f32": [_P, c_int64, _P, c_int64, _P, c_int64, c_int, c_int, c_int, _P],
     "mi_gemm_f32_swiglu_takes": [_P, c_int64, _P, c_int64, c_int, c_int, c_int],
-    "mi_gemm_f32_swiglu": [_P, c_int64, _P, c_int64, _P, c_int64, c_int, c_int, c_int, _P, c_float, _P],
-    "mi_gemm_f32_most_normed_rows": [],
-    "mi_gemm_f32_add_takes": [_P, c_int64, _P, c_int64, c_int, c_int, c_int],
-    "mi_gemm_f32_add": [_P, c_int64, _P, c_int64, _P, c_int64, c_int, c_int, c_int, _P],
+    "mi_gemm_f32_swiglu": [_P, c_int64, _P, c_int64, _P, c_int64, c_int, c_int, c_int, _P],
     "mi_gemm_f32_rope_takes": [_P, c_int64, _P, c_int64, c_int, c_int, c_int],
     "mi_gemm_f32_rope": [
-        _P, c_int64, _P, c_int64, _P, c_int64, _P, _P, _P, _P, _P, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, _P, c_float, _P,
+        _P, c_int64, _P, c_int64, _P, c_int64, _P, _P, _P, _P, _P, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int, _P,
     ],
     "mi_gemm_skinny_bf16": [_P, c_int64, _P, c_int64, _P, c_int64, c_int, c_int, c_int, _P],
     "mi_gemm_skinny_f32out_bf16": [_P, c_int64, _P, c_int64, _P, c_int64, c_int, c_int, c_int, c_float, _P],

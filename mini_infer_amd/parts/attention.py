@@ -169,15 +169,15 @@ class GQAttention(Mixer):
 
     def wants_scaled_rows(self, rows: int) -> bool:
         """Only where projection, rotation and cache write will run as the one kernel that
-        applies the rows' factors: few rows, whole heads rotated in half pairing."""
+        applies the rows' factors: few bfloat16 rows, whole heads rotated in half pairing."""
         layout = self.position.rotary_layout() if self.position is not None else None
-        takes = ops.scaled_rows_product_takes if self.dtype == torch.bfloat16 else ops.scaled_rows_product_takes_f32
         return (
-            self._same_widths
+            self.dtype == torch.bfloat16
+            and self._same_widths
             and self._plain_heads
             and layout == (self.head_dim, False)
             and self.head_dim % 32 == 0
-            and takes(rows, self.qkv.weight, self.hidden_size)
+            and ops.scaled_rows_product_takes(rows, self.qkv.weight, self.hidden_size)
         )
 
     def cache_needs(self, page_size: int) -> CacheNeeds:
@@ -347,10 +347,10 @@ class GQAttention(Mixer):
         """The output projection of what `_attend` returned; for few rows, where the block
         asked for it, not made here but handed on to the norm that follows."""
         assert self.out.weight is not None
-        if self.emit_pending_output:
+        if self.emit_pending_output and self.dtype == torch.bfloat16:
             rows = attended.tokens if isinstance(attended, ops.AttentionPieces) else attended.shape[0]
             q_width = self.num_heads * self.v_head_dim
-            if ops.pending_product_pays(rows, self.hidden_size, q_width, self.emit_partial_sums and self.dtype == torch.bfloat16):
+            if ops.pending_product_pays(rows, self.hidden_size, q_width, self.emit_partial_sums):
                 return ops.PendingProduct(attended, self.out.weight)
         if isinstance(attended, ops.AttentionPieces):
             return ops.linear_from_attention(attended, self.out.weight)

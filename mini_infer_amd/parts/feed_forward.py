@@ -49,8 +49,8 @@ class SwiGLU(FeedForward):
 
     def wants_scaled_rows(self, rows: int) -> bool:
         """Where the gated product runs as the weight-streaming kernel that applies the rows' factors."""
-        takes = ops.scaled_rows_product_takes if self.dtype == torch.bfloat16 else ops.scaled_rows_product_takes_f32
-        return self.activation == "silu" and takes(rows, self.gate_up.weight, self.hidden_size)
+        return (self.activation == "silu" and self.dtype == torch.bfloat16
+                and ops.scaled_rows_product_takes(rows, self.gate_up.weight, self.hidden_size))
 
     def joint_partner(self) -> "FeedForward | None":
         return self if self.activation == "silu" else None
@@ -76,8 +76,8 @@ class SwiGLU(FeedForward):
             act = ops.linear_geglu(x, self.gate_up.weight, steady=self.steady)
         if (
             self.emit_pending_output
-            and ops.pending_product_pays(act.shape[0], self.hidden_size, self.intermediate_size,
-                                         self.emit_partial_sums and self.dtype == torch.bfloat16)
+            and self.dtype == torch.bfloat16
+            and ops.pending_product_pays(act.shape[0], self.hidden_size, self.intermediate_size, self.emit_partial_sums)
         ):
             # few rows: the down product is left to the norm that follows (one kernel makes it,
             # adds it to the residual and begins the norm)

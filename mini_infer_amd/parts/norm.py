@@ -67,11 +67,9 @@ class RMSNorm(Norm):
                 and rows is None
                 and consumer is not None
                 and consumer.wants_scaled_rows(residual.shape[0])
+                and ops.linear_add_norm_takes(delta, residual, self.weight)
             ):
-                if ops.linear_add_norm_takes(delta, residual, self.weight):
-                    return ops.linear_add_norm(delta, residual, self.weight, self.eps)
-                if ops.linear_add_norm_f32_takes(delta, residual, self.weight):
-                    return ops.linear_add_norm_f32(delta, residual, self.weight, self.eps)
+                return ops.linear_add_norm(delta, residual, self.weight, self.eps)
             delta = delta.finish()
         return ops.add_rmsnorm(delta, residual, self.weight, self.eps, rows)
 

@@ -1650,34 +1650,6 @@ def test_latent_queries_are_rotated_in_place_only_when_asked_to(dim, spare):
     assert all(torch.equal(a, b) for a, b in zip(*made))
 
 
-@pytest.mark.parametrize("m,k,hidden,inter", [(1, 256, 64, 24), (3, 2048, 2048, 200), (4, 8192, 1000, 64), (2, 4096, 2080, 40), (4, 3072, 4096, 72)])
-def test_float32_norm_in_the_products_around_it(m, k, hidden, inter):
-    """A few float32 rows: the product that adds itself to the residual and the one that norms what it reads, against the norm's own launch.
-
-    A normed value is rounded once either way, at another place: by 2^-24 of it, so two of them differ by 2^-23; a product of `hidden`
-    terms of them carries that on as its square root times as much, and is rounded itself."""
-    from mini_infer_amd import ops
-    from mini_infer_amd.exceptions import KernelShapeError
-
-    torch.manual_seed(m * 100 + k)
-    eps = 1e-5
-    x, w = torch.randn(m, k, device="cuda"), torch.randn(hidden, k, device="cuda") / k ** 0.5
-    start, norm_w = torch.randn(m, hidden, device="cuda"), torch.rand(hidden, device="cuda") + 0.5
-    residual, apart = start.clone(), start.clone()
-    pending = ops.PendingProduct(x, w)
-    if k == 8192 or hidden % 32 == 0:
-        assert ops.linear_add_norm_f32_takes(pending, residual, norm_w)
-    rows = ops.linear_add_norm_f32(pending, residual, norm_w, eps)
-    normed = ops.add_rmsnorm(ops.linear(x, w), apart, norm_w, eps)
-    assert torch.equal(residual, apart)
-    assert torch.equal(rows.finish(), normed)
-    gate_up = torch.randn(2 * inter, hidden, device="cuda") / hidden ** 0.5
-    near = 2.0**-23 * hidden ** 0.5
-    torch.testing.assert_close(ops.linear_swiglu(rows, gate_up), ops.linear_swiglu(normed, gate_up), rtol=near, atol=near)
-    with pytest.raises(KernelShapeError):
-        ops.linear_add_norm_f32(ops.PendingProduct(torch.randn(5, k, device="cuda"), w), torch.zeros(5, hidden, device="cuda"), norm_w, eps)
-
-
 @pytest.mark.parametrize("m,hidden,heads,kv_heads,head_dim", [(1, 256, 2, 1, 16), (3, 2048, 6, 2, 64), (4, 8192, 3, 1, 32), (8, 1024, 4, 4, 128), (2, 64, 3, 0, 48)])
 @pytest.mark.parametrize("transposed", [False, True])
 def test_float32_rows_projected_rotated_and_written_as_one(m, hidden, heads, kv_heads, head_dim, transposed):
@@ -1699,22 +1671,6 @@ def test_float32_rows_projected_rotated_and_written_as_one(m, hidden, heads, kv_
     apart = ops.rope_kv_write(ops.linear(x, w), cos, sin, *where[0], rotary_dim=head_dim, **names)[:, : heads * head_dim]
     one = ops.qkv_rope_write_f32(x, w, cos, sin, *where[1], **names)
     assert torch.equal(one, apart) and all(torch.equal(ours, theirs) for ours, theirs in zip(caches[1], caches[0]))
-    if m > 4:
-        return
-    # with the norm still to be applied
-    norm_w = torch.rand(hidden, device="cuda") + 0.5
-    residual, again = x.clone(), x.clone()
-    last = ops.PendingProduct(torch.randn(m, 64, device="cuda"), torch.randn(hidden, 64, device="cuda"))
-    rows = ops.linear_add_norm_f32(last, residual, norm_w, 1e-6)
-    assert ops.qkv_rope_write_f32_takes(rows, w, head_dim, head_dim, False)
-    normed = ops.add_rmsnorm(last.finish(), again, norm_w, 1e-6)
-    for c in caches[0]:
-        c.zero_()
-    apart = ops.rope_kv_write(ops.linear(normed, w), cos, sin, *where[0], rotary_dim=head_dim, **names)[:, : heads * head_dim]
-    near = dict(rtol=0, atol=(3 + hidden ** 0.5) * 2.0**-24 * 8)
-    torch.testing.assert_close(ops.qkv_rope_write_f32(rows, w, cos, sin, *where[2], **names), apart, **near)
-    for ours, theirs in zip(caches[2], caches[0]):
-        torch.testing.assert_close(ours, theirs, **near)
 
 
 @pytest.mark.parametrize("m,hidden,heads,kv_heads,head_dim,page", [
