@@ -10,8 +10,8 @@
 // Both operands go straight from memory into LDS, 64 of K at a time, in a ring of STAGES; a row of a stage is 128 bytes (a whole cache
 // line: half lines, 32 of K at a time, hold as many lines up for half the bytes, 433 against 376 us for 2048 x 28672 x 4096), eight
 // chunks of 16, chunk c of row r at place c ^ (r % 8), so that the lanes that are served together find their pieces in
-// different banks.  Sums run over K from its beginning, 32 at a time: the order of the vendor library's kernels and of
-// one wave alone, so all tile shapes give the same bits as those.
+// different banks.  Sums run over K from its beginning, 32 at a time: the order of one wave alone, so all tile shapes give the same bits, and
+// the vendor library's kernels that do not cut K give them too (`turns_keep_the_order` in ops/kernels.py).
 #pragma once
 
 #include "gated_tile.h"

@@ -648,15 +648,27 @@ GATED_TILE_KINDS = {TURNS_SILU: 3, TURNS_CLAMPED: 4, TURNS_GELU: 5}  # of gemm_t
 TURNS_OUTPUTS_A_K = 400
 
 
-def _turns_take(x: torch.Tensor, weight: torch.Tensor) -> bool:
+def _turns_take(x: torch.Tensor, weight: torch.Tensor, steady: bool = False) -> bool:
     """Whether the product of these is made in the tiles of `gemm_turns_bf16`."""
-    return x.dim() == 2 and x.shape[0] >= TURNS_MIN_ROWS and turns_pay(x.shape[0], weight.shape[0], x.shape[1]) and _rows_of_bf16(x, weight)
+    if x.dim() != 2 or x.shape[0] < TURNS_MIN_ROWS or not turns_pay(x.shape[0], weight.shape[0], x.shape[1]) or not _rows_of_bf16(x, weight):
+        return False
+    return not steady or turns_keep_the_order(x.shape[0], weight.shape[0], x.shape[1], _compute_units(x.device))
+
+
+def turns_keep_the_order(m: int, n: int, k: int, cus: int = WHOLE_DEVICE_CUS) -> bool:
+    """Whether the vendor library, too, sums a bfloat16 product of more than 320 rows over K from its beginning, 32 at a time, so that
+    `gemm_turns_bf16` gives its bits: no more tiles of 256 x 256 than there are compute units, and K up to 8,192.  With more tiles some of its
+    kernels share the last ones out along K, with a longer K others cut it.  Measured: none of 15,000 products within these bounds differed (128 to
+    65,536 outputs in steps of 8 to 1,024, 321 to 8,192 rows, K from 64), nor any at each row count from 321 to 2,259 for the 27 matrices of
+    routed designs at 1B, 3B and 8B widths; of those beyond, 16384 x 3072 differs at 2,049 to 2,112 rows, 28672 x 4096 at 1,729 to 1,792, 4096 x 14336 at
+    1,537 to 2,080, and of 3,000 with K above 8,192 one in thirteen, the first at 9,216."""
+    return k <= 8192 and -(-m // 256) * -(-n // 256) <= cus
 
 
 def turns_pay(m: int, n: int, k: int) -> bool:
     """Whether a bfloat16 product of so many rows (n: gate and up together where it is gated, which is then one launch with its activation) is made in
-    the tiles of `gemm_turns_bf16`; otherwise `tiles_for`, `gated_tiles_for` or the vendor library.  Their sums have the same order, bit for bit, in all but a few of the library's kernels.  Microseconds of the library (or tiles, up to 1,024
-    rows) / these, weights from memory, over 12 matrices of 2048 x 2048 to 16384 x 2048 and 4096 x 14336:
+    the tiles of `gemm_turns_bf16`; otherwise `tiles_for`, `gated_tiles_for` or the vendor library (whose bits they mostly give: `turns_keep_the_order`).  Microseconds of the library (or
+    tiles, up to 1,024 rows) / these, weights from memory, over 12 matrices of 2048 x 2048 to 16384 x 2048 and 4096 x 14336:
 
         rows                400            640            1024           1501           2048           4096
         4096 x 14336        67 / 87        81 / 124       129 / 125      163 / 160      203 / 185      306 / 305
@@ -701,7 +713,7 @@ def _turns(act: int, x: torch.Tensor, weight: torch.Tensor, n: int, bias: torch.
 def _gated_as_one(act: int, x: torch.Tensor, weight: torch.Tensor, steady: bool, bias: torch.Tensor | None = None, limit: float = 0.0,
                   slope: float = 0.0) -> torch.Tensor | None:
     """The gated product of more than 32 rows with its activation as one launch of tiles where that pays, else None."""
-    if _turns_take(x, weight):
+    if _turns_take(x, weight, steady):
         return _turns(act, x, weight, weight.shape[0] // 2, bias, limit, slope)
     if steady or x.dim() != 2 or not SKINNY_WIDE_MAX_ROWS < x.shape[0] <= TILES_MAX_ROWS or not _rows_of_bf16(x, weight):
         return None
@@ -721,8 +733,8 @@ def linear(x: torch.Tensor, weight: torch.Tensor, partial_ok: bool = False, stea
     weight-streaming kernel, some tens to some hundreds of rows the tiles of `gemm_tiles_bf16` where they are faster
     (`tiles_for`), more rows mostly the tiles of `gemm_turns_bf16` (`turns_pay`); the rest goes to the vendor GEMM library through torch, as the
     reference's engine does (distributed/linear.py:167, `F.linear` -> the vendor BLAS).
-    With `partial_ok` the result may come as `PartialSums` where that pays.  `steady` (`Part.steady`): without the tiles of
-    `gemm_tiles_bf16`, so that the sums keep the order that they have in the library and in `gemm_turns_bf16`.
+    With `partial_ok` the result may come as `PartialSums` where that pays.  `steady` (`Part.steady`): above 16 rows the bits that the library gives,
+    so without the tiles of `gemm_tiles_bf16`, and in those of `gemm_turns_bf16` where they are the same (`turns_keep_the_order`).
     """
     if x.dtype == torch.float32:
         return gemm_f32(x, weight)
@@ -737,7 +749,7 @@ def linear(x: torch.Tensor, weight: torch.Tensor, partial_ok: bool = False, stea
         and skinny_gemm_takes(x.shape[0], x.shape[1], x.stride(0), weight.stride(0))
     ):
         return gemm_skinny_bf16(x, weight)
-    if _turns_take(x, weight):
+    if _turns_take(x, weight, steady):
         return _turns(TURNS_NONE, x, weight, weight.shape[0])
     if not steady and x.dim() == 2 and x.shape[0] <= TILES_MAX_ROWS and _rows_of_bf16(x, weight):
         m, n = x.shape[0], weight.shape[0]
@@ -889,7 +901,7 @@ def qkv_rope_write_many_plan(x: torch.Tensor, weight: torch.Tensor, head_dim: in
     if not isinstance(x, torch.Tensor) or interleaved or rotary_dim != head_dim or head_dim % 16 != 0 or not _rows_of_bf16(x, weight) or x.shape[1] % 64 != 0:
         return None
     m, n, k = x.shape[0], weight.shape[0], x.shape[1]
-    if _turns_take(x, weight):
+    if _turns_take(x, weight, steady):
         return -1
     if steady or in_pieces or m <= SKINNY_WIDE_MAX_ROWS:
         return None

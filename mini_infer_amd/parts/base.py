@@ -46,9 +46,9 @@ class Part:
     """
 
     graph_safe = False
-    # Set by the model on every part of a design with routed experts: products of more rows than stream their weights keep the
-    # order of sums over K that the vendor library's have (the library itself up to 320 rows, mostly `gemm_turns_bf16` above), and portions
-    # and single tokens attend in launches of their own.  The faster forms sum in another order,
+    # Set by the model on every part of a design with routed experts: products of more rows than stream their weights give the bits
+    # that the vendor library gives (the library itself up to 320 rows; above, `gemm_turns_bf16` where both sum in the same order,
+    # `ops.kernels.turns_keep_the_order`), and portions and single tokens attend in launches of their own.  The faster forms sum in another order,
     # no nearer to the exact sums and no farther, but where two experts' scores are close a rounding in front of the router chooses the
     # other one, and that token's logits are then 0.1 off what they were, a whole step's 0.03 (12 layers of 16 experts, 2 a token).
     steady = False

@@ -371,6 +371,35 @@ def test_products_of_many_rows_go_through_the_tiles_that_take_turns(m, n, k, mon
     assert taken == []
 
 
+@pytest.mark.parametrize("m, n, k", [(321, 1536, 64), (700, 520, 192), (1030, 2304, 512), (2048, 1024, 2048), (513, 4096, 576)])
+def test_tiles_that_take_turns_give_the_same_bits_in_every_form(m, n, k):
+    """All forms, the plan's launch, and the vendor library where it does not cut K."""
+    from mini_infer_amd.ops import kernels, library
+
+    a, w = _rand(m, k, dtype=torch.bfloat16, seed=50), _rand(n, k, dtype=torch.bfloat16, seed=51, scale=0.05)
+    planned = kernels._turns(kernels.TURNS_NONE, a, w, n)
+    for form in range(11):
+        assert library.load().mi_gemm_turns_rows(form) > 0
+        assert torch.equal(kernels._turns(kernels.TURNS_NONE, a, w, n, only=form), planned), form
+    assert kernels.turns_keep_the_order(m, n, k) and torch.equal(a @ w.t(), planned)
+
+
+@pytest.mark.parametrize("n, k", [(2048, 2048), (3072, 3072), (5120, 3072), (4096, 3072), (2112, 3072), (3072, 8192), (6144, 4096), (7168, 4096), (4096, 4096),
+                                  (4608, 1536), (4096, 512), (16384, 3072), (28672, 4096), (4096, 14336)])
+def test_steady_products_of_many_rows_are_the_librarys_bit_for_bit(n, k):
+    """The matrices of routed designs, at row counts within the bounds of `turns_keep_the_order` and beyond: the library cuts K of 16384 x 3072 at 2,060
+    rows, of 28672 x 4096 at 1,750, of 4096 x 14336 at 1,600."""
+    from mini_infer_amd import ops
+
+    w = _rand(n, k, dtype=torch.bfloat16, seed=53, scale=0.05)
+    for m in (321, 777, 1501, 1600, 1750, 2048, 2060):
+        a = _rand(m, k, dtype=torch.bfloat16, seed=52)
+        want = a @ w.t()
+        assert torch.equal(ops.linear(a, w, steady=True), want), m
+        if m in (321, 1600, 1750):
+            assert torch.equal(ops.linear_swiglu(a, w, steady=True), ops.silu_mul(want)), m
+
+
 @pytest.mark.parametrize("m,n,k", [(17, 3072, 3072), (33, 2048, 8192), (271, 3072, 8192), (100, 8192, 2048), (24, 1000, 8224), (400, 2048, 8192)])
 def test_linear_of_some_tens_to_some_hundreds_of_rows(m, n, k):
     """`linear` through tiles, with and without a consumer for the pieces; operands that the tiles do not take (rows off 16 bytes) go on

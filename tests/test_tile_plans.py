@@ -123,3 +123,11 @@ def test_the_rest_of_a_product_is_cut_where_whole_tiles_leave_units_idle():
                                             (2048, 4096, 14336, True), (1501, 2048, 8192, False), (2048, 2048, 8192, True), (512, 4096, 4128, False)])
 def test_products_that_go_to_the_tiles_that_take_turns(m, n, k, taken):
     assert kernels.turns_pay(m, n, k) == taken
+
+
+@pytest.mark.parametrize("m, n, k, kept", [(2048, 8192, 8192, True), (2049, 8192, 8192, False), (2048, 8193, 64, False), (321, 32768, 64, True), (321, 32769, 64, False),
+                                           (400, 4096, 8256, False), (1501, 5120, 3072, True), (1501, 16384, 3072, False), (65536, 256, 64, True)])
+def test_products_whose_order_of_sums_is_the_libraries_too(m, n, k, kept):
+    """Whole tiles of 256 x 256 are counted, and against the units that the device has."""
+    assert kernels.turns_keep_the_order(m, n, k) == kept
+    assert not kernels.turns_keep_the_order(m, n, k, 1) or m * n <= 256 * 256
