@@ -428,6 +428,25 @@ def test_expert_tiles_of_every_size(activation, rows, width, ff, counts, forms):
         assert (got[r] - want).abs().max() < 2 ** -6 * max(1.0, want.abs().max()), (r, e)
 
 
+def test_an_experts_rows_give_the_same_bits_however_they_are_cut():
+    """300 rows of one expert in tiles of 128, of 160, and of 256 and 64, as the rows of the others have it."""
+    from mini_infer_amd import ops
+
+    width, ff, mine = 192, 2048, 300
+    rng = np.random.default_rng(6)
+    x = dev(rng.standard_normal((mine + 15 * 150, width)), torch.bfloat16)
+    up = dev(rng.standard_normal((16, 2 * ff, width)) / np.sqrt(width), torch.bfloat16)
+    down = dev(rng.standard_normal((16, width, ff)) / np.sqrt(ff), torch.bfloat16)
+    results = []
+    for others, cut in (([], (0, 3, 100, 128)), ([40] * 15, (0, 2, 150, 160)), ([150] * 15, (1, 1, 44, 64))):
+        counts = [mine] + others
+        assert ops.kernels.expert_tile_cuts(counts, 2 * ff, width)[0] == cut
+        chosen = ints(np.repeat(np.arange(len(counts)), counts).tolist()).reshape(-1, 1)
+        rows, experts = chosen.shape[0], len(counts)
+        results.append(ops.experts_by_expert(x[:rows], up[:experts], down[:experts], chosen, torch.ones((rows, 1), device=DEV), tiles="lds")[:mine].clone())
+    assert torch.equal(results[0], results[1]) and torch.equal(results[0], results[2])
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 @pytest.mark.parametrize("scores", ["logistic", "softmax"])
 @pytest.mark.parametrize("tokens, width, outputs, experts, top, corrected, gated", [
