@@ -666,27 +666,41 @@ def turns_keep_the_order(m: int, n: int, k: int, cus: int = WHOLE_DEVICE_CUS) ->
 
 
 def turns_pay(m: int, n: int, k: int) -> bool:
-    """Whether a bfloat16 product of so many rows (n: gate and up together where it is gated, which is then one launch with its activation) is made in
-    the tiles of `gemm_turns_bf16`; otherwise `tiles_for`, `gated_tiles_for` or the vendor library (whose bits they mostly give: `turns_keep_the_order`).  Microseconds of the library (or
-    tiles, up to 1,024 rows) / these, weights from memory, over 12 matrices of 2048 x 2048 to 16384 x 2048 and 4096 x 14336:
+    """Whether a bfloat16 product of so many rows with something in its last step (an activation, n: gate and up together; a rotation) is made in
+    the tiles of `gemm_turns_bf16`; otherwise `tiles_for`, `gated_tiles_for` or the vendor library (whose bits they mostly give: `turns_keep_the_order`).
+    Plain products: `plain_turns_pay`.  Microseconds of the library / of these, plain, weights from memory (more of them in
+    profiles/products_of_many_rows.txt):
 
         rows                400            640            1024           1501           2048           4096
-        4096 x 14336        67 / 87        81 / 124       129 / 125      163 / 160      203 / 185      306 / 305
-        6144 x 4096         32 / 32        40 / 38        53 / 51        72 / 60        79 / 79        157 / 148
-        3072 x 8192         42 / 48        51 / 51        63 / 64        84 / 75        94 / 91        150 / 145
-        2048 x 8192         32 / 47        44 / 50        52 / 52        56 / 62        69 / 68        110 / 107
-        3072 x 3072         25 / 19        25 / 19        25 / 23        34 / 30        36 / 33        62 / 57
-        16384 x 2048        34 / 31        39 / 37        53 / 52        85 / 84        100 / 103      193 / 205
+        4096 x 14336        77 / 86        107 / 122      130 / 125      164 / 159      204 / 187      306 / 308
+        6144 x 4096         31 / 33        42 / 38        52 / 51        78 / 61        82 / 86        158 / 151
+        3072 x 8192         41 / 47        51 / 51        63 / 64        85 / 78        95 / 90        150 / 161
+        2048 x 8192         31 / 47        43 / 49        49 / 51        55 / 63        72 / 70        110 / 106
+        4096 x 4096         25.2 / 26.9    34 / 35        42 / 38        51 / 50        60 / 59        91 / 95
+        3072 x 3072         20.1 / 21.2    22.2 / 22.8    28.7 / 29.4    38 / 33        41 / 38        62 / 63
+        2048 x 2048         12.7 / 15.0    14.5 / 15.8    16.6 / 16.4    21.6 / 20.2    23.9 / 21.9    34 / 32
+        16384 x 2048        34 / 33        42 / 41        56 / 56        87 / 85        102 / 106      195 / 207
 
-    as a geometric mean over those matrices 1.08 up to 1,024 rows, 1.07 to 2,048, 1.05 beyond.  What they lose on is a long K with
-    few outputs: a block walks all of K, the library's smaller tiles and cut ranges finish earlier.  Left to those: fewer outputs than
-    `TURNS_OUTPUTS_A_K` for each element of K.  What is taken is at worst 0.94 as fast at these sizes (4096 x 4096 at 768 rows 33.2 / 35.5), and
-    of small matrices 1024 x 3072 at 2,048 rows 21.2 / 23.5, 512 x 512 at 500 rows 5.7 / 6.4, 1024 x 1024 at 1,100 11.1 / 9.8.
+    What they lose on is a long K with few outputs: a block walks all of K, the library's smaller tiles and cut ranges finish earlier.  Left to
+    those: fewer outputs than `TURNS_OUTPUTS_A_K` for each element of K.  From 321 rows on because `gemm_tiles_bf16` and its rules end there; the two have
+    not been compared with fewer rows.
 
     Gated, with the launch of the activation on the other side, gate|up 28672 x 4096 at 400 / 1,024 / 1,777 / 2,048 / 4,096 rows 106 / 203 / 432 / 373 / 693
     against 97 / 184 / 327 / 346 / 658, 16384 x 3072 60 / 94 / 166 / 173 / 330 against 48 / 79 / 144 / 152 / 300, 7168 x 4096 36 / 61 / 92 / 94 /
-    184 against 34 / 57 / 84 / 90 / 178: 1.12 up to 1,024 rows, 1.16 to 2,048, 1.14 beyond, and never slower from 321 rows on."""
+    184 against 34 / 57 / 84 / 90 / 178: 1.12 up to 1,024 rows, 1.16 to 2,048, 1.14 beyond
+    (measured again over 15 matrices of 1024 to 28672 rows, 1.08 as a geometric mean and at worst 0.91, 28672 x 4096 at 321 rows and 2048 x 2048 at 400)."""
     return m >= TURNS_MIN_ROWS and k % 64 == 0 and m * n >= TURNS_OUTPUTS_A_K * k
+
+
+def plain_turns_pay(m: int, n: int, k: int) -> bool:
+    """`turns_pay` for a product with nothing in its last step, where no launch is saved.  The library's kernels for K in whole 128s are faster where one
+    round of tiles leaves compute units idle: up to 4,096 outputs, K of 1,536 to 4,096 and fewer than 900 outputs for each element of K, library /
+    these 1536 x 1536 at 512 rows 10.5 / 13.4, 2048 x 2048 12.6 / 15.8, 3072 x 3072 20.3 / 22.9, 4096 x 4096 at 768 33.0 / 36.3, 1024 x 3072 at 1,501 18.9 /
+    22.6: over 56 such products of common sizes 0.94 and over 76 of random ones 0.94 as a geometric mean (0.78 to 1.20).  With other K it is these,
+    1.15 over 70.  Beside an attention's and a feed-forward's other products, 3072 x 3072 at 400 / 512 / 768 / 1,024 rows 20.6 / 22.1, 20.6 / 23.0, 26.4 /
+    30.2, 30.7 / 29.1.  Of 412 products of common sizes that are left to these 25 take more than 1.05 of the library's time (10240 x 8192 at 1,024
+    rows 137 / 154, 12288 x 4096 at 900 77 / 85, 16384 x 2048 at 4,096 195 / 207), the geometric mean is 1.07; of 2,464 of random sizes 5 %, the mean 1.15."""
+    return turns_pay(m, n, k) and (n > 4096 or not 1536 <= k <= 4096 or k % 128 != 0 or m * n >= 900 * k)
 
 
 def turns_plan(m: int, n: int, k: int, gated: bool = False, cus: int = WHOLE_DEVICE_CUS) -> tuple[list[int], float]:
@@ -731,7 +745,7 @@ def linear(x: torch.Tensor, weight: torch.Tensor, partial_ok: bool = False, stea
 
     float32 runs the hand-written true-float32 kernel.  bfloat16 with at most 16 rows (decode) runs the hand-written
     weight-streaming kernel, some tens to some hundreds of rows the tiles of `gemm_tiles_bf16` where they are faster
-    (`tiles_for`), more rows mostly the tiles of `gemm_turns_bf16` (`turns_pay`); the rest goes to the vendor GEMM library through torch, as the
+    (`tiles_for`), more rows mostly the tiles of `gemm_turns_bf16` (`plain_turns_pay`); the rest goes to the vendor GEMM library through torch, as the
     reference's engine does (distributed/linear.py:167, `F.linear` -> the vendor BLAS).
     With `partial_ok` the result may come as `PartialSums` where that pays.  `steady` (`Part.steady`): above 16 rows the bits that the library gives,
     so without the tiles of `gemm_tiles_bf16`, and in those of `gemm_turns_bf16` where they are the same (`turns_keep_the_order`).
@@ -749,7 +763,7 @@ def linear(x: torch.Tensor, weight: torch.Tensor, partial_ok: bool = False, stea
         and skinny_gemm_takes(x.shape[0], x.shape[1], x.stride(0), weight.stride(0))
     ):
         return gemm_skinny_bf16(x, weight)
-    if _turns_take(x, weight, steady):
+    if _turns_take(x, weight, steady) and plain_turns_pay(x.shape[0], weight.shape[0], x.shape[1]):
         return _turns(TURNS_NONE, x, weight, weight.shape[0])
     if not steady and x.dim() == 2 and x.shape[0] <= TILES_MAX_ROWS and _rows_of_bf16(x, weight):
         m, n = x.shape[0], weight.shape[0]

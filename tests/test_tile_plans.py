@@ -131,3 +131,12 @@ def test_products_whose_order_of_sums_is_the_libraries_too(m, n, k, kept):
     """Whole tiles of 256 x 256 are counted, and against the units that the device has."""
     assert kernels.turns_keep_the_order(m, n, k) == kept
     assert not kernels.turns_keep_the_order(m, n, k, 1) or m * n <= 256 * 256
+
+
+@pytest.mark.parametrize("m, n, k, gated, plain", [
+    (512, 2048, 2048, True, False), (900, 2048, 2048, True, True), (768, 4096, 4096, True, False), (900, 4096, 4096, True, True), (1501, 1024, 3072, True, False),
+    (512, 4097, 3072, True, True), (512, 3072, 3136, True, True), (512, 3072, 1472, True, True), (500, 512, 512, True, True), (2048, 4096, 14336, True, True),
+    (640, 4096, 14336, False, False)])
+def test_plain_products_with_few_outputs_for_their_k_are_the_librarys(m, n, k, gated, plain):
+    """With an activation or a rotation, whose launch is saved, they stay in tiles."""
+    assert kernels.turns_pay(m, n, k) == gated and kernels.plain_turns_pay(m, n, k) == plain
