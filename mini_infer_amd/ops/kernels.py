@@ -894,6 +894,33 @@ def qkv_rope_write(
     return q_out
 
 
+@functools.lru_cache(maxsize=8192)
+def rotary_tiles_for(m: int, n: int, k: int, cus: int = WHOLE_DEVICE_CUS) -> int | None:
+    """The tile shape where a rotary product of 33 to 1,024 rows is made in tiles, or None.  The tiles of `tiles_for` where those are whole.  Where
+    `linear` leaves the product to the vendor library, up to 320 rows the best whole tile, as that loses less to the library than the rotation's
+    launch takes; not where `linear` cuts K (10240 x 8192 at 100 rows in `qkv_rope_write_many_plan`), and not for a K above 4 times the
+    outputs, all of which a block would walk.  Microseconds of the two launches / this one, weights from memory:
+
+        rows             33             128            271            320
+        512 x 512        10.0 / 5.4     11.6 / 5.2     11.0 / 6.7     11.0 / 5.6
+        2304 x 768       11.3 / 6.3     12.4 / 6.3     12.6 / 8.3     12.5 / 7.3
+        3072 x 2048      15.4 / 10.1    18.6 / 10.9    18.0 / 13.4    18.0 / 13.1
+        768 x 3072       16.0 / 13.1    14.0 / 13.7    14.6 / 13.9    14.7 / 13.6
+        1536 x 4096      15.9 / 15.9    16.4 / 16.6    19.0 / 16.8    19.9 / 16.7
+        512 x 4096       15.4 / 15.6    16.3 / 15.6    14.5 / 16.0    14.7 / 15.1    (left to the two launches, as those below)
+        768 x 8192       15.7 / 27.5    18.4 / 28.5    24.0 / 27.8    24.1 / 28.0
+        512 x 14336      22.7 / 44.7    24.8 / 49.5    36.3 / 46.1    36.7 / 49.1
+
+    and of those that `tiles_for` refuses from 289 rows on, at 289 rows 5120 x 3072 27.3 / 24.5, 9216 x 3072 38.6 / 31.6, 12288 x 4096 59.2 / 48.5, 14336 x
+    4096 56.1 / 51.8, 15360 x 5120 68.2 / 66.4.  From 16,000 outputs on nothing was measured, and the launch is left as it was."""
+    plan = tiles_for(m, n, k, False, cus)
+    if plan is not None:
+        return plan[0] if plan[1] == 1 else None
+    if m >= TURNS_MIN_ROWS or n >= 16000 or k > 4 * n:
+        return None
+    return _tiles_plan(m, n, k, False, 1, False, 0.0, 0.0, cus)[1]
+
+
 def qkv_rope_write_many_plan(x: torch.Tensor, weight: torch.Tensor, head_dim: int, rotary_dim: int, interleaved: bool, steady: bool = False,
                              in_pieces: bool = False, others: tuple[torch.Tensor | None, ...] = ()) -> int | None:
     """How `qkv_rope_write_many` makes this product of many bfloat16 rows: the shape of its tiles, -1 for those of `gemm_turns_bf16`, or
@@ -908,8 +935,7 @@ def qkv_rope_write_many_plan(x: torch.Tensor, weight: torch.Tensor, head_dim: in
         6144 x 4096         25.0 / 20.8    32.1 / 27.0    33.6 / 28.7    39.7 / 34.6    58.3 / 52.6    90.4 / 83.8    308 / 283
         10240 x 8192        44.5 / 57.0    64.1 / 62.7    74.5 / 67.4    78.2 / 73.5    153 / 147      284 / 274      949 / 895
 
-    Up to 320 rows whole tiles are taken too where the library makes the product (3072 x 2048 above; 2304 x 768 11.3 to 13.3 / 6.3 to 8.3,
-    5120 x 3072 at 300 rows 27.1 / 25.4), as they lose less to it than the rotation's launch takes, but not where `linear` cuts K: 10240 x 8192 at 100 rows."""
+    Which tiles up to 320 rows: `rotary_tiles_for`."""
     if any(t is not None and t.data_ptr() % 16 != 0 for t in others):
         return None
     if not isinstance(x, torch.Tensor) or interleaved or rotary_dim != head_dim or head_dim % 16 != 0 or not _rows_of_bf16(x, weight) or x.shape[1] % 64 != 0:
@@ -919,11 +945,7 @@ def qkv_rope_write_many_plan(x: torch.Tensor, weight: torch.Tensor, head_dim: in
         return -1
     if steady or in_pieces or m <= SKINNY_WIDE_MAX_ROWS:
         return None
-    cus = _compute_units(x.device)
-    plan = tiles_for(m, n, k, False, cus)
-    if plan is None and m < TURNS_MIN_ROWS and n < 16000:
-        return _tiles_plan(m, n, k, False, 1, False, 0.0, 0.0, cus)[1]
-    return plan[0] if plan is not None and plan[1] == 1 else None
+    return rotary_tiles_for(m, n, k, _compute_units(x.device))
 
 
 def qkv_rope_write_many(

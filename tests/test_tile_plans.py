@@ -140,3 +140,18 @@ def test_products_whose_order_of_sums_is_the_libraries_too(m, n, k, kept):
 def test_plain_products_with_few_outputs_for_their_k_are_the_librarys(m, n, k, gated, plain):
     """With an activation or a rotation, whose launch is saved, they stay in tiles."""
     assert kernels.turns_pay(m, n, k) == gated and kernels.plain_turns_pay(m, n, k) == plain
+
+
+@pytest.mark.parametrize("m, n, k, made", [
+    (271, 5120, 3072, "whole"), (100, 6144, 4096, "whole"), (100, 10240, 8192, None),       # as `linear` has them: whole tiles, K cut
+    (33, 2304, 768, "own"), (320, 3072, 2048, "own"), (300, 15360, 5120, "own"), (100, 768, 3072, "own"), (100, 1536, 4096, "own"),
+    (100, 512, 4096, None), (64, 768, 8192, None), (320, 512, 14336, None),                 # a block would walk a long K alone
+    (300, 16384, 4096, None), (321, 2304, 768, None), (400, 768, 3072, None)])
+def test_tiles_of_rotary_products(m, n, k, made):
+    plan = kernels.tiles_for(m, n, k, False)
+    shape = kernels.rotary_tiles_for(m, n, k)
+    assert (shape is None) == (made is None)
+    if made == "whole":
+        assert plan == (shape, 1)
+    elif made == "own":
+        assert plan is None and kernels.tile_size(shape)[0] > 0
