@@ -1767,3 +1767,95 @@ def test_many_rows_projected_rotated_and_written_as_one(m, hidden, heads, kv_hea
         ops.qkv_rope_write_many(x[:, ::2], w[:, ::2], cos, sin, None, None, None, plan=-1, **names)
     assert ops.qkv_rope_write_many_plan(x, w, head_dim, head_dim, True) is None
     assert ops.qkv_rope_write_many_plan(x.float(), w.float(), head_dim, head_dim, False) is None
+
+
+@pytest.mark.parametrize("m, k, heads, kv_heads, head_dim, how, kind", [
+    (271, 3072, 24, 8, 128, {}, "tiles"), (97, 2048, 6, 1, 128, {}, "tiles"), (320, 768, 12, 12, 64, {}, "tiles"), (100, 2048, 16, 0, 64, {}, "tiles"),
+    (400, 768, 12, 12, 64, {}, "turns"), (512, 2048, 16, 8, 128, {}, "turns"), (700, 1024, 16, 0, 64, {}, "turns"),
+    (700, 1024, 16, 8, 64, {"steady": True}, "turns"), (400, 768, 12, 12, 64, {"in_pieces": True}, "turns"),
+    (271, 3072, 24, 8, 128, {"steady": True}, None), (271, 3072, 24, 8, 128, {"in_pieces": True}, None), (32, 3072, 24, 8, 128, {}, None),
+    (64, 8192, 4, 2, 64, {}, None), (330, 8192, 4, 2, 64, {}, None), (2060, 512, 64, 64, 128, {"steady": True}, None), (2060, 512, 64, 64, 128, {}, "turns"),
+    (300, 96, 4, 2, 64, {}, None), (271, 3072, 24, 8, 128, {"interleaved": True}, None), (271, 3072, 24, 8, 128, {"rotary_dim": 64}, None),
+    (271, 3072, 16, 8, 200, {}, None), (271, 3072, 24, 8, 128, {"off": True}, None)])
+def test_which_projections_are_rotated_in_their_tiles(m, k, heads, kv_heads, head_dim, how, kind):
+    """The plan from the public entry, and what it makes against the same tiles' plain product and `rope_kv_write`."""
+    from mini_infer_amd import ops
+    from mini_infer_amd.ops import kernels
+
+    n = (heads + 2 * kv_heads) * head_dim
+    x, w = _rand(m, k, dtype=torch.bfloat16, seed=60), _rand(n, k, dtype=torch.bfloat16, seed=61, scale=k ** -0.5)
+    angle = torch.rand(m, head_dim // 2, device="cuda") * 6
+    cos, sin = angle.cos(), angle.sin()
+    others = (cos, sin, torch.empty(9, device="cuda")[1:] if how.get("off") else None)
+    plan = ops.qkv_rope_write_many_plan(x, w, head_dim, how.get("rotary_dim", head_dim), how.get("interleaved", False), how.get("steady", False),
+                                        how.get("in_pieces", False), others)
+    assert (kind is None) == (plan is None) and (kind is None or (kind == "turns") == (plan == -1))
+    if plan is None:
+        return
+    product = kernels._turns(0, x, w, n) if plan < 0 else kernels._tiles(0, x, w, torch.empty((m, n), dtype=torch.bfloat16, device="cuda"), n, plan, 1)
+    slots = torch.randperm(m + 40, device="cuda").int()[:m].contiguous()
+    made = []
+    names = dict(q_heads=heads, kv_heads=kv_heads, head_dim=head_dim, v_transposed=True)
+    for as_one in (False, True):
+        pages = [torch.zeros(m // 16 + 4, max(kv_heads, 1), *shape, dtype=torch.bfloat16, device="cuda") for shape in ((16, head_dim), (head_dim, 16))]
+        where = (slots, *pages) if kv_heads else (None, None, None)
+        if as_one:
+            queries = ops.qkv_rope_write_many(x, w, cos, sin, *where, plan=plan, **names)
+        else:
+            queries = ops.rope_kv_write(product, cos, sin, *where, rotary_dim=head_dim, **names)[:, : heads * head_dim]
+        made.append([queries, *pages])
+    assert all(torch.equal(a, b) for a, b in zip(*made))
+
+
+LAUNCHES = ("mi_gemm_turns_rope", "mi_gemm_tiles_rope", "mi_gemm_f32_rope", "mi_gemm_turns_bf16", "mi_gemm_tiles_bf16", "mi_rope_kv_write")
+
+
+@pytest.mark.parametrize("dtype, steady, rows, rotates", [
+    (torch.float32, False, 1, "mi_gemm_f32_rope"), (torch.float32, False, 4, "mi_gemm_f32_rope"), (torch.float32, False, 5, "mi_gemm_f32_rope"),
+    (torch.float32, False, 8, "mi_gemm_f32_rope"), (torch.float32, False, 9, "mi_rope_kv_write"), (torch.float32, False, 100, "mi_rope_kv_write"),
+    (torch.bfloat16, False, 100, "mi_gemm_tiles_rope"), (torch.bfloat16, False, 320, "mi_gemm_tiles_rope"), (torch.bfloat16, False, 400, "mi_gemm_turns_rope"),
+    (torch.bfloat16, True, 100, "mi_rope_kv_write"), (torch.bfloat16, True, 400, "mi_gemm_turns_rope")])
+def test_what_a_models_step_launches(dtype, steady, rows, rotates, monkeypatch):
+    """A prompt of so many tokens (up to 9: so many requests, a token each) through a small Llama: which kernel rotates and writes q|k|v, in every layer, and no product of a steady
+    one in tiles of another order.  The logits against the same step where nothing is rotated in a product."""
+    from mini_infer_amd import ModelRunner, StepEntry, ops
+    from mini_infer_amd.models import architecture_for
+    from mini_infer_amd.ops import kernels, library
+
+    config = {"architectures": ["LlamaForCausalLM"], "num_hidden_layers": 2, "hidden_size": 512, "num_attention_heads": 8, "num_key_value_heads": 4,
+              "head_dim": 64, "intermediate_size": 1024, "vocab_size": 256, "rope_theta": 10000.0, "rms_norm_eps": 1e-5, "tie_word_embeddings": False,
+              "max_position_embeddings": 1024}
+    arch = architecture_for(config)
+    parsed = arch.parse_config(config)
+    model = arch.make_model(parsed, dtype, "cuda:0")
+    specs, generator = model.param_specs(), torch.Generator(device="cuda").manual_seed(7)
+    model.load_params(lambda name: (torch.randn(specs[name].shape, generator=generator, device="cuda") * (1.0 if len(specs[name].shape) == 1 else 0.05)).to(
+        torch.float32 if specs[name].dtype == "float32" else dtype))
+    for block in model.blocks:
+        for part in block.parts():
+            part.steady = steady
+    lib, taken = library.load(), []
+    for name in LAUNCHES:
+        monkeypatch.setattr(lib, name, lambda *a, name=name, launch=getattr(lib, name): (taken.append(name), launch(*a))[1])
+    tokens = torch.randint(0, 256, (rows,), generator=torch.Generator().manual_seed(8)).tolist()
+
+    def step():
+        runner = ModelRunner(model, parsed, num_blocks=40, block_size=16, max_concurrent=9)
+        if rows > 9:
+            return runner.step([StepEntry(0, tokens, [rows - 1])]).clone()
+        for i in range(rows):
+            runner.step([StepEntry(i, (tokens * 20)[:20], [])])
+        taken.clear()
+        return runner.step([StepEntry(i, tokens[i:i + 1], [0]) for i in range(rows)]).clone()
+
+    logits = step()
+    rotated = [name for name in taken if name in LAUNCHES[:3] + LAUNCHES[5:]]
+    assert set(rotated) == {rotates} and len(rotated) in (2, 4), taken  # (a short step runs once before it is recorded)
+    assert not steady or "mi_gemm_tiles_bf16" not in taken
+    monkeypatch.setattr(ops, "qkv_rope_write_many_plan", lambda *a: None)
+    monkeypatch.setattr(ops, "qkv_rope_write_f32_takes", lambda *a: False)
+    apart = step()
+    if dtype == torch.float32 or steady or rows > 320 or kernels.tiles_for(rows, 1024, 512, False):
+        assert torch.equal(logits, apart)
+    else:  # (one product a layer in another order of sums: a bfloat16 rounding, 2^-9, of q, k and v, carried through two layers)
+        assert (logits - apart).norm() < 2.0 ** -6 * apart.norm()
