@@ -38,8 +38,8 @@ constexpr int TILE_FEATURES = 256;
 static_assert(cut_rows(0) == turns_form(0).rows && cut_rows(1) == turns_form(1).rows && cut_rows(2) == turns_form(2).rows && cut_rows(3) == turns_form(3).rows);
 
 // Microseconds of a launch over n weight rows of k elements an expert: what the compute units multiply, the largest tiles first, and what they
-// bring in, of which neither hides the other quite.  Fitted to 50 spreads of pairs over experts of five sizes, weights from memory: the cut with the least of
-// these is 0.5 % slower than the best one on average, 8 % at worst.
+// bring in, of which neither hides the other quite.  Fitted to 48 spreads of pairs over experts of five sizes, weights from memory
+// (profiles/expert_tiles_cuts_times.txt): the cut with the least of these is 0.3 % slower than the best one on average, 8 % at worst.
 __host__ __device__ inline float launch_micros(const CutSums& sums, int n, int k, int cus) {
   const int feature_tiles = (n + TILE_FEATURES - 1) / TILE_FEATURES;
   constexpr float STEP[CUT_FORMS] = {0.84f, 1.04f, 1.15f, 1.30f};  // of 64 of K, with the pairs' rows from L2 and the weights from memory
@@ -155,8 +155,14 @@ __device__ __forceinline__ void make_tile(
   }
 }
 
-// ONCE: most experts have one row tile, so that nobody else reads its weights: past the caches (16 x 4096 x 3072 with 2,700 pairs 106 -> 98 us, and
-// 75 -> 67 with 400; with 12,000 pairs 265 -> 270).
+// ONCE: weights are read past the caches, which pays where few experts have a second row tile.  The host knows only how many pairs an expert gets on
+// average, and takes it up to 256; the cut, and with it who has one, is chosen later.  Microseconds through the caches / past them, gate and up:
+//     one tile an expert     16 x 4096 x 3072  40 an expert 79.8 / 71.0    130  91.6 / 84.1    230 (all alike) 102 / 92     64 x 2048 x 2048  150  168 / 159
+//     two for each           16 x 2048 x 2048  256 (all alike) 45.7 / 43.8
+//     for some               16 x 4096 x 3072  256 146 / 142    230 133 / 134      16 x 2048 x 2048  230  48.6 / 52.4
+//     beyond                 16 x 2048 x 2048  400 62.8 / 75.1    16 x 4096 x 3072  340 159 / 160     64 x 2048 x 2048  340  234 / 239
+// (the second tile of an expert runs at the same time as the first and often finds its weights on the way all the same; over 108 launches of up to 256
+// pairs an expert 0.93 to 1.24, one of 16 x 3072 x 2048 0.83, as a geometric mean 1.06; over 28 beyond 0.99).
 template <int MODE, bool ONCE>
 __global__ __launch_bounds__(512, 2) void expert_tiles_kernel(
     const bf16_t* __restrict__ src, int64_t src_stride, int src_div, const bf16_t* __restrict__ weight,

@@ -111,7 +111,7 @@ __device__ __forceinline__ int rotary_row_of(int row, int pairs, int head_dim) {
 // a tile of values in four times the instructions).  What bounds it: the tile leaves LDS as it would without the rotation, beside the angles from
 // L2 (asking for the next row's ahead of its turn measured the same).  The launch of rope_kv_write that it replaces read and wrote the projection once
 // more: 6.3 us a layer at 271 rows x 5120, 11.8 at 2,048 x 6144, against products some 3 and 5 us longer; a step of 15 single tokens beside 256 at 3B
-// sizes 4,275 -> 4,152 us, a prompt of 2,048 tokens at 8B sizes 25,634 -> 25,399 (in tiles that keep both rows of a pair in one wave, of which
+// sizes 4,281 -> 4,167 us (three times in turn, 1.026 to 1.030), a prompt of 2,048 tokens at 8B sizes 25,625 -> 25,370 (in tiles that keep both rows of a pair in one wave, of which
 // there are none 192 wide, 25,825 -> 25,705).
 template <class Pairs, int BM, int BN, int MADE, int THREADS>
 __device__ __forceinline__ void write_rotated(const bf16_t* made, const RotaryWrite& how, int r0, int m, int f0, int n) {

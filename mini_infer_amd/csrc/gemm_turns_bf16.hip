@@ -7,8 +7,9 @@
 // a half rounds of 256 x 256, and the half is a round of 128 x 256 (gated 369 us in four rounds, 346 so); 1777 rows three rounds and 16
 // tiles, cut into 64 rows (350, 327).  Results leave through LDS: in whole 16 bytes, and with little code (turns_product.h).
 //
-// Measured against the library, with the activation's launch where gated: `turns_pay` (ops/kernels.py).  A step of 2,048 tokens at 8B sizes (Llama)
-// 27,410 -> 26,058 us, of 12 layers with clamped feed-forwards 12,133 -> 11,040.
+// Measured against the library, with the activation's launch where gated: `turns_pay` and `plain_turns_pay` (ops/kernels.py).  Steps without these tiles and
+// with them, one machine in turn: 2,048 tokens at 8B sizes (Llama) 26,822 -> 25,461 us, of 12 layers with clamped feed-forwards 12,052 -> 11,266,
+// 1,777 tokens of 12 layers at 3B widths with four streams 8,692 -> 8,252, 1,501 with routed experts 6,231 -> 5,900.
 //
 // This stands where the reference's engine calls the vendor BLAS (distributed/linear.py:167) and where its SiLU * up kernel stands
 // (models/blocks/silu_mul_kernel.py:86-90).
@@ -104,7 +105,7 @@ TurnsPlan turns_plan(int m, int n, int k, bool gated, int only, int cus, double*
       if (turns_form(rest).features != form.features || form.rows % turns_form(rest).rows != 0 || (only >= 0 && rest != f)) continue;
       const int cut = form.rows / turns_form(rest).rows;
       const double multiplied = turns_rounds_micros(f, whole, each, k) + turns_rounds_micros(rest, (places - whole) * cut, each, k);
-      const double brought = turns_bytes_micros(f, 1, total + (int64_t)(places - whole) * 8 * (cut - 1), gated ? 2 * n : n, k);
+      const double brought = turns_bytes_micros(f, total + (int64_t)(places - whole) * 8 * (cut - 1), gated ? 2 * n : n, k);
       const double t = multiplied > brought ? multiplied : brought;
       if (*micros == 0.0 || t < *micros) *micros = t, best = {f, rest, cut, whole, places};
     }

@@ -296,13 +296,13 @@ __host__ __device__ constexpr TurnsForm turns_form(int i) {
 }
 
 // Microseconds of the rounds that `tiles` tiles of form f take on `each` compute units (of one XCD): the last one, where it does not fill them, is a
-// little shorter, because the card's power then lets the clock rise.  And of the bytes of `matrices` matrices of n rows of k elements that
-// `blocks` tiles read.
+// little shorter, because the card's power then lets the clock rise.  And of the bytes of n rows of W of k elements that `blocks` tiles read.  (The
+// microseconds of a step in the table above and these rates were fitted to profiles/turns_tiles_forms_times.txt.)
 __host__ __device__ inline float turns_rounds_micros(int f, int tiles, int each, int k) {
   if (tiles == 0) return 0.f;
   const int rounds = (tiles + each - 1) / each, idle = rounds * each - tiles;
   return ((float)rounds - 0.29f * (float)idle / (float)each) * ((float)(k / TURNS_K) * turns_form(f).step_micros + 3.4f);
 }
-__host__ __device__ inline float turns_bytes_micros(int f, int matrices, int64_t blocks, int n, int k) {
-  return 2.33e-7f * (float)matrices * (float)n * (float)k * 2.f + 0.73e-7f * (float)blocks * (float)k * ((float)turns_form(f).features * 2.f);
+__host__ __device__ inline float turns_bytes_micros(int f, int64_t blocks, int n, int k) {
+  return 2.33e-7f * (float)n * (float)k * 2.f + 0.73e-7f * (float)blocks * (float)k * ((float)turns_form(f).features * 2.f);
 }

@@ -682,8 +682,9 @@ def turns_pay(m: int, n: int, k: int) -> bool:
         16384 x 2048        34 / 33        42 / 41        56 / 56        87 / 85        102 / 106      195 / 207
 
     What they lose on is a long K with few outputs: a block walks all of K, the library's smaller tiles and cut ranges finish earlier.  Left to
-    those: fewer outputs than `TURNS_OUTPUTS_A_K` for each element of K.  From 321 rows on because `gemm_tiles_bf16` and its rules end there; the two have
-    not been compared with fewer rows.
+    those: fewer outputs than `TURNS_OUTPUTS_A_K` for each element of K.  From 321 rows on because `gemm_tiles_bf16` and its rules end there; with fewer rows
+    only one step's products were compared (271 rows, there / best form of these: gate|up 16384 x 3072 44.1 / 40.7, 5120 x 3072 21.4 / 22.0, 3072 x 3072 15.4 /
+    21.4, 3072 x 8192 26.4 / 47.6).
 
     Gated, with the launch of the activation on the other side, gate|up 28672 x 4096 at 400 / 1,024 / 1,777 / 2,048 / 4,096 rows 106 / 203 / 432 / 373 / 693
     against 97 / 184 / 327 / 346 / 658, 16384 x 3072 60 / 94 / 166 / 173 / 330 against 48 / 79 / 144 / 152 / 300, 7168 x 4096 36 / 61 / 92 / 94 /

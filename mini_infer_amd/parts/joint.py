@@ -13,8 +13,8 @@ both results are sums, the two last ones are one product with the matrices side 
 twice the size with the mixer's own work between them: at few rows the weights of a whole layer stream
 through two launches, and the first of them ends with everything that follows it row by row
 (`ops.layer_in`).  For many rows the pieces of a very large product were faster apart in the vendor library,
-which then made them all, so a prompt takes the parts' own views of the stacked matrices where they are (`apart_in`,
-`apart_out`).
+which then made them all, so a prompt takes the parts' own views of the stacked matrices there (`APART_IN_OUTPUTS`,
+`apart_out`); both ways' times stand at the limits.
 
 What a mixer that joins offers (`Mixer.can_join`): `joint_input` and `joint_output` (its first and
 last `Linear`), `joint_layout(ff, limit, slope)` (how the stacked rows lie), `rotation()`,
@@ -34,15 +34,18 @@ from mini_infer_amd.parts.base import FeedForward, LayerCache, Mixer, StepContex
 ROW_STEP = 8  # rows of stacked products and of joined inner rows begin on boundaries of as many elements
 
 
-# Where bfloat16 products are made apart (bfloat16 only; the 32-bit engine's own product has no such choice).
-# The first product, by rows x stacked features, microseconds together / apart at 8B and 1B widths:
-#     512 x 34592    147 / 128      1024 x 13088    96 / 108      256 x 34592     83 / 94
-#     2048 x 34592   466 / 430      2048 x 11296   255 / 155      2048 x 6176     59 / 61
-#     4096 x 34592   936 / 794      2048 x 19360   182 / 130      1024 x 19360    81 / 75
+# Where bfloat16 products are made apart (bfloat16 only; the 32-bit engine's own product has no such choice).  The limits were drawn when the vendor
+# library made them all; with the engine's own tiles in its place, microseconds together / apart:
+# the first product, by rows x stacked features at 8B and 1B widths (then)
+#     512 x 34592    142 / 132 (147 / 128)      1024 x 11168    45 / 54 ( 96 / 108)      256 x 34592     85 / 101 (83 / 94)
+#     2048 x 34592   431 / 436 (466 / 430)      2048 x 11168    82 / 81 (255 / 155)      2048 x 6176     46 / 57  (59 / 61)
+#     4096 x 34592   812 / 815 (936 / 794)      2048 x 19360   133 / 135 (182 / 130)     1024 x 19360    77 / 76  (81 / 75)
+#     1501 x 34592   331 / 344                  1501 x 19360    99 / 112
+# so above the limit they are level, and at some row counts together is faster by up to 14 %;
 APART_IN_OUTPUTS = 1 << 24
-# The last product, by rows and by K (3072 + 14336, 1536 + 8192, 3072 + 3584 into 4096 or 2048 features), 256 /
-# 512 / 2048 rows: 113 / 70, 176 / 100, 377 / 239; 28 / 43, 33 / 47, 78 / 87; 25 / 40, 41 / 45, 91 / 98.  (Up to
-# 128 rows a long K goes to the engine's own product in pieces.)
+# the last product, by K (3072 + 14336 into 4096 features, 1536 + 8192 and 3072 + 4096 into 2048) at 256 / 512 / 1501 / 2048 rows: 57 / 67, 87 / 122,
+# 295 / 199, 225 / 239 (then 113 / 70, 176 / 100 and 377 / 239 at 256, 512 and 2048); 26 / 33, 41 / 49, 72 / 79, 87 / 93; 21 / 32, 31 / 39, 61 / 66, 65 /
+# 71.  (Up to 128 rows a long K goes to the engine's own product in pieces.)
 APART_OUT_ROWS, APART_OUT_K = 128, 12288
 
 
