@@ -33,6 +33,8 @@
 
 #include <math.h>
 
+#include <type_traits>
+
 namespace {
 
 template <typename T>
@@ -642,6 +644,109 @@ __global__ __launch_bounds__(256) void expert_rows_mfma_kernel(
   }
 }
 
+// The same sums in the same order where the expert's rows lie on whole cache lines and a wave's quarter of K is whole pairs of steps (K a
+// multiple of 256): bound by reading the chosen experts' weights once, which are therefore read as whole lines, non-temporal (common.h).
+// An expert with more than 16 pairs has RT = 2 row tiles use each weight operand: its weights are then read once for 32 pairs, not for 16.
+// U steps are asked for before the first is used (8 instead of 4: within 1 %).  16 experts of 7168 x 4096 and 4096 x 3584, 8 tokens with two choices
+// each (some 550 and 275 MB): 99.4 -> 86.3 and 51.3 -> 43.9 us (6.4 TB/s); of 4096 x 3072 and 3072 x 2048, 64 tokens: 84.2 -> 67.7 and 46.3 -> 36.7.
+template <int MODE, int RT, int U>
+__device__ __forceinline__ void expert_lines(f32x4_e (*meet)[3][2][MI_WAVE], const bf16_t* __restrict__ src, int64_t src_stride, int src_div,
+                                             const bf16_t* __restrict__ weight, const int* __restrict__ listed, int begin, int end,
+                                             const float* __restrict__ pair_weight, bf16_t* __restrict__ out, int64_t out_stride, int k_dim, int features,
+                                             int f0) {
+  constexpr bool GATED = MODE == EXPERT_SILU_GATED;
+  constexpr int WT = GATED ? 2 : 1;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / MI_WAVE), lane = threadIdx.x % MI_WAVE;
+  const int col = lane % 16, quad = lane / 16;
+  uint32_t lower[WT], upper[WT];  // offsets of this lane's 16 bytes from the expert's first weight row (past the end: the last feature again)
+#pragma unroll
+  for (int t = 0; t < WT; ++t) {
+    const int row = f0 + line_row_of_lane(lane);
+    lower[t] = (uint32_t)(min(row, features - 1) + t * features) * (uint32_t)(k_dim * 2) + line_chunk_of_lane(lane);
+    upper[t] = (uint32_t)(min(row + 8, features - 1) + t * features) * (uint32_t)(k_dim * 2) + line_chunk_of_lane(lane);
+  }
+  const int quarter = k_dim / 128;  // steps of 32 a wave: even
+  const int lo = quarter * wave, hi = lo + quarter;
+  for (int chunk = begin; chunk < end; chunk += 16 * RT) {
+    int pair[RT];
+    const bf16_t* x_row[RT];
+#pragma unroll
+    for (int i = 0; i < RT; ++i) {  // (lanes past the expert's last pair read the chunk's first row; their sums are not written)
+      pair[i] = chunk + 16 * i + col < end ? listed[chunk + 16 * i + col] : -1;
+      x_row[i] = src + (int64_t)((pair[i] >= 0 ? pair[i] : listed[chunk]) / src_div) * src_stride + quad * 8;
+    }
+    f32x4_e acc[WT][RT];
+#pragma unroll
+    for (int t = 0; t < WT; ++t)
+#pragma unroll
+      for (int i = 0; i < RT; ++i) acc[t][i] = f32x4_e{0.f, 0.f, 0.f, 0.f};
+    auto some = [&](int step, auto count) {  // that many steps from `step` on
+      constexpr int N = decltype(count)::value;
+      bf16x8_t a[N][WT], b[N][RT];
+#pragma unroll
+      for (int u = 0; u < N; u += 2)
+#pragma unroll
+        for (int t = 0; t < WT; ++t) load_line_pair(weight, step + u, lower[t], upper[t], a[u][t], a[u + 1][t]);
+#pragma unroll
+      for (int u = 0; u < N; ++u)
+#pragma unroll
+        for (int i = 0; i < RT; ++i) b[u][i] = *reinterpret_cast<const bf16x8_t*>(x_row[i] + (step + u) * 32);
+#pragma unroll
+      for (int u = 0; u < N; u += 2) {
+#pragma unroll
+        for (int t = 0; t < WT; ++t) lines_to_operands(a[u][t], a[u + 1][t]);
+#pragma unroll
+        for (int v = 0; v < 2; ++v)
+#pragma unroll
+          for (int t = 0; t < WT; ++t)
+#pragma unroll
+            for (int i = 0; i < RT; ++i) acc[t][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u + v][t], b[u + v][i], acc[t][i], 0, 0, 0);
+      }
+    };
+    int step = lo;
+    for (; step + U <= hi; step += U) some(step, std::integral_constant<int, U>{});
+    for (; step < hi; step += 2) some(step, std::integral_constant<int, 2>{});
+    __syncthreads();  // (the last chunk's sums have been read)
+    if (wave > 0) {
+#pragma unroll
+      for (int t = 0; t < WT; ++t)
+#pragma unroll
+        for (int i = 0; i < RT; ++i) meet[t][wave - 1][i][lane] = acc[t][i];
+    }
+    __syncthreads();
+    if (wave > 0) continue;
+#pragma unroll
+    for (int i = 0; i < RT; ++i) {
+      if (pair[i] < 0) continue;
+#pragma unroll
+      for (int w = 0; w < 3; ++w)
+#pragma unroll
+        for (int t = 0; t < WT; ++t) acc[t][i] += meet[t][w][i][lane];
+      bf16_t* o = out + (int64_t)pair[i] * out_stride;
+      const float pw = MODE == EXPERT_SQUARED_RELU && pair_weight != nullptr ? pair_weight[pair[i]] : 1.f;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int f = f0 + 4 * quad + r;
+        if (f < features) o[f] = expert_feature<bf16_t, MODE, float>(acc[0][i][r], acc[WT - 1][i][r], pw);
+      }
+    }
+  }
+}
+
+template <int MODE>
+__global__ __launch_bounds__(256) void expert_lines_kernel(
+    const bf16_t* __restrict__ src, int64_t src_stride, int src_div, const bf16_t* __restrict__ weight,
+    int64_t expert_stride, const int* __restrict__ listed, const int* __restrict__ first,
+    const float* __restrict__ pair_weight, bf16_t* __restrict__ out, int64_t out_stride, int k_dim, int features) {
+  __shared__ f32x4_e meet[MODE == EXPERT_SILU_GATED ? 2 : 1][3][2][MI_WAVE];
+  const int e = blockIdx.y;
+  const int begin = first[e], end = first[e + 1];
+  if (begin >= end) return;  // nobody chose this expert (the whole block leaves)
+  const bf16_t* w = weight + (int64_t)e * expert_stride;
+  if (end - begin <= 16) expert_lines<MODE, 1, 4>(meet, src, src_stride, src_div, w, listed, begin, end, pair_weight, out, out_stride, k_dim, features, blockIdx.x * 16);
+  else expert_lines<MODE, 2, 4>(meet, src, src_stride, src_div, w, listed, begin, end, pair_weight, out, out_stride, k_dim, features, blockIdx.x * 16);
+}
+
 // Many rows an expert (a prompt): a block owns one expert and 64 of its output features, a wave 16 of
 // them over all of K, and the expert's listed pairs are taken 64 rows a pass: per step of 32 elements a wave
 // reads its 16 weight rows once (16 bytes a lane) and the four row tiles' input rows (the same for the
@@ -930,10 +1035,17 @@ extern "C" int mi_expert_rows(int dtype, int mode, const void* src, int64_t src_
   expert_rows_mfma_kernel<MODE><<<grid, 256, 0, stream>>>((const bf16_t*)src, src_stride, src_div, (const bf16_t*)weight, \
                                                           expert_stride, listed, first, pair_weight, (bf16_t*)out,    \
                                                           out_stride, k_dim, features)
+#define MI_LINES(MODE)                                                                                              \
+  expert_lines_kernel<MODE><<<grid, 256, 0, stream>>>((const bf16_t*)src, src_stride, src_div, (const bf16_t*)weight, \
+                                                      expert_stride, listed, first, pair_weight, (bf16_t*)out,        \
+                                                      out_stride, k_dim, features)
+    const bool lines = k_dim % 256 == 0 && (uintptr_t)weight % 128 == 0 && expert_stride < ((int64_t)1 << 30);  // (32-bit byte offsets)
     if (many_rows) MI_BY_MODE(MI_TILES);
+    else if (lines) MI_BY_MODE(MI_LINES);
     else MI_BY_MODE(MI_MFMA);
 #undef MI_TILES
 #undef MI_MFMA
+#undef MI_LINES
     MI_CHECK_LAUNCH("expert_rows_mfma");
     return MI_OK;
   }

@@ -413,6 +413,39 @@ def test_the_router_and_both_forms_of_the_experts(dtype, rows, width, ff, expert
         np.testing.assert_allclose(got, want, rtol=0, atol=tolerance(dtype, 8) * max(1.0, np.abs(want).max()))
 
 
+@pytest.mark.parametrize("activation", ["silu_gated", "squared_relu"])
+@pytest.mark.parametrize("width, ff, counts", [
+    (256, 256, [0, 1, 15, 16, 17]), (512, 264, [33, 0, 32, 31]), (1792, 512, [64, 2]), (3072, 40, [16, 49, 1]), (768, 1280, [5])])
+def test_experts_read_in_whole_lines_give_the_bits_of_those_read_in_pieces(activation, width, ff, counts):
+    """Whole cache lines and two tiles of 16 pairs a pass against 16-byte pieces and one tile (weights that do not begin on a line): the same
+    sums in the same order; and both against float64, as the tests of the other forms are."""
+    from mini_infer_amd import ops
+
+    rng = np.random.default_rng(width + ff)
+    experts, rows = len(counts), sum(counts)
+    features = 2 * ff if activation == "silu_gated" else ff
+    x = dev(rng.standard_normal((rows, width)), torch.bfloat16)
+
+    def off_lines(t):
+        room = torch.empty(t.numel() + 64, dtype=t.dtype, device=t.device)
+        at = (8 - room.data_ptr() // 2) % 64  # elements to 16 bytes behind a line
+        return room[at:at + t.numel()].view(t.shape).copy_(t)
+
+    up = dev(rng.standard_normal((experts, features, width)) / np.sqrt(width), torch.bfloat16)
+    down = dev(rng.standard_normal((experts, width, ff)) / np.sqrt(ff), torch.bfloat16)
+    picks = rng.permutation(np.repeat(np.arange(experts, dtype=np.int32), counts))
+    chosen, w = ints(picks.tolist()).reshape(rows, 1), torch.ones((rows, 1), device=DEV)
+    assert up.data_ptr() % 128 == 0 and off_lines(up).data_ptr() % 128 == 16
+    got = ops.experts_by_expert(x, up, down, chosen, w, tiles="rows", activation=activation)
+    assert torch.equal(got, ops.experts_by_expert(x, off_lines(up), off_lines(down), chosen, w, tiles="rows", activation=activation))
+    x64, u64, d64 = x.double().cpu(), up.double().cpu(), down.double().cpu()
+    for r in range(rows):
+        z = u64[picks[r]] @ x64[r]
+        act = torch.nn.functional.silu(z[:ff]) * z[ff:] if activation == "silu_gated" else torch.relu(z) ** 2
+        want = d64[picks[r]] @ act
+        assert (got[r].double().cpu() - want).abs().max() < 2 ** -6 * max(1.0, want.abs().max()), (r, picks[r])
+
+
 # ---------------------------------------------------------------------------------------------
 # each mixer and each feed-forward alone in a one-layer model
 # ---------------------------------------------------------------------------------------------
