@@ -51,6 +51,7 @@ struct ScanArgs {
   float* out;  // float32 [tokens, heads * vdim]
   const int* again;  // null, or one flag for 16 columns [requests][heads][ceil(vdim / 16)]: the columns to be taken
   int heads, groups, dim, vdim;
+  bool whole_runs;  // rows of q and k can be read a lane's run at a time
 };
 
 template <typename T>
@@ -95,6 +96,85 @@ __device__ __forceinline__ double lanes_sum(double v) {
 #pragma unroll
   for (int off = 1; off < L; off <<= 1) v += __shfl_xor(v, off, MI_WAVE);
   return v;
+}
+
+// R values of a row from `at` on as float32, zeros from `dim` on; `whole`: they can be read in pieces of 16 bytes (of all R where those are fewer), and dim
+// is a multiple of R.
+template <typename T, int R>
+__device__ __forceinline__ void run_of_row(const T* row, int at, int dim, bool whole, float (&v)[R]) {
+  if (whole) {
+    constexpr int V = sizeof(T) == 2 && R >= 8 ? 8 : 4;
+#pragma unroll
+    for (int i = 0; i < R; i += V) {
+      float some[V];
+      if constexpr (V == 8) {
+        const uint4 got = *reinterpret_cast<const uint4*>(row + (at < dim ? at + i : 0));
+        const uint32_t words[4] = {got.x, got.y, got.z, got.w};
+#pragma unroll
+        for (int w = 0; w < 4; ++w) some[2 * w] = __uint_as_float(words[w] << 16), some[2 * w + 1] = __uint_as_float(words[w] & 0xFFFF0000u);
+      } else {
+        mi_load_cols<T, V>(row + (at < dim ? at + i : 0), some);
+      }
+#pragma unroll
+      for (int j = 0; j < V; ++j) v[i + j] = at < dim ? some[j] : 0.f;
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < R; ++i) v[i] = at + i < dim ? to_f32(row[at + i]) : 0.f;
+  }
+}
+
+// One token of a request, a decay per head: bound by reading and writing its state.  Every lane reads what its rows of S need itself, beside the state;
+// nothing goes through LDS.  The arithmetic is that of the walk below, term by term.  40 requests of 64 heads of 128 x 64: 37.3 -> 34.2 us.  (With a
+// decay per channel each column's lanes would make all of their decays again, 16 heads of 128 x 256 46 -> 72 us: those share them through LDS.)
+template <typename T, int R, int L>
+__device__ __forceinline__ void decay_token(const ScanArgs& p, int64_t t, int slot, int head, int col0) {
+  using A = typename Wide<T>::type;
+  constexpr bool WIDE = sizeof(T) == 4;
+  const int part = threadIdx.x % L, col = col0 + threadIdx.x / L;
+  const bool live = col < p.vdim;
+  const int at = part * R, grp = head / (p.heads / p.groups);
+  float* mine = p.state + (int64_t)((slot < 0 || slot >= p.num_slots) ? p.num_slots : slot) * p.state_stride +
+                ((int64_t)head * p.vdim + (live ? col : 0)) * (R * L) + at;
+  float S[R], q[R], k[R];
+#pragma unroll
+  for (int i = 0; i < R; i += 4) {
+    const float4 got = *reinterpret_cast<const float4*>(mine + i);
+    S[i] = got.x, S[i + 1] = got.y, S[i + 2] = got.z, S[i + 3] = got.w;
+  }
+  run_of_row<T, R>((const T*)p.q + p.q_col + t * p.q_stride + (int64_t)grp * p.dim, at, p.dim, p.whole_runs, q);
+  run_of_row<T, R>((const T*)p.k + p.k_col + t * p.k_stride + (int64_t)grp * p.dim, at, p.dim, p.whole_runs, k);
+  const float raw = to_f32(((const T*)p.gate)[p.gate_col + t * p.gate_stride + head]), head_bias = p.gate_bias[head];
+  const float x = live ? to_f32(((const T*)p.v)[p.v_col + t * p.v_stride + (int64_t)head * p.vdim + col]) : 0.f;
+  const float skip = p.skip ? p.skip[head] : 0.f;
+  float a, dt;
+  if constexpr (WIDE) {
+    const double step = soft_plus<double>((double)raw + (double)head_bias);
+    a = (float)exp(-exp((double)p.rate[head]) * step);
+    dt = (float)step;
+  } else {
+    const float rate = expf(p.rate[head]) * 1.4426950408889634f;
+    dt = mi_soft_plus_fast(raw + head_bias);
+    a = __builtin_amdgcn_exp2f(-rate * dt);
+  }
+  const float vv = x * dt;
+  A acc = 0;
+#pragma unroll
+  for (int i = 0; i < R; ++i) {
+    const float qi = q[i] * p.q_scale;
+    S[i] = fmaf(k[i], vv, a * S[i]);
+    if constexpr (WIDE) acc = fma((double)S[i], (double)qi, acc);
+    else acc = fmaf(S[i], qi, acc);
+  }
+  acc = lanes_sum<L>(acc);
+  if (!live) return;
+  if (part == 0) {
+    if constexpr (WIDE) acc = fma((double)skip, (double)x, acc);
+    else acc = fmaf(skip, x, acc);
+    p.out[t * ((int64_t)p.heads * p.vdim) + (int64_t)head * p.vdim + col] = (float)acc;
+  }
+#pragma unroll
+  for (int i = 0; i < R; i += 4) *reinterpret_cast<float4*>(mine + i) = make_float4(S[i], S[i + 1], S[i + 2], S[i + 3]);
 }
 
 // Decoded tokens, short portions and the 32-bit engine; long portions of bfloat16 steps go in chunks (decay_chunks.hip).
@@ -177,10 +257,11 @@ __device__ __forceinline__ void decay_scan_columns(const ScanArgs& p, int b, int
       v_raw[i] = (tt < n && col0 + cc < p.vdim) ? to_f32(v_rows[(int64_t)(t0 + tt) * p.v_stride + cc]) : 0.f;
     }
   };
-  auto put = [&]() {
+  auto put = [&](int n) {
 #pragma unroll
     for (int i = 0; i < EACH; ++i) {
       const int e = tid + i * 256, tt = e / DP, d = e % DP;
+      if (i * 256 >= n * DP) continue;  // (a tile of few tokens: no decays of others)
       const int at = tt * LP + d + (d / R) * (RUN - R);
       q_lds[at] = q_raw[i] * p.q_scale;
       k_lds[at] = k_raw[i];
@@ -241,7 +322,7 @@ __device__ __forceinline__ void decay_scan_columns(const ScanArgs& p, int b, int
   for (int t0 = first; t0 < last; t0 += SCAN_TILE) {
     const int n = min(SCAN_TILE, last - t0);
     __syncthreads();  // the last tile has been walked
-    put();
+    put(n);
     __syncthreads();
     if (t0 + SCAN_TILE < last) ask(t0 + SCAN_TILE, min(SCAN_TILE, last - t0 - SCAN_TILE));  // (waits in registers through the walk)
     auto step = [&](int tt, const Operands& o) {
@@ -279,9 +360,25 @@ __device__ __forceinline__ void decay_scan_columns(const ScanArgs& p, int b, int
   }
 }
 
+// Blocks: a request's heads and columns side by side, so that they spread over the XCDs (workgroups are dealt to the 8 of them in turn), and the last
+// request first: a step's long portion commonly comes last, and its chain should not begin when everything else is done.  With the requests
+// side by side every eighth block was the long portion's where requests come in 8s: 31 single tokens beside 64 of 64 heads of 128 x 64 184 us, so 34;
+// 16 heads of 128 x 256 254 / 66.  Heads go round before columns: a head's column blocks then share an XCD's L2 (512 tokens of 64 heads 144 us, 164
+// the other way).
 template <typename T, int MODE, int R, int L>
-__global__ __launch_bounds__(256) void decay_scan_kernel(ScanArgs p) {
-  decay_scan_columns<T, MODE, R, L, false>(p, blockIdx.x, blockIdx.y, blockIdx.z * (256 / L));
+__global__ __launch_bounds__(256) void decay_scan_kernel(ScanArgs p, int requests) {
+  constexpr int COLS = 256 / L;
+  const int each = p.heads * ((p.vdim + COLS - 1) / COLS);
+  const int b = requests - 1 - (int)(blockIdx.x / each), rest = (int)(blockIdx.x % each);
+  const int head = rest % p.heads, col0 = rest / p.heads * COLS;
+  if constexpr (MODE == DECAY_PER_HEAD) {
+    const int first = p.cu[b];
+    if (p.cu[b + 1] - first == 1) {
+      decay_token<T, R, L>(p, first, p.slots[b], head, col0);
+      return;
+    }
+  }
+  decay_scan_columns<T, MODE, R, L, false>(p, b, head, col0);
 }
 
 // the same for columns that the chunks' walk has flagged
@@ -310,11 +407,17 @@ inline void scan_shape(int dim, int* rows, int* lanes) {
 }
 
 template <typename T, int MODE>
-int launch_scan(const ScanArgs& p, int requests, hipStream_t stream) {
+int launch_scan(ScanArgs p, int requests, hipStream_t stream) {
   int rows, lanes;
   scan_shape(p.dim, &rows, &lanes);
-  dim3 grid(requests, p.heads, ceil_div(p.vdim, 256 / lanes));
-#define MI_SCAN(RR, LL) decay_scan_kernel<T, MODE, RR, LL><<<grid, 256, 0, stream>>>(p)
+  const int piece = min(16, rows * (int)sizeof(T));
+  auto in_pieces = [&](const void* row, int64_t stride, int col) {
+    return ((uintptr_t)row + (uintptr_t)col * sizeof(T)) % piece == 0 && stride * sizeof(T) % piece == 0;
+  };
+  p.whole_runs = p.dim % rows == 0 && in_pieces(p.q, p.q_stride, p.q_col) && in_pieces(p.k, p.k_stride, p.k_col);
+  const int64_t grid = (int64_t)requests * p.heads * ceil_div(p.vdim, 256 / lanes);
+  MI_REQUIRE(grid < ((int64_t)1 << 31), "decay_scan: %lld blocks are too many", (long long)grid);
+#define MI_SCAN(RR, LL) decay_scan_kernel<T, MODE, RR, LL><<<(unsigned)grid, 256, 0, stream>>>(p, requests)
   if (rows == 4) MI_SCAN(4, 4);
   else if (rows == 8 && lanes == 4) MI_SCAN(8, 4);
   else if (rows == 8 && lanes == 8) MI_SCAN(8, 8);
@@ -470,7 +573,7 @@ extern "C" int mi_decay_scan(int dtype, int mode, const void* q, int64_t q_strid
   p.q_col = q_col, p.k_col = k_col, p.v_col = v_col, p.gate_col = gate_col;
   p.gate_bias = gate_bias, p.rate = rate, p.skip = skip, p.inv_tau = inv_tau, p.q_scale = q_scale;
   p.state = state, p.state_stride = state_stride, p.cu = cu, p.slots = slots, p.num_slots = num_slots, p.out = out, p.again = nullptr;
-  p.heads = heads, p.groups = groups, p.dim = dim, p.vdim = vdim;
+  p.heads = heads, p.groups = groups, p.dim = dim, p.vdim = vdim, p.whole_runs = false;
   if (dtype == MI_F32) return mode == 0 ? launch_scan<float, DECAY_PER_CHANNEL>(p, num_requests, stream)
                                         : launch_scan<float, DECAY_PER_HEAD>(p, num_requests, stream);
   return mode == 0 ? launch_scan<bf16_t, DECAY_PER_CHANNEL>(p, num_requests, stream)
@@ -488,7 +591,7 @@ int mi_decay_scan_again(int mode, const void* q, int64_t q_stride, int q_col, co
   p.q_col = q_col, p.k_col = k_col, p.v_col = v_col, p.gate_col = gate_col;
   p.gate_bias = gate_bias, p.rate = rate, p.skip = skip, p.inv_tau = inv_tau, p.q_scale = q_scale;
   p.state = state, p.state_stride = state_stride, p.cu = cu, p.slots = slots, p.num_slots = num_slots, p.out = out, p.again = again;
-  p.heads = heads, p.groups = groups, p.dim = dim, p.vdim = vdim;
+  p.heads = heads, p.groups = groups, p.dim = dim, p.vdim = vdim, p.whole_runs = false;
   return mode == 0 ? launch_scan_again<DECAY_PER_CHANNEL>(p, num_requests, stream) : launch_scan_again<DECAY_PER_HEAD>(p, num_requests, stream);
 }
 

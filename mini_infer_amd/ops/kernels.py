@@ -2445,17 +2445,18 @@ def delta_state_shape(heads: int, dim: int, vdim: int) -> tuple[int, int, int]:
 # Microseconds of a recurrence over a step's rows with keys of up to so many columns: token by token (the launches, a request and a
 # token on a full chip, a token of the longest portion) and in chunks of 32 (the launches, a request on a full chip, a chunk of the
 # longest portion).  Fitted to 1,508 measured pairs: 1 to 100 requests of 8 to 512 tokens, single tokens beside one portion, 4 to 80
-# heads of 64 to 512 columns; half of the times are within 5 %.
+# heads of 64 to 512 columns; half of the times are within 5 %.  (A request's share of the decays token by token: fitted to 8 to 80 single
+# tokens of 16 to 64 heads since their blocks spread over the XCDs; beside a portion these expect 10 to 25 % more than is measured.)
 _SCAN_TIMES = {
     ("delta", 64): (6.95, 0.89, 0.093, 0.288, 18.3, 2.33, 1.82),
     ("delta", 128): (8.39, 2.13, 0.161, 0.428, 21, 3.14, 2.26),
     ("delta", 256): (7.82, 3.4, 0.288, 0.62, 24.7, 7.38, 4.32),
-    ("per_head", 64): (3.85, 0.356, 0.0355, 0.252, 13.4, 0.971, 1.13),
-    ("per_head", 128): (3.43, 0.851, 0.0864, 0.303, 14, 1.68, 1.52),
-    ("per_head", 256): (2.44, 2.06, 0.19, 0.472, 16.4, 3.59, 2.36),
-    ("per_channel", 64): (3.98, 0.361, 0.0473, 0.267, 17.5, 1.57, 1.05),
-    ("per_channel", 128): (3.28, 1.18, 0.121, 0.348, 23.4, 2.35, 1.71),
-    ("per_channel", 256): (1.11, 3.09, 0.256, 0.58, 31.6, 5.51, 3.08),
+    ("per_head", 64): (3.85, 0.33, 0.0355, 0.252, 13.4, 0.971, 1.13),
+    ("per_head", 128): (3.43, 0.61, 0.0864, 0.303, 14, 1.68, 1.52),
+    ("per_head", 256): (2.44, 1.65, 0.19, 0.472, 16.4, 3.59, 2.36),
+    ("per_channel", 64): (3.98, 0.32, 0.0473, 0.267, 17.5, 1.57, 1.05),
+    ("per_channel", 128): (3.28, 0.775, 0.121, 0.348, 23.4, 2.35, 1.71),
+    ("per_channel", 256): (1.11, 2.1, 0.256, 0.58, 31.6, 5.51, 3.08),
 }
 
 
@@ -2466,10 +2467,6 @@ def scan_times(kind: str, tokens: int, requests: int, longest: int | None, heads
     launches, request, token, chain, chunk_launches, chunk_request, chunk_chain = _SCAN_TIMES[kind, 64 if dim <= 64 else 128 if dim <= 128 else 256]
     longest = max(1, tokens - requests + 1) if longest is None else longest
     full = heads * -(-vdim // 16) / 256  # of the chip, by one request
-    if kind != "delta" and requests % 8 == 0 and longest * requests >= 2 * tokens:
-        # (that kernel's blocks go round the requests first, so of 8, 16, .. requests one has all its blocks on one of the 8 XCDs: 256
-        # tokens of 48 heads of 128 x 64 beside 15 single tokens take 288 microseconds, beside 14 or 16 of them 95)
-        chain *= max(1.0, 4 * full)
     walked = launches + request * requests * full + max(token * tokens * full, chain * longest)
     return walked, chunk_launches + chunk_request * requests * full + chunk_chain * longest / 32
 

@@ -336,3 +336,35 @@ def test_a_recorded_step_is_not_taken_for_single_tokens():
         made.append((ops.gated_delta(qkv, proj, 0, heads, 2 * heads, a_log, dt_bias, weight, state, cu, torch.arange(count, dtype=torch.int32, device=DEV),
                                      heads=heads, kv_heads=heads, dim=dim, vdim=dim, eps=1e-6), state))
     assert torch.equal(made[0][0], made[1][0]) and torch.equal(made[0][1], made[1][1])
+
+
+@pytest.mark.parametrize("heads,groups,dim,vdim", [(4, 2, 64, 64), (6, 3, 96, 80), (2, 1, 256, 250), (3, 3, 20, 30), (2, 2, 128, 128), (2, 1, 12, 7)])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("odd", [False, True])
+def test_decay_scan_of_single_tokens_gives_the_bits_of_portions(monkeypatch, heads, groups, dim, vdim, dtype, odd):
+    """A decay per head: three tokens of a request in steps of one beside other portions, each with its state from memory, and as one portion
+    (row runs read in pieces of 16 bytes and one by one); requests without tokens and one without a slot between them."""
+    from mini_infer_amd import ops
+    from mini_infer_amd.ops import kernels
+
+    monkeypatch.setattr(kernels, "chunked_scan_pays", lambda *sizes: False)
+    g = torch.Generator(device=DEV).manual_seed(5)
+    rows = [_rows(g, 3, 2 * groups * dim + heads * vdim + heads, odd).to(dtype) for _ in range(2)]  # of the two requests that are followed
+    bias, rate, skip = (torch.randn(heads, generator=g, device=DEV) for _ in range(3))
+    state = _state(g, 6, ops.decay_state_shape(heads, dim, vdim), dim)
+
+    def step(parts, slots, into):
+        x = torch.cat([p for p in parts if p is not None])
+        if odd:
+            x = torch.nn.functional.pad(x, (1, 0))[:, 1:]
+        cu = _boundaries([0 if p is None else p.shape[0] for p in parts])
+        return ops.decay_scan(x, 0, x, groups * dim, x, 2 * groups * dim, x, 2 * groups * dim + heads * vdim, bias, into, cu,
+                              torch.tensor(slots, dtype=torch.int32, device=DEV), heads=heads, groups=groups, dim=dim, vdim=vdim, per_head=True,
+                              rate=rate, skip=skip)
+
+    whole, single = state.clone(), state.clone()
+    out = step([rows[0], None, rows[1]], [3, 0, 1], whole)
+    for t in range(3):
+        got = step([rows[0][t:t + 1], None, rows[0][:2], rows[1][t:t + 1]], [3, 0, -1, 1], single)
+        assert torch.equal(got[0], out[t]) and torch.equal(got[3], out[3 + t])
+    assert torch.equal(single[:-1], whole[:-1])
