@@ -84,66 +84,109 @@ __global__ __launch_bounds__(256) void short_conv_kernel(
   }
 }
 
-// Long steps whose rows are read four columns at a time: a thread takes CONV_RUN consecutive rows of
-// four channels with the last taps-1 inputs in registers, so a row is read once per run and not once per
-// tap.  The arithmetic is that of short_conv_kernel, term by term.
-#define CONV_RUN 16
-
-template <typename T, int TAPS>
-__global__ __launch_bounds__(256) void short_conv_runs_kernel(
-    const T* __restrict__ x, int64_t x_stride, const float* __restrict__ w, const T* __restrict__ tail,
-    int64_t tail_stride, const int* __restrict__ cu, const int* __restrict__ slots,
-    const int* __restrict__ token_request, T* __restrict__ y, int64_t y_stride, int channels, int num_tokens,
+// Rows that can be read four columns at a time, with 2 to 4 taps: convolution and tail as one launch, whatever the step holds.  Bound by the latency of its
+// loads: a thread makes RUN consecutive rows of four channels, and all they need is asked for at once.  (A walk over 16 rows a thread with the tail's launch
+// behind it, which stood here above 64 rows, took 22 + 4.2 us for 555 + 20 rows of 2,304 channels, one over a request's rows up to 64 21 us for
+// two requests of 25.)  The arithmetic is that of short_conv_kernel, term by term.
+//
+// A request's tail is read for its first BACK rows and written anew; both by the thread that makes the first of them, so that no other reads
+// what it overwrites: rows 1 .. BACK-1 of a request are made by whoever makes its row 0, also past the end of the run that that one lies in.
+template <typename T, int TAPS, int RUN>
+__global__ __launch_bounds__(256) void short_conv_rows_kernel(
+    const T* __restrict__ x, int64_t x_stride, const float* __restrict__ w, T* tail, int64_t tail_stride, const int* __restrict__ cu,
+    const int* __restrict__ slots, const int* __restrict__ token_request, T* __restrict__ y, int64_t y_stride, int channels, int num_tokens,
     int num_slots, const float* __restrict__ bias, int add_input) {
   using A = typename ConvSum<T>::type;
   constexpr int BACK = TAPS - 1;
-  const int c = (blockIdx.x * blockDim.x + threadIdx.x) * 4;
+  const int c = (blockIdx.y * blockDim.x + threadIdx.x) * 4;
   if (c >= channels) return;
-  const int t0 = blockIdx.y * CONV_RUN, t1 = min(num_tokens, t0 + CONV_RUN);
-  A wc[TAPS][4], start[4];
-  float window[BACK > 0 ? BACK : 1][4];  // window[j]: the input `BACK - j` rows ago
+  const int t0 = blockIdx.x * RUN;
+  float wc[4][TAPS], start[4];
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
-    start[e] = bias ? (A)bias[c + e] : (A)0;
+    start[e] = bias ? bias[c + e] : 0.f;
     if constexpr (TAPS == 4) {  // (a channel's taps at once: one by one every load would touch a line a lane)
-      float taps_of[4];
-      mi_load_cols<float, 4>(w + (int64_t)(c + e) * 4, taps_of);
-#pragma unroll
-      for (int j = 0; j < 4; ++j) wc[j][e] = (A)taps_of[j];
+      mi_load_cols<float, 4>(w + (int64_t)(c + e) * 4, wc[e]);
     } else {
 #pragma unroll
-      for (int j = 0; j < TAPS; ++j) wc[j][e] = (A)w[(int64_t)(c + e) * TAPS + j];
+      for (int j = 0; j < TAPS; ++j) wc[e][j] = w[(int64_t)(c + e) * TAPS + j];
     }
   }
-  int of = -1;  // the request the window belongs to
-  for (int t = t0; t < t1; ++t) {
-    const int b = token_request[t];
-    if (b != of) {
-      of = b;
-      const int i = t - cu[b];
-      const int slot = slots[b];
-      const T* mine = tail + (int64_t)((slot < 0 || slot >= num_slots) ? num_slots : slot) * tail_stride;
-#pragma unroll
-      for (int j = 0; j < BACK; ++j) {
-        const int at = i - BACK + j;
-        if (at >= 0) mi_load_cols<T, 4>(x + (int64_t)(t - BACK + j) * x_stride + c, window[j]);
-        else mi_load_cols<T, 4>(mine + (int64_t)(BACK + at) * channels + c, window[j]);
-      }
-    }
-    float now[4], made[4];
-    mi_load_cols<T, 4>(x + (int64_t)t * x_stride + c, now);
+  auto make = [&](int t, const float (&in)[TAPS][4]) {  // in[j]: the row BACK - j ago
+    float made[4];
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
-      A sum = start[e];
+      A sum = (A)start[e];
 #pragma unroll
-      for (int j = 0; j < BACK; ++j) sum = fma(wc[j][e], (A)window[j][e], sum);
-      sum = fma(wc[BACK][e], (A)now[e], sum);
-      made[e] = conv_result(sum, now[e], add_input);
-#pragma unroll
-      for (int j = 0; j + 1 < BACK; ++j) window[j][e] = window[j + 1][e];
-      if constexpr (BACK > 0) window[BACK - 1][e] = now[e];
+      for (int j = 0; j < TAPS; ++j) sum = fma((A)wc[e][j], (A)in[j][e], sum);
+      made[e] = conv_result(sum, in[BACK][e], add_input);
     }
     mi_store_cols<T, 4>(y + (int64_t)t * y_stride + c, made);
+  };
+  const int b0 = token_request[t0], first0 = cu[b0];
+  if (t0 - first0 >= BACK && t0 + RUN <= min(num_tokens, cu[b0 + 1])) {  // inside a request, away from its first rows
+    float rows[RUN + BACK][4];
+#pragma unroll
+    for (int i = 0; i < RUN + BACK; ++i) mi_load_cols<T, 4>(x + (int64_t)(t0 - BACK + i) * x_stride + c, rows[i]);
+#pragma unroll
+    for (int i = 0; i < RUN; ++i) {
+      float in[TAPS][4];
+#pragma unroll
+      for (int j = 0; j < TAPS; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) in[j][e] = rows[i + j][e];
+      make(t0 + i, in);
+    }
+    return;
+  }
+  const int t1 = min(num_tokens, t0 + RUN);
+  int t = t0;
+  if (t0 > first0 && t0 - first0 < BACK) t = first0 + BACK;  // (made with the request's row 0, as far as they are its)
+  if (t > cu[b0 + 1]) t = cu[b0 + 1];
+  while (t < t1) {  // the part of a request from row t on
+    const int b = token_request[t], first = cu[b], end = cu[b + 1];
+    const int upto = min(end, t == first ? max(t1, first + BACK) : t1);
+    const int slot = slots[b];
+    T* mine = tail + (int64_t)((slot < 0 || slot >= num_slots) ? num_slots : slot) * tail_stride + c;
+    float window[TAPS][4], old[BACK][4], next[BACK][4];
+    const bool begins = t == first;
+#pragma unroll
+    for (int j = 0; j < BACK; ++j) {
+      if (begins) mi_load_cols<T, 4>(mine + (int64_t)j * channels, window[j]);
+      else mi_load_cols<T, 4>(x + (int64_t)(t - BACK + j) * x_stride + c, window[j]);
+    }
+    if (begins) {
+#pragma unroll
+      for (int j = 0; j < BACK; ++j) {
+        const int at = end - BACK + j;
+        if (at >= first) mi_load_cols<T, 4>(x + (int64_t)at * x_stride + c, next[j]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) old[j][e] = window[j][e];
+      }
+    }
+    for (; t < upto; ++t) {
+      mi_load_cols<T, 4>(x + (int64_t)t * x_stride + c, window[BACK]);
+      make(t, window);
+#pragma unroll
+      for (int j = 0; j < BACK; ++j)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) window[j][e] = window[j + 1][e];
+    }
+    if (begins) {
+#pragma unroll
+      for (int j = 0; j < BACK; ++j) {
+        const int at = end - BACK + j;
+        if (at < first) {  // a short portion: what is still of the tail before it
+#pragma unroll
+          for (int i = 0; i < BACK; ++i)
+            if (i == end - first + j) {
+#pragma unroll
+              for (int e = 0; e < 4; ++e) next[j][e] = old[i][e];
+            }
+        }
+        mi_store_cols<T, 4>(mine + (int64_t)j * channels, next[j]);
+      }
+    }
   }
 }
 
@@ -647,6 +690,37 @@ extern "C" int mi_short_conv(int dtype, const void* x, int64_t x_stride, const f
   MI_REQUIRE(num_requests <= 65535, "short_conv: too many requests");
   MI_REQUIRE(dtype == MI_F32 || dtype == MI_BF16, "short_conv: unknown dtype %d", dtype);
   if (num_tokens == 0 || num_requests == 0) return MI_OK;
+  const size_t elem = dtype == MI_F32 ? 4 : 2;
+  if (taps >= 2 && taps <= 4 && channels % 4 == 0 && x_stride % 4 == 0 && y_stride % 4 == 0 && tail_stride % 4 == 0 &&
+      ((uintptr_t)x | (uintptr_t)y | (uintptr_t)tail) % (4 * elem) == 0 && (uintptr_t)w % 16 == 0 && channels <= 65535 * 1024) {
+    // Rows a thread: more of them read a row 4, 1.75 and 1.4 times, fewer are more threads with shorter ways to memory.  Microseconds with 4 / 8: 1,777 x
+    // 3,328 11.7 / 12.4, 2,048 x 6,144 16.7 / 14.8; with 1 / 8: 673 x 3,072 6.7 / 8.9.
+    const int64_t values = (int64_t)num_tokens * channels;
+    const int run = values <= 2500000 ? 1 : values <= 8000000 ? 4 : 8;
+    dim3 grid(ceil_div(num_tokens, run), ceil_div(channels, 1024));
+#define MI_CONV_OF(T, TAPS, RUN)                                                                                       \
+  short_conv_rows_kernel<T, TAPS, RUN><<<grid, 256, 0, stream>>>((const T*)x, x_stride, w, (T*)tail, tail_stride, cu,  \
+                                                                 slots, token_request, (T*)y, y_stride, channels, num_tokens, num_slots, bias, add_input)
+#define MI_CONV_ROWS(T, TAPS)                  \
+  do {                                         \
+    if (run == 1) MI_CONV_OF(T, TAPS, 1);      \
+    else if (run == 4) MI_CONV_OF(T, TAPS, 4); \
+    else MI_CONV_OF(T, TAPS, 8);               \
+  } while (0)
+    if (dtype == MI_F32) {
+      if (taps == 2) MI_CONV_ROWS(float, 2);
+      else if (taps == 3) MI_CONV_ROWS(float, 3);
+      else MI_CONV_ROWS(float, 4);
+    } else {
+      if (taps == 2) MI_CONV_ROWS(bf16_t, 2);
+      else if (taps == 3) MI_CONV_ROWS(bf16_t, 3);
+      else MI_CONV_ROWS(bf16_t, 4);
+    }
+#undef MI_CONV_ROWS
+#undef MI_CONV_OF
+    MI_CHECK_LAUNCH("short_conv_rows");
+    return MI_OK;
+  }
   const int blocks = ceil_div(channels, 256);
   if (num_tokens <= SHORT_CONV_WALK_ROWS) {
     dim3 grid(blocks, num_requests);
@@ -659,28 +733,7 @@ extern "C" int mi_short_conv(int dtype, const void* x, int64_t x_stride, const f
     MI_CHECK_LAUNCH("short_conv_walk");
     return MI_OK;
   }
-  const size_t elem = dtype == MI_F32 ? 4 : 2;
-  const bool runs = taps >= 2 && taps <= 4 && channels % 4 == 0 && x_stride % 4 == 0 && y_stride % 4 == 0 && tail_stride % 4 == 0 &&
-                    ((uintptr_t)x | (uintptr_t)y | (uintptr_t)tail) % (4 * elem) == 0 && (uintptr_t)w % 16 == 0 &&
-                    ceil_div(num_tokens, CONV_RUN) <= 65535;
-  if (runs) {
-    dim3 grid(ceil_div(channels, 1024), ceil_div(num_tokens, CONV_RUN));
-#define MI_CONV_RUNS(T, TAPS)                                                                                            \
-  short_conv_runs_kernel<T, TAPS><<<grid, 256, 0, stream>>>((const T*)x, x_stride, w, (const T*)tail, tail_stride, cu,   \
-                                                            slots, token_request, (T*)y, y_stride, channels, num_tokens, \
-                                                            num_slots, bias, add_input)
-    if (dtype == MI_F32) {
-      if (taps == 2) MI_CONV_RUNS(float, 2);
-      else if (taps == 3) MI_CONV_RUNS(float, 3);
-      else MI_CONV_RUNS(float, 4);
-    } else {
-      if (taps == 2) MI_CONV_RUNS(bf16_t, 2);
-      else if (taps == 3) MI_CONV_RUNS(bf16_t, 3);
-      else MI_CONV_RUNS(bf16_t, 4);
-    }
-#undef MI_CONV_RUNS
-  }
-  for (int first = runs ? num_tokens : 0; first < num_tokens; first += 65535) {
+  for (int first = 0; first < num_tokens; first += 65535) {
     dim3 grid(blocks, min(65535, num_tokens - first));
     if (dtype == MI_F32)
       short_conv_kernel<float><<<grid, 256, 0, stream>>>((const float*)x, x_stride, w, (const float*)tail, tail_stride, cu,

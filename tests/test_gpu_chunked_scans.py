@@ -368,3 +368,27 @@ def test_decay_scan_of_single_tokens_gives_the_bits_of_portions(monkeypatch, hea
         got = step([rows[0][t:t + 1], None, rows[0][:2], rows[1][t:t + 1]], [3, 0, -1, 1], single)
         assert torch.equal(got[0], out[t]) and torch.equal(got[3], out[3 + t])
     assert torch.equal(single[:-1], whole[:-1])
+
+
+@pytest.mark.parametrize("lengths,channels", [([1, 2, 3, 0, 4, 1, 5, 9, 1], 12), ([70], 1028), ([3, 1] * 8 + [17, 6, 1, 2], 96),
+                                              ([1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 300, 3], 8192), ([2, 1, 3, 990, 13, 4, 1, 1, 29], 8192)])
+@pytest.mark.parametrize("taps", [2, 3, 4])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_short_conv_of_rows_in_fours_gives_the_bits_of_the_general_form(lengths, channels, taps, dtype):
+    """One, four and eight rows a thread (by the step's size), requests that begin and end anywhere in them, twice in a row so that tails are carried:
+    against rows off 16 bytes, which take the launches that stand for any layout."""
+    from mini_infer_amd import ops
+
+    g = torch.Generator(device=DEV).manual_seed(sum(lengths))
+    requests, tokens = len(lengths), sum(lengths)
+    w, bias = torch.randn(channels, taps, generator=g, device=DEV), torch.randn(channels, generator=g, device=DEV)
+    slots = torch.randperm(requests, generator=g, device=DEV).int()
+    of = torch.repeat_interleave(torch.arange(requests, device=DEV), torch.tensor(lengths, device=DEV)).int()
+    tail = torch.randn(requests + 1, taps - 1, channels, generator=g, device=DEV).to(dtype)
+    other = tail.clone()
+    for _ in range(2):
+        x = torch.randn(tokens, channels, generator=g, device=DEV).to(dtype)
+        off = torch.empty(tokens, channels + 1, dtype=dtype, device=DEV)[:, :channels].copy_(x)
+        assert torch.equal(ops.short_conv(x, channels, w, tail, _boundaries(lengths), slots, of, bias=bias),
+                           ops.short_conv(off, channels, w, other, _boundaries(lengths), slots, of, bias=bias))
+        assert torch.equal(tail, other)
