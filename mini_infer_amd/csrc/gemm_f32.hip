@@ -39,6 +39,11 @@ __device__ __forceinline__ float4 four_of_row(const float* row, int at, int k) {
                      at + 3 < k ? row[at + 3] : 0.f);
 }
 
+// What lies between the matrices of one head and the next where a launch makes the products of several side by side (elements).
+struct Heads {
+  int64_t a, w, c;
+};
+
 // Many rows: a block of 4 waves owns BM x 64 outputs, STAGE slices of both operands in LDS, the next ones in
 // flight in registers.  With 64 cycles an instruction the LDS is idle most of the time, so small tiles cost
 // nothing.  BM = 64 (a wave 32 x 32), one slice a stage, where there are at least four blocks a CU to cover one
@@ -47,12 +52,13 @@ __device__ __forceinline__ float4 four_of_row(const float* row, int at, int k) {
 template <int BM, int STAGE, bool ALIGNED>
 __global__ __launch_bounds__(256) void gemm_f32_kernel(const float* __restrict__ a, int64_t lda,
                                                        const float* __restrict__ w, int64_t ldw,
-                                                       float* __restrict__ c, int64_t ldc, int m, int n, int k) {
+                                                       float* __restrict__ c, int64_t ldc, int m, int n, int k, Heads heads) {
   constexpr int LDS_ROW = STAGE * SLICE + 4;  // floats: 16-byte reads of 16 rows fall on different banks
   constexpr int CT = BM == 64 ? 2 : 1;  // 16-column tiles of a wave (it has two tiles of rows)
   constexpr int AL = STAGE * BM / 32, WL = STAGE * BN / 32;  // 16-byte pieces a thread stages
   __shared__ __attribute__((aligned(16))) float a_s[BM][LDS_ROW];
   __shared__ __attribute__((aligned(16))) float w_s[BN][LDS_ROW];
+  a += (int64_t)blockIdx.z * heads.a, w += (int64_t)blockIdx.z * heads.w, c += (int64_t)blockIdx.z * heads.c;
   const int tid = threadIdx.x, wave = tid / MI_WAVE, lane = tid % MI_WAVE;
   const int row0 = blockIdx.y * BM, col0 = blockIdx.x * BN;
   const int wave_row = BM == 64 ? wave / 2 * 32 : 0, wave_col = BM == 64 ? wave % 2 * 32 : wave * 16;
@@ -164,7 +170,8 @@ __device__ __forceinline__ float4 four_in_flight(const float* row, int at, int k
   return make_float4(__uint_as_float(bits[0]), __uint_as_float(bits[1]), __uint_as_float(bits[2]), __uint_as_float(bits[3]));
 }
 
-// Few rows (decode; those that gemm_f32_few_kernel does not take): bound by reading W once.  A block owns 16 * RT rows and 16 * FT features; its 8 waves take
+// Up to a few hundred rows (those that gemm_f32_few_kernel does not take): bound by the matrix instruction, or by what a CU brings in where there are few
+// rows.  A block owns 16 * RT rows and 16 * FT features, as many as leave a block for every CU (f32_micros); its 8 waves take
 // one run of K each (the order above), every wave streams its part of the weights from memory, two slices ahead,
 // and the runs' sums meet in LDS.  LINES: whole lines of W, non-temporal, brought into operand order by lane
 // exchanges (common.h): rows of W on 128 bytes, K a multiple of 32, A on 16 bytes.  PIECES: 16 bytes a load in operand order
@@ -175,10 +182,16 @@ enum { VALUES = 0, PIECES = 1, LINES = 2 };
 template <int RT, int FT, int FORM>
 __global__ __launch_bounds__(SEGMENTS * MI_WAVE) void gemm_f32_rows_kernel(const float* __restrict__ a, int64_t lda,
                                                             const float* __restrict__ w, int64_t ldw,
-                                                            float* __restrict__ c, int64_t ldc, int m, int n, int k) {
-  __shared__ double sums[SEGMENTS][RT * FT][16][17];
+                                                            float* __restrict__ c, int64_t ldc, int m, int n, int k, int row_tiles, int total, Heads heads) {
+  constexpr int AT_ONCE = RT * FT < 4 ? RT * FT : 4;  // tiles whose runs' sums meet in LDS at a time
+  __shared__ double sums[SEGMENTS][AT_ONCE][16][17];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / MI_WAVE), lane = threadIdx.x % MI_WAVE;
-  const int col0 = blockIdx.x * 16 * FT;
+  // (consecutive places go to one XCD: the row tiles that read the same rows of W run at the same time behind one L2)
+  const int place = row_tiles > 1 ? (int)(blockIdx.x % 8 * (gridDim.x / 8) + blockIdx.x / 8) : (int)blockIdx.x;
+  if (place >= total) return;
+  const int row0 = place % row_tiles * (16 * RT), col0 = place / row_tiles * (16 * FT);
+  a += (int64_t)blockIdx.y * heads.a + (int64_t)row0 * lda, w += (int64_t)blockIdx.y * heads.w, c += (int64_t)blockIdx.y * heads.c + (int64_t)row0 * ldc;
+  m -= row0;
   const int r = lane % 16, quad = lane / 16;
   const float* a_row[RT];
   f64x4_t acc[RT][FT];
@@ -280,18 +293,20 @@ __global__ __launch_bounds__(SEGMENTS * MI_WAVE) void gemm_f32_rows_kernel(const
     }
   }
 #pragma unroll
-  for (int i = 0; i < RT; ++i)
+  for (int t0 = 0; t0 < RT * FT; t0 += AT_ONCE) {
+    if (t0 > 0) __syncthreads();
 #pragma unroll
-    for (int f = 0; f < FT; ++f)
+    for (int t = t0; t < t0 + AT_ONCE; ++t)
 #pragma unroll
-      for (int e = 0; e < 4; ++e) sums[wave][i * FT + f][4 * e + quad][r] = acc[i][f][e];
-  __syncthreads();
-  for (int at = threadIdx.x; at < 256 * RT * FT; at += SEGMENTS * MI_WAVE) {
-    const int tile = at / 256, row = tile / FT * 16 + at / 16 % 16, col = col0 + tile % FT * 16 + at % 16;
-    double total = 0.0;
+      for (int e = 0; e < 4; ++e) sums[wave][t - t0][4 * e + quad][r] = acc[t / FT][t % FT][e];
+    __syncthreads();
+    for (int at = threadIdx.x; at < 256 * AT_ONCE; at += SEGMENTS * MI_WAVE) {
+      const int tile = t0 + at / 256, row = tile / FT * 16 + at / 16 % 16, col = col0 + tile % FT * 16 + at % 16;
+      double whole = 0.0;
 #pragma unroll
-    for (int s = 0; s < SEGMENTS; ++s) total += sums[s][tile][at / 16 % 16][at % 16];
-    if (row < m && col < n) c[(int64_t)row * ldc + col] = (float)total;
+      for (int s = 0; s < SEGMENTS; ++s) whole += sums[s][at / 256][at / 16 % 16][at % 16];
+      if (row < m && col < n) c[(int64_t)row * ldc + col] = (float)whole;
+    }
   }
 }
 
@@ -317,7 +332,7 @@ __global__ __launch_bounds__(SEGMENTS * MI_WAVE) void gemm_f32_rows_kernel(const
 // 1,571, but that rounds elsewhere than the norm's launch in front of more rows: a request's logits changed when a fifth one joined.  The
 // factor first, its sum in the order of that launch, has every block add up all rows' squares: o, norm and gate|up of 3 rows at those sizes 33.6 ->
 // 38.6 us.)
-enum { FEW_PLAIN = 0, FEW_GATED = 1, FEW_ROPE = 2 };
+enum { FEW_PLAIN = 0, FEW_GATED = 1, FEW_ROPE = 2, FEW_HEADS = 3 };  // (FEW_HEADS: plain, a product a head)
 
 struct FewRows {  // what FEW_ROPE has beside the product (see the entry)
   const float *cos_t, *sin_t;  // [m][half]
@@ -329,7 +344,8 @@ struct FewRows {  // what FEW_ROPE has beside the product (see the entry)
 template <int G, int FEATURES, int KIND = FEW_PLAIN>
 __global__ __launch_bounds__(SEGMENTS * MI_WAVE) void gemm_f32_few_kernel(const float* __restrict__ a, int64_t lda,
                                                            const float* __restrict__ w, int64_t ldw,
-                                                           float* __restrict__ c, int64_t ldc, int m, int n, int k, int chunk, FewRows with) {
+                                                           float* __restrict__ c, int64_t ldc, int m, int n, int k, int chunk, FewRows with, Heads heads) {
+  if constexpr (KIND == FEW_HEADS) a += (int64_t)blockIdx.y * heads.a, w += (int64_t)blockIdx.y * heads.w, c += (int64_t)blockIdx.y * heads.c;
   extern __shared__ __attribute__((aligned(16))) float4 staged[];  // [wave][slice of the chunk][group of rows][half][piece of K][row]
   __shared__ double sums[SEGMENTS][G][MI_WAVE];
   constexpr int AHEAD = G == 1 ? 4 : 2;
@@ -451,19 +467,19 @@ __global__ __launch_bounds__(SEGMENTS * MI_WAVE) void gemm_f32_few_kernel(const 
 
 template <int BM, int STAGE>
 static void launch_tiles(const float* a, int64_t lda, const float* w, int64_t ldw, float* c, int64_t ldc, int m, int n,
-                         int k, bool aligned, hipStream_t stream) {
-  dim3 grid(ceil_div(n, BN), ceil_div(m, BM));
-  if (aligned) gemm_f32_kernel<BM, STAGE, true><<<grid, 256, 0, stream>>>(a, lda, w, ldw, c, ldc, m, n, k);
-  else gemm_f32_kernel<BM, STAGE, false><<<grid, 256, 0, stream>>>(a, lda, w, ldw, c, ldc, m, n, k);
+                         int k, bool aligned, int count, const Heads& heads, hipStream_t stream) {
+  dim3 grid(ceil_div(n, BN), ceil_div(m, BM), count);
+  if (aligned) gemm_f32_kernel<BM, STAGE, true><<<grid, 256, 0, stream>>>(a, lda, w, ldw, c, ldc, m, n, k, heads);
+  else gemm_f32_kernel<BM, STAGE, false><<<grid, 256, 0, stream>>>(a, lda, w, ldw, c, ldc, m, n, k, heads);
 }
 
 template <int G, int FEATURES, int KIND = FEW_PLAIN>
 static void launch_few(const float* a, int64_t lda, const float* w, int64_t ldw, float* c, int64_t ldc, int m, int n, int k,
-                       hipStream_t stream, const FewRows& with = FewRows()) {
+                       hipStream_t stream, const FewRows& with = FewRows(), int count = 1, const Heads& heads = Heads()) {
   const int chunk = min(segment_slices(k), 16 / G);
   const int blocks = KIND == FEW_ROPE ? (with.q_heads + 2 * with.kv_heads) * (with.head_dim / 16) : ceil_div(n, KIND == FEW_GATED ? 8 : FEATURES);
-  gemm_f32_few_kernel<G, FEATURES, KIND><<<blocks, SEGMENTS * MI_WAVE, SEGMENTS * chunk * G * 32 * sizeof(float4), stream>>>(
-      a, lda, w, ldw, c, ldc, m, n, k, chunk, with);
+  gemm_f32_few_kernel<G, FEATURES, KIND><<<dim3(blocks, count), SEGMENTS * MI_WAVE, SEGMENTS * chunk * G * 32 * sizeof(float4), stream>>>(
+      a, lda, w, ldw, c, ldc, m, n, k, chunk, with, heads);
 }
 
 // A launch of a kind for one or two groups of four rows.
@@ -476,11 +492,12 @@ static void launch_few_of(const float* a, int64_t lda, const float* w, int64_t l
 
 template <int RT, int FT>
 static void launch_rows(const float* a, int64_t lda, const float* w, int64_t ldw, float* c, int64_t ldc, int m, int n,
-                        int k, int form, hipStream_t stream) {
-  const int grid = ceil_div(n, 16 * FT), block = SEGMENTS * MI_WAVE;
-  if (form == LINES) gemm_f32_rows_kernel<RT, FT, LINES><<<grid, block, 0, stream>>>(a, lda, w, ldw, c, ldc, m, n, k);
-  else if (form == PIECES) gemm_f32_rows_kernel<RT, FT, PIECES><<<grid, block, 0, stream>>>(a, lda, w, ldw, c, ldc, m, n, k);
-  else gemm_f32_rows_kernel<RT, FT, VALUES><<<grid, block, 0, stream>>>(a, lda, w, ldw, c, ldc, m, n, k);
+                        int k, int form, int count, const Heads& heads, hipStream_t stream) {
+  const int row_tiles = ceil_div(m, 16 * RT), total = row_tiles * ceil_div(n, 16 * FT), block = SEGMENTS * MI_WAVE;
+  dim3 grid(row_tiles > 1 ? ceil_div(total, 8) * 8 : total, count);
+  if (form == LINES) gemm_f32_rows_kernel<RT, FT, LINES><<<grid, block, 0, stream>>>(a, lda, w, ldw, c, ldc, m, n, k, row_tiles, total, heads);
+  else if (form == PIECES) gemm_f32_rows_kernel<RT, FT, PIECES><<<grid, block, 0, stream>>>(a, lda, w, ldw, c, ldc, m, n, k, row_tiles, total, heads);
+  else gemm_f32_rows_kernel<RT, FT, VALUES><<<grid, block, 0, stream>>>(a, lda, w, ldw, c, ldc, m, n, k, row_tiles, total, heads);
 }
 
 // Whether gemm_f32_few_kernel is the faster one (figures there).
@@ -535,47 +552,113 @@ extern "C" int mi_gemm_f32_rope(const float* a, int64_t lda, const float* w, int
   return MI_OK;
 }
 
-// Which kernel, with microseconds at rows x N x K (weights from memory; 3 rows: in one 16 x 16 product, for groups of four see
-// gemm_f32_few_kernel).  Before: 64-bit multiply-adds on the vector
-// pipe, 4 x 4 outputs a thread, and a kernel of its own for up to 16 rows only.
-//     3 x 2048 x 2048     75.6 ->   9.0     20 x  2048 x 2048   317 ->  15.0     509 x  2048 x 2048    327 ->  82
-//     3 x 16384 x 2048     107 ->  30.7     20 x 16384 x 2048   349 ->  46.0     509 x  3072 x 2048    378 -> 117
-//     3 x 128256 x 2048    419 ->   192     60 x  2048 x 2048   320 ->  26.3     509 x 16384 x 2048   1060 -> 580
-//     3 x 2048 x 8192      322 ->  28.1     60 x 16384 x 2048   355 -> 102       509 x  2048 x 8192   1340 -> 316
-// 3 rows of 16,384 features and more run at the rate of a large copy; 580 us is 59 TFLOP/s, where the vendor
-// library's 64-bit product reaches 64.  Two tiles of features a wave from 8,192 on (fewer blocks below that would
-// leave CUs idle).  Up to 32 rows the streaming kernel always (20 x 128256 x 2048: 325 against 320 for the tiles,
-// 20 x 16384: 46 against 66); up to 64 rows where there are few features (60 x 2048: 26 against 64; 60 x 128256:
-// 810 against 580, every block reads all the rows' activations).  Rows off whole lines, 16-byte pieces (single values waited for one
+// Before the 64-bit matrix instruction (64-bit multiply-adds on the vector pipe, 4 x 4 outputs a thread), microseconds at rows x N x K, weights from
+// memory: 20 x 2048 x 2048 317, 60 x 16384 x 2048 355, 509 x 16384 x 2048 1060 -> 580 (59 TFLOP/s, where the vendor library's 64-bit product
+// reaches 64), 509 x 2048 x 8192 1340 -> 316.  Rows off whole lines, 16-byte pieces (single values waited for one
 // by one before): 1 x 128256 x 2052 684 -> 267, 32 rows 1,410 -> 509; 16 x 4096 x 4096, rows not on a line, 66 -> 23; single values, 8 x
 // 32000 x 4095 415 -> 218.
-extern "C" int mi_gemm_f32(const float* a, int64_t lda, const float* w, int64_t ldw, float* c,
-                           int64_t ldc, int m, int n, int k, hipStream_t stream) {
-  MI_REQUIRE(m >= 0 && n > 0 && k > 0, "gemm_f32: bad sizes m=%d n=%d k=%d", m, n, k);
+
+// The kernels that a call may take: the 16s of rows and of features that a block of gemm_f32_rows_kernel makes, then the others.
+#define F32_ROWS_FORMS(X) X(0, 1, 1) X(1, 1, 2) X(2, 2, 1) X(3, 2, 2) X(4, 4, 1) X(5, 4, 2)
+enum { F32_ROWS = 6, F32_FEW = 6, F32_TILES_32 = 7, F32_TILES_64 = 8, F32_FORMS = 9 };
+
+// Microseconds that a form is expected to take: the rounds of its blocks over the compute units, with the cycles a block is on the matrix pipe (a
+// slice is 128 for each of its 16 x 16 products) and those it loses on converting and moving its operands.  Tiles beside one another on a CU cover
+// one another's waits, one by itself does not.  Within 12 % of what 9 to 256 rows of 3072, 2048 and 16384 x 2048 and of 2048 x 8192 took.
+static double f32_micros(int form, int m, int n, int k, int count, int cus) {
+  const int slices = ceil_div(k, SLICE);
+  auto rounds = [&](int rows, int features) { return (double)ceil_div64((int64_t)ceil_div(m, rows) * ceil_div(n, features) * count, cus); };
+  if (form == F32_TILES_32) {
+    const double r = rounds(32, BN);
+    return (r > 1 ? 0.56 * r + 0.22 : 0.77) * slices;
+  }
+  if (form == F32_TILES_64) {
+    const double r = rounds(64, BN);
+    return (r > 1 ? 1.1 * r + 0.39 : 1.44) * slices;
+  }
+  constexpr int of[F32_ROWS][2] = {
+#define X(I, RT, FT) {RT, FT},
+      F32_ROWS_FORMS(X)
+#undef X
+  };
+  const int rt = of[form][0], ft = of[form][1];
+  const double r = rounds(16 * rt, 16 * ft);
+  return 4.0 + r * (r > 2 ? 1.1 : 1.0) * slices * (128 * rt * ft + 30 * (rt + ft)) / 2100.0;
+}
+
+// The form of m rows for which the four-row products are not taken: the one that is expected to be the fastest.  (All give the same bits.)  Microseconds
+// of what stood here before (up to 32 rows, or 64 with less than 8,192 features, all rows a block; above, tiles through LDS) and this one, weights
+// from memory:
+//     rows            25             64             96             128            256
+//     2048 x 2048     15.1 / 9.6     27.5 / 15.0    50.9 / 22.3    51.3 / 23.6    51.8 / 43.7
+//     3072 x 2048     15.8 / 15.3    28.3 / 22.4    51.1 / 32.8    51.3 / 36.2    82.1 / 67.2
+//     16384 x 2048    51.4 / 50.3    89.4 / 87.6    123 / 122      161 / 160      303 / 303
+//     2048 x 8192     50.1 / 31.5    91.0 / 51.5    195 / 77.7     196 / 83.5     199 / 148
+static int f32_form(int m, int n, int k, int count, int cus) {
+  int best = F32_TILES_64;
+  if (m > 32 * 65535) return best;
+  double least = f32_micros(best, m, n, k, count, cus);
+  for (int form = 0; form < F32_FORMS; ++form) {
+    if (form == F32_FEW || form == F32_TILES_64) continue;
+    const double t = f32_micros(form, m, n, k, count, cus);
+    if (t < least) least = t, best = form;
+  }
+  return best;
+}
+
+// `count` products side by side, `heads` apart; only: a form, or -1.
+static int gemm_f32(const float* a, int64_t lda, const float* w, int64_t ldw, float* c, int64_t ldc, int m, int n, int k, int count, const Heads& heads,
+                    int only, hipStream_t stream) {
+  MI_REQUIRE(m >= 0 && n > 0 && k > 0 && count >= 1 && count <= 65535, "gemm_f32: bad sizes m=%d n=%d k=%d, %d of them", m, n, k, count);
   MI_REQUIRE(lda >= k && ldw >= k && ldc >= n, "gemm_f32: a row stride is shorter than its row");
   MI_REQUIRE(ceil_div(m, 64) <= 65535, "gemm_f32: m=%d is too large for one call", m);
   if (m == 0) return MI_OK;
-  const bool a16 = lda % 4 == 0 && (uintptr_t)a % 16 == 0, w16 = ldw % 4 == 0 && (uintptr_t)w % 16 == 0;
-  const bool wide = n >= 8192;
-  if (m <= 32 || (m <= 64 && !wide)) {
-    const bool lines = whole_lines(a, lda, w, ldw, k, 32);
-    const int form = lines ? LINES : a16 && w16 && k % 4 == 0 ? PIECES : VALUES;
-    const bool half_empty = ceil_div(n, 16) <= 128;
-    if (lines && few_rows_take(m, k)) {
-      if (m > 4) half_empty ? launch_few<2, 8>(a, lda, w, ldw, c, ldc, m, n, k, stream) : launch_few<2, 16>(a, lda, w, ldw, c, ldc, m, n, k, stream);
-      else half_empty ? launch_few<1, 8>(a, lda, w, ldw, c, ldc, m, n, k, stream) : launch_few<1, 16>(a, lda, w, ldw, c, ldc, m, n, k, stream);
-    } else if (m > 32) launch_rows<4, 1>(a, lda, w, ldw, c, ldc, m, n, k, form, stream);
-    else if (m > 16) launch_rows<2, 1>(a, lda, w, ldw, c, ldc, m, n, k, form, stream);
-    else if (wide) launch_rows<1, 2>(a, lda, w, ldw, c, ldc, m, n, k, form, stream);
-    else launch_rows<1, 1>(a, lda, w, ldw, c, ldc, m, n, k, form, stream);
-    MI_CHECK_LAUNCH("gemm_f32 (few rows)");
-    return MI_OK;
-  }
+  const bool a16 = lda % 4 == 0 && (uintptr_t)a % 16 == 0 && (count == 1 || heads.a % 4 == 0), w16 = ldw % 4 == 0 && (uintptr_t)w % 16 == 0 && (count == 1 || heads.w % 4 == 0);
+  const bool lines = whole_lines(a, lda, w, ldw, k, 32) && (count == 1 || (heads.a % 4 == 0 && heads.w % 32 == 0));
+  const bool few = lines && few_rows_take(m, k);
+  const int form = only >= 0 ? only : few ? (int)F32_FEW : f32_form(m, n, k, count, max(8, mi_compute_units()));
   const bool aligned = a16 && w16 && k % 4 == 0;
-  const bool many_blocks = (int64_t)ceil_div(n, BN) * ceil_div(m, 64) >= 1024 || m > 32 * 65535;
-  if (many_blocks) launch_tiles<64, 1>(a, lda, w, ldw, c, ldc, m, n, k, aligned, stream);
-  else if (segment_slices(k) % 4 == 0) launch_tiles<32, 4>(a, lda, w, ldw, c, ldc, m, n, k, aligned, stream);
-  else launch_tiles<32, 1>(a, lda, w, ldw, c, ldc, m, n, k, aligned, stream);
+  const int how = lines ? LINES : aligned ? PIECES : VALUES;
+  MI_REQUIRE(form < F32_FORMS && (form != F32_FEW || few), "gemm_f32: form %d does not take m=%d k=%d", form, m, k);
+  if (form == F32_FEW) {
+    const bool half_empty = (int64_t)ceil_div(n, 16) * count <= 128;
+#define MI_FEW(FEATURES, KIND)                                                                                          \
+  do {                                                                                                                  \
+    if (m > 4) launch_few<2, FEATURES, KIND>(a, lda, w, ldw, c, ldc, m, n, k, stream, FewRows(), count, heads);         \
+    else launch_few<1, FEATURES, KIND>(a, lda, w, ldw, c, ldc, m, n, k, stream, FewRows(), count, heads);               \
+  } while (0)
+    if (count > 1 && half_empty) MI_FEW(8, FEW_HEADS);
+    else if (count > 1) MI_FEW(16, FEW_HEADS);
+    else if (half_empty) MI_FEW(8, FEW_PLAIN);
+    else MI_FEW(16, FEW_PLAIN);
+#undef MI_FEW
+  } else if (form == F32_TILES_64) {
+    launch_tiles<64, 1>(a, lda, w, ldw, c, ldc, m, n, k, aligned, count, heads, stream);
+  } else if (form == F32_TILES_32) {
+    if (segment_slices(k) % 4 == 0) launch_tiles<32, 4>(a, lda, w, ldw, c, ldc, m, n, k, aligned, count, heads, stream);
+    else launch_tiles<32, 1>(a, lda, w, ldw, c, ldc, m, n, k, aligned, count, heads, stream);
+  }
+#define X(I, RT, FT) \
+  else if (form == I) launch_rows<RT, FT>(a, lda, w, ldw, c, ldc, m, n, k, how, count, heads, stream);
+  F32_ROWS_FORMS(X)
+#undef X
   MI_CHECK_LAUNCH("gemm_f32");
   return MI_OK;
+}
+
+extern "C" int mi_gemm_f32(const float* a, int64_t lda, const float* w, int64_t ldw, float* c, int64_t ldc, int m, int n, int k, hipStream_t stream) {
+  return gemm_f32(a, lda, w, ldw, c, ldc, m, n, k, 1, {}, -1, stream);
+}
+
+// The same in one of its forms (those that do not take the sizes refuse them).
+extern "C" int mi_gemm_f32_as(int form, const float* a, int64_t lda, const float* w, int64_t ldw, float* c, int64_t ldc, int m, int n, int k,
+                              hipStream_t stream) {
+  MI_REQUIRE(form >= 0, "gemm_f32: form %d", form);
+  return gemm_f32(a, lda, w, ldw, c, ldc, m, n, k, 1, {}, form, stream);
+}
+
+// A product a head: a, w and c of head h lie h times a_head, w_head and c_head elements further on.
+extern "C" int mi_gemm_f32_heads(const float* a, int64_t lda, int64_t a_head, const float* w, int64_t ldw, int64_t w_head, float* c, int64_t ldc,
+                                 int64_t c_head, int m, int n, int k, int heads, hipStream_t stream) {
+  return gemm_f32(a, lda, w, ldw, c, ldc, m, n, k, heads, {a_head, w_head, c_head}, -1, stream);
 }

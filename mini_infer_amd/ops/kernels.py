@@ -2675,7 +2675,7 @@ def linear_per_head(x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor, we
     stride).  With `gate` [T, heads, N] the result (rounded to the element type) is multiplied by
     `logistic(gate)`.
 
-    float32: the true-float32 product, head by head.  bfloat16: up to `PER_HEAD_MAX_ROWS` rows that are
+    float32: the true-float32 products of all heads as one launch.  bfloat16: up to `PER_HEAD_MAX_ROWS` rows that are
     read 16 bytes at a time run as one kernel, gate included; otherwise one batched product of the
     vendor library, whose right operand is `weight_kn` (`weight` with its last two axes exchanged,
     [heads, K, N], contiguous; made here if it is not given)."""
@@ -2694,9 +2694,8 @@ def linear_per_head(x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor, we
         return
     lib = library.load()
     if x.dtype == torch.float32:
-        for h in range(heads):
-            library.check(lib.mi_gemm_f32(_ptr(x[:, h]), x.stride(0), _ptr(weight[h]), weight.stride(1), _ptr(out[:, h]),
-                                          out.stride(0), tokens, n, k, _stream()))
+        library.check(lib.mi_gemm_f32_heads(_ptr(x), x.stride(0), x.stride(1), _ptr(weight), weight.stride(1), weight.stride(0), _ptr(out),
+                                            out.stride(0), out.stride(1), tokens, n, k, heads, _stream()))
     elif (tokens <= PER_HEAD_MAX_ROWS and k % 8 == 0 and x.stride(0) % 8 == 0 and x.stride(1) % 8 == 0 and x.data_ptr() % 16 == 0
           and weight.is_contiguous() and weight.data_ptr() % 16 == 0):
         library.check(lib.mi_per_head_bf16(

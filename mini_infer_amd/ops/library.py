@@ -33,6 +33,8 @@ _SIGNATURES: dict[str, list] = {
     ],
     "mi_silu_mul": [c_int, _P, _P, c_int, c_int, _P],
     "mi_gemm_f32": [_P, c_int64, _P, c_int64, _P, c_int64, c_int, c_int, c_int, _P],
+    "mi_gemm_f32_as": [c_int, _P, c_int64, _P, c_int64, _P, c_int64, c_int, c_int, c_int, _P],
+    "mi_gemm_f32_heads": [_P, c_int64, c_int64, _P, c_int64, c_int64, _P, c_int64, c_int64, c_int, c_int, c_int, c_int, _P],
     "mi_gemm_f32_swiglu_takes": [_P, c_int64, _P, c_int64, c_int, c_int, c_int],
     "mi_gemm_f32_swiglu": [_P, c_int64, _P, c_int64, _P, c_int64, c_int, c_int, c_int, _P],
     "mi_gemm_f32_rope_takes": [_P, c_int64, _P, c_int64, c_int, c_int, c_int],

@@ -325,7 +325,7 @@ def test_products_in_tiles_that_take_turns(form):
         finite = slice(0, m - 1 if m > 2 else m)
         exact = (a.double() @ w.double().T)[finite]
         # (float32 sums of k products, then one rounding to 8 bits)
-        bound = 2.0 ** -23 * k * (a.double().abs() @ w.double().abs().T)[finite] + 2.0 ** -8 * exact.abs() + 1e-30
+        bound = 2.0 ** -23 * k * (a.double().abs() @ w.double().abs().T)[finite] + 2.0 ** -8 * exact.abs() + 1e-12
         out = made(kernels.TURNS_NONE, a, w, 2 * n)[finite]
         assert ((out.double() - exact).abs() <= bound).all(), (m, n, k)
         for spare in (3, -2 * n % 8 + 8):
@@ -1859,3 +1859,43 @@ def test_what_a_models_step_launches(dtype, steady, rows, rotates, monkeypatch):
         assert torch.equal(logits, apart)
     else:  # (one product a layer in another order of sums: a bfloat16 rounding, 2^-9, of q, k and v, carried through two layers)
         assert (logits - apart).norm() < 2.0 ** -6 * apart.norm()
+
+
+@pytest.mark.parametrize("m", [1, 7, 15, 17, 33, 63, 65, 130])
+@pytest.mark.parametrize("n, k", [(16, 32), (37, 96), (200, 288), (64, 2048), (520, 4128), (130, 31), (33, 260)])
+def test_every_form_of_the_float32_product_gives_the_same_bits(m, n, k):
+    """Tiles of every size, in whole lines, in pieces and value by value, with rows and features beside whole tiles: the same order of the same
+    64-bit sums; and against float64, which they round once (2^-24)."""
+    from mini_infer_amd import ops
+    from mini_infer_amd.ops import library
+    from mini_infer_amd.ops.kernels import _ptr, _stream
+
+    g = torch.Generator(device="cuda").manual_seed(m * n + k)
+    wide = torch.randn(n, (k + 31) // 32 * 32 + 32, generator=g, device="cuda")
+    lib = library.load()
+    a = torch.randn(m, k, generator=g, device="cuda")
+    for first in (0, 4, 1):  # rows of W on a line, on 16 bytes, on neither
+        w = wide[:, first : first + k]
+        want = a.double() @ w.double().t()
+        exact = want.float()
+        got = ops.gemm_f32(a, w)
+        assert ((got - exact).abs() <= 2.0 ** -23 * exact.abs() + 1e-12).all()
+        for form in (0, 1, 2, 3, 4, 5, 7, 8):
+            out = torch.full((m, n + 2), 7.0, device="cuda")
+            library.check(lib.mi_gemm_f32_as(form, _ptr(a), a.stride(0), _ptr(w), w.stride(0), _ptr(out), out.stride(0), m, n, k, _stream()))
+            assert torch.equal(out[:, :n], got) and (out[:, n:] == 7).all(), (first, form)
+
+
+@pytest.mark.parametrize("tokens", [1, 3, 5, 8, 9, 17, 40, 130])
+@pytest.mark.parametrize("heads, k, n", [(1, 64, 256), (32, 64, 256), (5, 256, 64), (3, 10, 22), (40, 36, 12)])
+def test_float32_products_of_all_heads_are_those_of_each(tokens, heads, k, n):
+    from mini_infer_amd import ops
+
+    g = torch.Generator(device="cuda").manual_seed(tokens + heads)
+    x = torch.randn(tokens, heads, k + 8, generator=g, device="cuda")[:, :, :k]
+    w = torch.randn(heads, n, k, generator=g, device="cuda")
+    out = torch.zeros(tokens, heads, n + 4, device="cuda")
+    ops.linear_per_head(x, w, out[:, :, :n])
+    for h in range(heads):
+        assert torch.equal(out[:, h, :n], ops.gemm_f32(x[:, h], w[h]))
+    assert (out[:, :, n:] == 0).all()
