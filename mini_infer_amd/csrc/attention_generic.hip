@@ -466,11 +466,13 @@ static int attn_generic_launch(const void* q, int64_t q_row_stride, const void* 
   const size_t lds = sizeof(S) * GT * head_dim;
   const bool vec = head_dim % 16 == 0 && v_dim % 16 == 0 && v_row_stride % 16 == 0;
   // Four waves a range in the 32-bit path where one wave a range is fewer than two waves a SIMD (decode; values of
-  // up to 128 dims, which the merging's LDS holds) and the ranges are long enough for the blocks, of which three run
+  // up to 256 dims, which the merging's LDS holds) and the ranges are long enough for the blocks, of which three run
   // on a CU at once instead of twelve.  Microseconds a layer with one wave and with four: 24 heads of 128 over 8: 30 tokens of
   // 100 positions (240 blocks) 40 / 36, 60 of 200 113 / 47, 100 of 100 (800 blocks) 63 / 74, 100 of 200 115 / 82, 200 of 100 (1,600)
   // 69 / 108, 200 of 400 313 / 299; 32 heads of 64 over 8: 30 of 200 44 / 20, 100 of 100 30 / 35, 200 of 200 60 / 60.  (One wave before
   // its loads were batched: a prompt of 509 tokens 247, then 148; such prompts now take attention_prompt_f32.hip, 66.)
+  //
+  // Values of up to 256 dims (latent rows of 288, 32 heads): 4 tokens of up to 300 positions 88 -> 33 us a layer, 128 of up to 153 (1,024 blocks) 95 -> 68.
   //
   // Up to three blocks a CU a wave has one or two 64s of keys and its time is the waits one after another, so that more loads in flight
   // (DEEP) are worth two blocks a CU at once instead of three; for values of up to 64 dims, of which less is in flight, as long as two
@@ -484,7 +486,7 @@ static int attn_generic_launch(const void* q, int64_t q_row_stride, const void* 
   if (window > 0) keys = keys < window ? keys : window;
   if (mask_chunk > 0) keys = keys < mask_chunk ? keys : mask_chunk;
   keys = ceil_div64(keys, num_splits);
-  const bool four = sizeof(S) == 8 && v_dim <= 128 && blocks < 2048 && keys > MI_WAVE * ceil_div64(blocks, 768);
+  const bool four = sizeof(S) == 8 && v_dim <= 256 && blocks < 2048 && keys > MI_WAVE * ceil_div64(blocks, 768);
 #define MI_ATTN_LAUNCH_WAVES(VPL, VEC, WAVES, DEEP, LDS)                                          \
   attn_generic_kernel<T, VPL, VEC, WAVES, DEEP><<<grid, WAVES * MI_WAVE, LDS, stream>>>(                \
       (const T*)q, q_row_stride, (const T*)k_pages, (const T*)v_pages, block_table, max_blocks,   \
@@ -493,10 +495,10 @@ static int attn_generic_launch(const void* q, int64_t q_row_stride, const void* 
       softcap, sinks, (const T*)gate, gate_row_stride)
 #define MI_ATTN_LAUNCH(VPL, VEC)                                                                  \
   do {                                                                                            \
-    if constexpr (sizeof(S) == 8 && VPL <= 2) {                                                   \
-      if (four) {                                                                                 \
-        const size_t merge = 3 * GT * (VPL + 1) * MI_WAVE * sizeof(S) + 4 * GT * sizeof(float);   \
-        if (VEC && blocks <= (VPL == 1 ? 512 : 768)) MI_ATTN_LAUNCH_WAVES(VPL, VEC, 4, VEC, lds + merge); \
+    if constexpr (sizeof(S) == 8 && VPL <= 4) {                                                   \
+      const size_t merge = 3 * GT * (VPL + 1) * MI_WAVE * sizeof(S) + 4 * GT * sizeof(float);     \
+      if (four && lds + merge <= 64 * 1024) {                                                     \
+        if (VEC && VPL <= 2 && blocks <= (VPL == 1 ? 512 : 768)) MI_ATTN_LAUNCH_WAVES(VPL, VEC, 4, (VEC && VPL <= 2), lds + merge); \
         else MI_ATTN_LAUNCH_WAVES(VPL, VEC, 4, false, lds + merge);                               \
         break;                                                                                    \
       }                                                                                           \

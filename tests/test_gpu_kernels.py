@@ -1899,3 +1899,29 @@ def test_float32_products_of_all_heads_are_those_of_each(tokens, heads, k, n):
     for h in range(heads):
         assert torch.equal(out[:, h, :n], ops.gemm_f32(x[:, h], w[h]))
     assert (out[:, :, n:] == 0).all()
+
+
+@pytest.mark.parametrize("head_dim, v_dim", [(288, 256), (200, 144), (256, 250), (130, 130), (96, 64)])
+@pytest.mark.parametrize("contexts", [[1, 64, 65], [300, 7, 129, 256, 257], [700]])
+@pytest.mark.parametrize("window", [None, 100])
+def test_float32_attention_over_wide_value_rows(head_dim, v_dim, contexts, window):
+    """Values of up to 256 dims inside rows of keys, one key head, as few tokens as decoding brings (four waves share a range) and ends of
+    64s: against float64, of which float32 results are one rounding (and one of each range's part) away."""
+    from mini_infer_amd import ops
+
+    g = torch.Generator(device="cuda").manual_seed(head_dim + sum(contexts))
+    page, heads, tokens = 16, 6, len(contexts)
+    width = -(-max(contexts) // page)
+    pages = torch.randn(tokens * width, 1, page, head_dim, generator=g, device="cuda")
+    table = torch.randperm(tokens * width, generator=g, device="cuda").int().view(tokens, width)
+    q = torch.randn(tokens, heads * head_dim, generator=g, device="cuda")
+    of = torch.arange(tokens, dtype=torch.int32, device="cuda")
+    positions = torch.tensor(contexts, dtype=torch.int32, device="cuda") - 1
+    cu = torch.arange(tokens + 1, dtype=torch.int32, device="cuda")
+    got = ops.paged_attention(q, pages, None, table, of, positions, cu, cu.tolist(), q_heads=heads, kv_heads=1, head_dim=head_dim, scale=0.11,
+                              window=window, max_seq_len=max(contexts), v_head_dim=v_dim)
+    for t, n in enumerate(contexts):
+        keys = pages[table[t].long()].view(-1, head_dim)[max(0, n - window) if window else 0 : n].double()
+        p = torch.softmax(q[t].double().view(heads, head_dim) @ keys.t() * 0.11, -1)
+        want = p @ keys[:, :v_dim]
+        assert (got[t].double().view(heads, v_dim) - want).abs().max() < 2.0 ** -21 * want.abs().max()
