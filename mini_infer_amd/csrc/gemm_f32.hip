@@ -17,19 +17,9 @@
 // What bounds it: the 64-bit matrix instruction (16x16x4) takes 64 cycles a SIMD, 76 TFLOP/s on
 // the whole part (the vector pipe's 64-bit multiply-add reached 51, and needs a widened operand
 // in registers for every one of them; the instruction shares it among 16 products).
-#include "common.h"
+#include "gemm_f32_lines.h"
 
-typedef double f64x4_t __attribute__((ext_vector_type(4)));
-
-#define SEGMENTS 8
-#define SLICE 32       // values of K a step: one 128-byte line of a row
 #define BN 64
-
-static __host__ __device__ inline int segment_slices(int k) { return (k + SEGMENTS * SLICE - 1) / (SEGMENTS * SLICE); }
-
-__device__ __forceinline__ f64x4_t mma(float a, float w, f64x4_t acc) {
-  return __builtin_amdgcn_mfma_f64_16x16x4f64((double)a, (double)w, acc, 0, 0, 0);
-}
 
 // four values of a row from `at` on, zeros past its end
 template <bool ALIGNED>
@@ -213,46 +203,7 @@ __global__ __launch_bounds__(SEGMENTS * MI_WAVE) void gemm_f32_rows_kernel(const
       lower[f] = (uint32_t)min(row, most) * (uint32_t)(ldw * 4) + line_chunk_of_lane(lane);
       upper[f] = (uint32_t)min(row + 8, most) * (uint32_t)(ldw * 4) + line_chunk_of_lane(lane);
     }
-    const float* w_block = w + (int64_t)col0 * ldw;
-    constexpr int AHEAD = 2;
-    bf16x8_t lo[AHEAD][FT], hi[AHEAD][FT];  // 16-byte pieces; what they hold is float32
-    float4 av[AHEAD][RT][2];
-    auto fetch = [&](int slot, int slice) {
-#pragma unroll
-      for (int f = 0; f < FT; ++f) load_line_pair(w_block, 2 * (int64_t)slice, lower[f], upper[f], lo[slot][f], hi[slot][f]);
-#pragma unroll
-      for (int i = 0; i < RT; ++i) {
-        av[slot][i][0] = *reinterpret_cast<const float4*>(a_row[i] + slice * SLICE + 4 * quad);
-        av[slot][i][1] = *reinterpret_cast<const float4*>(a_row[i] + slice * SLICE + 16 + 4 * quad);
-      }
-    };
-#pragma unroll
-    for (int s = 0; s < AHEAD; ++s)
-      if (first + s < last) fetch(s, first + s);
-    for (int at = first; at < last; at += AHEAD) {
-#pragma unroll
-      for (int s = 0; s < AHEAD; ++s) {
-        if (at + s < last) {
-          float wv[FT][2][4], xv[RT][2][4];
-#pragma unroll
-          for (int f = 0; f < FT; ++f) {
-            lines_to_operands(lo[s][f], hi[s][f]);
-            __builtin_memcpy(wv[f][0], &lo[s][f], 16);
-            __builtin_memcpy(wv[f][1], &hi[s][f], 16);
-          }
-          __builtin_memcpy(xv, av[s], sizeof(xv));
-          if (at + s + AHEAD < last) fetch(s, at + s + AHEAD);
-#pragma unroll
-          for (int half = 0; half < 2; ++half)
-#pragma unroll
-            for (int e = 0; e < 4; ++e)
-#pragma unroll
-              for (int i = 0; i < RT; ++i)
-#pragma unroll
-                for (int f = 0; f < FT; ++f) acc[i][f] = mma(xv[i][half][e], wv[f][half][e], acc[i][f]);
-        }
-      }
-    }
+    lines_product<RT, FT>(w + (int64_t)col0 * ldw, lower, upper, a_row, first, last, acc);
   } else {
     constexpr int AHEAD = 2;
     const float* w_row[FT];

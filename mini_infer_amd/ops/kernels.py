@@ -3485,6 +3485,14 @@ def expert_tiles_take(x: torch.Tensor, ff: int) -> bool:
     return x.dtype == torch.bfloat16 and bool(lib.mi_expert_tiles_take(x.shape[1])) and bool(lib.mi_expert_tiles_take(ff))
 
 
+def expert_lines_take_f32(gate_up: torch.Tensor, down: torch.Tensor) -> bool:
+    """Whether float32 experts are read in whole lines for the matrix instruction (both products), which is faster than the products sorted by expert
+    at every size."""
+    lib = library.load()
+    return gate_up.dtype == torch.float32 and all(
+        bool(lib.mi_expert_lines_f32_take(_ptr(w), w.shape[2], w.shape[1] * w.shape[2])) for w in (gate_up, down))
+
+
 def expert_tile_cuts(counts: list[int], weight_rows: int, k: int, cus: int = WHOLE_DEVICE_CUS) -> list[tuple[int, int, int, int]]:
     """For each expert with `counts` pairs: the full tiles of 256 of them, the tiles behind those, the pairs in each of these and the rows of
     their form, in a launch of the tiles staged through LDS with `weight_rows` (gate and up together) of `k` elements an expert."""

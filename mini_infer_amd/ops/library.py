@@ -185,6 +185,7 @@ _SIGNATURES: dict[str, list] = {
         c_int, c_int, c_int, _P, _P,
     ],
     "mi_expert_tiles_take": [c_int],
+    "mi_expert_lines_f32_take": [_P, c_int, c_int64],
     "mi_gemm_turns_plan": [c_int, c_int, c_int, c_int, c_int, _P, _P],
     "mi_gemm_turns_rows": [c_int],
     "mi_gemm_turns_features": [c_int],

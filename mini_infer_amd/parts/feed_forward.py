@@ -405,6 +405,8 @@ class RoutedExperts(FeedForward):
             return False  # (the sorted form reads the experts' row counts on the host)
         if ops.expert_tiles_take(x, self.intermediate_size):
             return False  # (tiles over the device's own list of rows are faster at every size)
+        if x.dtype == torch.float32 and ops.expert_lines_take_f32(self.gate_up, self.down) and ops.experts_by_expert_take(x, self.gate_up, self.activation):
+            return False  # (and so are the blocks of float32 experts over that list)
         element = 2 if self.dtype == torch.bfloat16 else 4
         expert_bytes = (3 if self.gated else 2) * self.intermediate_size * self.hidden_size * element
         return x.shape[0] * self.top * expert_bytes > self.experts * self.GROUPED_BYTES_PER_EXPERT

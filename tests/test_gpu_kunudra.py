@@ -446,6 +446,32 @@ def test_experts_read_in_whole_lines_give_the_bits_of_those_read_in_pieces(activ
         assert (got[r].double().cpu() - want).abs().max() < 2 ** -6 * max(1.0, want.abs().max()), (r, picks[r])
 
 
+@pytest.mark.parametrize("activation", ["silu_gated", "squared_relu"])
+@pytest.mark.parametrize("width, ff, counts", [
+    (32, 64, [0, 1, 15, 16, 17]), (288, 96, [33, 0, 32, 31]), (2048, 40, [64, 2]), (64, 4128, [16, 49, 1])])
+def test_float32_experts_on_the_matrix_cores(activation, width, ff, counts):
+    """Rows in whole lines (of 40 features the second product is not: the general form), runs of K that are short or missing, one and two tiles
+    of 16 pairs a pass: against float64.  Both products round once to float32, the activation once more."""
+    from mini_infer_amd import ops
+
+    rng = np.random.default_rng(width + ff)
+    experts, rows = len(counts), sum(counts)
+    features = 2 * ff if activation == "silu_gated" else ff
+    x, up, down = (dev(rng.standard_normal(shape) / np.sqrt(shape[-1]), torch.float32)
+                   for shape in ((rows, width), (experts, features, width), (experts, width, ff)))
+    x *= width ** 0.5
+    picks = rng.permutation(np.repeat(np.arange(experts, dtype=np.int32), counts))
+    chosen, w = ints(picks.tolist()).reshape(rows, 1), torch.ones((rows, 1), device=DEV)
+    assert ops.expert_lines_take_f32(up, down) == (ff % 32 == 0)
+    got = ops.experts_by_expert(x, up, down, chosen, w, activation=activation).double().cpu()
+    x64, u64, d64 = x.double().cpu(), up.double().cpu(), down.double().cpu()
+    for r in range(rows):
+        z = u64[picks[r]] @ x64[r]
+        act = torch.nn.functional.silu(z[:ff]) * z[ff:] if activation == "silu_gated" else torch.relu(z) ** 2
+        want = d64[picks[r]] @ act
+        assert (got[r] - want).norm() < 2 ** -22 * want.norm() + 1e-9, (r, picks[r])
+
+
 # ---------------------------------------------------------------------------------------------
 # each mixer and each feed-forward alone in a one-layer model
 # ---------------------------------------------------------------------------------------------
