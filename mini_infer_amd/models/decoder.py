@@ -54,7 +54,8 @@ class DecoderModel:
         self.head = HEADS.lookup(head["kind"])(head, dtype, device, shared)
         self.stream_vectors: dict[str, torch.Tensor] = {}  # float32 [rows, hidden], by checkpoint name
         layer_parts = [part for block in self.blocks for part in block.parts()]
-        if any(getattr(part, "routes", False) for part in layer_parts):
+        self.steady = any(getattr(part, "routes", False) for part in layer_parts)
+        if self.steady:
             for part in layer_parts:
                 part.steady = True
         # a product whose output only ever meets norms that can add up its pieces may leave them apart
