@@ -183,8 +183,8 @@ __global__ __launch_bounds__(256, MODE == DELTA || DT > 2 ? 1 : 2) void walk_ker
   }
   const int slot = p.slots[b];
   const int row0 = 16 * DT * wave;  // of S
-  float* mine = p.state + (int64_t)((slot < 0 || slot >= p.num_slots) ? p.num_slots : slot) * p.state_stride +
-                ((int64_t)head * p.vdim + (live ? col : 0)) * PAD + row0 + 4 * quad;
+  const bool kept = live && slot >= 0 && slot < p.num_slots;  // (without a slot: from the spare row, which stays as it is)
+  float* mine = p.state + (int64_t)(kept ? slot : p.num_slots) * p.state_stride + ((int64_t)head * p.vdim + (live ? col : 0)) * PAD + row0 + 4 * quad;
   f32x4_t S[DT];
 #pragma unroll
   for (int d = 0; d < DT; ++d) S[d] = live ? *reinterpret_cast<const f32x4_t*>(mine + 16 * d) : f32x4_t{0.f, 0.f, 0.f, 0.f};
@@ -331,7 +331,7 @@ __global__ __launch_bounds__(256, MODE == DELTA || DT > 2 ? 1 : 2) void walk_ker
   for (int d = 0; d < DT; ++d) zeros += 0.f * S[d];
   const bool again = __syncthreads_or(!((zeros[0] + zeros[1]) + (zeros[2] + zeros[3]) == 0.f));
   if (threadIdx.x == 0) *flag = again;
-  if (live && !again) {
+  if (kept && !again) {
 #pragma unroll
     for (int d = 0; d < DT; ++d) *reinterpret_cast<f32x4_t*>(mine + 16 * d) = S[d];
   }

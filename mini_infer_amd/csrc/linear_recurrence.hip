@@ -124,28 +124,36 @@ __device__ __forceinline__ void run_of_row(const T* row, int at, int dim, bool w
   }
 }
 
-// One token of a request, a decay per head: bound by reading and writing its state.  Every lane reads what its rows of S need itself, beside the state;
-// nothing goes through LDS.  The arithmetic is that of the walk below, term by term.  40 requests of 64 heads of 128 x 64: 37.3 -> 34.2 us.  (With a
-// decay per channel each column's lanes would make all of their decays again, 16 heads of 128 x 256 46 -> 72 us: those share them through LDS.)
-template <typename T, int R, int L>
+// One token of a request, a decay per head: bound by reading and writing its state.  Every lane reads what its rows of S need itself, beside the state
+// of G times 256 / L columns, which is all asked for at once: with G = 1 a block had 8 KB on the way, and the blocks went in rounds of 4 us each.
+// The arithmetic is that of the walk below, term by term.  64 heads of 128 x 64, states from memory, G = 1 / 4: 34 requests 37.8 / 33.7 us, of them in a
+// recorded step of 64 57.3 / 40.2, 64 requests 65.6 / 56.8 (4.7 TB/s).  (With a decay per channel, made once a wave and shared through LDS, 34
+// requests of 16 heads of 128 x 256 46 us; the walk takes 43.)
+template <typename T, int R, int L, int G>
 __device__ __forceinline__ void decay_token(const ScanArgs& p, int64_t t, int slot, int head, int col0) {
   using A = typename Wide<T>::type;
   constexpr bool WIDE = sizeof(T) == 4;
-  const int part = threadIdx.x % L, col = col0 + threadIdx.x / L;
-  const bool live = col < p.vdim;
-  const int at = part * R, grp = head / (p.heads / p.groups);
-  float* mine = p.state + (int64_t)((slot < 0 || slot >= p.num_slots) ? p.num_slots : slot) * p.state_stride +
-                ((int64_t)head * p.vdim + (live ? col : 0)) * (R * L) + at;
-  float S[R], q[R], k[R];
+  constexpr int DP = R * L, COLS = 256 / L;
+  const int part = threadIdx.x % L, at = part * R, grp = head / (p.heads / p.groups);
+  const bool kept = slot >= 0 && slot < p.num_slots;  // (else a row that fills a recorded step: from the spare row, which stays as it is)
+  float* state = p.state + (int64_t)(kept ? slot : p.num_slots) * p.state_stride + (int64_t)head * p.vdim * DP + at;
+  float S[G][R], q[R], k[R], x[G];
+  int col[G];
 #pragma unroll
-  for (int i = 0; i < R; i += 4) {
-    const float4 got = *reinterpret_cast<const float4*>(mine + i);
-    S[i] = got.x, S[i + 1] = got.y, S[i + 2] = got.z, S[i + 3] = got.w;
+  for (int g = 0; g < G; ++g) {
+    col[g] = col0 + g * COLS + threadIdx.x / L;
+#pragma unroll
+    for (int i = 0; i < R; i += 4) {  // (past the last column: that one again, not written)
+      const float4 got = *reinterpret_cast<const float4*>(state + (int64_t)min(col[g], p.vdim - 1) * DP + i);
+      S[g][i] = got.x, S[g][i + 1] = got.y, S[g][i + 2] = got.z, S[g][i + 3] = got.w;
+    }
   }
   run_of_row<T, R>((const T*)p.q + p.q_col + t * p.q_stride + (int64_t)grp * p.dim, at, p.dim, p.whole_runs, q);
   run_of_row<T, R>((const T*)p.k + p.k_col + t * p.k_stride + (int64_t)grp * p.dim, at, p.dim, p.whole_runs, k);
+  const T* v_row = (const T*)p.v + p.v_col + t * p.v_stride + (int64_t)head * p.vdim;
+#pragma unroll
+  for (int g = 0; g < G; ++g) x[g] = to_f32(v_row[min(col[g], p.vdim - 1)]);
   const float raw = to_f32(((const T*)p.gate)[p.gate_col + t * p.gate_stride + head]), head_bias = p.gate_bias[head];
-  const float x = live ? to_f32(((const T*)p.v)[p.v_col + t * p.v_stride + (int64_t)head * p.vdim + col]) : 0.f;
   const float skip = p.skip ? p.skip[head] : 0.f;
   float a, dt;
   if constexpr (WIDE) {
@@ -157,24 +165,30 @@ __device__ __forceinline__ void decay_token(const ScanArgs& p, int64_t t, int sl
     dt = mi_soft_plus_fast(raw + head_bias);
     a = __builtin_amdgcn_exp2f(-rate * dt);
   }
-  const float vv = x * dt;
-  A acc = 0;
 #pragma unroll
-  for (int i = 0; i < R; ++i) {
-    const float qi = q[i] * p.q_scale;
-    S[i] = fmaf(k[i], vv, a * S[i]);
-    if constexpr (WIDE) acc = fma((double)S[i], (double)qi, acc);
-    else acc = fmaf(S[i], qi, acc);
-  }
-  acc = lanes_sum<L>(acc);
-  if (!live) return;
-  if (part == 0) {
-    if constexpr (WIDE) acc = fma((double)skip, (double)x, acc);
-    else acc = fmaf(skip, x, acc);
-    p.out[t * ((int64_t)p.heads * p.vdim) + (int64_t)head * p.vdim + col] = (float)acc;
-  }
+  for (int i = 0; i < R; ++i) q[i] *= p.q_scale;
 #pragma unroll
-  for (int i = 0; i < R; i += 4) *reinterpret_cast<float4*>(mine + i) = make_float4(S[i], S[i + 1], S[i + 2], S[i + 3]);
+  for (int g = 0; g < G; ++g) {
+    const float vv = x[g] * dt;
+    A acc = 0;
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+      S[g][i] = fmaf(k[i], vv, a * S[g][i]);
+      if constexpr (WIDE) acc = fma((double)S[g][i], (double)q[i], acc);
+      else acc = fmaf(S[g][i], q[i], acc);
+    }
+    acc = lanes_sum<L>(acc);
+    if (col[g] >= p.vdim) continue;
+    if (part == 0) {
+      if constexpr (WIDE) acc = fma((double)skip, (double)x[g], acc);
+      else acc = fmaf(skip, x[g], acc);
+      p.out[t * ((int64_t)p.heads * p.vdim) + (int64_t)head * p.vdim + col[g]] = (float)acc;
+    }
+    if (!kept) continue;
+#pragma unroll
+    for (int i = 0; i < R; i += 4)
+      *reinterpret_cast<float4*>(state + (int64_t)col[g] * DP + i) = make_float4(S[g][i], S[g][i + 1], S[g][i + 2], S[g][i + 3]);
+  }
 }
 
 // Decoded tokens, short portions and the 32-bit engine; long portions of bfloat16 steps go in chunks (decay_chunks.hip).
@@ -210,8 +224,8 @@ __device__ __forceinline__ void decay_scan_columns(const ScanArgs& p, int b, int
   // (of columns taken again the flagged ones: the others' states have been advanced)
   if constexpr (AGAIN) live = live && p.again[((int64_t)b * p.heads + head) * ((p.vdim + 15) / 16) + min(col, p.vdim - 1) / 16] != 0;
   const int slot = p.slots[b];
-  float* mine = p.state + (int64_t)((slot < 0 || slot >= p.num_slots) ? p.num_slots : slot) * p.state_stride +
-                ((int64_t)head * p.vdim + (live ? col : 0)) * DP + part * R;
+  const bool kept = slot >= 0 && slot < p.num_slots;  // (see decay_token)
+  float* mine = p.state + (int64_t)(kept ? slot : p.num_slots) * p.state_stride + ((int64_t)head * p.vdim + (live ? col : 0)) * DP + part * R;
   float S[R];
 #pragma unroll
   for (int i = 0; i < R; i += 4) {
@@ -354,7 +368,7 @@ __device__ __forceinline__ void decay_scan_columns(const ScanArgs& p, int b, int
       }
     }
   }
-  if (live) {
+  if (live && kept) {
 #pragma unroll
     for (int i = 0; i < R; i += 4) *reinterpret_cast<float4*>(mine + i) = make_float4(S[i], S[i + 1], S[i + 2], S[i + 3]);
   }
@@ -365,20 +379,21 @@ __device__ __forceinline__ void decay_scan_columns(const ScanArgs& p, int b, int
 // side by side every eighth block was the long portion's where requests come in 8s: 31 single tokens beside 64 of 64 heads of 128 x 64 184 us, so 34;
 // 16 heads of 128 x 256 254 / 66.  Heads go round before columns: a head's column blocks then share an XCD's L2 (512 tokens of 64 heads 144 us, 164
 // the other way).
-template <typename T, int MODE, int R, int L>
+// G: column blocks that a single token's block takes together (the other G - 1 leave at once); where there are enough blocks for that, launch_scan.
+template <typename T, int MODE, int R, int L, int G>
 __global__ __launch_bounds__(256) void decay_scan_kernel(ScanArgs p, int requests) {
   constexpr int COLS = 256 / L;
   const int each = p.heads * ((p.vdim + COLS - 1) / COLS);
   const int b = requests - 1 - (int)(blockIdx.x / each), rest = (int)(blockIdx.x % each);
-  const int head = rest % p.heads, col0 = rest / p.heads * COLS;
+  const int head = rest % p.heads, col_block = rest / p.heads;
   if constexpr (MODE == DECAY_PER_HEAD) {
     const int first = p.cu[b];
     if (p.cu[b + 1] - first == 1) {
-      decay_token<T, R, L>(p, first, p.slots[b], head, col0);
+      if (col_block % G == 0) decay_token<T, R, L, G>(p, first, p.slots[b], head, col_block * COLS);
       return;
     }
   }
-  decay_scan_columns<T, MODE, R, L, false>(p, b, head, col0);
+  decay_scan_columns<T, MODE, R, L, false>(p, b, head, col_block * COLS);
 }
 
 // the same for columns that the chunks' walk has flagged
@@ -407,7 +422,7 @@ inline void scan_shape(int dim, int* rows, int* lanes) {
 }
 
 template <typename T, int MODE>
-int launch_scan(ScanArgs p, int requests, hipStream_t stream) {
+int launch_scan(ScanArgs p, int tokens, int requests, hipStream_t stream) {
   int rows, lanes;
   scan_shape(p.dim, &rows, &lanes);
   const int piece = min(16, rows * (int)sizeof(T));
@@ -417,7 +432,15 @@ int launch_scan(ScanArgs p, int requests, hipStream_t stream) {
   p.whole_runs = p.dim % rows == 0 && in_pieces(p.q, p.q_stride, p.q_col) && in_pieces(p.k, p.k_stride, p.k_col);
   const int64_t grid = (int64_t)requests * p.heads * ceil_div(p.vdim, 256 / lanes);
   MI_REQUIRE(grid < ((int64_t)1 << 31), "decay_scan: %lld blocks are too many", (long long)grid);
-#define MI_SCAN(RR, LL) decay_scan_kernel<T, MODE, RR, LL><<<(unsigned)grid, 256, 0, stream>>>(p, requests)
+  constexpr int TOGETHER = MODE == DECAY_PER_HEAD ? 4 : 1;
+  // (two rounds of what the CUs hold; 24 requests of 32 heads of 64 columns, 3,072 blocks, take the same either way.  Beside a long portion, whose
+  // chain the larger blocks hold up, one: 38 tokens beside 73, a step of 12 layers 2,910 / 2,928 us.)
+  const bool together = grid >= 4096 && tokens <= requests;
+#define MI_SCAN(RR, LL)                                                                                               \
+  do {                                                                                                                \
+    if (together) decay_scan_kernel<T, MODE, RR, LL, TOGETHER><<<(unsigned)grid, 256, 0, stream>>>(p, requests);      \
+    else decay_scan_kernel<T, MODE, RR, LL, 1><<<(unsigned)grid, 256, 0, stream>>>(p, requests);                      \
+  } while (0)
   if (rows == 4) MI_SCAN(4, 4);
   else if (rows == 8 && lanes == 4) MI_SCAN(8, 4);
   else if (rows == 8 && lanes == 8) MI_SCAN(8, 8);
@@ -574,10 +597,10 @@ extern "C" int mi_decay_scan(int dtype, int mode, const void* q, int64_t q_strid
   p.gate_bias = gate_bias, p.rate = rate, p.skip = skip, p.inv_tau = inv_tau, p.q_scale = q_scale;
   p.state = state, p.state_stride = state_stride, p.cu = cu, p.slots = slots, p.num_slots = num_slots, p.out = out, p.again = nullptr;
   p.heads = heads, p.groups = groups, p.dim = dim, p.vdim = vdim, p.whole_runs = false;
-  if (dtype == MI_F32) return mode == 0 ? launch_scan<float, DECAY_PER_CHANNEL>(p, num_requests, stream)
-                                        : launch_scan<float, DECAY_PER_HEAD>(p, num_requests, stream);
-  return mode == 0 ? launch_scan<bf16_t, DECAY_PER_CHANNEL>(p, num_requests, stream)
-                   : launch_scan<bf16_t, DECAY_PER_HEAD>(p, num_requests, stream);
+  if (dtype == MI_F32) return mode == 0 ? launch_scan<float, DECAY_PER_CHANNEL>(p, num_tokens, num_requests, stream)
+                                        : launch_scan<float, DECAY_PER_HEAD>(p, num_tokens, num_requests, stream);
+  return mode == 0 ? launch_scan<bf16_t, DECAY_PER_CHANNEL>(p, num_tokens, num_requests, stream)
+                   : launch_scan<bf16_t, DECAY_PER_HEAD>(p, num_tokens, num_requests, stream);
 }
 
 int mi_decay_scan_again(int mode, const void* q, int64_t q_stride, int q_col, const void* k, int64_t k_stride, int k_col, const void* v,

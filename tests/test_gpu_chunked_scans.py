@@ -338,7 +338,8 @@ def test_a_recorded_step_is_not_taken_for_single_tokens():
     assert torch.equal(made[0][0], made[1][0]) and torch.equal(made[0][1], made[1][1])
 
 
-@pytest.mark.parametrize("heads,groups,dim,vdim", [(4, 2, 64, 64), (6, 3, 96, 80), (2, 1, 256, 250), (3, 3, 20, 30), (2, 2, 128, 128), (2, 1, 12, 7)])
+@pytest.mark.parametrize("heads,groups,dim,vdim", [(4, 2, 64, 64), (6, 3, 96, 80), (2, 1, 256, 250), (3, 3, 20, 30), (2, 2, 128, 128), (2, 1, 12, 7), (300, 3, 40, 70),
+                                                   (520, 2, 128, 20)])  # (with so many heads a token's block takes four times the columns)
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("odd", [False, True])
 def test_decay_scan_of_single_tokens_gives_the_bits_of_portions(monkeypatch, heads, groups, dim, vdim, dtype, odd):
@@ -365,8 +366,9 @@ def test_decay_scan_of_single_tokens_gives_the_bits_of_portions(monkeypatch, hea
     whole, single = state.clone(), state.clone()
     out = step([rows[0], None, rows[1]], [3, 0, 1], whole)
     for t in range(3):
-        got = step([rows[0][t:t + 1], None, rows[0][:2], rows[1][t:t + 1]], [3, 0, -1, 1], single)
-        assert torch.equal(got[0], out[t]) and torch.equal(got[3], out[3 + t])
+        portion = rows[0][:2] if t == 1 else None  # (steps of single tokens, and one with a portion)
+        got = step([rows[0][t:t + 1], None, portion, rows[1][t:t + 1]], [3, 0, -1, 1], single)
+        assert torch.equal(got[0], out[t]) and torch.equal(got[-1], out[3 + t])
     assert torch.equal(single[:-1], whole[:-1])
 
 
@@ -392,3 +394,42 @@ def test_short_conv_of_rows_in_fours_gives_the_bits_of_the_general_form(lengths,
         assert torch.equal(ops.short_conv(x, channels, w, tail, _boundaries(lengths), slots, of, bias=bias),
                            ops.short_conv(off, channels, w, other, _boundaries(lengths), slots, of, bias=bias))
         assert torch.equal(tail, other)
+
+
+@pytest.mark.parametrize("kind", ["decay", "channels", "delta"])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("chunks", [False, True])
+@pytest.mark.parametrize("lengths", [[1, 1, 1, 1], [1, 40, 2, 33]])
+def test_requests_without_a_slot_start_from_the_spare_row_and_leave_it_as_it_is(monkeypatch, kind, dtype, chunks, lengths):
+    """Rows that only fill a recorded step: what they would give with a slot that holds what the spare row does, while no row of the state is
+    written for them."""
+    from mini_infer_amd import ops
+    from mini_infer_amd.ops import kernels
+
+    if chunks and dtype == torch.float32:
+        pytest.skip("chunks are of bfloat16 rows")
+    monkeypatch.setattr(kernels, "chunked_scan_pays", lambda *sizes: chunks)
+    heads, dim, vdim, tokens = 4, 128, 64, sum(lengths)
+    g = torch.Generator(device=DEV).manual_seed(3)
+    x = torch.randn(tokens, 4 * heads * (dim + vdim), generator=g, device=DEV).to(dtype)
+    bias, rate = torch.randn(heads * dim, generator=g, device=DEV), torch.rand(heads, generator=g, device=DEV)
+    shape = ops.delta_state_shape(heads, dim, vdim) if kind == "delta" else ops.decay_state_shape(heads, dim, vdim)
+    state = torch.randn(6, *shape, generator=g, device=DEV)
+    state[4] = state[5]
+    cu = _boundaries(lengths)
+
+    def step(slots, into):
+        slots = torch.tensor(slots, dtype=torch.int32, device=DEV)
+        if kind == "delta":
+            return ops.gated_delta(x, x, 0, heads, 2 * heads, rate, bias[:heads], torch.ones(vdim, device=DEV), into, cu, slots, heads=heads, kv_heads=heads,
+                                   dim=dim, vdim=vdim, eps=1e-6)
+        per_head = kind == "decay"
+        return ops.decay_scan(x, 0, x, heads * dim, x, 2 * heads * dim, x, 2 * heads * dim + heads * vdim, bias[: heads if per_head else heads * dim], into, cu,
+                              slots, heads=heads, groups=heads, dim=dim, vdim=vdim, per_head=per_head, rate=rate if per_head else None)
+
+    left, zeros = state.clone(), state.clone()
+    got, want = step([2, -1, 0, -1], left), None
+    rows = [torch.arange(int(cu[b]), int(cu[b + 1]), device=DEV) for b in range(4)]
+    want = step([2, 4, 0, 3], zeros)
+    assert torch.equal(got[rows[0]], want[rows[0]]) and torch.equal(got[rows[1]], want[rows[1]]) and torch.equal(got[rows[2]], want[rows[2]])
+    assert torch.equal(left[[0, 2]], zeros[[0, 2]]) and torch.equal(left[[1, 3, 4, 5]], state[[1, 3, 4, 5]])
