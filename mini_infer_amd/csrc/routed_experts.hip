@@ -148,13 +148,23 @@ __device__ __forceinline__ void rank_outputs(A* mine, const float* __restrict__ 
   }
 }
 
+// A token that only fills its step (its request has no slot): it goes to no expert, or it would have their weights read.
+struct StepOwners {
+  const int *token_request, *slots;  // null: all tokens are someone's
+};
+__device__ __forceinline__ void drop_idle(const StepOwners& owners, int t, int* __restrict__ chosen, float* __restrict__ weights, int outputs, int top, int lane) {
+  if (owners.slots == nullptr || owners.slots[owners.token_request[t]] >= 0) return;
+  if (lane == 0)  // (which has written them)
+    for (int k = 0; k < top; ++k) chosen[k] = outputs, weights[k] = 0.f;
+}
+
 // R tokens a block: their rows wait in LDS while every wave walks router rows (16 bytes a lane, each
 // router row read once for all R tokens), then wave r ranks token r's outputs.
 template <typename T, int R>
 __global__ __launch_bounds__(1024) void route_top_k_kernel(
     const T* __restrict__ x, int64_t x_stride, const float* __restrict__ router, const float* __restrict__ correction,
     const float* __restrict__ gate_row, int* __restrict__ chosen, float* __restrict__ weights,
-    float* __restrict__ shared_gate, int num_tokens, int width, int outputs, int top, float route_scale, int scores) {
+    float* __restrict__ shared_gate, int num_tokens, int width, int outputs, int top, float route_scale, int scores, StepOwners owners) {
   using A = typename SumOf<T>::type;
   extern __shared__ __align__(16) unsigned char lds_bytes[];
   A* z = reinterpret_cast<A*>(lds_bytes);                         // [R][outputs + 1]
@@ -226,6 +236,7 @@ __global__ __launch_bounds__(1024) void route_top_k_kernel(
     A* mine = z + r * (outputs + 1);
     if (gate_row != nullptr && lane == 0) shared_gate[t] = (float)((A)1 / ((A)1 + exp_of(-mine[outputs])));
     rank_outputs<A>(mine, correction, chosen + (int64_t)t * top, weights + (int64_t)t * top, outputs, top, route_scale, scores, lane);
+    drop_idle(owners, t, chosen + (int64_t)t * top, weights + (int64_t)t * top, outputs, top, lane);
   }
 }
 
@@ -456,7 +467,7 @@ __global__ __launch_bounds__(1024) void route_list_kernel(const float* __restric
                                                           int* __restrict__ chosen, float* __restrict__ weights,
                                                           float* __restrict__ shared_gate, int* __restrict__ listed,
                                                           int* __restrict__ first, int num_tokens, int outputs, int total,
-                                                          int experts, int top, float route_scale, int scores) {
+                                                          int experts, int top, float route_scale, int scores, StepOwners owners) {
   extern __shared__ __align__(16) unsigned char lds_bytes[];
   float* z = reinterpret_cast<float*>(lds_bytes);                        // [waves][outputs]
   __shared__ int count[MI_SORT_MAX_EXPERTS + 1];
@@ -468,6 +479,7 @@ __global__ __launch_bounds__(1024) void route_list_kernel(const float* __restric
     __builtin_amdgcn_wave_barrier();
     if (total > outputs && lane == 0) shared_gate[t] = 1.f / (1.f + expf(-logits[(int64_t)t * total + outputs]));
     rank_outputs<float>(mine, correction, chosen + t * top, weights + t * top, outputs, top, route_scale, scores, lane);
+    drop_idle(owners, t, chosen + t * top, weights + t * top, outputs, top, lane);
   }
   __syncthreads();  // (what this block's waves have written to `chosen` is there for all of them)
   const int pairs = num_tokens * top;
@@ -903,9 +915,12 @@ __global__ __launch_bounds__(256) void weighted_squared_relu_kernel(const T* __r
 
 }  // namespace
 
-extern "C" int mi_route_top_k(int dtype, const void* x, int64_t x_stride, const float* router, const float* correction,
-                              const float* gate_row, int* chosen, float* weights, float* shared_gate, int num_tokens,
-                              int width, int outputs, int top, float route_scale, int scores, hipStream_t stream) {
+// token_request, slots (both or neither): tokens of requests without a slot get the choice `outputs`, which is no expert, with weight 0.
+extern "C" int mi_route_top_k_of(int dtype, const void* x, int64_t x_stride, const float* router, const float* correction,
+                                 const float* gate_row, int* chosen, float* weights, float* shared_gate, const int* token_request, const int* slots,
+                                 int num_tokens, int width, int outputs, int top, float route_scale, int scores, hipStream_t stream) {
+  MI_REQUIRE((token_request == nullptr) == (slots == nullptr), "route_top_k: the tokens' requests come with their slots");
+  const StepOwners owners = {token_request, slots};
   MI_REQUIRE(num_tokens >= 0 && width > 0 && x_stride >= width, "route_top_k: bad sizes tokens=%d width=%d", num_tokens, width);
   MI_REQUIRE(outputs > 0 && outputs <= MI_ROUTER_MAX_OUTPUTS && top > 0 && top <= outputs,
              "route_top_k: %d router outputs (at most %d) of which %d are chosen", outputs, MI_ROUTER_MAX_OUTPUTS, top);
@@ -928,7 +943,7 @@ extern "C" int mi_route_top_k(int dtype, const void* x, int64_t x_stride, const 
 #define MI_ROUTE(T, R)                                                                                               \
   route_top_k_kernel<T, R><<<blocks, threads, lds_for(R), stream>>>((const T*)x, x_stride, router, correction, gate_row, \
                                                                     chosen, weights, shared_gate, num_tokens, width,    \
-                                                                    outputs, top, route_scale, scores)
+                                                                    outputs, top, route_scale, scores, owners)
   if (dtype == MI_F32) {
     if (per_block == 4) MI_ROUTE(float, 4);
     else if (per_block == 2) MI_ROUTE(float, 2);
@@ -941,6 +956,13 @@ extern "C" int mi_route_top_k(int dtype, const void* x, int64_t x_stride, const 
 #undef MI_ROUTE
   MI_CHECK_LAUNCH("route_top_k");
   return MI_OK;
+}
+
+extern "C" int mi_route_top_k(int dtype, const void* x, int64_t x_stride, const float* router, const float* correction,
+                              const float* gate_row, int* chosen, float* weights, float* shared_gate, int num_tokens,
+                              int width, int outputs, int top, float route_scale, int scores, hipStream_t stream) {
+  return mi_route_top_k_of(dtype, x, x_stride, router, correction, gate_row, chosen, weights, shared_gate, nullptr, nullptr, num_tokens, width, outputs,
+                           top, route_scale, scores, stream);
 }
 
 // act: [num_tokens * top, ff]; rows of pairs whose expert is an identity expert are not written.  mode: 1 silu
@@ -1042,11 +1064,11 @@ extern "C" int mi_route_few_takes(int num_tokens, int width, int outputs, int to
          outputs > 0 && outputs <= MI_ROUTER_MAX_OUTPUTS;
 }
 
-// mi_route_top_k and mi_expert_sort for few bfloat16 tokens in two launches; `logits`: scratch
+// mi_route_top_k_of and mi_expert_sort for few bfloat16 tokens in two launches; `logits`: scratch
 // [num_tokens, outputs + (gate row ? 1 : 0)] floats.
-extern "C" int mi_route_few(const void* x, int64_t x_stride, const float* router, const float* correction, const float* gate_row,
-                            float* logits, int* chosen, float* weights, float* shared_gate, int* listed, int* first,
-                            int num_tokens, int width, int outputs, int experts, int top, float route_scale, int scores,
+extern "C" int mi_route_few_of(const void* x, int64_t x_stride, const float* router, const float* correction, const float* gate_row,
+                            float* logits, int* chosen, float* weights, float* shared_gate, int* listed, int* first, const int* token_request,
+                            const int* slots, int num_tokens, int width, int outputs, int experts, int top, float route_scale, int scores,
                             hipStream_t stream) {
   MI_REQUIRE(mi_route_few_takes(num_tokens, width, outputs, top) && x_stride >= width && x_stride % 4 == 0 && (uintptr_t)x % 8 == 0 &&
                  is_aligned16(router) && is_aligned16(gate_row),
@@ -1054,15 +1076,25 @@ extern "C" int mi_route_few(const void* x, int64_t x_stride, const float* router
   MI_REQUIRE(top > 0 && top <= outputs && experts > 0 && experts <= outputs, "route_few: %d of %d outputs, %d experts", top, outputs, experts);
   MI_REQUIRE(scores >= SCORES_SOFTMAX && scores <= SCORES_CHOSEN_SOFTMAX, "route_few: unknown scores %d", scores);
   MI_REQUIRE(gate_row == nullptr || shared_gate != nullptr, "route_few: a gate row needs a place for the gates");
+  MI_REQUIRE((token_request == nullptr) == (slots == nullptr), "route_few: the tokens' requests come with their slots");
   const int total = outputs + (gate_row != nullptr ? 1 : 0);
   route_logits_kernel<<<dim3(total, ceil_div(num_tokens, 8)), 256, 0, stream>>>((const bf16_t*)x, x_stride, router, gate_row, logits,
                                                                                num_tokens, width, outputs, total);
   MI_CHECK_LAUNCH("route_logits");
   const int threads = min(1024, num_tokens * MI_WAVE);
   route_list_kernel<<<1, threads, (size_t)(threads / MI_WAVE) * outputs * 4, stream>>>(
-      logits, correction, chosen, weights, shared_gate, listed, first, num_tokens, outputs, total, experts, top, route_scale, scores);
+      logits, correction, chosen, weights, shared_gate, listed, first, num_tokens, outputs, total, experts, top, route_scale, scores,
+      StepOwners{token_request, slots});
   MI_CHECK_LAUNCH("route_list");
   return MI_OK;
+}
+
+extern "C" int mi_route_few(const void* x, int64_t x_stride, const float* router, const float* correction, const float* gate_row,
+                            float* logits, int* chosen, float* weights, float* shared_gate, int* listed, int* first,
+                            int num_tokens, int width, int outputs, int experts, int top, float route_scale, int scores,
+                            hipStream_t stream) {
+  return mi_route_few_of(x, x_stride, router, correction, gate_row, logits, chosen, weights, shared_gate, listed, first, nullptr, nullptr, num_tokens, width,
+                         outputs, experts, top, route_scale, scores, stream);
 }
 
 // Rows a block keeps in LDS at a time for rows of k_dim elements (0: such rows do not fit).

@@ -3306,7 +3306,7 @@ def _list_pairs(chosen: torch.Tensor, lists: ExpertLists, pairs: int, experts: i
 
 def route_top_k(
     x: torch.Tensor, router: torch.Tensor, correction: torch.Tensor | None, gate_row: torch.Tensor | None, *, top: int,
-    route_scale: float, scores: str = "softmax", experts: int | None = None,
+    route_scale: float, scores: str = "softmax", experts: int | None = None, owners: tuple[torch.Tensor, torch.Tensor] | None = None,
 ) -> "tuple[torch.Tensor, torch.Tensor, torch.Tensor | None] | tuple[torch.Tensor, torch.Tensor, torch.Tensor | None, ExpertLists]":
     """Per row of `x` [T, W]: scores `softmax(router @ x)` over all router outputs (`router` float32
     [outputs, W]), the `top` outputs with the largest `score + correction` (`correction` float32
@@ -3318,7 +3318,8 @@ def route_top_k(
 
     With `experts` (how many of the outputs are real experts) a fourth result is the list of (row, choice) pairs
     by expert that `experts_by_expert` works from: for few bfloat16 rows it is made in the same launch
-    that ranks the outputs."""
+    that ranks the outputs.  `owners`: every row's request and every request's slot (int32): rows of requests without a slot (below 0: they only
+    fill a recorded step) choose no expert: their choice is `outputs`, with weight 0."""
     if scores not in ROUTER_SCORES:
         raise KernelShapeError(f"route_top_k: scores {scores!r}; built: {ROUTER_SCORES}")
     _need_cuda(x, router, correction, gate_row)
@@ -3337,6 +3338,14 @@ def route_top_k(
         raise KernelShapeError(f"route_top_k: one correction per router output, got {correction.numel()} for {outputs}")
     if gate_row is not None and gate_row.numel() != width:
         raise KernelShapeError(f"route_top_k: the gate row has {gate_row.numel()} entries for {width} columns")
+    token_request, slots = (None, None) if owners is None else owners
+    if owners is not None:
+        _need_cuda(token_request, slots)
+        for name, t in (("token_request", token_request), ("slots", slots)):
+            _need_contiguous(name, t)
+            _need_int32(name, t)
+        if token_request.numel() != tokens:
+            raise KernelShapeError(f"route_top_k: one request a row, got {token_request.numel()} for {tokens}")
     chosen = torch.empty((tokens, top), dtype=torch.int32, device=x.device)
     weights = torch.empty((tokens, top), dtype=torch.float32, device=x.device)
     gates = torch.empty((tokens,), dtype=torch.float32, device=x.device) if gate_row is not None else None
@@ -3350,15 +3359,15 @@ def route_top_k(
         if (x.dtype == torch.bfloat16 and lib.mi_route_few_takes(tokens, width, outputs, int(top)) and x.stride(0) % 4 == 0
                 and x.data_ptr() % 8 == 0 and router.data_ptr() % 16 == 0 and (gate_row is None or gate_row.data_ptr() % 16 == 0)):
             logits = torch.empty((tokens, outputs + (gate_row is not None)), dtype=torch.float32, device=x.device)
-            library.check(lib.mi_route_few(
+            library.check(lib.mi_route_few_of(
                 _ptr(x), x.stride(0), _ptr(router), _ptr(correction), _ptr(gate_row), _ptr(logits), _ptr(chosen), _ptr(weights),
-                _ptr(gates), _ptr(lists.listed), _ptr(lists.first), tokens, width, outputs, experts, int(top), float(route_scale),
+                _ptr(gates), _ptr(lists.listed), _ptr(lists.first), _ptr(token_request), _ptr(slots), tokens, width, outputs, experts, int(top), float(route_scale),
                 ROUTER_SCORES.index(scores), _stream()))
             return chosen, weights, gates, lists
     library.check(
-        library.load().mi_route_top_k(
+        library.load().mi_route_top_k_of(
             _dtype_code(x), _ptr(x), x.stride(0), _ptr(router), _ptr(correction), _ptr(gate_row), _ptr(chosen), _ptr(weights),
-            _ptr(gates), tokens, width, outputs, int(top), float(route_scale), ROUTER_SCORES.index(scores), _stream(),
+            _ptr(gates), _ptr(token_request), _ptr(slots), tokens, width, outputs, int(top), float(route_scale), ROUTER_SCORES.index(scores), _stream(),
         )
     )
     if lists is not None:

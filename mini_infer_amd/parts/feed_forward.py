@@ -423,9 +423,14 @@ class RoutedExperts(FeedForward):
         grouped = self._grouped(x, ctx)
         by_expert = not grouped and (self.force_form == "by_expert" or (
             self.force_form is None and ops.experts_by_expert_take(x, self.gate_up, self.activation)))
+        # Rows that only fill a recorded step choose no expert, whose weights would be read for them (3 requests decoding in a step of 4, 12 layers of 16
+        # experts at 8B widths 2,305 -> 2,142 us); not where a norm adds all of a row's choices up.
+        owners = None
+        if by_expert and not self.leave_rows_apart and x.is_cuda and torch.cuda.is_current_stream_capturing():
+            owners = (ctx.token_request, ctx.state_slots)
         chosen, weights, gates, *lists = ops.route_top_k(
             x, self.router, self.correction, self.shared_gate_row, top=self.top, route_scale=self.route_scale, scores=self.scores,
-            experts=self.experts if by_expert else None)
+            experts=self.experts if by_expert else None, owners=owners)
         shared = None
         if self.shared is not None and not self.partner_joined:
             shared = self.shared.forward(x, ctx)

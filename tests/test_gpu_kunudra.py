@@ -472,6 +472,26 @@ def test_float32_experts_on_the_matrix_cores(activation, width, ff, counts):
         assert (got[r] - want).norm() < 2 ** -22 * want.norm() + 1e-9, (r, picks[r])
 
 
+@pytest.mark.parametrize("rows, width, outputs, experts, top, dtype", [
+    (1, 64, 18, 16, 2, "bfloat16"), (32, 256, 18, 16, 2, "bfloat16"), (33, 256, 5, 5, 3, "bfloat16"), (200, 64, 7, 4, 1, "bfloat16"), (8, 64, 18, 16, 2, "float32")])
+def test_rows_that_only_fill_a_step_choose_no_expert(rows, width, outputs, experts, top, dtype):
+    """Every third request without a slot, two rows a request: the other rows' choices, weights and places in the lists are as they were."""
+    from mini_infer_amd import ops
+
+    rng = np.random.default_rng(rows)
+    x, router = dev(rng.standard_normal((rows, width)), TORCH[dtype]), dev(rng.standard_normal((outputs, width)))
+    of = ints([r // 2 for r in range(rows)])
+    slots = ints([-1 if b % 3 == 1 else b for b in range(-(-rows // 2))])
+    idle = (slots[of.long()] < 0).cpu()
+    chosen, weights, _, lists = ops.route_top_k(x, router, None, None, top=top, route_scale=1.3, experts=experts)
+    got, got_weights, _, got_lists = ops.route_top_k(x, router, None, None, top=top, route_scale=1.3, experts=experts, owners=(of, slots))
+    assert torch.equal(got.cpu()[~idle], chosen.cpu()[~idle]) and torch.equal(got_weights.cpu()[~idle], weights.cpu()[~idle])
+    assert (got.cpu()[idle] == outputs).all() and (got_weights.cpu()[idle] == 0).all()
+    first, listed = got_lists.first.tolist(), got_lists.listed.tolist()
+    for e in range(experts):
+        assert sorted(listed[first[e]:first[e + 1]]) == [p for p in range(rows * top) if not idle[p // top] and int(chosen.view(-1)[p]) == e]
+
+
 # ---------------------------------------------------------------------------------------------
 # each mixer and each feed-forward alone in a one-layer model
 # ---------------------------------------------------------------------------------------------
