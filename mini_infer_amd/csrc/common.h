@@ -105,8 +105,9 @@ __device__ __forceinline__ bf16x8_t load_line(const void* matrix, int64_t first_
   return __builtin_nontemporal_load((global_chunk*)((global_bytes*)base_bits + at));
 }
 
-// The two loads of a pair of k-steps, non-temporal: base (uniform, kept in scalar registers) + the
-// lane's offsets.
+// The two loads of a pair of k-steps, non-temporal unless other blocks read the same rows (ONCE false): base (uniform, kept in
+// scalar registers) + the lane's offsets.
+template <bool ONCE = true>
 __device__ __forceinline__ void load_line_pair(const void* matrix, int64_t first_kstep, uint32_t lower_at,
                                                uint32_t upper_at, bf16x8_t& lower_rows, bf16x8_t& upper_rows) {
   using global_bytes = const __attribute__((address_space(1))) char;
@@ -117,8 +118,13 @@ __device__ __forceinline__ void load_line_pair(const void* matrix, int64_t first
   // (opaque to the compiler, or it widens the offsets to 64 bits once and for all and adds
   // whole addresses in vector registers for every load)
   asm("" : "+v"(lower_at), "+v"(upper_at));
-  lower_rows = __builtin_nontemporal_load((global_chunk*)(base + lower_at));
-  upper_rows = __builtin_nontemporal_load((global_chunk*)(base + upper_at));
+  if constexpr (ONCE) {
+    lower_rows = __builtin_nontemporal_load((global_chunk*)(base + lower_at));
+    upper_rows = __builtin_nontemporal_load((global_chunk*)(base + upper_at));
+  } else {
+    lower_rows = *(global_chunk*)(base + lower_at);
+    upper_rows = *(global_chunk*)(base + upper_at);
+  }
 }
 
 // (float32 elements: evaluated in 64-bit and rounded once; the float32 exponential and two more

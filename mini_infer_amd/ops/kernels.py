@@ -552,6 +552,22 @@ def _tiles(kind: int, x: torch.Tensor, weight: torch.Tensor, out: torch.Tensor, 
     return out
 
 
+def _whole_lines(x: torch.Tensor, weight: torch.Tensor) -> bool:
+    """Whether `gemm_rows_bf16` takes these (matrices that `_rows_of_bf16` has passed)."""
+    lib = library.load()
+    return bool(lib.mi_gemm_rows_take(_ptr(x), x.stride(0), _ptr(weight), weight.stride(0), x.shape[0], weight.shape[0], x.shape[1]))
+
+
+def _few_rows(form: int, x: torch.Tensor, weight: torch.Tensor) -> torch.Tensor:
+    """One launch of `gemm_rows_bf16`."""
+    out = torch.empty((x.shape[0], weight.shape[0]), dtype=torch.bfloat16, device=x.device)
+    library.check(
+        library.load().mi_gemm_rows_bf16(form, _ptr(x), x.stride(0), _ptr(weight), weight.stride(0), _ptr(out), out.stride(0), x.shape[0],
+                                         weight.shape[0], x.shape[1], _stream())
+    )
+    return out
+
+
 def linear_partial_sums(x: torch.Tensor, weight: torch.Tensor) -> PartialSums:
     """`x @ weight.T` for up to 128 bfloat16 rows as float32 sums over ranges of K; the ranges, and the order in which each is
     summed, depend on the matrix alone."""
@@ -615,6 +631,38 @@ def tiles_for(m: int, n: int, k: int, partial_ok: bool, cus: int = WHOLE_DEVICE_
     if m > 320 and micros > 0.88 * whole or m > 288 and ranges == 1 and max(n, k) > 4096:
         return None
     return shape, ranges
+
+
+SMALL_PRODUCT = 8_000_000  # elements of W
+SMALL_SUM_LAUNCH_MICROS = 2.0
+
+
+@functools.lru_cache(maxsize=8192)
+def small_product_plan(m: int, n: int, k: int, cus: int = WHOLE_DEVICE_CUS) -> tuple[int | None, int, int] | None:
+    """(form of `gemm_rows_bf16` or None, tile shape and ranges of K where its operands do not suit it) of a whole bfloat16 product of more rows than
+    `gemm_skinny_bf16` takes, where that is faster than what `tiles_for` says; None: as that says.
+
+    Matrices of fewer than 8,000,000 elements up to 320 rows, which `tiles_for` leaves to the vendor library: microseconds there / so (more of them at
+    the top of csrc/gemm_rows_bf16.hip), weights from memory, 3072 x 2048 at 128 / 192 / 256 / 320 rows 14.7 / 10.5, 21.5 / 12.6, 13.4 / 13.1, 13.5 / 13.2, 2048 x 2048
+    11.4 / 8.4, 12.0 / 10.1, 12.1 / 10.0, 12.9 / 12.5, 1024 x 1024 at 32 to 320 rows 8.1 / 3.7 to 6.2.  Not above 64 rows with K from 3,072 on, where a block walks
+    all of it: 1024 x 3072 at 96 / 256 rows 9.9 / 9.7 and 10.3 / 13.3, 2048 x 3072 10.9 / 11.4 and 16.0 / 13.7.  Up to 96 rows and 4,096 features larger ones too, cut
+    where the sum's launch, 2 microseconds in a recorded step, is counted as what it takes: 3072 x 3072 at 64 rows 14.3 / 11.6, 4096 x 4096 at 96 17.9 /
+    17.2.  Up to 32 rows those of more features in the forms of `gemm_rows_bf16`: 8192 x 3072 at 17 / 32 rows 17.1 / 13.0 and 17.9 / 15.1, 6144 x 3072 15.4 / 11.8 and 16.1 /
+    13.4, 8192 x 4096 18.7 / 15.5 and 20.1 / 17.5 (above, products with a rotation share their tiles with plain ones: `rotary_tiles_for`)."""
+    small = n * k < SMALL_PRODUCT
+    if not SKINNY_MAX_ROWS < m < TURNS_MIN_ROWS or small and m > 64 and k >= 3072:
+        return None
+    cut = small or n <= 4096 and m <= 96
+    if not cut and m > SKINNY_WIDE_MAX_ROWS:
+        return None
+    form, micros = ctypes.c_int(), ctypes.c_float()
+    library.check(library.load().mi_gemm_rows_plan(m, n, k, cus, ctypes.addressof(form), ctypes.addressof(micros)))
+    tiles, shape, ranges = _tiles_plan(m, n, k, False, 16, False, SMALL_SUM_LAUNCH_MICROS if cut else SUM_LAUNCH_MICROS, m * n * 4 / SUM_BYTES_A_MICRO, cus)
+    if ranges > 1 and not cut:
+        tiles -= SUM_LAUNCH_MICROS - SMALL_SUM_LAUNCH_MICROS  # (the ranges are those of `tiles_for`)
+    if micros.value < tiles:
+        return form.value, shape, ranges
+    return (None, shape, ranges) if cut else None
 
 
 def tile_size(shape: int) -> tuple[int, int]:
@@ -746,8 +794,9 @@ def linear(x: torch.Tensor, weight: torch.Tensor, partial_ok: bool = False, stea
 
     float32 runs the hand-written true-float32 kernel.  bfloat16 with at most 16 rows (decode) runs the hand-written
     weight-streaming kernel, some tens to some hundreds of rows the tiles of `gemm_tiles_bf16` where they are faster
-    (`tiles_for`), more rows mostly the tiles of `gemm_turns_bf16` (`plain_turns_pay`); the rest goes to the vendor GEMM library through torch, as the
-    reference's engine does (distributed/linear.py:167, `F.linear` -> the vendor BLAS).
+    (`tiles_for`), some tens with a small matrix `gemm_rows_bf16` (`small_product_plan`), more rows mostly the tiles of `gemm_turns_bf16`
+    (`plain_turns_pay`); the rest goes to the vendor GEMM library through torch, as the reference's engine does
+    (distributed/linear.py:167, `F.linear` -> the vendor BLAS).
     With `partial_ok` the result may come as `PartialSums` where that pays.  `steady` (`Part.steady`): above 16 rows the bits that the library gives,
     so without the tiles of `gemm_tiles_bf16`, and in those of `gemm_turns_bf16` where they are the same (`turns_keep_the_order`).
     """
@@ -768,7 +817,10 @@ def linear(x: torch.Tensor, weight: torch.Tensor, partial_ok: bool = False, stea
         return _turns(TURNS_NONE, x, weight, weight.shape[0])
     if not steady and x.dim() == 2 and x.shape[0] <= TILES_MAX_ROWS and _rows_of_bf16(x, weight):
         m, n = x.shape[0], weight.shape[0]
-        plan = tiles_for(m, n, x.shape[1], partial_ok, _compute_units(x.device))
+        small = None if partial_ok else small_product_plan(m, n, x.shape[1], _compute_units(x.device))
+        if small is not None and small[0] is not None and _whole_lines(x, weight):
+            return _few_rows(small[0], x, weight)
+        plan = small[1:] if small is not None else tiles_for(m, n, x.shape[1], partial_ok, _compute_units(x.device))
         if plan is not None:
             if plan[1] == 1:
                 return _tiles(0, x, weight, torch.empty((m, n), dtype=torch.bfloat16, device=x.device), n, *plan)

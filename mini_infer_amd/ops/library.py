@@ -43,6 +43,11 @@ _SIGNATURES: dict[str, list] = {
     ],
     "mi_gemm_skinny_bf16": [_P, c_int64, _P, c_int64, _P, c_int64, c_int, c_int, c_int, _P],
     "mi_gemm_skinny_f32out_bf16": [_P, c_int64, _P, c_int64, _P, c_int64, c_int, c_int, c_int, c_float, _P],
+    "mi_gemm_rows_plan": [c_int, c_int, c_int, c_int, _P, _P],
+    "mi_gemm_rows_take": [_P, c_int64, _P, c_int64, c_int, c_int, c_int],
+    "mi_gemm_rows_rows": [c_int],
+    "mi_gemm_rows_features": [c_int],
+    "mi_gemm_rows_bf16": [c_int, _P, c_int64, _P, c_int64, _P, c_int64, c_int, c_int, c_int, _P],
     "mi_gemm_tiles_plan": [c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_float, c_int, _P, _P, _P],
     "mi_gemm_tiles_rows": [c_int],
     "mi_gemm_tiles_features": [c_int],

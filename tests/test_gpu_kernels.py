@@ -400,6 +400,44 @@ def test_steady_products_of_many_rows_are_the_librarys_bit_for_bit(n, k):
             assert torch.equal(ops.linear_swiglu(a, w, steady=True), ops.silu_mul(want)), m
 
 
+@pytest.mark.parametrize("m, n, k", [(17, 40, 64), (31, 2048, 2048), (32, 1000, 576), (33, 515, 1088), (64, 3072, 2048), (100, 258, 4160), (256, 1024, 192)])
+def test_products_of_some_tens_of_rows_whose_waves_share_k(m, n, k):
+    """Every form, waves without a share of K and uneven ones, strided operands, tails of rows and features; nothing is written beside the output.
+    `linear` takes the planned one, and other kernels where W does not lie in whole cache lines."""
+    from mini_infer_amd import ops
+    from mini_infer_amd.exceptions import KernelShapeError
+    from mini_infer_amd.ops import kernels, library
+
+    lib = library.load()
+    a, w = _rand(m, k + 24, dtype=torch.bfloat16, seed=61)[:, :k], _rand(n, k + 64, dtype=torch.bfloat16, seed=62, scale=0.05)[:, :k]
+    exact = a.double() @ w.double().T
+    # half a bfloat16 unit, and k float32 roundings of the sums of magnitudes (eight of those more where the waves meet)
+    bound = exact.abs() * 2.0 ** -8 + (k + 8) * 2.0 ** -24 * (a.double().abs() @ w.double().abs().T)
+
+    def made(form, spare):
+        out = torch.full((m, n + spare), 7.0, dtype=torch.bfloat16, device="cuda")
+        library.check(lib.mi_gemm_rows_bf16(form, a.data_ptr(), a.stride(0), w.data_ptr(), w.stride(0), out.data_ptr(), out.stride(0), m, n, k,
+                                            torch.cuda.current_stream().cuda_stream))
+        assert (out[:, n:] == 7.0).all()
+        return out[:, :n]
+
+    form, first = 0, made(0, 0)
+    while lib.mi_gemm_rows_rows(form):
+        for spare in (0, 3, -n % 8 + 8):
+            got = made(form, spare)
+            assert torch.equal(got, first) and ((got.double() - exact).abs() <= bound).all(), (form, spare)
+        form += 1
+    assert form == 3
+    with pytest.raises(KernelShapeError):
+        made(form, 0)
+    plan = kernels.small_product_plan(m, n, k)
+    got = ops.linear(a, w)
+    assert ((got.double() - exact).abs() <= bound).all()
+    assert plan is None or plan[0] is None or torch.equal(got, first)
+    off = _rand(n * (k + 8) + 8, dtype=torch.bfloat16, seed=63)[8:].view(n, k + 8)[:, :k].copy_(w)  # rows on 16 bytes
+    assert not kernels._whole_lines(a, off) and ((ops.linear(a, off).double() - exact).abs() <= bound).all()
+
+
 @pytest.mark.parametrize("m,n,k", [(17, 3072, 3072), (33, 2048, 8192), (271, 3072, 8192), (100, 8192, 2048), (24, 1000, 8224), (400, 2048, 8192)])
 def test_linear_of_some_tens_to_some_hundreds_of_rows(m, n, k):
     """`linear` through tiles, with and without a consumer for the pieces; operands that the tiles do not take (rows off 16 bytes) go on

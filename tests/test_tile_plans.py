@@ -155,3 +155,14 @@ def test_tiles_of_rotary_products(m, n, k, made):
         assert plan == (shape, 1)
     elif made == "own":
         assert plan is None and kernels.tile_size(shape)[0] > 0
+
+
+@pytest.mark.parametrize("m, n, k, plan", [
+    (16, 2048, 2048, None), (17, 2048, 2048, "rows"), (32, 1024, 1024, "rows"), (128, 2048, 2048, "rows"), (64, 3072, 2048, "rows"),
+    (192, 3072, 2048, "whole"), (320, 1024, 1024, "whole"), (321, 1024, 1024, None),                                   # small matrices
+    (64, 2048, 3072, "cut"), (96, 2048, 3072, None), (64, 3072, 3072, "cut"), (97, 4096, 4096, None),                  # a longer K
+    (17, 8192, 4096, "rows"), (32, 8192, 3072, "rows"), (33, 8192, 3072, None), (32, 28672, 4096, None)])             # more features
+def test_products_with_small_matrices(m, n, k, plan):
+    got = kernels.small_product_plan(m, n, k)
+    made = None if got is None else "rows" if got[0] is not None else "whole" if got[2] == 1 else "cut"
+    assert made == plan
