@@ -171,7 +171,7 @@ __global__ __launch_bounds__(256, MODE == DELTA || DT > 2 ? 1 : 2) void walk_ker
   __shared__ f32x4_t parts[2][4][SUMS][MI_WAVE];
   __shared__ __align__(16) Shared<MODE> shared[2];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / MI_WAVE), lane = threadIdx.x % MI_WAVE;
-  const int head = blockIdx.x % p.heads, b = blockIdx.y;
+  const int head = blockIdx.x % p.heads, b = gridDim.y - 1 - blockIdx.y;
   const uint32_t r = lane % 16, quad = lane / 16;
   const int col = blockIdx.x / p.heads * 16 + r;
   const bool live = col < p.vdim;
