@@ -68,6 +68,23 @@ __device__ __forceinline__ int first_chunk(int cu_b, int b) { return cu_b / CHUN
 static inline int64_t chunk_count(int tokens, int requests) { return (int64_t)tokens / CHUNK + requests; }
 static inline int64_t flag_count(int requests, int heads, int vdim) { return (int64_t)requests * heads * ceil_div(vdim, 16); }
 
+// Of a request's only token the first launch leaves what walk_one_token reads and nothing else: row 0 of q and k (without DELTA: k as row 1 of q), the
+// first value of W, of T w and of both factors, and the fade.  One thread a channel makes it.
+//
+// The sums over a block of 256 threads, the same in all of them; `scratch`: 4 * N floats.
+template <int N>
+__device__ __forceinline__ void sum_of_block(float (&v)[N], float* scratch) {
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+#pragma unroll
+    for (int off = 1; off < MI_WAVE; off <<= 1) v[i] += __shfl_xor(v[i], off, MI_WAVE);
+    if (threadIdx.x % MI_WAVE == 0) scratch[threadIdx.x / MI_WAVE * N + i] = v[i];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < N; ++i) v[i] = (scratch[i] + scratch[N + i]) + (scratch[2 * N + i] + scratch[3 * N + i]);
+}
+
 // Which request a chunk number belongs to: all threads of the block call this; -1: no request's.
 __device__ __forceinline__ int request_of_chunk(int chunk, const int* __restrict__ cu, int requests, int* shared_answer) {
   if (threadIdx.x == 0) *shared_answer = -1;
@@ -160,6 +177,99 @@ struct Shared {
   float factor[2 * CHUNK];
 };
 
+// A request's only token, for G column blocks of 16 at once: bound by the state's bytes, and as a chunk of one token a block had 8 KB of them on the way
+// while it brought in 40 KB of operands.  Every wave keeps its rows of S as in the walk.  Steps with single tokens beside a long portion, all of them in chunks
+// / so: 34 and 500 of the delta rule with 32 heads of 128 x 128 (12 layers, half of them of the rule) 5,625 / 5,036 us, 25 and 400 with 24 heads 3,278 / 2,902, 34 and 700
+// with 64 heads of 128 x 64 8,551 / 7,847 (the long portion's blocks first in both: before that 8,847).
+template <int DT, int MODE, int G>
+__device__ __forceinline__ void walk_one_token(const WalkArgs& p, float* sums, int b, int first, int head, int block0) {
+  constexpr int PAD = 64 * DT;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / MI_WAVE), lane = threadIdx.x % MI_WAVE;
+  const int r = lane % 16, quad = lane / 16, row0 = 16 * DT * wave + 4 * quad;
+  const int slot = p.slots[b], blocks = (p.vdim + 15) / 16;
+  const bool kept = slot >= 0 && slot < p.num_slots;
+  float* state = p.state + (int64_t)(kept ? slot : p.num_slots) * p.state_stride + (int64_t)head * p.vdim * PAD + row0;
+  const int64_t chunk = first_chunk(first, b), rows = chunk * p.made.shares + head / (p.heads / p.made.shares), of = chunk * p.heads + head;
+  f32x4_t S[G][DT];
+  float v[G];
+  const bf16_t* v_row = p.v + (int64_t)first * p.v_stride + p.v_col + (int64_t)head * p.vdim;
+#pragma unroll
+  for (int g = 0; g < G; ++g) {
+    const int col = min((block0 + g) * 16 + r, p.vdim - 1);  // (past the last column: that one again, not written)
+#pragma unroll
+    for (int d = 0; d < DT; ++d) S[g][d] = *reinterpret_cast<const f32x4_t*>(state + (int64_t)col * PAD + 16 * d);
+    v[g] = to_f32(v_row[col]);
+  }
+  float4 q[DT], k[DT], fade[DT];
+#pragma unroll
+  for (int d = 0; d < DT; ++d) {
+    q[d] = load4(p.made.q + rows * CHUNK * PAD + row0 + 16 * d);
+    k[d] = load4((MODE == DELTA ? p.made.k : p.made.q + PAD) + rows * CHUNK * PAD + row0 + 16 * d);
+    if constexpr (MODE == PER_CHANNEL) fade[d] = load4(p.made.fade + of * PAD + row0 + 16 * d);
+  }
+  const float* factor = p.made.factor + of * 2 * CHUNK;
+  const float decay = MODE == PER_CHANNEL ? 1.f : factor[0], tail = MODE == PER_CHANNEL ? 1.f : factor[CHUNK];
+  const float within = p.made.within[of * CHUNK * CHUNK], solve = MODE == DELTA ? p.made.solve[of * CHUNK * CHUNK] : 1.f;
+  const float skip = (MODE == PER_HEAD && p.skip) ? p.skip[head] : 0.f;
+#pragma unroll
+  for (int g = 0; g < G; ++g) {
+    float qs = 0.f, ks = 0.f;
+#pragma unroll
+    for (int d = 0; d < DT; ++d) {
+      qs = fmaf(q[d].x, S[g][d][0], fmaf(q[d].y, S[g][d][1], fmaf(q[d].z, S[g][d][2], fmaf(q[d].w, S[g][d][3], qs))));
+      if constexpr (MODE == DELTA) ks = fmaf(k[d].x, S[g][d][0], fmaf(k[d].y, S[g][d][1], fmaf(k[d].z, S[g][d][2], fmaf(k[d].w, S[g][d][3], ks))));
+    }
+#pragma unroll
+    for (int off = 16; off < MI_WAVE; off <<= 1) {
+      qs += __shfl_xor(qs, off, MI_WAVE);
+      if constexpr (MODE == DELTA) ks += __shfl_xor(ks, off, MI_WAVE);
+    }
+    if (quad == 0) {
+      sums[(wave * G + g) * 32 + r] = qs;
+      if constexpr (MODE == DELTA) sums[(wave * G + g) * 32 + 16 + r] = ks;
+    }
+  }
+  __syncthreads();
+  int odd = 0;  // column blocks that do not end finite, a bit each
+#pragma unroll
+  for (int g = 0; g < G; ++g) {
+    auto whole = [&](int at) { return (sums[g * 32 + at] + sums[(G + g) * 32 + at]) + (sums[(2 * G + g) * 32 + at] + sums[(3 * G + g) * 32 + at]); };
+    float u = v[g];
+    if constexpr (MODE == DELTA) u = solve * (u - decay * whole(16 + r));
+    const float add = MODE == PER_CHANNEL ? u : tail * u;
+    float zeros = 0.f;
+#pragma unroll
+    for (int d = 0; d < DT; ++d) {
+      if constexpr (MODE == PER_CHANNEL) S[g][d] = scaled(fade[d], S[g][d]);
+      else S[g][d] *= decay;
+      S[g][d] = f32x4_t{fmaf(k[d].x, add, S[g][d][0]), fmaf(k[d].y, add, S[g][d][1]), fmaf(k[d].z, add, S[g][d][2]), fmaf(k[d].w, add, S[g][d][3])};
+#pragma unroll
+      for (int e = 0; e < 4; ++e) zeros = fmaf(0.f, S[g][d][e], zeros);
+    }
+    odd |= (__ballot(!(zeros == 0.f)) != 0) << g;
+    const int col = (block0 + g) * 16 + r;
+    if (wave * 4 + quad == g && col < p.vdim) {
+      float read = fmaf(within, u, decay * whole(r));
+      if constexpr (MODE == PER_HEAD) read = fmaf(skip, v[g], read);
+      p.out[(int64_t)first * p.heads * p.vdim + (int64_t)head * p.vdim + col] = read;
+    }
+  }
+  __syncthreads();  // (the sums have been read)
+  int* odd_of = reinterpret_cast<int*>(sums);
+  if (lane == 0) odd_of[wave] = odd;
+  __syncthreads();
+  odd = (odd_of[0] | odd_of[1]) | (odd_of[2] | odd_of[3]);
+  if (threadIdx.x < G && block0 + (int)threadIdx.x < blocks) p.again[((int64_t)b * p.heads + head) * blocks + block0 + threadIdx.x] = odd >> threadIdx.x & 1;
+  if (!kept) return;
+#pragma unroll
+  for (int g = 0; g < G; ++g) {
+    const int col = (block0 + g) * 16 + r;
+    if (col >= p.vdim || (odd >> g & 1)) continue;
+#pragma unroll
+    for (int d = 0; d < DT; ++d) *reinterpret_cast<f32x4_t*>(state + (int64_t)col * PAD + 16 * d) = S[g][d];
+  }
+}
+
 // grid: heads * column blocks (the heads side by side, so that an XCD's blocks share their chunk data), requests; 256 threads.
 // DT: 16-row tiles of S a wave keeps; pad = 64 * DT.  One wave a SIMD walks, so what a chunk costs is what a wave issues:
 // addresses are a base that is the same for the wave plus a lane's offset made once, without branches (at the end of
@@ -179,6 +289,12 @@ __global__ __launch_bounds__(256, MODE == DELTA || DT > 2 ? 1 : 2) void walk_ker
   int* flag = p.again + ((int64_t)b * p.heads + head) * ((p.vdim + 15) / 16) + blockIdx.x / p.heads;
   if (last <= first) {
     if (threadIdx.x == 0) *flag = 0;
+    return;
+  }
+  if (last - first == 1) {  // (the other blocks of those that go together have nothing to do)
+    constexpr int TOGETHER = MODE == DELTA ? 8 : 4;
+    static_assert(sizeof(parts) >= sizeof(float) * 4 * TOGETHER * 32, "the sums fit");
+    if (blockIdx.x / p.heads % TOGETHER == 0) walk_one_token<DT, MODE, TOGETHER>(p, reinterpret_cast<float*>(parts), b, first, head, blockIdx.x / p.heads);
     return;
   }
   const int slot = p.slots[b];

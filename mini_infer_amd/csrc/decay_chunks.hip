@@ -32,6 +32,24 @@ __global__ __launch_bounds__(256) void head_decay_chunk_kernel(RowArgs p, Made m
   if (b < 0) return;
   const int t0 = p.cu[b] + (chunk - first_chunk(p.cu[b], b)) * CHUNK, nt = min(CHUNK, p.cu[b + 1] - t0);
   const int tid = threadIdx.x, wave = tid / MI_WAVE, lane = tid % MI_WAVE;
+  if (p.cu[b + 1] - p.cu[b] == 1) {
+    if (blockIdx.z > 0) return;
+    const int64_t row = t0, at = tid < p.dim ? (int64_t)share * p.dim + tid : -1;
+    const float q = at >= 0 ? to_f32(p.q[row * p.q_stride + p.q_col + at]) : 0.f, k = at >= 0 ? to_f32(p.k[row * p.k_stride + p.k_col + at]) : 0.f;
+    float sums[2] = {q * p.q_scale * k, fmaf(0.f, k, 0.f * q)};
+    sum_of_block(sums, qk_s);
+    float* rows = made.q + ((int64_t)chunk * made.shares + share) * CHUNK * PAD;
+    if (tid < PAD) rows[tid] = q * p.q_scale, rows[PAD + tid] = k;
+    for (int h = share * (p.heads / p.groups) + tid; h < (share + 1) * (p.heads / p.groups); h += 256) {
+      const int64_t of = (int64_t)chunk * p.heads + h;
+      const float dt = mi_soft_plus_fast(to_f32(p.gate[row * p.gate_stride + p.gate_col + h]) + p.gate_bias[h]);
+      const float sum = -(expf(p.rate[h]) * 1.4426950408889634f * dt), whole = __builtin_amdgcn_exp2f(0.f * sum);  // (1, or NaN)
+      made.factor[of * 2 * CHUNK] = __builtin_amdgcn_exp2f(sum);
+      made.factor[of * 2 * CHUNK + CHUNK] = whole * dt + sums[1];
+      made.within[of * CHUNK * CHUNK] = whole * sums[0] * dt;
+    }
+    return;
+  }
   {
     const int token = tid / 8, sub = tid % 8;
     const int64_t row = t0 + min(token, nt - 1);
@@ -120,6 +138,23 @@ __global__ __launch_bounds__(256) void channel_decay_chunk_kernel(RowArgs p, Mad
   const int t0 = p.cu[b] + (chunk - first_chunk(p.cu[b], b)) * CHUNK, nt = min(CHUNK, p.cu[b + 1] - t0);
   const int tid = threadIdx.x, share = head / (p.heads / p.groups);
   int odd = 0;
+  if (p.cu[b + 1] - p.cu[b] == 1) {
+    const bool in = tid < p.dim;
+    const int64_t row = t0, at = (int64_t)share * p.dim + tid;
+    const float q = in ? to_f32(p.q[row * p.q_stride + p.q_col + at]) : 0.f, k = in ? to_f32(p.k[row * p.k_stride + p.k_col + at]) : 0.f;
+    const float a = in ? mi_channel_decay(to_f32(p.gate[row * p.gate_stride + p.gate_col + (int64_t)head * p.dim + tid]) + p.gate_bias[(int64_t)head * p.dim + tid],
+                                          p.inv_tau) : 1.f;
+    odd = __syncthreads_or(!(fmaf(0.f, q, 0.f * k) + 0.f * a == 0.f));
+    float sums[1] = {q * p.q_scale * k};
+    sum_of_block(sums, channel_lds);
+    float* rows = made.q + ((int64_t)chunk * made.shares + head) * CHUNK * PAD;
+    if (tid < PAD) {
+      rows[tid] = q * p.q_scale * a, rows[PAD + tid] = k;
+      made.fade[((int64_t)chunk * p.heads + head) * PAD + tid] = odd ? NAN : a;
+    }
+    if (tid == 0) made.within[((int64_t)chunk * p.heads + head) * CHUNK * CHUNK] = sums[0];
+    return;
+  }
   {
     const int token = tid / 8, sub = tid % 8;
     const int64_t row = t0 + min(token, nt - 1);

@@ -30,6 +30,26 @@ __global__ __launch_bounds__(256) void delta_chunk_kernel(const bf16_t* __restri
   if (b < 0) return;
   const int t0 = cu[b] + (chunk - first_chunk(cu[b], b)) * CHUNK, nt = min(CHUNK, cu[b + 1] - t0);
   const int tid = threadIdx.x, wave = tid / MI_WAVE, lane = tid % MI_WAVE;
+  if (cu[b + 1] - cu[b] == 1) {
+    const bf16_t* row = qkv + (int64_t)t0 * qkv_stride + share * dim;
+    const float q = tid < dim ? to_f32(row[tid]) : 0.f, k = tid < dim ? to_f32(row[kv_heads * dim + tid]) : 0.f;
+    float sums[3] = {q * q, k * k, q * k};
+    sum_of_block(sums, lds);
+    const float q_inv = rsqrtf(sums[0] + 1e-6f) * (1.0f / sqrtf((float)dim)), k_inv = rsqrtf(sums[1] + 1e-6f);
+    const int64_t at = ((int64_t)chunk * made.shares + share) * CHUNK * PAD + tid;
+    if (tid < PAD) made.q[at] = q * q_inv, made.k[at] = k * k_inv;
+    for (int h = share * (heads / kv_heads) + tid; h < (share + 1) * (heads / kv_heads); h += 256) {
+      const int64_t of = (int64_t)chunk * heads + h;
+      const bf16_t* p = proj + (int64_t)t0 * proj_stride;
+      const float z = to_f32(p[col_a + h]) + dt_bias[h];
+      const float gate = -(expf(a_log[h]) * (z > 20.f ? z : log1pf(expf(z))));
+      made.factor[of * 2 * CHUNK] = expf(gate);
+      made.factor[of * 2 * CHUNK + CHUNK] = expf(0.f * gate);
+      made.within[of * CHUNK * CHUNK] = expf(0.f * gate) * (sums[2] * q_inv * k_inv);
+      made.solve[of * CHUNK * CHUNK] = 1.f / (1.f + expf(-to_f32(p[col_b + h])));
+    }
+    return;
+  }
   {
     const int token = tid / 8, sub = tid % 8;
     const bf16_t* row = qkv + (int64_t)(t0 + min(token, nt - 1)) * qkv_stride + share * dim;

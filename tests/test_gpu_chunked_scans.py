@@ -270,6 +270,50 @@ def test_what_is_not_finite_goes_token_by_token(monkeypatch, kind, what, dim, vd
     assert out[: 50 if name == "state" else at].isfinite().all()
 
 
+@pytest.mark.parametrize("lengths", [[1] * 5 + [40], [33, 1, 0, 1]])
+@pytest.mark.parametrize("heads,shared,dim,vdim", [(4, 2, 64, 64), (2, 2, 128, 128), (6, 3, 96, 80), (2, 1, 256, 250), (4, 1, 40, 30), (18, 2, 64, 130)])
+@pytest.mark.parametrize("kind", ["delta", "per_head", "per_channel"])
+def test_single_tokens_beside_portions_in_chunks(monkeypatch, kind, lengths, heads, shared, dim, vdim):
+    """Whole and partial groups of the column blocks that a single token's block takes together."""
+    if kind == "delta":
+        test_gated_delta_in_chunks(monkeypatch, lengths, heads, shared, dim, vdim, True, False)
+    else:
+        test_decaying_state_in_chunks(monkeypatch, lengths, heads, shared, dim, vdim, True, kind == "per_head", False)
+
+
+@pytest.mark.parametrize("dim,vdim", [(64, 64), (128, 200)])
+@pytest.mark.parametrize("kind", ["delta", "per_head", "per_channel"])
+def test_single_tokens_that_are_not_finite(monkeypatch, kind, dim, vdim):
+    """Beside a portion in chunks: as `test_what_is_not_finite_goes_token_by_token`, a request for each kind of it."""
+    from mini_infer_amd import ops
+
+    heads, groups, lengths, column = 4, 2, [1] * 8 + [40], vdim - 3
+    tokens, requests = sum(lengths), len(lengths)
+    g = torch.Generator(device=DEV).manual_seed(18)
+    q, k, v = (torch.randn(tokens, n, generator=g, device=DEV).bfloat16() for n in (groups * dim, groups * dim, heads * vdim))
+    per_channel = heads * dim if kind == "per_channel" else heads
+    gate = torch.randn(tokens, per_channel, generator=g, device=DEV).bfloat16()
+    state = _state(g, requests, ops.delta_state_shape(heads, dim, vdim) if kind == "delta" else ops.decay_state_shape(heads, dim, vdim), dim)
+    v[0, vdim + column], v[1, column], k[2, 7], q[3, 7] = float("inf"), float("nan"), float("inf"), float("-inf")
+    gate[4, 0], gate[5, 0], gate[6, 0], state[7, 1, column, 3] = float("inf"), float("-inf"), float("nan"), float("inf")
+    cu, slots = _boundaries(lengths), torch.arange(requests, dtype=torch.int32, device=DEV)
+    if kind == "delta":
+        proj = torch.cat([torch.randn(tokens, heads, generator=g, device=DEV).bfloat16(), gate, torch.randn(tokens, heads * vdim, generator=g, device=DEV).bfloat16()], 1)
+        names = dict(heads=heads, kv_heads=groups, dim=dim, vdim=vdim, eps=1e-6)
+        made = _both(monkeypatch, lambda s: ops.gated_delta(torch.cat([q, k, v], 1), proj, 0, heads, 2 * heads, torch.zeros(heads, device=DEV),
+                                                            torch.full((heads,), -2.0, device=DEV), torch.ones(vdim, device=DEV), s, cu, slots, **names), state)
+    else:
+        names = dict(heads=heads, groups=groups, dim=dim, vdim=vdim, per_head=kind == "per_head", inv_tau=0.0625,
+                     rate=torch.zeros(heads, device=DEV) if kind == "per_head" else None)
+        made = _both(monkeypatch, lambda s: ops.decay_scan(q, 0, k, 0, v, 0, gate, 0, torch.zeros(per_channel, device=DEV), s, cu, slots, **names), state)
+    for got, walked in zip(*made):
+        got, walked = got.double(), walked.double()
+        assert torch.equal(got.isnan(), walked.isnan()) and torch.equal(got.isinf(), walked.isinf()) and torch.equal(got[got.isinf()], walked[walked.isinf()])
+        finite = walked.isfinite()
+        # (the read-out of the delta rule is rounded to bfloat16, else as above)
+        assert float((got - walked)[finite].norm() / walked[finite].norm()) < (2.0 ** -7 if kind == "delta" and got.dim() == 2 else 8e-7)
+
+
 @pytest.mark.parametrize("kind", ["delta", "per_head", "per_channel"])
 @pytest.mark.parametrize("lengths,known,chunks", [
     ([300], True, True), ([300], False, True), ([1] * 15 + [300], True, True), ([64] * 20, False, True),
