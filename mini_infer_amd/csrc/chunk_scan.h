@@ -270,33 +270,18 @@ __device__ __forceinline__ void walk_one_token(const WalkArgs& p, float* sums, i
   }
 }
 
-// grid: heads * column blocks (the heads side by side, so that an XCD's blocks share their chunk data), requests; 256 threads.
-// DT: 16-row tiles of S a wave keeps; pad = 64 * DT.  One wave a SIMD walks, so what a chunk costs is what a wave issues:
-// addresses are a base that is the same for the wave plus a lane's offset made once, without branches (at the end of
-// one everything in flight would be waited for) and multiplications.
+// One wave a SIMD walks, so what a chunk costs is what a wave issues: addresses are a base that is the same for the wave plus a lane's offset made
+// once, without branches (at the end of one everything in flight would be waited for) and multiplications.
 template <int DT, int MODE>
-__global__ __launch_bounds__(256, MODE == DELTA || DT > 2 ? 1 : 2) void walk_kernel(WalkArgs p) {
+__device__ __forceinline__ void walk_portion(const WalkArgs& p, f32x4_t (*parts)[4][MODE == DELTA ? 4 : 2][MI_WAVE], Shared<MODE>* shared, int b, int first, int last,
+                                             int head, int block) {
   constexpr int PAD = 64 * DT;
   constexpr int SUMS = MODE == DELTA ? 4 : 2;
-  __shared__ f32x4_t parts[2][4][SUMS][MI_WAVE];
-  __shared__ __align__(16) Shared<MODE> shared[2];
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / MI_WAVE), lane = threadIdx.x % MI_WAVE;
-  const int head = blockIdx.x % p.heads, b = gridDim.y - 1 - blockIdx.y;
   const uint32_t r = lane % 16, quad = lane / 16;
-  const int col = blockIdx.x / p.heads * 16 + r;
+  const int col = block * 16 + r;
   const bool live = col < p.vdim;
-  const int first = p.cu[b], last = p.cu[b + 1];
-  int* flag = p.again + ((int64_t)b * p.heads + head) * ((p.vdim + 15) / 16) + blockIdx.x / p.heads;
-  if (last <= first) {
-    if (threadIdx.x == 0) *flag = 0;
-    return;
-  }
-  if (last - first == 1) {  // (the other blocks of those that go together have nothing to do)
-    constexpr int TOGETHER = MODE == DELTA ? 8 : 4;
-    static_assert(sizeof(parts) >= sizeof(float) * 4 * TOGETHER * 32, "the sums fit");
-    if (blockIdx.x / p.heads % TOGETHER == 0) walk_one_token<DT, MODE, TOGETHER>(p, reinterpret_cast<float*>(parts), b, first, head, blockIdx.x / p.heads);
-    return;
-  }
+  int* flag = p.again + ((int64_t)b * p.heads + head) * ((p.vdim + 15) / 16) + block;
   const int slot = p.slots[b];
   const int row0 = 16 * DT * wave;  // of S
   const bool kept = live && slot >= 0 && slot < p.num_slots;  // (without a slot: from the spare row, which stays as it is)
@@ -453,12 +438,106 @@ __global__ __launch_bounds__(256, MODE == DELTA || DT > 2 ? 1 : 2) void walk_ker
   }
 }
 
+// The item-th piece of work of a launch: requests of several tokens first, a piece a head and block of 16 columns (the heads side by side, so that an XCD's
+// blocks share their chunk data), then the others, a piece a head and TOGETHER column blocks; each from the last request on, as a step's long portion
+// commonly comes last and its chain should not begin when everything else is done (20 single tokens beside 555 of 32 heads of 128 x 64: 55 us, so 38).
+// False: there are fewer.  All lanes get the same answer.
+struct Piece {
+  int b, first, last, head, block;
+};
+__device__ __forceinline__ bool find_piece(const int* __restrict__ cu, int requests, int heads, int many_each, int one_each, int together, int item, Piece& piece) {
+  const int lane = threadIdx.x % MI_WAVE;
+  int many = 0, from = 0, first = 0, last = 0;
+  auto load = [&](int base) {  // (up to 64 requests: once)
+    from = base;
+    const int b = requests - 1 - base - lane;
+    first = b >= 0 ? cu[b] : 0, last = b >= 0 ? cu[b + 1] : 0;
+  };
+  load(0);
+  auto find = [&](bool of_many, int which) {  // request number `which` of its kind from the last on
+    for (int base = 0; base < requests; base += MI_WAVE) {
+      if (base != from) load(base);
+      const bool is = requests - 1 - base - lane >= 0 && (last - first > 1) == of_many;
+      const uint64_t mask = __ballot(is);
+      const int count = __popcll(mask);
+      if (of_many) many += count;
+      if (which < count) {
+        const int at = __ffsll(__ballot(is && (int)__builtin_amdgcn_mbcnt_hi((uint32_t)(mask >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)mask, 0)) == which)) - 1;
+        piece.b = requests - 1 - base - at;
+        piece.first = __builtin_amdgcn_readlane(first, at);
+        piece.last = __builtin_amdgcn_readlane(last, at);
+        return true;
+      }
+      which -= count;
+    }
+    return false;
+  };
+  if (find(true, item / many_each)) {
+    piece.head = item % many_each % heads, piece.block = item % many_each / heads;
+    return true;
+  }
+  item -= many * many_each;
+  piece.head = item % one_each % heads, piece.block = item % one_each / heads * together;
+  return find(false, item / one_each);
+}
+
+// 256 threads.  DT: 16-row tiles of S a wave keeps; pad = 64 * DT.  grid: heads * column blocks, requests; or, where most requests are known to bring one
+// token (launch_walk), as many blocks as there are pieces of work, of which a block takes every gridDim.x-th.  (Blocks that find nothing to do are not
+// free: each waits for the place of one that works.  31 single tokens beside 64, a block for each request / for each piece: a decay per channel, 16 heads of
+// 128 x 256 66.5 / 54, 8 heads 62.7 / 41; delta rule, 24 heads of 128 x 128 52.2 / 47.6, 8 of 256 x 256 124 / 64, 32 of 128 x 128 55 / 56; a decay per head, 64
+// heads of 128 x 64 43 / 45.  The search costs 1 us.)
+template <int DT, int MODE, bool SEARCH>
+__global__ __launch_bounds__(256, MODE == DELTA || DT > 2 ? 1 : 2) void walk_kernel(WalkArgs p, int requests) {
+  constexpr int TOGETHER = MODE == DELTA ? 8 : 4;
+  __shared__ f32x4_t parts[2][4][MODE == DELTA ? 4 : 2][MI_WAVE];
+  __shared__ __align__(16) Shared<MODE> shared[2];
+  static_assert(sizeof(parts) >= sizeof(float) * 4 * TOGETHER * 32, "a single token's sums fit");
+  const int blocks = (p.vdim + 15) / 16;
+  auto make = [&](const Piece& at) {
+    if (at.last - at.first > 1) {
+      walk_portion<DT, MODE>(p, parts, shared, at.b, at.first, at.last, at.head, at.block);
+    } else if (at.block % TOGETHER == 0) {
+      if (at.last - at.first == 1) walk_one_token<DT, MODE, TOGETHER>(p, reinterpret_cast<float*>(parts), at.b, at.first, at.head, at.block);
+      else if (threadIdx.x < TOGETHER && at.block + (int)threadIdx.x < blocks) p.again[((int64_t)at.b * p.heads + at.head) * blocks + at.block + threadIdx.x] = 0;
+    }
+  };
+  Piece at;
+  if constexpr (SEARCH) {
+    const int one_each = p.heads * ((blocks + TOGETHER - 1) / TOGETHER);
+    for (int item = blockIdx.x; find_piece(p.cu, requests, p.heads, p.heads * blocks, one_each, TOGETHER, item, at); item += gridDim.x) {
+      if (item != (int)blockIdx.x) __syncthreads();  // (the last piece's sums have been read)
+      make(at);
+    }
+  } else {
+    at.b = requests - 1 - (int)blockIdx.y, at.head = blockIdx.x % p.heads, at.block = blockIdx.x / p.heads;
+    at.first = p.cu[at.b], at.last = p.cu[at.b + 1];
+    make(at);
+  }
+}
+
 template <int MODE>
-static int launch_walk(const WalkArgs& p, int pad, int requests, hipStream_t stream) {
-  dim3 grid(p.heads * ceil_div(p.vdim, 16), requests);
-  if (pad == 64) walk_kernel<1, MODE><<<grid, 256, 0, stream>>>(p);
-  else if (pad == 128) walk_kernel<2, MODE><<<grid, 256, 0, stream>>>(p);
-  else walk_kernel<4, MODE><<<grid, 256, 0, stream>>>(p);
+static int launch_walk(const WalkArgs& p, int pad, int tokens, int requests, int longest, hipStream_t stream) {
+  constexpr int TOGETHER = MODE == DELTA ? 8 : 4;
+  const int blocks = ceil_div(p.vdim, 16), others = requests - 1;
+  // requests of several tokens: where every one brings a token those that bring more; not known: as if there were one long portion, with a few
+  // rounds of blocks in case there are more
+  const int many = longest == 1 ? requests : longest == 0 ? 1 : 1 + max(0, min(others, tokens - longest - others));
+  const int64_t all = (int64_t)requests * p.heads * blocks, a_few_rounds = 8 * mi_compute_units();
+  const int64_t pieces = (int64_t)p.heads * ((int64_t)many * blocks + (int64_t)(requests - many) * ceil_div(blocks, TOGETHER));
+  MI_REQUIRE(all < ((int64_t)1 << 30), "chunk_walk: %d requests of %d heads", requests, p.heads);
+  // (a decay per head, and the delta rule where a request has a block for each compute unit, are as fast or up to 5 % faster with a block for each request)
+  constexpr bool SEARCHED = MODE != PER_HEAD;
+  const bool search = SEARCHED && (MODE == PER_CHANNEL || p.heads * blocks < mi_compute_units()) && many < requests && all > a_few_rounds;
+  const dim3 grid = search ? dim3((unsigned)(longest == 0 ? max(pieces, a_few_rounds) : pieces)) : dim3(p.heads * blocks, requests);
+#define MI_WALK(DT)                                                                                  \
+  do {                                                                                               \
+    if (search) walk_kernel<DT, MODE, SEARCHED><<<grid, 256, 0, stream>>>(p, requests);              \
+    else walk_kernel<DT, MODE, false><<<grid, 256, 0, stream>>>(p, requests);                        \
+  } while (0)
+  if (pad == 64) MI_WALK(1);
+  else if (pad == 128) MI_WALK(2);
+  else MI_WALK(4);
+#undef MI_WALK
   MI_CHECK_LAUNCH("chunk_walk");
   return MI_OK;
 }

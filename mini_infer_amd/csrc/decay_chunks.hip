@@ -241,12 +241,12 @@ extern "C" int64_t mi_decay_scan_chunks_scratch(int mode, int num_tokens, int nu
          flag_count(num_requests, heads, vdim);
 }
 
-// As mi_decay_scan for bfloat16, with `scratch` on 16 bytes.
+// As mi_decay_scan for bfloat16, with `scratch` on 16 bytes; longest: tokens of the longest portion, 0: not known.
 extern "C" int mi_decay_scan_chunks(int mode, const void* q, int64_t q_stride, int q_col, const void* k, int64_t k_stride, int k_col,
                                     const void* v, int64_t v_stride, int v_col, const void* gate, int64_t gate_stride, int gate_col,
                                     const float* gate_bias, const float* rate, const float* skip, float inv_tau, float q_scale,
                                     float* state, int64_t state_stride, const int* cu, const int* slots, int num_slots, float* scratch,
-                                    float* out, int num_tokens, int num_requests, int heads, int groups, int dim, int vdim,
+                                    float* out, int num_tokens, int num_requests, int longest, int heads, int groups, int dim, int vdim,
                                     hipStream_t stream) {
   const int bad = mi_decay_scan_check(MI_BF16, mode, q_stride, q_col, k_stride, k_col, v_stride, v_col, gate_stride, gate_col, gate_bias,
                                       rate, state, state_stride, num_slots, num_tokens, num_requests, heads, groups, dim, vdim);
@@ -293,7 +293,8 @@ extern "C" int mi_decay_scan_chunks(int mode, const void* q, int64_t q_stride, i
   p.v = (const bf16_t*)v, p.v_stride = v_stride, p.v_col = v_col, p.skip = skip;
   p.state = state, p.state_stride = state_stride, p.cu = cu, p.slots = slots, p.num_slots = num_slots;
   p.out = out, p.again = again, p.heads = heads, p.vdim = vdim;
-  const int walked = mode == PER_CHANNEL ? launch_walk<PER_CHANNEL>(p, pad, num_requests, stream) : launch_walk<PER_HEAD>(p, pad, num_requests, stream);
+  const int walked = mode == PER_CHANNEL ? launch_walk<PER_CHANNEL>(p, pad, num_tokens, num_requests, longest, stream)
+                                         : launch_walk<PER_HEAD>(p, pad, num_tokens, num_requests, longest, stream);
   if (walked != MI_OK) return walked;
   return mi_decay_scan_again(mode, q, q_stride, q_col, k, k_stride, k_col, v, v_stride, v_col, gate, gate_stride, gate_col, gate_bias, rate,
                              skip, inv_tau, q_scale, state, state_stride, cu, slots, num_slots, out, again, num_requests, heads, groups, dim,

@@ -166,12 +166,12 @@ extern "C" int64_t mi_gated_delta_chunks_scratch(int num_tokens, int num_request
          flag_count(num_requests, heads, vdim);
 }
 
-// As mi_gated_delta for bfloat16, with `scratch` on 16 bytes.
+// As mi_gated_delta for bfloat16, with `scratch` on 16 bytes; longest: tokens of the longest portion, 0: not known.
 extern "C" int mi_gated_delta_chunks(const void* qkv, int64_t qkv_stride, const void* proj, int64_t proj_stride, int col_b, int col_a,
                                      int col_g, const float* a_log, const float* dt_bias, const float* norm_weight, float* state,
                                      int64_t state_stride, const int* cu, const int* slots, float* readout, float* scratch, void* out,
-                                     int64_t out_stride, int num_tokens, int num_requests, int heads, int kv_heads, int dim, int vdim,
-                                     int dim_pad, float eps, int num_slots, hipStream_t stream) {
+                                     int64_t out_stride, int num_tokens, int num_requests, int longest, int heads, int kv_heads, int dim,
+                                     int vdim, int dim_pad, float eps, int num_slots, hipStream_t stream) {
   const int bad = mi_gated_delta_check(qkv_stride, proj_stride, col_b, col_a, col_g, state, state_stride, out_stride, num_requests, heads,
                                        kv_heads, dim, vdim, dim_pad, eps, num_slots);
   if (bad != MI_OK) return bad;
@@ -203,7 +203,7 @@ extern "C" int mi_gated_delta_chunks(const void* qkv, int64_t qkv_stride, const 
   p.skip = nullptr;
   p.state = state, p.state_stride = state_stride, p.cu = cu, p.slots = slots, p.num_slots = num_slots;
   p.out = readout, p.again = again, p.heads = heads, p.vdim = vdim;
-  const int walked = launch_walk<DELTA>(p, dim_pad, num_requests, stream);
+  const int walked = launch_walk<DELTA>(p, dim_pad, num_tokens, num_requests, longest, stream);
   if (walked != MI_OK) return walked;
   const int redone = mi_delta_again(qkv, qkv_stride, proj, proj_stride, col_b, col_a, a_log, dt_bias, state, state_stride, cu, slots, readout,
                                     again, num_requests, heads, kv_heads, dim, vdim, num_slots, stream);

@@ -2496,38 +2496,43 @@ def delta_state_shape(heads: int, dim: int, vdim: int) -> tuple[int, int, int]:
 
 # Microseconds of a recurrence over a step's rows with keys of up to so many columns: token by token (the launches, a request and a
 # token on a full chip, a token of the longest portion) and in chunks of 32 (the launches, a request on a full chip, a chunk of the
-# longest portion).  Fitted to 1,508 measured pairs: 1 to 100 requests of 8 to 512 tokens, single tokens beside one portion, 4 to 80
+# longest portion, a request of one token on a full chip).  Fitted to 1,508 measured pairs: 1 to 100 requests of 8 to 512 tokens, single tokens beside one portion, 4 to 80
 # heads of 64 to 512 columns; half of the times are within 5 %.  (A request's share of the decays token by token: fitted to 8 to 80 single
-# tokens of 16 to 64 heads since their blocks spread over the XCDs; beside a portion these expect 10 to 25 % more than is measured.)
+# tokens of 16 to 64 heads since their blocks spread over the XCDs; beside a portion these expect 10 to 25 % more than is measured.  Single tokens in chunks: 210 steps of 4 to 100
+# beside a portion of 32 to 600, within 7 %.)
 _SCAN_TIMES = {
-    ("delta", 64): (6.95, 0.89, 0.093, 0.288, 18.3, 2.33, 1.82),
-    ("delta", 128): (8.39, 2.13, 0.161, 0.428, 21, 3.14, 2.26),
-    ("delta", 256): (7.82, 3.4, 0.288, 0.62, 24.7, 7.38, 4.32),
-    ("per_head", 64): (3.85, 0.33, 0.0355, 0.252, 13.4, 0.971, 1.13),
-    ("per_head", 128): (3.43, 0.61, 0.0864, 0.303, 14, 1.68, 1.52),
-    ("per_head", 256): (2.44, 1.65, 0.19, 0.472, 16.4, 3.59, 2.36),
-    ("per_channel", 64): (3.98, 0.32, 0.0473, 0.267, 17.5, 1.57, 1.05),
-    ("per_channel", 128): (3.28, 0.775, 0.121, 0.348, 23.4, 2.35, 1.71),
-    ("per_channel", 256): (1.11, 2.1, 0.256, 0.58, 31.6, 5.51, 3.08),
+    ("delta", 64): (6.95, 0.89, 0.093, 0.288, 18.3, 2.33, 1.82, 0.778),
+    ("delta", 128): (8.39, 2.13, 0.161, 0.428, 21, 3.14, 2.26, 0.851),
+    ("delta", 256): (7.82, 3.4, 0.288, 0.62, 24.7, 7.38, 4.32, 1.56),
+    ("per_head", 64): (3.85, 0.33, 0.0355, 0.252, 13.4, 0.971, 1.13, 0.419),
+    ("per_head", 128): (3.43, 0.61, 0.0864, 0.303, 14, 1.68, 1.52, 0.787),
+    ("per_head", 256): (2.44, 1.65, 0.19, 0.472, 16.4, 3.59, 2.36, 1.36),
+    ("per_channel", 64): (3.98, 0.32, 0.0473, 0.267, 17.5, 1.57, 1.05, 0.563),
+    ("per_channel", 128): (3.28, 0.775, 0.121, 0.348, 23.4, 2.35, 1.71, 0.751),
+    ("per_channel", 256): (1.11, 2.1, 0.256, 0.58, 31.6, 5.51, 3.08, 1.49),
 }
 
 
 def scan_times(kind: str, tokens: int, requests: int, longest: int | None, heads: int, dim: int, vdim: int) -> tuple[float, float]:
     """About how many microseconds a recurrence takes token by token and in chunks.  A long portion is a chain of tokens (0.3 to 0.45
-    microseconds each at keys of 128) or of chunks (1.5 to 2.3), but a chunk costs the same with one token in it.  `longest`: tokens
+    microseconds each at keys of 128) or of chunks (1.5 to 2.3); a portion's chunk costs the same with fewer tokens in it, a single token less.  `longest`: tokens
     of the step's longest portion; None (a recorded step): as if it were one portion beside single tokens, a scheduler's ordinary step."""
-    launches, request, token, chain, chunk_launches, chunk_request, chunk_chain = _SCAN_TIMES[kind, 64 if dim <= 64 else 128 if dim <= 128 else 256]
+    launches, request, token, chain, chunk_launches, chunk_request, chunk_chain, chunk_single = _SCAN_TIMES[kind, 64 if dim <= 64 else 128 if dim <= 128 else 256]
     longest = max(1, tokens - requests + 1) if longest is None else longest
     full = heads * -(-vdim // 16) / 256  # of the chip, by one request
     walked = launches + request * requests * full + max(token * tokens * full, chain * longest)
-    return walked, chunk_launches + chunk_request * requests * full + chunk_chain * longest / 32
+    if tokens <= requests:  # (single tokens: there are launches for these)
+        return walked, math.inf
+    # (requests of several tokens: the longest, and as many others as there are tokens beyond one for each)
+    singles = requests - 1 - max(0, min(requests - 1, tokens - longest - (requests - 1)))
+    return walked, chunk_launches + (chunk_request * (requests - singles) + chunk_single * singles) * full + chunk_chain * longest / 32
 
 
 def chunked_scan_pays(walked: float, chunked: float, widest: int) -> bool:
     """Whether a recurrence over a step's rows is taken 32 tokens at a time on the matrix cores rather than token by token, from
     what `scan_times` expects of the two.  At this margin 1 of 1,508 measured steps is slower than token by token (6 %), and
     together they are 1.17 times as fast (1.19 with the better one each time).  Microseconds, token by token against in chunks, of
-    the delta rule with 32 heads of 128 x 128: 2,048 tokens 887 / 181, 70 tokens 39 / 29, 256 beside 15 single tokens 161 / 83, 16
+    the delta rule with 32 heads of 128 x 128: 2,048 tokens 887 / 181, 70 tokens 39 / 29, 256 beside 16 single tokens 160 / 56, 64 beside 31 97 / 56, 16
     portions of 32 116 / 74, not taken: 4 of 20 33 / 33, 16 of 8 60 / 70, 100 of 4 243 / 331; a decay per head, 48 heads of 128 x 64:
     2,048 tokens 705 / 117, 16 portions of 32 43 / 36, not taken: 16 of 16 25 / 36; per channel, 12 heads of 128 x 256: 2,048 tokens
     818 / 125, 32 portions of 32 112 / 75, not taken: 4 of 64 29 / 37.  `widest`: values from one row to the next of the widest operand
@@ -2581,7 +2586,7 @@ def gated_delta(
                 lib.mi_gated_delta_chunks(
                     _ptr(qkv), qkv.stride(0), _ptr(proj), proj.stride(0), int(col_b), int(col_a), int(col_g),
                     _ptr(a_log), _ptr(dt_bias), _ptr(norm_weight), _ptr(state), state.stride(0), _ptr(cu_seqlens), _ptr(slots),
-                    _ptr(readout), _ptr(scratch), _ptr(out), out.stride(0), qkv.shape[0], requests, heads, kv_heads, dim, vdim, shape[2],
+                    _ptr(readout), _ptr(scratch), _ptr(out), out.stride(0), qkv.shape[0], requests, longest or 0, heads, kv_heads, dim, vdim, shape[2],
                     float(eps), state.shape[0] - 1, _stream(),
                 )
             )
@@ -3009,7 +3014,7 @@ def decay_scan(
                     int(per_head), _ptr(q), q.stride(0), int(q_col), _ptr(k), k.stride(0), int(k_col), _ptr(v), v.stride(0), int(v_col),
                     _ptr(gate), gate.stride(0), int(gate_col), _ptr(gate_bias), _ptr(rate), _ptr(skip), float(inv_tau), float(q_scale),
                     _ptr(state), state.stride(0), _ptr(cu_seqlens), _ptr(slots), state.shape[0] - 1, _ptr(scratch), _ptr(out), tokens,
-                    requests, heads, groups, dim, vdim, _stream(),
+                    requests, longest or 0, heads, groups, dim, vdim, _stream(),
                 )
             )
             return out

@@ -14,7 +14,7 @@ from pathlib import Path
 from mini_infer_amd.exceptions import ExtensionMissingError, KernelShapeError
 from mini_infer_amd.ops import build as _build
 
-ABI_VERSION = 54
+ABI_VERSION = 55
 
 _lib: ctypes.CDLL | None = None
 _lib_path: Path | None = None
@@ -130,7 +130,7 @@ _SIGNATURES: dict[str, list] = {
     ],
     "mi_gated_delta_chunks": [
         _P, c_int64, _P, c_int64, c_int, c_int, c_int, _P, _P, _P, _P, c_int64, _P, _P, _P, _P, _P, c_int64, c_int, c_int, c_int, c_int,
-        c_int, c_int, c_int, c_float, c_int, _P,
+        c_int, c_int, c_int, c_int, c_float, c_int, _P,
     ],
     "mi_gated_delta_chunks_scratch": [c_int, c_int, c_int, c_int, c_int, c_int],
     "mi_gated_delta_rows": [c_int, c_int],
@@ -148,7 +148,7 @@ _SIGNATURES: dict[str, list] = {
     ],
     "mi_decay_scan_chunks": [
         c_int, _P, c_int64, c_int, _P, c_int64, c_int, _P, c_int64, c_int, _P, c_int64, c_int, _P, _P, _P, c_float,
-        c_float, _P, c_int64, _P, _P, c_int, _P, _P, c_int, c_int, c_int, c_int, c_int, c_int, _P,
+        c_float, _P, c_int64, _P, _P, c_int, _P, _P, c_int, c_int, c_int, c_int, c_int, c_int, c_int, _P,
     ],
     "mi_decay_scan_chunks_scratch": [c_int, c_int, c_int, c_int, c_int, c_int, c_int],
     "mi_decay_scan_dim_pad": [c_int],
