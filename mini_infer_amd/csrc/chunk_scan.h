@@ -34,10 +34,10 @@
 // tokens before it, quotients behind a decay of zero are infinity less infinity, and a chunk's decays together may be zero, which
 // makes NaN of an infinite state that each by itself leaves infinite.  Whatever is not finite in the state, the values, the
 // gates, and (for the delta rule by itself, else through the factors) in queries and keys stays in S to the end: products with
-// zero keep it.  So where a block's S does not end finite it leaves the state as it found it and sets its flag, and a last
-// launch takes the flagged columns again with the token-by-token kernel.  That launch costs 3 us where nothing is flagged, and the
-// barrier at a block's end 0.3 us; sums of what a chunk adds and of Q S0, the same in all waves and without a barrier, cost more
-// (77.6 us for the 70 of a decay per head).
+// zero keep it.  So where a block's S does not end finite it leaves the state as it found it and takes its columns again, token by token (walk_by_token).
+// (A launch of their own behind the walk for columns that it had flagged: 4.6 us of every call.  Three prompts of 80 tokens, 12 layers, 2,165 / 2,126 us, of
+// 67 at 8B widths 4,135 / 4,090, one token beside 144 1,548 / 1,530.)  The barrier at a block's end costs 0.3 us;
+// sums of what a chunk adds and of Q S0, the same in all waves and without a barrier, cost more (77.6 us for the 70 of a decay per head).
 #pragma once
 #include "common.h"
 
@@ -66,7 +66,6 @@ struct Made {
 // the chunks of request b from one request to the next.
 __device__ __forceinline__ int first_chunk(int cu_b, int b) { return cu_b / CHUNK + b; }
 static inline int64_t chunk_count(int tokens, int requests) { return (int64_t)tokens / CHUNK + requests; }
-static inline int64_t flag_count(int requests, int heads, int vdim) { return (int64_t)requests * heads * ceil_div(vdim, 16); }
 
 // Of a request's only token the first launch leaves what walk_one_token reads and nothing else: row 0 of q and k (without DELTA: k as row 1 of q), the
 // first value of W, of T w and of both factors, and the fade.  One thread a channel makes it.
@@ -134,7 +133,6 @@ struct WalkArgs {
   const int *cu, *slots;
   int num_slots;
   float* out;  // float32 [tokens, heads * vdim]
-  int* again;  // [requests][heads][column blocks of 16]: 1 where the columns are to be taken token by token
   int heads, vdim;
 };
 constexpr int64_t MAX_ROW = 1 << 24;
@@ -181,12 +179,13 @@ struct Shared {
 // while it brought in 40 KB of operands.  Every wave keeps its rows of S as in the walk.  Steps with single tokens beside a long portion, all of them in chunks
 // / so: 34 and 500 of the delta rule with 32 heads of 128 x 128 (12 layers, half of them of the rule) 5,625 / 5,036 us, 25 and 400 with 24 heads 3,278 / 2,902, 34 and 700
 // with 64 heads of 128 x 64 8,551 / 7,847 (the long portion's blocks first in both: before that 8,847).
+// Returns the column blocks that did not end finite and whose state is as it was, a bit each.
 template <int DT, int MODE, int G>
-__device__ __forceinline__ void walk_one_token(const WalkArgs& p, float* sums, int b, int first, int head, int block0) {
+__device__ __forceinline__ int walk_one_token(const WalkArgs& p, float* sums, int b, int first, int head, int block0) {
   constexpr int PAD = 64 * DT;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / MI_WAVE), lane = threadIdx.x % MI_WAVE;
   const int r = lane % 16, quad = lane / 16, row0 = 16 * DT * wave + 4 * quad;
-  const int slot = p.slots[b], blocks = (p.vdim + 15) / 16;
+  const int slot = p.slots[b];
   const bool kept = slot >= 0 && slot < p.num_slots;
   float* state = p.state + (int64_t)(kept ? slot : p.num_slots) * p.state_stride + (int64_t)head * p.vdim * PAD + row0;
   const int64_t chunk = first_chunk(first, b), rows = chunk * p.made.shares + head / (p.heads / p.made.shares), of = chunk * p.heads + head;
@@ -259,21 +258,23 @@ __device__ __forceinline__ void walk_one_token(const WalkArgs& p, float* sums, i
   if (lane == 0) odd_of[wave] = odd;
   __syncthreads();
   odd = (odd_of[0] | odd_of[1]) | (odd_of[2] | odd_of[3]);
-  if (threadIdx.x < G && block0 + (int)threadIdx.x < blocks) p.again[((int64_t)b * p.heads + head) * blocks + block0 + threadIdx.x] = odd >> threadIdx.x & 1;
-  if (!kept) return;
+  if (kept) {
 #pragma unroll
-  for (int g = 0; g < G; ++g) {
-    const int col = (block0 + g) * 16 + r;
-    if (col >= p.vdim || (odd >> g & 1)) continue;
+    for (int g = 0; g < G; ++g) {
+      const int col = (block0 + g) * 16 + r;
+      if (col >= p.vdim || (odd >> g & 1)) continue;
 #pragma unroll
-    for (int d = 0; d < DT; ++d) *reinterpret_cast<f32x4_t*>(state + (int64_t)col * PAD + 16 * d) = S[g][d];
+      for (int d = 0; d < DT; ++d) *reinterpret_cast<f32x4_t*>(state + (int64_t)col * PAD + 16 * d) = S[g][d];
+    }
   }
+  return odd;
 }
 
 // One wave a SIMD walks, so what a chunk costs is what a wave issues: addresses are a base that is the same for the wave plus a lane's offset made
 // once, without branches (at the end of one everything in flight would be waited for) and multiplications.
+// Returns whether S did not end finite; the state is then as it was.
 template <int DT, int MODE>
-__device__ __forceinline__ void walk_portion(const WalkArgs& p, f32x4_t (*parts)[4][MODE == DELTA ? 4 : 2][MI_WAVE], Shared<MODE>* shared, int b, int first, int last,
+__device__ __forceinline__ bool walk_portion(const WalkArgs& p, f32x4_t (*parts)[4][MODE == DELTA ? 4 : 2][MI_WAVE], Shared<MODE>* shared, int b, int first, int last,
                                              int head, int block) {
   constexpr int PAD = 64 * DT;
   constexpr int SUMS = MODE == DELTA ? 4 : 2;
@@ -281,7 +282,6 @@ __device__ __forceinline__ void walk_portion(const WalkArgs& p, f32x4_t (*parts)
   const uint32_t r = lane % 16, quad = lane / 16;
   const int col = block * 16 + r;
   const bool live = col < p.vdim;
-  int* flag = p.again + ((int64_t)b * p.heads + head) * ((p.vdim + 15) / 16) + block;
   const int slot = p.slots[b];
   const int row0 = 16 * DT * wave;  // of S
   const bool kept = live && slot >= 0 && slot < p.num_slots;  // (without a slot: from the spare row, which stays as it is)
@@ -431,10 +431,72 @@ __device__ __forceinline__ void walk_portion(const WalkArgs& p, f32x4_t (*parts)
 #pragma unroll
   for (int d = 0; d < DT; ++d) zeros += 0.f * S[d];
   const bool again = __syncthreads_or(!((zeros[0] + zeros[1]) + (zeros[2] + zeros[3]) == 0.f));
-  if (threadIdx.x == 0) *flag = again;
   if (kept && !again) {
 #pragma unroll
     for (int d = 0; d < DT; ++d) *reinterpret_cast<f32x4_t*>(mine + 16 * d) = S[d];
+  }
+  return again;
+}
+
+// 16 columns token by token, for what is not finite: 16 lanes a column, 4 * DT rows a lane, every operand read and made by each lane itself, in the arithmetic of
+// the token-by-token kernels.  It is not fast, 2,048 tokens with a NaN 2.3 to 4.8 ms where those kernels take 0.9: a launch of theirs for it, nearly always with nothing
+// to do, was a step of 12 such layers' 1 to 2 %.  Rows: what brings a token's operands (Rows::operands in the .hip files: rows at .. at + R of q, k and the decays, and the
+// step size or write strength).
+template <int CTRL>
+__device__ __forceinline__ float lane_moved(float v) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true));
+}
+__device__ __forceinline__ float sum_of_16(float v) {  // (neighbours, pairs, the mirror images inside 8 and inside 16 lanes)
+  v += lane_moved<0xB1>(v);
+  v += lane_moved<0x4E>(v);
+  v += lane_moved<0x141>(v);
+  return v + lane_moved<0x140>(v);
+}
+template <int DT, int MODE, typename Rows>
+__device__ __forceinline__ void walk_by_token(const WalkArgs& p, const Rows& rows, int b, int first, int last, int head, int block) {
+  constexpr int R = 4 * DT, PAD = 64 * DT;
+  const int part = threadIdx.x % 16, col = block * 16 + threadIdx.x / 16, slot = p.slots[b];
+  const bool live = col < p.vdim, kept = live && slot >= 0 && slot < p.num_slots;
+  const int column = live ? col : p.vdim - 1;
+  float* mine = p.state + (int64_t)(kept ? slot : p.num_slots) * p.state_stride + ((int64_t)head * p.vdim + column) * PAD + part * R;
+  constexpr int BATCH = MODE == PER_CHANNEL || DT > 2 ? 2 : 4;  // tokens whose operands are asked for together (more: registers of the whole kernel)
+  float S[R];
+#pragma unroll
+  for (int i = 0; i < R; ++i) S[i] = mine[i];
+  const float skip = (MODE == PER_HEAD && p.skip) ? p.skip[head] : 0.f;
+  for (int t0 = first; t0 < last; t0 += BATCH) {
+    float q[BATCH][R], k[BATCH][R], a[BATCH][R], step[BATCH], x[BATCH];
+#pragma unroll
+    for (int n = 0; n < BATCH; ++n) {  // (past the last token that one again)
+      const int t = min(t0 + n, last - 1);
+      x[n] = to_f32(p.v[(int64_t)t * p.v_stride + p.v_col + (int64_t)head * p.vdim + column]);
+      step[n] = rows.template operands<R>(t, head, p.heads, part * R, q[n], k[n], a[n]);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int n = 0; n < BATCH; ++n) {
+      if (t0 + n >= last) break;
+      float u = step[n] * x[n];
+      if constexpr (MODE == DELTA) {
+        float seen = 0.f;
+#pragma unroll
+        for (int i = 0; i < R; ++i) seen = fmaf(S[i], k[n][i], seen);
+        u = step[n] * (x[n] - sum_of_16(seen) * a[n][0]);
+      }
+      float read = 0.f;
+#pragma unroll
+      for (int i = 0; i < R; ++i) {
+        S[i] = fmaf(k[n][i], u, a[n][i] * S[i]);
+        read = fmaf(S[i], q[n][i], read);
+      }
+      read = sum_of_16(read);
+      if constexpr (MODE == PER_HEAD) read = fmaf(skip, x[n], read);
+      if (part == 0 && live) p.out[((int64_t)(t0 + n) * p.heads + head) * p.vdim + col] = read;
+    }
+  }
+  if (kept) {
+#pragma unroll
+    for (int i = 0; i < R; ++i) mine[i] = S[i];
   }
 }
 
@@ -486,20 +548,20 @@ __device__ __forceinline__ bool find_piece(const int* __restrict__ cu, int reque
 // free: each waits for the place of one that works.  31 single tokens beside 64, a block for each request / for each piece: a decay per channel, 16 heads of
 // 128 x 256 66.5 / 54, 8 heads 62.7 / 41; delta rule, 24 heads of 128 x 128 52.2 / 47.6, 8 of 256 x 256 124 / 64, 32 of 128 x 128 55 / 56; a decay per head, 64
 // heads of 128 x 64 43 / 45.  The search costs 1 us.)
-template <int DT, int MODE, bool SEARCH>
-__global__ __launch_bounds__(256, MODE == DELTA || DT > 2 ? 1 : 2) void walk_kernel(WalkArgs p, int requests) {
+template <int DT, int MODE, bool SEARCH, typename Rows>
+__global__ __launch_bounds__(256, MODE == DELTA || DT > 2 ? 1 : 2) void walk_kernel(WalkArgs p, Rows rows, int requests) {
   constexpr int TOGETHER = MODE == DELTA ? 8 : 4;
   __shared__ f32x4_t parts[2][4][MODE == DELTA ? 4 : 2][MI_WAVE];
   __shared__ __align__(16) Shared<MODE> shared[2];
   static_assert(sizeof(parts) >= sizeof(float) * 4 * TOGETHER * 32, "a single token's sums fit");
   const int blocks = (p.vdim + 15) / 16;
   auto make = [&](const Piece& at) {
-    if (at.last - at.first > 1) {
-      walk_portion<DT, MODE>(p, parts, shared, at.b, at.first, at.last, at.head, at.block);
-    } else if (at.block % TOGETHER == 0) {
-      if (at.last - at.first == 1) walk_one_token<DT, MODE, TOGETHER>(p, reinterpret_cast<float*>(parts), at.b, at.first, at.head, at.block);
-      else if (threadIdx.x < TOGETHER && at.block + (int)threadIdx.x < blocks) p.again[((int64_t)at.b * p.heads + at.head) * blocks + at.block + threadIdx.x] = 0;
-    }
+    int odd = 0;
+    if (at.last - at.first > 1) odd = walk_portion<DT, MODE>(p, parts, shared, at.b, at.first, at.last, at.head, at.block);
+    else if (at.last - at.first == 1 && at.block % TOGETHER == 0)
+      odd = walk_one_token<DT, MODE, TOGETHER>(p, reinterpret_cast<float*>(parts), at.b, at.first, at.head, at.block);
+    for (int g = 0; odd >> g != 0; ++g)
+      if ((odd >> g & 1) && at.block + g < blocks) walk_by_token<DT, MODE>(p, rows, at.b, at.first, at.last, at.head, at.block + g);
   };
   Piece at;
   if constexpr (SEARCH) {
@@ -515,8 +577,8 @@ __global__ __launch_bounds__(256, MODE == DELTA || DT > 2 ? 1 : 2) void walk_ker
   }
 }
 
-template <int MODE>
-static int launch_walk(const WalkArgs& p, int pad, int tokens, int requests, int longest, hipStream_t stream) {
+template <int MODE, typename Rows>
+static int launch_walk(const WalkArgs& p, const Rows& rows, int pad, int tokens, int requests, int longest, hipStream_t stream) {
   constexpr int TOGETHER = MODE == DELTA ? 8 : 4;
   const int blocks = ceil_div(p.vdim, 16), others = requests - 1;
   // requests of several tokens: where every one brings a token those that bring more; not known: as if there were one long portion, with a few
@@ -531,8 +593,8 @@ static int launch_walk(const WalkArgs& p, int pad, int tokens, int requests, int
   const dim3 grid = search ? dim3((unsigned)(longest == 0 ? max(pieces, a_few_rounds) : pieces)) : dim3(p.heads * blocks, requests);
 #define MI_WALK(DT)                                                                                  \
   do {                                                                                               \
-    if (search) walk_kernel<DT, MODE, SEARCHED><<<grid, 256, 0, stream>>>(p, requests);              \
-    else walk_kernel<DT, MODE, false><<<grid, 256, 0, stream>>>(p, requests);                        \
+    if (search) walk_kernel<DT, MODE, SEARCHED><<<grid, 256, 0, stream>>>(p, rows, requests);        \
+    else walk_kernel<DT, MODE, false><<<grid, 256, 0, stream>>>(p, rows, requests);                  \
   } while (0)
   if (pad == 64) MI_WALK(1);
   else if (pad == 128) MI_WALK(2);

@@ -245,23 +245,6 @@ __device__ __forceinline__ void mi_write_page_rows(T* v_pages, int t, int page, 
   }
 }
 
-// Blocks of a launch that looks for flagged work and usually finds none.
-constexpr int AGAIN_BLOCKS = 512;
-
-// Calls take(i) for every i < total with flagged(i), an item a block at a time; all 256 threads of the block call this.
-template <typename F, typename G>
-__device__ __forceinline__ void mi_take_flagged(int64_t total, F flagged, G take) {
-  for (int64_t base = blockIdx.x; base < total; base += (int64_t)256 * gridDim.x) {
-    const int64_t mine = base + (int64_t)threadIdx.x * gridDim.x;
-    if (!__syncthreads_or(mine < total && flagged(mine))) continue;
-    for (int64_t i = base; i < min(total, base + (int64_t)256 * gridDim.x); i += gridDim.x) {
-      if (!flagged(i)) continue;
-      take(i);
-      __syncthreads();
-    }
-  }
-}
-
 // The two elements of a head that are rotated together.  Each is one product, rounded, and one fused multiply-add; which of an element's two products
 // is rounded shows in its last bit, and left to the compiler that differed from kernel to kernel.
 __device__ __forceinline__ void mi_rotate(float x0, float x1, float c, float s, float& y0, float& y1) {

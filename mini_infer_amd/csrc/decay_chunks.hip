@@ -20,6 +20,37 @@ struct RowArgs {
   bool eights;  // rows of q, k (and the channels' gates) lie on 16 bytes in whole 8s
 };
 
+// What walk_by_token reads.
+template <int MODE>
+struct TokenRows {
+  RowArgs p;
+  template <int R>
+  __device__ __forceinline__ float operands(int t, int head, int heads, int at, float (&q)[R], float (&k)[R], float (&a)[R]) const {
+    const int64_t row = t, share = head / (heads / p.groups) * (int64_t)p.dim;
+    const bf16_t* gate = p.gate + row * p.gate_stride + p.gate_col;
+    float decay = 0.f, step = 1.f;
+    if constexpr (MODE == PER_HEAD) {
+      step = mi_soft_plus_fast(to_f32(gate[head]) + p.gate_bias[head]);
+      decay = __builtin_amdgcn_exp2f(-(expf(p.rate[head]) * 1.4426950408889634f) * step);
+    }
+    const bf16_t *q_row = p.q + row * p.q_stride + p.q_col + share, *k_row = p.k + row * p.k_stride + p.k_col + share;
+#pragma unroll
+    for (int i = 0; i < R; ++i) {  // (without branches, past the last channel that one again)
+      const int d = min(at + i, p.dim - 1);
+      const bool in = at + i < p.dim;
+      const float qv = to_f32(q_row[d]) * p.q_scale, kv = to_f32(k_row[d]);
+      q[i] = in ? qv : 0.f, k[i] = in ? kv : 0.f;
+      if constexpr (MODE == PER_HEAD) {
+        a[i] = decay;
+      } else {
+        const float av = mi_channel_decay(to_f32(gate[(int64_t)head * p.dim + d]) + p.gate_bias[(int64_t)head * p.dim + d], p.inv_tau);
+        a[i] = in ? av : 0.f;
+      }
+    }
+    return step;
+  }
+};
+
 // a decay per head: one block per (chunk, group of rows, 8 heads of the group), 4 waves
 template <int DT>
 __global__ __launch_bounds__(256) void head_decay_chunk_kernel(RowArgs p, Made made) {
@@ -116,11 +147,6 @@ __global__ __launch_bounds__(256) void head_decay_chunk_kernel(RowArgs p, Made m
       within[i * CHUNK] = i >= i0 ? __builtin_amdgcn_exp2f((float)(sum_i - sum)) * qk_s[i * (CHUNK + 4) + i0] * dt : 0.f;
     }
   }
-}
-
-template <int CTRL>
-__device__ __forceinline__ float lane_moved(float v) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true));
 }
 
 // a decay per key channel: one block per (chunk, head).  Everything is a running product of decays down the chunk's
@@ -237,8 +263,7 @@ extern "C" int64_t mi_decay_scan_chunks_scratch(int mode, int num_tokens, int nu
   const int pad = mi_decay_scan_dim_pad(dim);
   if (num_tokens <= 0 || num_requests <= 0 || num_requests > 65535 || dim > 256 || pad < 64 || heads <= 0 || heads > 65535 || groups <= 0 || vdim <= 0) return 0;
   return chunk_count(num_tokens, num_requests) * ((int64_t)2 * made_shares(mode, heads, groups) * CHUNK * pad +
-                                                  (int64_t)heads * (CHUNK * CHUNK + (mode == PER_CHANNEL ? pad : 2 * CHUNK))) +
-         flag_count(num_requests, heads, vdim);
+                                                  (int64_t)heads * (CHUNK * CHUNK + (mode == PER_CHANNEL ? pad : 2 * CHUNK)));
 }
 
 // As mi_decay_scan for bfloat16, with `scratch` on 16 bytes; longest: tokens of the longest portion, 0: not known.
@@ -262,7 +287,6 @@ extern "C" int mi_decay_scan_chunks(int mode, const void* q, int64_t q_stride, i
   made.fade = made.within + chunks * heads * CHUNK * CHUNK;
   made.factor = made.fade + (mode == PER_CHANNEL ? chunks * heads * pad : 0);
   made.k = made.solve = nullptr;
-  int* again = reinterpret_cast<int*>(made.factor + (mode == PER_CHANNEL ? 0 : chunks * heads * 2 * CHUNK));
   made.shares = made_shares(mode, heads, groups);
   RowArgs a;
   a.q = (const bf16_t*)q, a.k = (const bf16_t*)k, a.gate = (const bf16_t*)gate;
@@ -292,11 +316,7 @@ extern "C" int mi_decay_scan_chunks(int mode, const void* q, int64_t q_stride, i
   p.made = made;
   p.v = (const bf16_t*)v, p.v_stride = v_stride, p.v_col = v_col, p.skip = skip;
   p.state = state, p.state_stride = state_stride, p.cu = cu, p.slots = slots, p.num_slots = num_slots;
-  p.out = out, p.again = again, p.heads = heads, p.vdim = vdim;
-  const int walked = mode == PER_CHANNEL ? launch_walk<PER_CHANNEL>(p, pad, num_tokens, num_requests, longest, stream)
-                                         : launch_walk<PER_HEAD>(p, pad, num_tokens, num_requests, longest, stream);
-  if (walked != MI_OK) return walked;
-  return mi_decay_scan_again(mode, q, q_stride, q_col, k, k_stride, k_col, v, v_stride, v_col, gate, gate_stride, gate_col, gate_bias, rate,
-                             skip, inv_tau, q_scale, state, state_stride, cu, slots, num_slots, out, again, num_requests, heads, groups, dim,
-                             vdim, stream);
+  p.out = out, p.heads = heads, p.vdim = vdim;
+  return mode == PER_CHANNEL ? launch_walk<PER_CHANNEL>(p, TokenRows<PER_CHANNEL>{a}, pad, num_tokens, num_requests, longest, stream)
+                             : launch_walk<PER_HEAD>(p, TokenRows<PER_HEAD>{a}, pad, num_tokens, num_requests, longest, stream);
 }

@@ -10,6 +10,31 @@ namespace {
 
 using namespace chunk_scan;
 
+// What walk_by_token reads.
+struct TokenRows {
+  const bf16_t *qkv, *proj;
+  int64_t qkv_stride, proj_stride;
+  int col_b, col_a, kv_heads, dim;
+  const float *a_log, *dt_bias;
+  template <int R>
+  __device__ __forceinline__ float operands(int t, int head, int heads, int at, float (&q)[R], float (&k)[R], float (&a)[R]) const {
+    const bf16_t *row = qkv + (int64_t)t * qkv_stride + head / (heads / kv_heads) * dim, *gates = proj + (int64_t)t * proj_stride + head;
+    float qq = 0.f, kk = 0.f;
+#pragma unroll
+    for (int i = 0; i < R; ++i) {
+      const int d = min(at + i, dim - 1);  // (without branches, past the last channel that one again)
+      const float qv = to_f32(row[d]), kv = to_f32(row[kv_heads * dim + d]);
+      q[i] = at + i < dim ? qv : 0.f, k[i] = at + i < dim ? kv : 0.f;
+      qq = fmaf(q[i], q[i], qq), kk = fmaf(k[i], k[i], kk);
+    }
+    const float q_inv = rsqrtf(sum_of_16(qq) + 1e-6f) * (1.0f / sqrtf((float)dim)), k_inv = rsqrtf(sum_of_16(kk) + 1e-6f);
+    const float z = to_f32(gates[col_a]) + dt_bias[head], decay = expf(-expf(a_log[head]) * (z > 20.f ? z : log1pf(expf(z))));
+#pragma unroll
+    for (int i = 0; i < R; ++i) q[i] *= q_inv, k[i] *= k_inv, a[i] = decay;
+    return 1.f / (1.f + expf(-to_f32(gates[col_b])));
+  }
+};
+
 // 256 threads: 8 of them bring one token's q and k rows in and make them unit vectors; then a wave makes a 16 x 16
 // tile of each product; then a wave takes a head at a time.  The sums of the decays' logarithms are carried in
 // 64-bit: a quotient is the exponential of a difference of two of them, and they grow with the chunk while it may
@@ -162,8 +187,7 @@ __global__ __launch_bounds__(256) void delta_chunk_kernel(const bf16_t* __restri
 extern "C" int64_t mi_gated_delta_chunks_scratch(int num_tokens, int num_requests, int heads, int kv_heads, int dim, int vdim) {
   if (num_tokens <= 0 || num_requests <= 0 || dim > 256 || vdim > 256 || vdim <= 0 || heads <= 0 || kv_heads <= 0 || kv_heads > 65535) return 0;
   const int pad = mi_gated_delta_rows(dim, vdim);
-  return chunk_count(num_tokens, num_requests) * ((int64_t)3 * kv_heads * CHUNK * pad + (int64_t)heads * (2 * CHUNK * CHUNK + 2 * CHUNK)) +
-         flag_count(num_requests, heads, vdim);
+  return chunk_count(num_tokens, num_requests) * ((int64_t)3 * kv_heads * CHUNK * pad + (int64_t)heads * (2 * CHUNK * CHUNK + 2 * CHUNK));
 }
 
 // As mi_gated_delta for bfloat16, with `scratch` on 16 bytes; longest: tokens of the longest portion, 0: not known.
@@ -185,7 +209,6 @@ extern "C" int mi_gated_delta_chunks(const void* qkv, int64_t qkv_stride, const 
   made.within = made.kt + rows, made.solve = made.within + chunks * heads * CHUNK * CHUNK;
   made.factor = made.solve + chunks * heads * CHUNK * CHUNK;
   made.fade = nullptr;
-  int* again = reinterpret_cast<int*>(made.factor + chunks * heads * 2 * CHUNK);
   made.shares = kv_heads;
   dim3 grid((unsigned)chunks, kv_heads);
 #define MI_DELTA_CHUNKS(DT)                                                                                              \
@@ -202,11 +225,9 @@ extern "C" int mi_gated_delta_chunks(const void* qkv, int64_t qkv_stride, const 
   p.v = (const bf16_t*)qkv, p.v_stride = qkv_stride, p.v_col = 2 * kv_heads * dim;
   p.skip = nullptr;
   p.state = state, p.state_stride = state_stride, p.cu = cu, p.slots = slots, p.num_slots = num_slots;
-  p.out = readout, p.again = again, p.heads = heads, p.vdim = vdim;
-  const int walked = launch_walk<DELTA>(p, dim_pad, num_tokens, num_requests, longest, stream);
+  p.out = readout, p.heads = heads, p.vdim = vdim;
+  const TokenRows rows_of = {(const bf16_t*)qkv, (const bf16_t*)proj, qkv_stride, proj_stride, col_b, col_a, kv_heads, dim, a_log, dt_bias};
+  const int walked = launch_walk<DELTA>(p, rows_of, dim_pad, num_tokens, num_requests, longest, stream);
   if (walked != MI_OK) return walked;
-  const int redone = mi_delta_again(qkv, qkv_stride, proj, proj_stride, col_b, col_a, a_log, dt_bias, state, state_stride, cu, slots, readout,
-                                    again, num_requests, heads, kv_heads, dim, vdim, num_slots, stream);
-  if (redone != MI_OK) return redone;
   return mi_delta_readout_norm(MI_BF16, readout, proj, proj_stride, col_g, norm_weight, out, out_stride, num_tokens, heads, vdim, eps, stream);
 }

@@ -496,21 +496,6 @@ __global__ __launch_bounds__(256) void gated_delta_kernel(
                                   heads, kv_heads, dim, vdim, num_slots, blockIdx.x / chunks, blockIdx.x % chunks, blockIdx.y);
 }
 
-// the same for columns that the chunks' walk has flagged
-template <int ROWS>
-__global__ __launch_bounds__(256) void gated_delta_again_kernel(
-    const bf16_t* __restrict__ qkv, int64_t qkv_stride, const bf16_t* __restrict__ proj, int64_t proj_stride, int col_b,
-    int col_a, const float* __restrict__ a_log, const float* __restrict__ dt_bias, float* __restrict__ state,
-    int64_t state_stride, const int* __restrict__ cu, const int* __restrict__ slots, float* __restrict__ readout,
-    const int* __restrict__ again, int requests, int heads, int kv_heads, int dim, int vdim, int chunks, int num_slots) {
-  mi_take_flagged(
-      (int64_t)requests * heads * chunks, [&](int64_t i) { return again[i] != 0; },
-      [&](int64_t i) {
-        gated_delta_columns<bf16_t, 16, ROWS>(qkv, qkv_stride, proj, proj_stride, col_b, col_a, a_log, dt_bias, state, state_stride, cu, slots,
-                                              readout, heads, kv_heads, dim, vdim, num_slots, i / chunks % heads, i % chunks, i / chunks / heads);
-      });
-}
-
 // The read-outs of a step, head by head: divided by their root mean square over the head's
 // columns, times a weight per column, times silu of the output gate's projection.  A wave a head.
 template <typename T>
@@ -789,25 +774,6 @@ int mi_gated_delta_check(int64_t qkv_stride, int64_t proj_stride, int col_b, int
              "gated_delta: the gates' columns lie outside a row of the projections");
   MI_REQUIRE(eps > 0.f, "gated_delta: eps must be positive, got %g", (double)eps);
   MI_REQUIRE(num_slots >= 1 && num_requests <= 65535, "gated_delta: bad slot or request count");
-  return MI_OK;
-}
-
-int mi_delta_again(const void* qkv, int64_t qkv_stride, const void* proj, int64_t proj_stride, int col_b, int col_a, const float* a_log,
-                   const float* dt_bias, float* state, int64_t state_stride, const int* cu, const int* slots, float* readout,
-                   const int* again, int num_requests, int heads, int kv_heads, int dim, int vdim, int num_slots, hipStream_t stream) {
-  int lanes = 0, rows = 0;
-  delta_layout(dim, vdim, &lanes, &rows);
-  const int chunks = ceil_div(vdim, 256 / lanes);  // (of 16 columns, as the flags)
-  const int grid = (int)min((int64_t)AGAIN_BLOCKS, (int64_t)num_requests * heads * chunks);
-#define MI_DELTA_AGAIN(ROWS)                                                                                                      \
-  gated_delta_again_kernel<ROWS><<<grid, 256, 0, stream>>>((const bf16_t*)qkv, qkv_stride, (const bf16_t*)proj, proj_stride, col_b, \
-                                                           col_a, a_log, dt_bias, state, state_stride, cu, slots, readout, again,  \
-                                                           num_requests, heads, kv_heads, dim, vdim, chunks, num_slots)
-  if (rows == 4) MI_DELTA_AGAIN(4);
-  else if (rows == 8) MI_DELTA_AGAIN(8);
-  else MI_DELTA_AGAIN(16);
-#undef MI_DELTA_AGAIN
-  MI_CHECK_LAUNCH("gated_delta (again)");
   return MI_OK;
 }
 

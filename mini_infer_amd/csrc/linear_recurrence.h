@@ -9,14 +9,6 @@ int mi_decay_scan_check(int dtype, int mode, int64_t q_stride, int q_col, int64_
                         int64_t gate_stride, int gate_col, const float* gate_bias, const float* rate, const float* state,
                         int64_t state_stride, int num_slots, int num_tokens, int num_requests, int heads, int groups, int dim, int vdim);
 
-// The token-by-token kernel over a step's bfloat16 rows, sizes checked, for the columns whose flag in `again` (one for 16 columns,
-// [requests][heads][ceil(vdim / 16)]) is set.
-int mi_decay_scan_again(int mode, const void* q, int64_t q_stride, int q_col, const void* k, int64_t k_stride, int k_col, const void* v,
-                        int64_t v_stride, int v_col, const void* gate, int64_t gate_stride, int gate_col, const float* gate_bias,
-                        const float* rate, const float* skip, float inv_tau, float q_scale, float* state, int64_t state_stride,
-                        const int* cu, const int* slots, int num_slots, float* out, const int* again, int num_requests, int heads,
-                        int groups, int dim, int vdim, hipStream_t stream);
-
 // log(1 + e) for 0 <= e <= 1 on the hardware's logarithm (one ulp), with the series where 1 + e
 // would round e away
 __device__ __forceinline__ float mi_log1p_small(float e) {

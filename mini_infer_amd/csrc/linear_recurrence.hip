@@ -49,7 +49,6 @@ struct ScanArgs {
   const int *cu, *slots;
   int num_slots;
   float* out;  // float32 [tokens, heads * vdim]
-  const int* again;  // null, or one flag for 16 columns [requests][heads][ceil(vdim / 16)]: the columns to be taken
   int heads, groups, dim, vdim;
   bool whole_runs;  // rows of q and k can be read a lane's run at a time
 };
@@ -198,7 +197,7 @@ __device__ __forceinline__ void decay_token(const ScanArgs& p, int64_t t, int sl
 // step sizes in LDS, and the walk reads LDS only, each token's operands one token ahead.  In LDS
 // a lane's run of R entries is followed by four unused ones where runs of 32 or 64 bytes would
 // otherwise meet 2 or 4 to a bank in a 16-byte read of all lanes.
-template <typename T, int MODE, int R, int L, bool AGAIN>
+template <typename T, int MODE, int R, int L>
 __device__ __forceinline__ void decay_scan_columns(const ScanArgs& p, int b, int head, int col0) {
   using A = typename Wide<T>::type;
   constexpr bool WIDE = sizeof(T) == 4;
@@ -218,11 +217,9 @@ __device__ __forceinline__ void decay_scan_columns(const ScanArgs& p, int b, int
   const int tid = threadIdx.x;
   const int grp = head / (p.heads / p.groups);
   const int part = tid % L, c = tid / L, col = col0 + c;
-  bool live = col < p.vdim;
+  const bool live = col < p.vdim;
   const int first = p.cu[b], last = p.cu[b + 1];
   if (last <= first) return;
-  // (of columns taken again the flagged ones: the others' states have been advanced)
-  if constexpr (AGAIN) live = live && p.again[((int64_t)b * p.heads + head) * ((p.vdim + 15) / 16) + min(col, p.vdim - 1) / 16] != 0;
   const int slot = p.slots[b];
   const bool kept = slot >= 0 && slot < p.num_slots;  // (see decay_token)
   float* mine = p.state + (int64_t)(kept ? slot : p.num_slots) * p.state_stride + ((int64_t)head * p.vdim + (live ? col : 0)) * DP + part * R;
@@ -393,23 +390,7 @@ __global__ __launch_bounds__(256) void decay_scan_kernel(ScanArgs p, int request
       return;
     }
   }
-  decay_scan_columns<T, MODE, R, L, false>(p, b, head, col_block * COLS);
-}
-
-// the same for columns that the chunks' walk has flagged
-template <int MODE, int R, int L>
-__global__ __launch_bounds__(256) void decay_scan_again_kernel(ScanArgs p, int requests) {
-  constexpr int COLS = 256 / L;
-  const int flags = (p.vdim + 15) / 16, blocks = (p.vdim + COLS - 1) / COLS;
-  mi_take_flagged(
-      (int64_t)requests * p.heads * blocks,
-      [&](int64_t i) {
-        const int* of = p.again + i / blocks * flags;
-        bool any = false;
-        for (int f = i % blocks * (COLS / 16); f < min((int)(i % blocks + 1) * (COLS / 16), flags); ++f) any = any || of[f] != 0;
-        return any;
-      },
-      [&](int64_t i) { decay_scan_columns<bf16_t, MODE, R, L, true>(p, i / blocks / p.heads, i / blocks % p.heads, i % blocks * COLS); });
+  decay_scan_columns<T, MODE, R, L>(p, b, head, col_block * COLS);
 }
 
 // rows per lane and lanes per column for a head whose keys are `dim` wide
@@ -448,21 +429,6 @@ int launch_scan(ScanArgs p, int tokens, int requests, hipStream_t stream) {
   else MI_SCAN(16, 16);
 #undef MI_SCAN
   MI_CHECK_LAUNCH("decay_scan");
-  return MI_OK;
-}
-
-// (chunks take keys of 33 columns and more)
-template <int MODE>
-int launch_scan_again(const ScanArgs& p, int requests, hipStream_t stream) {
-  int rows, lanes;
-  scan_shape(p.dim, &rows, &lanes);
-  const int grid = (int)min((int64_t)AGAIN_BLOCKS, (int64_t)requests * p.heads * ceil_div(p.vdim, 256 / lanes));
-#define MI_SCAN(RR, LL) decay_scan_again_kernel<MODE, RR, LL><<<grid, 256, 0, stream>>>(p, requests)
-  if (lanes == 8) MI_SCAN(8, 8);
-  else if (rows == 8) MI_SCAN(8, 16);
-  else MI_SCAN(16, 16);
-#undef MI_SCAN
-  MI_CHECK_LAUNCH("decay_scan (again)");
   return MI_OK;
 }
 
@@ -595,27 +561,12 @@ extern "C" int mi_decay_scan(int dtype, int mode, const void* q, int64_t q_strid
   p.q_stride = q_stride, p.k_stride = k_stride, p.v_stride = v_stride, p.gate_stride = gate_stride;
   p.q_col = q_col, p.k_col = k_col, p.v_col = v_col, p.gate_col = gate_col;
   p.gate_bias = gate_bias, p.rate = rate, p.skip = skip, p.inv_tau = inv_tau, p.q_scale = q_scale;
-  p.state = state, p.state_stride = state_stride, p.cu = cu, p.slots = slots, p.num_slots = num_slots, p.out = out, p.again = nullptr;
+  p.state = state, p.state_stride = state_stride, p.cu = cu, p.slots = slots, p.num_slots = num_slots, p.out = out;
   p.heads = heads, p.groups = groups, p.dim = dim, p.vdim = vdim, p.whole_runs = false;
   if (dtype == MI_F32) return mode == 0 ? launch_scan<float, DECAY_PER_CHANNEL>(p, num_tokens, num_requests, stream)
                                         : launch_scan<float, DECAY_PER_HEAD>(p, num_tokens, num_requests, stream);
   return mode == 0 ? launch_scan<bf16_t, DECAY_PER_CHANNEL>(p, num_tokens, num_requests, stream)
                    : launch_scan<bf16_t, DECAY_PER_HEAD>(p, num_tokens, num_requests, stream);
-}
-
-int mi_decay_scan_again(int mode, const void* q, int64_t q_stride, int q_col, const void* k, int64_t k_stride, int k_col, const void* v,
-                        int64_t v_stride, int v_col, const void* gate, int64_t gate_stride, int gate_col, const float* gate_bias,
-                        const float* rate, const float* skip, float inv_tau, float q_scale, float* state, int64_t state_stride,
-                        const int* cu, const int* slots, int num_slots, float* out, const int* again, int num_requests, int heads,
-                        int groups, int dim, int vdim, hipStream_t stream) {
-  ScanArgs p;
-  p.q = q, p.k = k, p.v = v, p.gate = gate;
-  p.q_stride = q_stride, p.k_stride = k_stride, p.v_stride = v_stride, p.gate_stride = gate_stride;
-  p.q_col = q_col, p.k_col = k_col, p.v_col = v_col, p.gate_col = gate_col;
-  p.gate_bias = gate_bias, p.rate = rate, p.skip = skip, p.inv_tau = inv_tau, p.q_scale = q_scale;
-  p.state = state, p.state_stride = state_stride, p.cu = cu, p.slots = slots, p.num_slots = num_slots, p.out = out, p.again = again;
-  p.heads = heads, p.groups = groups, p.dim = dim, p.vdim = vdim, p.whole_runs = false;
-  return mode == 0 ? launch_scan_again<DECAY_PER_CHANNEL>(p, num_requests, stream) : launch_scan_again<DECAY_PER_HEAD>(p, num_requests, stream);
 }
 
 // o float32 [tokens, width]; gate [tokens, >= width] in the element type (row stride, from its first column);
