@@ -45,6 +45,14 @@ struct PairedHow<2> {
   using type = RotaryWrite;
 };
 
+// Where rows of W are a multiple of 4 KB apart, blocks that walk K in step all ask the same memory channels; gated products and the output head then begin
+// a step later from tile to tile, and go round.  Microseconds, from the beginning / so: gate|up 16384 x 2048 at 33 / 48 / 96 / 192 rows 16.5, 16.6, 19.3, 25.1 / 14.1, 14.1,
+// 18.8, 24.5, 28672 x 4096 48.1, 48.8, 52.5, 64.9 / 43.4, 44.7, 48.9, 63.5; 128256 x 2048 at 17 / 32 / 64 / 128 102, 109, 125, 135 / 90, 96, 107, 107, x 4096
+// 176, 182, 202, 219 / 173, 178, 196, 218, 64128 x 6144 145, 154, 169, 174 / 125, 131, 145, 146.  (Of 16384 x 3072, 28672 x 5120 and 128256 x 1024 the same or 3 % more; five
+// or eight steps later for one: 128256 x 4096 189 and 176.  Ranges of K, which begin apart: the same.  Plain whole products and those with a rotation give the
+// same bits as one another, which have their rows of W in other tiles: from the beginning.)
+__device__ __forceinline__ bool turned(int kind, int64_t ldw) { return kind >= 2 && ldw % 2048 == 0; }
+
 // (the second bound: two blocks a CU where LDS holds two)
 template <class T, int PAIRED, bool ONCE, bool ODD>
 __global__ __launch_bounds__(T::THREADS, T::RING * 4 <= 163840 ? 2 : 1) void gemm_tiles_kernel(
@@ -69,7 +77,8 @@ __global__ __launch_bounds__(T::THREADS, T::RING * 4 <= 163840 ? 2 : 1) void gem
       [&](int r) {
         if constexpr (PAIRED == PAIRED_ROTARY) return w + (int64_t)rotary_row_of(GatedTile<T::NT>::row_of(r, f0, n), n, how.head_dim) * ldw;
         else return w + (int64_t)(PAIRED == PAIRED_GATED ? GatedTile<T::NT>::row_of(r, f0, n) : min(f0 + r, n - 1)) * ldw;
-      });
+      },
+      !ODD && PAIRED != PAIRED_ROTARY && turned(kind, ldw) ? feature_tile % (part.halves / 2) : 0);
   if constexpr (PAIRED == PAIRED_ROTARY) {
     tile.leave(ring);
     write_rotated<GatedTile<T::NT>, T::BM, T::BN, T::MADE, T::THREADS>(ring, how, r0, m, f0, n);

@@ -286,6 +286,27 @@ def test_products_in_tiles(shape):
                 assert torch.equal(made(5, a, w, n, torch.bfloat16, spare=spare)[finite], ops.gated_mul(out[:, :n], out[:, n:], "gelu_tanh")[finite])
 
 
+@pytest.mark.parametrize("shape", [0, 1, 3, 6, 9, 11, 13])
+@pytest.mark.parametrize("k", [64, 192, 480, 2048])
+def test_tiles_that_begin_a_step_later_than_their_neighbours(shape, k):
+    """An output head and gated products whose rows of W are 4 KB apart: more tiles than steps of K, K of one step and, which begins like the others, of odd 32s."""
+    from mini_infer_amd.ops import kernels
+
+    bm, bn = kernels.tile_size(shape)
+    m, n = bm + 3, bn * (35 if bn <= 64 else 5)
+    a, w = _rand(m, k, dtype=torch.bfloat16, seed=71), _rand(2 * n, 2048, dtype=torch.bfloat16, seed=72, scale=0.05)[:, :k]
+    exact = a.double() @ w.double().T
+    # (as test_products_in_tiles: sums of k terms, one rounding to 8 bits; in the activation half a unit of each factor and of the result)
+    summed = 2.0 ** -23 * (k + 1) * (a.double().abs() @ w.double().abs().T) + 1e-30
+    logits = kernels._tiles(2, a, w, torch.empty(m, 2 * n, device=DEV), 2 * n, shape, 1, 0.25)
+    assert ((logits.double() * 4 - exact).abs() <= summed + 2.0 ** -8 * exact.abs()).all()
+    gated = kernels._tiles(3, a, w, torch.empty(m, n, dtype=torch.bfloat16, device=DEV), n, shape, 1).double()
+    g, u = exact[:, :n], exact[:, n:]
+    off_g, off_u = (e + 2.0 ** -8 * x.abs() for e, x in ((summed[:, :n], g), (summed[:, n:], u)))
+    wanted = torch.nn.functional.silu(g) * u  # (|silu'| <= 1.1, |silu(g)| <= |g|)
+    assert ((gated - wanted).abs() <= 1.1 * off_g * (u.abs() + off_u) + g.abs() * off_u + 2.0 ** -8 * wanted.abs() + 1e-6).all()
+
+
 def test_every_form_of_the_tiles_that_take_turns_is_tested():
     from mini_infer_amd.ops import library
 
