@@ -30,7 +30,7 @@
 
 #include <mutex>
 
-#define GT 4  // query heads handled together by one wave
+constexpr int HEADS_TOGETHER = 4;  // query heads of a wave (GT)
 
 template <typename T, int N>
 struct alignas(sizeof(T) * N) Pack {
@@ -72,7 +72,7 @@ __device__ __forceinline__ float from_lane(float v, int lane) {
 // measured at attn_generic_launch.
 // DEEP (several waves, rows in whole 16s): 32 value rows are asked for at once instead of 8, the first of them with the first
 // values of the key rows, before the scores; measured at attn_generic_launch.
-template <typename T, int VPL, bool VEC, int WAVES, bool DEEP = false>
+template <typename T, int VPL, bool VEC, int WAVES, bool DEEP = false, int GT = HEADS_TOGETHER>
 __global__ __launch_bounds__(64 * WAVES) void attn_generic_kernel(
     const T* __restrict__ q, int64_t q_row_stride, const T* __restrict__ k_pages,
     const T* __restrict__ v_pages, const int* __restrict__ block_table, int max_blocks,
@@ -461,6 +461,7 @@ static int attn_generic_launch(const void* q, int64_t q_row_stride, const void* 
   if (v_dim <= 0) v_dim = head_dim;
   if (v_row_stride <= 0) v_row_stride = v_dim;
   const int group = q_heads / kv_heads;
+  constexpr int GT = HEADS_TOGETHER;
   dim3 grid(num_tokens, kv_heads * ceil_div(group, GT), num_splits);
   using S = typename SumType<T>::type;
   const size_t lds = sizeof(S) * GT * head_dim;
@@ -487,8 +488,15 @@ static int attn_generic_launch(const void* q, int64_t q_row_stride, const void* 
   if (mask_chunk > 0) keys = keys < mask_chunk ? keys : mask_chunk;
   keys = ceil_div64(keys, num_splits);
   const bool four = sizeof(S) == 8 && v_dim <= 256 && blocks < 2048 && keys > MI_WAVE * ceil_div64(blocks, 768);
-#define MI_ATTN_LAUNCH_WAVES(VPL, VEC, WAVES, DEEP, LDS)                                          \
-  attn_generic_kernel<T, VPL, VEC, WAVES, DEEP><<<grid, WAVES * MI_WAVE, LDS, stream>>>(                \
+  // One head a block instead of four where that is at most two blocks a CU, the 32-bit path: four heads are four times the work on the way through a wave's
+  // keys, and the CUs are idle (the same bits; keys and values are read by as many blocks as there are heads, from L2).  Microseconds, four heads / one: 32 heads of
+  // 64 over 8, 1 / 3 / 6 tokens of 100 positions 14.5 / 10.5, of 600 28.3 / 20.6, 22.2, 26.8, 1 of 2,000 29.6 / 23.5 (3: 768 blocks, 30.5 / 35.1), 12 of 100 14.6 / 12.1;
+  // 24 heads of 128 over 8, 3 of 600 35.9 / 29.8; latent rows of 288, 32 heads, 3 of 100 / 600 32.2 / 19.4, 62.6 / 41.7.
+  // Values of up to 64 dims in one or two ranges up to four blocks a CU: 32 of 100 (1,024 blocks) 14.7 / 13.1, 12 of 300 (768) 24.4 / 20.8; 48 of 100 17.4 / 22.2.
+  const bool one = sizeof(S) == 8 && v_dim <= 256 && group > 1 &&
+                   (int64_t)num_tokens * q_heads * num_splits <= (v_dim <= 64 && num_splits <= 2 ? 1024 : 512);
+#define MI_ATTN_LAUNCH_WAVES(VPL, VEC, WAVES, DEEP, LDS, ...)                                     \
+  attn_generic_kernel<T, VPL, VEC, WAVES, DEEP, ##__VA_ARGS__><<<grid, WAVES * MI_WAVE, LDS, stream>>>( \
       (const T*)q, q_row_stride, (const T*)k_pages, (const T*)v_pages, block_table, max_blocks,   \
       token_request, positions, (T*)out, out_row_stride, part_acc, part_ml, q_heads, kv_heads,    \
       head_dim, page_size, scale, window, num_splits, slopes, v_dim, v_row_stride, has_sink, sink_logit, mask_chunk, \
@@ -496,6 +504,12 @@ static int attn_generic_launch(const void* q, int64_t q_row_stride, const void* 
 #define MI_ATTN_LAUNCH(VPL, VEC)                                                                  \
   do {                                                                                            \
     if constexpr (sizeof(S) == 8 && VPL <= 4) {                                                   \
+      const size_t a_head = sizeof(S) * head_dim + 3 * (VPL + 1) * MI_WAVE * sizeof(S) + 4 * sizeof(float); \
+      if (one) {                                                                                  \
+        grid.y = q_heads;                                                                         \
+        MI_ATTN_LAUNCH_WAVES(VPL, VEC, 4, (VEC && VPL <= 2), a_head, 1);                          \
+        break;                                                                                    \
+      }                                                                                           \
       const size_t merge = 3 * GT * (VPL + 1) * MI_WAVE * sizeof(S) + 4 * GT * sizeof(float);     \
       if (four && lds + merge <= 64 * 1024) {                                                     \
         if (VEC && VPL <= 2 && blocks <= (VPL == 1 ? 512 : 768)) MI_ATTN_LAUNCH_WAVES(VPL, VEC, 4, (VEC && VPL <= 2), lds + merge); \
@@ -541,7 +555,7 @@ static int attn_generic_check(int dtype, int64_t q_row_stride, int max_blocks, i
   MI_REQUIRE(num_splits >= 1 && num_splits <= 64, "attn_generic: num_splits=%d must be 1..64", num_splits);
   MI_REQUIRE(q_row_stride >= (int64_t)q_heads * head_dim && out_row_stride >= (int64_t)q_heads * v_dim,
              "attn_generic: row strides shorter than q_heads*head_dim");
-  MI_REQUIRE(kv_heads * ceil_div(q_heads / kv_heads, GT) <= 65535, "attn_generic: too many heads");
+  MI_REQUIRE(kv_heads * ceil_div(q_heads / kv_heads, HEADS_TOGETHER) <= 65535, "attn_generic: too many heads");
   MI_REQUIRE(dtype == MI_F32 || dtype == MI_BF16, "attn_generic: unknown dtype %d", dtype);
   return MI_OK;
 }

@@ -1960,6 +1960,45 @@ def test_float32_products_of_all_heads_are_those_of_each(tokens, heads, k, n):
     assert (out[:, :, n:] == 0).all()
 
 
+@pytest.mark.parametrize("heads, kv_heads, head_dim, v_dim", [(8, 2, 64, 64), (6, 2, 128, 128), (20, 2, 22, 30), (16, 1, 288, 256)])
+@pytest.mark.parametrize("context", [5, 64, 101, 700])
+def test_float32_attention_a_head_a_block_gives_the_bits_of_four(heads, kv_heads, head_dim, v_dim, context):
+    """A token by itself (a block for each head) as one of many (four heads a block), with groups of fewer than four heads and ones that are not whole fours; the
+    keys in ranges and not."""
+    from mini_infer_amd.ops import kernels
+
+    page, many = 16, 1024 // heads + 1
+    pages = -(-context // page)
+    k_pages = _rand(pages + 2, kv_heads, page, head_dim, seed=81)
+    v_pages = _rand(pages + 2, kv_heads, page, v_dim, seed=82)
+    table = torch.randperm(pages, generator=torch.Generator().manual_seed(83)).to(torch.int32).to(DEV)[None]
+    q = _rand(many, heads * head_dim, seed=84)
+
+    def attended(rows, splits):
+        n = rows.shape[0]
+        out = torch.empty(n, heads * v_dim, device=DEV)
+        names = dict(q_heads=heads, kv_heads=kv_heads, head_dim=head_dim, v_head_dim=v_dim, scale=head_dim ** -0.5, window=None, max_seq_len=context,
+                     v_transposed=False, slopes=None, sink_logit=None, out=out)
+        own = kernels.attention_splits
+        kernels.attention_splits = lambda *a: splits
+        try:
+            return kernels._paged_attention_general(rows, k_pages, v_pages, table, torch.zeros(n, dtype=torch.int32, device=DEV),
+                                                    torch.full((n,), context - 1, dtype=torch.int32, device=DEV), **names)
+        finally:
+            kernels.attention_splits = own
+
+    for splits in (1, 3):
+        together = attended(q, splits)
+        for row in (0, many - 1):
+            assert torch.equal(attended(q[row : row + 1], splits)[0], together[row]), (splits, row)
+        if splits == 1:
+            keys, values = (x[table[0].long()].transpose(1, 2).reshape(pages * page, kv_heads, -1)[:context].double() for x in (k_pages, v_pages))
+            scores = torch.einsum("hd,chd->hc", q[0].view(heads, head_dim).double(), keys.repeat_interleave(heads // kv_heads, 1)) * head_dim ** -0.5
+            exact = torch.einsum("hc,chd->hd", scores.softmax(1), values.repeat_interleave(heads // kv_heads, 1)).flatten()
+            # (weights and result rounded to float32 once each)
+            assert (together[0].double() - exact).norm() < 3e-7 * exact.norm()
+
+
 @pytest.mark.parametrize("head_dim, v_dim", [(288, 256), (200, 144), (256, 250), (130, 130), (96, 64)])
 @pytest.mark.parametrize("contexts", [[1, 64, 65], [300, 7, 129, 256, 257], [700]])
 @pytest.mark.parametrize("window", [None, 100])
