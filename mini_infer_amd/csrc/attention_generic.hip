@@ -492,9 +492,8 @@ static int attn_generic_launch(const void* q, int64_t q_row_stride, const void* 
   // keys, and the CUs are idle (the same bits; keys and values are read by as many blocks as there are heads, from L2).  Microseconds, four heads / one: 32 heads of
   // 64 over 8, 1 / 3 / 6 tokens of 100 positions 14.5 / 10.5, of 600 28.3 / 20.6, 22.2, 26.8, 1 of 2,000 29.6 / 23.5 (3: 768 blocks, 30.5 / 35.1), 12 of 100 14.6 / 12.1;
   // 24 heads of 128 over 8, 3 of 600 35.9 / 29.8; latent rows of 288, 32 heads, 3 of 100 / 600 32.2 / 19.4, 62.6 / 41.7.
-  // Values of up to 64 dims in one or two ranges up to four blocks a CU: 32 of 100 (1,024 blocks) 14.7 / 13.1, 12 of 300 (768) 24.4 / 20.8; 48 of 100 17.4 / 22.2.
-  const bool one = sizeof(S) == 8 && v_dim <= 256 && group > 1 &&
-                   (int64_t)num_tokens * q_heads * num_splits <= (v_dim <= 64 && num_splits <= 2 ? 1024 : 512);
+  // (Up to four blocks a CU, values of up to 64 dims in one or two ranges: 32 tokens of 100 positions 14.7 / 13.1, but a step of 28 new ones beside one of 73 2,275 / 2,287.)
+  const bool one = sizeof(S) == 8 && v_dim <= 256 && group > 1 && (int64_t)num_tokens * q_heads * num_splits <= 512;
 #define MI_ATTN_LAUNCH_WAVES(VPL, VEC, WAVES, DEEP, LDS, ...)                                     \
   attn_generic_kernel<T, VPL, VEC, WAVES, DEEP, ##__VA_ARGS__><<<grid, WAVES * MI_WAVE, LDS, stream>>>( \
       (const T*)q, q_row_stride, (const T*)k_pages, (const T*)v_pages, block_table, max_blocks,   \

@@ -1967,7 +1967,7 @@ def test_float32_attention_a_head_a_block_gives_the_bits_of_four(heads, kv_heads
     keys in ranges and not."""
     from mini_infer_amd.ops import kernels
 
-    page, many = 16, 1024 // heads + 1
+    page, many = 16, 512 // heads + 1
     pages = -(-context // page)
     k_pages = _rand(pages + 2, kv_heads, page, head_dim, seed=81)
     v_pages = _rand(pages + 2, kv_heads, page, v_dim, seed=82)
