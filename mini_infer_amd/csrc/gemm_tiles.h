@@ -51,10 +51,10 @@ struct PairedHow<2> {
 // 176, 182, 202, 219 / 173, 178, 196, 218, 64128 x 6144 145, 154, 169, 174 / 125, 131, 145, 146.  (Of 16384 x 3072, 28672 x 5120 and 128256 x 1024 the same or 3 % more; five
 // or eight steps later for one: 128256 x 4096 189 and 176.  Ranges of K, which begin apart: the same.  Plain whole products and those with a rotation give the
 // same bits as one another, which have their rows of W in other tiles: from the beginning.)
-__device__ __forceinline__ bool turned(int kind, int64_t ldw) { return kind >= 2 && ldw % 2048 == 0; }
+static bool turned(int kind, int64_t ldw) { return kind >= 2 && ldw % 2048 == 0; }
 
 // (the second bound: two blocks a CU where LDS holds two)
-template <class T, int PAIRED, bool ONCE, bool ODD>
+template <class T, int PAIRED, bool ONCE, bool ODD, bool ROUND>
 __global__ __launch_bounds__(T::THREADS, T::RING * 4 <= 163840 ? 2 : 1) void gemm_tiles_kernel(
     const bf16_t* __restrict__ a, int64_t lda, const bf16_t* __restrict__ w, int64_t ldw, void* __restrict__ out, int64_t ldc,
     int kind, float scale, const typename PairedHow<PAIRED>::type how, bool vec, int m, int n, int k, int steps_each, int row_tiles, int feature_tiles,
@@ -72,13 +72,13 @@ __global__ __launch_bounds__(T::THREADS, T::RING * 4 <= 163840 ? 2 : 1) void gem
   a += part.first * 32;
   w += part.first * 32;
   T tile;
-  tile.template run<ONCE, ODD>(
+  tile.template run<ONCE, ODD, ROUND>(
       ring, part.halves, [&](int r) { return a + (int64_t)min(r0 + r, m - 1) * lda; },
       [&](int r) {
         if constexpr (PAIRED == PAIRED_ROTARY) return w + (int64_t)rotary_row_of(GatedTile<T::NT>::row_of(r, f0, n), n, how.head_dim) * ldw;
         else return w + (int64_t)(PAIRED == PAIRED_GATED ? GatedTile<T::NT>::row_of(r, f0, n) : min(f0 + r, n - 1)) * ldw;
       },
-      !ODD && PAIRED != PAIRED_ROTARY && turned(kind, ldw) ? feature_tile % (part.halves / 2) : 0);
+      ROUND ? feature_tile % (part.halves / 2) : 0);
   if constexpr (PAIRED == PAIRED_ROTARY) {
     tile.leave(ring);
     write_rotated<GatedTile<T::NT>, T::BM, T::BN, T::MADE, T::THREADS>(ring, how, r0, m, f0, n);
@@ -143,7 +143,10 @@ template <class T, int PAIRED, bool ODD>
 static void gemm_tiles_launch(const GemmTilesLaunch& l) {
   const int row_tiles = ceil_div(l.m, T::BM), feature_tiles = ceil_div(l.n, PAIRED != PAIRED_NOT ? T::BN / 2 : T::BN);
   const int total = row_tiles * feature_tiles * ceil_div(ceil_div(l.k, 64), l.steps_each);
-  const auto kernel = row_tiles == 1 ? gemm_tiles_kernel<T, PAIRED, true, ODD> : gemm_tiles_kernel<T, PAIRED, false, ODD>;
+  auto kernel = row_tiles == 1 ? gemm_tiles_kernel<T, PAIRED, true, ODD, false> : gemm_tiles_kernel<T, PAIRED, false, ODD, false>;
+  if constexpr (!ODD && PAIRED != PAIRED_ROTARY) {
+    if (turned(l.kind, l.ldw)) kernel = row_tiles == 1 ? gemm_tiles_kernel<T, PAIRED, true, false, true> : gemm_tiles_kernel<T, PAIRED, false, false, true>;
+  }
   const auto& how = [&]() -> const auto& {
     if constexpr (PAIRED == PAIRED_ROTARY) return l.rotary;
     else return l.how;

@@ -74,10 +74,10 @@ struct TileProduct {
 
   // acc = the tile's sums over `halves` pieces of 32 of K (at least one); a_row(r) and w_row(r) give the first of them of the tile's
   // row r, 0 <= r < BM, BN, on 16 bytes and readable.  ONCE: nobody else reads these rows of W (they are then read past the
-  // caches: 4 % at 64 rows; not where several row tiles share them).  ODD: `halves` may be odd.  begin: the step (of 64) that comes first, after the last
-  // one step 0 follows; 0 with ODD.  (Both known when
-  // compiling: a branch in the loop for either cost 5 to 20 %.)
-  template <bool ONCE, bool ODD, typename RowA, typename RowW>
+  // caches: 4 % at 64 rows; not where several row tiles share them).  ODD: `halves` may be odd.  ROUND: begin at the step (of 64) `begin`, after the last
+  // one step 0 follows; not with ODD.  (All known when
+  // compiling: a branch in the loop for either of the first two cost 5 to 20 %, going round 1 % of a step of 271 tokens at 3072 wide that does not.)
+  template <bool ONCE, bool ODD, bool ROUND = false, typename RowA, typename RowW>
   __device__ __forceinline__ void run(bf16_t* ring, int halves, RowA a_row, RowW w_row, int begin = 0) {
     const int steps = ODD ? (halves + 1) / 2 : halves / 2;
     const bf16_t* src[MOST];
@@ -92,8 +92,10 @@ struct TileProduct {
       else src[j] = nullptr;  // (not fetched)
     }
     int fetched = 0, left = steps - begin;
+    if constexpr (ROUND) {
 #pragma unroll
-    for (int j = 0; j < MOST; ++j) src[j] += begin * STEP_K;
+      for (int j = 0; j < MOST; ++j) src[j] += begin * STEP_K;
+    }
     auto fetch = [&](int slot) {
       if (ODD && ++fetched == steps && halves % 2 != 0) {  // the last 32 of K have no other half: the first one again, not multiplied
 #pragma unroll
@@ -101,7 +103,7 @@ struct TileProduct {
           if (((lane % 8) ^ ((wave + j * WAVES) * 8 + row_of) % 8) >= 4) src[j] -= STEP_K / 2;
       }
       bf16_t* to = ring + slot * STAGE + wave * 512;
-      const int add = --left == 0 ? STEP_K - steps * STEP_K : STEP_K;
+      const int add = ROUND && --left == 0 ? STEP_K - steps * STEP_K : STEP_K;
 #pragma unroll
       for (int j = 0; j < MOST; ++j) {
         if (j < EACH || wave < REST) {
