@@ -54,7 +54,7 @@ struct PairedHow<2> {
 static bool turned(int kind, int64_t ldw) { return kind >= 2 && ldw % 2048 == 0; }
 
 // (the second bound: two blocks a CU where LDS holds two)
-template <class T, int PAIRED, bool ONCE, bool ODD, bool ROUND>
+template <class T, int PAIRED, bool ONCE, bool ODD, bool ROUND, bool EIGHTHS = false>
 __global__ __launch_bounds__(T::THREADS, T::RING * 4 <= 163840 ? 2 : 1) void gemm_tiles_kernel(
     const bf16_t* __restrict__ a, int64_t lda, const bf16_t* __restrict__ w, int64_t ldw, void* __restrict__ out, int64_t ldc,
     int kind, float scale, const typename PairedHow<PAIRED>::type how, bool vec, int m, int n, int k, int steps_each, int row_tiles, int feature_tiles,
@@ -72,13 +72,13 @@ __global__ __launch_bounds__(T::THREADS, T::RING * 4 <= 163840 ? 2 : 1) void gem
   a += part.first * 32;
   w += part.first * 32;
   T tile;
-  tile.template run<ONCE, ODD, ROUND>(
-      ring, part.halves, [&](int r) { return a + (int64_t)min(r0 + r, m - 1) * lda; },
-      [&](int r) {
-        if constexpr (PAIRED == PAIRED_ROTARY) return w + (int64_t)rotary_row_of(GatedTile<T::NT>::row_of(r, f0, n), n, how.head_dim) * ldw;
-        else return w + (int64_t)(PAIRED == PAIRED_GATED ? GatedTile<T::NT>::row_of(r, f0, n) : min(f0 + r, n - 1)) * ldw;
-      },
-      ROUND ? feature_tile % (part.halves / 2) : 0);
+  const auto a_row = [&](int r) { return a + (int64_t)min(r0 + r, m - 1) * lda; };
+  const auto w_row = [&](int r) {
+    if constexpr (PAIRED == PAIRED_ROTARY) return w + (int64_t)rotary_row_of(GatedTile<T::NT>::row_of(r, f0, n), n, how.head_dim) * ldw;
+    else return w + (int64_t)(PAIRED == PAIRED_GATED ? GatedTile<T::NT>::row_of(r, f0, n) : min(f0 + r, n - 1)) * ldw;
+  };
+  if constexpr (EIGHTHS) tile.template run_eighths<ROUND>(ring, part.halves, a_row, w_row, feature_tile % 4);
+  else tile.template run<ONCE, ODD, ROUND>(ring, part.halves, a_row, w_row, ROUND ? feature_tile % (part.halves / 2) : 0);
   if constexpr (PAIRED == PAIRED_ROTARY) {
     tile.leave(ring);
     write_rotated<GatedTile<T::NT>, T::BM, T::BN, T::MADE, T::THREADS>(ring, how, r0, m, f0, n);
@@ -139,13 +139,21 @@ struct GemmTilesLaunch {
   hipStream_t stream;
 };
 
-template <class T, int PAIRED, bool ODD>
+template <class T, int PAIRED, bool ODD, bool EIGHTHS = false>
 static void gemm_tiles_launch(const GemmTilesLaunch& l) {
   const int row_tiles = ceil_div(l.m, T::BM), feature_tiles = ceil_div(l.n, PAIRED != PAIRED_NOT ? T::BN / 2 : T::BN);
   const int total = row_tiles * feature_tiles * ceil_div(ceil_div(l.k, 64), l.steps_each);
-  auto kernel = row_tiles == 1 ? gemm_tiles_kernel<T, PAIRED, true, ODD, false> : gemm_tiles_kernel<T, PAIRED, false, ODD, false>;
+  auto kernel = gemm_tiles_kernel<T, PAIRED, true, ODD, false, EIGHTHS>;
+  if constexpr (!EIGHTHS) {  // (of eighths: one row tile)
+    if (row_tiles > 1) kernel = gemm_tiles_kernel<T, PAIRED, false, ODD, false>;
+  }
   if constexpr (!ODD && PAIRED != PAIRED_ROTARY) {
-    if (turned(l.kind, l.ldw)) kernel = row_tiles == 1 ? gemm_tiles_kernel<T, PAIRED, true, false, true> : gemm_tiles_kernel<T, PAIRED, false, false, true>;
+    if (turned(l.kind, l.ldw)) {
+      kernel = gemm_tiles_kernel<T, PAIRED, true, false, true, EIGHTHS>;
+      if constexpr (!EIGHTHS) {
+        if (row_tiles > 1) kernel = gemm_tiles_kernel<T, PAIRED, false, false, true>;
+      }
+    }
   }
   const auto& how = [&]() -> const auto& {
     if constexpr (PAIRED == PAIRED_ROTARY) return l.rotary;
@@ -157,3 +165,4 @@ static void gemm_tiles_launch(const GemmTilesLaunch& l) {
 
 // gemm_tiles_gated_bf16.hip
 void gemm_tiles_gated_launch(int shape, bool odd, const GemmTilesLaunch& l);
+void gemm_tiles_eighths_launch(int features, const GemmTilesLaunch& l);

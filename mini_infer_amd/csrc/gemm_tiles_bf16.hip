@@ -100,22 +100,26 @@ extern "C" int mi_gemm_tiles_take(int m, int n, int k, int64_t lda, int64_t ldw)
              : 0;
 }
 
-// kind, out: as at the top; n: features written (kinds 3 to 5: W has 2 n rows).  part of kind 1: [ranges][m][n], contiguous.
+// kind, out: as at the top; n: features written (kinds 3 to 5: W has 2 n rows; 8 ranges of these: shapes 0 and 1, whole, the sums of K's eighths added
+// in order).  part of kind 1: [ranges][m][n], contiguous.
 extern "C" int mi_gemm_tiles_bf16(int kind, const void* a, int64_t lda, const void* w, int64_t ldw, void* out, int64_t ldc, float scale,
                                   const float* bias, float limit, float slope, int m, int n, int k, int shape, int ranges, hipStream_t stream) {
   MI_REQUIRE(mi_gemm_tiles_take(m, n, k, lda, ldw) && ((uintptr_t)a | (uintptr_t)w) % 16 == 0,
              "gemm_tiles_bf16: takes K a multiple of 32 and rows on 16 bytes; got m=%d n=%d k=%d lda=%lld ldw=%lld", m, n, k, (long long)lda,
              (long long)ldw);
-  MI_REQUIRE(kind >= 0 && kind <= 5 && (kind != 4 || limit > 0.f) && shape >= 0 && shape < SHAPE_COUNT && ranges >= 1 && ranges <= MOST_RANGES && (kind == 1 || ranges == 1) &&
+  const bool eighths = kind >= 3 && ranges == 8;
+  MI_REQUIRE(!eighths || (m <= 32 && k % 512 == 0 && shape >= 0 && shape <= 1), "gemm_tiles_bf16: eighths of K of m=%d k=%d, shape %d", m, k, shape);
+  MI_REQUIRE(kind >= 0 && kind <= 5 && (kind != 4 || limit > 0.f) && shape >= 0 && shape < SHAPE_COUNT && ranges >= 1 && ranges <= MOST_RANGES && (kind == 1 || ranges == 1 || eighths) &&
                  (kind == 1 || ldc >= n),
              "gemm_tiles_bf16: kind %d, shape %d, %d ranges", kind, shape, ranges);
-  const int steps = ceil_div(k, 64), each = ceil_div(steps, ranges);
-  MI_REQUIRE(ceil_div(steps, each) == ranges, "gemm_tiles_bf16: %d steps of K do not make %d ranges", steps, ranges);
+  const int steps = ceil_div(k, 64), each = eighths ? steps : ceil_div(steps, ranges);
+  MI_REQUIRE(eighths || ceil_div(steps, each) == ranges, "gemm_tiles_bf16: %d steps of K do not make %d ranges", steps, ranges);
   const int element = kind == 1 || kind == 2 ? 4 : 2, at_once = kind >= 3 ? 8 : 4;
   const bool vec = (uintptr_t)out % (at_once * element) == 0 && (kind == 1 ? n : ldc) % at_once == 0;
   const GemmTilesLaunch l = {a, w, out, lda, ldw, ldc, kind, scale, {bias, limit, slope}, {}, vec, m, n, k, each, stream};
   const bool odd = k % 64 != 0;  // (one shape for these: nothing real is made so)
-  if (kind >= 3) gemm_tiles_gated_launch(shape, odd, l);
+  if (eighths) gemm_tiles_eighths_launch(SHAPES[shape].features, l);
+  else if (kind >= 3) gemm_tiles_gated_launch(shape, odd, l);
   else if (odd) gemm_tiles_launch<TileProduct<GEMM_TILE_ODD_SHAPE>, PAIRED_NOT, true>(l);
   else SHAPES[shape].launch(l);
   MI_CHECK_LAUNCH("gemm_tiles_bf16");

@@ -191,6 +191,149 @@ struct TileProduct {
     }
   }
 
+  // The same sums as eight waves that take an eighth of K each and add theirs in order: halves % 16 == 0.  Of the two waves along K one takes the even
+  // eighths, one the odd: a place in the ring holds 64 of K of an even one and the 64 as far into the one behind it.  W is read past the caches.
+  // ROUND: begin at pair of eighths `begin` (of 4).  Two eighths at a time, as a wave that sums all of them has twice the reads and products between two
+  // barriers: [16384 x 3072 | 2048] at 32 rows so 20.9 and 15.1 us, with waves that sum whole eighths in turn 21.0 and 17.2, in the order of `run` 19.5 and 14.2.
+  template <bool ROUND, typename RowA, typename RowW>
+  __device__ __forceinline__ void run_eighths(bf16_t* ring, int halves, RowA a_row, RowW w_row, int begin) {
+    static_assert(WK == 2 && STAGES % 2 == 0 && WM * WN * 4 * NT * MT * MI_WAVE * 8 <= RING, "the sums that change hands fit");
+    constexpr int PLACES = STAGES / 2;
+    const int each = halves / 16, rounds = 4 * each;  // steps of 64 of an eighth, of two eighths in turn
+    const bf16_t* src[MOST];
+    const int row_of = lane / 8;
+#pragma unroll
+    for (int j = 0; j < MOST; ++j) {
+      const int r = (wave + j * WAVES) * 8 + row_of;
+      const int chunk = (lane % 8) ^ (r % 8);
+      if ((wave + j * WAVES) * 8 < BM) src[j] = a_row(r) + chunk * 8;
+      else if (wave + j * WAVES < LOADS) src[j] = w_row(r - BM) + chunk * 8;
+      else src[j] = nullptr;  // (not fetched)
+      if (ROUND) src[j] += begin * each * (2 * STEP_K);
+    }
+    int left = each, pair = ROUND ? begin : 0;  // of what is fetched
+    auto fetch = [&](int place) {
+      bf16_t* to = ring + place * (2 * STAGE) + wave * 512;
+      int add = STEP_K;
+      if (--left == 0) {
+        left = each;
+        add += each * STEP_K;
+        if (ROUND && ++pair == 4) pair = 0, add -= 8 * each * STEP_K;
+      }
+#pragma unroll
+      for (int j = 0; j < MOST; ++j) {
+        if (j < EACH || wave < REST) {
+#pragma unroll
+          for (int odd = 0; odd < 2; ++odd) {
+            if ((wave + j * WAVES) * 8 >= BM) __builtin_amdgcn_global_load_lds((global_void*)(src[j] + odd * each * STEP_K), (lds_void*)(to + odd * STAGE + j * (WAVES * 512)), 16, 0, 2);
+            else __builtin_amdgcn_global_load_lds((global_void*)(src[j] + odd * each * STEP_K), (lds_void*)(to + odd * STAGE + j * (WAVES * 512)), 16, 0, 0);
+          }
+        }
+        src[j] += add;
+      }
+    };
+    // waits until at most `newer` (PLACES - 1 or fewer) places' loads of this wave are outstanding
+    auto wait_places = [&](int newer) {
+      if (newer >= 2) {
+        if (REST > 0 && wave < REST) outstanding<2 * 2 * MOST>();
+        else outstanding<2 * 2 * EACH>();
+      } else if (newer == 1) {
+        if (REST > 0 && wave < REST) outstanding<2 * MOST>();
+        else outstanding<2 * EACH>();
+      } else {
+        outstanding<0>();
+      }
+    };
+    static_assert(PLACES == 3, "as wait_places counts");
+#pragma unroll
+    for (int s = 0; s < PLACES; ++s)
+      if (s < rounds) fetch(s);
+    f32x4_t sums[4][NT][MT];  // of this wave's eighths
+#pragma unroll
+    for (int n = 0; n < NT; ++n)
+#pragma unroll
+      for (int m = 0; m < MT; ++m) acc[n][m] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+    bf16x8_t wf[2][NT], af[2][MT];
+    const bf16_t* a_at = ring + wk * STAGE + (wm * MT * 16 + col) * STEP_K;
+    const bf16_t* w_at = ring + wk * STAGE + (BM + wn * NT * 16 + col) * STEP_K;
+    auto read = [&](int set, int place, int half) {
+      const int at = place * (2 * STAGE) + ((half * 4 + quad) ^ (col % 8)) * 8;
+#pragma unroll
+      for (int n = 0; n < NT; ++n) wf[set][n] = *reinterpret_cast<const bf16x8_t*>(w_at + n * 16 * STEP_K + at);
+#pragma unroll
+      for (int m = 0; m < MT; ++m) af[set][m] = *reinterpret_cast<const bf16x8_t*>(a_at + m * 16 * STEP_K + at);
+    };
+    auto multiply = [&](int set) {
+      __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+      for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int n = 0; n < NT; ++n) acc[n][m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[set][n], af[set][m], acc[n][m], 0, 0, 0);
+      __builtin_amdgcn_s_setprio(0);
+    };
+    int place = 0, done = ROUND ? begin : 0, part_left = each;
+    wait_places(min(rounds, PLACES) - 1);
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    read(0, 0, 0);
+    for (int round = 0; round < rounds; ++round) {
+      read(1, place, 1);
+      __builtin_amdgcn_sched_barrier(0);
+      multiply(0);
+      __builtin_amdgcn_sched_barrier(0);
+      const int before = place;
+      place = place + 1 == PLACES ? 0 : place + 1;
+      if (round + 1 < rounds) {  // the next place is in LDS for all waves, and nobody reads this one any more: it is filled anew
+        wait_places(min(rounds - 2 - round, PLACES - 2));
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        if (round + PLACES < rounds) fetch(before);
+        read(0, place, 0);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      multiply(1);
+      __builtin_amdgcn_sched_barrier(0);
+      if (--part_left == 0) {
+        part_left = each;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          if (done == i) {
+#pragma unroll
+            for (int n = 0; n < NT; ++n)
+#pragma unroll
+              for (int m = 0; m < MT; ++m) sums[i][n][m] = acc[n][m];
+          }
+        done = done == 3 ? 0 : done + 1;
+#pragma unroll
+        for (int n = 0; n < NT; ++n)
+#pragma unroll
+          for (int m = 0; m < MT; ++m) acc[n][m] = f32x4_t{0.f, 0.f, 0.f, 0.f};
+      }
+    }
+    __syncthreads();
+    f32x4_t* to = reinterpret_cast<f32x4_t*>(ring) + ((wm * WN + wn) * 4 * NT * MT) * MI_WAVE + lane;
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int n = 0; n < NT; ++n)
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+          if (!mine(m)) to[((i * NT + n) * MT + m) * MI_WAVE] = sums[i][n][m];
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int n = 0; n < NT; ++n)
+#pragma unroll
+        for (int m = 0; m < MT; ++m)
+          if (mine(m)) {
+            const f32x4_t other = to[((i * NT + n) * MT + m) * MI_WAVE];
+            acc[n][m] += wk == 0 ? sums[i][n][m] : other;
+            acc[n][m] += wk == 0 ? other : sums[i][n][m];
+          }
+  }
+
   // The sums rounded to bfloat16 as rows of the tile in `ring`, MADE elements apart; all threads see them afterwards.
   __device__ __forceinline__ void leave(bf16_t* ring) {
     __syncthreads();

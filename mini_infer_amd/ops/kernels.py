@@ -475,7 +475,8 @@ def skinny_gemm_takes(m: int, k: int, lda: int, ldw: int, max_rows: int = SKINNY
 
 # The gated product and the q|k|v product with rotation and cache write take two tiles of 16
 # rows: up to 32 rows they measured faster than the vendor product followed by `silu_mul` /
-# `rope_kv_write` (8B sizes 12-21 %, 3B sizes 3-22 %), with 48 and 64 rows level or slower.
+# `rope_kv_write` (8B sizes 12-21 %, 3B sizes 3-22 %), with 48 and 64 rows level or slower.  (Of gated products these rows are tiles with the same sums
+# where `gated_eighths_for` says so.)
 SKINNY_WIDE_MAX_ROWS = 32
 
 
@@ -673,11 +674,8 @@ def tile_size(shape: int) -> tuple[int, int]:
 
 @functools.lru_cache(maxsize=8192)
 def gated_tiles_for(m: int, n: int, k: int, cus: int = WHOLE_DEVICE_CUS) -> int | None:
-    """The tile shape where the gated product of n features is made in tiles, or None.  Up to 32 rows the streaming product
-    (`gemm_skinny_swiglu_bf16`) stands, in whose sums a row's result does not depend on how many other rows there are (tiles of 32 x 64 are
-    faster where they are a block a compute unit on most of them, gate|up at 17 / 24 / 32 rows 16384 x 3072 22.6 / 22.3 / 23.6 us against
-    19.3 / 18.7 / 19.1, 11008 x 2048 12.9 / 13.8 / 15.1 against 11.6 / 11.9 / 12.3, and level or slower elsewhere, 28672 x 4096 43.7 / 45.9 /
-    47.1 against 48.7 / 47.4 / 47.4).  Above, measured against the vendor product and the activation's launch, tiles are 1.0 to 1.9 times as fast up to
+    """The tile shape where the gated product of n features is made in tiles, or None.  Up to 32 rows `gated_eighths_for` says, whose tiles keep the sums of
+    the streaming product (`gemm_skinny_swiglu_bf16`), in which a row's result does not depend on how many other rows there are.  Above, measured against the vendor product and the activation's launch, tiles are 1.0 to 1.9 times as fast up to
     160 rows, and beyond as long as tiles of up to 192 x 128 are what pays (7168 x 4096 at 256 rows 32.5 against 43.8, 16384 x 2048 at
     271 / 320 29.4 / 30.8 against 33.3 / 33.9; with the clamped activation 16384 x 3072 at 64 / 200 / 300 rows 24.7 / 39.9 / 46.5 against 22.1 / 36.1
     / 44.1); where there is work for larger ones the library is faster by as much as 1.3 (28672 x 4096 at 193 rows 86.9 / 72.3, 57344 x 8192 at 161 /
@@ -688,6 +686,22 @@ def gated_tiles_for(m: int, n: int, k: int, cus: int = WHOLE_DEVICE_CUS) -> int 
     if m > 160 and tile_size(shape)[0] * tile_size(shape)[1] > 192 * 128:
         return None
     return shape
+
+
+GATED_EIGHTHS = 8  # ranges of K by which `_tiles` knows them
+
+
+def gated_eighths_for(m: int, n: int, k: int, cus: int = WHOLE_DEVICE_CUS) -> int | None:
+    """The tile shape (0: 64 wide, 1: 128) where the gated product of 17 to 32 rows is made in tiles that sum K in eighths, bit for bit what the streaming
+    product gives, or None.  Microseconds, streaming / so, at 17 and 32 rows, weights from memory: gate|up 16384 x 3072 22.4 / 20.3 and 23.8 / 20.9, x 2048 17.9 / 14.8
+    and 19.6 / 15.1, x 1024 10.3 / 9.4 and 10.9 / 9.8, 28672 x 5120 61.1 / 54.5 and 73.7 / 55.8, x 4096 44.9 / 44.7 and 51.2 / 44.6, x 3072 36.7 / 34.0 and 42.7 / 34.7, 11008
+    x 2048 13.7 / 13.5 and 16.2 / 14.0, 10240 x 3072 17.4 / 16.8 and 19.7 / 17.7.  Tiles 64 wide while each has a compute unit (16384 x 3072 at 32 rows 20.9,
+    128 wide 27.3; 18432 x 3072 32.4 / 31.5).  Not with fewer features (7168 x 4096 15.7 / 19.0 and 19.0 / 19.8), nor where rows of W are 8 KB apart and the eighths that are read
+    together 1 KB, unless the tiles are many (12288 x 4096 23.0 / 25.4, 20480 x 4096 36.7 / 39.9, 22016 x 4096 40.9 / 40.2), nor where these are 2 KB
+    (57344 x 8192 153 / 192)."""
+    if not SKINNY_MAX_ROWS < m <= SKINNY_WIDE_MAX_ROWS or k % 512 or not 1024 <= k <= 5120 or n < (11_000 if k % 4096 == 0 else 5_000):
+        return None
+    return 0 if -(-n // 32) <= cus else 1
 
 
 TURNS_MIN_ROWS = 321
@@ -775,18 +789,19 @@ def _turns(act: int, x: torch.Tensor, weight: torch.Tensor, n: int, bias: torch.
 
 def _gated_as_one(act: int, x: torch.Tensor, weight: torch.Tensor, steady: bool, bias: torch.Tensor | None = None, limit: float = 0.0,
                   slope: float = 0.0) -> torch.Tensor | None:
-    """The gated product of more than 32 rows with its activation as one launch of tiles where that pays, else None."""
+    """The gated product of more than 16 rows with its activation as one launch of tiles where that pays, else None."""
     if _turns_take(x, weight, steady):
         return _turns(act, x, weight, weight.shape[0] // 2, bias, limit, slope)
-    if steady or x.dim() != 2 or not SKINNY_WIDE_MAX_ROWS < x.shape[0] <= TILES_MAX_ROWS or not _rows_of_bf16(x, weight):
+    if x.dim() != 2 or not SKINNY_MAX_ROWS < x.shape[0] <= TILES_MAX_ROWS or steady and x.shape[0] > SKINNY_WIDE_MAX_ROWS or not _rows_of_bf16(x, weight):
         return None
     _need_cuda(x, weight, bias)
     m, n = x.shape[0], weight.shape[0] // 2
-    shape = gated_tiles_for(m, n, x.shape[1], _compute_units(x.device))
+    few = m <= SKINNY_WIDE_MAX_ROWS
+    shape = (gated_eighths_for if few else gated_tiles_for)(m, n, x.shape[1], _compute_units(x.device))
     if shape is None:
         return None
     out = torch.empty((m, n), dtype=torch.bfloat16, device=x.device)
-    return _tiles(GATED_TILE_KINDS[act], x, weight, out, n, shape, 1, bias=bias, limit=limit, slope=slope)
+    return _tiles(GATED_TILE_KINDS[act], x, weight, out, n, shape, GATED_EIGHTHS if few else 1, bias=bias, limit=limit, slope=slope)
 
 
 def linear(x: torch.Tensor, weight: torch.Tensor, partial_ok: bool = False, steady: bool = False) -> torch.Tensor | PartialSums:
@@ -1046,7 +1061,7 @@ def qkv_rope_write_many(
 def linear_swiglu(x: "torch.Tensor | ScaledRows", gate_up_weight: torch.Tensor, steady: bool = False) -> torch.Tensor:
     """`silu(x @ gate.T) * (x @ up.T)` with `gate_up_weight` = [gate; up] stacked, [2I, K].
 
-    bfloat16 with at most 32 rows, up to some hundreds where that is faster (`gated_tiles_for`) and most of more (`turns_pay`) runs as ONE
+    bfloat16 with at most 32 rows (`gated_eighths_for`), up to some hundreds where that is faster (`gated_tiles_for`) and most of more (`turns_pay`) runs as ONE
     hand-written kernel (the product with the activation in its last step), and so do up to 8 float32 rows (4 of a long K);
     otherwise the product and `silu_mul` run in turn.  Both ways round the two products to the element type before the activation, so given
     the same rows a token's result does not depend on which one ran.  `x` may be

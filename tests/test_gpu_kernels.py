@@ -520,6 +520,26 @@ def test_linear_leaves_partial_sums_only_where_asked_and_where_it_pays():
         ops.linear_partial_sums(_rand(129, 64, dtype=torch.bfloat16), _rand(16, 64, dtype=torch.bfloat16))
 
 
+@pytest.mark.parametrize("m, n, k", [(17, 5000, 1024), (32, 8192, 3072), (31, 5127, 2048), (18, 8193, 1536), (25, 11003, 4096), (32, 9000, 2560), (20, 8200, 5120)])
+def test_gated_products_of_17_to_32_rows_in_eighths_of_k_give_the_streaming_bits(monkeypatch, m, n, k):
+    """Tiles of both widths, with a last one of few features, begun at any pair of eighths or not, each row as in a product of at most 16."""
+    from mini_infer_amd import ops
+    from mini_infer_amd.ops import kernels
+
+    taken = []
+    own = kernels._tiles
+    monkeypatch.setattr(kernels, "_tiles", lambda kind, *rest, **more: (taken.append((kind, rest[5])), own(kind, *rest, **more))[1])
+    a, w = _rand(m, k + 64, dtype=torch.bfloat16, seed=61)[:, :k], _rand(2 * n, k, dtype=torch.bfloat16, seed=62, scale=0.05)
+    bias = _rand(2 * n, seed=63, dtype=torch.float32)
+    got = [f(steady) for steady in (False, True) for f in (
+        lambda s: ops.linear_swiglu(a, w, steady=s), lambda s: ops.linear_geglu(a, w, steady=s), lambda s: ops.linear_clamped_glu(a, w, bias, 2.0, 1.702, steady=s))]
+    assert taken == [(3, kernels.GATED_EIGHTHS), (5, kernels.GATED_EIGHTHS), (4, kernels.GATED_EIGHTHS)] * 2
+    both = torch.cat([ops.gemm_skinny_bf16(a[at:at + 16], w) for at in range(0, m, 16)])
+    want = [ops.silu_mul(both), ops.gated_mul(both[:, :n], both[:, n:], "gelu_tanh"), ops.clamped_glu(both, bias, 2.0, 1.702)]
+    for i, x in enumerate(got):
+        assert torch.equal(x, want[i % 3]), i
+
+
 @pytest.mark.parametrize(
     "m,inter,k",
     [(1, 14336, 4096), (8, 14336, 4096), (16, 160, 64), (7, 301, 96), (13, 4100, 160), (3, 5, 32), (9, 8192, 3072),
