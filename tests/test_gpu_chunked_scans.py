@@ -314,6 +314,56 @@ def test_single_tokens_that_are_not_finite(monkeypatch, kind, dim, vdim):
         assert float((got - walked)[finite].norm() / walked[finite].norm()) < (2.0 ** -7 if kind == "delta" and got.dim() == 2 else 8e-7)
 
 
+# Requests in this order: single ones, portions and empty ones on both sides of the 64th from the end; more portions than a step of unknown division has blocks for.
+MANY_REQUESTS = [[1] * 40 + [70], [1] * 10 + [33, 0] + [1] * 20 + [0, 0, 40] + [1] * 45 + [0, 65], [40, 33] * 32 + [1] * 20, [2] * 30 + [1] * 70 + [97]]
+
+
+@pytest.mark.parametrize("lengths", MANY_REQUESTS)
+@pytest.mark.parametrize("heads,shared,dim,vdim", [(16, 4, 64, 128), (18, 3, 96, 80), (6, 1, 256, 250)])
+@pytest.mark.parametrize("known", [True, False])
+@pytest.mark.parametrize("kind", ["delta", "per_channel"])
+def test_chunks_of_steps_with_as_many_blocks_as_there_is_work(monkeypatch, kind, known, heads, shared, dim, vdim, lengths):
+    """Where a walk's blocks find their pieces of work themselves (csrc/chunk_scan.h, launch_walk): every piece once, and those that a block makes one after
+    another do not meet; a single token, a portion and a state that are not finite among them, and a request without a slot."""
+    from mini_infer_amd import ops
+
+    cus = torch.cuda.get_device_properties(DEV).multi_processor_count
+    blocks, tokens, requests, longest = -(-vdim // 16), sum(lengths), len(lengths), max(lengths) if known else None
+    assert requests * heads * blocks > 8 * cus and (kind != "delta" or heads * blocks < cus)
+    portions = [b for b in range(requests) if lengths[b] > 1]
+    many = 1 if longest is None else 1 + min(requests - 1, tokens - longest - (requests - 1))
+    if many == requests:
+        pytest.skip("a block for each request and its columns where the portions may be as many as the requests")
+    if lengths is MANY_REQUESTS[2] and not known and dim != 96:
+        assert heads * (len(portions) * blocks + 20 * 2) > 8 * cus  # (so blocks take a second piece)
+    g = torch.Generator(device=DEV).manual_seed(31)
+    q, k, v = (torch.randn(tokens, n, generator=g, device=DEV).bfloat16() for n in (shared * dim, shared * dim, heads * vdim))
+    gate = torch.randn(tokens, heads * dim if kind == "per_channel" else heads, generator=g, device=DEV).bfloat16()
+    state = _state(g, requests, ops.delta_state_shape(heads, dim, vdim) if kind == "delta" else ops.decay_state_shape(heads, dim, vdim), dim)
+    cu = _boundaries(lengths)
+    slots = torch.randperm(requests, generator=g, device=DEV).int()
+    single, portion = lengths.index(1), portions[-1]
+    slots[lengths.index(1, single + 1)] = -1
+    v[int(cu[single]), vdim + 3], v[int(cu[portion]) + 1, vdim - 1] = float("nan"), float("inf")
+    state[slots[lengths.index(1, single + 2)].long(), heads - 1, vdim - 1, 5] = float("inf")
+    if kind == "delta":
+        qkv = torch.cat([q, k, v], 1)
+        proj = torch.cat([torch.randn(tokens, heads, generator=g, device=DEV).bfloat16(), gate, torch.randn(tokens, heads * vdim, generator=g, device=DEV).bfloat16()], 1)
+        names = dict(heads=heads, kv_heads=shared, dim=dim, vdim=vdim, eps=1e-6, longest=longest)
+        call = lambda s: ops.gated_delta(qkv, proj, 0, heads, 2 * heads, torch.zeros(heads, device=DEV), torch.full((heads,), -2.0, device=DEV),  # noqa: E731
+                                         torch.ones(vdim, device=DEV), s, cu, slots, **names)
+    else:
+        names = dict(heads=heads, groups=shared, dim=dim, vdim=vdim, per_head=False, rate=None, inv_tau=0.0625, longest=longest)
+        call = lambda s: ops.decay_scan(q, 0, k, 0, v, 0, gate, 0, torch.zeros(heads * dim, device=DEV), s, cu, slots, **names)  # noqa: E731
+    (out, left), (out_walked, left_walked) = _both(monkeypatch, call, state)
+    for got, walked in ((out.double(), out_walked.double()), (left.double(), left_walked.double())):
+        assert torch.equal(got.isnan(), walked.isnan()) and torch.equal(got.isinf(), walked.isinf()) and torch.equal(got[got.isinf()], walked[walked.isinf()])
+        finite = walked.isfinite()
+        # (as test_what_is_not_finite_goes_token_by_token; a piece left out or made twice is some 1e-2)
+        assert float((got - walked)[finite].norm() / walked[finite].norm()) < (2.0 ** -7 if kind == "delta" and got.dim() == 2 else 8e-7)
+    assert torch.equal(left[requests:], state[requests:])
+
+
 @pytest.mark.parametrize("kind", ["delta", "per_head", "per_channel"])
 @pytest.mark.parametrize("lengths,known,chunks", [
     ([300], True, True), ([300], False, True), ([1] * 15 + [300], True, True), ([64] * 20, False, True),
