@@ -438,10 +438,13 @@ __device__ __forceinline__ bool walk_portion(const WalkArgs& p, f32x4_t (*parts)
   return again;
 }
 
-// 16 columns token by token, for what is not finite: 16 lanes a column, 4 * DT rows a lane, every operand read and made by each lane itself, in the arithmetic of
-// the token-by-token kernels.  It is not fast, 2,048 tokens with a NaN 2.3 to 4.8 ms where those kernels take 0.9: a launch of theirs for it, nearly always with nothing
-// to do, was a step of 12 such layers' 1 to 2 %.  Rows: what brings a token's operands (Rows::operands in the .hip files: rows at .. at + R of q, k and the decays, and the
-// step size or write strength).
+// 16 columns token by token, for what is not finite: 16 lanes a column, 4 * DT rows a lane, in the arithmetic of the token-by-token kernels.  Tokens go in tiles
+// through LDS (`room`, the walk's own), the threads side by side along the channels, and a token's operands are read one token ahead.  The next tile is not
+// asked for while one is walked, and few of a tile's values at a time: it is the registers of the whole kernel, and with them the waves on a CU, that this must not
+// raise (the next tile in registers: 3 waves a SIMD instead of 4 with a decay per channel of 64).  Microseconds of a scan, 2,048 tokens with a NaN, as a launch of the
+// token-by-token kernels behind the walk / here with every lane reading and making its operands itself / so: delta rule, 32 heads of 128 x 128 1,103 / 2,699 / 1,062, 8 of
+// 256 x 256 1,606 / 9,342 / 1,722; a decay per head, 48 of 128 x 64 927 / 2,297 / 824; per channel, 12 of 128 x 256 984 / 4,713 / 879, 8 of 256 x 256 1,551 / 13,422 / 1,659.
+// TokenRows in the .hip files: what a token's operands are.
 template <int CTRL>
 __device__ __forceinline__ float lane_moved(float v) {
   return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true));
@@ -452,51 +455,103 @@ __device__ __forceinline__ float sum_of_16(float v) {  // (neighbours, pairs, th
   v += lane_moved<0x141>(v);
   return v + lane_moved<0x140>(v);
 }
+
+template <int DT, int MODE>
+struct TokenTile {
+  static constexpr int TOKENS = 32 / DT;
+  float q[TOKENS * 64 * DT], k[TOKENS * 64 * DT], a[MODE == PER_CHANNEL ? TOKENS * 64 * DT : 4];
+  float v[TOKENS][16], decay[TOKENS], step[TOKENS];
+};
+
 template <int DT, int MODE, typename Rows>
-__device__ __forceinline__ void walk_by_token(const WalkArgs& p, const Rows& rows, int b, int first, int last, int head, int block) {
-  constexpr int R = 4 * DT, PAD = 64 * DT;
-  const int part = threadIdx.x % 16, col = block * 16 + threadIdx.x / 16, slot = p.slots[b];
+__device__ __forceinline__ void walk_by_token(const WalkArgs& p, const Rows& rows, TokenTile<DT, MODE>& room, int b, int first, int last, int head, int block) {
+  constexpr int R = 4 * DT, PAD = 64 * DT, TOKENS = TokenTile<DT, MODE>::TOKENS;
+  const int part = threadIdx.x % 16, column = threadIdx.x / 16, col = block * 16 + column, slot = p.slots[b];
   const bool live = col < p.vdim, kept = live && slot >= 0 && slot < p.num_slots;
-  const int column = live ? col : p.vdim - 1;
-  float* mine = p.state + (int64_t)(kept ? slot : p.num_slots) * p.state_stride + ((int64_t)head * p.vdim + column) * PAD + part * R;
-  constexpr int BATCH = MODE == PER_CHANNEL || DT > 2 ? 2 : 4;  // tokens whose operands are asked for together (more: registers of the whole kernel)
-  float S[R];
+  float* mine = p.state + (int64_t)(kept ? slot : p.num_slots) * p.state_stride + ((int64_t)head * p.vdim + (live ? col : p.vdim - 1)) * PAD + part * R;
+  f32x4_t S[DT];
 #pragma unroll
-  for (int i = 0; i < R; ++i) S[i] = mine[i];
+  for (int d = 0; d < DT; ++d) S[d] = *reinterpret_cast<const f32x4_t*>(mine + 4 * d);
   const float skip = (MODE == PER_HEAD && p.skip) ? p.skip[head] : 0.f;
-  for (int t0 = first; t0 < last; t0 += BATCH) {
-    float q[BATCH][R], k[BATCH][R], a[BATCH][R], step[BATCH], x[BATCH];
+  struct Of {
+    float4 q[DT], k[DT], a[MODE == PER_CHANNEL ? DT : 1];
+    float x, decay, step;
+  };
+  auto read = [&](int i) {
+    Of o;
 #pragma unroll
-    for (int n = 0; n < BATCH; ++n) {  // (past the last token that one again)
-      const int t = min(t0 + n, last - 1);
-      x[n] = to_f32(p.v[(int64_t)t * p.v_stride + p.v_col + (int64_t)head * p.vdim + column]);
-      step[n] = rows.template operands<R>(t, head, p.heads, part * R, q[n], k[n], a[n]);
+    for (int d = 0; d < DT; ++d) {
+      o.q[d] = load4(&room.q[i * PAD + part * R + 4 * d]);
+      o.k[d] = load4(&room.k[i * PAD + part * R + 4 * d]);
+      if constexpr (MODE == PER_CHANNEL) o.a[d] = load4(&room.a[i * PAD + part * R + 4 * d]);
     }
-    __builtin_amdgcn_sched_barrier(0);
+    o.x = room.v[i][column], o.decay = MODE == PER_CHANNEL ? 1.f : room.decay[i], o.step = MODE == PER_CHANNEL ? 1.f : room.step[i];
+    return o;
+  };
+  for (int t0 = first; t0 < last; t0 += TOKENS) {
+    const int n = min(TOKENS, last - t0);
+    lds_barrier();  // the last tile, or what stood here before it, has been read
+    {
+      const int d = threadIdx.x % PAD, from = min(d, rows.width() - 1);  // (past the last channel that one again, as zeros)
+#pragma unroll 4
+      for (int token = threadIdx.x / PAD; token < TOKENS; token += 256 / PAD) {  // (past the last token that one again)
+        const int64_t t = t0 + min(token, n - 1);
+        float q, k;
+        rows.channel(t, head, p.heads, from, q, k);
+        room.q[token * PAD + d] = d == from ? q : 0.f, room.k[token * PAD + d] = d == from ? k : 0.f;
+        if constexpr (MODE == PER_CHANNEL) room.a[token * PAD + d] = rows.channel_gate(t, head, from);
+      }
+      if constexpr (MODE == PER_CHANNEL) {  // (the gates that this thread has left)
+        const float bias = rows.channel_bias(head, from);
+#pragma unroll 2
+        for (int token = threadIdx.x / PAD; token < TOKENS; token += 256 / PAD) {
+          const float a = rows.channel_decay(room.a[token * PAD + d] + bias);
+          room.a[token * PAD + d] = d == from ? a : 0.f;
+        }
+      } else if (threadIdx.x < n) {
+        rows.head_gates(t0 + threadIdx.x, head, room.decay[threadIdx.x], room.step[threadIdx.x]);
+      }
+      for (int token = column; token < n; token += 16)
+        room.v[token][part] = to_f32(p.v[(int64_t)(t0 + token) * p.v_stride + p.v_col + (int64_t)head * p.vdim + min(block * 16 + part, p.vdim - 1)]);
+    }
+    lds_barrier();
+    if constexpr (MODE == DELTA) {  // unit vectors: 8 * DT lanes a token, 8 channels a lane
+      float *q = &room.q[threadIdx.x * 8], *k = &room.k[threadIdx.x * 8], qq = 0.f, kk = 0.f;
 #pragma unroll
-    for (int n = 0; n < BATCH; ++n) {
-      if (t0 + n >= last) break;
-      float u = step[n] * x[n];
+      for (int i = 0; i < 8; ++i) qq = fmaf(q[i], q[i], qq), kk = fmaf(k[i], k[i], kk);
+#pragma unroll
+      for (int off = 1; off < 8 * DT; off <<= 1) qq += __shfl_xor(qq, off, MI_WAVE), kk += __shfl_xor(kk, off, MI_WAVE);
+      const float q_inv = rsqrtf(qq + 1e-6f) * (1.0f / sqrtf((float)rows.width())), k_inv = rsqrtf(kk + 1e-6f);
+#pragma unroll
+      for (int i = 0; i < 8; ++i) q[i] *= q_inv, k[i] *= k_inv;
+      lds_barrier();
+    }
+    Of now = read(0);
+    for (int i = 0; i < n; ++i) {
+      const Of next = read(min(i + 1, n - 1));
+      float u = now.step * now.x;
       if constexpr (MODE == DELTA) {
         float seen = 0.f;
 #pragma unroll
-        for (int i = 0; i < R; ++i) seen = fmaf(S[i], k[n][i], seen);
-        u = step[n] * (x[n] - sum_of_16(seen) * a[n][0]);
+        for (int d = 0; d < DT; ++d) seen = fmaf(S[d][0], now.k[d].x, fmaf(S[d][1], now.k[d].y, fmaf(S[d][2], now.k[d].z, fmaf(S[d][3], now.k[d].w, seen))));
+        u = now.step * (now.x - sum_of_16(seen) * now.decay);
       }
-      float read = 0.f;
+      float out = 0.f;
 #pragma unroll
-      for (int i = 0; i < R; ++i) {
-        S[i] = fmaf(k[n][i], u, a[n][i] * S[i]);
-        read = fmaf(S[i], q[n][i], read);
+      for (int d = 0; d < DT; ++d) {
+        const float4 a = MODE == PER_CHANNEL ? now.a[d] : make_float4(now.decay, now.decay, now.decay, now.decay);
+        S[d] = f32x4_t{fmaf(now.k[d].x, u, a.x * S[d][0]), fmaf(now.k[d].y, u, a.y * S[d][1]), fmaf(now.k[d].z, u, a.z * S[d][2]), fmaf(now.k[d].w, u, a.w * S[d][3])};
+        out = fmaf(S[d][0], now.q[d].x, fmaf(S[d][1], now.q[d].y, fmaf(S[d][2], now.q[d].z, fmaf(S[d][3], now.q[d].w, out))));
       }
-      read = sum_of_16(read);
-      if constexpr (MODE == PER_HEAD) read = fmaf(skip, x[n], read);
-      if (part == 0 && live) p.out[((int64_t)(t0 + n) * p.heads + head) * p.vdim + col] = read;
+      out = sum_of_16(out);
+      if constexpr (MODE == PER_HEAD) out = fmaf(skip, now.x, out);
+      if (part == 0 && live) p.out[((int64_t)(t0 + i) * p.heads + head) * p.vdim + col] = out;
+      now = next;
     }
   }
   if (kept) {
 #pragma unroll
-    for (int i = 0; i < R; ++i) mine[i] = S[i];
+    for (int d = 0; d < DT; ++d) *reinterpret_cast<f32x4_t*>(mine + 4 * d) = S[d];
   }
 }
 
@@ -551,17 +606,22 @@ __device__ __forceinline__ bool find_piece(const int* __restrict__ cu, int reque
 template <int DT, int MODE, bool SEARCH, typename Rows>
 __global__ __launch_bounds__(256, MODE == DELTA || DT > 2 ? 1 : 2) void walk_kernel(WalkArgs p, Rows rows, int requests) {
   constexpr int TOGETHER = MODE == DELTA ? 8 : 4;
-  __shared__ f32x4_t parts[2][4][MODE == DELTA ? 4 : 2][MI_WAVE];
-  __shared__ __align__(16) Shared<MODE> shared[2];
-  static_assert(sizeof(parts) >= sizeof(float) * 4 * TOGETHER * 32, "a single token's sums fit");
+  struct Walked {
+    f32x4_t parts[2][4][MODE == DELTA ? 4 : 2][MI_WAVE];
+    Shared<MODE> shared[2];
+  };
+  __shared__ __align__(16) unsigned char room[sizeof(Walked)];
+  Walked& walked = *reinterpret_cast<Walked*>(room);
+  static_assert(sizeof(walked.parts) >= sizeof(float) * 4 * TOGETHER * 32 && sizeof(TokenTile<DT, MODE>) <= sizeof(Walked), "single tokens' sums and tiles of tokens fit");
   const int blocks = (p.vdim + 15) / 16;
   auto make = [&](const Piece& at) {
     int odd = 0;
-    if (at.last - at.first > 1) odd = walk_portion<DT, MODE>(p, parts, shared, at.b, at.first, at.last, at.head, at.block);
+    if (at.last - at.first > 1) odd = walk_portion<DT, MODE>(p, walked.parts, walked.shared, at.b, at.first, at.last, at.head, at.block);
     else if (at.last - at.first == 1 && at.block % TOGETHER == 0)
-      odd = walk_one_token<DT, MODE, TOGETHER>(p, reinterpret_cast<float*>(parts), at.b, at.first, at.head, at.block);
+      odd = walk_one_token<DT, MODE, TOGETHER>(p, reinterpret_cast<float*>(room), at.b, at.first, at.head, at.block);
     for (int g = 0; odd >> g != 0; ++g)
-      if ((odd >> g & 1) && at.block + g < blocks) walk_by_token<DT, MODE>(p, rows, at.b, at.first, at.last, at.head, at.block + g);
+      if ((odd >> g & 1) && at.block + g < blocks)
+        walk_by_token<DT, MODE>(p, rows, *reinterpret_cast<TokenTile<DT, MODE>*>(room), at.b, at.first, at.last, at.head, at.block + g);
   };
   Piece at;
   if constexpr (SEARCH) {

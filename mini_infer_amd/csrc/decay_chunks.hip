@@ -20,35 +20,24 @@ struct RowArgs {
   bool eights;  // rows of q, k (and the channels' gates) lie on 16 bytes in whole 8s
 };
 
-// What walk_by_token reads.
+// What walk_by_token takes of a token.
 template <int MODE>
 struct TokenRows {
   RowArgs p;
-  template <int R>
-  __device__ __forceinline__ float operands(int t, int head, int heads, int at, float (&q)[R], float (&k)[R], float (&a)[R]) const {
-    const int64_t row = t, share = head / (heads / p.groups) * (int64_t)p.dim;
-    const bf16_t* gate = p.gate + row * p.gate_stride + p.gate_col;
-    float decay = 0.f, step = 1.f;
-    if constexpr (MODE == PER_HEAD) {
-      step = mi_soft_plus_fast(to_f32(gate[head]) + p.gate_bias[head]);
-      decay = __builtin_amdgcn_exp2f(-(expf(p.rate[head]) * 1.4426950408889634f) * step);
-    }
-    const bf16_t *q_row = p.q + row * p.q_stride + p.q_col + share, *k_row = p.k + row * p.k_stride + p.k_col + share;
-#pragma unroll
-    for (int i = 0; i < R; ++i) {  // (without branches, past the last channel that one again)
-      const int d = min(at + i, p.dim - 1);
-      const bool in = at + i < p.dim;
-      const float qv = to_f32(q_row[d]) * p.q_scale, kv = to_f32(k_row[d]);
-      q[i] = in ? qv : 0.f, k[i] = in ? kv : 0.f;
-      if constexpr (MODE == PER_HEAD) {
-        a[i] = decay;
-      } else {
-        const float av = mi_channel_decay(to_f32(gate[(int64_t)head * p.dim + d]) + p.gate_bias[(int64_t)head * p.dim + d], p.inv_tau);
-        a[i] = in ? av : 0.f;
-      }
-    }
-    return step;
+  __device__ __forceinline__ void channel(int64_t t, int head, int heads, int d, float& q, float& k) const {
+    const int64_t at = head / (heads / p.groups) * (int64_t)p.dim + d;
+    q = to_f32(p.q[t * p.q_stride + p.q_col + at]) * p.q_scale, k = to_f32(p.k[t * p.k_stride + p.k_col + at]);
   }
+  __device__ __forceinline__ float channel_gate(int64_t t, int head, int d) const {
+    return to_f32(p.gate[t * p.gate_stride + p.gate_col + (int64_t)head * p.dim + d]);
+  }
+  __device__ __forceinline__ float channel_bias(int head, int d) const { return p.gate_bias[(int64_t)head * p.dim + d]; }
+  __device__ __forceinline__ float channel_decay(float z) const { return mi_channel_decay(z, p.inv_tau); }
+  __device__ __forceinline__ void head_gates(int64_t t, int head, float& decay, float& step) const {
+    step = mi_soft_plus_fast(to_f32(p.gate[t * p.gate_stride + p.gate_col + head]) + p.gate_bias[head]);
+    decay = __builtin_amdgcn_exp2f(-(expf(p.rate[head]) * 1.4426950408889634f) * step);
+  }
+  __device__ __forceinline__ int width() const { return p.dim; }
 };
 
 // a decay per head: one block per (chunk, group of rows, 8 heads of the group), 4 waves

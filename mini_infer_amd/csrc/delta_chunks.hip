@@ -10,29 +10,23 @@ namespace {
 
 using namespace chunk_scan;
 
-// What walk_by_token reads.
+// What walk_by_token takes of a token (it makes the unit vectors).
 struct TokenRows {
   const bf16_t *qkv, *proj;
   int64_t qkv_stride, proj_stride;
   int col_b, col_a, kv_heads, dim;
   const float *a_log, *dt_bias;
-  template <int R>
-  __device__ __forceinline__ float operands(int t, int head, int heads, int at, float (&q)[R], float (&k)[R], float (&a)[R]) const {
-    const bf16_t *row = qkv + (int64_t)t * qkv_stride + head / (heads / kv_heads) * dim, *gates = proj + (int64_t)t * proj_stride + head;
-    float qq = 0.f, kk = 0.f;
-#pragma unroll
-    for (int i = 0; i < R; ++i) {
-      const int d = min(at + i, dim - 1);  // (without branches, past the last channel that one again)
-      const float qv = to_f32(row[d]), kv = to_f32(row[kv_heads * dim + d]);
-      q[i] = at + i < dim ? qv : 0.f, k[i] = at + i < dim ? kv : 0.f;
-      qq = fmaf(q[i], q[i], qq), kk = fmaf(k[i], k[i], kk);
-    }
-    const float q_inv = rsqrtf(sum_of_16(qq) + 1e-6f) * (1.0f / sqrtf((float)dim)), k_inv = rsqrtf(sum_of_16(kk) + 1e-6f);
-    const float z = to_f32(gates[col_a]) + dt_bias[head], decay = expf(-expf(a_log[head]) * (z > 20.f ? z : log1pf(expf(z))));
-#pragma unroll
-    for (int i = 0; i < R; ++i) q[i] *= q_inv, k[i] *= k_inv, a[i] = decay;
-    return 1.f / (1.f + expf(-to_f32(gates[col_b])));
+  __device__ __forceinline__ void channel(int64_t t, int head, int heads, int d, float& q, float& k) const {
+    const bf16_t* row = qkv + t * qkv_stride + head / (heads / kv_heads) * dim + d;
+    q = to_f32(row[0]), k = to_f32(row[kv_heads * dim]);
   }
+  __device__ __forceinline__ void head_gates(int64_t t, int head, float& decay, float& step) const {
+    const bf16_t* gates = proj + t * proj_stride + head;
+    const float z = to_f32(gates[col_a]) + dt_bias[head];
+    decay = expf(-expf(a_log[head]) * (z > 20.f ? z : log1pf(expf(z))));
+    step = 1.f / (1.f + expf(-to_f32(gates[col_b])));
+  }
+  __device__ __forceinline__ int width() const { return dim; }
 };
 
 // 256 threads: 8 of them bring one token's q and k rows in and make them unit vectors; then a wave makes a 16 x 16
