@@ -50,7 +50,7 @@ struct ScanArgs {
   int num_slots;
   float* out;  // float32 [tokens, heads * vdim]
   int heads, groups, dim, vdim;
-  bool whole_runs;  // rows of q and k can be read a lane's run at a time
+  bool tokens_alone;  // a request's only token goes through decay_token (launch_scan)
 };
 
 template <typename T>
@@ -97,29 +97,23 @@ __device__ __forceinline__ double lanes_sum(double v) {
   return v;
 }
 
-// R values of a row from `at` on as float32, zeros from `dim` on; `whole`: they can be read in pieces of 16 bytes (of all R where those are fewer), and dim
-// is a multiple of R.
+// R values of a row from `at` on as float32, zeros from `dim` (a multiple of R) on; the row can be read in pieces of 16 bytes, of all R where those are fewer.
 template <typename T, int R>
-__device__ __forceinline__ void run_of_row(const T* row, int at, int dim, bool whole, float (&v)[R]) {
-  if (whole) {
-    constexpr int V = sizeof(T) == 2 && R >= 8 ? 8 : 4;
+__device__ __forceinline__ void run_of_row(const T* row, int at, int dim, float (&v)[R]) {
+  constexpr int V = sizeof(T) == 2 && R >= 8 ? 8 : 4;
 #pragma unroll
-    for (int i = 0; i < R; i += V) {
-      float some[V];
-      if constexpr (V == 8) {
-        const uint4 got = *reinterpret_cast<const uint4*>(row + (at < dim ? at + i : 0));
-        const uint32_t words[4] = {got.x, got.y, got.z, got.w};
+  for (int i = 0; i < R; i += V) {
+    float some[V];
+    if constexpr (V == 8) {
+      const uint4 got = *reinterpret_cast<const uint4*>(row + (at < dim ? at + i : 0));
+      const uint32_t words[4] = {got.x, got.y, got.z, got.w};
 #pragma unroll
-        for (int w = 0; w < 4; ++w) some[2 * w] = __uint_as_float(words[w] << 16), some[2 * w + 1] = __uint_as_float(words[w] & 0xFFFF0000u);
-      } else {
-        mi_load_cols<T, V>(row + (at < dim ? at + i : 0), some);
-      }
-#pragma unroll
-      for (int j = 0; j < V; ++j) v[i + j] = at < dim ? some[j] : 0.f;
+      for (int w = 0; w < 4; ++w) some[2 * w] = __uint_as_float(words[w] << 16), some[2 * w + 1] = __uint_as_float(words[w] & 0xFFFF0000u);
+    } else {
+      mi_load_cols<T, V>(row + (at < dim ? at + i : 0), some);
     }
-  } else {
 #pragma unroll
-    for (int i = 0; i < R; ++i) v[i] = at + i < dim ? to_f32(row[at + i]) : 0.f;
+    for (int j = 0; j < V; ++j) v[i + j] = at < dim ? some[j] : 0.f;
   }
 }
 
@@ -147,8 +141,8 @@ __device__ __forceinline__ void decay_token(const ScanArgs& p, int64_t t, int sl
       S[g][i] = got.x, S[g][i + 1] = got.y, S[g][i + 2] = got.z, S[g][i + 3] = got.w;
     }
   }
-  run_of_row<T, R>((const T*)p.q + p.q_col + t * p.q_stride + (int64_t)grp * p.dim, at, p.dim, p.whole_runs, q);
-  run_of_row<T, R>((const T*)p.k + p.k_col + t * p.k_stride + (int64_t)grp * p.dim, at, p.dim, p.whole_runs, k);
+  run_of_row<T, R>((const T*)p.q + p.q_col + t * p.q_stride + (int64_t)grp * p.dim, at, p.dim, q);
+  run_of_row<T, R>((const T*)p.k + p.k_col + t * p.k_stride + (int64_t)grp * p.dim, at, p.dim, k);
   const T* v_row = (const T*)p.v + p.v_col + t * p.v_stride + (int64_t)head * p.vdim;
 #pragma unroll
   for (int g = 0; g < G; ++g) x[g] = to_f32(v_row[min(col[g], p.vdim - 1)]);
@@ -385,7 +379,7 @@ __global__ __launch_bounds__(256) void decay_scan_kernel(ScanArgs p, int request
   const int head = rest % p.heads, col_block = rest / p.heads;
   if constexpr (MODE == DECAY_PER_HEAD) {
     const int first = p.cu[b];
-    if (p.cu[b + 1] - first == 1) {
+    if (p.tokens_alone && p.cu[b + 1] - first == 1) {
       if (col_block % G == 0) decay_token<T, R, L, G>(p, first, p.slots[b], head, col_block * COLS);
       return;
     }
@@ -406,17 +400,22 @@ template <typename T, int MODE>
 int launch_scan(ScanArgs p, int tokens, int requests, hipStream_t stream) {
   int rows, lanes;
   scan_shape(p.dim, &rows, &lanes);
-  const int piece = min(16, rows * (int)sizeof(T));
-  auto in_pieces = [&](const void* row, int64_t stride, int col) {
-    return ((uintptr_t)row + (uintptr_t)col * sizeof(T)) % piece == 0 && stride * sizeof(T) % piece == 0;
-  };
-  p.whole_runs = p.dim % rows == 0 && in_pieces(p.q, p.q_stride, p.q_col) && in_pieces(p.k, p.k_stride, p.k_col);
   const int64_t grid = (int64_t)requests * p.heads * ceil_div(p.vdim, 256 / lanes);
   MI_REQUIRE(grid < ((int64_t)1 << 31), "decay_scan: %lld blocks are too many", (long long)grid);
   constexpr int TOGETHER = MODE == DECAY_PER_HEAD ? 4 : 1;
   // (two rounds of what the CUs hold; 24 requests of 32 heads of 64 columns, 3,072 blocks, take the same either way.  Beside a long portion, whose
   // chain the larger blocks hold up, one: 38 tokens beside 73, a step of 12 layers 2,910 / 2,928 us.)
   const bool together = grid >= 4096 && tokens <= requests;
+  // Single tokens by decay_token: where rows of q and k are read a lane's run at a time, in float32 only four column blocks together and keys of more than 64.
+  // Microseconds as in a walk / so, a decay per head, from memory: bfloat16, 64 heads of 128 x 64, 8 / 40 requests 11.5 / 10.1 and 44.9 / 35.9, 48 of 64 x 64 6.0 / 5.4 and
+  // 19.8 / 17.0; value by value 64 of 100 x 64 at 8 11.4 / 17.0, 24 of 200 x 256 33.5 / 61.5 and 121 / 183, 64 of 256 x 64 24.1 / 50.2 and 88.8 / 116; float32, 64 of
+  // 128 x 64 at 40 49.3 / 37.3, at 8 13.7 / 14.2, beside a portion 46 / 54, 48 of 64 x 64 at 40 19.2 / 22.6, 64 of 256 x 64 at 8 / 40 23.6 / 28.1 and 90.6 / 83.7.
+  const int piece = min(16, rows * (int)sizeof(T));
+  auto in_pieces = [&](const void* row, int64_t stride, int col) {
+    return ((uintptr_t)row + (uintptr_t)col * sizeof(T)) % piece == 0 && stride * sizeof(T) % piece == 0;
+  };
+  p.tokens_alone = p.dim % rows == 0 && in_pieces(p.q, p.q_stride, p.q_col) && in_pieces(p.k, p.k_stride, p.k_col) &&
+                   (sizeof(T) == 2 || (together && p.dim > 64));
 #define MI_SCAN(RR, LL)                                                                                               \
   do {                                                                                                                \
     if (together) decay_scan_kernel<T, MODE, RR, LL, TOGETHER><<<(unsigned)grid, 256, 0, stream>>>(p, requests);      \
@@ -562,7 +561,7 @@ extern "C" int mi_decay_scan(int dtype, int mode, const void* q, int64_t q_strid
   p.q_col = q_col, p.k_col = k_col, p.v_col = v_col, p.gate_col = gate_col;
   p.gate_bias = gate_bias, p.rate = rate, p.skip = skip, p.inv_tau = inv_tau, p.q_scale = q_scale;
   p.state = state, p.state_stride = state_stride, p.cu = cu, p.slots = slots, p.num_slots = num_slots, p.out = out;
-  p.heads = heads, p.groups = groups, p.dim = dim, p.vdim = vdim, p.whole_runs = false;
+  p.heads = heads, p.groups = groups, p.dim = dim, p.vdim = vdim, p.tokens_alone = false;
   if (dtype == MI_F32) return mode == 0 ? launch_scan<float, DECAY_PER_CHANNEL>(p, num_tokens, num_requests, stream)
                                         : launch_scan<float, DECAY_PER_HEAD>(p, num_tokens, num_requests, stream);
   return mode == 0 ? launch_scan<bf16_t, DECAY_PER_CHANNEL>(p, num_tokens, num_requests, stream)

@@ -506,6 +506,33 @@ def test_decay_scan_of_single_tokens_gives_the_bits_of_portions(monkeypatch, hea
     assert torch.equal(single[:-1], whole[:-1])
 
 
+def test_decay_scan_of_single_tokens_costs_little_more_off_16_bytes(monkeypatch):
+    """Rows of q and k that cannot be read 16 bytes at a time: 1.1 times the time of those that can (1.5 times where every lane read its own value by value)."""
+    from mini_infer_amd import ops
+    from mini_infer_amd.ops import kernels
+
+    monkeypatch.setattr(kernels, "chunked_scan_pays", lambda *sizes: False)
+    heads, dim, vdim, requests = 64, 256, 256, 8
+    g = torch.Generator(device=DEV).manual_seed(37)
+    bias, rate = torch.zeros(heads, device=DEV), torch.zeros(heads, device=DEV)
+    state = _state(g, requests, ops.decay_state_shape(heads, dim, vdim), dim)
+    cu, slots = _boundaries([1] * requests), torch.arange(requests, dtype=torch.int32, device=DEV)
+    took = []
+    for odd in (False, True):
+        q, k, v, gate = (_rows(g, requests, n, odd) for n in (dim, dim, heads * vdim, heads))
+        times = []
+        for _ in range(6):
+            begin, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            begin.record()
+            for _ in range(10):
+                ops.decay_scan(q, 0, k, 0, v, 0, gate, 0, bias, state, cu, slots, heads=heads, groups=1, dim=dim, vdim=vdim, per_head=True, rate=rate)
+            end.record()
+            end.synchronize()
+            times.append(begin.elapsed_time(end))
+        took.append(min(times))
+    assert took[1] < 1.3 * took[0], took
+
+
 @pytest.mark.parametrize("lengths,channels", [([1, 2, 3, 0, 4, 1, 5, 9, 1], 12), ([70], 1028), ([3, 1] * 8 + [17, 6, 1, 2], 96),
                                               ([1, 2, 3, 4, 5, 6, 7, 8, 9, 10, 300, 3], 8192), ([2, 1, 3, 990, 13, 4, 1, 1, 29], 8192)])
 @pytest.mark.parametrize("taps", [2, 3, 4])
