@@ -513,45 +513,57 @@ extern "C" int mi_gemm_f32_rope(const float* a, int64_t lda, const float* w, int
 #define F32_ROWS_FORMS(X) X(0, 1, 1) X(1, 1, 2) X(2, 2, 1) X(3, 2, 2) X(4, 4, 1) X(5, 4, 2)
 enum { F32_ROWS = 6, F32_FEW = 6, F32_TILES_32 = 7, F32_TILES_64 = 8, F32_FORMS = 9 };
 
-// Microseconds that a form is expected to take: the rounds of its blocks over the compute units, with the cycles a block is on the matrix pipe (a
-// slice is 128 for each of its 16 x 16 products) and those it loses on converting and moving its operands.  Tiles beside one another on a CU cover
-// one another's waits, one by itself does not.  Within 12 % of what 9 to 256 rows of 3072, 2048 and 16384 x 2048 and of 2048 x 8192 took.
-static double f32_micros(int form, int m, int n, int k, int count, int cus) {
+// Microseconds that a form is expected to take, for operands that are read value by value, in pieces and in lines.  The rows' kernel: a launch; for every
+// two rounds of its blocks over the compute units (two of them are on one at a time) the loads of a wave's slices one after another; for every round a block's
+// slices on one matrix pipe (waves w and w + 4 share one) with its 16 x 16 products and their operands, and what its sums and its end take.  The tiles: a launch and for
+// every slice a first round and the others.  Fitted to 3,110 products of 1 to 600 rows, 16 to 20,000 features and K 32 to 9,000, each in every form: half of the times are
+// within 6 % (11 % value by value) for the rows' kernel and 4 % for the tiles.
+struct RowsCost {
+  double launch, trip, round, tile, product, operand;
+};
+struct TilesCost {
+  double launch, only, each, rest;
+};
+static double f32_micros(int form, int how, int m, int n, int k, int count, int cus) {
+  static const RowsCost rows_cost[3] = {{2.08, 0.557, 0, 0.0466, 0.0546, 0.0849}, {2.41, 0.139, 0.0215, 0.0994, 0.0678, 0.0238}, {2.58, 0.0654, 0.117, 0.139, 0.0653, 0.0144}};
+  static const TilesCost tiles_64[3] = {{3.04, 1.83, 1.41, 0.396}, {3.18, 1.43, 1.29, 0}, {2.89, 1.45, 1.17, 0.246}};
+  static const TilesCost tiles_32[3][2] = {  // one slice a stage, four
+      {{2.67, 1.18, 0.779, 0.286}, {5.89, 1.12, 0.803, 0}}, {{2.75, 0.893, 0.67, 0.14}, {5.01, 0.749, 0.559, 0.127}}, {{2.62, 0.897, 0.627, 0.285}, {4.59, 0.741, 0.553, 0.127}}};
   const int slices = ceil_div(k, SLICE);
   auto rounds = [&](int rows, int features) { return (double)ceil_div64((int64_t)ceil_div(m, rows) * ceil_div(n, features) * count, cus); };
-  if (form == F32_TILES_32) {
-    const double r = rounds(32, BN);
-    return (r > 1 ? 0.56 * r + 0.22 : 0.77) * slices;
-  }
-  if (form == F32_TILES_64) {
-    const double r = rounds(64, BN);
-    return (r > 1 ? 1.1 * r + 0.39 : 1.44) * slices;
+  if (form == F32_TILES_32 || form == F32_TILES_64) {
+    const TilesCost& c = form == F32_TILES_64 ? tiles_64[how] : tiles_32[how][segment_slices(k) % 4 == 0];
+    const double r = rounds(form == F32_TILES_64 ? 64 : 32, BN);
+    return c.launch + slices * (r > 1 ? c.each * r + c.rest : c.only);
   }
   constexpr int of[F32_ROWS][2] = {
 #define X(I, RT, FT) {RT, FT},
       F32_ROWS_FORMS(X)
 #undef X
   };
-  const int rt = of[form][0], ft = of[form][1];
+  const RowsCost& c = rows_cost[how];
+  const int rt = of[form][0], ft = of[form][1], run = segment_slices(k), on_a_pipe = ceil_div(slices, run) > 4 ? 2 * run : run;
   const double r = rounds(16 * rt, 16 * ft);
-  return 4.0 + r * (r > 2 ? 1.1 : 1.0) * slices * (128 * rt * ft + 30 * (rt + ft)) / 2100.0;
+  return c.launch + ceil(r / 2) * run * c.trip + r * (c.round + c.tile * rt * ft + 4 * on_a_pipe * (c.product * rt * ft + c.operand * (rt + ft)));
 }
 
-// The form of m rows for which the four-row products are not taken: the one that is expected to be the fastest.  (All give the same bits.)  Microseconds
-// of what stood here before (up to 32 rows, or 64 with less than 8,192 features, all rows a block; above, tiles through LDS) and this one, weights
-// from memory:
+// The form of m rows for which the four-row products are not taken: the one that is expected to be the fastest.  (All give the same bits.)  Over the
+// products that the times are fitted to, as geometric means of the fastest form's time, in lines / in pieces / value by value: all rows a block up to 32 rows, or 64 with
+// less than 8,192 features, and tiles above 1.35 / 1.23 / 1.16; by times that know neither a tile's launch nor how operands are read 1.08 / 1.14 / 1.13 (13 x 512
+// x 160 6.8 for 3.5 us, 2 x 1024 x 145 8.2 / 4.0, 232 x 6418 x 1024 value by value 167 / 116); so 1.01 / 1.015 / 1.01.  In lines, weights from memory,
+// before forms in blocks of rows / so:
 //     rows            25             64             96             128            256
 //     2048 x 2048     15.1 / 9.6     27.5 / 15.0    50.9 / 22.3    51.3 / 23.6    51.8 / 43.7
 //     3072 x 2048     15.8 / 15.3    28.3 / 22.4    51.1 / 32.8    51.3 / 36.2    82.1 / 67.2
 //     16384 x 2048    51.4 / 50.3    89.4 / 87.6    123 / 122      161 / 160      303 / 303
 //     2048 x 8192     50.1 / 31.5    91.0 / 51.5    195 / 77.7     196 / 83.5     199 / 148
-static int f32_form(int m, int n, int k, int count, int cus) {
+static int f32_form(int how, int m, int n, int k, int count, int cus) {
   int best = F32_TILES_64;
   if (m > 32 * 65535) return best;
-  double least = f32_micros(best, m, n, k, count, cus);
+  double least = f32_micros(best, how, m, n, k, count, cus);
   for (int form = 0; form < F32_FORMS; ++form) {
     if (form == F32_FEW || form == F32_TILES_64) continue;
-    const double t = f32_micros(form, m, n, k, count, cus);
+    const double t = f32_micros(form, how, m, n, k, count, cus);
     if (t < least) least = t, best = form;
   }
   return best;
@@ -567,9 +579,9 @@ static int gemm_f32(const float* a, int64_t lda, const float* w, int64_t ldw, fl
   const bool a16 = lda % 4 == 0 && (uintptr_t)a % 16 == 0 && (count == 1 || heads.a % 4 == 0), w16 = ldw % 4 == 0 && (uintptr_t)w % 16 == 0 && (count == 1 || heads.w % 4 == 0);
   const bool lines = whole_lines(a, lda, w, ldw, k, 32) && (count == 1 || (heads.a % 4 == 0 && heads.w % 32 == 0));
   const bool few = lines && few_rows_take(m, k);
-  const int form = only >= 0 ? only : few ? (int)F32_FEW : f32_form(m, n, k, count, max(8, mi_compute_units()));
   const bool aligned = a16 && w16 && k % 4 == 0;
   const int how = lines ? LINES : aligned ? PIECES : VALUES;
+  const int form = only >= 0 ? only : few ? (int)F32_FEW : f32_form(how, m, n, k, count, max(8, mi_compute_units()));
   MI_REQUIRE(form < F32_FORMS && (form != F32_FEW || few), "gemm_f32: form %d does not take m=%d k=%d", form, m, k);
   if (form == F32_FEW) {
     const bool half_empty = (int64_t)ceil_div(n, 16) * count <= 128;

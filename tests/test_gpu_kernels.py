@@ -1965,6 +1965,41 @@ def test_every_form_of_the_float32_product_gives_the_same_bits(m, n, k):
             assert torch.equal(out[:, :n], got) and (out[:, n:] == 7).all(), (first, form)
 
 
+@pytest.mark.parametrize("m, n, k, first", [(13, 512, 160, 0), (43, 4096, 224, 0), (2, 1024, 145, 1), (11, 82, 140, 4), (136, 2048, 2048, 1), (232, 6418, 1024, 1),
+                                            (150, 8192, 908, 4), (25, 2048, 2048, 0), (256, 2048, 8192, 0), (509, 3072, 2048, 0)])
+def test_the_form_of_a_float32_product_is_near_the_fastest(m, n, k, first):
+    """A few slices of K and many, operands in whole lines, in pieces and value by value; recorded, so that the host's part is not in it."""
+    from mini_infer_amd import ops
+    from mini_infer_amd.ops import library
+    from mini_infer_amd.ops.kernels import _ptr, _stream
+
+    lib = library.load()
+    wide = torch.randn(n, (k + 31) // 32 * 32 + 32, device="cuda")
+    a, w, out = torch.randn(m, k, device="cuda"), wide[:, first : first + k], torch.empty(m, n, device="cuda")
+
+    def micros(product):
+        product()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            for _ in range(20):
+                product()
+        times = []
+        for _ in range(6):
+            begin, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            begin.record()
+            graph.replay()
+            end.record()
+            end.synchronize()
+            times.append(begin.elapsed_time(end) * 50)
+        return min(times)
+
+    def in_form(form):
+        library.check(lib.mi_gemm_f32_as(form, _ptr(a), a.stride(0), _ptr(w), w.stride(0), _ptr(out), n, m, n, k, _stream()))
+
+    fastest = min(micros(lambda form=form: in_form(form)) for form in (0, 1, 2, 3, 4, 5, 7, 8))
+    assert micros(lambda: ops.gemm_f32(a, w)) < 1.3 * fastest
+
+
 @pytest.mark.parametrize("tokens", [1, 3, 5, 8, 9, 17, 40, 130])
 @pytest.mark.parametrize("heads, k, n", [(1, 64, 256), (32, 64, 256), (5, 256, 64), (3, 10, 22), (40, 36, 12)])
 def test_float32_products_of_all_heads_are_those_of_each(tokens, heads, k, n):
