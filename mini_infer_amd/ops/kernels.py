@@ -3567,11 +3567,30 @@ def expert_tiles_take(x: torch.Tensor, ff: int) -> bool:
 
 
 def expert_lines_take_f32(gate_up: torch.Tensor, down: torch.Tensor) -> bool:
-    """Whether float32 experts are read in whole lines for the matrix instruction (both products), which is faster than the products sorted by expert
-    at every size."""
+    """Whether float32 experts are read in whole lines for the matrix instruction (both products)."""
     lib = library.load()
     return gate_up.dtype == torch.float32 and all(
         bool(lib.mi_expert_lines_f32_take(_ptr(w), w.shape[2], w.shape[1] * w.shape[2])) for w in (gate_up, down))
+
+
+def sorted_f32_experts_pay(pairs: int, experts: int, width: int, ff: int, gated: bool, cus: int = WHOLE_DEVICE_CUS) -> bool:
+    """Whether `experts_grouped` is faster than `experts_by_expert` with float32 experts in whole lines, by the time that each is expected to take: blocks of 32 pairs
+    reach 45 TFLOP/s while there are as many of them as compute units, a product an expert 71 behind the launches and what the host reads.  Fitted to 4,038 measured
+    pairs of 4 to 64 experts of 512 to 4,096 x 256 to 4,096, 16 to 1,500 rows each, with the margin 0.4 % off the better one (1.7 % without sorting, at worst 2.5
+    times as slow).  Microseconds in blocks / sorted: 4 experts, 1024 x 4096, 400 / 1,000 / 4,096 tokens of two choices 647 / 667, 1,496 / 1,116, 6,014 / 3,975; 8 of
+    2048 x 4096, 400 / 4,096 965 / 1,164, 8,445 / 7,750; 16 of 2048 x 2048, 400 / 2,048 555 / 818, 2,285 / 2,436; 64 of 2048 x 1024, six choices, 4,096 7,011 / 8,227."""
+    rows = pairs / experts
+    if rows < 1:
+        return False
+
+    def idle(blocks: int) -> float:
+        return -(-blocks // cus) * cus / blocks
+
+    first, second = ((4 if gated else 2) * pairs * width * ff / 1e6, 2 * pairs * width * ff / 1e6)  # MFLOP
+    passes = -(-math.ceil(rows) // 32) * 32 / rows if rows < 64 else 1 + 16 / rows
+    blocks = 37 + passes * (first * idle(experts * -(-ff // (16 if gated else 32))) + second * idle(experts * -(-width // 32))) / 45.5
+    one_by_one = 183 + 21.5 * experts + (first + second) * (1 + 32 / rows) / 70.9 + 5.4 * pairs * (width + (2 if gated else 1) * ff) / 1e6
+    return one_by_one < 0.88 * blocks
 
 
 def expert_tile_cuts(counts: list[int], weight_rows: int, k: int, cus: int = WHOLE_DEVICE_CUS) -> list[tuple[int, int, int, int]]:

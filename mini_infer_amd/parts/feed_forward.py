@@ -310,7 +310,8 @@ class RoutedExperts(FeedForward):
     expert's weights are streamed once for up to eight of its rows at a time (sizes that are not read
     16 bytes at a time work each pair on its own instead, the expert's weights read by index).  Many
     rows (bfloat16, rows in steps of 64 elements) run over tiles of 128 of an expert's rows staged through
-    LDS, from the same list; sizes those do not take are sorted by expert and every chosen expert runs the
+    LDS, from the same list; float32 (whole lines) goes on in blocks of 32 of an expert's rows up to some hundreds of them
+    (`ops.sorted_f32_experts_pay`); what none of these takes is sorted by expert and every chosen expert runs the
     engine's own products once over all its rows.  Router, correction and the shared expert's gate row stay float32."""
 
     graph_safe = True
@@ -406,7 +407,8 @@ class RoutedExperts(FeedForward):
         if ops.expert_tiles_take(x, self.intermediate_size):
             return False  # (tiles over the device's own list of rows are faster at every size)
         if x.dtype == torch.float32 and ops.expert_lines_take_f32(self.gate_up, self.down) and ops.experts_by_expert_take(x, self.gate_up, self.activation):
-            return False  # (and so are the blocks of float32 experts over that list)
+            # (and so are the blocks of float32 experts over that list up to some hundreds of rows an expert)
+            return ops.sorted_f32_experts_pay(x.shape[0] * self.top, self.experts, self.hidden_size, self.intermediate_size, self.gated)
         element = 2 if self.dtype == torch.bfloat16 else 4
         expert_bytes = (3 if self.gated else 2) * self.intermediate_size * self.hidden_size * element
         return x.shape[0] * self.top * expert_bytes > self.experts * self.GROUPED_BYTES_PER_EXPERT

@@ -166,3 +166,29 @@ def test_products_with_small_matrices(m, n, k, plan):
     got = kernels.small_product_plan(m, n, k)
     made = None if got is None else "rows" if got[0] is not None else "whole" if got[2] == 1 else "cut"
     assert made == plan
+
+
+@pytest.mark.parametrize("tokens, experts, top, width, ff, gated, pays", [
+    (1, 16, 2, 2048, 2048, True, False), (400, 16, 2, 2048, 2048, True, False), (2048, 16, 2, 2048, 2048, True, False), (4096, 64, 6, 2048, 1024, True, False),
+    (400, 4, 2, 1024, 4096, True, False), (1000, 4, 2, 1024, 4096, True, True), (4096, 4, 2, 1024, 4096, True, True), (4096, 8, 2, 2048, 4096, True, True),
+    (3, 64, 1, 512, 256, False, False), (4096, 4, 4, 512, 4096, False, True)])
+def test_float32_experts_of_many_rows_are_sorted(monkeypatch, tokens, experts, top, width, ff, gated, pays):
+    """On both sides of the line (measured at its rule), through the layer's own choice where a step is not recorded."""
+    import torch
+
+    from mini_infer_amd import ops
+    from mini_infer_amd.parts import feed_forward
+
+    assert kernels.sorted_f32_experts_pay(tokens * top, experts, width, ff, gated) == pays
+    layer = feed_forward.RoutedExperts(width, ff, experts, top, torch.float32, "cpu", activation="silu_gated" if gated else "squared_relu")
+    rows = 2 * ff if gated else ff
+    layer.gate_up, layer.down = torch.empty((experts, rows, width), device="meta"), torch.empty((experts, width, ff), device="meta")
+    x = torch.empty((tokens, width), device="meta")
+
+    class Step:
+        host_cu_seqlens_q = [0, tokens]
+
+    for name, answer in {"expert_tiles_take": False, "expert_lines_take_f32": True, "experts_by_expert_take": True}.items():
+        monkeypatch.setattr(ops, name, lambda *a, answer=answer: answer)
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    assert layer._grouped(x, Step) == pays
