@@ -1114,10 +1114,11 @@ extern "C" int mi_expert_lines_f32_take(const void* weight, int k_dim, int64_t e
 // mode 1 (silu gated): weight [experts, 2 * features, k_dim], out[pair, f] = silu(gate_f . row) * (up_f . row) with
 // the row of pair p at src[p / src_div]; mode 2: weight [experts, features, k_dim], out[pair, f] =
 // relu(pair_weight[pair] * (w_f . row))^2 (pair_weight null: 1); mode 0: out[pair, f] = w_f . row.
-// many_rows = 1 (bfloat16 with k_dim a multiple of 32 only): blocks of 64 features that take 64 rows a pass.
+// form = 1: in bfloat16 with k_dim a multiple of 32 blocks of 64 features that take 64 rows a pass, in float32 four rows a pass also where
+// whole lines are taken.
 extern "C" int mi_expert_rows(int dtype, int mode, const void* src, int64_t src_stride, int src_div, const void* weight,
                               const int* listed, const int* first, const float* pair_weight, void* out, int64_t out_stride,
-                              int experts, int k_dim, int features, int many_rows, hipStream_t stream) {
+                              int experts, int k_dim, int features, int form, hipStream_t stream) {
   MI_REQUIRE(experts > 0 && experts <= 65535 && k_dim > 0 && features > 0 && src_div > 0 && src_stride >= k_dim && out_stride >= features,
              "expert_rows: bad sizes experts=%d k=%d features=%d", experts, k_dim, features);
   MI_REQUIRE(dtype == MI_F32 || dtype == MI_BF16, "expert_rows: unknown dtype %d", dtype);
@@ -1149,7 +1150,7 @@ extern "C" int mi_expert_rows(int dtype, int mode, const void* src, int64_t src_
                                                       expert_stride, listed, first, pair_weight, (bf16_t*)out,        \
                                                       out_stride, k_dim, features)
     const bool lines = k_dim % 256 == 0 && (uintptr_t)weight % 128 == 0 && expert_stride < ((int64_t)1 << 30);  // (32-bit byte offsets)
-    if (many_rows) MI_BY_MODE(MI_TILES);
+    if (form) MI_BY_MODE(MI_TILES);
     else if (lines) MI_BY_MODE(MI_LINES);
     else MI_BY_MODE(MI_MFMA);
 #undef MI_TILES
@@ -1158,7 +1159,7 @@ extern "C" int mi_expert_rows(int dtype, int mode, const void* src, int64_t src_
     MI_CHECK_LAUNCH("expert_rows_mfma");
     return MI_OK;
   }
-  if (dtype == MI_F32 && mi_expert_lines_f32_take(weight, k_dim, expert_stride)) {
+  if (dtype == MI_F32 && form == 0 && mi_expert_lines_f32_take(weight, k_dim, expert_stride)) {
     dim3 blocks(ceil_div(features, mode == EXPERT_SILU_GATED ? 16 : 32), experts);
 #define MI_LINES_F32(MODE)                                                                                                     \
   expert_lines_f32_kernel<MODE><<<blocks, SEGMENTS * MI_WAVE, 0, stream>>>((const float*)src, src_stride, src_div, (const float*)weight, expert_stride, \

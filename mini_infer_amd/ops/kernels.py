@@ -3593,6 +3593,19 @@ def sorted_f32_experts_pay(pairs: int, experts: int, width: int, ff: int, gated:
     return one_by_one < 0.88 * blocks
 
 
+def f32_experts_by_fours(pairs: int, experts: int, k: int, features: int, gated: bool) -> bool:
+    """Whether a product of float32 experts in whole lines is made four of an expert's rows a pass all the same.  The matrix instruction takes 16 rows where an expert
+    has one or two, and reaches 4.0 to 4.6 TB/s of weights; four rows a pass reach 5.5 once a launch reads much (and have more blocks where one has few of 32
+    features).  Microseconds in lines / by fours, one product, random choices: 64 experts of 4096 x 2048 (gate and up), 12 / 67 pairs 94 / 81 and 300 / 248, 16 of
+    them, 24 pairs 90 / 82; 8 experts, 1 pair 15.8 / 17.4.  Over 7,081 measured products (1 to 1,600 pairs, K 256 to 4,096) lines alone take 0.756 of the time by fours and are 7 % slower in
+    1,210 of them, so 0.746 and 126 (the better one each time 0.734)."""
+    if pairs >= 3 * experts:
+        return False
+    used = experts * (1 - (1 - 1 / experts) ** pairs)
+    many_bytes = k > 512 and used * (2 if gated else 1) * features * k * 4 > 64e6
+    return many_bytes or not gated and k >= 1792 and used * -(-features // 32) < 128
+
+
 def expert_tile_cuts(counts: list[int], weight_rows: int, k: int, cus: int = WHOLE_DEVICE_CUS) -> list[tuple[int, int, int, int]]:
     """For each expert with `counts` pairs: the full tiles of 256 of them, the tiles behind those, the pairs in each of these and the rows of
     their form, in a launch of the tiles staged through LDS with `weight_rows` (gate and up together) of `k` elements an expert."""
@@ -3648,7 +3661,6 @@ def experts_by_expert(
         tiles = expert_tiles_for(x, pairs, experts, ff)
     elif tiles not in EXPERT_TILES or (tiles == "lds" and not expert_tiles_take(x, ff)):
         raise KernelShapeError(f"experts_by_expert: tiles {tiles!r} for rows of {width} and {ff} {x.dtype}")
-    many = int(tiles == "direct")
     if tiles == "lds":
         plan = lists.plan
         if plan is None:
@@ -3659,10 +3671,13 @@ def experts_by_expert(
         library.check(lib.mi_expert_tiles(0, _ptr(act), ff, 1, _ptr(down), _ptr(listed), _ptr(plan), None, _ptr(made),
                                           width, pairs, experts, ff, width, _stream()))
     else:
+        forms = [int(tiles == "direct")] * 2
+        if x.dtype == torch.float32:
+            forms = [int(f32_experts_by_fours(pairs, experts, width, ff, mode == 1)), int(f32_experts_by_fours(pairs, experts, ff, width, False))]
         library.check(lib.mi_expert_rows(code, mode, _ptr(x), x.stride(0), top, _ptr(gate_up), _ptr(listed), _ptr(first),
-                                         _ptr(on_input), _ptr(act), ff, experts, width, ff, many, _stream()))
+                                         _ptr(on_input), _ptr(act), ff, experts, width, ff, forms[0], _stream()))
         library.check(lib.mi_expert_rows(code, 0, _ptr(act), ff, 1, _ptr(down), _ptr(listed), _ptr(first), None, _ptr(made),
-                                         width, experts, ff, width, many, _stream()))
+                                         width, experts, ff, width, forms[1], _stream()))
     if not combine:
         return SummedRows(made, top) if on_output is None else WeightedRows(made, weights)
     rows = ExpertRows(made, chosen, on_output, x, shared, shared_gate, experts, top)

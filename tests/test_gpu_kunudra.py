@@ -492,6 +492,25 @@ def test_rows_that_only_fill_a_step_choose_no_expert(rows, width, outputs, exper
         assert sorted(listed[first[e]:first[e + 1]]) == [p for p in range(rows * top) if not idle[p // top] and int(chosen.view(-1)[p]) == e]
 
 
+@pytest.mark.parametrize("activation", ["silu_gated", "squared_relu"])
+@pytest.mark.parametrize("width, ff, counts", [(2048, 512, [0, 1, 3, 4, 5]), (1056, 1792, [9, 0, 1])])
+def test_float32_experts_in_lines_and_by_fours(monkeypatch, activation, width, ff, counts):
+    """The two forms of a float32 product of few rows: each product one rounding of 64-bit sums, in other orders."""
+    from mini_infer_amd import ops
+    from mini_infer_amd.ops import kernels
+
+    rng = np.random.default_rng(width)
+    experts, rows, features = len(counts), sum(counts), 2 * ff if activation == "silu_gated" else ff
+    x, up, down = (dev(rng.standard_normal(shape) / np.sqrt(shape[-1]), torch.float32)
+                   for shape in ((rows, width), (experts, features, width), (experts, width, ff)))
+    chosen, w = ints(np.repeat(np.arange(experts), counts).tolist()).reshape(rows, 1), torch.ones((rows, 1), device=DEV)
+    made = []
+    for fours in (False, True):
+        monkeypatch.setattr(kernels, "f32_experts_by_fours", lambda *sizes, fours=fours: fours)
+        made.append(ops.experts_by_expert(x, up, down, chosen, w, activation=activation).double())
+    assert (made[0] - made[1]).norm() < 2 ** -22 * made[0].norm()
+
+
 # ---------------------------------------------------------------------------------------------
 # each mixer and each feed-forward alone in a one-layer model
 # ---------------------------------------------------------------------------------------------

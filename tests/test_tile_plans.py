@@ -192,3 +192,10 @@ def test_float32_experts_of_many_rows_are_sorted(monkeypatch, tokens, experts, t
         monkeypatch.setattr(ops, name, lambda *a, answer=answer: answer)
     monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
     assert layer._grouped(x, Step) == pays
+
+
+@pytest.mark.parametrize("pairs, experts, k, features, gated, fours", [
+    (1, 16, 2048, 2048, True, False), (12, 64, 2048, 2048, True, True), (24, 16, 2048, 2048, True, True), (47, 16, 2048, 2048, True, True), (48, 16, 2048, 2048, True, False),
+    (12, 64, 512, 8192, True, False), (2, 16, 2048, 512, False, True), (2, 16, 2048, 512, True, False), (2, 16, 1024, 512, False, False), (1, 1, 4096, 4096, False, True)])
+def test_which_float32_experts_are_read_for_four_rows(pairs, experts, k, features, gated, fours):
+    assert kernels.f32_experts_by_fours(pairs, experts, k, features, gated) == fours
