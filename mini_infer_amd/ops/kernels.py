@@ -639,9 +639,9 @@ SMALL_SUM_LAUNCH_MICROS = 2.0
 
 
 @functools.lru_cache(maxsize=8192)
-def small_product_plan(m: int, n: int, k: int, cus: int = WHOLE_DEVICE_CUS) -> tuple[int | None, int, int] | None:
-    """(form of `gemm_rows_bf16` or None, tile shape and ranges of K where its operands do not suit it) of a whole bfloat16 product of more rows than
-    `gemm_skinny_bf16` takes, where that is faster than what `tiles_for` says; None: as that says.
+def small_product_plan(m: int, n: int, k: int, cus: int = WHOLE_DEVICE_CUS, lines: bool = True) -> tuple[int | None, int, int] | None:
+    """(form of `gemm_rows_bf16` or None, tile shape and ranges of K) of a whole bfloat16 product of more rows than
+    `gemm_skinny_bf16` takes, where that is faster than what `tiles_for` says; None: as that says.  `lines`: whether the operands suit `gemm_rows_bf16`.
 
     Matrices of fewer than 8,000,000 elements up to 320 rows, which `tiles_for` leaves to the vendor library: microseconds there / so (more of them at
     the top of csrc/gemm_rows_bf16.hip), weights from memory, 3072 x 2048 at 128 / 192 / 256 / 320 rows 14.7 / 10.5, 21.5 / 12.6, 13.4 / 13.1, 13.5 / 13.2, 2048 x 2048
@@ -649,16 +649,27 @@ def small_product_plan(m: int, n: int, k: int, cus: int = WHOLE_DEVICE_CUS) -> t
     all of it: 1024 x 3072 at 96 / 256 rows 9.9 / 9.7 and 10.3 / 13.3, 2048 x 3072 10.9 / 11.4 and 16.0 / 13.7.  Up to 96 rows and 4,096 features larger ones too, cut
     where the sum's launch, 2 microseconds in a recorded step, is counted as what it takes: 3072 x 3072 at 64 rows 14.3 / 11.6, 4096 x 4096 at 96 17.9 /
     17.2.  Up to 32 rows those of more features in the forms of `gemm_rows_bf16`: 8192 x 3072 at 17 / 32 rows 17.1 / 13.0 and 17.9 / 15.1, 6144 x 3072 15.4 / 11.8 and 16.1 /
-    13.4, 8192 x 4096 18.7 / 15.5 and 20.1 / 17.5 (above, products with a rotation share their tiles with plain ones: `rotary_tiles_for`)."""
-    small = n * k < SMALL_PRODUCT
-    if not SKINNY_MAX_ROWS < m < TURNS_MIN_ROWS or small and m > 64 and k >= 3072:
+    13.4, 8192 x 4096 18.7 / 15.5 and 20.1 / 17.5 (above, products with a rotation share their tiles with plain ones: `rotary_tiles_for`).
+
+    Features that are no multiple of four are not cut, as ranges of them are written value by value (497 x 8192 at 29 rows 16.9 for the library's 9.2, 1434 x 3072 at 35
+    13.9 / 7.8), and with K from 3,072 on left to the library; where rows of W do not lie in whole lines, to it as well up to 32 rows (tiles up to 1.8
+    times as slow), and so are 512 to 2,047 values of K with fewer than 1,024 features, of which it makes 512 x 1024 at 18 rows in 5.7 and tiles in 7.6.  Of 7,011 measured
+    products (17 to 320 rows, 64 to 8,192 features and K) this takes 0.685 of the time by `tiles_for` alone and 12 are 7 %
+    slower (249 with cuts of any number of features)."""
+    small, fours = n * k < SMALL_PRODUCT, n % 4 == 0
+    if not SKINNY_MAX_ROWS < m < TURNS_MIN_ROWS or small and k >= 3072 and (m > 64 or not fours):
         return None
-    cut = small or n <= 4096 and m <= 96
+    cut = small or fours and n <= 4096 and m <= 96
     if not cut and m > SKINNY_WIDE_MAX_ROWS:
         return None
+    tiles, shape, ranges = _tiles_plan(m, n, k, False, 16 if fours or not small else 1, False, SMALL_SUM_LAUNCH_MICROS if cut else SUM_LAUNCH_MICROS,
+                                       m * n * 4 / SUM_BYTES_A_MICRO, cus)
+    if not lines:
+        if small and (not fours and m <= SKINNY_WIDE_MAX_ROWS or 512 <= k < 2048 and n < 1024):
+            return None
+        return (None, shape, ranges) if cut else None
     form, micros = ctypes.c_int(), ctypes.c_float()
     library.check(library.load().mi_gemm_rows_plan(m, n, k, cus, ctypes.addressof(form), ctypes.addressof(micros)))
-    tiles, shape, ranges = _tiles_plan(m, n, k, False, 16, False, SMALL_SUM_LAUNCH_MICROS if cut else SUM_LAUNCH_MICROS, m * n * 4 / SUM_BYTES_A_MICRO, cus)
     if ranges > 1 and not cut:
         tiles -= SUM_LAUNCH_MICROS - SMALL_SUM_LAUNCH_MICROS  # (the ranges are those of `tiles_for`)
     if micros.value < tiles:
@@ -832,10 +843,13 @@ def linear(x: torch.Tensor, weight: torch.Tensor, partial_ok: bool = False, stea
         return _turns(TURNS_NONE, x, weight, weight.shape[0])
     if not steady and x.dim() == 2 and x.shape[0] <= TILES_MAX_ROWS and _rows_of_bf16(x, weight):
         m, n = x.shape[0], weight.shape[0]
-        small = None if partial_ok else small_product_plan(m, n, x.shape[1], _compute_units(x.device))
-        if small is not None and small[0] is not None and _whole_lines(x, weight):
-            return _few_rows(small[0], x, weight)
-        plan = small[1:] if small is not None else tiles_for(m, n, x.shape[1], partial_ok, _compute_units(x.device))
+        cus = _compute_units(x.device)
+        small = None if partial_ok else small_product_plan(m, n, x.shape[1], cus)
+        if small is not None and small[0] is not None:
+            if _whole_lines(x, weight):
+                return _few_rows(small[0], x, weight)
+            small = small_product_plan(m, n, x.shape[1], cus, False)
+        plan = small[1:] if small is not None else tiles_for(m, n, x.shape[1], partial_ok, cus)
         if plan is not None:
             if plan[1] == 1:
                 return _tiles(0, x, weight, torch.empty((m, n), dtype=torch.bfloat16, device=x.device), n, *plan)

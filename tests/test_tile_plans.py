@@ -163,7 +163,20 @@ def test_tiles_of_rotary_products(m, n, k, made):
     (64, 2048, 3072, "cut"), (96, 2048, 3072, None), (64, 3072, 3072, "cut"), (97, 4096, 4096, None),                  # a longer K
     (17, 8192, 4096, "rows"), (32, 8192, 3072, "rows"), (33, 8192, 3072, None), (32, 28672, 4096, None)])             # more features
 def test_products_with_small_matrices(m, n, k, plan):
-    got = kernels.small_product_plan(m, n, k)
+    check_small_plan(m, n, k, plan)
+
+
+@pytest.mark.parametrize("m, n, k, lines, plan", [
+    (29, 497, 8192, True, None), (29, 496, 8192, True, "cut"), (35, 1434, 3072, True, None), (45, 2046, 2048, True, "rows"), (80, 3070, 2560, True, "whole"),
+    (200, 3071, 2048, True, "whole"), (64, 2730, 4096, True, None),                              # features that no range writes four at a time
+    (20, 512, 1024, False, None), (40, 512, 2000, False, None), (40, 512, 480, False, "whole"), (40, 1024, 1024, False, "whole"), (24, 2050, 1024, False, None),
+    (40, 2050, 1024, False, "whole"), (24, 2048, 1024, False, "whole"), (64, 3072, 3072, False, "cut"), (24, 8192, 3072, False, None)])  # rows of W off whole lines
+def test_products_with_small_matrices_that_are_not_multiples(m, n, k, lines, plan):
+    check_small_plan(m, n, k, plan, lines)
+
+
+def check_small_plan(m, n, k, plan, lines=True):
+    got = kernels.small_product_plan(m, n, k, lines=lines)
     made = None if got is None else "rows" if got[0] is not None else "whole" if got[2] == 1 else "cut"
     assert made == plan
 
