@@ -51,7 +51,14 @@ struct PairedHow<2> {
 // 176, 182, 202, 219 / 173, 178, 196, 218, 64128 x 6144 145, 154, 169, 174 / 125, 131, 145, 146.  (Of 16384 x 3072, 28672 x 5120 and 128256 x 1024 the same or 3 % more; five
 // or eight steps later for one: 128256 x 4096 189 and 176.  Ranges of K, which begin apart: the same.  Plain whole products and those with a rotation give the
 // same bits as one another, which have their rows of W in other tiles: from the beginning.)
-static bool turned(int kind, int64_t ldw) { return kind >= 2 && ldw % 2048 == 0; }
+//
+// Not with so few tiles that the channels are not what they wait for (1,024 features x 4096 at 66 rows 14.8 / 15.9, 512 x 8192 at 109 25.2 / 27.5), not with several
+// tiles of rows to few of features, whose blocks read the same rows of W, and not in tiles 64 wide where rows of W are an odd multiple of 8 KB apart, whose
+// halves of 32 features then meet again (4,096 features x 4096 at 33 / 48 rows 17.6 / 19.7 and 18.9 / 21.4, 8,192 at 33 / 96 1.15 times as long, 18,432 1.2; in tiles
+// 128 wide 0.8 to 0.95).
+static bool turned(int kind, int64_t ldw, int tile_width, int feature_tiles) {
+  return kind >= 2 && ldw % 2048 == 0 && feature_tiles > 128 && !(tile_width == 64 && ldw % 8192 == 4096);
+}
 
 // (the second bound: two blocks a CU where LDS holds two)
 template <class T, int PAIRED, bool ONCE, bool ODD, bool ROUND, bool EIGHTHS = false>
@@ -148,7 +155,7 @@ static void gemm_tiles_launch(const GemmTilesLaunch& l) {
     if (row_tiles > 1) kernel = gemm_tiles_kernel<T, PAIRED, false, ODD, false>;
   }
   if constexpr (!ODD && PAIRED != PAIRED_ROTARY) {
-    if (turned(l.kind, l.ldw)) {
+    if (turned(l.kind, l.ldw, T::BN, feature_tiles)) {
       kernel = gemm_tiles_kernel<T, PAIRED, true, false, true, EIGHTHS>;
       if constexpr (!EIGHTHS) {
         if (row_tiles > 1) kernel = gemm_tiles_kernel<T, PAIRED, false, false, true>;

@@ -293,8 +293,23 @@ def test_tiles_that_begin_a_step_later_than_their_neighbours(shape, k):
     from mini_infer_amd.ops import kernels
 
     bm, bn = kernels.tile_size(shape)
-    m, n = bm + 3, bn * (35 if bn <= 64 else 5)
-    a, w = _rand(m, k, dtype=torch.bfloat16, seed=71), _rand(2 * n, 2048, dtype=torch.bfloat16, seed=72, scale=0.05)[:, :k]
+    check_tiles_of_rows_4_kb_apart(shape, bm + 3, bn * (35 if bn <= 64 else 5), k)
+
+
+@pytest.mark.parametrize("shape", range(14))
+@pytest.mark.parametrize("k, row_tiles, feature_tiles", [(2048, 1, 129), (2048, 2, 131), (256, 1, 200), (64, 1, 210), (4096, 1, 130)])
+def test_many_tiles_that_begin_a_step_later_than_their_neighbours(shape, k, row_tiles, feature_tiles):
+    """On the side of the rule where they do (some of these, by the width and the rows of their tiles, begin like the others)."""
+    from mini_infer_amd.ops import kernels
+
+    bm, bn = kernels.tile_size(shape)
+    check_tiles_of_rows_4_kb_apart(shape, bm * row_tiles - 1, bn // 2 * feature_tiles - 3, k, stride=max(k, 2048))
+
+
+def check_tiles_of_rows_4_kb_apart(shape, m, n, k, stride=2048):
+    from mini_infer_amd.ops import kernels
+
+    a, w = _rand(m, k, dtype=torch.bfloat16, seed=71), _rand(2 * n, stride, dtype=torch.bfloat16, seed=72, scale=0.05)[:, :k]
     exact = a.double() @ w.double().T
     # (as test_products_in_tiles: sums of k terms, one rounding to 8 bits; in the activation half a unit of each factor and of the result)
     summed = 2.0 ** -23 * (k + 1) * (a.double().abs() @ w.double().abs().T) + 1e-30
