@@ -55,7 +55,10 @@ def bucket_of(value: int, minimum: int = 1) -> int:
 def mixed_bucket_of(value: int, minimum: int = 1) -> int:
     """The bucket of a mixed step's tokens or requests: a power of two, or above 32 one and a half of one.  Every row that only fills its bucket goes through
     all layers: 84 tokens in 96 rows instead of 128 are 5,599 -> 4,864 us in float32 at 1B widths, 80 of two prompts at 8B 5,276 -> 4,771, 33 of
-    one in 48 instead of 64 4,232 -> 4,049, 160 in 192 instead of 256 at 3B 3,962 -> 3,681."""
+    one in 48 instead of 64 4,232 -> 4,049, 160 in 192 instead of 256 at 3B 3,962 -> 3,681.
+
+    What they cost: the first step of a bucket takes 5 to 9 ms longer, and its graph keeps 22 to 54 MiB (Llama) or 24 to 90 (Zekonex) at 3B widths for as long as
+    the runner.  Steps of every size are recorded in at most 8 buckets of tokens and 12 of requests for each width of the tables, of powers of two alone in 5 and 9."""
     bucket = bucket_of(value, minimum)
     return bucket // 4 * 3 if bucket > 32 and value <= bucket // 4 * 3 else bucket
 
