@@ -2524,49 +2524,50 @@ def delta_state_shape(heads: int, dim: int, vdim: int) -> tuple[int, int, int]:
 
 
 # Microseconds of a recurrence over a step's rows with keys of up to so many columns: token by token (the launches, a request and a
-# token on a full chip, a token of the longest portion) and in chunks of 32 (the launches, a request on a full chip, a chunk of the
-# longest portion, a request of one token on a full chip).  Fitted to 1,508 measured pairs: 1 to 100 requests of 8 to 512 tokens, single tokens beside one portion, 4 to 80
-# heads of 64 to 512 columns; half of the times are within 5 %.  (A request's share of the decays token by token: fitted to 8 to 80 single
-# tokens of 16 to 64 heads since their blocks spread over the XCDs; beside a portion these expect 10 to 25 % more than is measured.  Single tokens in chunks: 210 steps of 4 to 100
-# beside a portion of 32 to 600, within 7 %.)
+# token on a full chip, a token of the longest portion) and in chunks of 32 (the launches, a request of several tokens on a full chip, a chunk of the
+# longest portion, a request of one token on a full chip, a portion's chunk on a full chip).  Fitted to 6,000 measured pairs of the kernels as they are: 1 to 100 requests
+# of 8 to 4,096 tokens, single tokens beside one portion and beside several, 4 to 80 heads of 64 to 512 columns, keys of 48 to 256, shared by 1 to 4 heads of a delta rule and by up to
+# all of a decay per head; states from memory; of the times token by token 41 % are within 5 %, of those in chunks 36 %.
 _SCAN_TIMES = {
-    ("delta", 64): (6.95, 0.89, 0.093, 0.288, 18.3, 2.33, 1.82, 0.778),
-    ("delta", 128): (8.39, 2.13, 0.161, 0.428, 21, 3.14, 2.26, 0.851),
-    ("delta", 256): (7.82, 3.4, 0.288, 0.62, 24.7, 7.38, 4.32, 1.56),
-    ("per_head", 64): (3.85, 0.33, 0.0355, 0.252, 13.4, 0.971, 1.13, 0.419),
-    ("per_head", 128): (3.43, 0.61, 0.0864, 0.303, 14, 1.68, 1.52, 0.787),
-    ("per_head", 256): (2.44, 1.65, 0.19, 0.472, 16.4, 3.59, 2.36, 1.36),
-    ("per_channel", 64): (3.98, 0.32, 0.0473, 0.267, 17.5, 1.57, 1.05, 0.563),
-    ("per_channel", 128): (3.28, 0.775, 0.121, 0.348, 23.4, 2.35, 1.71, 0.751),
-    ("per_channel", 256): (1.11, 2.1, 0.256, 0.58, 31.6, 5.51, 3.08, 1.49),
+    ("delta", 64): (5.69, 1.08, 0.109, 0.312, 17.2, 1.73, 1.72, 0.751, 2.1),
+    ("delta", 128): (6.41, 2.12, 0.208, 0.431, 19.6, 2.49, 2.32, 1.19, 3.21),
+    ("delta", 256): (6.86, 3.07, 0.333, 0.638, 24.6, 5.23, 4.01, 2.39, 6.53),
+    ("per_head", 64): (3.2, 0.336, 0.0448, 0.251, 10.4, 0.867, 1.11, 0.446, 0.787),
+    ("per_head", 128): (3.26, 0.752, 0.113, 0.284, 12.1, 1.42, 1.41, 0.876, 1.39),
+    ("per_head", 256): (3.97, 1.68, 0.228, 0.443, 15.8, 3.08, 2.23, 1.74, 2.74),
+    ("per_channel", 64): (2.96, 0.374, 0.0557, 0.273, 16.0, 0.994, 1.03, 0.669, 1.0),
+    ("per_channel", 128): (3.03, 0.928, 0.162, 0.341, 22.3, 1.77, 1.5, 1.17, 1.92),
+    ("per_channel", 256): (3.94, 1.76, 0.388, 0.559, 32.6, 4.11, 2.9, 2.41, 5.19),
 }
 
 
 def scan_times(kind: str, tokens: int, requests: int, longest: int | None, heads: int, dim: int, vdim: int) -> tuple[float, float]:
     """About how many microseconds a recurrence takes token by token and in chunks.  A long portion is a chain of tokens (0.3 to 0.45
-    microseconds each at keys of 128) or of chunks (1.5 to 2.3); a portion's chunk costs the same with fewer tokens in it, a single token less.  `longest`: tokens
-    of the step's longest portion; None (a recorded step): as if it were one portion beside single tokens, a scheduler's ordinary step."""
-    launches, request, token, chain, chunk_launches, chunk_request, chunk_chain, chunk_single = _SCAN_TIMES[kind, 64 if dim <= 64 else 128 if dim <= 128 else 256]
+    microseconds each at keys of 128) or of chunks (1.4 to 2.3), many of them fill the chip; a portion's chunk costs the same with fewer tokens in it, a single token
+    less.  `longest`: tokens of the step's longest portion; None (a recorded step): as if it were one portion beside single tokens, a scheduler's ordinary step."""
+    launches, request, token, chain, chunk_launches, chunk_request, chunk_chain, chunk_single, chunk = _SCAN_TIMES[kind, 64 if dim <= 64 else 128 if dim <= 128 else 256]
     longest = max(1, tokens - requests + 1) if longest is None else longest
     full = heads * -(-vdim // 16) / 256  # of the chip, by one request
     walked = launches + request * requests * full + max(token * tokens * full, chain * longest)
     if tokens <= requests:  # (single tokens: there are launches for these)
         return walked, math.inf
-    # (requests of several tokens: the longest, and as many others as there are tokens beyond one for each)
-    singles = requests - 1 - max(0, min(requests - 1, tokens - longest - (requests - 1)))
-    return walked, chunk_launches + (chunk_request * (requests - singles) + chunk_single * singles) * full + chunk_chain * longest / 32
+    # (requests of several tokens: the longest, and as few others as hold the tokens beyond one for each)
+    more = tokens - longest - (requests - 1)
+    singles = requests - 1 - max(0, min(requests - 1, -(-more // max(1, longest - 1))))
+    chunks = max(chunk_chain * -(-longest // 32), chunk * (tokens - singles) / 32 * full)
+    return walked, chunk_launches + (chunk_request * (requests - singles) + chunk_single * singles) * full + chunks
 
 
 def chunked_scan_pays(walked: float, chunked: float, widest: int) -> bool:
     """Whether a recurrence over a step's rows is taken 32 tokens at a time on the matrix cores rather than token by token, from
-    what `scan_times` expects of the two.  At this margin 1 of 1,508 measured steps is slower than token by token (6 %), and
-    together they are 1.17 times as fast (1.19 with the better one each time).  Microseconds, token by token against in chunks, of
-    the delta rule with 32 heads of 128 x 128: 2,048 tokens 887 / 181, 70 tokens 39 / 29, 256 beside 16 single tokens 160 / 56, 64 beside 31 97 / 56, 16
-    portions of 32 116 / 74, not taken: 4 of 20 33 / 33, 16 of 8 60 / 70, 100 of 4 243 / 331; a decay per head, 48 heads of 128 x 64:
-    2,048 tokens 705 / 117, 16 portions of 32 43 / 36, not taken: 16 of 16 25 / 36; per channel, 12 heads of 128 x 256: 2,048 tokens
-    818 / 125, 32 portions of 32 112 / 75, not taken: 4 of 64 29 / 37.  `widest`: values from one row to the next of the widest operand
+    what `scan_times` expects of the two.  At this margin 75 of the 6,000 measured steps are slower than token by token (at worst 1.5 times), and
+    as a geometric mean they are 1.540 times as fast (1.552 with the better one each time).  Microseconds, token by token against in chunks, of
+    the delta rule with 32 heads of 128 x 128: 2,048 tokens 891 / 206, 70 tokens 38 / 28, 256 beside 16 single tokens 168 / 60, 64 beside 31 110 / 60, 16
+    portions of 32 132 / 94, not taken: 4 of 20 35 / 35, 16 of 8 65 / 82, 100 of 4 264 / 399; a decay per head, 48 heads of 128 x 64:
+    2,048 tokens 730 / 113, 16 portions of 32 54 / 36, not taken: 16 of 16 32 / 36; per channel, 12 heads of 128 x 256: 2,048 tokens
+    835 / 129, 32 portions of 32 135 / 83, not taken: 4 of 64 35 / 37.  `widest`: values from one row to the next of the widest operand
     or result; the chunks' kernels reach over their 32 rows in 32 bits."""
-    return chunked < 0.85 * walked and widest < 2**24
+    return chunked < 0.9 * walked and widest < 2**24
 
 
 def gated_delta(

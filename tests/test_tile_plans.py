@@ -212,3 +212,13 @@ def test_float32_experts_of_many_rows_are_sorted(monkeypatch, tokens, experts, t
     (12, 64, 512, 8192, True, False), (2, 16, 2048, 512, False, True), (2, 16, 2048, 512, True, False), (2, 16, 1024, 512, False, False), (1, 1, 4096, 4096, False, True)])
 def test_which_float32_experts_are_read_for_four_rows(pairs, experts, k, features, gated, fours):
     assert kernels.f32_experts_by_fours(pairs, experts, k, features, gated) == fours
+
+
+@pytest.mark.parametrize("kind, dim, heads, vdim, requests, tokens, longest, walked, chunked", [
+    ("delta", 96, 31, 256, 59, 208, 115, 325, 155), ("per_channel", 200, 22, 512, 18, 302, 265, 408, 188), ("delta", 64, 14, 256, 39, 328, 218, 123, 57),
+    ("per_head", 128, 15, 256, 29, 532, 191, 108, 60), ("per_head", 128, 48, 64, 1, 2048, 2048, 730, 113), ("delta", 128, 32, 128, 32, 95, 64, 110, 60),
+    ("per_head", 128, 48, 64, 16, 256, 16, 32, 36), ("delta", 128, 32, 128, 100, 400, 4, 264, 399), ("delta", 128, 32, 128, 16, 128, 8, 65, 82)])
+def test_scans_go_the_way_that_was_measured_to_be_faster(kind, dim, heads, vdim, requests, tokens, longest, walked, chunked):
+    """Single tokens beside one portion and beside several, of which only the longest is known, prompts, and short portions (microseconds as measured)."""
+    expected = kernels.scan_times(kind, tokens, requests, longest, heads, dim, vdim)
+    assert kernels.chunked_scan_pays(*expected, heads * vdim) == (chunked < walked)
