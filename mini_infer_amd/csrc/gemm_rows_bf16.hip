@@ -163,9 +163,8 @@ extern "C" int mi_gemm_rows_take(const void* a, int64_t lda, const void* w, int6
              : 0;
 }
 
-// Rows and features of a form (0: there is none of that number).
+// Rows of a form (0: there is none of that number).
 extern "C" int mi_gemm_rows_rows(int form) { return form >= 0 && form < FORM_COUNT ? FORMS[form].rows : 0; }
-extern "C" int mi_gemm_rows_features(int form) { return form >= 0 && form < FORM_COUNT ? FORMS[form].features : 0; }
 
 extern "C" int mi_gemm_rows_bf16(int form, const void* a, int64_t lda, const void* w, int64_t ldw, void* out, int64_t ldc, int m, int n, int k,
                                  hipStream_t stream) {

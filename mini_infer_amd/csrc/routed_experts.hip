@@ -916,9 +916,9 @@ __global__ __launch_bounds__(256) void weighted_squared_relu_kernel(const T* __r
 }  // namespace
 
 // token_request, slots (both or neither): tokens of requests without a slot get the choice `outputs`, which is no expert, with weight 0.
-extern "C" int mi_route_top_k_of(int dtype, const void* x, int64_t x_stride, const float* router, const float* correction,
-                                 const float* gate_row, int* chosen, float* weights, float* shared_gate, const int* token_request, const int* slots,
-                                 int num_tokens, int width, int outputs, int top, float route_scale, int scores, hipStream_t stream) {
+extern "C" int mi_route_top_k(int dtype, const void* x, int64_t x_stride, const float* router, const float* correction,
+                              const float* gate_row, int* chosen, float* weights, float* shared_gate, const int* token_request, const int* slots,
+                              int num_tokens, int width, int outputs, int top, float route_scale, int scores, hipStream_t stream) {
   MI_REQUIRE((token_request == nullptr) == (slots == nullptr), "route_top_k: the tokens' requests come with their slots");
   const StepOwners owners = {token_request, slots};
   MI_REQUIRE(num_tokens >= 0 && width > 0 && x_stride >= width, "route_top_k: bad sizes tokens=%d width=%d", num_tokens, width);
@@ -956,13 +956,6 @@ extern "C" int mi_route_top_k_of(int dtype, const void* x, int64_t x_stride, con
 #undef MI_ROUTE
   MI_CHECK_LAUNCH("route_top_k");
   return MI_OK;
-}
-
-extern "C" int mi_route_top_k(int dtype, const void* x, int64_t x_stride, const float* router, const float* correction,
-                              const float* gate_row, int* chosen, float* weights, float* shared_gate, int num_tokens,
-                              int width, int outputs, int top, float route_scale, int scores, hipStream_t stream) {
-  return mi_route_top_k_of(dtype, x, x_stride, router, correction, gate_row, chosen, weights, shared_gate, nullptr, nullptr, num_tokens, width, outputs,
-                           top, route_scale, scores, stream);
 }
 
 // act: [num_tokens * top, ff]; rows of pairs whose expert is an identity expert are not written.  mode: 1 silu
@@ -1064,9 +1057,9 @@ extern "C" int mi_route_few_takes(int num_tokens, int width, int outputs, int to
          outputs > 0 && outputs <= MI_ROUTER_MAX_OUTPUTS;
 }
 
-// mi_route_top_k_of and mi_expert_sort for few bfloat16 tokens in two launches; `logits`: scratch
+// mi_route_top_k and mi_expert_sort for few bfloat16 tokens in two launches; `logits`: scratch
 // [num_tokens, outputs + (gate row ? 1 : 0)] floats.
-extern "C" int mi_route_few_of(const void* x, int64_t x_stride, const float* router, const float* correction, const float* gate_row,
+extern "C" int mi_route_few(const void* x, int64_t x_stride, const float* router, const float* correction, const float* gate_row,
                             float* logits, int* chosen, float* weights, float* shared_gate, int* listed, int* first, const int* token_request,
                             const int* slots, int num_tokens, int width, int outputs, int experts, int top, float route_scale, int scores,
                             hipStream_t stream) {
@@ -1087,14 +1080,6 @@ extern "C" int mi_route_few_of(const void* x, int64_t x_stride, const float* rou
       StepOwners{token_request, slots});
   MI_CHECK_LAUNCH("route_list");
   return MI_OK;
-}
-
-extern "C" int mi_route_few(const void* x, int64_t x_stride, const float* router, const float* correction, const float* gate_row,
-                            float* logits, int* chosen, float* weights, float* shared_gate, int* listed, int* first,
-                            int num_tokens, int width, int outputs, int experts, int top, float route_scale, int scores,
-                            hipStream_t stream) {
-  return mi_route_few_of(x, x_stride, router, correction, gate_row, logits, chosen, weights, shared_gate, listed, first, nullptr, nullptr, num_tokens, width,
-                         outputs, experts, top, route_scale, scores, stream);
 }
 
 // Rows a block keeps in LDS at a time for rows of k_dim elements (0: such rows do not fit).

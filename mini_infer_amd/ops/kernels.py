@@ -3446,13 +3446,13 @@ def route_top_k(
         if (x.dtype == torch.bfloat16 and lib.mi_route_few_takes(tokens, width, outputs, int(top)) and x.stride(0) % 4 == 0
                 and x.data_ptr() % 8 == 0 and router.data_ptr() % 16 == 0 and (gate_row is None or gate_row.data_ptr() % 16 == 0)):
             logits = torch.empty((tokens, outputs + (gate_row is not None)), dtype=torch.float32, device=x.device)
-            library.check(lib.mi_route_few_of(
+            library.check(lib.mi_route_few(
                 _ptr(x), x.stride(0), _ptr(router), _ptr(correction), _ptr(gate_row), _ptr(logits), _ptr(chosen), _ptr(weights),
                 _ptr(gates), _ptr(lists.listed), _ptr(lists.first), _ptr(token_request), _ptr(slots), tokens, width, outputs, experts, int(top), float(route_scale),
                 ROUTER_SCORES.index(scores), _stream()))
             return chosen, weights, gates, lists
     library.check(
-        library.load().mi_route_top_k_of(
+        library.load().mi_route_top_k(
             _dtype_code(x), _ptr(x), x.stride(0), _ptr(router), _ptr(correction), _ptr(gate_row), _ptr(chosen), _ptr(weights),
             _ptr(gates), _ptr(token_request), _ptr(slots), tokens, width, outputs, int(top), float(route_scale), ROUTER_SCORES.index(scores), _stream(),
         )

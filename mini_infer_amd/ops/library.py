@@ -14,7 +14,7 @@ from pathlib import Path
 from mini_infer_amd.exceptions import ExtensionMissingError, KernelShapeError
 from mini_infer_amd.ops import build as _build
 
-ABI_VERSION = 55
+ABI_VERSION = 56
 
 _lib: ctypes.CDLL | None = None
 _lib_path: Path | None = None
@@ -46,7 +46,6 @@ _SIGNATURES: dict[str, list] = {
     "mi_gemm_rows_plan": [c_int, c_int, c_int, c_int, _P, _P],
     "mi_gemm_rows_take": [_P, c_int64, _P, c_int64, c_int, c_int, c_int],
     "mi_gemm_rows_rows": [c_int],
-    "mi_gemm_rows_features": [c_int],
     "mi_gemm_rows_bf16": [c_int, _P, c_int64, _P, c_int64, _P, c_int64, c_int, c_int, c_int, _P],
     "mi_gemm_tiles_plan": [c_int, c_int, c_int, c_int, c_int, c_int, c_float, c_float, c_int, _P, _P, _P],
     "mi_gemm_tiles_rows": [c_int],
@@ -171,13 +170,9 @@ _SIGNATURES: dict[str, list] = {
         c_int, _P, c_int64, _P, _P, _P, c_int64, _P, _P, _P, _P, c_int, c_int, c_int, c_int, c_int, c_int, c_int, c_int,
         c_float, _P,
     ],
-    "mi_route_top_k": [c_int, _P, c_int64, _P, _P, _P, _P, _P, _P, c_int, c_int, c_int, c_int, c_float, c_int, _P],
-    "mi_route_top_k_of": [c_int, _P, c_int64, _P, _P, _P, _P, _P, _P, _P, _P, c_int, c_int, c_int, c_int, c_float, c_int, _P],
+    "mi_route_top_k": [c_int, _P, c_int64, _P, _P, _P, _P, _P, _P, _P, _P, c_int, c_int, c_int, c_int, c_float, c_int, _P],
     "mi_route_few_takes": [c_int, c_int, c_int, c_int],
     "mi_route_few": [
-        _P, c_int64, _P, _P, _P, _P, _P, _P, _P, _P, _P, c_int, c_int, c_int, c_int, c_int, c_float, c_int, _P,
-    ],
-    "mi_route_few_of": [
         _P, c_int64, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P, c_int, c_int, c_int, c_int, c_int, c_float, c_int, _P,
     ],
     "mi_expert_gate_up": [c_int, c_int, _P, c_int64, _P, _P, _P, _P, c_int, c_int, c_int, c_int, c_int, _P],

@@ -14,7 +14,7 @@ from mini_infer_amd.ops import library
 # version -> digest of every entry point's argument types
 DIGESTS = {37: "19d70346842e0dd7", 38: "5f985cd6095e4c7f", 39: "18d3fc0198a35211", 40: "6851cd991bfce4b8", 41: "9803e53b3110fced", 42: "d01bdc89bd271a04", 43: "613ab1a77867ce37", 44: "2a63e0010ae073e1",
            45: "f6d5abd47b7311f0", 46: "bc507a4251d57fa7", 47: "eefedaa760aa714e", 48: "8e751a64dde672ba", 49: "550e0b8ef907056e",
-           50: "80c3c74b33a8dc1c", 51: "60445bc43334f58b", 52: "4d1ac4af3a9083a1", 53: "2bbae5280632fa47", 54: "146144b8444c2820", 55: "21fcb354686890c1"}
+           50: "80c3c74b33a8dc1c", 51: "60445bc43334f58b", 52: "4d1ac4af3a9083a1", 53: "2bbae5280632fa47", 54: "146144b8444c2820", 55: "21fcb354686890c1", 56: "1165b637a929ca89"}
 
 
 def test_the_version_changes_with_the_arguments():
