@@ -371,11 +371,12 @@ __device__ __forceinline__ void decay_scan_columns(const ScanArgs& p, int b, int
 // 16 heads of 128 x 256 254 / 66.  Heads go round before columns: a head's column blocks then share an XCD's L2 (512 tokens of 64 heads 144 us, 164
 // the other way).
 // G: column blocks that a single token's block takes together (the other G - 1 leave at once); where there are enough blocks for that, launch_scan.
+// first_block: of this launch (a launch has no more than 2^32 threads).
 template <typename T, int MODE, int R, int L, int G>
-__global__ __launch_bounds__(256) void decay_scan_kernel(ScanArgs p, int requests) {
+__global__ __launch_bounds__(256) void decay_scan_kernel(ScanArgs p, int requests, uint32_t first_block) {
   constexpr int COLS = 256 / L;
-  const int each = p.heads * ((p.vdim + COLS - 1) / COLS);
-  const int b = requests - 1 - (int)(blockIdx.x / each), rest = (int)(blockIdx.x % each);
+  const uint32_t each = p.heads * ((p.vdim + COLS - 1) / COLS), at = first_block + blockIdx.x;
+  const int b = requests - 1 - (int)(at / each), rest = (int)(at % each);
   const int head = rest % p.heads, col_block = rest / p.heads;
   if constexpr (MODE == DECAY_PER_HEAD) {
     const int first = p.cu[b];
@@ -396,12 +397,14 @@ inline void scan_shape(int dim, int* rows, int* lanes) {
   else *rows = 16, *lanes = 16;
 }
 
+constexpr int64_t MOST_BLOCKS = ((int64_t)1 << 24) - 1;  // of 256 threads
+
 template <typename T, int MODE>
 int launch_scan(ScanArgs p, int tokens, int requests, hipStream_t stream) {
   int rows, lanes;
   scan_shape(p.dim, &rows, &lanes);
   const int64_t grid = (int64_t)requests * p.heads * ceil_div(p.vdim, 256 / lanes);
-  MI_REQUIRE(grid < ((int64_t)1 << 31), "decay_scan: %lld blocks are too many", (long long)grid);
+  MI_REQUIRE(grid < ((int64_t)1 << 32), "decay_scan: %lld blocks are too many", (long long)grid);
   constexpr int TOGETHER = MODE == DECAY_PER_HEAD ? 4 : 1;
   // (two rounds of what the CUs hold; 24 requests of 32 heads of 64 columns, 3,072 blocks, take the same either way.  Beside a long portion, whose
   // chain the larger blocks hold up, one: 38 tokens beside 73, a step of 12 layers 2,910 / 2,928 us.)
@@ -416,16 +419,19 @@ int launch_scan(ScanArgs p, int tokens, int requests, hipStream_t stream) {
   };
   p.tokens_alone = p.dim % rows == 0 && in_pieces(p.q, p.q_stride, p.q_col) && in_pieces(p.k, p.k_stride, p.k_col) &&
                    (sizeof(T) == 2 || (together && p.dim > 64));
-#define MI_SCAN(RR, LL)                                                                                               \
-  do {                                                                                                                \
-    if (together) decay_scan_kernel<T, MODE, RR, LL, TOGETHER><<<(unsigned)grid, 256, 0, stream>>>(p, requests);      \
-    else decay_scan_kernel<T, MODE, RR, LL, 1><<<(unsigned)grid, 256, 0, stream>>>(p, requests);                      \
+#define MI_SCAN(RR, LL)                                                                                                    \
+  do {                                                                                                                     \
+    if (together) decay_scan_kernel<T, MODE, RR, LL, TOGETHER><<<blocks, 256, 0, stream>>>(p, requests, (uint32_t)first);  \
+    else decay_scan_kernel<T, MODE, RR, LL, 1><<<blocks, 256, 0, stream>>>(p, requests, (uint32_t)first);                  \
   } while (0)
-  if (rows == 4) MI_SCAN(4, 4);
-  else if (rows == 8 && lanes == 4) MI_SCAN(8, 4);
-  else if (rows == 8 && lanes == 8) MI_SCAN(8, 8);
-  else if (rows == 8 && lanes == 16) MI_SCAN(8, 16);
-  else MI_SCAN(16, 16);
+  for (int64_t first = 0; first < grid; first += MOST_BLOCKS) {
+    const unsigned blocks = (unsigned)min(MOST_BLOCKS, grid - first);
+    if (rows == 4) MI_SCAN(4, 4);
+    else if (rows == 8 && lanes == 4) MI_SCAN(8, 4);
+    else if (rows == 8 && lanes == 8) MI_SCAN(8, 8);
+    else if (rows == 8 && lanes == 16) MI_SCAN(8, 16);
+    else MI_SCAN(16, 16);
+  }
 #undef MI_SCAN
   MI_CHECK_LAUNCH("decay_scan");
   return MI_OK;

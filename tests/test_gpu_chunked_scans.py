@@ -506,6 +506,27 @@ def test_decay_scan_of_single_tokens_gives_the_bits_of_portions(monkeypatch, hea
     assert torch.equal(single[:-1], whole[:-1])
 
 
+def test_decay_scan_of_more_blocks_than_a_launch_holds():
+    """257 requests of 65,535 heads are 2^24 blocks and more: the same as in two steps."""
+    from mini_infer_amd import ops
+
+    heads, dim, vdim, requests = 65535, 12, 1, 257
+    g = torch.Generator(device=DEV).manual_seed(41)
+    qk, v, gate = (torch.randn(requests, n, generator=g, device=DEV).bfloat16() for n in (2 * dim, heads * vdim, heads))
+    bias, rate = torch.zeros(heads, device=DEV), torch.zeros(heads, device=DEV)
+    state = _state(g, 1, ops.decay_state_shape(heads, dim, vdim), dim)
+    slots = torch.full((requests,), -1, dtype=torch.int32, device=DEV)
+    slots[0], slots[200] = 0, 1
+
+    def scan(at, end, into):
+        return ops.decay_scan(qk[at:end], 0, qk[at:end], dim, v[at:end], 0, gate[at:end], 0, bias, into, _boundaries([1] * (end - at)), slots[at:end].contiguous(),
+                              heads=heads, groups=1, dim=dim, vdim=vdim, per_head=True, rate=rate)
+
+    whole, parts = state.clone(), state.clone()
+    out = scan(0, requests, whole)
+    assert torch.equal(out, torch.cat([scan(0, 130, parts), scan(130, requests, parts)])) and torch.equal(whole, parts) and not torch.equal(whole, state)
+
+
 def test_decay_scan_of_single_tokens_costs_little_more_off_16_bytes(monkeypatch):
     """Rows of q and k that cannot be read 16 bytes at a time: 1.1 times the time of those that can (1.5 times where every lane read its own value by value)."""
     from mini_infer_amd import ops
