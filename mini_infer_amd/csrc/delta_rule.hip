@@ -679,7 +679,7 @@ extern "C" int mi_short_conv(int dtype, const void* x, int64_t x_stride, const f
   if (num_tokens == 0 || num_requests == 0) return MI_OK;
   const size_t elem = dtype == MI_F32 ? 4 : 2;
   if (taps >= 2 && taps <= 4 && channels % 4 == 0 && x_stride % 4 == 0 && y_stride % 4 == 0 && tail_stride % 4 == 0 &&
-      ((uintptr_t)x | (uintptr_t)y | (uintptr_t)tail) % (4 * elem) == 0 && (uintptr_t)w % 16 == 0 && channels <= 65535 * 1024) {
+      ((uintptr_t)x | (uintptr_t)y | (uintptr_t)tail) % (4 * elem) == 0 && (uintptr_t)w % 16 == 0 && channels <= 65535 * 1024 && num_tokens < 1 << 24) {
     // Rows a thread: more of them read a row 4, 1.75 and 1.4 times, fewer are more threads with shorter ways to memory.  Microseconds with 4 / 8: 1,777 x
     // 3,328 11.7 / 12.4, 2,048 x 6,144 16.7 / 14.8; with 1 / 8: 673 x 3,072 6.7 / 8.9.
     const int64_t values = (int64_t)num_tokens * channels;

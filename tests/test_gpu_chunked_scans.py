@@ -527,6 +527,22 @@ def test_decay_scan_of_more_blocks_than_a_launch_holds():
     assert torch.equal(out, torch.cat([scan(0, 130, parts), scan(130, requests, parts)])) and torch.equal(whole, parts) and not torch.equal(whole, state)
 
 
+def test_short_conv_of_more_rows_than_a_launch_holds():
+    """2^27 + 9 rows of four channels: the last ones, which come behind 2^24 blocks of 8."""
+    from mini_infer_amd import ops
+
+    tokens, channels, g = 2**27 + 9, 4, torch.Generator(device=DEV).manual_seed(43)
+    x = torch.zeros(tokens, channels, dtype=torch.bfloat16, device=DEV)
+    x[-40:] = torch.randn(40, channels, generator=g, device=DEV).bfloat16()
+    taps = torch.randn(channels, 4, generator=g, device=DEV)
+    tail = torch.zeros(2, 3, channels, dtype=torch.bfloat16, device=DEV)
+    cu, slots, of = _boundaries([tokens]), torch.zeros(1, dtype=torch.int32, device=DEV), torch.zeros(tokens, dtype=torch.int32, device=DEV)
+    got = ops.short_conv(x, channels, taps, tail, cu, slots, of)
+    last, own = x[-60:].contiguous(), torch.zeros(2, 3, channels, dtype=torch.bfloat16, device=DEV)
+    want = ops.short_conv(last, channels, taps, own, _boundaries([60]), slots, of[:60].contiguous())
+    assert torch.equal(got[-60:], want) and torch.equal(tail[0], own[0]) and not got[:-60].any()
+
+
 def test_decay_scan_of_single_tokens_costs_little_more_off_16_bytes(monkeypatch):
     """Rows of q and k that cannot be read 16 bytes at a time: 1.1 times the time of those that can (1.5 times where every lane read its own value by value)."""
     from mini_infer_amd import ops
