@@ -924,7 +924,7 @@ def qkv_rope_write(
     queries [M, q_heads*head_dim]; rotated keys and values go to their slots.  `kv_heads=0`
     with the query rows of the weight alone projects and rotates queries only.  The result
     is that of `linear` followed by `rope_kv_write` (both round the product to bfloat16
-    before rotating).  `x` may be `ScaledRows`: the rows' factors are then applied to the
+    before rotating; above 16 rows `linear` may sum in another order).  `x` may be `ScaledRows`: the rows' factors are then applied to the
     products' sums before they are rounded.
     """
     scaled = x if isinstance(x, ScaledRows) else None
@@ -979,26 +979,31 @@ def qkv_rope_write(
 @functools.lru_cache(maxsize=8192)
 def rotary_tiles_for(m: int, n: int, k: int, cus: int = WHOLE_DEVICE_CUS) -> int | None:
     """The tile shape where a rotary product of 33 to 1,024 rows is made in tiles, or None.  The tiles of `tiles_for` where those are whole.  Where
-    `linear` leaves the product to the vendor library, up to 320 rows the best whole tile, as that loses less to the library than the rotation's
-    launch takes; not where `linear` cuts K (10240 x 8192 at 100 rows in `qkv_rope_write_many_plan`), and not for a K above 4 times the
-    outputs, all of which a block would walk.  Microseconds of the two launches / this one, weights from memory:
+    that leaves the product to the vendor library, up to 320 rows the best whole tile, as that loses less than the rotation's
+    launch takes; not where it cuts K (10240 x 8192 at 100 rows in `qkv_rope_write_many_plan`), not for a K above 4 times the
+    outputs, all of which a block would walk, and up to 64 rows not above twice, of which `linear` then makes ranges or the sums of eight waves
+    (`small_product_plan`).  Microseconds of the two launches / this one, weights from memory:
 
-        rows             33             128            271            320
-        512 x 512        10.0 / 5.4     11.6 / 5.2     11.0 / 6.7     11.0 / 5.6
-        2304 x 768       11.3 / 6.3     12.4 / 6.3     12.6 / 8.3     12.5 / 7.3
-        3072 x 2048      15.4 / 10.1    18.6 / 10.9    18.0 / 13.4    18.0 / 13.1
-        768 x 3072       16.0 / 13.1    14.0 / 13.7    14.6 / 13.9    14.7 / 13.6
-        1536 x 4096      15.9 / 15.9    16.4 / 16.6    19.0 / 16.8    19.9 / 16.7
-        512 x 4096       15.4 / 15.6    16.3 / 15.6    14.5 / 16.0    14.7 / 15.1    (left to the two launches, as those below)
-        768 x 8192       15.7 / 27.5    18.4 / 28.5    24.0 / 27.8    24.1 / 28.0
-        512 x 14336      22.7 / 44.7    24.8 / 49.5    36.3 / 46.1    36.7 / 49.1
+        rows             33             64             128            271            320
+        512 x 512        6.7 / 5.2      6.8 / 5.2      6.9 / 5.2      7.8 / 6.5      7.8 / 5.3
+        2304 x 768       9.1 / 6.3      9.2 / 6.4      10.2 / 6.5     12.0 / 8.5     12.2 / 7.4
+        3072 x 2048      13.6 / 10.3    13.7 / 11.2    15.0 / 11.0    17.8 / 13.5    18.2 / 13.4
+        2048 x 3072      13.7 / 13.1    15.1 / 14.7    16.0 / 14.4
+        768 x 3072       10.2 / 12.8    10.6 / 12.7    12.2 / 12.8    13.3 / 13.4    13.4 / 12.5    (up to 64 rows the two launches)
+        1536 x 4096      13.4 / 16.0    14.9 / 17.3    17.1 / 17.2    19.6 / 17.1    20.6 / 17.2
+        512 x 4096       11.4 / 15.7    12.6 / 15.8    16.3 / 15.8    14.6 / 16.2    14.6 / 15.2    (left to the two launches, as those below)
+        768 x 8192       13.1 / 27.7    14.8 / 29.1    19.3 / 28.9    24.8 / 28.2    25.0 / 28.6
+        512 x 14336      14.7 / 45.3    14.8 / 50.6    24.9 / 50.0    36.3 / 46.7    36.3 / 49.8
 
-    and of those that `tiles_for` refuses from 289 rows on, at 289 rows 5120 x 3072 27.3 / 24.5, 9216 x 3072 38.6 / 31.6, 12288 x 4096 59.2 / 48.5, 14336 x
-    4096 56.1 / 51.8, 15360 x 5120 68.2 / 66.4.  From 16,000 outputs on nothing was measured, and the launch is left as it was."""
+    and of those that `tiles_for` refuses from 289 rows on, at 289 rows 5120 x 3072 28.9 / 25.5, 9216 x 3072 41.7 / 34.0, 12288 x 4096 59.6 / 54.8, 14336 x
+    4096 59.2 / 55.9, 15360 x 5120 73.5 / 69.1.  From 16,000 outputs on nothing was measured, and the launch is left as it was.
+
+    `linear` by itself sums some of these in another order up to 96 rows (ranges of K, eight waves), and is slower with the rotation's launch all the same: 3072 x
+    3072 at 64 / 80 / 96 rows 16.6 / 15.0, 17.8 / 14.1, 19.1 / 14.9, 4096 x 4096 at 80 / 96 20.2 / 16.8, 21.9 / 18.1, 4096 x 2048 at 48 / 64 14.1 / 10.7, 14.6 / 11.3."""
     plan = tiles_for(m, n, k, False, cus)
     if plan is not None:
         return plan[0] if plan[1] == 1 else None
-    if m >= TURNS_MIN_ROWS or n >= 16000 or k > 4 * n:
+    if m >= TURNS_MIN_ROWS or n >= 16000 or k > 4 * n or m <= 64 and k > 2 * n:
         return None
     return _tiles_plan(m, n, k, False, 1, False, 0.0, 0.0, cus)[1]
 
@@ -1009,13 +1014,14 @@ def qkv_rope_write_many_plan(x: torch.Tensor, weight: torch.Tensor, head_dim: in
     None: left to `linear` and `rope_kv_write`.  Whole heads of a multiple of 16, rotated in half pairing.  `others`: the tensors that it reads and
     writes beside these, which have to lie on 16 bytes.
 
-    Where `linear` makes whole tiles these are they, with the same results.  Microseconds of the two launches / this one, weights from memory:
+    Where `linear` makes whole tiles these are they, with the same results (where it sums in another order: `rotary_tiles_for`).  Microseconds of the two
+    launches / this one, weights from memory:
 
         rows                100            200            271            330            1000           2048           8192
-        3072 x 2048         16.3 / 10.5    17.3 / 12.3    18.1 / 13.3    20.7 / 15.9    26.4 / 21.2    35.3 / 29.3    103 / 86
-        5120 x 3072         21.0 / 16.3    24.1 / 19.6    26.9 / 22.4    27.4 / 22.5    45.0 / 40.3    69.8 / 64.7    217 / 194
-        6144 x 4096         25.0 / 20.8    32.1 / 27.0    33.6 / 28.7    39.7 / 34.6    58.3 / 52.6    90.4 / 83.8    308 / 283
-        10240 x 8192        44.5 / 57.0    64.1 / 62.7    74.5 / 67.4    78.2 / 73.5    153 / 147      284 / 274      949 / 895
+        3072 x 2048         14.4 / 10.6    17.1 / 12.6    17.5 / 13.5    19.7 / 16.3    27.3 / 21.7    37.0 / 31.5    109 / 93
+        5120 x 3072         22.1 / 17.1    25.4 / 20.5    27.2 / 22.6    28.0 / 23.3    45.7 / 41.6    71.4 / 67.1    227 / 206
+        6144 x 4096         27.0 / 22.2    33.3 / 28.0    34.8 / 29.9    40.7 / 35.5    58.4 / 53.2    96.0 / 90.1    326 / 305
+        10240 x 8192        47.8 / 61.6    67.5 / 66.6    77.1 / 72.8    78.6 / 73.6    162 / 153      300 / 289      1013 / 953
 
     Which tiles up to 320 rows: `rotary_tiles_for`."""
     if any(t is not None and t.data_ptr() % 16 != 0 for t in others):

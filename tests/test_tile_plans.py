@@ -146,6 +146,7 @@ def test_plain_products_with_few_outputs_for_their_k_are_the_librarys(m, n, k, g
     (271, 5120, 3072, "whole"), (100, 6144, 4096, "whole"), (100, 10240, 8192, None),       # as `linear` has them: whole tiles, K cut
     (33, 2304, 768, "own"), (320, 3072, 2048, "own"), (300, 15360, 5120, "own"), (100, 768, 3072, "own"), (100, 1536, 4096, "own"),
     (100, 512, 4096, None), (64, 768, 8192, None), (320, 512, 14336, None),                 # a block would walk a long K alone
+    (33, 768, 3072, None), (64, 1536, 4096, None), (64, 2048, 3072, "own"), (65, 768, 3072, "own"),  # `linear` in ranges, or eight waves
     (300, 16384, 4096, None), (321, 2304, 768, None), (400, 768, 3072, None)])
 def test_tiles_of_rotary_products(m, n, k, made):
     plan = kernels.tiles_for(m, n, k, False)
@@ -155,6 +156,17 @@ def test_tiles_of_rotary_products(m, n, k, made):
         assert plan == (shape, 1)
     elif made == "own":
         assert plan is None and kernels.tile_size(shape)[0] > 0
+
+
+@pytest.mark.parametrize("m, n, k, linear", [(64, 3072, 3072, "cut"), (96, 4096, 4096, "cut"), (48, 4096, 2048, "rows"), (64, 3072, 2048, "rows"), (80, 3072, 2048, "whole"),
+                                             (100, 3072, 3072, "whole"), (200, 3072, 2048, "whole")])
+def test_rotary_products_whose_plain_ones_are_made_otherwise(m, n, k, linear):
+    """Whole tiles, whatever `linear` by itself takes, which with the rotation's launch behind it is slower."""
+    small = kernels.small_product_plan(m, n, k)
+    form, shape, ranges = (None, *kernels.tiles_for(m, n, k, False)) if small is None else small
+    assert linear == ("rows" if form is not None else "whole" if ranges == 1 else "cut")
+    rotary = kernels.rotary_tiles_for(m, n, k)
+    assert rotary is not None and (linear != "whole" or rotary == shape)
 
 
 @pytest.mark.parametrize("m, n, k, plan", [
