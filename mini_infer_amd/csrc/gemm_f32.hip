@@ -544,13 +544,14 @@ static double f32_micros(int form, int how, int m, int n, int k, int count, int 
   const RowsCost& c = rows_cost[how];
   const int rt = of[form][0], ft = of[form][1], run = segment_slices(k), on_a_pipe = ceil_div(slices, run) > 4 ? 2 * run : run;
   const double r = rounds(16 * rt, 16 * ft);
-  return c.launch + ceil(r / 2) * run * c.trip + r * (c.round + c.tile * rt * ft + 4 * on_a_pipe * (c.product * rt * ft + c.operand * (rt + ft)));
+  const double t = c.launch + ceil(r / 2) * run * c.trip + r * (c.round + c.tile * rt * ft + 4 * on_a_pipe * (c.product * rt * ft + c.operand * (rt + ft)));
+  return r > 1 && run <= 4 && rt * ft >= 4 ? 1.15 * t : t;  // (large blocks in several rounds end and begin more than they multiply)
 }
 
 // The form of m rows for which the four-row products are not taken: the one that is expected to be the fastest.  (All give the same bits.)  Over the
 // products that the times are fitted to, as geometric means of the fastest form's time, in lines / in pieces / value by value: all rows a block up to 32 rows, or 64 with
 // less than 8,192 features, and tiles above 1.35 / 1.23 / 1.16; by times that know neither a tile's launch nor how operands are read 1.08 / 1.14 / 1.13 (13 x 512
-// x 160 6.8 for 3.5 us, 2 x 1024 x 145 8.2 / 4.0, 232 x 6418 x 1024 value by value 167 / 116); so 1.01 / 1.015 / 1.01.  In lines, weights from memory,
+// x 160 6.8 for 3.5 us, 2 x 1024 x 145 8.2 / 4.0, 232 x 6418 x 1024 value by value 167 / 116); so 1.008 / 1.013 / 1.010.  In lines, weights from memory,
 // before forms in blocks of rows / so:
 //     rows            25             64             96             128            256
 //     2048 x 2048     15.1 / 9.6     27.5 / 15.0    50.9 / 22.3    51.3 / 23.6    51.8 / 43.7

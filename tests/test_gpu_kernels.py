@@ -1981,7 +1981,7 @@ def test_every_form_of_the_float32_product_gives_the_same_bits(m, n, k):
 
 
 @pytest.mark.parametrize("m, n, k, first", [(13, 512, 160, 0), (43, 4096, 224, 0), (2, 1024, 145, 1), (11, 82, 140, 4), (136, 2048, 2048, 1), (232, 6418, 1024, 1),
-                                            (150, 8192, 908, 4), (25, 2048, 2048, 0), (256, 2048, 8192, 0), (509, 3072, 2048, 0)])
+                                            (150, 8192, 908, 4), (504, 3072, 512, 0), (383, 4096, 512, 0), (25, 2048, 2048, 0), (256, 2048, 8192, 0), (509, 3072, 2048, 0)])
 def test_the_form_of_a_float32_product_is_near_the_fastest(m, n, k, first):
     """A few slices of K and many, operands in whole lines, in pieces and value by value; recorded, so that the host's part is not in it."""
     from mini_infer_amd import ops
