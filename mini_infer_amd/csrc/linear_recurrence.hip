@@ -184,6 +184,10 @@ __device__ __forceinline__ void decay_token(const ScanArgs& p, int64_t t, int sl
   }
 }
 
+// whether a launch may have single tokens go through decay_token (in float32 launch_scan has the walk take them with one column block a block)
+template <typename T, int MODE, int R, int L, int G>
+constexpr bool MAY_BE_ALONE = MODE == DECAY_PER_HEAD && (sizeof(T) == 2 || (G > 1 && R * L > 64));
+
 // Decoded tokens, short portions and the 32-bit engine; long portions of bfloat16 steps go in chunks (decay_chunks.hip).
 // 256 threads keep 256 / L columns of a head's S, L lanes a column, R rows a lane.  Tokens are
 // taken SCAN_TILE at a time: a tile's rows are asked of memory while the tile before it is
@@ -370,22 +374,24 @@ __device__ __forceinline__ void decay_scan_columns(const ScanArgs& p, int b, int
 // side by side every eighth block was the long portion's where requests come in 8s: 31 single tokens beside 64 of 64 heads of 128 x 64 184 us, so 34;
 // 16 heads of 128 x 256 254 / 66.  Heads go round before columns: a head's column blocks then share an XCD's L2 (512 tokens of 64 heads 144 us, 164
 // the other way).
-// G: column blocks that a single token's block takes together (the other G - 1 leave at once); where there are enough blocks for that, launch_scan.
-// first_block: of this launch (a launch has no more than 2^32 threads).
+// The blocks are the launch's own three dimensions: in one row, divided up by every block, and with decay_token also where none goes through it, small
+// ones held up by both, 48 float32 requests of 64 heads of 16 x 64 13.2 us, so 11.2.
+// G: column blocks that a block takes, a single token's together, other requests' one after another (launch_scan says where).  With a block for every
+// column block, of which a single token's first took four and the others left at once, all work was on a quarter of the compute units with 8 heads:
+// 64 requests of 8 heads of 128 x 512 135 us, so 53, as one at a time 59.
 template <typename T, int MODE, int R, int L, int G>
-__global__ __launch_bounds__(256) void decay_scan_kernel(ScanArgs p, int requests, uint32_t first_block) {
+__global__ __launch_bounds__(256) void decay_scan_kernel(ScanArgs p, int last_request, int first_col_block) {
   constexpr int COLS = 256 / L;
-  const uint32_t each = p.heads * ((p.vdim + COLS - 1) / COLS), at = first_block + blockIdx.x;
-  const int b = requests - 1 - (int)(at / each), rest = (int)(at % each);
-  const int head = rest % p.heads, col_block = rest / p.heads;
-  if constexpr (MODE == DECAY_PER_HEAD) {
+  const int b = last_request - (int)blockIdx.z, head = blockIdx.x, col0 = (first_col_block + (int)blockIdx.y) * (G * COLS);
+  if constexpr (MAY_BE_ALONE<T, MODE, R, L, G>) {
     const int first = p.cu[b];
     if (p.tokens_alone && p.cu[b + 1] - first == 1) {
-      if (col_block % G == 0) decay_token<T, R, L, G>(p, first, p.slots[b], head, col_block * COLS);
+      decay_token<T, R, L, G>(p, first, p.slots[b], head, col0);
       return;
     }
   }
-  decay_scan_columns<T, MODE, R, L>(p, b, head, col_block * COLS);
+#pragma unroll 1
+  for (int g = 0; g < G && (g == 0 || col0 + g * COLS < p.vdim); ++g) decay_scan_columns<T, MODE, R, L>(p, b, head, col0 + g * COLS);
 }
 
 // rows per lane and lanes per column for a head whose keys are `dim` wide
@@ -397,18 +403,14 @@ inline void scan_shape(int dim, int* rows, int* lanes) {
   else *rows = 16, *lanes = 16;
 }
 
-constexpr int64_t MOST_BLOCKS = ((int64_t)1 << 24) - 1;  // of 256 threads
+constexpr int MOST_BLOCKS = 65535;  // of a launch's second and third dimension
 
 template <typename T, int MODE>
 int launch_scan(ScanArgs p, int tokens, int requests, hipStream_t stream) {
   int rows, lanes;
   scan_shape(p.dim, &rows, &lanes);
-  const int64_t grid = (int64_t)requests * p.heads * ceil_div(p.vdim, 256 / lanes);
-  MI_REQUIRE(grid < ((int64_t)1 << 32), "decay_scan: %lld blocks are too many", (long long)grid);
-  constexpr int TOGETHER = MODE == DECAY_PER_HEAD ? 4 : 1;
-  // (two rounds of what the CUs hold; 24 requests of 32 heads of 64 columns, 3,072 blocks, take the same either way.  Beside a long portion, whose
-  // chain the larger blocks hold up, one: 38 tokens beside 73, a step of 12 layers 2,910 / 2,928 us.)
-  const bool together = grid >= 4096 && tokens <= requests;
+  constexpr int TOGETHER = MODE == DECAY_PER_HEAD ? 4 : 1;  // column blocks
+  const int col_blocks = ceil_div(p.vdim, 256 / lanes);
   // Single tokens by decay_token: where rows of q and k are read a lane's run at a time, in float32 only four column blocks together and keys of more than 64.
   // Microseconds as in a walk / so, a decay per head, from memory: bfloat16, 64 heads of 128 x 64, 8 / 40 requests 11.5 / 10.1 and 44.9 / 35.9, 48 of 64 x 64 6.0 / 5.4 and
   // 19.8 / 17.0; value by value 64 of 100 x 64 at 8 11.4 / 17.0, 24 of 200 x 256 33.5 / 61.5 and 121 / 183, 64 of 256 x 64 24.1 / 50.2 and 88.8 / 116; float32, 64 of
@@ -417,15 +419,21 @@ int launch_scan(ScanArgs p, int tokens, int requests, hipStream_t stream) {
   auto in_pieces = [&](const void* row, int64_t stride, int col) {
     return ((uintptr_t)row + (uintptr_t)col * sizeof(T)) % piece == 0 && stride * sizeof(T) % piece == 0;
   };
-  p.tokens_alone = p.dim % rows == 0 && in_pieces(p.q, p.q_stride, p.q_col) && in_pieces(p.k, p.k_stride, p.k_col) &&
-                   (sizeof(T) == 2 || (together && p.dim > 64));
-#define MI_SCAN(RR, LL)                                                                                                    \
-  do {                                                                                                                     \
-    if (together) decay_scan_kernel<T, MODE, RR, LL, TOGETHER><<<blocks, 256, 0, stream>>>(p, requests, (uint32_t)first);  \
-    else decay_scan_kernel<T, MODE, RR, LL, 1><<<blocks, 256, 0, stream>>>(p, requests, (uint32_t)first);                  \
+  p.tokens_alone = p.dim % rows == 0 && in_pieces(p.q, p.q_stride, p.q_col) && in_pieces(p.k, p.k_stride, p.k_col);
+  // Four column blocks together from two rounds of what the CUs hold on; 24 requests of 32 heads of 64 columns, 3,072 blocks, take the same either way.  Beside a long
+  // portion, whose chain the larger blocks hold up, one: 38 tokens beside 73, a step of 12 layers 2,910 / 2,928 us.  (A head's last block would read for four
+  // whatever it holds: heads of whole fours only.)
+  const bool together = TOGETHER > 1 && p.tokens_alone && (sizeof(T) == 2 || p.dim > 64) && tokens <= requests &&
+                        (int64_t)requests * p.heads * col_blocks >= 4096 && col_blocks % TOGETHER == 0;
+  MI_REQUIRE(p.heads < (1 << 24), "decay_scan: %d heads are too many", p.heads);
+  const int each = together ? col_blocks / TOGETHER : col_blocks;
+#define MI_SCAN(RR, LL)                                                                                              \
+  do {                                                                                                               \
+    if (together) decay_scan_kernel<T, MODE, RR, LL, TOGETHER><<<grid, 256, 0, stream>>>(p, requests - 1 - r, c);     \
+    else decay_scan_kernel<T, MODE, RR, LL, 1><<<grid, 256, 0, stream>>>(p, requests - 1 - r, c);                     \
   } while (0)
-  for (int64_t first = 0; first < grid; first += MOST_BLOCKS) {
-    const unsigned blocks = (unsigned)min(MOST_BLOCKS, grid - first);
+  for (int r = 0; r < requests; r += MOST_BLOCKS) for (int c = 0; c < each; c += MOST_BLOCKS) {
+    const dim3 grid(p.heads, min(MOST_BLOCKS, each - c), min(MOST_BLOCKS, requests - r));
     if (rows == 4) MI_SCAN(4, 4);
     else if (rows == 8 && lanes == 4) MI_SCAN(8, 4);
     else if (rows == 8 && lanes == 8) MI_SCAN(8, 8);

@@ -473,7 +473,9 @@ def test_a_recorded_step_is_not_taken_for_single_tokens():
 
 
 @pytest.mark.parametrize("heads,groups,dim,vdim", [(4, 2, 64, 64), (6, 3, 96, 80), (2, 1, 256, 250), (3, 3, 20, 30), (2, 2, 128, 128), (2, 1, 12, 7), (300, 3, 40, 70),
-                                                   (520, 2, 128, 20)])  # (with so many heads a token's block takes four times the columns)
+                                                   (520, 2, 128, 20),
+                                                   # four column blocks together: 4,096 blocks and more, a multiple of four a head
+                                                   (300, 3, 40, 128), (300, 3, 20, 200), (270, 2, 128, 60), (258, 1, 256, 64), (130, 1, 12, 512)])
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 @pytest.mark.parametrize("odd", [False, True])
 def test_decay_scan_of_single_tokens_gives_the_bits_of_portions(monkeypatch, heads, groups, dim, vdim, dtype, odd):
@@ -506,11 +508,12 @@ def test_decay_scan_of_single_tokens_gives_the_bits_of_portions(monkeypatch, hea
     assert torch.equal(single[:-1], whole[:-1])
 
 
-def test_decay_scan_of_more_blocks_than_a_launch_holds():
-    """257 requests of 65,535 heads are 2^24 blocks and more: the same as in two steps."""
+@pytest.mark.parametrize("heads,requests", [(65535, 257), (2, 65540)])
+def test_decay_scan_of_more_blocks_than_a_launch_holds(heads, requests):
+    """2^24 blocks and more, and more requests than a launch's third dimension takes: the same as in two steps."""
     from mini_infer_amd import ops
 
-    heads, dim, vdim, requests = 65535, 12, 1, 257
+    dim, vdim = 12, 1
     g = torch.Generator(device=DEV).manual_seed(41)
     qk, v, gate = (torch.randn(requests, n, generator=g, device=DEV).bfloat16() for n in (2 * dim, heads * vdim, heads))
     bias, rate = torch.zeros(heads, device=DEV), torch.zeros(heads, device=DEV)
@@ -541,6 +544,29 @@ def test_short_conv_of_more_rows_than_a_launch_holds():
     last, own = x[-60:].contiguous(), torch.zeros(2, 3, channels, dtype=torch.bfloat16, device=DEV)
     want = ops.short_conv(last, channels, taps, own, _boundaries([60]), slots, of[:60].contiguous())
     assert torch.equal(got[-60:], want) and torch.equal(tail[0], own[0]) and not got[:-60].any()
+
+
+def test_decay_scan_of_single_tokens_takes_few_heads_as_fast_as_many():
+    """64 requests of 134 MB of states in 8 heads of 512 columns and in 64 of 64: 1.0 times (2.4 times where one block in four had work)."""
+    from mini_infer_amd import ops
+
+    dim, requests, g, took = 128, 64, torch.Generator(device=DEV).manual_seed(47), []
+    cu, slots = _boundaries([1] * requests), torch.arange(requests, dtype=torch.int32, device=DEV)
+    for heads, vdim in ((64, 64), (8, 512)):
+        bias, rate = torch.zeros(heads, device=DEV), torch.zeros(heads, device=DEV)
+        state = _state(g, requests, ops.decay_state_shape(heads, dim, vdim), dim)
+        q, k, v, gate = (_rows(g, requests, n, False) for n in (dim, dim, heads * vdim, heads))
+        times = []
+        for _ in range(6):
+            begin, end = (torch.cuda.Event(enable_timing=True) for _ in range(2))
+            begin.record()
+            for _ in range(10):
+                ops.decay_scan(q, 0, k, 0, v, 0, gate, 0, bias, state, cu, slots, heads=heads, groups=1, dim=dim, vdim=vdim, per_head=True, rate=rate)
+            end.record()
+            end.synchronize()
+            times.append(begin.elapsed_time(end))
+        took.append(min(times))
+    assert took[1] < 1.4 * took[0], took
 
 
 def test_decay_scan_of_single_tokens_costs_little_more_off_16_bytes(monkeypatch):
