@@ -475,7 +475,7 @@ static int attn_generic_launch(const void* q, int64_t q_row_stride, const void* 
   //
   // Values of 129 to 256 dims, of which fewer blocks are on a CU, one wave / four: latent rows of 288, 32 heads, 4 tokens of up to 300 positions 88 / 33 us a layer, 128 of
   // up to 153 (1,024 blocks) 95 / 68; by blocks and keys of a range, 336 x 307 178 / 81, 960 x 290 213 / 179, 1,184 x 264 201 / 175, 544 x 72 44 / 57, 1,372 x 272 214 / 245, 1,488 x
-  // 459 360 / 291, 1,776 x 320 192 / 280, 1,760 x 278 232 / 294, 1,920 x 549 311 / 341.
+  // 459 360 / 291, 1,568 x 573 412 / 468, 1,776 x 320 192 / 280, 1,760 x 278 232 / 294, 1,920 x 549 311 / 341.
   //
   // Up to three blocks a CU a wave has one or two 64s of keys and its time is the waits one after another, so that more loads in flight
   // (DEEP) are worth two blocks a CU at once instead of three; for values of up to 64 dims, of which less is in flight, as long as two
@@ -490,7 +490,7 @@ static int attn_generic_launch(const void* q, int64_t q_row_stride, const void* 
   if (mask_chunk > 0) keys = keys < mask_chunk ? keys : mask_chunk;
   keys = ceil_div64(keys, num_splits);
   const bool four = sizeof(S) == 8 && (v_dim <= 128 ? blocks < 2048 && keys > MI_WAVE * ceil_div64(blocks, 768)
-                                       : v_dim <= 256 && (blocks <= 1200 ? keys > MI_WAVE * ceil_div64(blocks, 512) : blocks < 1600 && keys > 400));
+                                       : v_dim <= 256 && (blocks <= 1200 ? keys > MI_WAVE * ceil_div64(blocks, 512) : blocks <= 1536 && keys > 400));
   // One head a block instead of four where that is at most two blocks a CU, the 32-bit path: four heads are four times the work on the way through a wave's
   // keys, and the CUs are idle (the same bits; keys and values are read by as many blocks as there are heads, from L2).  Microseconds, four heads / one: 32 heads of
   // 64 over 8, 1 / 3 / 6 tokens of 100 positions 14.5 / 10.5, of 600 28.3 / 20.6, 22.2, 26.8, 1 of 2,000 29.6 / 23.5 (3: 768 blocks, 30.5 / 35.1), 12 of 100 14.6 / 12.1;
